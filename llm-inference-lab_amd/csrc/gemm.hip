@@ -30,9 +30,10 @@
 //       issuing MFMAs, both operands loaded from global memory straight into LDS
 //       (gemm_bf16_pingpong): 1.1 to 1.17 PF/s where the tiles above reach 0.9 to 0.97.
 //     (products of few rows, as in decode steps, have kernels of their own in decode.hip)
-//   float32: a plain FMA kernel (tiles of 64x64 to 128x128, 4x4 to 8x8 outputs per thread) and, for up to 64
-//     rows, one in which a wave owns four rows of W and its lanes split the inner size:
-//     true 32-bit products and sums, no matrix-core shortcut.
+//   float32: numbers split into three bfloat16 parts for the matrix cores, 32-bit products and sums
+//     as exact as plain FMAs (gemm_f32_split_kernel); a plain FMA kernel beside it as its
+//     reference (tiles of 64x64 to 128x128, 4x4 to 8x8 outputs per thread); for up to 64 rows one in
+//     which a wave owns four rows of W and its lanes split the inner size.
 //
 // Fragment layout of the 16x16x32 MFMA (wave of 64 lanes, lane l):
 //   A operand: row l%16, k = 8*(l/16) .. +7      B operand: column l%16, same k
@@ -819,129 +820,277 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   }
 }
 
-// Many rows in float32 on the matrix cores: v_mfma_f32_32x32x2_f32 multiplies and sums in
-// true 32 bits (no reduced-precision mode) at twice the rate of unpacked FMAs and with one
-// LDS read per operand and instruction.  BM x BN outputs per block of four waves (2 x 2);
-// both operands through LDS in steps of 16 of the inner size (rows padded to 17 floats:
-// the lanes of an instruction read one number each from 32 consecutive rows without
-// bank conflicts), the next step's numbers on their way from memory meanwhile.  The
-// product is taken transposed, C^T[n, m] = W x^T, so that a lane holds one row m of the
-// output and 16 of its columns, four and four next to each other, and for SWIGLU the gate
-// and the up value of an output in the same lane.
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
-template <int EPI, int BM, int BN>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ A,
-                                                             const float* __restrict__ W, EpiArgs e, int M,
-                                                             int N, int K, int vec) {
-  constexpr int KT = 16, LD = KT + 1;
-  constexpr int TM = BM / 64, TN = BN / 64;            // 32 x 32 tiles per wave along m and n
-  constexpr int LA = BM * KT / 4 / 256, LB = BN * KT / 4 / 256;     // 16-byte pieces per thread and step
-  __shared__ float Xs[BM * LD];
-  __shared__ float Ws[BN * LD];
+// Many rows in float32: the products are taken by the bfloat16 matrix instructions without giving
+// up a bit of the operands.  A float32 number is the sum of three bfloat16 numbers, x = h + m + l (h =
+// x rounded to nearest, m = x - h rounded, l the rest: 24 bits of significand in three times 8, the
+// differences exact), and x w = h_x h_w + h_x m_w + m_x h_w + m_x m_w + h_x l_w + l_x h_w up to terms below
+// 2^-24 of |x w|, less than what one rounding of a 32-bit sum costs.  Every bfloat16 product is
+// exact in float32 and the sums are float32; an instruction adds 32 of them where
+// v_mfma_f32_32x32x2_f32 adds 2, so fewer roundings meet in a sum (relative error of a product of
+// normal numbers against 64 bits: inner size 896 4.5e-7, 5.4e-7 with the float32 instructions; 4,864 1.1e-6
+// and 1.25e-6, 6e-7 in three pieces).  Six instructions at 16 times the rate of the float32 ones, measured
+// against tiles of v_mfma_f32_32x32x2_f32 (which this replaces; 157 TFLOP/s is what those could reach): 1,531
+// rows of 9728 x 896 186 us against 266 (144 TFLOP/s of 32-bit products), of 896 x 4864 in three pieces 81
+// against 215, 4,000 rows of 17920 x 1536 1,348 against 1,831, 65 rows of 1536 x 8960 48 in eight pieces against 252.
+// What bounds it: in full rounds the power limit (0.98 PFLOP/s of bfloat16 products), in a round by itself
+// a step's trip through LDS (1.3 us where its matrix instructions need 0.7).
+//
+// BM x BN outputs per block of WM x WN waves, steps of 32 of the inner size.  A thread
+// fetches eight numbers of a row as they lie in memory, three steps ahead, splits them in registers and
+// puts the three parts down in LDS in fragment order, [16 rows][part][lane][8], so that writes
+// and reads are 1 KB of consecutive bytes a wave.  Lane (c, g) of a fragment holds the numbers 4 g
+// .. 4 g + 3 and 16 + 4 g .. of its row's 32 (the order inside a step is free, both operands share
+// it), so that four lanes read 64 consecutive bytes.  Two stages of LDS: the next step is split and put down
+// between the matrix instructions of this one, a barrier a step.  The product is taken transposed, C^T = W
+// x^T, so that a lane holds four neighbouring columns of a row, and for SWIGLU the gate and the up
+// value of an output.
+//
+// Numbers that bfloat16 would round to infinity (3.396e38 and above, and infinity itself) have no
+// such parts: a block that meets one takes its outputs again with plain FMAs at the end.  (NaN needs no
+// care: all three parts are NaN.)
+constexpr float SPLIT_LIMIT = 3.3961775e38f;       // the smallest number that rounds to infinity in bfloat16
+template <int EPI, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const float* __restrict__ A,
+                                                                const float* __restrict__ W, EpiArgs e, int M,
+                                                                int N, int K, int vec) {
+  constexpr int BK = 32, NW = WM * WN;
+  constexpr int TM = BM / 16 / WM, TN = BN / 16 / WN;    // 16 x 16 tiles per wave along m and n
+  constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW;    // pieces of eight numbers per thread and step
+  static_assert(LA >= 1 && LB >= 1 && LA * NW * 16 == BM && LB * NW * 16 == BN && TN % 2 == 0, "pieces");
+  constexpr int STAGE = (BM + BN) / 16 * 3072;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
+  __shared__ int s_big;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int r32 = lane & 31, kk = lane >> 5;
-  floatx16 acc[TN][TM];
+  const int wm = wave % WM, wn = wave / WM;
+  int bx = blockIdx.x, by = blockIdx.y;
+  {                                                      // a band of column tiles per die, as above
+    const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
+    const int lin = by * gx + bx;
+    const int whole = total & ~7;
+    const int mapped = lin < whole ? (lin & 7) * (whole >> 3) + (lin >> 3) : lin;
+    bx = mapped / gy;
+    by = mapped - bx * gy;
+  }
+  const int m0 = by * BM, n0 = bx * BN;
+  const int c = lane & 15, g = lane >> 4;
+  // this block's range of the inner size (PART: its group's share, whole steps)
+  int k_begin = 0, k_end = K;
+  if constexpr (EPI == EPI_PART) {
+    k_begin = min(K, (int)blockIdx.z * e.kt_per_split * BK);
+    k_end = min(K, k_begin + e.kt_per_split * BK);
+    e.out = (float*)e.out + (size_t)blockIdx.z * e.part_stride;
+    if (blockIdx.z > 0) e.bias = nullptr;
+  }
+  if (tid == 0) s_big = 0;
+
+  floatx4 acc[TN][TM];
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // piece x of a thread: row (wave + NW x) * 16 + c of the tile, numbers 4 g .. and 16 + 4 g .. of the step
+  const float* ap[LA];
+  const float* bp[LB];
 #pragma unroll
-      for (int x = 0; x < 16; ++x) acc[j][i][x] = 0.f;
-  floatx4 ra[LA], rb[LB];
-  // piece p of a tile: row p / 4, numbers 4 (p % 4) .. + 3 of the step
-  auto fetch = [&](int k0) {
+  for (int x = 0; x < LA; ++x) ap[x] = A + (size_t)min(m0 + (wave + NW * x) * 16 + c, M - 1) * K;
 #pragma unroll
-    for (int x = 0; x < LA; ++x) {
-      const int p = tid + x * 256, row = p >> 2, kq = (p & 3) * 4;
-      const float* src = A + (size_t)min(m0 + row, M - 1) * K + k0 + kq;
-      if (vec && k0 + kq + 4 <= K) ra[x] = *(const floatx4*)src;
-      else
+  for (int x = 0; x < LB; ++x) bp[x] = W + (size_t)min(n0 + (wave + NW * x) * 16 + c, N - 1) * K;
+  struct Pieces {
+    floatx4 a[LA][2], b[LB][2];
+  };
+  auto guarded = [&](const float* row, int k) {
+    floatx4 v;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) ra[x][c] = k0 + kq + c < K ? src[c] : 0.f;
-    }
+    for (int q = 0; q < 4; ++q) v[q] = k + q < k_end ? row[k + q] : 0.f;
+    return v;
+  };
+  auto fetch = [&](Pieces& r, int k0) {
+    if (vec && k0 + BK <= k_end) {
 #pragma unroll
-    for (int x = 0; x < LB; ++x) {
-      const int p = tid + x * 256, row = p >> 2, kq = (p & 3) * 4;
-      const float* src = W + (size_t)min(n0 + row, N - 1) * K + k0 + kq;
-      if (vec && k0 + kq + 4 <= K) rb[x] = *(const floatx4*)src;
-      else
+      for (int x = 0; x < LB; ++x) {
+        r.b[x][0] = *(const floatx4*)(bp[x] + k0 + 4 * g);
+        r.b[x][1] = *(const floatx4*)(bp[x] + k0 + 16 + 4 * g);
+      }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) rb[x][c] = k0 + kq + c < K ? src[c] : 0.f;
+      for (int x = 0; x < LA; ++x) {
+        r.a[x][0] = *(const floatx4*)(ap[x] + k0 + 4 * g);
+        r.a[x][1] = *(const floatx4*)(ap[x] + k0 + 16 + 4 * g);
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < LB; ++x) {
+        r.b[x][0] = guarded(bp[x], k0 + 4 * g);
+        r.b[x][1] = guarded(bp[x], k0 + 16 + 4 * g);
+      }
+#pragma unroll
+      for (int x = 0; x < LA; ++x) {
+        r.a[x][0] = guarded(ap[x], k0 + 4 * g);
+        r.a[x][1] = guarded(ap[x], k0 + 16 + 4 * g);
+      }
     }
   };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += KT) {
-    __syncthreads();
+  float biggest = 0.f;
+  auto split = [&](const floatx4 (&v)[2], char* to) {
+    bf16x8 h, m, l;
 #pragma unroll
-    for (int x = 0; x < LA; ++x) {
-      const int p = tid + x * 256, row = p >> 2, kq = (p & 3) * 4;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) Xs[row * LD + kq + c] = ra[x][c];
+    for (int q = 0; q < 8; ++q) {
+      const float x = v[q >> 2][q & 3];
+      biggest = fmaxf(biggest, fabsf(x));
+      h[q] = (bf16_t)x;
+      const float r = x - (float)h[q];
+      m[q] = (bf16_t)r;
+      l[q] = (bf16_t)(r - (float)m[q]);
     }
+    *(bf16x8*)to = h;
+    *(bf16x8*)(to + 1024) = m;
+    *(bf16x8*)(to + 2048) = l;
+  };
+  auto stash = [&](const Pieces& r, int stage) {
+    char* to = smem + stage * STAGE + lane * 16;
 #pragma unroll
-    for (int x = 0; x < LB; ++x) {
-      const int p = tid + x * 256, row = p >> 2, kq = (p & 3) * 4;
+    for (int x = 0; x < LA; ++x) split(r.a[x], to + (wave + NW * x) * 3072);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) Ws[row * LD + kq + c] = rb[x][c];
-    }
-    __syncthreads();
-    if (k0 + KT < K) fetch(k0 + KT);
+    for (int x = 0; x < LB; ++x) split(r.b[x], to + (BM / 16 + wave + NW * x) * 3072);
+  };
+  auto multiply = [&](int stage, auto between) {
+    const char* xs = smem + stage * STAGE + lane * 16;
+    const char* ws = xs + BM / 16 * 3072;
+    bf16x8 xf[3][TM], wf[3][TN];
+    auto parts = [&](int p) {
 #pragma unroll
-    for (int s2 = 0; s2 < KT; s2 += 2) {
-      float wv[TN], xv[TM];
+      for (int i = 0; i < TM; ++i) xf[p][i] = *(const bf16x8*)(xs + ((wm * TM + i) * 3 + p) * 1024);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) wv[j] = Ws[(wn * (BN / 2) + j * 32 + r32) * LD + s2 + kk];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) xv[i] = Xs[(wm * (BM / 2) + i * 32 + r32) * LD + s2 + kk];
+      for (int j = 0; j < TN; ++j) wf[p][j] = *(const bf16x8*)(ws + ((wn * TN + j) * 3 + p) * 1024);
+    };
+    auto products = [&](int pw, int px) {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
-          acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[j], xv[i], acc[j][i], 0, 0, 0);
+          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[pw][j], xf[px][i], acc[j][i], 0, 0, 0);
+    };
+    parts(1);
+    parts(0);
+    parts(2);
+    products(1, 1);            // m_w m_x
+    between();
+    products(1, 0);
+    products(0, 1);
+    products(2, 0);
+    products(0, 2);
+    products(0, 0);            // h_w h_x
+  };
+
+  // Step t lies in stage t % 2; it is put there while step t - 1 is multiplied, from registers
+  // that were asked for three steps ahead.
+  const int steps = (k_end - k_begin + BK - 1) / BK;
+  if (steps > 0) {
+    Pieces r0, r1;
+    fetch(r0, k_begin);
+    fetch(r1, k_begin + BK);
+    stash(r0, 0);
+    fetch(r0, k_begin + 2 * BK);
+    __syncthreads();
+    for (int t = 0; t < steps; t += 2) {
+      const int k0 = k_begin + t * BK;
+      multiply(0, [&]() { stash(r1, 1); });          // (past the last step: zeros, never read)
+      fetch(r1, k0 + 3 * BK);
+      __syncthreads();
+      if (t + 1 >= steps) break;
+      multiply(1, [&]() { stash(r0, 0); });
+      fetch(r0, k0 + 4 * BK);
+      __syncthreads();
     }
   }
-  // lane (r32, kk) holds, of every 32 x 32 tile, output row m = r32 and the columns
-  // n = 8 (x / 4) + 4 kk + x % 4 for x = 0 .. 15
+  if (biggest >= SPLIT_LIMIT) s_big = 1;      // (any thread's; the same value from all)
+  __syncthreads();
+  if (s_big) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const float* xrow = A + (size_t)min(m0 + (wm * TM + i) * 16 + c, M - 1) * K;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        for (int x = 0; x < 4; ++x) {
+          const float* wrow = W + (size_t)min(n0 + (wn * TN + j) * 16 + 4 * g + x, N - 1) * K;
+          float sum = 0.f;
+          for (int k = k_begin; k < k_end; ++k) sum = fmaf(xrow[k], wrow[k], sum);
+          acc[j][i][x] = sum;
+        }
+    }
+  }
+  // lane (c, g) holds, of every 16 x 16 tile, output row m = c and the columns n = 4 g .. 4 g + 3
+  const bool whole_pieces = (e.ldo & 3) == 0 && ((uintptr_t)e.out & 15) == 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int m = m0 + wm * (BM / 2) + i * 32 + r32;
+    const int m = m0 + (wm * TM + i) * 16 + c;
     if (m >= M) continue;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int nb = n0 + wn * (BN / 2) + j * 32;
+      const int nb = n0 + (wn * TN + j) * 16;
       if constexpr (EPI == EPI_SWIGLU) {
-        // columns 0 .. 15 of the 32 are gate, 16 .. 31 the up values of the same outputs
+        // tiles of columns alternate: gate, up of the same 16 outputs
+        if (j & 1) continue;
+        const int o = (nb >> 5) * 16 + 4 * g;
+        floatx4 v;
 #pragma unroll
-        for (int x = 0; x < 8; ++x) {
-          const int o = (nb >> 5) * 16 + 8 * (x >> 2) + 4 * kk + (x & 3);
-          if (o < e.n_out) ((float*)e.out)[(size_t)m * e.ldo + o] = pair_exact_f(acc[j][i][x], acc[j][i][x + 8], e);
-        }
+        for (int x = 0; x < 4; ++x) v[x] = pair_exact_f(acc[j][i][x], acc[j + 1][i][x], e);
+        float* dst = (float*)e.out + (size_t)m * e.ldo + o;
+        if (whole_pieces && o + 4 <= e.n_out) *(floatx4*)dst = v;
+        else
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            if (o + x < e.n_out) dst[x] = v[x];
       } else {
+        const int n = nb + 4 * g;
+        floatx4 v = acc[j][i];
+        if (e.bias)
 #pragma unroll
-        for (int x = 0; x < 16; ++x) {
-          const int n = nb + 8 * (x >> 2) + 4 * kk + (x & 3);
-          if (n < N) epi_store<float, EPI>(e, m, n, acc[j][i][x]);
+          for (int x = 0; x < 4; ++x) v[x] += load_vec(e.bias, e.bias_bf16, min(n + x, N - 1));
+        if (EPI == EPI_STORE && e.act)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v[x] = relu2_f(v[x]);
+        float* dst = (float*)e.out + (size_t)m * e.ldo + n;
+        if (whole_pieces && n + 4 <= N) {
+          if (EPI == EPI_RESID) v += *(const floatx4*)dst;
+          *(floatx4*)dst = v;
+        } else {
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            if (n + x < N) dst[x] = (EPI == EPI_RESID ? dst[x] : 0.f) + v[x];
         }
       }
     }
   }
 }
 
-// The largest tile that still gives every compute unit a block.
+// The tile of a float32 product of many rows, and into how many pieces along the inner size one that adds
+// into the stream is cut.
+struct F32Plan {
+  int bm, pieces;
+};
+static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int min_steps);
+
+template <int EPI>
+static void launch_f32_split(int bm, const float* A, const float* W, const EpiArgs& e, int M, int N, int K, int pieces,
+                             hipStream_t stream) {
+  const int vec = (K % 4 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);
+  const dim3 grid((N + bm - 1) / bm, (M + bm - 1) / bm, pieces);
+  if (bm == 128)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 128, 128, 2, 4>), grid, dim3(512), 0, stream, A, W, e, M, N, K, vec);
+  else
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 64, 64, 2, 2>), grid, dim3(256), 0, stream, A, W, e, M, N, K, vec);
+}
+
+// Products of many rows in float32: the matrix cores, or (debug) the plain FMA kernel, their reference, with
+// the largest tile that still gives every compute unit a block.
 template <int EPI>
 static void launch_f32_tiled(const float* A, const float* W, const EpiArgs& e, int M, int N, int K,
                              int num_cus, hipStream_t stream) {
   const int vec = (K % 4 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);
   auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  if (g_f32_fma == 0) {       // the matrix cores (the plain FMA kernels below stay as their reference)
-    if (blocks(128, 128) >= num_cus)
-      hipLaunchKernelGGL((gemm_f32_mfma_kernel<EPI, 128, 128>), dim3((N + 127) / 128, (M + 127) / 128), dim3(256),
-                         0, stream, A, W, e, M, N, K, vec);
-    else
-      hipLaunchKernelGGL((gemm_f32_mfma_kernel<EPI, 64, 64>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0,
-                         stream, A, W, e, M, N, K, vec);
+  if (g_f32_fma == 0) {
+    launch_f32_split<EPI>(f32_plan(M, N, K, num_cus, 1, 1).bm, A, W, e, M, N, K, 1, stream);
     return;
   }
   if (blocks(128, 128) >= num_cus)
@@ -1190,6 +1339,40 @@ extern "C" void llmlab_debug_gemm_tile(int tile) {
   g_pp_min_rows = tile <= -256 ? -tile : 512;
 }
 
+// By an estimate of the time, fitted to a sweep of seven matrices of two model shapes at 65 to 4,000 rows
+// whole and in up to eight pieces (within 12 % of the measurement; its picks lose 0.1 % on average, 5 % at most, to the best of the sweep).  A block of the 128 x
+// 128 tile is alone on its unit, rounds are whole; of the 64 x 64 tile three share one, whose first is slow by
+// itself (0.86 us a step for its own chain of trips, 0.58 where others fill the gaps).
+static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int min_steps) {
+  const int steps = (K + 31) / 32;
+  F32Plan best{0, 1};
+  double least = 0.0;
+  for (int bm = 64; bm <= 128; bm += 64) {
+    if (g_force_tile == 64 && bm != 64) continue;
+    if ((g_force_tile == 128 || g_force_tile == 129) && bm != 128) continue;
+    for (int pieces = 1; pieces <= max_pieces; ++pieces) {
+      const int s = (steps + pieces - 1) / pieces;
+      if (pieces > 1 && s < min_steps) break;
+      const double share = (double)((M + bm - 1) / bm) * ((N + bm - 1) / bm) * pieces / num_cus;
+      const double whole = ceil(share - 1e-9);
+      double t;
+      if (bm == 128) {
+        t = whole * (5.4 + s * (1.31 + 0.12 * (share < 1.0 ? share : 1.0)));
+      } else {
+        const double shared = (share <= 3.0 ? whole : share) * (1.0 + 0.58 * s);
+        t = 2.0 + 0.863 * s;
+        if (shared > t && whole > 1.0) t = shared;
+      }
+      if (pieces > 1) t += pieces * ((double)M * N * 2.2e-6 + 0.3);      // (their way through memory to the next reader)
+      if (best.bm == 0 || t < least) {
+        least = t;
+        best = F32Plan{bm, pieces};
+      }
+    }
+  }
+  return best;
+}
+
 static int choose_tile(int M, int N, int K, int num_cus) {
   if (g_force_tile == 64) return TILE_64;
   if (g_force_tile == 130) return TILE_64x128;
@@ -1413,6 +1596,14 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   out[1] = best_kind;
 }
 
+// The same for a float32 product (of more rows than the few-row kernel takes).
+extern "C" void llmlab_linear_plan_f32(int M, int N, int K, int num_cus, int max_pieces, int min_steps_per_piece,
+                                       int* out) {
+  const F32Plan plan = f32_plan(M, N, K, num_cus > 0 ? num_cus : 256, max_pieces, min_steps_per_piece);
+  out[0] = plan.pieces;
+  out[1] = plan.bm == 128 ? TILE_128 : TILE_64;
+}
+
 // q/k/v projection of many rows with bias, rotation and cache write in the epilogue
 // (bfloat16).  The tile is chosen as for any product; the head size must divide it.
 extern "C" int llmlab_linear_qkv(const void* x, const void* w, const void* bias, int bias_dtype, void* q_out,
@@ -1449,14 +1640,24 @@ extern "C" int llmlab_linear_tile(int M, int N, int K, int num_cus) {
 }
 
 // parts[z] = x[:, K_z] . W[:, K_z]^T for `ksplit` ranges K_z of the inner size (whole K
-// tiles of 64 each); bias in parts[0].  bfloat16 only; `tile` as llmlab_linear_plan gives it.
-extern "C" int llmlab_linear_partials(const void* x, const void* w, float* parts, const void* bias,
+// tiles of 64 each, in float32 whole steps of 32); bias in parts[0].  `tile` as llmlab_linear_plan gives it.
+extern "C" int llmlab_linear_partials(const void* x, const void* w, int dtype, float* parts, const void* bias,
                                       int bias_dtype, int M, int N, int K, int ldo, int ksplit,
                                       size_t part_stride, int tile, hipStream_t stream) {
-  LLMLAB_REQUIRE(M >= 0 && N > 0 && K > 0 && K % 8 == 0, "linear_partials: bad sizes M=%d N=%d K=%d", M, N, K);
+  LLMLAB_REQUIRE(M >= 0 && N > 0 && K > 0 && (dtype == DT_F32 || K % 8 == 0), "linear_partials: bad sizes M=%d N=%d K=%d",
+                 M, N, K);
   LLMLAB_REQUIRE(ksplit >= 1 && ksplit <= 16 && ldo >= N && part_stride >= (size_t)M * ldo,
                  "linear_partials: %d pieces, row stride %d", ksplit, ldo);
   LLMLAB_REQUIRE(tile >= TILE_64 && tile < TILE_KINDS, "linear_partials: unknown tile %d", tile);
+  if (dtype == DT_F32) {
+    LLMLAB_REQUIRE(tile == TILE_64 || tile == TILE_128, "linear_partials(float32): tile %d", tile);
+    if (M == 0) return 0;
+    const int steps = (K + 31) / 32;
+    EpiArgs e{parts, bias, bias_dtype == DT_BF16, ldo, N, (steps + ksplit - 1) / ksplit, part_stride};
+    launch_f32_split<EPI_PART>(tile == TILE_128 ? 128 : 64, (const float*)x, (const float*)w, e, M, N, K, ksplit, stream);
+    LLMLAB_LAUNCH_CHECK("linear_partials(float32)");
+    return 0;
+  }
   LLMLAB_REQUIRE(((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0),
                  "linear_partials: operands must be 16-byte aligned");
   if (M == 0) return 0;

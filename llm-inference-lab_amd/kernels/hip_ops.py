@@ -189,7 +189,7 @@ class HipOps:
             self.device = torch.device("cuda", torch.cuda.current_device())
         self._core = self._load(build.core_library())
         self._declare_core()
-        if self._core.llmlab_abi_version() != 9:
+        if self._core.llmlab_abi_version() != 10:
             raise RuntimeError("kernel library and Python bindings disagree on the interface")
         self._attn: Dict[int, ctypes.CDLL] = {}
         self._mixer_libs: Dict[str, ctypes.CDLL] = {}
@@ -244,14 +244,15 @@ class HipOps:
                                         _c_int, _c_int, _c_int, _c_int, _c_ptr]
         c.llmlab_linear_tile.argtypes = [_c_int, _c_int, _c_int, _c_int]
         c.llmlab_linear_tile.restype = _c_int
-        c.llmlab_linear_partials.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
+        c.llmlab_linear_partials.argtypes = [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                              _c_int, _c_int, _c_size, _c_int, _c_ptr]
         c.llmlab_qkv_from_pieces.argtypes = [_c_ptr, _c_int, _c_size, _c_int, _c_ptr, _c_int, _c_int, _c_int,
                                              _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                                              _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr]
         c.llmlab_qkv_from_pieces.restype = _c_int
-        c.llmlab_linear_plan.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr]
-        c.llmlab_linear_plan.restype = None
+        for plan in (c.llmlab_linear_plan, c.llmlab_linear_plan_f32):
+            plan.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr]
+            plan.restype = None
         c.llmlab_skinny_linear.argtypes = [
             _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr,
             _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
@@ -687,16 +688,16 @@ class HipOps:
         [n, k]^T`` should be cut so that it spreads over the chip: a narrow output
         gives too few blocks otherwise, and a compute unit draws only so much from
         memory.  1: do not cut."""
-        if dtype != torch.bfloat16 or rows <= 0:
+        if rows <= 0 or (dtype != torch.bfloat16 and rows <= self.FEW_ROWS):
             return 1
-        if self.pieces_by_tiles(rows, n, k):
+        if dtype != torch.bfloat16 or self.pieces_by_tiles(rows, n, k):
             # many rows, tiled kernel: its own estimate (rounds of blocks over the chip times
             # the K tiles of a block, plus a write and a read of the result for every piece)
-            if k % 8:
+            if dtype == torch.bfloat16 and k % 8:
                 return 1
             if self.rules.forced_tiled_pieces:
                 return max(1, min(self.rules.forced_tiled_pieces, (k + 63) // 64, self.MAX_SPLITS))
-            return self._linear_plan(rows, n, k)[0]
+            return self._linear_plan(rows, n, k, dtype)[0]
         if rows > self.split_max_rows:
             return 1
         strips, steps = (n + 15) // 16, (k + 31) // 32
@@ -717,17 +718,20 @@ class HipOps:
         want = self.num_cus // max(strips, 1)
         return max(1, min(want, most))
 
-    def _linear_plan(self, rows: int, n: int, k: int):
+    def _linear_plan(self, rows: int, n: int, k: int, dtype=torch.bfloat16):
         """(pieces, tile) for a many-row product that adds into float32 rows."""
         out = (_c_int * 2)()
-        self._core.llmlab_linear_plan(rows, n, k, self.num_cus, self.MAX_SPLITS, self.rules.min_tiles_per_split, out)
+        plan = self._core.llmlab_linear_plan if dtype == torch.bfloat16 else self._core.llmlab_linear_plan_f32
+        plan(rows, n, k, self.num_cus, self.MAX_SPLITS, self.rules.min_tiles_per_split, out)
         return out[0], out[1]
 
     def linear_partials(self, x, w, parts: torch.Tensor, splits: int, bias=None) -> PendingSums:
         """``parts[s] = x[:, K_s] w[:, K_s]^T`` for the ``splits`` pieces ``K_s`` of the inner
         size (bias in piece 0): the product without the final sum."""
-        self._need(x, "linear input", torch.bfloat16)
+        self._need(x, "linear input")
         w = self._weight(w, "linear weight")
+        if x.dtype != w.dtype:
+            raise TypeError(f"linear_partials: input is {x.dtype} but the weight is {w.dtype}")
         m, k = x.shape
         n = w.shape[0]
         if (w.shape[1] != k or parts.dtype != torch.float32 or parts.dim() != 3 or parts.shape[0] < splits
@@ -737,16 +741,16 @@ class HipOps:
                              f"parts {tuple(parts.shape)} for {splits} pieces do not fit")
         if not 1 <= splits <= self.MAX_SPLITS:
             raise ValueError(f"linear_partials: {splits} pieces")
-        if not self.pieces_by_tiles(m, n, k):
+        if x.dtype == torch.bfloat16 and not self.pieces_by_tiles(m, n, k):
             self._skinny(x, False, None, None, 0.0, w, bias, EPI_PART, parts, m, n, k, parts.stride(1), n,
                          ksplit=splits, part_stride=parts.stride(0))
         else:
             if bias is not None:
                 self._need(bias, "bias")
             self._call(self._core.llmlab_linear_partials,
-                self._ptr(x), self._ptr(w), self._ptr(parts), self._ptr(bias),
+                self._ptr(x), self._ptr(w), _dt(x), self._ptr(parts), self._ptr(bias),
                 _dt(bias) if bias is not None else 0, m, n, k, parts.stride(1), splits, parts.stride(0),
-                self._linear_plan(m, n, k)[1], self._stream())
+                self._linear_plan(m, n, k, x.dtype)[1], self._stream())
         return PendingSums(parts, splits)
 
     def add_pending(self, x: torch.Tensor, pending: PendingSums) -> None:
@@ -877,7 +881,7 @@ class HipOps:
                 self._need(b_qkv, "bias")
             parts = self.workspace[:pieces * rows * n].view(pieces, rows, n)
             self._call(self._core.llmlab_linear_partials,
-                self._ptr(h), self._ptr(w_qkv), self._ptr(parts), None, 0, rows, n, k, n, pieces,
+                self._ptr(h), self._ptr(w_qkv), _dt(h), self._ptr(parts), None, 0, rows, n, k, n, pieces,
                 rows * n, tile, self._stream())
             self._call(self._core.llmlab_qkv_from_pieces,
                 self._ptr(parts), pieces, rows * n, n, self._ptr(b_qkv),

@@ -1,0 +1,64 @@
+"""The float32 products of many rows that split every number into three bfloat16 parts
+(``gemm_f32_split_kernel``): both tiles, whole and in pieces, against 64 bits at the edges of the
+tiles, with numbers of very different sizes, and with numbers that have no such parts."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llm_inference_lab_amd.kernels.hip_ops import HipOps
+    return HipOps(DEV)
+
+
+def rnd(shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed))
+
+
+def bound(x, w):
+    """What 32-bit sums of ``k`` products in any order may be off by: ``k`` roundings (and, of the split, the
+    three left-out terms, below two more) of half a unit of the sum of the absolute products."""
+    return (x.shape[1] + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+
+
+@pytest.mark.parametrize("tile", [64, 128, None])
+@pytest.mark.parametrize("m,n,k", [(65, 64, 32), (66, 65, 33), (127, 63, 31), (128, 128, 64), (129, 130, 100),
+                                   (192, 257, 1), (193, 36, 1153)])
+def test_against_64_bits(ops, tile, m, n, k):
+    # (sizes spread over 2^-30 .. 2^30: all three parts of a number matter)
+    x = rnd((m, k), 1) * torch.exp2(torch.randint(-30, 31, (m, k), generator=torch.Generator().manual_seed(2)).float())
+    w = rnd((n, k), 3)
+    want, limit = x.double() @ w.double().T, bound(x, w)
+    dx, dw = x.to(DEV), ops.prepare_weight(w.to(DEV))
+    with ops.debug.force(gemm_tile=tile):
+        out = torch.empty(m, n, device=DEV)
+        ops.linear_logits(dx, dw, out)
+        assert bool(((out.cpu().double() - want).abs() <= limit).all())
+        for pieces in (2, 3):
+            parts = torch.full((pieces, m, n), float("nan"), device=DEV)
+            ops.linear_partials(dx, dw, parts, pieces)
+            got = parts.cpu().double().sum(0)
+            assert bool(((got - want).abs() <= limit).all()), f"{pieces} pieces"
+
+
+@pytest.mark.parametrize("tile", [64, 128])
+def test_numbers_without_parts(ops, tile):
+    """Infinities, numbers that bfloat16 rounds to infinity and NaN: as plain 32-bit FMAs give them."""
+    m, n, k = 70, 66, 40
+    x, w = rnd((m, k), 5), rnd((n, k), 6)
+    x[3, 7], x[10, 0], x[20, 39], x[65, 1] = float("inf"), 3.4e38, float("nan"), -float("inf")
+    w[:, 0] = 1e-38 * w[:, 0]
+    want = x.double() @ w.double().T
+    out = torch.empty(m, n, device=DEV)
+    with ops.debug.force(gemm_tile=tile):
+        ops.linear_logits(x.to(DEV), w.to(DEV), out)
+    got = out.cpu().double()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    limit = torch.where(fine, bound(x, w), torch.zeros(()).double())
+    assert bool(((got - want).abs()[fine] <= limit[fine]).all())
