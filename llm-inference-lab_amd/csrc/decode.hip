@@ -1,5 +1,5 @@
 // Matrix products for few rows (decode steps and short portions; up to 1,024 rows of
-// a small matrix, in tiles of 16 to 64 rows), bfloat16, gfx950.  At this size a step is bound by launch count and by memory
+// a small matrix, in tiles of 16 to 64 rows), gfx950.  At this size a step is bound by launch count and by memory
 // latency, not by arithmetic, so one kernel does what the general path does in
 // three or four:
 //
@@ -60,19 +60,19 @@
 enum { SK_STORE = 0, SK_RESID = 1, SK_F32 = 2, SK_SWIGLU = 3, SK_QKV = 4, SK_PART = 5 };
 
 struct SkinnyArgs {
-  const void* x;        // NORM: float32 rows of the residual stream; else bfloat16 [M, K]
+  const void* x;        // NORM: float32 rows of the residual stream; else [M, K] in the compute type
   const int* x_rows;    // NORM only, optional: row of x for each m (final norm of wanted rows)
   const void* norm_w;   // NORM: [K]
-  const bf16_t* W;      // [N, K]
+  const void* W;        // [N, K]: bfloat16 packed in fragment order, float32 row by row
   const void* bias;     // [N] or null
-  void* out;            // STORE/SWIGLU: bf16 [M, ldo]; RESID/F32: float [M, ldo]; QKV: bf16 q [M, ldo]
+  void* out;            // STORE/SWIGLU, QKV (q): compute type [M, ldo]; RESID/F32: float [M, ldo]
   // QKV epilogue
   const float* inv_freq;   // [d/2] or null (no rotation)
   const int* positions;    // [M]
   const int* row_req;      // [M]
   const int* table;        // block table
-  bf16_t* kcache;          // may be null: q only is produced, k and v heads are skipped
-  bf16_t* vcache;
+  void* kcache;            // may be null: q only is produced, k and v heads are skipped
+  void* vcache;
   int M, N, K, ldo, n_out;
   int norm_w_bf16, bias_bf16;
   int nsb, kw;
@@ -109,11 +109,72 @@ __device__ __forceinline__ float sk_gelu_tanh(float z) {
 
 // act(gate) * up; the clamped pair: g = min(gate, limit), u = up held within -limit .. limit,
 // g * sigmoid(slope * g) * (u + shift)
+// (bfloat16 results by the hardware's exponential, float32 results by the library's functions)
+template <typename T>
 __device__ __forceinline__ float sk_pair(float g, float u, const SkinnyArgs& a) {
+  if constexpr (sizeof(T) == 4) {
+    if (a.act == 2) {
+      const float t = 0.7978845608028654f * (g + 0.044715f * g * g * g);
+      return 0.5f * g * (1.f + tanhf(t)) * u;
+    }
+    if (a.act != 3) return g / (1.f + expf(-g)) * u;
+    g = fminf(g, a.limit);
+    return g / (1.f + expf(-a.slope * g)) * (fminf(fmaxf(u, -a.limit), a.limit) + a.shift);
+  }
   if (a.act != 3) return (a.act == 2 ? sk_gelu_tanh(g) : sk_silu(g)) * u;
   g = fminf(g, a.limit);
   return g / (1.f + __expf(-a.slope * g)) * (fminf(fmaxf(u, -a.limit), a.limit) + a.shift);
 }
+
+// What a step of the inner size is: 16 rows of W by 64 bytes, 16 bytes a lane.  bfloat16: 32 numbers, one
+// matrix instruction.  float32: 16 numbers, four (lane (c, g) holds the numbers 4 g .. 4 g + 3 of row c; instruction
+// e contracts the e-th of all four groups, the same four numbers of both operands), 32-bit products and sums in
+// sixteen running sums that meet at the end: the order of a tree, so that a sum is as exact as the one of
+// the kernel whose lanes split the inner size (relative error against 64 bits 1.0e-7 to 1.8e-7 where that has 0.9e-7 to
+// 2.2e-7; one running sum: 2e-7 to 8.5e-7).  W lies row by row, so that a load of a wave is 16 pieces of 64 bytes; packed
+// like bfloat16 it would be 8 to 20 % faster (8 rows of 9728 x 896 13.8 us against 15.0), which every other reader
+// of the matrix would have to learn.  8 / 64 rows of 9728 x 896 15 / 31 us (17.4 / 59 by that kernel), of 896 x
+// 4864 in four pieces 8.5 / 24 (12.7 / 26), of 151936 x 896 106 / 287 (150 / 1,120), and the norm, the rotation and the
+// writing of the cache ride along: a decode step of eight requests of the 0.5B shape 2.20 -> 1.37 ms.
+template <typename T>
+struct SkStep;
+template <>
+struct SkStep<bf16_t> {
+  typedef bf16x8 frag;
+  static constexpr int LEN = 32, PER = 8, SUMS = 1;
+  static __device__ __forceinline__ void mul(frag x, frag w, floatx4* acc, int) {
+    acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, w, acc[0], 0, 0, 0);
+  }
+};
+template <>
+struct SkStep<float> {
+  typedef floatx4 frag;
+  static constexpr int LEN = 16, PER = 4, SUMS = 16;
+  static __device__ __forceinline__ void mul(frag x, frag w, floatx4* acc, int step) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      floatx4& sum = acc[(step & 3) * 4 + e];
+      sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], w[e], sum, 0, 0, 0);
+    }
+  }
+};
+// eight neighbouring numbers
+template <typename T>
+struct Sk8;
+template <>
+struct Sk8<bf16_t> {
+  bf16x8 v;
+  __device__ __forceinline__ void load(const bf16_t* p) { v = *(const bf16x8*)p; }
+  __device__ __forceinline__ void store(bf16_t* p) const { *(bf16x8*)p = v; }
+  __device__ __forceinline__ void set(int i, float f) { v[i] = (bf16_t)f; }
+};
+template <>
+struct Sk8<float> {
+  floatx4 lo, hi;
+  __device__ __forceinline__ void load(const float* p) { lo = *(const floatx4*)p; hi = *(const floatx4*)(p + 4); }
+  __device__ __forceinline__ void store(float* p) const { *(floatx4*)p = lo; *(floatx4*)(p + 4) = hi; }
+  __device__ __forceinline__ void set(int i, float f) { if (i < 4) lo[i] = f; else hi[i - 4] = f; }
+};
 
 // Loads of W (and of x where it is not staged) run R steps ahead of the MFMAs in a
 // ring of registers that is refilled slot by slot, so a wave always has R loads
@@ -130,7 +191,7 @@ __host__ __device__ constexpr int sk_ring(int mb, bool stage) {
 }
 
 constexpr int SK_STAGE_U_PIECES = 1;
-constexpr int SK_APAD = 8;   // padding of a staged row, in elements: 16-byte reads of 8 lanes cover all banks
+constexpr int SK_APAD = 16;  // padding of a staged row, in bytes: 16-byte reads of 8 lanes cover all banks
 
 // floats of LDS before the staged rows (host and device must agree)
 __host__ __device__ inline size_t sk_float_words(int nsb, int kw, int mb, int M, int epi) {
@@ -142,9 +203,11 @@ __host__ __device__ inline size_t sk_float_words(int nsb, int kw, int mb, int M,
   return (f + 3) & ~(size_t)3;
 }
 
-template <int MB, int EPI, bool NORM, bool STAGE>
+template <typename T, int MB, int EPI, bool NORM, bool STAGE>
 __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(SkinnyArgs a) {
   static_assert(STAGE || !NORM, "the fused norm needs the staged rows");
+  using S = SkStep<T>;
+  using Frag = typename S::frag;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   // Rows in tiles of 16 MB: a block sees its tile as if it were the whole product,
   // through pointers moved to the tile's first row.  The tiles of one set of columns
@@ -161,11 +224,11 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     if (NORM && a.x_rows) a.x_rows += m0;       // (the pieces owed are then found by these numbers too)
     else {
       a.x = NORM ? (const void*)((const float*)a.x + (size_t)m0 * a.K)
-                 : (const void*)((const bf16_t*)a.x + (size_t)m0 * a.K);
+                 : (const void*)((const T*)a.x + (size_t)m0 * a.K);
       a.pend += (size_t)m0 * a.pend_ld;
     }
     constexpr bool OUT32 = EPI == SK_RESID || EPI == SK_F32 || EPI == SK_PART;
-    a.out = OUT32 ? (void*)((float*)a.out + (size_t)m0 * a.ldo) : (void*)((bf16_t*)a.out + (size_t)m0 * a.ldo);
+    a.out = OUT32 ? (void*)((float*)a.out + (size_t)m0 * a.ldo) : (void*)((T*)a.out + (size_t)m0 * a.ldo);
     if constexpr (EPI == SK_QKV) {
       a.positions += m0;
       if (a.row_req) a.row_req += m0;
@@ -183,7 +246,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   const int bidx = (EPI == SK_PART) ? col_block - ksp * nblk : col_block;
   const int n0 = bidx * cols;
   const int K = a.K, M = a.M;
-  const int steps = (K + 31) >> 5;      // K steps of 32; W is packed and zero-padded to this
+  const int steps = (K + S::LEN - 1) / S::LEN;     // bfloat16: W is packed and zero-padded to this; float32: whole steps
 
   float* part = smem;                                   // [kw*nsb][MB][64][4]
   float* inv = part + (size_t)kw * nsb * MB * 256;      // [MB*16]
@@ -193,8 +256,8 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   int* s_page = s_pos + MB * 16;                        // [MB*16]
   float* s_freq = (float*)(s_page + MB * 16);           // [128]
   float* tile = s_freq + 128;                           // [M][cols]   (SWIGLU, QKV)
-  bf16_t* As = (bf16_t*)(smem + sk_float_words(nsb, kw, MB, M, EPI));   // [M][steps*32 + SK_APAD]
-  const int lda = steps * 32 + SK_APAD;
+  T* As = (T*)(smem + sk_float_words(nsb, kw, MB, M, EPI));   // [M][steps * S::LEN + padding]
+  const int lda = steps * S::LEN + SK_APAD / (int)sizeof(T);
 
   // QKV with qsplit > 1: block = (head, p); its two strips are columns p*16.. and
   // d/2 + p*16.. of the head, i.e. both halves of the rotary pairs
@@ -211,14 +274,16 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   // one again, and what comes of it is dropped by the epilogue)
   int wstrip = (EPI == SK_QKV) ? (qhead * a.d + head_col(strip * 16)) >> 4 : bidx * nsb + strip;
   wstrip = min(wstrip, ((a.N + 15) >> 4) - 1);
-  const bf16_t* wp = a.W + (size_t)wstrip * steps * 512 + lane * 8;
+  constexpr bool PACKED = sizeof(T) == 2;
+  const T* wp = PACKED ? (const T*)a.W + (size_t)wstrip * steps * 512 + lane * 8
+                       : (const T*)a.W + (size_t)min(wstrip * 16 + c, a.N - 1) * K + g * S::PER;
   // this block's K steps (all of them, or its group's share), split over its waves
   const int gsteps = (EPI == SK_PART) ? (steps + a.ksplit - 1) / a.ksplit : steps;
   const int g_begin = ksp * gsteps, g_end = min(steps, g_begin + gsteps);
   const int per = (max(g_end - g_begin, 0) + kw - 1) / kw;
   const int s_begin = g_begin + ks * per;
   const int s_end = min(g_end, s_begin + per);
-  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const Frag zero = {};
   const floatx4 fzero = {0.f, 0.f, 0.f, 0.f};
 
   // ---- what the epilogue needs from global memory, fetched now
@@ -257,15 +322,19 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     }
   }
 
-  floatx4 acc[MB];
+  floatx4 acc[MB][S::SUMS];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) acc[mb] = fzero;
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int i = 0; i < S::SUMS; ++i) acc[mb][i] = fzero;
 
   // Loads in the ring are unconditional (a step past the end reads the last tile
   // again and is multiplied by zeros): a load under a branch makes the compiler wait
   // for every load in flight at the join, and the stream stalls once per round.
-  auto wload = [&](int st) { return *(const bf16x8*)(wp + (size_t)max(0, min(st, steps - 1)) * 512); };
-  bf16x8 b[R];
+  auto wload = [&](int st) {
+    return *(const Frag*)(wp + (size_t)max(0, min(st, steps - 1)) * (PACKED ? 512 : S::LEN));
+  };
+  Frag b[R];
 
   if constexpr (STAGE) {
 #pragma unroll
@@ -273,7 +342,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     // ---- the first weight tiles are on their way; stage the rows of x
     // Fewer rows than waves: `wpr` waves share a row, each taking every wpr-th run of 64
     // chunks (one wave alone would walk a long row in many trips while the others wait)
-    const int chunks = K >> 3, chunks_pad = steps * 4;
+    const int chunks = K >> 3, chunks_pad = steps * (S::LEN / 8);
     int wpr = 1;
     while (2 * wpr * M <= nwaves) wpr *= 2;
     // A wave walks its part of a row U chunks at a time: the loads of all U (the row, the
@@ -286,7 +355,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       const int stride = 64 * wpr;
       for (int unit = wave; unit < M * wpr; unit += nwaves) {
         const int r = unit / wpr, sub = unit - r * wpr;
-        bf16_t* dst = As + (size_t)r * lda;
+        T* dst = As + (size_t)r * lda;
         if constexpr (NORM) {
           const float* src = (const float*)a.x + (size_t)(a.x_rows ? a.x_rows[r] : r) * K;
           float ssq = 0.f;
@@ -342,14 +411,14 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
                   wv[4 + j] = w1[u][j];
                 }
               }
-              bf16x8 av;
+              Sk8<T> av;
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
                 ssq += p[u][j] * p[u][j] + q[u][j] * q[u][j];
-                av[j] = (bf16_t)(p[u][j] * wv[j]);
-                av[4 + j] = (bf16_t)(q[u][j] * wv[4 + j]);
+                av.set(j, p[u][j] * wv[j]);
+                av.set(4 + j, q[u][j] * wv[4 + j]);
               }
-              *(bf16x8*)(dst + chs[u] * 8) = av;
+              av.store(dst + chs[u] * 8);
             }
           }
           ssq = wave_sum(ssq);
@@ -358,18 +427,18 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
             else s_ssq[unit] = ssq;       // (M * wpr <= 16 waves)
           }
         } else {
-          const bf16_t* src = (const bf16_t*)a.x + (size_t)r * K;
+          const T* src = (const T*)a.x + (size_t)r * K;
           for (int ch0 = sub * 64 + lane; ch0 < chunks; ch0 += U * stride) {
-            bf16x8 v[U];
+            Sk8<T> v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = *(const bf16x8*)(src + min(ch0 + u * stride, chunks - 1) * 8);
+            for (int u = 0; u < U; ++u) v[u].load(src + min(ch0 + u * stride, chunks - 1) * 8);
 #pragma unroll
             for (int u = 0; u < U; ++u)
-              if (ch0 + u * stride < chunks) *(bf16x8*)(dst + (ch0 + u * stride) * 8) = v[u];
+              if (ch0 + u * stride < chunks) v[u].store(dst + (ch0 + u * stride) * 8);
           }
         }
         if (sub == 0)
-          for (int ch = chunks + lane; ch < chunks_pad; ch += 64) *(bf16x8*)(dst + ch * 8) = zero;
+          for (int ch = chunks + lane; ch < chunks_pad; ch += 64) Sk8<T>{}.store(dst + ch * 8);
       }
     };
     // (with pieces owed, two chunks' loads are as many registers as four without)
@@ -394,9 +463,9 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     }
     // rows past M are not staged: their lanes read the last row, and what they
     // compute lands in rows of the result that nobody reads
-    const bf16_t* arow[MB];
+    const T* arow[MB];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) arow[mb] = As + (size_t)min(mb * 16 + c, M - 1) * lda + g * 8;
+    for (int mb = 0; mb < MB; ++mb) arow[mb] = As + (size_t)min(mb * 16 + c, M - 1) * lda + g * S::PER;
     int s0 = s_begin;
     for (; s0 + R < s_end; s0 += R) {       // rounds that refill the ring
 #pragma unroll
@@ -404,8 +473,8 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
         const int st = s0 + u;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
-          const bf16x8 av = *(const bf16x8*)(arow[mb] + st * 32);
-          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b[u], acc[mb], 0, 0, 0);
+          const Frag av = *(const Frag*)(arow[mb] + st * S::LEN);
+          S::mul(av, b[u], acc[mb], u);
         }
         b[u] = wload(min(st + R, s_end - 1));
         __builtin_amdgcn_sched_barrier(0);
@@ -414,19 +483,19 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
 #pragma unroll
     for (int u = 0; u < R; ++u) {           // the last round drains it
       const int st = s0 + u;
-      const bf16x8 bu = st < s_end ? b[u] : zero;
+      const Frag bu = st < s_end ? b[u] : zero;
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        const bf16x8 av = *(const bf16x8*)(arow[mb] + min(st, steps - 1) * 32);
-        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bu, acc[mb], 0, 0, 0);
+        const Frag av = *(const Frag*)(arow[mb] + min(st, steps - 1) * S::LEN);
+        S::mul(av, bu, acc[mb], u);
       }
     }
   } else {
-    // ---- rows of x (bfloat16) straight from global memory, in the same ring; a
+    // ---- rows of x (compute type) straight from global memory, in the same ring; a
     // piece past K or a row past M reads a valid piece instead: it meets zeros of
     // the padded W, or lands in a row of the result that nobody reads
-    const bf16_t* xb[MB];
-    const bf16_t* x_rows = (const bf16_t*)a.x;
+    const T* xb[MB];
+    const T* x_rows = (const T*)a.x;
     if constexpr (EPI == SK_PART) {
       int seg = 0;
 #pragma unroll
@@ -436,9 +505,9 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) xb[mb] = x_rows + (size_t)min(mb * 16 + c, M - 1) * K;
     auto xload = [&](int st, int mb) {
-      return *(const bf16x8*)(xb[mb] + min(max(0, min(st, steps - 1)) * 32 + g * 8, K - 8));
+      return *(const Frag*)(xb[mb] + min(max(0, min(st, steps - 1)) * S::LEN + g * S::PER, K - S::PER));
     };
-    bf16x8 ab[R][MB];
+    Frag ab[R][MB];
 #pragma unroll
     for (int u = 0; u < R; ++u) {     // in the order in which the loop below refills the ring
       const int st = min(s_begin + u, s_end - 1);
@@ -454,7 +523,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
         const int st = s0 + u;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
-          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab[u][mb], b[u], acc[mb], 0, 0, 0);
+          S::mul(ab[u][mb], b[u], acc[mb], u);
         const int nx = min(st + R, s_end - 1);
         b[u] = wload(nx);
 #pragma unroll
@@ -464,17 +533,21 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     }
 #pragma unroll
     for (int u = 0; u < R; ++u) {           // the last round drains it
-      const bf16x8 bu = s0 + u < s_end ? b[u] : zero;
+      const Frag bu = s0 + u < s_end ? b[u] : zero;
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ab[u][mb], bu, acc[mb], 0, 0, 0);
+      for (int mb = 0; mb < MB; ++mb) S::mul(ab[u][mb], bu, acc[mb], u);
     }
   }
 
   // ---- partial sums to LDS
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-    *(floatx4*)(part + (((size_t)wave * MB + mb) * 64 + lane) * 4) = acc[mb];
+  for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+    for (int half = S::SUMS / 2; half > 0; half >>= 1)
+#pragma unroll
+      for (int i = 0; i < half; ++i) acc[mb][i] += acc[mb][half + i];
+    *(floatx4*)(part + (((size_t)wave * MB + mb) * 64 + lane) * 4) = acc[mb][0];
+  }
   __syncthreads();
   // ---- reduce over the K slices in a fixed order; epilogue
   for (int idx = threadIdx.x; idx < M * cols; idx += blockDim.x) {
@@ -491,7 +564,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       tile[idx] = sum;
     } else if (nn < a.N) {
       const size_t at = (size_t)m * a.ldo + nn;
-      if (EPI == SK_STORE) ((bf16_t*)a.out)[at] = (bf16_t)(a.act ? fmaxf(sum, 0.f) * fmaxf(sum, 0.f) : sum);
+      if (EPI == SK_STORE) ((T*)a.out)[at] = from_float<T>(a.act ? fmaxf(sum, 0.f) * fmaxf(sum, 0.f) : sum);
       else if (EPI == SK_RESID) {
         float old = resid_old;
         if (idx != (int)threadIdx.x) {
@@ -514,7 +587,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       const int pr = j >> 4, cc = j & 15;
       const float gv = tile[m * cols + pr * 32 + cc], uv = tile[m * cols + pr * 32 + 16 + cc];
       const int o = ((n0 >> 5) + pr) * 16 + cc;
-      if (o < a.n_out) ((bf16_t*)a.out)[(size_t)m * a.ldo + o] = (bf16_t)sk_pair(gv, uv, a);
+      if (o < a.n_out) ((T*)a.out)[(size_t)m * a.ldo + o] = from_float<T>(sk_pair<T>(gv, uv, a));
     }
   }
   if constexpr (EPI == SK_QKV) {
@@ -530,29 +603,35 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       float lo = tile[m * cols + il], hi = tile[m * cols + il + half];
       const int pos = s_pos[m];
       if ((is_q || is_k) && a.inv_freq) {
-        // bfloat16 results: the hardware sine and cosine of r = frac(angle / 2 pi)
-        float r = (float)pos * s_freq[i] * 0.15915494309189535f;
-        r -= floorf(r);
-        const float s = __builtin_amdgcn_sinf(r), co = __builtin_amdgcn_cosf(r);
+        float s, co;
+        if constexpr (sizeof(T) == 4) {
+          sincosf((float)pos * s_freq[i], &s, &co);
+        } else {
+          // bfloat16 results: the hardware sine and cosine of r = frac(angle / 2 pi)
+          float r = (float)pos * s_freq[i] * 0.15915494309189535f;
+          r -= floorf(r);
+          s = __builtin_amdgcn_sinf(r);
+          co = __builtin_amdgcn_cosf(r);
+        }
         const float nlo = lo * co - hi * s, nhi = hi * co + lo * s;
         lo = nlo;
         hi = nhi;
       }
       if (is_q) {
-        bf16_t* dst = (bf16_t*)a.out + (size_t)m * a.ldo + (size_t)head * d;
-        dst[i] = (bf16_t)lo;
-        dst[i + dhalf] = (bf16_t)hi;
+        T* dst = (T*)a.out + (size_t)m * a.ldo + (size_t)head * d;
+        dst[i] = from_float<T>(lo);
+        dst[i + dhalf] = from_float<T>(hi);
       } else if (a.kcache) {
         const size_t page = (size_t)s_page[m];
         const int off = pos % a.page_size;
         if (is_k) {
-          bf16_t* dst = a.kcache + (page * a.nkv + (head - a.nq)) * (size_t)a.page_size * d;
-          dst[kcache_index(off, i, d)] = (bf16_t)lo;
-          dst[kcache_index(off, i + dhalf, d)] = (bf16_t)hi;
+          T* dst = (T*)a.kcache + (page * a.nkv + (head - a.nq)) * (size_t)a.page_size * d;
+          dst[kcache_index(off, i, d)] = from_float<T>(lo);
+          dst[kcache_index(off, i + dhalf, d)] = from_float<T>(hi);
         } else {
-          bf16_t* dst = a.vcache + (page * a.nkv + (head - a.nq - a.nkv)) * (size_t)a.page_size * d;
-          dst[vcache_index(off, i, d)] = (bf16_t)lo;
-          dst[vcache_index(off, i + dhalf, d)] = (bf16_t)hi;
+          T* dst = (T*)a.vcache + (page * a.nkv + (head - a.nq - a.nkv)) * (size_t)a.page_size * d;
+          dst[vcache_index(off, i, d)] = from_float<T>(lo);
+          dst[vcache_index(off, i + dhalf, d)] = from_float<T>(hi);
         }
       }
     }
@@ -560,9 +639,10 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
 }
 
 // ---------------------------------------------------------------- dispatch
-static size_t skinny_lds_bytes(int nsb, int kw, int mb, int M, int K, int epi, bool stage) {
+// (`width`: bytes of a number of W and of the staged rows, 2 or 4)
+static size_t skinny_lds_bytes(int nsb, int kw, int mb, int M, int K, int epi, bool stage, int width) {
   size_t bytes = sk_float_words(nsb, kw, mb, M, epi) * sizeof(float);
-  if (stage) bytes += (size_t)M * ((K + 31) / 32 * 32 + SK_APAD) * sizeof(bf16_t);
+  if (stage) bytes += (size_t)M * ((size_t)(K + 31) / 32 * 32 * width + SK_APAD);
   return bytes;
 }
 
@@ -571,9 +651,9 @@ static const size_t SK_LDS_LIMIT = 152 * 1024;
 // Most rows of a call (tiles of at most 64 rows, a block each per set of columns).
 constexpr int SK_MAX_ROWS = 1024;
 
-template <int MB, int EPI, bool NORM, bool STAGE>
+template <typename T, int MB, int EPI, bool NORM, bool STAGE>
 static int skinny_launch(const SkinnyArgs& a, int blocks, size_t lds, hipStream_t stream) {
-  auto kernel = skinny_block_kernel<MB, EPI, NORM, STAGE>;
+  auto kernel = skinny_block_kernel<T, MB, EPI, NORM, STAGE>;
   if (lds > 48 * 1024) {
     static size_t raised = 0;     // per instantiation
     if (lds > raised) {
@@ -591,20 +671,21 @@ static int skinny_launch(const SkinnyArgs& a, int blocks, size_t lds, hipStream_
 }
 
 template <int EPI, bool NORM, bool STAGE>
-static int skinny_launch_mb(const SkinnyArgs& a, int mb, int blocks, size_t lds, hipStream_t stream) {
-  if (mb == 1) return skinny_launch<1, EPI, NORM, STAGE>(a, blocks, lds, stream);
-  if (mb == 2) return skinny_launch<2, EPI, NORM, STAGE>(a, blocks, lds, stream);
-  return skinny_launch<4, EPI, NORM, STAGE>(a, blocks, lds, stream);
+static int skinny_launch_mb(const SkinnyArgs& a, int width, int mb, int blocks, size_t lds, hipStream_t stream) {
+  if (width == 4) return skinny_launch<float, 1, EPI, NORM, STAGE>(a, blocks, lds, stream);     // (tiles of 16 rows only)
+  if (mb == 1) return skinny_launch<bf16_t, 1, EPI, NORM, STAGE>(a, blocks, lds, stream);
+  if (mb == 2) return skinny_launch<bf16_t, 2, EPI, NORM, STAGE>(a, blocks, lds, stream);
+  return skinny_launch<bf16_t, 4, EPI, NORM, STAGE>(a, blocks, lds, stream);
 }
 
 template <int EPI, bool NORM>
-static int skinny_launch_stage(const SkinnyArgs& a, bool stage, int mb, int blocks, size_t lds,
+static int skinny_launch_stage(const SkinnyArgs& a, int width, bool stage, int mb, int blocks, size_t lds,
                                hipStream_t stream) {
   if constexpr (NORM) {
-    return skinny_launch_mb<EPI, true, true>(a, mb, blocks, lds, stream);   // the norm is staged always
+    return skinny_launch_mb<EPI, true, true>(a, width, mb, blocks, lds, stream);   // the norm is staged always
   } else {
-    if (stage) return skinny_launch_mb<EPI, false, true>(a, mb, blocks, lds, stream);
-    return skinny_launch_mb<EPI, false, false>(a, mb, blocks, lds, stream);
+    if (stage) return skinny_launch_mb<EPI, false, true>(a, width, mb, blocks, lds, stream);
+    return skinny_launch_mb<EPI, false, false>(a, width, mb, blocks, lds, stream);
   }
 }
 
@@ -635,8 +716,8 @@ static inline int sk_tiles(int M, int mb) { return (M + 16 * mb - 1) / (16 * mb)
 // bandwidth would suggest, so spreading the matrix over all units matters most),
 // or the memory round trips of a wave if those take longer.
 static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, int tiles, int N, int K, int d,
-                                      int num_cus, int ksplit, double* cost_out) {
-  const int steps = ((K + 31) / 32 + ksplit - 1) / ksplit;     // per K group of blocks
+                                      int num_cus, int ksplit, int width, double* cost_out) {
+  const int steps = ((K + 31) / 32 + ksplit - 1) / ksplit * (width / 2);     // per K group of blocks
   const int strips = (N + 15) / 16;
   const int max_waves = mb >= 4 ? 8 : 16;
   SkinnyShape best{0, 0, false, 1, mb};
@@ -654,7 +735,7 @@ static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, in
     for (int kw = 1; kw * nsb <= max_waves && kw <= steps; ++kw) {
       for (int st = norm ? 1 : 0; st < (epilogue == SK_PART ? 1 : 2); ++st) {     // pieces of K: no staging
         const bool stage = st == 1;
-        const size_t lds = skinny_lds_bytes(nsb, kw, mb, M, K, epilogue, stage);
+        const size_t lds = skinny_lds_bytes(nsb, kw, mb, M, K, epilogue, stage, width);
         if (lds > SK_LDS_LIMIT) continue;
         const int blocks = (strips + nsb - 1) / nsb * ksplit * tiles;     // (for QKV: heads, or heads * d/32)
         const int per_cu = (blocks + num_cus - 1) / num_cus;       // blocks the busiest unit runs
@@ -670,7 +751,7 @@ static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, in
         // (fitted twice: a large matrix is bound by what the waves of a unit keep in
         // flight, up to about 50 GB/s; a small one by latencies, which the lower figures
         // stand for)
-        const bool large = (double)N * K * 2.0 >= 64e6;
+        const bool large = (double)N * K * width >= 64e6;
         double rate = (large ? 3.2e3 : 3.5e3) * resident * nsb * kw;
         // (more than one tile of rows of a wide output: all but the first tile of a set of
         // columns find W in the L2 of their die, and sixteen waves a block draw what eight
@@ -678,8 +759,8 @@ static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, in
         // with 4 x 2; a narrow output gains nothing from more slices)
         const double cap = (large || (tiles > 1 && strips >= num_cus)) ? 50.0e3 : 25.0e3;
         if (rate > cap) rate = cap;
-        const double t_stream = per_cu * (16.0 * nsb * K * 2.0) / rate;
-        const double x_bytes = (double)(stage ? 1 : 2 * nsb) * M * K * (norm ? 4.0 : 2.0);
+        const double t_stream = per_cu * (16.0 * nsb * K * width) / rate;
+        const double x_bytes = (double)(stage ? 1 : 2 * nsb) * M * K * (norm ? 4.0 : width);
         const double t_x = per_cu * x_bytes / 50.0e3;
         const int per = (steps + kw - 1) / kw;
         const int u = sk_ring(mb, stage);
@@ -704,12 +785,12 @@ static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, in
 // blocks, each of which stages (and norms) fewer rows, and W is read once per tile
 // (from the cache after the first).
 static SkinnyShape skinny_choose(int epilogue, bool norm, int M, int N, int K, int d, int num_cus,
-                                 int ksplit = 1) {
+                                 int ksplit = 1, int width = 2) {
   SkinnyShape best{0, 0, false, 1, 1};
   double best_cost = 1e30;
   // (q/k/v of more than 64 rows: tiles of 16 rows, measured; 576 rows of 1152 x 896 take
   // 13.4 us so, 16.4 in tiles of 32 and 26 in tiles of 64)
-  const int mb_max = M <= 16 || (epilogue == SK_QKV && M > 64) ? 1 : (M <= 32 ? 2 : 4);
+  const int mb_max = width == 4 || M <= 16 || (epilogue == SK_QKV && M > 64) ? 1 : (M <= 32 ? 2 : 4);
   for (int mb = mb_max; mb >= 1; mb >>= 1) {
     if (g_force_mb > 0 && (g_force_epi < 0 || g_force_epi == epilogue) && mb != g_force_mb &&
         !(g_force_mb > mb_max && mb == mb_max))
@@ -717,7 +798,7 @@ static SkinnyShape skinny_choose(int epilogue, bool norm, int M, int N, int K, i
     const int tiles = sk_tiles(M, mb);
     double cost;
     const SkinnyShape s = skinny_choose_tile(epilogue, norm, mb, M < 16 * mb ? M : 16 * mb, tiles, N, K, d,
-                                             num_cus, ksplit, &cost);
+                                             num_cus, ksplit, width, &cost);
     if (s.nsb > 0 && cost < best_cost) {
       best_cost = cost;
       best = s;
@@ -744,7 +825,7 @@ extern "C" void llmlab_skinny_shape(int epilogue, int norm, int M, int N, int K,
 //   segs > 1 (SK_PART): the strips of 16 rows of W below seg_ends[0] multiply x, the ones from there to
 //     below seg_ends[1] x + seg_stride, and so on (seg_ends: segs - 1 numbers in host memory)
 extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, const void* norm_w,
-                                    int norm_w_dtype, float eps, const void* w, const void* bias,
+                                    int norm_w_dtype, float eps, const void* w, int dtype, const void* bias,
                                     int bias_dtype, int epilogue, void* out, int M, int N, int K,
                                     int ldo, int n_out, const float* inv_freq, const int* positions,
                                     const int* row_req, const int* table, int table_stride,
@@ -756,7 +837,9 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   LLMLAB_REQUIRE(segs <= 1 || (segs <= 8 && seg_ends && epilogue == SK_PART && seg_stride % 8 == 0),
                  "skinny_linear: up to 8 segments with inputs of their own, in pieces, got %d", segs);
   LLMLAB_REQUIRE(M >= 0 && M <= SK_MAX_ROWS, "skinny_linear: takes at most %d rows, got %d", SK_MAX_ROWS, M);
-  LLMLAB_REQUIRE(N > 0 && K > 0 && K % 8 == 0, "skinny_linear: bad sizes N=%d K=%d (K must be a multiple of 8)", N, K);
+  LLMLAB_REQUIRE(N > 0 && K > 0 && K % (dtype == DT_F32 ? 16 : 8) == 0,
+                 "skinny_linear: bad sizes N=%d K=%d (K must be a multiple of 8, in float32 of 16)", N, K);
+  const int width = dtype == DT_F32 ? 4 : 2;
   // (6 at this interface: STORE through the squared relu; 7: the paired product with a gelu gate;
   // 8: the clamped pair)
   const int act = epilogue == 6 ? 1 : epilogue == 7 ? 2 : epilogue == 8 ? 3 : 0;
@@ -790,7 +873,7 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
     LLMLAB_REQUIRE(n_out == N, "skinny_linear: n_out %d != N %d", n_out, N);
   }
   LLMLAB_REQUIRE(ldo >= (epilogue == SK_QKV ? nq * d : n_out), "skinny_linear: output stride too small");
-  SkinnyShape shape = skinny_choose(epilogue, norm != 0, M, N, K, d, num_cus, ksplit);
+  SkinnyShape shape = skinny_choose(epilogue, norm != 0, M, N, K, d, num_cus, ksplit, width);
   const int mb = shape.mb, tiles = sk_tiles(M, mb), tile_rows = M < 16 * mb ? M : 16 * mb;
   const bool forced = g_force_epi < 0 || g_force_epi == epilogue;
   if (forced && g_force_nsb > 0 && epilogue != SK_QKV) shape.nsb = g_force_nsb;
@@ -802,14 +885,14 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   if (forced && g_force_stage >= 0) shape.stage = norm || (g_force_stage != 0 && epilogue != SK_PART);
   LLMLAB_REQUIRE(shape.nsb > 0 && shape.kw > 0,
                  "skinny_linear: no block shape fits N=%d K=%d M=%d (16 rows of x to stage: %zu bytes of LDS)",
-                 N, K, M, (size_t)(M < 16 ? M : 16) * ((K + 31) / 32 * 32 + SK_APAD) * sizeof(bf16_t));
-  const size_t lds = skinny_lds_bytes(shape.nsb, shape.kw, mb, tile_rows, K, epilogue, shape.stage);
+                 N, K, M, (size_t)(M < 16 ? M : 16) * ((size_t)(K + 31) / 32 * 32 * width + SK_APAD));
+  const size_t lds = skinny_lds_bytes(shape.nsb, shape.kw, mb, tile_rows, K, epilogue, shape.stage, width);
   LLMLAB_REQUIRE(lds <= SK_LDS_LIMIT && shape.nsb * shape.kw <= (mb >= 4 ? 8 : 16),
                  "skinny_linear: block shape %dx%d does not fit", shape.nsb, shape.kw);
   // (only a forced shape can fail these: a gate strip and its up strip share a block, and
   // every K slice has a step)
   LLMLAB_REQUIRE(!(epilogue == SK_SWIGLU && shape.nsb % 2 != 0) &&
-                     shape.kw <= ((K + 31) / 32 + ksplit - 1) / ksplit,
+                     shape.kw <= ((K + 31) / 32 + ksplit - 1) / ksplit * (width / 2),
                  "skinny_linear: block shape %dx%d does not fit this product", shape.nsb, shape.kw);
   const int blocks = (N + 16 * shape.nsb - 1) / (16 * shape.nsb) * ksplit;
   SkinnyArgs a;
@@ -821,9 +904,9 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   a.qsplit = shape.qsplit;
   a.act = act;
   a.limit = limit; a.slope = slope; a.shift = shift;
-  a.x = x; a.x_rows = x_rows; a.norm_w = norm_w; a.W = (const bf16_t*)w; a.bias = bias; a.out = out;
+  a.x = x; a.x_rows = x_rows; a.norm_w = norm_w; a.W = w; a.bias = bias; a.out = out;
   a.inv_freq = inv_freq; a.positions = positions; a.row_req = row_req; a.table = table;
-  a.kcache = (bf16_t*)kcache; a.vcache = (bf16_t*)vcache;
+  a.kcache = kcache; a.vcache = vcache;
   a.M = M; a.N = N; a.K = K; a.ldo = ldo; a.n_out = n_out;
   a.norm_w_bf16 = norm_w_dtype == DT_BF16; a.bias_bf16 = bias_dtype == DT_BF16;
   a.nsb = shape.nsb; a.kw = shape.kw; a.nq = nq; a.nkv = nkv; a.d = d; a.table_stride = table_stride;
@@ -831,19 +914,19 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   int rc = 0;
   if (norm) {
     switch (epilogue) {
-      case SK_F32: rc = skinny_launch_stage<SK_F32, true>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_SWIGLU: rc = skinny_launch_stage<SK_SWIGLU, true>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_QKV: rc = skinny_launch_stage<SK_QKV, true>(a, shape.stage, mb, blocks, lds, stream); break;
+      case SK_F32: rc = skinny_launch_stage<SK_F32, true>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_SWIGLU: rc = skinny_launch_stage<SK_SWIGLU, true>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_QKV: rc = skinny_launch_stage<SK_QKV, true>(a, width, shape.stage, mb, blocks, lds, stream); break;
       default: LLMLAB_REQUIRE(false, "skinny_linear: epilogue %d has no fused norm", epilogue);
     }
   } else {
     switch (epilogue) {
-      case SK_STORE: rc = skinny_launch_stage<SK_STORE, false>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_RESID: rc = skinny_launch_stage<SK_RESID, false>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_F32: rc = skinny_launch_stage<SK_F32, false>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_SWIGLU: rc = skinny_launch_stage<SK_SWIGLU, false>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_QKV: rc = skinny_launch_stage<SK_QKV, false>(a, shape.stage, mb, blocks, lds, stream); break;
-      case SK_PART: rc = skinny_launch_stage<SK_PART, false>(a, false, mb, blocks, lds, stream); break;
+      case SK_STORE: rc = skinny_launch_stage<SK_STORE, false>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_RESID: rc = skinny_launch_stage<SK_RESID, false>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_F32: rc = skinny_launch_stage<SK_F32, false>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_SWIGLU: rc = skinny_launch_stage<SK_SWIGLU, false>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_QKV: rc = skinny_launch_stage<SK_QKV, false>(a, width, shape.stage, mb, blocks, lds, stream); break;
+      case SK_PART: rc = skinny_launch_stage<SK_PART, false>(a, width, false, mb, blocks, lds, stream); break;
       default: LLMLAB_REQUIRE(false, "skinny_linear: epilogue %d needs the norm", epilogue);
     }
   }

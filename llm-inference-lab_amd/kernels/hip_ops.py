@@ -40,6 +40,9 @@ def _dt(t: torch.Tensor) -> int:
     raise TypeError(f"kernels take float32 or bfloat16 tensors, got {t.dtype}")
 
 
+_DTYPE_CODES = {torch.float32: DT_F32, torch.bfloat16: DT_BF16}
+
+
 class KernelError(RuntimeError):
     pass
 
@@ -254,7 +257,7 @@ class HipOps:
             plan.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr]
             plan.restype = None
         c.llmlab_skinny_linear.argtypes = [
-            _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr,
+            _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_ptr,
             _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
             _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
             _c_ptr, _c_int, _c_int, _c_size, _c_int, _c_size, _c_int, _c_ptr, _c_size, _c_float, _c_float, _c_float, _c_ptr]
@@ -528,7 +531,8 @@ class HipOps:
         ldo = out.stride(0) if m > 1 else max(out.stride(0), n_out)
         # few rows: the block kernel that splits K inside a block; from 17 rows on only
         # for narrow outputs (the tiled kernel has too few tiles there), measured
-        if x.dtype == torch.bfloat16 and (m <= 16 or (n < 8192 and self.few_rows_take(m, n, k))):
+        if ((self.few_rows_take_float32(m, k) and (x.data_ptr() | w.data_ptr()) % 16 == 0) if x.dtype == torch.float32
+                else m <= 16 or (n < 8192 and self.few_rows_take(m, n, k))):
             self._skinny(x, False, None, None, 0.0, w, bias, epilogue, out, m, n, k, ldo, n_out,
                          pending=pending, constants=constants)
             return
@@ -587,19 +591,32 @@ class HipOps:
         tiles = (rows + self.FUSE_TILE_ROWS - 1) // self.FUSE_TILE_ROWS
         return (rows <= min(self.rules.few_rows_max, self.FUSED_MAX_ROWS)
                 and 2.0 * outer * inner * tiles < self.rules.few_rows_read_bytes)
+
+    def few_rows_take_float32(self, rows: int, inner: int) -> bool:
+        """The same for a float32 product (whole steps of 16 of the inner size).  One or two rows are faster
+        by the kernel whose lanes split the inner size (``gemm_f32_rows_kernel``; 896 x 896 at 1 / 4 / 8 rows: 3.4 /
+        4.9 / 6.9 us so, 4.9 / 5.3 / 5.4 in pieces here; 896 x 4864: 5.9 / 9.0 / 12.5 and 7.2 / 7.7 / 8.3)."""
+        return inner % 16 == 0 and self.SPLIT_LANES_ROWS_FLOAT32 < rows <= self.FEW_ROWS
+
+    SPLIT_LANES_ROWS_FLOAT32 = 2
     STAGE_BYTES = 118 * 1024      # most LDS the staged rows of a fused kernel may take
 
     def can_fuse(self, rows: int, dtype, inner: int, outer: Optional[int] = None) -> bool:
-        """Whether the fused few-row kernels take this step: bfloat16, few rows, a tile
-        of rows (``inner`` wide) fits the staging buffer in LDS, and beyond one tile the
+        """Whether the fused few-row kernels take this step: few rows, a tile
+        of rows (``inner`` wide, in float32 whole steps of 16) fits the staging buffer in LDS, and beyond one tile the
         matrix (``outer`` rows) is a small one."""
-        if dtype != torch.bfloat16 or not 0 < rows <= min(max(self.FEW_ROWS, self.rules.few_rows_max), self.FUSED_MAX_ROWS):
+        if not 0 < rows <= min(max(self.FEW_ROWS, self.rules.few_rows_max), self.FUSED_MAX_ROWS):
             return False
+        width = 2
+        if dtype == torch.float32:
+            if rows > self.FEW_ROWS or inner % 16:
+                return False
+            width = 4
         tiles = (rows + self.FUSE_TILE_ROWS - 1) // self.FUSE_TILE_ROWS
         limit = self.rules.fuse_read_bytes if rows <= self.FEW_ROWS else self.rules.few_rows_read_bytes
-        if tiles > 1 and (outer is None or 2.0 * outer * inner * tiles >= limit):
+        if tiles > 1 and (outer is None or float(width) * outer * inner * tiles >= limit):
             return False
-        return min(rows, self.FUSE_TILE_ROWS) * ((inner + 31) // 32 * 32 + 8) * 2 <= self.STAGE_BYTES
+        return min(rows, self.FUSE_TILE_ROWS) * ((inner + 31) // 32 * 32 * width + 16) <= self.STAGE_BYTES
 
     def _skinny(self, x, norm, x_rows, norm_w, eps, w, bias, epilogue, out, m, n, k, ldo, n_out,
                 qkv=None, pending: Optional[PendingSums] = None, ksplit: int = 1,
@@ -624,7 +641,7 @@ class HipOps:
                      ptr(qkv["v_cache"]), qkv["nq"], qkv["nkv"], qkv["d"])
         self._call(self._core.llmlab_skinny_linear,
             x.data_ptr(), 1 if norm else 0, self._ptr(x_rows), self._ptr(norm_w),
-            _dt(norm_w) if norm_w is not None else 0, float(eps), w.data_ptr(), self._ptr(bias),
+            _dt(norm_w) if norm_w is not None else 0, float(eps), w.data_ptr(), _DTYPE_CODES[w.dtype], self._ptr(bias),
             _dt(bias) if bias is not None else 0, epilogue, out.data_ptr(), m, n, k, ldo, n_out,
             *heads, self.num_cus, pend[0], pend[1], pend[2], pend[3], int(ksplit),
             int(part_stride), *(segments or (1, None, 0)), *constants, self._stream())
@@ -683,14 +700,18 @@ class HipOps:
         """Whether a product left in pieces is cut by the tiled kernel (else by the few-row one)."""
         return rows > self.FEW_ROWS or (rows > self.FUSE_TILE_ROWS and 2.0 * n * k >= self.rules.tiled_pieces_bytes)
 
+    def _pieces_by_tiles(self, rows: int, n: int, k: int, dtype) -> bool:
+        """(float32: what the few-row kernel does not take is cut by the tiled one)"""
+        return not self.few_rows_take_float32(rows, k) if dtype == torch.float32 else self.pieces_by_tiles(rows, n, k)
+
     def split_count(self, rows: int, dtype, n: int, k: int) -> int:
         """Into how many pieces along the inner size a few-row product ``[rows, k] x
         [n, k]^T`` should be cut so that it spreads over the chip: a narrow output
         gives too few blocks otherwise, and a compute unit draws only so much from
         memory.  1: do not cut."""
-        if rows <= 0 or (dtype != torch.bfloat16 and rows <= self.FEW_ROWS):
+        if rows <= 0 or (dtype == torch.float32 and rows <= self.FEW_ROWS and (k % 16 or rows <= self.SPLIT_LANES_ROWS_FLOAT32)):
             return 1
-        if dtype != torch.bfloat16 or self.pieces_by_tiles(rows, n, k):
+        if self._pieces_by_tiles(rows, n, k, dtype):
             # many rows, tiled kernel: its own estimate (rounds of blocks over the chip times
             # the K tiles of a block, plus a write and a read of the result for every piece)
             if dtype == torch.bfloat16 and k % 8:
@@ -698,7 +719,7 @@ class HipOps:
             if self.rules.forced_tiled_pieces:
                 return max(1, min(self.rules.forced_tiled_pieces, (k + 63) // 64, self.MAX_SPLITS))
             return self._linear_plan(rows, n, k, dtype)[0]
-        if rows > self.split_max_rows:
+        if rows > self.split_max_rows and dtype != torch.float32:
             return 1
         strips, steps = (n + 15) // 16, (k + 31) // 32
         most = min(steps // self.rules.min_steps_per_split, self.MAX_SPLITS)
@@ -716,6 +737,10 @@ class HipOps:
                     return p
             return 1
         want = self.num_cus // max(strips, 1)
+        if dtype == torch.float32 and rows > self.split_max_rows:
+            # (the pieces of so many rows are folded by the norm, more of them cost the next product nothing: 48 / 64
+            # rows of 1536 x 8960 46 / 55 us in eight, 58 / 58 in two, 71 / 71 whole)
+            want = max(want, k // 1120)
         return max(1, min(want, most))
 
     def _linear_plan(self, rows: int, n: int, k: int, dtype=torch.bfloat16):
@@ -741,7 +766,7 @@ class HipOps:
                              f"parts {tuple(parts.shape)} for {splits} pieces do not fit")
         if not 1 <= splits <= self.MAX_SPLITS:
             raise ValueError(f"linear_partials: {splits} pieces")
-        if x.dtype == torch.bfloat16 and not self.pieces_by_tiles(m, n, k):
+        if not self._pieces_by_tiles(m, n, k, x.dtype):
             self._skinny(x, False, None, None, 0.0, w, bias, EPI_PART, parts, m, n, k, parts.stride(1), n,
                          ksplit=splits, part_stride=parts.stride(0))
         else:
@@ -767,15 +792,14 @@ class HipOps:
         self._need(x, "residual stream", torch.float32)
         self._need(norm_w, "norm weight")
         w = self._weight(w, "weight")
-        if w.dtype != torch.bfloat16:
-            raise TypeError("the fused few-row kernels are bfloat16 kernels")
         k = x.shape[1]
         if norm_w.numel() != k or w.shape[1] != k:
             raise ValueError(f"fused norm + product: x {tuple(x.shape)}, norm weight "
                              f"{tuple(norm_w.shape)}, w {tuple(w.shape)} do not fit")
-        if k % 8 != 0:
+        whole = 16 if w.dtype == torch.float32 else 8
+        if k % whole != 0:
             raise UnsupportedSizeError(
-                f"bfloat16 matrix products need an inner size that is a multiple of 8, got {k}")
+                f"the fused kernels need an inner size that is a multiple of {whole} in this data type, got {k}")
         if not 0 < rows <= self.FUSED_MAX_ROWS:
             raise ValueError(f"the fused kernels take 1..{self.FUSED_MAX_ROWS} rows, got {rows}")
         return w, k
@@ -785,7 +809,8 @@ class HipOps:
         n = (num_heads + 2 * num_kv_heads) * head_dim
         if w_qkv.shape[0] != n or tuple(q_out.shape) != (rows, num_heads * head_dim):
             raise ValueError(f"{what}: weight or output shape does not fit the heads")
-        self._need(q_out, "q output", torch.bfloat16)
+        dtype = w_qkv.dtype
+        self._need(q_out, "q output", dtype)
         self._need(positions, "positions", torch.int32)
         if positions.numel() < rows:
             raise ValueError(f"{what}: one position per row")
@@ -800,7 +825,7 @@ class HipOps:
             if (tuple(k_cache.shape) != (pages, num_kv_heads, page_size, head_dim)
                     or tuple(v_cache.shape) != (pages, num_kv_heads, head_dim, page_size)
                     or not k_cache.is_contiguous() or not v_cache.is_contiguous()
-                    or k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16
+                    or k_cache.dtype != dtype or v_cache.dtype != dtype
                     or row_req.numel() < rows):
                 raise ValueError(f"{what}: cache tensors do not have the paged layout")
         return n
@@ -910,7 +935,7 @@ class HipOps:
                           activation: str = "silu") -> None:
         rows, inter = out.shape
         w_gate_up, k = self._fused_common(x, norm_w, w_gate_up, rows)
-        self._need(out, "SwiGLU output", torch.bfloat16)
+        self._need(out, "SwiGLU output", w_gate_up.dtype)
         if x.shape[0] != rows or w_gate_up.shape[0] != 2 * ((inter + 15) // 16 * 16):
             raise ValueError("fused_norm_swiglu: shapes do not fit")
         self._skinny(x, True, None, norm_w, eps, w_gate_up, None, GATE_EPILOGUES[activation], out, rows,

@@ -161,7 +161,7 @@ class GQAAttention(Mixer):
         if rms is not None:
             # few rows: norm, the three projections, bias, rotation and the cache
             # write are one kernel
-            q = ctx.scratch("attention.q", (rows, self.q_size), self.dtype)
+            q = ctx.scratch("attention.qkv", (rows, self.q_size), self.dtype)
             # pieces still owed to the stream are added as its rows are read, and folded
             # in by the output projection below
             pending = getattr(ctx, "pending", None)
@@ -176,7 +176,7 @@ class GQAAttention(Mixer):
             # more rows: the norm on its own, then one kernel for the rest
             if isinstance(h, NormedInput):
                 h = h.tensor()
-            q = ctx.scratch("attention.q", (rows, self.q_size), self.dtype)
+            q = ctx.scratch("attention.qkv", (rows, self.q_size), self.dtype)
             ops.qkv_rope_cache(h, self.w_qkv, self.b_qkv, self.num_heads, self.num_kv_heads,
                                self.head_dim, table, ctx.positions, ctx.row_req, group.block_table,
                                group.page_size, k_cache, v_cache, q)
