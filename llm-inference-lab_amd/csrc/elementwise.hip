@@ -489,37 +489,161 @@ extern "C" int llmlab_add_pending(float* x, const float* pend, int splits, size_
 
 // ------------------------------------------------------------- layer norm
 // y = (x - mean(x)) * rsqrt(var(x) + eps) * w with var the mean of the squared
-// deviations (taken about the mean, in a pass of its own), no bias; all in float32.
+// deviations (taken about the mean, in a pass of its own over registers), no bias; all in float32.
 // ADD false: out[i, :] = T(y) for x row rows[i] (or i).  ADD true: the float32 stream
 // resid[i, :] += y, and, if copy is given, copy[i, :] = T(resid[i, :]) after the sum: what
-// the next reader of the stream multiplies with.
-template <typename T, bool ADD>
-__global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict__ x, const void* __restrict__ w,
-                                                        int w_bf16, float eps, T* __restrict__ out,
-                                                        float* __restrict__ resid, T* __restrict__ copy,
-                                                        const int* __restrict__ rows, int hidden) {
-  __shared__ float red[17];
-  const int i = blockIdx.x;
+// the next reader of the stream multiplies with.  x may be a result that a product left in
+// pieces: row i is the sum of x[s][i, :], s < splits, in their order.
+//
+// A thread keeps its first KEEP groups of W numbers (of the row, the weight and the stream) in
+// registers, all asked for at once, so that a row costs one trip to memory; what lies beyond is
+// read again.  Few rows are bound by that trip: a row is spread over as many threads as it has
+// groups of four, its pieces come G at a time (16 rows of 2048: in three strided passes of 256 threads
+// 6.2 us back to back and 10.8 in a decode step, 3.0 and 4.2 so).  Many rows are bound by the memory rate:
+// ONE_WAVE, a wave a row and no barrier at all (with the stream's copy, 1,900 rows of 896 7.1 -> 5.4 us, 4.4 TB/s;
+// 2,048 of 2048 14.3 -> 10.2).
+template <typename T, bool ADD, bool VEC, bool ONE_WAVE, int KEEP, int G>
+__global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
+    const float* __restrict__ x, int splits, size_t stride, const void* __restrict__ w, int w_bf16, float eps,
+    T* __restrict__ out, float* __restrict__ resid, T* __restrict__ copy, const int* __restrict__ rows, int n_rows,
+    int hidden) {
+  constexpr int W = VEC ? 4 : 1;
+  __shared__ float red[ONE_WAVE ? 1 : 32];
+  const int i = ONE_WAVE ? (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6) : (int)blockIdx.x;
+  if (ONE_WAVE && i >= n_rows) return;                     // (a wave's row is its own: no barrier below)
+  const int t = ONE_WAVE ? (int)threadIdx.x & 63 : (int)threadIdx.x, step = (ONE_WAVE ? 64 : (int)blockDim.x) * W;
   const float* src = x + (size_t)(rows ? rows[i] : i) * hidden;
-  float s = 0.f;
-  for (int c = threadIdx.x; c < hidden; c += blockDim.x) s += src[c];
-  const float mean = block_sum(s, red) / (float)hidden;
-  float v = 0.f;
-  for (int c = threadIdx.x; c < hidden; c += blockDim.x) {
-    const float d = src[c] - mean;
-    v += d * d;
-  }
-  const float inv = 1.0f / sqrtf(block_sum(v, red) / (float)hidden + eps);
-  for (int c = threadIdx.x; c < hidden; c += blockDim.x) {
-    const float y = (src[c] - mean) * inv * load_vec(w, w_bf16, c);
-    if (ADD) {
-      const float t = resid[(size_t)i * hidden + c] + y;
-      resid[(size_t)i * hidden + c] = t;
-      if (copy) copy[(size_t)i * hidden + c] = from_float<T>(t);
+  struct alignas(4 * W) Group {
+    float v[W];
+  };
+  auto get = [](const float* p) {
+    Group g;
+    if constexpr (VEC) *(floatx4*)g.v = *(const floatx4*)p;
+    else g.v[0] = *p;
+    return g;
+  };
+  // (loads unconditional: past the last piece the last one again, not added)
+  auto whole = [&](int c) {
+    Group sum = get(src + c);
+    for (int s0 = 1; s0 < splits; s0 += G) {
+      Group p[G];
+#pragma unroll
+      for (int j = 0; j < G; ++j) p[j] = get(src + min(s0 + j, splits - 1) * stride + c);
+#pragma unroll
+      for (int j = 0; j < G; ++j)
+#pragma unroll
+        for (int e = 0; e < W; ++e) sum.v[e] += s0 + j < splits ? p[j].v[e] : 0.f;
+    }
+    return sum;
+  };
+  auto weights = [&](int c) {
+    Group g;
+    if constexpr (VEC) {
+      if (!w_bf16) return get((const float*)w + c);
+      const bf16x4 b = *(const bf16x4*)((const bf16_t*)w + c);
+#pragma unroll
+      for (int e = 0; e < W; ++e) g.v[e] = (float)b[e];
     } else {
-      out[(size_t)i * hidden + c] = from_float<T>(y);
+      g.v[0] = load_vec(w, w_bf16, c);
+    }
+    return g;
+  };
+  auto total = [&](float v, int which) {
+    v = wave_sum(v);
+    if constexpr (!ONE_WAVE) {
+      if ((threadIdx.x & 63) == 0) red[which * 16 + (threadIdx.x >> 6)] = v;
+      __syncthreads();
+      v = 0.f;
+      for (int k = 0; k < (int)(blockDim.x >> 6); ++k) v += red[which * 16 + k];
+    }
+    return v;
+  };
+  Group keep[KEEP], wk[KEEP], old[KEEP];
+  float s = 0.f;
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    const int c = t * W + j * step;
+    if (c < hidden) {
+      keep[j] = whole(c);
+      wk[j] = weights(c);
+      if (ADD) old[j] = get(resid + (size_t)i * hidden + c);
+#pragma unroll
+      for (int e = 0; e < W; ++e) s += keep[j].v[e];
     }
   }
+  for (int c = t * W + KEEP * step; c < hidden; c += step) {
+    const Group g = whole(c);
+#pragma unroll
+    for (int e = 0; e < W; ++e) s += g.v[e];
+  }
+  const float mean = total(s, 0) / (float)hidden;
+  float v = 0.f;
+  auto deviate = [&](const Group& g) {
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      const float d = g.v[e] - mean;
+      v += d * d;
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j)
+    if (t * W + j * step < hidden) deviate(keep[j]);
+  for (int c = t * W + KEEP * step; c < hidden; c += step) deviate(whole(c));
+  const float inv = 1.0f / sqrtf(total(v, 1) / (float)hidden + eps);
+  auto put = [&](int c, const Group& g, const Group& wg, const Group& og) {
+    typedef T Out __attribute__((ext_vector_type(W)));
+    Group y;
+    Out o;
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      y.v[e] = (g.v[e] - mean) * inv * wg.v[e];
+      if (ADD) y.v[e] += og.v[e];
+      o[e] = from_float<T>(y.v[e]);
+    }
+    if (ADD) {
+      float* dst = resid + (size_t)i * hidden + c;
+      if constexpr (VEC) *(floatx4*)dst = *(const floatx4*)y.v;
+      else *dst = y.v[0];
+      if (copy) *(Out*)(copy + (size_t)i * hidden + c) = o;
+    } else {
+      *(Out*)(out + (size_t)i * hidden + c) = o;
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    const int c = t * W + j * step;
+    if (c < hidden) put(c, keep[j], wk[j], old[j]);
+  }
+  for (int c = t * W + KEEP * step; c < hidden; c += step)
+    put(c, whole(c), weights(c), ADD ? get(resid + (size_t)i * hidden + c) : Group{});
+}
+
+template <typename T, bool ADD>
+static void launch_layernorm(const float* x, int splits, size_t stride, const void* w, int w_bf16, float eps, T* out,
+                             float* resid, T* copy, const int* rows, int n_rows, int hidden, hipStream_t stream) {
+  const bool vec = hidden % 4 == 0 && stride % 4 == 0 && (((uintptr_t)x | (uintptr_t)resid) & 15) == 0 &&
+                   (((uintptr_t)out | (uintptr_t)copy) & (4 * sizeof(T) - 1)) == 0 &&
+                   ((uintptr_t)w & (w_bf16 ? 7 : 15)) == 0;
+  // A wave a row where the rows fill the chip and a row fits a wave's registers; else a block, whose
+  // threads cover the row in one group each.
+  if (vec && n_rows > 512 && hidden <= 2048) {
+    if (hidden <= 1024)
+      hipLaunchKernelGGL((layernorm_kernel<T, ADD, true, true, 4, 1>), dim3((n_rows + 3) / 4), dim3(256), 0, stream, x,
+                         splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
+    else
+      hipLaunchKernelGGL((layernorm_kernel<T, ADD, true, true, 8, 1>), dim3((n_rows + 3) / 4), dim3(256), 0, stream, x,
+                         splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
+    return;
+  }
+  int threads = 64;
+  while (threads < 1024 && threads * (vec ? 4 : 1) < hidden) threads += 64;
+  if (n_rows > 128 && threads > 256) threads = 256;
+  if (vec)
+    hipLaunchKernelGGL((layernorm_kernel<T, ADD, true, false, 4, 4>), dim3(n_rows), dim3(threads), 0, stream, x, splits,
+                       stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
+  else
+    hipLaunchKernelGGL((layernorm_kernel<T, ADD, false, false, 4, 4>), dim3(n_rows), dim3(threads), 0, stream, x,
+                       splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
 }
 
 // out: n_out rows of the compute dtype; rows: which rows of x (null: all in order).
@@ -528,27 +652,31 @@ extern "C" int llmlab_layernorm(const float* x, const void* w, int w_dtype, floa
   LLMLAB_REQUIRE(n_out >= 0 && hidden > 0, "layernorm: bad sizes n=%d hidden=%d", n_out, hidden);
   if (n_out == 0) return 0;
   if (out_dtype == DT_BF16)
-    hipLaunchKernelGGL((layernorm_kernel<bf16_t, false>), dim3(n_out), dim3(256), 0, stream, x, w, w_dtype == DT_BF16,
-                       eps, (bf16_t*)out, (float*)nullptr, (bf16_t*)nullptr, rows, hidden);
+    launch_layernorm<bf16_t, false>(x, 1, 0, w, w_dtype == DT_BF16, eps, (bf16_t*)out, nullptr, nullptr, rows, n_out,
+                                    hidden, stream);
   else
-    hipLaunchKernelGGL((layernorm_kernel<float, false>), dim3(n_out), dim3(256), 0, stream, x, w, w_dtype == DT_BF16,
-                       eps, (float*)out, (float*)nullptr, (float*)nullptr, rows, hidden);
+    launch_layernorm<float, false>(x, 1, 0, w, w_dtype == DT_BF16, eps, (float*)out, nullptr, nullptr, rows, n_out,
+                                   hidden, stream);
   LLMLAB_LAUNCH_CHECK("layernorm");
   return 0;
 }
 
-// resid += layernorm(y); copy (may be null, of copy_dtype) receives the new rows of resid.
-extern "C" int llmlab_layernorm_add(const float* y, const void* w, int w_dtype, float eps, float* resid, void* copy,
-                                    int copy_dtype, int n_rows, int hidden, hipStream_t stream) {
+// resid += layernorm(y), y the sum of `splits` pieces `stride` numbers apart; copy (may be null, of copy_dtype)
+// receives the new rows of resid.
+extern "C" int llmlab_layernorm_add(const float* y, int splits, size_t stride, const void* w, int w_dtype, float eps,
+                                    float* resid, void* copy, int copy_dtype, int n_rows, int hidden,
+                                    hipStream_t stream) {
   LLMLAB_REQUIRE(n_rows >= 0 && hidden > 0, "layernorm_add: bad sizes n=%d hidden=%d", n_rows, hidden);
   LLMLAB_REQUIRE(y != resid, "layernorm_add: the sublayer's output and the stream are two buffers");
+  LLMLAB_REQUIRE(splits == 1 || (splits > 1 && stride >= (size_t)n_rows * hidden),
+                 "layernorm_add: %d pieces do not follow each other", splits);
   if (n_rows == 0) return 0;
   if (copy_dtype == DT_BF16)
-    hipLaunchKernelGGL((layernorm_kernel<bf16_t, true>), dim3(n_rows), dim3(256), 0, stream, y, w, w_dtype == DT_BF16,
-                       eps, (bf16_t*)nullptr, resid, (bf16_t*)copy, (const int*)nullptr, hidden);
+    launch_layernorm<bf16_t, true>(y, splits, stride, w, w_dtype == DT_BF16, eps, nullptr, resid, (bf16_t*)copy, nullptr,
+                                   n_rows, hidden, stream);
   else
-    hipLaunchKernelGGL((layernorm_kernel<float, true>), dim3(n_rows), dim3(256), 0, stream, y, w, w_dtype == DT_BF16,
-                       eps, (float*)nullptr, resid, (float*)copy, (const int*)nullptr, hidden);
+    launch_layernorm<float, true>(y, splits, stride, w, w_dtype == DT_BF16, eps, nullptr, resid, (float*)copy, nullptr,
+                                  n_rows, hidden, stream);
   LLMLAB_LAUNCH_CHECK("layernorm_add");
   return 0;
 }

@@ -265,8 +265,8 @@ class HipOps:
         c.llmlab_add_pending.restype = _c_int
         c.llmlab_layernorm.argtypes = [_c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_ptr]
         c.llmlab_layernorm.restype = _c_int
-        c.llmlab_layernorm_add.argtypes = [_c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
-                                           _c_ptr]
+        c.llmlab_layernorm_add.argtypes = [_c_ptr, _c_int, _c_size, _c_ptr, _c_int, _c_float, _c_ptr, _c_ptr, _c_int, _c_int,
+                                           _c_int, _c_ptr]
         c.llmlab_layernorm_add.restype = _c_int
         c.llmlab_activation.argtypes = [_c_ptr, _c_ptr, _c_int, _c_int, _c_long, _c_ptr]
         c.llmlab_activation.restype = _c_int
@@ -1086,9 +1086,15 @@ class HipOps:
         self._call(self._core.llmlab_layernorm, self._ptr(x), self._ptr(weight), _dt(weight), float(eps),
                    self._ptr(out), _dt(out), self._ptr(rows), n_out, hidden, self._stream())
 
+    LAYERNORM_ADDS_PIECES = True
+
     def layernorm_add(self, y, weight, eps, resid, copy=None) -> None:
-        """``resid += layernorm(y)`` on the float32 stream; ``copy`` (compute dtype, same shape)
-        receives the stream's new rows for the product that reads them next."""
+        """``resid += layernorm(y)`` on the float32 stream (``y`` float32, or ``PendingSums`` whose pieces are
+        summed on the way); ``copy`` (compute dtype, same shape) receives the stream's new rows for the
+        product that reads them next."""
+        splits, stride = 1, 0
+        if isinstance(y, PendingSums):
+            splits, stride, y = y.splits, y.parts.stride(0), y.parts[0]
         self._need(y, "sublayer output", torch.float32)
         self._need(resid, "residual stream", torch.float32)
         self._need(weight, "norm weight")
@@ -1100,7 +1106,7 @@ class HipOps:
             self._need(copy, "copy of the stream")
             if tuple(copy.shape) != (rows, hidden):
                 raise ValueError("layernorm_add: the copy has the stream's shape")
-        self._call(self._core.llmlab_layernorm_add, self._ptr(y), self._ptr(weight), _dt(weight), float(eps),
+        self._call(self._core.llmlab_layernorm_add, self._ptr(y), splits, stride, self._ptr(weight), _dt(weight), float(eps),
                    self._ptr(resid), self._ptr(copy), _dt(copy) if copy is not None else DT_F32, rows, hidden,
                    self._stream())
 

@@ -186,9 +186,13 @@ class SublayerNormBlock(Block):
 
     def _sublayer(self, part, norm, h, residual, ctx, *entry):
         y = ctx.scratch("block.sublayer_out", tuple(residual.shape), torch.float32)
-        if hasattr(part, "forward_pending") and getattr(norm, "adds_pieces", False):
-            pieces = part.forward_pending(h, y, ctx, *entry)      # (a product left in pieces is summed by the norm)
-            return y if pieces is None else pieces
+        if getattr(norm, "adds_pieces", False):      # (a product left in pieces is summed by the norm)
+            leave = getattr(part, "forward_pending", None)
+            if leave is None and entry and not self.token_shift:      # (a mixer)
+                leave = getattr(part, "forward_split", None)
+            if leave is not None:
+                pieces = leave(h, y, ctx, *entry)
+                return y if pieces is None else pieces
         if part.writes_output:
             part.forward_into(h, y, ctx, *entry)
         else:

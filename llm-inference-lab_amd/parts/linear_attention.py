@@ -224,6 +224,13 @@ class GatedLinearAttention(ScanMixer):
         self.norm_weight = pad_heads(tensors[t["out_norm"]].float(), 1, self.file_value_dim, self.value_dim).contiguous()
 
     def forward_into(self, h, out, ctx, entry):
+        self.ops.linear_logits(self._mixed(h, ctx, entry), self.w_o, out)
+
+    def forward_split(self, h, out, ctx, entry):
+        return self._product_split(self._mixed(h, ctx, entry), self.w_o, out, ctx)
+
+    def _mixed(self, h, ctx, entry):
+        """The gated heads' outputs of this step's rows, side by side, in the compute dtype."""
         ops, rows, o = self.ops, h.shape[0], self.offsets
         proj = ctx.scratch("linear_attention.proj", (rows, self.in_size), torch.float32)
         ops.linear_logits(h, self.w_in, proj)
@@ -238,10 +245,9 @@ class GatedLinearAttention(ScanMixer):
         def in_chunks(mixed):
             ops.gla_decay(proj[:, o["decay_down"]:], self.decay_rank, self.w_decay, self.b_decay, self.tau, decay, as_log=True)
             self._in_chunks(proj, ctx, entry, off, decay, self.norm_weight, self.norm_eps, "silu", self.q_scale, mixed)
-        mixed = self._recur(proj, ctx, entry, off, self.norm_weight, self.norm_eps, "silu", self.q_scale, many_rows,
-                            in_chunks, self.decay_rank,
-                            decay=(o["decay_down"], self.decay_rank, self.w_decay, self.b_decay, "sigmoid", self.tau))
-        ops.linear_logits(mixed, self.w_o, out)
+        return self._recur(proj, ctx, entry, off, self.norm_weight, self.norm_eps, "silu", self.q_scale, many_rows,
+                           in_chunks, self.decay_rank,
+                           decay=(o["decay_down"], self.decay_rank, self.w_decay, self.b_decay, "sigmoid", self.tau))
 
     def weight_bytes(self):
         return sum(w.numel() * w.element_size()

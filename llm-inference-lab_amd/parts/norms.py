@@ -106,8 +106,14 @@ class LayerNorm(Norm):
     def forward(self, x, out, rows=None):
         self.ops.layernorm(x, self.weight, self.eps, out, rows)
 
+    @property
+    def adds_pieces(self):
+        """Whether ``add_into`` takes a result left in pieces as well (``PendingSums``)."""
+        return getattr(self.ops, "LAYERNORM_ADDS_PIECES", False)
+
     def add_into(self, y, stream, copy=None):
-        """``stream += norm(y)``; ``copy`` (compute dtype) receives the stream's new rows."""
+        """``stream += norm(y)`` (``y`` float32 or ``PendingSums``); ``copy`` (compute dtype) receives the stream's new
+        rows."""
         self.ops.layernorm_add(y, self.weight, self.eps, stream, copy)
 
     def weight_bytes(self):
