@@ -333,8 +333,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
   constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
   constexpr int TM = WTM / 16, TN = WTN / 16;
   constexpr int KCH = BK / 8;                // 16-byte chunks in a row of a tile
-  constexpr int A_CHUNKS = BM * KCH / NT;    // chunks of x per thread
-  static_assert(A_CHUNKS >= 1 && BM * KCH % NT == 0, "tile too small");
+  constexpr int A_CHUNKS = (BM * KCH + NT - 1) / NT;    // chunks of x per thread (past the tile's last: that one again)
+  static_assert(BM * KCH >= NT, "tile too small");
+  auto chunk_of = [&](int i) { return BM * KCH % NT == 0 ? (int)threadIdx.x + i * NT : min((int)threadIdx.x + i * NT, BM * KCH - 1); };
   // three stages of LDS for x: the tile after the next is put in while this one is
   // multiplied and the next one's fragments are read, one barrier per tile
   constexpr int A_STAGE = BM * LDS_STRIDE;
@@ -413,14 +414,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
   if constexpr (GROUPED) {
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const int m = min(m0 + (tid + i * NT) / KCH, M - 1);
+      const int m = min(m0 + chunk_of(i) / KCH, M - 1);
       gathered[i] = e.g_rows ? max(e.g_rows[m], 0) : m;
     }
   }
   auto fetch = [&](int slot, int k0) {
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const int ch = tid + i * NT, row = ch / KCH, kc = (ch % KCH) * 8;
+      const int ch = chunk_of(i), row = ch / KCH, kc = (ch % KCH) * 8;
       const int m = GROUPED ? gathered[i] : min(m0 + row, M - 1), k = min(k0 + kc, K - 8);
       ra[slot][i] = *(const bf16x8*)(A + (size_t)m * K + k);
     }
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
     bf16_t* As = As2 + stage * A_STAGE;
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const int ch = tid + i * NT, row = ch / KCH, kc = (ch % KCH) * 8;
+      const int ch = chunk_of(i), row = ch / KCH, kc = (ch % KCH) * 8;
       *(bf16x8*)(As + row * LDS_STRIDE + kc) = ra[slot][i];
     }
   };
@@ -1278,18 +1279,21 @@ constexpr int F32_ROWS_MAX = 64;     // up to here the few-row kernel (the tiled
 // bytes a microsecond, the chip 5.3e6 at most (one tile of rows, 17 to 64 of them, of
 // matrices from 9 to 283 MB, in 4 or 8 pieces: the estimate is within 2 us of the
 // measurement).
-enum { TILE_64 = 0, TILE_64x128 = 1, TILE_128 = 2, TILE_128x256 = 3, TILE_256 = 4, TILE_192 = 5, TILE_KINDS = 6 };
+enum { TILE_64 = 0, TILE_64x128 = 1, TILE_128 = 2, TILE_128x256 = 3, TILE_256 = 4, TILE_192 = 5, TILE_KINDS = 6,
+       // chosen by their own rule (one_round_tile) for whole products
+       TILE_64x96 = 6, TILE_64x160 = 7, TILE_64x224 = 8, TILE_128x160 = 9, TILE_ALL = 10 };
 struct TileModel {
   int bm, bn;
   double L, f, tk, resident, stream;
   int whole_rounds;
 };
-static const TileModel TILE_MODELS[TILE_KINDS] = {{64, 64, 6.39, 0.79, 0.289, 1.0, 20e3, 0},
+static const TileModel TILE_MODELS[TILE_ALL] = {{64, 64, 6.39, 0.79, 0.289, 1.0, 20e3, 0},
                                                   {64, 128, 6.54, 0.71, 0.5, 1.5, 27e3, 0},
                                                   {128, 128, 8.0, 0.48, 0.66, 1.0, 24e3, 0},
                                                   {128, 256, 0.0, 6.16, 0.945, 1.0, 24e3, 1},
                                                   {256, 256, 0.0, 9.2, 1.8, 1.0, 24e3, 1},
-                                                  {192, 256, 0.0, 9.2, 1.4, 1.0, 24e3, 1}};
+                                                  {192, 256, 0.0, 9.2, 1.4, 1.0, 24e3, 1},
+                                                  {64, 96}, {64, 160}, {64, 224}, {128, 160}};
 constexpr double CHIP_STREAM = 5.3e6;     // bytes a microsecond
 
 // The tiles of the two groups of waves: whole rounds of one block a unit; with 256 rows a
@@ -1325,7 +1329,7 @@ static double tile_cost(int kind, int M, int N, int K, int num_cus, int pieces) 
 
 // Debug interface (kernels/debug.py): a tile can be forced, for tests and measurements
 // (0 = choose; 64, 130 = 64 x 128, 129 = 128 x 128, 131 = 128 x 256, 132 = 256 x 256, 133 =
-// 192 x 256; -131 = choose among the first three; -256 and below: the tiles of two groups
+// 192 x 256, 134 / 135 / 136 = 64 x 96 / 160 / 224, 137 = 128 x 160; -131 = choose among the first three; -256 and below: the tiles of two groups
 // of waves from so many rows on).
 static int g_force_tile = 0, g_without_wide = 0, g_pp_min_rows = 512;
 // The 128 x 256 tile is weighed from so many rows on.  (By the product alone it would pay from
@@ -1337,6 +1341,32 @@ extern "C" void llmlab_debug_gemm_tile(int tile) {
   g_force_tile = tile > 0 ? tile : 0;
   g_without_wide = tile == -131;
   g_pp_min_rows = tile <= -256 ? -tile : 512;
+}
+
+// Up to 128 rows of a wide matrix: the product is bound by the read of W, every compute unit draws its
+// share at the same rate, and what matters is that all of them draw until the end: one round of
+// blocks that nearly fills the chip, each wave with 32 columns of its own.  The width that does that,
+// 32 times 3, 4, 5 or 7, is the narrowest whose blocks find a unit each (-1: none does, or the round would
+// leave a fifth of the units, of the narrowest tile three tenths, without a block).  Inner sizes from 1,536 up,
+// measured against the best of the other tiles / the estimates' pick: 64 rows of 37888 x 3584 (160 columns,
+// 237 blocks) 57 us against 70 / 70, of 22016 x 2048 (96, 230) 26.2 / 27.2 / 27.8, of 17920 x 1536 (96, 187)
+// 19.6 / 20.9 / 22.9, of 27648 x 5120 (128, 216) 62 / 62 / 69, of 55296 x 5120 (224, 247) 105 / 109 / 109; 17 rows
+// the same; 128 rows of 37888 x 3584 in one tile of rows (160) 70 / 78 / 79, of 17920 x 1536 in two (2 x 112
+// blocks) 23.9 / 27.1 / 27.3.
+static int one_round_tile(int M, int N, int K, int num_cus) {
+  if (M > 128 || K < 1024) return -1;
+  auto fills = [&](int width, int tiles, double least) {
+    const long blocks = (long)((N + width - 1) / width) * tiles;
+    return blocks <= num_cus && blocks >= least * num_cus;
+  };
+  if (M > 64) {
+    if (fills(160, 1, 0.8)) return TILE_128x160;
+    return fills(160, 2, 0.8) ? TILE_64x160 : -1;
+  }
+  if (fills(96, 1, 0.7)) return TILE_64x96;
+  if (fills(128, 1, 0.8)) return TILE_64x128;
+  if (fills(160, 1, 0.8)) return TILE_64x160;
+  return fills(224, 1, 0.8) ? TILE_64x224 : -1;
 }
 
 // By an estimate of the time, fitted to a sweep of seven matrices of two model shapes at 65 to 4,000 rows
@@ -1450,6 +1480,18 @@ static int choose_tile(int M, int N, int K, int num_cus) {
   return best;
 }
 
+// The tile of a product that is neither cut into pieces nor written into the cache by heads (those need a
+// width that heads divide): the rule for few rows of a wide matrix, else the estimates.
+static int plain_tile(int M, int N, int K, int num_cus) {
+  if (g_force_tile >= 134 && g_force_tile <= 137) return TILE_64x96 + (g_force_tile - 134);
+  const int one_round = g_force_tile == 0 && !g_without_wide ? one_round_tile(M, N, K, num_cus) : -1;
+  return one_round >= 0 ? one_round : choose_tile(M, N, K, num_cus);
+}
+// ... its width (for tests)
+extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
+  return TILE_MODELS[plain_tile(M, N, K, num_cus > 0 ? num_cus : 256)].bn;
+}
+
 template <int EPI>
 static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArgs& e, int M, int N, int K,
                         int pieces, hipStream_t stream) {
@@ -1463,11 +1505,19 @@ static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArg
     hipLaunchKernelGGL((gemm_bf16_tiled<128, 128, 64, 1, 4, EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
   else if (kind == TILE_128x256)
     hipLaunchKernelGGL((gemm_bf16_tiled<128, 256, 64, 1, 8, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
-  else {
-    if (kind == TILE_256)
-      hipLaunchKernelGGL((gemm_bf16_pingpong<256, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
-    else
-      hipLaunchKernelGGL((gemm_bf16_pingpong<192, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  else if (kind == TILE_256)
+    hipLaunchKernelGGL((gemm_bf16_pingpong<256, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  else if (kind == TILE_192)
+    hipLaunchKernelGGL((gemm_bf16_pingpong<192, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  if constexpr (EPI != EPI_QKV && EPI != EPI_PART) {      // (plain_tile: whole products only)
+    if (kind == TILE_64x96)
+      hipLaunchKernelGGL((gemm_bf16_tiled<64, 96, 64, 1, 3, EPI>), grid, dim3(192), 0, stream, A, W, e, M, N, K);
+    else if (kind == TILE_64x160)
+      hipLaunchKernelGGL((gemm_bf16_tiled<64, 160, 64, 1, 5, EPI>), grid, dim3(320), 0, stream, A, W, e, M, N, K);
+    else if (kind == TILE_64x224)
+      hipLaunchKernelGGL((gemm_bf16_tiled<64, 224, 64, 1, 7, EPI>), grid, dim3(448), 0, stream, A, W, e, M, N, K);
+    else if (kind == TILE_128x160)
+      hipLaunchKernelGGL((gemm_bf16_tiled<128, 160, 64, 1, 5, EPI>), grid, dim3(320), 0, stream, A, W, e, M, N, K);
   }
 }
 
@@ -1699,7 +1749,7 @@ extern "C" int llmlab_linear(const void* x, const void* w, int dtype, int epilog
                    "linear(bfloat16): operands must be 16-byte aligned");
     const bf16_t* A = (const bf16_t*)x;
     const bf16_t* W = (const bf16_t*)w;
-    const int kind = choose_tile(M, N, K, num_cus);
+    const int kind = plain_tile(M, N, K, num_cus);
     switch (epilogue) {
       case EPI_STORE: launch_tile<EPI_STORE>(kind, A, W, e, M, N, K, 1, stream); break;
       case EPI_RESID: launch_tile<EPI_RESID>(kind, A, W, e, M, N, K, 1, stream); break;
