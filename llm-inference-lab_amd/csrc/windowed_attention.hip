@@ -1020,6 +1020,7 @@ struct MfmaArgs {
   int splits; float* part_o; float* part_ml;      // (decoding) [rows, heads, splits, E] and [rows, heads, splits, 2]
   Gate gate;
   int mode;                                       // MODE_SOFTMAX, or MODE_SIGMOID (sink: the bias of the scores)
+  int most_shares;                                // (decoding) the shares that a row of any length may be cut into
 };
 
 // Prompts: a wave takes 16 consecutive rows and one head, a block four such tiles.  Rows of
@@ -1356,7 +1357,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
 // one key/value head (16 at a time) and one of `splits` shares of the row's key tiles, so that
 // few rows still fill the chip.  With one share the result is final; else the share's
 // maximum, denominator and unnormalised sum go to part_ml / part_o for the merge kernel.
-// The sink enters the first share only.
+// The sink enters the first share only.  How a row's keys are cut follows from the row alone (two tiles a share
+// at least, `most_shares` at most), not from `splits`, which holds for the step's longest row: a step
+// replayed from a graph has shares for a longer one (the others weigh zero in the merge, exactly), and sums the
+// same numbers in the same order.
 template <int DC, int EB>
 __global__ __launch_bounds__(64) void sink_window_attention_grouped_kernel(MfmaArgs a) {
   constexpr int D = 32 * DC, E = 16 * EB;
@@ -1387,7 +1391,8 @@ __global__ __launch_bounds__(64) void sink_window_attention_grouped_kernel(MfmaA
 #pragma unroll
   for (int eb = 0; eb < EB; ++eb) run.o[eb] = floatx4{0.f, 0.f, 0.f, 0.f};
   const KeyTiles kt(pos, pos, a.mask);
-  const int per = (kt.tiles + a.splits - 1) / a.splits;
+  const int shares = min(min((kt.tiles + 1) / 2, a.most_shares), a.splits);
+  const int per = (kt.tiles + shares - 1) / shares;
   const int t_begin = z * per, t_end = (z + 1) * per < kt.tiles ? (z + 1) * per : kt.tiles;
   attend_tiles<DC, EB>(kt, t_begin, t_end, qf, head_ok, pos, a.table + (size_t)b * a.max_pages, a.page_size, a.n_kv, g,
                        a.k_cache, a.v_cache, a.mask, a.scale, run, a.mode, bias);
@@ -1545,7 +1550,7 @@ extern "C" int llmlab_sink_window_attention(const void* q, int dtype, int rows, 
   if (long_from > 0) {
     MfmaArgs a{(const bf16_t*)q, rows, n_heads, n_kv, (const bf16_t*)k_cache, (const bf16_t*)v_cache, table, max_pages,
                page_size, positions, row_req, mask, sink, scale, (bf16_t*)out, q_start, long_from, 1,
-               nullptr, nullptr, gates, mode};
+               nullptr, nullptr, gates, mode, 1};
     if (launches & 2) {
       // heads that read the same keys and values share the tiles a block stages in LDS
       const int group = n_heads / n_kv;
@@ -1560,15 +1565,17 @@ extern "C" int llmlab_sink_window_attention(const void* q, int dtype, int rows, 
       // shorter than two tiles of 32 keys, and no more than the scratch holds
       const int group = n_heads / n_kv, per_group = (group + 15) / 16;
       const long waves = (long)rows * n_kv * per_group;
-      const int tiles = (max_keys + 31) / 32 + 1;
-      long splits = (4L * num_cus + waves - 1) / waves;
-      if (splits > tiles / 2) splits = tiles / 2;
+      const int tiles = (max_keys + 31) / 32 + 1 + (keep_first > 0 ? 1 : 0);      // (no row has more, but for a cut
+                                                                                  // window's: its last share is longer)
+      long most = (4L * num_cus + waves - 1) / waves;
       const size_t per_split = (size_t)rows * n_heads * (E + 2);
-      if (workspace == nullptr) splits = 1;
-      else if (splits * per_split > workspace_floats) splits = (long)(workspace_floats / per_split);
-      if (splits < 1) splits = 1;
-      if (splits > MERGE_MAX_SPLITS) splits = MERGE_MAX_SPLITS;
+      if (workspace == nullptr) most = 1;
+      else if (most * per_split > workspace_floats) most = (long)(workspace_floats / per_split);
+      if (most < 1) most = 1;
+      if (most > MERGE_MAX_SPLITS) most = MERGE_MAX_SPLITS;
+      const long splits = tiles / 2 < 1 ? 1 : (tiles / 2 < most ? tiles / 2 : most);
       a.splits = (int)splits;
+      a.most_shares = (int)most;
       a.part_o = workspace;
       a.part_ml = workspace ? workspace + (size_t)rows * n_heads * splits * E : nullptr;
       LLMLAB_REQUIRE(n_kv * per_group <= 65535, "sink_window_attention: too many heads");
