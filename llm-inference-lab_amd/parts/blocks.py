@@ -7,7 +7,7 @@ import torch
 
 from ..config.spec import PartSpec
 from ..weights.loader import TensorSpec, MATRIX, VECTOR, INIT_ZEROS
-from .base import Block, Part, NormedInput
+from .base import Block, Part, NormedInput, NormedPair
 from .registry import register_part, build_part
 
 
@@ -192,6 +192,9 @@ class SublayerNormBlock(Block):
                 leave = getattr(part, "forward_split", None)
             if leave is not None:
                 pieces = leave(h, y, ctx, *entry)
+                if isinstance(pieces, NormedPair) and not getattr(norm, "adds_pairs", True):
+                    self.ops.normed_sum(y, pieces.y1, pieces.w1, pieces.a, pieces.y2, pieces.w2, pieces.b, pieces.eps)
+                    return y
                 return y if pieces is None else pieces
         if part.writes_output:
             part.forward_into(h, y, ctx, *entry)

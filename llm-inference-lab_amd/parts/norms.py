@@ -106,6 +106,8 @@ class LayerNorm(Norm):
     def forward(self, x, out, rows=None):
         self.ops.layernorm(x, self.weight, self.eps, out, rows)
 
+    adds_pairs = False      # ``add_into`` takes no ``NormedPair``: its sum is made before
+
     @property
     def adds_pieces(self):
         """Whether ``add_into`` takes a result left in pieces as well (``PendingSums``)."""

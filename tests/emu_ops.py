@@ -253,9 +253,12 @@ class EmuOps:
         v = x.float() if rows is None else x.float()[rows.long()]
         out.copy_(self._layernorm(v, weight, eps).to(out.dtype))
 
+    LAYERNORM_ADDS_PIECES = True
+
     def layernorm_add(self, y, weight, eps, resid, copy=None):
         self._count("layernorm_add")
-        resid.add_(self._layernorm(y.float(), weight, eps))
+        v = self._owed(y) if isinstance(y, PendingSums) else y.float()
+        resid.add_(self._layernorm(v, weight, eps))
         if copy is not None:
             copy.copy_(resid.to(copy.dtype))
 
