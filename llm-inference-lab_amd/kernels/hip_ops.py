@@ -1094,6 +1094,8 @@ class HipOps:
         product that reads them next."""
         splits, stride = 1, 0
         if isinstance(y, PendingSums):
+            if y.parts.dim() != 3 or not 1 <= y.splits <= y.parts.shape[0]:
+                raise ValueError(f"layernorm_add: {y.splits} pieces of {tuple(y.parts.shape)}")
             splits, stride, y = y.splits, y.parts.stride(0), y.parts[0]
         self._need(y, "sublayer output", torch.float32)
         self._need(resid, "residual stream", torch.float32)

@@ -154,3 +154,24 @@ def test_models_whose_products_are_cut(backend, dtype, design, name):
             err = torch.cat([(got[rid].double() - want[rid].double()).flatten() for rid in seqs])
             assert float(err.square().mean().sqrt()) <= bounds.TOL_BF16[0] and float(err.abs().max()) <= bounds.TOL_BF16[1]
     assert made[10 ** 6] == 0 and (made[1] > 0) == (backend == "hip" or dtype == "bf16")
+
+
+@pytest.mark.parametrize("shape,splits", [((2, 3, 8), 3), ((1, 3, 8), 2), ((2, 3, 8), 0), ((3, 8), 1)])
+def test_pieces_that_are_not_there(shape, splits):
+    """A layer norm of more pieces than the buffer holds is refused before any launch."""
+    from llm_inference_lab_amd.kernels.hip_ops import HipOps
+    from llm_inference_lab_amd.parts.base import PendingSums
+    ops = HipOps.__new__(HipOps)          # (its checks alone: no library, no GPU)
+    ops.device = torch.device("cpu")
+
+    class Library:
+        llmlab_layernorm_add = None
+    ops._core = Library()
+    launched = []
+    ops._call = lambda *a: launched.append(a)
+    ops._stream = lambda: None
+    with pytest.raises(ValueError):
+        ops.layernorm_add(PendingSums(torch.zeros(shape), splits), torch.ones(8), 1e-6, torch.zeros(3, 8))
+    assert not launched
+    ops.layernorm_add(PendingSums(torch.zeros(2, 3, 8), 2), torch.ones(8), 1e-6, torch.zeros(3, 8))
+    assert len(launched) == 1
