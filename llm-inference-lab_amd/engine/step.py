@@ -170,12 +170,15 @@ class StepContext:
                                        f"available after the weights and the cache")
             self.scratch_bytes += need - (0 if buf is None else buf.numel() * width)
             self.scratch_allocations += 1
-            buf = None                      # give the old one back before taking the new
-            self._scratch.pop(key, None)
+            if buf is not None:
+                # (a buffer asked for the first time leaves the others where they are: the calls written
+                # down and the graphs captured so far stay as they are)
+                self.scratch_version += 1
+                self._views = {k: v for k, v in self._views.items() if (k[0], k[1]) != key}
+                buf = None                  # give the old one back before taking the new
+                self._scratch.pop(key, None)
             buf = torch.empty(max(count, 1), dtype=dtype, device=self.device)
             self._scratch[key] = buf
-            self.scratch_version += 1
-            self._views = {k: v for k, v in self._views.items() if (k[0], k[1]) != key}
         view = buf[:count].view(shape)
         if len(self._views) < 4096 and isinstance(shape, tuple):
             self._views[(name, dtype, shape)] = view

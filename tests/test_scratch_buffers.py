@@ -1,0 +1,52 @@
+"""Scratch buffers asked for in the middle of a run: a new one moves none of the others, so the calls that a block
+has written down stay and later blocks' are written down; one that grows moves, and drops them."""
+import pytest
+import torch
+
+import helpers as H
+import vivevik_cases as V
+from emu_ops import EmuOps
+
+
+def vivevik(**kw):
+    return V.make_engine("P", 1, "bf16", ops=EmuOps(), device="cpu", **kw)
+
+
+def test_first_decode_step_writes_all_blocks_down():
+    """A prompt of many rows cuts no product; the first decode step does and asks for the pieces' buffers: its
+    blocks' calls are written down all the same, and the second step makes them from the list."""
+    engine = vivevik()
+    engine.ops.rules.min_steps_per_split = 1
+    ids = V.random_ids(V.config_of("P"), 72, 3)
+    request = engine.open("r")
+    engine.step([H.lab.StepEntry(request, ids[:70], [])])
+    made = engine.step_fn.ctx.scratch_allocations
+    prompt = engine.model.launches_recorded
+    keeping = sum(engine.model.blocks[v.block].keeps_launches for v in engine.model.entries)
+    engine.step([H.lab.StepEntry(request, [ids[70]], [0])])
+    assert engine.step_fn.ctx.scratch_allocations > made
+    assert engine.model.launches_recorded - prompt == keeping > 0
+    replayed = engine.model.launches_replayed
+    engine.step([H.lab.StepEntry(request, [ids[71]], [0])])
+    assert engine.model.launches_replayed - replayed == keeping
+    engine.close(request)
+
+
+def test_a_buffer_that_grows_moves(monkeypatch):
+    ctx = vivevik().step_fn.ctx
+    small = ctx.scratch("a", (4, 4), torch.float32)
+    assert ctx.scratch("a", (2, 4), torch.float32).data_ptr() == small.data_ptr()
+    before = ctx.scratch_version
+    ctx.scratch("b", (4, 4), torch.float32)
+    assert ctx.scratch_version == before
+    ctx.scratch("a", (8, 4), torch.float32)
+    assert ctx.scratch_version == before + 1
+
+    def full(*args, **kw):
+        raise RuntimeError("no memory")
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", lambda *a, **kw: full() if a and a[0] == 64 else torch.zeros(*a, **kw))
+        with pytest.raises(RuntimeError):
+            ctx.scratch("a", (16, 4), torch.float32)
+    assert ctx.scratch_version == before + 2          # (the old one has been given back: nothing may still point at it)
+    assert ctx.scratch("a", (8, 4), torch.float32).shape == (8, 4)
