@@ -334,8 +334,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
   constexpr int TM = WTM / 16, TN = WTN / 16;
   constexpr int KCH = BK / 8;                // 16-byte chunks in a row of a tile
   constexpr int A_CHUNKS = (BM * KCH + NT - 1) / NT;    // chunks of x per thread (past the tile's last: that one again)
+  constexpr bool EVEN = BM * KCH % NT == 0;
   static_assert(BM * KCH >= NT, "tile too small");
-  auto chunk_of = [&](int i) { return BM * KCH % NT == 0 ? (int)threadIdx.x + i * NT : min((int)threadIdx.x + i * NT, BM * KCH - 1); };
   // three stages of LDS for x: the tile after the next is put in while this one is
   // multiplied and the next one's fragments are read, one barrier per tile
   constexpr int A_STAGE = BM * LDS_STRIDE;
@@ -414,14 +414,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
   if constexpr (GROUPED) {
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const int m = min(m0 + chunk_of(i) / KCH, M - 1);
+      const int m = min(m0 + (EVEN ? tid + i * NT : min(tid + i * NT, BM * KCH - 1)) / KCH, M - 1);
       gathered[i] = e.g_rows ? max(e.g_rows[m], 0) : m;
     }
   }
   auto fetch = [&](int slot, int k0) {
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const int ch = chunk_of(i), row = ch / KCH, kc = (ch % KCH) * 8;
+      const int ch = EVEN ? tid + i * NT : min(tid + i * NT, BM * KCH - 1), row = ch / KCH, kc = (ch % KCH) * 8;
       const int m = GROUPED ? gathered[i] : min(m0 + row, M - 1), k = min(k0 + kc, K - 8);
       ra[slot][i] = *(const bf16x8*)(A + (size_t)m * K + k);
     }
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
     bf16_t* As = As2 + stage * A_STAGE;
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
-      const int ch = chunk_of(i), row = ch / KCH, kc = (ch % KCH) * 8;
+      const int ch = EVEN ? tid + i * NT : min(tid + i * NT, BM * KCH - 1), row = ch / KCH, kc = (ch % KCH) * 8;
       *(bf16x8*)(As + row * LDS_STRIDE + kc) = ra[slot][i];
     }
   };
