@@ -822,7 +822,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 }
 
 // Many rows in float32: the products are taken by the bfloat16 matrix instructions without giving
-// up a bit of the operands.  A float32 number is the sum of three bfloat16 numbers, x = h + m + l (h =
+// up a bit of the operands.  A float32 number of 2^-110 to 3.39e38 is the sum of three bfloat16 numbers, x = h + m + l (h =
 // x rounded to nearest, m = x - h rounded, l the rest: 24 bits of significand in three times 8, the
 // differences exact), and x w = h_x h_w + h_x m_w + m_x h_w + m_x m_w + h_x l_w + l_x h_w up to terms below
 // 2^-24 of |x w|, less than what one rounding of a 32-bit sum costs.  Every bfloat16 product is
@@ -846,10 +846,12 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // x^T, so that a lane holds four neighbouring columns of a row, and for SWIGLU the gate and the up
 // value of an output.
 //
-// Numbers that bfloat16 would round to infinity (3.396e38 and above, and infinity itself) have no
-// such parts: a block that meets one takes its outputs again with plain FMAs at the end.  (NaN needs no
-// care: all three parts are NaN.)
-constexpr float SPLIT_LIMIT = 3.3961775e38f;       // the smallest number that rounds to infinity in bfloat16
+// Two ranges have no such parts.  Of numbers below 2^-110 the last bits fall under bfloat16's smallest number, 2^-133
+// (the sum of the parts is then off by 2.4e-7 of the number at 2^-112, 9.5e-4 at 2^-124): it shows in what the third
+// part is rounded from, whose lower half is not zero.  And numbers that bfloat16 rounds to infinity (3.396e38 and above,
+// infinity itself), like products of parts that overflow where the whole product does not, or overflow with both
+// signs, leave an output that is not finite.  A block that meets either takes its outputs again on
+// v_mfma_f32_16x16x4_f32, operands straight from memory: true 32-bit products over the whole range.
 template <int EPI, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const float* __restrict__ A,
                                                                 const float* __restrict__ W, EpiArgs e, int M,
@@ -860,7 +862,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
   static_assert(LA >= 1 && LB >= 1 && LA * NW * 16 == BM && LB * NW * 16 == BN && TN % 2 == 0, "pieces");
   constexpr int STAGE = (BM + BN) / 16 * 3072;
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
-  __shared__ int s_big;
+  __shared__ int s_again;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % WM, wn = wave / WM;
   int bx = blockIdx.x, by = blockIdx.y;
@@ -882,7 +884,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
     e.out = (float*)e.out + (size_t)blockIdx.z * e.part_stride;
     if (blockIdx.z > 0) e.bias = nullptr;
   }
-  if (tid == 0) s_big = 0;
+  if (tid == 0) s_again = 0;
 
   floatx4 acc[TN][TM];
 #pragma unroll
@@ -931,17 +933,18 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
       }
     }
   };
-  float biggest = 0.f;
+  unsigned rest = 0;
   auto split = [&](const floatx4 (&v)[2], char* to) {
     bf16x8 h, m, l;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       const float x = v[q >> 2][q & 3];
-      biggest = fmaxf(biggest, fabsf(x));
       h[q] = (bf16_t)x;
       const float r = x - (float)h[q];
       m[q] = (bf16_t)r;
-      l[q] = (bf16_t)(r - (float)m[q]);
+      const float s = r - (float)m[q];
+      l[q] = (bf16_t)s;
+      rest |= __float_as_uint(s);      // (its lower half is zero where bfloat16 holds it)
     }
     *(bf16x8*)to = h;
     *(bf16x8*)(to + 1024) = m;
@@ -1004,20 +1007,43 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
       __syncthreads();
     }
   }
-  if (biggest >= SPLIT_LIMIT) s_big = 1;      // (any thread's; the same value from all)
+  bool again = (rest & 0xffffu) != 0;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) again |= !(fabsf(acc[j][i][x]) < __builtin_inff());
+  if (again) s_again = 1;      // (any thread's; the same value from all)
   __syncthreads();
-  if (s_big) {
+  if (s_again) {
+    // lane (c, g) holds the numbers 4 g .. 4 g + 3 of 16 of its row; an instruction contracts one of each group
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const float* xrow = A + (size_t)min(m0 + (wm * TM + i) * 16 + c, M - 1) * K;
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        for (int x = 0; x < 4; ++x) {
-          const float* wrow = W + (size_t)min(n0 + (wn * TN + j) * 16 + 4 * g + x, N - 1) * K;
-          float sum = 0.f;
-          for (int k = k_begin; k < k_end; ++k) sum = fmaf(xrow[k], wrow[k], sum);
-          acc[j][i][x] = sum;
-        }
+      for (int i = 0; i < TM; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k0 = k_begin; k0 < k_end; k0 += 16) {
+      const int k = k0 + 4 * g;
+      const bool whole = vec && k0 + 16 <= k_end;
+      floatx4 xf[TM], wf[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const float* row = A + (size_t)min(m0 + (wm * TM + i) * 16 + c, M - 1) * K;
+        xf[i] = whole ? *(const floatx4*)(row + k) : guarded(row, k);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const float* row = W + (size_t)min(n0 + (wn * TN + j) * 16 + c, N - 1) * K;
+        wf[j] = whole ? *(const floatx4*)(row + k) : guarded(row, k);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][e], xf[i][e], acc[j][i], 0, 0, 0);
     }
   }
   // lane (c, g) holds, of every 16 x 16 tile, output row m = c and the columns n = 4 g .. 4 g + 3

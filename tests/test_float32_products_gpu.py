@@ -62,3 +62,53 @@ def test_numbers_without_parts(ops, tile):
     fine = want.isfinite()
     limit = torch.where(fine, bound(x, w), torch.zeros(()).double())
     assert bool(((got - want).abs()[fine] <= limit[fine]).all())
+
+
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("m,n,k", [(70, 66, 40), (129, 130, 100), (65, 64, 33)])
+@pytest.mark.parametrize("size", [-100, -104, -107, -110, -111, -112, -116, -120, -124, -126, -140])
+def test_small_numbers(ops, tile, m, n, k, size):
+    """Numbers whose last bits lie under bfloat16's smallest (or that are below float32's smallest normal number), in
+    one row among ordinary ones, in a few places among zeros, and on the other side of the product."""
+    x, w = rnd((m, k), 7), rnd((n, k), 8) * 2.0 ** 90
+    x[3] *= 2.0 ** size
+    alone = torch.arange(m - 9, m)
+    x[alone] = 0
+    x[alone, alone % k] = rnd((9,), 11) * 2.0 ** size
+    for a, b in ((x, w), (w, x)):
+        want, limit = a.double() @ b.double().T, bound(a, b)
+        # (a product below float32's smallest normal number is a whole number of its steps, 2^-149)
+        limit = limit + a.shape[1] * 2.0 ** -149
+        one = (a != 0).sum(1, keepdim=True) * (b != 0).sum(1) < 2 * a.shape[1]      # (a product alone: no sum to round)
+        limit = torch.where(one, 4 * 2.0 ** -24 * want.abs() + 2.0 ** -149, limit)
+        out = torch.empty(a.shape[0], b.shape[0], device=DEV)
+        with ops.debug.force(gemm_tile=tile):
+            ops.linear_logits(a.to(DEV), b.to(DEV), out)
+            parts = torch.full((2, a.shape[0], b.shape[0]), float("nan"), device=DEV)
+            ops.linear_partials(a.to(DEV), b.to(DEV), parts, 2)
+        assert bool(((out.cpu().double() - want).abs() <= limit).all())
+        assert bool(((parts.cpu().double().sum(0) - want).abs() <= limit).all())
+
+
+@pytest.mark.parametrize("tile", [64, 128])
+def test_sums_that_overflow(ops, tile):
+    """Numbers that have parts and a product past the largest float32: infinite, not NaN; a product just below it,
+    whose leading parts' product is past it: finite."""
+    m, n, k = 70, 66, 40
+    x, w = rnd((m, k), 9), rnd((n, k), 10)
+    x[0], x[1], x[2] = 0, 0, 0
+    x[0, 5], w[:33, 5] = 1e38, 1003000.0
+    x[1, 6], w[7, 6] = 1e30, 1.0037e12
+    root = 2.0 ** 64 * (1 - 2.0 ** -10)          # (its leading part is 2^64)
+    x[2, 9], w[11, 9] = root, root
+    want = (x.double() @ w.double().T)
+    limit = bound(x, w)
+    want = torch.where(want.abs() >= 2.0 ** 128 * (1 - 2.0 ** -25), want.sign() * float("inf"), want)
+    assert bool(want[0, :33].isinf().all()) and bool(want[1, 7].isinf()) and bool(want[2, 11].isfinite())
+    out = torch.empty(m, n, device=DEV)
+    with ops.debug.force(gemm_tile=tile):
+        ops.linear_logits(x.to(DEV), w.to(DEV), out)
+    got = out.cpu().double()
+    fine = want.isfinite()
+    assert torch.equal(got[~fine], want[~fine])
+    assert bool(((got - want).abs()[fine] <= limit[fine]).all())
