@@ -142,6 +142,7 @@ template <>
 struct SkStep<bf16_t> {
   typedef bf16x8 frag;
   static constexpr int LEN = 32, PER = 8, SUMS = 1;
+  static constexpr bool KEEPS_INF = false;
   static __device__ __forceinline__ void mul(frag x, frag w, floatx4* acc, int) {
     acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, w, acc[0], 0, 0, 0);
   }
@@ -150,6 +151,7 @@ template <>
 struct SkStep<float> {
   typedef floatx4 frag;
   static constexpr int LEN = 16, PER = 4, SUMS = 16;
+  static constexpr bool KEEPS_INF = true;      // (a step past the end is zeros of both operands: an infinity of x met by a zero would be NaN)
   static __device__ __forceinline__ void mul(frag x, frag w, floatx4* acc, int step) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -486,7 +488,8 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       const Frag bu = st < s_end ? b[u] : zero;
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        const Frag av = *(const Frag*)(arow[mb] + min(st, steps - 1) * S::LEN);
+        Frag av = *(const Frag*)(arow[mb] + min(st, steps - 1) * S::LEN);
+        if constexpr (S::KEEPS_INF) av = st < s_end ? av : zero;
         S::mul(av, bu, acc[mb], u);
       }
     }
@@ -535,7 +538,11 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     for (int u = 0; u < R; ++u) {           // the last round drains it
       const Frag bu = s0 + u < s_end ? b[u] : zero;
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) S::mul(ab[u][mb], bu, acc[mb], u);
+      for (int mb = 0; mb < MB; ++mb) {
+        Frag av = ab[u][mb];
+        if constexpr (S::KEEPS_INF) av = s0 + u < s_end ? av : zero;
+        S::mul(av, bu, acc[mb], u);
+      }
     }
   }
 

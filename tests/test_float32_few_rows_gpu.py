@@ -99,3 +99,56 @@ def test_fused_norm_qkv(ops, m, d, nq, nkv):
         p, off = int(table[r, int(positions[r]) // page]), int(positions[r]) % page
         assert float((keys[p, :, off].double() - turned[r, nq:nq + nkv]).abs().max()) <= limit
         assert float((values[p, :, :, off].double() - y[r, nq + nkv:]).abs().max()) <= limit
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 16, 16), (5, 17, 896), (16, 100, 48), (17, 130, 160), (64, 31, 1600)])
+def test_infinities(ops, m, n, k):
+    """An infinity among the inputs gives an infinity, NaN gives NaN, in their rows alone: in every epilogue, whole
+    and in pieces, wherever in the row it lies (the last steps of a wave's share are filled up with zeros)."""
+    x, w = rnd((m, k), 15), rnd((n, k), 16)
+    x[0, k - 1], x[1, 0], x[2, k // 2] = float("inf"), -float("inf"), float("nan")
+    want = x.double() @ w.double().T
+    limit = (k + 16) * 2.0 ** -24 * (x[3:].double().abs() @ w.double().abs().T)
+    dx, dw = x.to(DEV), w.to(DEV)
+    for what in ("store", "logits", "stream", "pieces"):
+        out = torch.zeros(m, n, device=DEV)
+        if what == "store":
+            ops.linear(dx, dw, out)
+        elif what == "logits":
+            ops.linear_logits(dx, dw, out)
+        elif what == "stream":
+            ops.linear_residual(dx, dw, out)
+        else:
+            parts = torch.full((2, m, n), float("nan"), device=DEV)
+            ops.linear_partials(dx, dw, parts, 2)
+            out = parts.sum(0)
+        got = out.cpu().double()
+        assert torch.equal(got[:2], want[:2]) and bool(got[2].isnan().all()), what
+        assert bool(((got[3:] - want[3:]).abs() <= limit).all()), what
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "clamped"])
+@pytest.mark.parametrize("m,k,inter", [(3, 64, 20), (16, 96, 16), (21, 160, 48)])
+def test_pairs(ops, activation, m, k, inter):
+    """The three pairs of gate and up value, from far below zero to far above."""
+    x, gate, up = rnd((m, k), 17, 3.0), rnd((inter, k), 18, 0.5), rnd((inter, k), 19, 0.5)
+    out = torch.empty(m, inter, device=DEV)
+    constants = (7.0, 1.702, 1.0) if activation == "clamped" else None
+    assert ops.few_rows_take_float32(m, k)
+    ops.linear_swiglu(x.to(DEV), interleave_gate_up(gate, up).to(DEV), out, activation, constants)
+    g, u = x.double() @ gate.double().T, x.double() @ up.double().T
+    # the sums are off by e_g and e_u; |slope| of each activation is at most 1.2 (silu 1.1, tanh gelu 1.13, the clamped
+    # 1.1), its own evaluation a few units of the result, and the tanh form's 1 + tanh one unit of the gate's number where it cancels
+    unit = (k + 16) * 2.0 ** -24
+    e_g, e_u = (unit * (x.double().abs() @ t.double().abs().T) for t in (gate, up))
+    if activation == "clamped":
+        limit, slope, shift = constants
+        g = g.clamp(max=limit)
+        v = g * torch.sigmoid(slope * g)
+        u = u.clamp(-limit, limit) + shift
+    elif activation == "silu":
+        v = g * torch.sigmoid(g)
+    else:
+        v = 0.5 * g * (1 + torch.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3)))
+    bound = 1.2 * e_g * u.abs() + e_u * v.abs() + 2.0 ** -20 * (v * u).abs() + 2.0 ** -23 * (g * u).abs() + 1e-12
+    assert bool(((out.cpu().double() - v * u).abs() <= bound).all())
