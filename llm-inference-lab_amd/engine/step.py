@@ -184,6 +184,13 @@ class StepContext:
             self._views[(name, dtype, shape)] = view
         return view
 
+    def scratch_or_none(self, name: str, shape: Tuple[int, ...], dtype: torch.dtype) -> Optional[torch.Tensor]:
+        """The same for a buffer that a step can do without: None where no memory is left for it."""
+        try:
+            return self.scratch(name, shape, dtype)
+        except ScratchExhausted:
+            return None
+
     def _memory_available(self) -> Optional[int]:
         if torch.device(self.device).type != "cuda":
             return None

@@ -8,7 +8,7 @@ import torch
 
 from ..config.spec import PartSpec
 from ..weights.loader import TensorSpec, MATRIX, VECTOR, INIT_NORM
-from .base import Mixer, KVCacheSpec, CacheSpec, PageTensor, NormedInput, PendingSums, project_normed
+from .base import Mixer, KVCacheSpec, CacheSpec, PageTensor, NormedInput, PendingSums, pieces_buffer, project_normed
 from .registry import register_part, build_part
 
 
@@ -231,10 +231,10 @@ class GQAAttention(Mixer):
         splits = 1
         if getattr(ctx, "pending", 0) is None and ops.pieces_by_tiles(rows, self.hidden_size, self.q_size):
             splits = ops.split_count(rows, self.dtype, self.hidden_size, self.q_size)
-        if splits > 1:
+        parts = pieces_buffer(ctx, "attention.pieces", (splits, rows, self.hidden_size)) if splits > 1 else None
+        if parts is not None:
             # some rows of a large matrix: cut along the inner size, the pieces left for the
             # norm that reads the stream next
-            parts = ctx.scratch("attention.pieces", (splits, rows, self.hidden_size), torch.float32)
             ctx.pending = ops.linear_partials(out, self.w_o, parts, splits, self.b_o)
         else:
             ops.linear_residual(out, self.w_o, residual, self.b_o)

@@ -182,6 +182,12 @@ class PendingSums:
         self.parts, self.splits = parts, int(splits)
 
 
+def pieces_buffer(ctx, name: str, shape) -> Optional[torch.Tensor]:
+    """Scratch for a product left in pieces, or None where the step has no memory left for it: the product
+    is then taken whole, which needs none."""
+    return getattr(ctx, "scratch_or_none", ctx.scratch)(name, shape, torch.float32)
+
+
 class ChosenSums:
     """A result that is a weighted sum of experts' results, not summed yet: row ``r`` is ``sum_k weights[r, k] *
     rows[place_of[r, k], :]``, the choices in their order (a place below zero: none).  Whoever takes it sums it
@@ -303,8 +309,8 @@ class Mixer(Part):
         inner size, the pieces themselves (``PendingSums``; ``out`` is not written)."""
         rows, width = out.shape
         splits = self.ops.split_count(rows, self.dtype, width, x.shape[1])
-        if splits > 1:
-            parts = ctx.scratch("mixer.pieces", (splits, rows, width), torch.float32)
+        parts = pieces_buffer(ctx, "mixer.pieces", (splits, rows, width)) if splits > 1 else None
+        if parts is not None:
             return self.ops.linear_partials(x, w, parts, splits)
         self.ops.linear_logits(x, w, out)
         return None

@@ -6,7 +6,7 @@ from typing import Dict
 import torch
 
 from ..weights.loader import TensorSpec, MATRIX, VECTOR, INIT_NORM
-from .base import FeedForward, NormedInput
+from .base import FeedForward, NormedInput, pieces_buffer
 from .registry import register_part
 
 PAIR = 16   # rows of the gate matrix and of the up matrix alternate in runs of 16
@@ -110,8 +110,8 @@ class SwiGLU(FeedForward):
         act = ctx.scratch("swiglu.act", (rows, self.kernel_size), self.dtype)
         self.ops.linear_swiglu(h, self.w_gate_up, act, *self._act())
         splits = self.ops.split_count(rows, self.dtype, self.hidden_size, self.kernel_size)
-        if splits > 1:
-            parts = ctx.scratch("swiglu.pieces", (splits, rows, self.hidden_size), torch.float32)
+        parts = pieces_buffer(ctx, "swiglu.pieces", (splits, rows, self.hidden_size)) if splits > 1 else None
+        if parts is not None:
             return self.ops.linear_partials(act, self.w_down, parts, splits)
         self.ops.linear_logits(act, self.w_down, out)
         return None
@@ -129,10 +129,12 @@ class SwiGLU(FeedForward):
                 h = h.tensor()
             self.ops.linear_swiglu(h, self.w_gate_up, act, *self._act())
         splits = self.ops.split_count(rows, self.dtype, self.hidden_size, self.kernel_size)
+        parts = None
         if splits > 1 and hasattr(ctx, "pending") and ctx.pending is None:
             # a narrow output: the product is cut along the inner size so that it spreads
             # over the chip, and its pieces are left for the next reader of the stream
-            parts = ctx.scratch("swiglu.pieces", (splits, rows, self.hidden_size), torch.float32)
+            parts = pieces_buffer(ctx, "swiglu.pieces", (splits, rows, self.hidden_size))
+        if parts is not None:
             ctx.pending = self.ops.linear_partials(act, self.w_down, parts, splits)
         else:
             self.ops.linear_residual(act, self.w_down, residual, None)
@@ -206,8 +208,8 @@ class DenseFeedForward(FeedForward):
             h = h.tensor()
         rows, act = h.shape[0], self._activated(h, ctx)
         splits = self.ops.split_count(rows, self.dtype, self.hidden_size, self.kernel_size)
-        if splits > 1:
-            parts = ctx.scratch("dense_ffn.pieces", (splits, rows, self.hidden_size), torch.float32)
+        parts = pieces_buffer(ctx, "dense_ffn.pieces", (splits, rows, self.hidden_size)) if splits > 1 else None
+        if parts is not None:
             return self.ops.linear_partials(act, self.w_down, parts, splits)
         self.ops.linear_logits(act, self.w_down, out)
         return None

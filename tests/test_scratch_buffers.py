@@ -50,3 +50,26 @@ def test_a_buffer_that_grows_moves(monkeypatch):
             ctx.scratch("a", (16, 4), torch.float32)
     assert ctx.scratch_version == before + 2          # (the old one has been given back: nothing may still point at it)
     assert ctx.scratch("a", (8, 4), torch.float32).shape == (8, 4)
+
+
+@pytest.mark.parametrize("backend", ["emu", pytest.param("hip", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("design,name", [("vivevik", "P"), ("qwen2", "B")])
+def test_no_memory_left_for_pieces(backend, dtype, design, name):
+    """A step that fits while its products are taken whole still runs when the rules would cut them and nothing
+    is left for the pieces: the same bits as whole."""
+    cases = V if design == "vivevik" else H
+    kw = dict(ops=EmuOps(), device="cpu") if backend == "emu" else {}
+    engine = cases.make_engine(name, 1, dtype, **kw)
+    ids = cases.random_ids(cases.config_of(name), 21, 3)
+    outs = []
+    for least in (10 ** 6, 1):
+        engine.ops.rules.min_steps_per_split = least
+        request = engine.open(least)
+        outs.append([engine.step([H.lab.StepEntry(request, ids[:20], [19])]).clone(),
+                     engine.step([H.lab.StepEntry(request, ids[20:], [0])]).clone()])
+        engine.close(request)
+        engine.step_fn.ctx._memory_available = lambda: 0
+    made = engine.step_fn.ctx.scratch_allocations
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    assert engine.step_fn.ctx.scratch_allocations == made
