@@ -825,7 +825,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // up a bit of the operands.  A float32 number of 2^-110 to 3.39e38 is the sum of three bfloat16 numbers, x = h + m + l (h =
 // x rounded to nearest, m = x - h rounded, l the rest: 24 bits of significand in three times 8, the
 // differences exact), and x w = h_x h_w + h_x m_w + m_x h_w + m_x m_w + h_x l_w + l_x h_w up to terms below
-// 2^-24 of |x w|, less than what one rounding of a 32-bit sum costs.  Every bfloat16 product is
+// 2^-24 of |x w|, less than what one rounding of a 32-bit sum costs (three of the nine part products are left out: about
+// 2^-26 of a product, so that a product by itself is within two roundings, not one).  Every bfloat16 product is
 // exact in float32 and the sums are float32; an instruction adds 32 of them where
 // v_mfma_f32_32x32x2_f32 adds 2, so fewer roundings meet in a sum (relative error of a product of
 // normal numbers against 64 bits: inner size 896 4.5e-7, 5.4e-7 with the float32 instructions; 4,864 1.1e-6
@@ -1373,11 +1374,14 @@ extern "C" void llmlab_debug_gemm_tile(int tile) {
 // share at the same rate, and what matters is that all of them draw until the end: one round of
 // blocks that nearly fills the chip, each wave with 32 columns of its own.  The width that does that,
 // 32 times 3, 4, 5 or 7, is the narrowest whose blocks find a unit each (-1: none does, or the round would
-// leave a fifth of the units, of the narrowest tile three tenths, without a block).  Inner sizes from 1,536 up,
-// measured against the best of the other tiles / the estimates' pick: 64 rows of 37888 x 3584 (160 columns,
+// leave a fifth of the units, of the narrowest tile three tenths, without a block).
+// Measured against the best of the other tiles / the estimates' pick: 64 rows of 37888 x 3584 (160 columns,
 // 237 blocks) 57 us against 70 / 70, of 22016 x 2048 (96, 230) 26.2 / 27.2 / 27.8, of 17920 x 1536 (96, 187)
 // 19.6 / 20.9 / 22.9, of 27648 x 5120 (128, 216) 62 / 62 / 69, of 55296 x 5120 (224, 247) 105 / 109 / 109; 17 rows
-// the same; 128 rows of 37888 x 3584 in one tile of rows (160) 70 / 78 / 79, of 17920 x 1536 in two (2 x 112
+// the same.  Short inner sizes: 17 / 64 rows of 24448 x 1024 (96) 15.3 / 16.8 against 15.9 / 16.8 by the estimates, of
+// 37888 x 1024 (160) 20.3 / 21.8 against 21.6 / 24.2; 128 columns lose at 1,024 (28672: 16.9 / 18.4 against 16.2 / 17.3)
+// and not at 1,152 (18.6 / 19.9 and 18.8 / 20.9); 224 lose until 2,048 (49152 x 1152: 26.9 / 28.5 against 25.3 / 28.5, x
+// 2048: 40.3 / 42.2 and 38.7 / 42.5) and not at 3,072 (56.1 / 60.7 and 56.8 / 62.5).  128 rows of 37888 x 3584 in one tile of rows (160) 70 / 78 / 79, of 17920 x 1536 in two (2 x 112
 // blocks) 23.9 / 27.1 / 27.3.
 static int one_round_tile(int M, int N, int K, int num_cus) {
   if (M > 128 || K < 1024) return -1;
@@ -1390,9 +1394,9 @@ static int one_round_tile(int M, int N, int K, int num_cus) {
     return fills(160, 2, 0.8) ? TILE_64x160 : -1;
   }
   if (fills(96, 1, 0.7)) return TILE_64x96;
-  if (fills(128, 1, 0.8)) return TILE_64x128;
+  if (K >= 1152 && fills(128, 1, 0.8)) return TILE_64x128;
   if (fills(160, 1, 0.8)) return TILE_64x160;
-  return fills(224, 1, 0.8) ? TILE_64x224 : -1;
+  return K >= 3072 && fills(224, 1, 0.8) ? TILE_64x224 : -1;
 }
 
 // By an estimate of the time, fitted to a sweep of seven matrices of two model shapes at 65 to 4,000 rows
@@ -1444,7 +1448,7 @@ static int choose_tile(int M, int N, int K, int num_cus) {
   const long wide = (N + 127) / 128;
   if (M <= 64 && wide >= num_cus) return TILE_64x128;
   // ... and of a matrix of 32,768 to 65,536 rows the 128 x 256 tile (96 / 128 rows of 37888 x
-  // 3584: 81 / 77 us against 83 / 84; of 59136 x 8192: 195 / 201 against 200 / 209; a decode
+  // 3584: 81 / 77 us against 83 / 84, and 70 in the one round of one_round_tile, which whole products ask first; of 59136 x 8192: 195 / 201 against 200 / 209; a decode
   // step of 128 requests of the 7B shape 6.99 -> 6.86 ms, of the 32B shape 24.8 -> 24.4; a
   // vocabulary of 152,064 gains nothing from it)
   if (M > 64 && M <= 128 && N >= 32768 && N <= 65536 && K >= 1024 && !g_without_wide) return TILE_128x256;

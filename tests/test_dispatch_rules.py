@@ -92,13 +92,49 @@ def test_measured_decisions(core, m, n, k, want):
 
 
 def test_one_tile_of_rows_of_a_wide_matrix(core):
-    """65 to 128 rows: the tile of a product that does not add into the stream (gate and up, the
-    logits), measured inside decode steps of 96 and 128 requests."""
+    """Up to 128 rows: the tile that the estimates pick, measured inside decode steps of 96 and 128 requests.  (A
+    product that is neither cut nor written by heads follows it only where no width makes one round of blocks:
+    ``test_one_round_of_blocks``.)"""
     assert core.llmlab_linear_tile(128, 37888, 3584, CUS) == 256      # 128 x 256: 77 us against 84
     assert core.llmlab_linear_tile(96, 55296, 5120, CUS) == 256
     assert core.llmlab_linear_tile(128, 152064, 3584, CUS) == 128     # a vocabulary gains nothing from it
     assert core.llmlab_linear_tile(128, 27648, 5120, CUS) == 128
     assert core.llmlab_linear_tile(64, 37888, 3584, CUS) == 128       # (64 x 128)
+
+
+@pytest.mark.parametrize("m,n,k,columns", [
+    # (measured: see the comment at the rule in csrc/gemm.hip)
+    (64, 37888, 3584, 160), (17, 37888, 3584, 160), (64, 22016, 2048, 96), (64, 17920, 1536, 96),
+    (64, 27648, 5120, 128), (64, 55296, 5120, 224), (128, 37888, 3584, 160), (128, 17920, 1536, 160),
+    # 128 columns from an inner size of 1,152 on, 224 from 3,072 on (below, the estimates' picks are faster)
+    (17, 28672, 1152, 128), (17, 28672, 1024, 64), (32, 49152, 3072, 224), (32, 49152, 2048, 128), (17, 24448, 1024, 96),
+    # no width makes a round: what the estimates pick
+    (128, 55296, 5120, 256), (128, 152064, 3584, 128), (64, 152064, 3584, 128), (64, 4608, 3584, 64),
+])
+def test_one_round_of_blocks(core, m, n, k, columns):
+    """The tile of gate and up, of logits and of other whole products of up to 128 rows."""
+    assert core.llmlab_plain_tile(m, n, k, CUS) == columns
+
+
+def test_one_round_of_blocks_is_one_round(core):
+    """Over sizes drawn at random: where the tile is not the one that the estimates pick, its blocks find a compute unit
+    each and leave few without one; beyond 128 rows and at short inner sizes it is the estimates' always."""
+    rng = random.Random(7)
+    differs = 0
+    for _ in range(5000):
+        m = rng.choice([rng.randint(17, 64), rng.randint(65, 128), rng.randint(129, 3000)])
+        n, k = rng.randint(64, 70000), 8 * rng.randint(16, 1500)
+        cus = rng.choice([CUS, 304, 64])
+        columns, estimates = core.llmlab_plain_tile(m, n, k, cus), core.llmlab_linear_tile(m, n, k, cus)
+        if m > 128 or k < 1024:
+            assert columns == estimates, (m, n, k)
+        if columns == estimates:
+            continue
+        differs += 1
+        assert columns in ((96, 128, 160, 224) if m <= 64 else (160,)), (m, n, k)
+        rounds = [(n + columns - 1) // columns * tiles / cus for tiles in ((1,) if m <= 64 else (1, 2))]
+        assert any((0.7 if columns == 96 else 0.8) <= r <= 1.0 for r in rounds), (m, n, k, columns)
+    assert differs > 300
 
 
 def test_block_shapes_of_products_of_few_rows(core):

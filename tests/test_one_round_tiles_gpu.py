@@ -51,7 +51,7 @@ def test_epilogues(ops, tile, m, n, k):
                      <= 1.1 * sums(gate) * u.abs() + sums(up) * g.abs() + full.abs() / 128 + 1e-6).all())
 
 
-@pytest.mark.parametrize("m,n,k,columns", [(17, 24448, 1024, 96), (64, 37888, 1024, 160), (40, 49000, 1024, 224),
+@pytest.mark.parametrize("m,n,k,columns", [(17, 24448, 1024, 96), (64, 37888, 1024, 160), (40, 49000, 3072, 224),
                                            (65, 37888, 1024, 160), (128, 17920, 1024, 160), (64, 152064, 1024, 128)])
 def test_one_round_of_blocks(ops, m, n, k, columns):
     """The chosen width, and one product by it against the same product by another tile."""
