@@ -1309,10 +1309,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
 // one key/value head (16 at a time) and one of `splits` shares of the row's key tiles, so that
 // few rows still fill the chip.  With one share the result is final; else the share's
 // maximum, denominator and unnormalised sum go to part_ml / part_o for the merge kernel.
-// The sink enters the first share only.  How a row's keys are cut follows from the row alone (two tiles a share
-// at least, `most_shares` at most), not from `splits`, which holds for the step's longest row: a step
-// replayed from a graph has shares for a longer one (the others weigh zero in the merge, exactly), and sums the
-// same numbers in the same order.
+// The sink enters the first share only.  How a row's keys are cut follows from the row's length and from `most_shares`
+// (two tiles a share at least, so many shares at most: by the number of rows of the launch, the compute units and
+// the scratch), not from the longest history that the step announces, which `splits` holds for: a step replayed from
+// a graph has shares for a longer one (the others weigh zero in the merge, exactly), and sums the same numbers in
+// the same order.  Beside another number of rows a row may be cut otherwise.
 template <int DC, int EB>
 __global__ __launch_bounds__(64) void sink_window_attention_grouped_kernel(MfmaArgs a) {
   constexpr int D = 32 * DC, E = 16 * EB;

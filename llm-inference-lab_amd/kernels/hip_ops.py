@@ -739,7 +739,9 @@ class HipOps:
         want = self.num_cus // max(strips, 1)
         if dtype == torch.float32 and rows > self.split_max_rows:
             # (the pieces of so many rows are folded by the norm, more of them cost the next product nothing: 48 / 64
-            # rows of 1536 x 8960 46 / 55 us in eight, 58 / 58 in two, 71 / 71 whole)
+            # rows of 1536 x 8960, the norm behind it included, 50 / 58 us in eight, 62 / 61 in two, 73 / 74 whole; of 2048 x
+            # 11008 in eight 85 / 90 against 93 / 92 whole, 78 / 93 in two; of 3584 x 18944 217 / 243 against 217 / 285; of
+            # 896 x 4864 in four 23 / 27 against 26 / 26)
             want = max(want, k // 1120)
         return max(1, min(want, most))
 

@@ -1,5 +1,6 @@
-"""The shares that a decoding row's keys are cut into follow from the row alone: a step that is told of longer
-histories (as one replayed from a graph is) gives the same bits."""
+"""The shares that a decoding row's keys are cut into follow from the row and the number of rows of the launch, not
+from the longest history announced: a step that is told of longer ones (as one replayed from a graph is) gives the
+same bits."""
 import pytest
 import torch
 
