@@ -1394,7 +1394,7 @@ static int one_round_tile(int M, int N, int K, int num_cus) {
     return fills(160, 2, 0.8) ? TILE_64x160 : -1;
   }
   if (fills(96, 1, 0.7)) return TILE_64x96;
-  if (K >= 1152 && fills(128, 1, 0.8)) return TILE_64x128;
+  if (fills(128, 1, 0.8)) return K >= 1152 ? TILE_64x128 : -1;
   if (fills(160, 1, 0.8)) return TILE_64x160;
   return K >= 3072 && fills(224, 1, 0.8) ? TILE_64x224 : -1;
 }

@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import collections
 import dataclasses
+import math
 import time
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -185,7 +186,15 @@ class StepContext:
         return view
 
     def scratch_or_none(self, name: str, shape: Tuple[int, ...], dtype: torch.dtype) -> Optional[torch.Tensor]:
-        """The same for a buffer that a step can do without: None where no memory is left for it."""
+        """The same for a buffer that a step can do without: None where no memory is left for it (or where it would
+        be made while a graph is captured: the eager step before has gone without it, and so does the graph)."""
+        hit = self._views.get((name, dtype, shape))
+        if hit is not None:
+            return hit
+        buf = self._scratch.get((name, dtype))
+        if ((buf is None or buf.numel() < math.prod(shape)) and torch.device(self.device).type == "cuda"
+                and torch.cuda.is_current_stream_capturing()):
+            return None
         try:
             return self.scratch(name, shape, dtype)
         except ScratchExhausted:

@@ -73,3 +73,31 @@ def test_no_memory_left_for_pieces(backend, dtype, design, name):
     made = engine.step_fn.ctx.scratch_allocations
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
     assert engine.step_fn.ctx.scratch_allocations == made
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_no_memory_left_for_pieces_under_capture(dtype):
+    """Memory that turns up while a graph is captured makes no buffer inside it: the graph does what the eager
+    step before it did, at every replay."""
+    runs = []
+    for graph in (False, True):
+        engine = V.make_engine("P", 1, dtype, graph=graph)
+        ids = V.random_ids(V.config_of("P"), 40, 5)
+        engine.ops.rules.min_steps_per_split = 10 ** 6
+        requests = [engine.open(i) for i in range(3)]
+        engine.step([H.lab.StepEntry(r, ids[:20 + i], [19]) for i, r in enumerate(requests)])
+        engine.step([H.lab.StepEntry(r, [ids[29]], [0]) for r in requests])
+        ctx = engine.step_fn.ctx
+        if graph:
+            engine.ops.rules.min_steps_per_split = 1
+            ctx._memory_available = lambda: (1 << 40) if torch.cuda.is_current_stream_capturing() else 0
+        outs = []
+        for i in range(6):
+            outs.append(engine.step([H.lab.StepEntry(r, [ids[30 + i]], [0]) for r in requests]).clone())
+            torch.cuda.synchronize()
+        if graph:
+            assert engine.step_fn.graph_captures > 0 and engine.step_fn.graph_replays > 0
+            assert not any(name.endswith(".pieces") for name, _ in ctx._scratch)
+        runs.append(outs)
+    assert all(torch.equal(a, b) for a, b in zip(*runs))
