@@ -165,7 +165,7 @@ class StepContext:
         if buf is None or buf.numel() < count:
             width = torch.empty((), dtype=dtype).element_size()
             need = max(count, 1) * width
-            have = self._memory_available()
+            have = self._memory_available(need)
             if have is not None and need > have:
                 raise ScratchExhausted(f"scratch buffer '{name}' needs {need} bytes; {have} bytes are "
                                        f"available after the weights and the cache")
@@ -200,10 +200,14 @@ class StepContext:
         except ScratchExhausted:
             return None
 
-    def _memory_available(self) -> Optional[int]:
+    def _memory_available(self, enough: int) -> Optional[int]:
+        """Bytes that a new buffer could take (``enough`` or more if there are so many, without asking the
+        allocator, whose statistics cost six times what the question to the GPU does)."""
         if torch.device(self.device).type != "cuda":
             return None
         free, _ = torch.cuda.mem_get_info(self.device)
+        if free >= enough:
+            return int(free)
         stats = torch.cuda.memory_stats(self.device)
         reusable = stats.get("reserved_bytes.all.current", 0) - stats.get("allocated_bytes.all.current", 0)
         return int(free) + max(0, int(reusable))

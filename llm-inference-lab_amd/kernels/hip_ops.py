@@ -1098,13 +1098,21 @@ class HipOps:
         if isinstance(y, PendingSums):
             if y.parts.dim() != 3 or not 1 <= y.splits <= y.parts.shape[0]:
                 raise ValueError(f"layernorm_add: {y.splits} pieces of {tuple(y.parts.shape)}")
-            splits, stride, y = y.splits, y.parts.stride(0), y.parts[0]
-        self._need(y, "sublayer output", torch.float32)
+            splits, y = y.splits, y.parts
+            stride = y.stride(0)
+            # (the first piece's rows follow each other, so do the others'; a slice of it costs 3 us a call)
+            self._need(y, "sublayer output", torch.float32, contiguous=False)
+            if (y.stride(1) != y.shape[2] and y.shape[1] > 1) or (y.stride(2) != 1 and y.shape[2] > 1):
+                raise ValueError("sublayer output must be contiguous")
+            shape = tuple(y.shape[1:])
+        else:
+            self._need(y, "sublayer output", torch.float32)
+            shape = tuple(y.shape)
         self._need(resid, "residual stream", torch.float32)
         self._need(weight, "norm weight")
         rows, hidden = resid.shape
-        if tuple(y.shape) != (rows, hidden) or weight.numel() != hidden or y.data_ptr() == resid.data_ptr():
-            raise ValueError(f"layernorm_add: y {tuple(y.shape)}, weight {tuple(weight.shape)}, stream "
+        if shape != (rows, hidden) or weight.numel() != hidden or y.data_ptr() == resid.data_ptr():
+            raise ValueError(f"layernorm_add: y {shape}, weight {tuple(weight.shape)}, stream "
                              f"{tuple(resid.shape)} do not fit (and are two buffers)")
         if copy is not None:
             self._need(copy, "copy of the stream")

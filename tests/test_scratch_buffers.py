@@ -69,7 +69,7 @@ def test_no_memory_left_for_pieces(backend, dtype, design, name):
         outs.append([engine.step([H.lab.StepEntry(request, ids[:20], [19])]).clone(),
                      engine.step([H.lab.StepEntry(request, ids[20:], [0])]).clone()])
         engine.close(request)
-        engine.step_fn.ctx._memory_available = lambda: 0
+        engine.step_fn.ctx._memory_available = lambda enough: 0
     made = engine.step_fn.ctx.scratch_allocations
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
     assert engine.step_fn.ctx.scratch_allocations == made
@@ -91,7 +91,7 @@ def test_no_memory_left_for_pieces_under_capture(dtype):
         ctx = engine.step_fn.ctx
         if graph:
             engine.ops.rules.min_steps_per_split = 1
-            ctx._memory_available = lambda: (1 << 40) if torch.cuda.is_current_stream_capturing() else 0
+            ctx._memory_available = lambda enough: (1 << 40) if torch.cuda.is_current_stream_capturing() else 0
         outs = []
         for i in range(6):
             outs.append(engine.step([H.lab.StepEntry(r, [ids[30 + i]], [0]) for r in requests]).clone())
