@@ -832,8 +832,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // normal numbers against 64 bits: inner size 896 4.5e-7, 5.4e-7 with the float32 instructions; 4,864 1.1e-6
 // and 1.25e-6, 6e-7 in three pieces).  Six instructions at 16 times the rate of the float32 ones, measured
 // against tiles of v_mfma_f32_32x32x2_f32 (which this replaces; 157 TFLOP/s is what those could reach): 1,531
-// rows of 9728 x 896 186 us against 266 (144 TFLOP/s of 32-bit products), of 896 x 4864 in three pieces 81
-// against 215, 4,000 rows of 17920 x 1536 1,348 against 1,831, 65 rows of 1536 x 8960 48 in eight pieces against 252.
+// rows of 9728 x 896 181 us against 266 (147 TFLOP/s of 32-bit products), of 896 x 4864 in three pieces 82
+// against 215, 4,000 rows of 17920 x 1536 1,305 against 1,831, 65 rows of 1536 x 8960 42 in eight pieces against 252.
 // What bounds it: in full rounds the power limit (0.98 PFLOP/s of bfloat16 products), in a round by itself
 // a step's trip through LDS (1.3 us where its matrix instructions need 0.7).
 //
@@ -852,7 +852,9 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // part is rounded from, whose lower half is not zero.  And numbers that bfloat16 rounds to infinity (3.396e38 and above,
 // infinity itself), like products of parts that overflow where the whole product does not, or overflow with both
 // signs, leave an output that is not finite.  A block that meets either takes its outputs again on
-// v_mfma_f32_16x16x4_f32, operands straight from memory: true 32-bit products over the whole range.
+// v_mfma_f32_16x16x4_f32, operands straight from memory: true 32-bit products over the whole range (1,531 rows of 9728 x
+// 896 with such a number in every block 654 us).  (The split is the one of Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 artificial intelligence datatype for higher-precision computations", 2019.)
 template <int EPI, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const float* __restrict__ A,
                                                                 const float* __restrict__ W, EpiArgs e, int M,
