@@ -28,7 +28,7 @@
 //     * the largest products (from 1024 rows on, where its blocks fill the chip): a 256x256
 //       tile whose eight waves form two groups that alternate between reading LDS and
 //       issuing MFMAs, both operands loaded from global memory straight into LDS
-//       (gemm_bf16_pingpong): 1.1 to 1.17 PF/s where the tiles above reach 0.9 to 0.97.
+//       (gemm_bf16_pingpong): 1.1 to 1.25 PF/s where the tiles above reach 0.9 to 0.97.
 //     (products of few rows, as in decode steps, have kernels of their own in decode.hip)
 //   float32: numbers split into three bfloat16 parts for the matrix cores, 32-bit products and sums
 //     as exact as plain FMAs (gemm_f32_split_kernel); a plain FMA kernel beside it as its
@@ -530,19 +530,31 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
 
 // ============================================================ bf16, 256 x 256 by two groups of waves
 // The largest products.  Eight waves, each with a 128 x 64 part of a 256 x 256 tile; both
-// operands come by direct loads from global memory into LDS (no registers in between), in
-// steps of 32 of the inner size, four stages of 32 KB.  The lanes of a load address the
-// 16-byte pieces of one MFMA fragment (16 rows of x, or one 1 KB tile of the packed W), which
-// the hardware lays down lane after lane: LDS holds fragments, and a fragment read is 1 KB
-// of consecutive bytes.  The waves form two groups with a wave on every SIMD each, half a
-// step apart: between two barriers one group reads its twelve fragments and issues its
+// operands come by direct loads from global memory into LDS (no registers in between).  The
+// waves form two groups with a wave on every SIMD each, half a step (32 of the inner size)
+// apart: between two barriers one group reads its twelve fragments and issues its
 // loads while the other issues its 32 MFMAs, then they change roles, so that the reads of
 // LDS and the matrix instructions of a compute unit overlap by construction and not by
 // the luck of the scheduler (all eight waves in step: 975 TF/s on 8192 x 37888 x 3584,
-// the groups apart: 1065; the 128 x 256 tile of the kernel above: 966).  Under this load
-// the chip holds 1.45 to 1.85 GHz, and a step takes 1340 clocks where the MFMAs alone
-// need 1024.  A block fills a compute unit; the epilogue takes the two halves of the rows
-// through LDS one after the other.
+// the groups apart: 1065; the 128 x 256 tile of the kernel above: 966).  A block fills a
+// compute unit; the epilogue takes the two halves of the rows through LDS one after the other.
+//
+// What bounds it is the way of x to the compute units, line by line: with 1 KB of consecutive
+// memory a load in place of rows the same loop is 20 % faster.  W has such tiles (packed:
+// one load, one fragment, in a ring of four steps).  A load of x takes 8 rows of 128 bytes, two
+// steps of the inner size, neighbouring lanes in the same row, so that a load touches eight lines
+// and takes them whole; with one fragment a load (16 rows of 64 bytes, neighbouring lanes in
+// different rows) it touched 64 half lines, and 2367 rows of 37888 x 3584 took 597 us instead of 522,
+// of 3584 x 18944 322 instead of 286, 2048 of 22016 x 2048 191 instead of 169, of 3584 x 18944
+// 317 instead of 273 (16 rows of 64 bytes with neighbouring lanes in one row: 539, 280, 178, 319).
+// A piece of x is half of the tile's rows of two steps: NG of them in a ring, one fetched a step,
+// each by the step NG - 2 later at the latest.  Six make the 256 x 256 tile's LDS full; the tile
+// that writes the cache needs room for positions and biases and has five.
+// In LDS a row of a load lies as 128 bytes, its eight pieces of 16 bytes exchanged by the row's
+// number: a fragment read, 16 rows of one piece each, then meets every bank once.
+// A ring of five or six steps of W instead of four, or blocks that begin at different steps of the
+// inner size (to spread the channels of memory), change nothing; four waves of 128 x 128, whose
+// fragments for the next step are read between this one's MFMAs, are as fast and no faster.
 //
 // The direct loads are written in assembly: the compiler then knows nothing of them, the
 // waits (vmcnt) are placed by hand, and the loop holds no other load that it would count.
@@ -556,11 +568,12 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   static_assert(BM == 256 || BM == 192, "a wave has 128 or 96 rows");
   constexpr int BN = 256, NT = 512, HALF = 128;
   constexpr int TM = BM / 32;                           // blocks of 16 rows of a wave
-  constexpr int XF = BM / 16;                           // fragments of x in a step
-  constexpr int STAGE = (XF + BN / 16) * 1024;          // bytes: the fragments of x, then 16 of W
+  constexpr int NG = BM == 256 && EPI == EPI_QKV ? 5 : 6;      // pieces of x in LDS
+  constexpr int PIECE = BM / 2 * 128;                   // bytes: half of the rows, two steps
+  constexpr int W_AT = NG * PIECE, W_STEP = (BN / 16) * 1024;
   constexpr int C_STRIDE = BN + 4;
   constexpr size_t C_BYTES = (size_t)HALF * C_STRIDE * sizeof(float);
-  __shared__ __attribute__((aligned(1024))) char smem[C_BYTES > 4 * STAGE ? C_BYTES : 4 * STAGE];
+  __shared__ __attribute__((aligned(1024))) char smem[C_BYTES > W_AT + 4 * W_STEP ? C_BYTES : W_AT + 4 * W_STEP];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2;                             // waves 0-3 and 4-7: one of each on every SIMD
@@ -593,33 +606,39 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
       s_bias[i] = (e.bias && n0 + i < N) ? load_vec(e.bias, e.bias_bf16, n0 + i) : 0.f;
   }
 
-  // Per step a wave fetches four fragments (three of x with BM = 192): the even waves of x,
-  // the odd ones of W (so that both groups fetch both).  Rows past M, strips past N and pieces past K read a
-  // valid piece instead: they land in rows and columns that nobody stores, or meet the
+  // Per step a wave fetches four times 1 KB (three times of x with BM = 192): the even waves of x,
+  // the odd ones of W (so that both groups fetch both).  Rows past M, strips past N and numbers past K read a
+  // valid place instead: they land in rows and columns that nobody stores, or meet the
   // zeros of the padded W.
   const int T = (K + 31) >> 5, nstrips = (N + 15) >> 4;
   const bool fetches_x = (wave & 1) == 0;
   const int quarter = wave >> 1;
-  constexpr int NFX = XF / 4;                           // fragments of x that one of its four waves fetches
-  const bf16_t* src[4];
+  constexpr int NFX = BM / 64;                          // loads of a piece of x by each of its four waves
+  unsigned off[2][4];                                   // bytes from the tile's rows of x (by half) or of W
+  int shift[4];                                         // (of x) the numbers of k that `off` holds
   unsigned dst[4];
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     if (fetches_x) {
-      const int f = min(quarter * NFX + i, XF - 1);
-      src[i] = A + (size_t)min(m0 + f * 16 + c, M - 1) * K;
-      dst[i] = lds0 + f * 1024;
+      const int b = min(quarter * NFX + i, BM / 16 - 1);
+      shift[i] = ((lane & 7) ^ (((b & 1) << 2) | (lane >> 4))) * 8;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        off[h][i] = ((unsigned)(min(m0 + h * (BM / 2) + b * 8 + (lane >> 3), M - 1) - m0) * (unsigned)K + shift[i]) * 2u;
+      dst[i] = lds0 + b * 1024;
     } else {
       const int f = quarter * 4 + i;
-      src[i] = W + (size_t)min((n0 >> 4) + f, nstrips - 1) * T * 512 + lane * 8;
-      dst[i] = lds0 + (XF + f) * 1024;
+      off[0][i] = (unsigned)(min((n0 >> 4) + f, nstrips - 1) - (n0 >> 4)) * (unsigned)T * 1024u + lane * 16u;
+      dst[i] = lds0 + W_AT + f * 1024;
     }
   }
-  auto load_to_lds = [&](const bf16_t* from, unsigned to) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+  const char* const xbase = (const char*)(A + (size_t)m0 * K);
+  const char* const wbase = (const char*)(W + (size_t)(n0 >> 4) * T * 512);
+  auto load_to_lds = [&](unsigned at, const char* base, unsigned to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
-                 : "v"(from), "s"(to)
+                 : "v"(at), "s"(base), "s"(to)
                  : "memory", "m0");
   };
   // this block's steps: all of them, or (PART) its group's share of the inner size from
@@ -631,22 +650,31 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
     e.out = (float*)e.out + (size_t)blockIdx.z * e.part_stride;
     if (blockIdx.z > 0) e.bias = nullptr;
   }
-  auto fetch = [&](int stage, int step) {
-    const int t = min(first + step, T - 1);
-    if (fetches_x) {
-      const size_t off = (size_t)min(t * 32 + g * 8, K - 8);
+  // piece q of x: half q % 2 (given as a constant) of the rows, steps q and q + 1 of an even q
+  auto fetch_x = [&](int q, int half, unsigned slot) {
+    const int k = (first + (q & ~1)) * 32;
+    if (k + 64 <= K) {
+      const char* base = xbase + (size_t)k * 2;
 #pragma unroll
-      for (int i = 0; i < NFX; ++i) load_to_lds(src[i] + off, dst[i] + stage * STAGE);
+      for (int i = 0; i < NFX; ++i) load_to_lds(off[half][i], base, dst[i] + slot);
     } else {
-      const size_t off = (size_t)t * 512;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) load_to_lds(src[i] + off, dst[i] + stage * STAGE);
+      for (int i = 0; i < NFX; ++i)
+        load_to_lds(off[half][i] + (unsigned)(min(k + shift[i], K - 8) - shift[i]) * 2u, xbase, dst[i] + slot);
     }
   };
-  // lgkmcnt(0) and vmcnt(the loads of two steps): what a wave waits for before a barrier
-  auto wait_all_but_two_steps = [&]() {
-    if (NFX == 4 || !fetches_x) __builtin_amdgcn_s_waitcnt(0x0070 | 8);
-    else __builtin_amdgcn_s_waitcnt(0x0070 | (2 * NFX));
+  auto fetch_w = [&](int stage, int step) {
+    const char* base = wbase + (size_t)min(first + step, T - 1) * 1024;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_to_lds(off[0][i], base, dst[i] + stage * W_STEP);
+  };
+  // What a wave waits for before a barrier: its reads of LDS, and of its loads those that the next
+  // step reads: of W all but two steps; of x, before an even step, all but the pieces
+  // after that step's two (an odd step reads the same pieces as the step before).
+  auto wait_loads = [&](bool even_next) {
+    if (!fetches_x) __builtin_amdgcn_s_waitcnt(0x0070 | 8);
+    else if (even_next) __builtin_amdgcn_s_waitcnt(0x0070 | ((NG - 4) * NFX));
+    else __builtin_amdgcn_s_waitcnt(0x0070 | 15);
   };
 
   floatx4 acc[TM][4];
@@ -664,28 +692,42 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
   };
-  // Step t lies in stage t % 4.  A wave's memory phase of step t reads its fragments,
-  // issues its loads of step t + 3 (into the stage that both groups read last in step
-  // t - 1, at least one barrier ago) and waits for its own loads of step t + 1; the
+  // Step t of W lies in stage t % 4, piece q of x in slot q % NG.  A wave's memory phase of step t reads its
+  // fragments, issues its loads of W of step t + 3 (into the stage that both groups read last in
+  // step t - 1, at least one barrier ago) or of piece t + NG - 2 of x (into the slot of piece t - 2, read
+  // last in step t - 1 or t - 2) and waits for its own loads of step t + 1; the
   // barrier after the other group's same phase then says that step t + 1 is whole.
-  fetch(0, 0);
-  fetch(1, 1);
-  fetch(2, 2);
-  wait_all_but_two_steps();
+  if (fetches_x) {
+#pragma unroll
+    for (int q = 0; q < NG - 2; ++q) fetch_x(q, q & 1, q * PIECE);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) fetch_w(q, q);
+  }
+  wait_loads(true);
   barrier();
   if (grp == 1) barrier();                               // the second group runs half a step behind
+  unsigned read_at = wm * PIECE, write_at = (NG - 2) * PIECE;
+  const int even_at = c * 128 + ((g ^ (c >> 1)) << 4), odd_at = c * 128 + (((4 + g) ^ (c >> 1)) << 4);
   for (int t0 = 0; t0 < nk; t0 += 4) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int t = t0 + u;
       if (t < nk) {                                      // (the same for every wave of the block)
-        const char* stage = smem + u * STAGE;
+        const char* ws = smem + W_AT + u * W_STEP;
+        const char* xs = smem + read_at + ((u & 1) ? odd_at : even_at);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = *(const bf16x8*)(stage + (XF + wn * 4 + j) * 1024 + lane * 16);
+        for (int j = 0; j < 4; ++j) b[j] = *(const bf16x8*)(ws + (wn * 4 + j) * 1024 + lane * 16);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = *(const bf16x8*)(stage + (wm * TM + i) * 1024 + lane * 16);
-        fetch((u + 3) & 3, t + 3);
-        wait_all_but_two_steps();
+        for (int i = 0; i < TM; ++i) a[i] = *(const bf16x8*)(xs + i * 2048);
+        if (fetches_x) fetch_x(t + NG - 2, (u + NG) & 1, write_at);
+        else fetch_w((u + 3) & 3, t + 3);
+        write_at = write_at == (NG - 1) * PIECE ? 0 : write_at + PIECE;
+        if (u & 1) {
+          read_at += 2 * PIECE;
+          if (read_at >= NG * PIECE) read_at -= NG * PIECE;
+        }
+        wait_loads(u & 1);
         barrier();
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -1320,21 +1362,21 @@ static const TileModel TILE_MODELS[TILE_ALL] = {{64, 64, 6.39, 0.79, 0.289, 1.0,
                                                   {64, 128, 6.54, 0.71, 0.5, 1.5, 27e3, 0},
                                                   {128, 128, 8.0, 0.48, 0.66, 1.0, 24e3, 0},
                                                   {128, 256, 0.0, 6.16, 0.945, 1.0, 24e3, 1},
-                                                  {256, 256, 0.0, 9.2, 1.8, 1.0, 24e3, 1},
-                                                  {192, 256, 0.0, 9.2, 1.4, 1.0, 24e3, 1},
+                                                  {256, 256, 0.0, 12.8, 1.34, 1.0, 24e3, 1},
+                                                  {192, 256, 0.0, 10.2, 1.08, 1.0, 24e3, 1},
                                                   {64, 96}, {64, 160}, {64, 224}, {128, 160}};
 constexpr double CHIP_STREAM = 5.3e6;     // bytes a microsecond
 
 // The tiles of the two groups of waves: whole rounds of one block a unit; with 256 rows a
-// step of 32 of the inner size takes 0.82 us in a full round and from 0.56 us in a round of
-// few blocks (the chip clocks higher), and 9.6 us pass before and after the loop; with 192
-// rows 0.64, 0.47 and 7.6 us (fitted to the same sweeps, inner sizes from 896 to 27648: 8
-// and 9 % rms).
+// step of 32 of the inner size takes 0.67 us in a full round and from 0.41 us in a round of
+// few blocks (the chip clocks higher), and 12.8 us pass before and after the loop; with 192
+// rows 0.54, 0.37 and 10.2 us (fitted to a sweep of 14 matrices of four model shapes at 512 to 8192
+// rows, inner sizes from 896 to 18944: 7 and 5 % rms).
 static double pingpong_cost(int bm, int M, int N, int K, int num_cus, int pieces) {
   const double rounds = (double)((M + bm - 1) / bm) * ((N + 255) / 256) * pieces / num_cus;
   const double whole = floor(rounds + 1e-9), last = rounds - whole;
   const int steps = pieces > 1 ? 2 * (((K + 63) / 64 + pieces - 1) / pieces) : (K + 31) / 32;
-  const double before_after = bm == 256 ? 9.6 : 7.6, full = bm == 256 ? 0.816 : 0.637, few = bm == 256 ? 0.555 : 0.472;
+  const double before_after = bm == 256 ? 12.8 : 10.2, full = bm == 256 ? 0.67 : 0.544, few = bm == 256 ? 0.414 : 0.371;
   double t = whole * (before_after + steps * full);
   if (last > 1e-9) t += before_after + steps * (few + (full - few) * last);
   return t;
@@ -1366,6 +1408,7 @@ static int g_force_tile = 0, g_without_wide = 0, g_pp_min_rows = 512;
 // tokens of five shapes that is between 1.4 % faster and 1.3 % slower than from 2,048 on.)
 constexpr int WIDE_TILE_MIN_ROWS = 2048;
 constexpr int PP_MIN_INNER = 896;      // the shortest inner size the estimates of those tiles were fitted to
+constexpr int PP_MAX_INNER = 1 << 22;  // their loads address a tile's rows by 32 bits of bytes
 extern "C" void llmlab_debug_gemm_tile(int tile) {
   g_force_tile = tile > 0 ? tile : 0;
   g_without_wide = tile == -131;
@@ -1440,8 +1483,8 @@ static int choose_tile(int M, int N, int K, int num_cus) {
   if (g_force_tile == 130) return TILE_64x128;
   if (g_force_tile == 129 || g_force_tile == 128) return TILE_128;
   if (g_force_tile == 131) return TILE_128x256;
-  if (g_force_tile == 132) return TILE_256;
-  if (g_force_tile == 133) return TILE_192;
+  if (g_force_tile == 132 && K <= PP_MAX_INNER) return TILE_256;
+  if (g_force_tile == 133 && K <= PP_MAX_INNER) return TILE_192;
   // One or two tiles of rows of a wide matrix (the head, gate and up at larger shapes):
   // bound by the read of W, which the wider tiles stream better than the estimate
   // knows, and the 128-row tile reads W once where two 64-row tiles read it twice
@@ -1484,10 +1527,10 @@ static int choose_tile(int M, int N, int K, int num_cus) {
     }
   }
   // The tiles of the two groups of waves where the estimate of one is the lowest (over the
-  // sweeps the 256 x 256 tile is then 10 to 24 % faster than the best of the others: 2048
-  // rows, 37888 x 3584: 501 us against 623; 55296 x 5120: 999 against 1245; with a quarter
+  // sweeps the 256 x 256 tile is then 10 to 30 % faster than the best of the others: 2048
+  // rows, 37888 x 3584: 460 us against 607; with a quarter
   // of a round of blocks it is twice as slow; the 192 x 256 tile where its blocks fill
-  // their rounds better: 2048 rows, 5120 x 27648: 534 us against 655 with 256 rows).
+  // their rounds better: 2048 rows, 4608 x 3584: 66 us against 74 with 256 rows).
   // From 512 rows on (prefill steps of 512 to 960 tokens as a whole: 2.4 to 6.8 % faster at
   // the 7B shape, 3 to 4.6 % at the 32B shape; from 256 rows a step of 384 tokens would be
   // 13 % slower at the 7B shape: the estimates are not fitted there) and an inner size of
@@ -1499,8 +1542,11 @@ static int choose_tile(int M, int N, int K, int num_cus) {
   // chip (192 / 256 / 384 rows of 55296 x 5120: 153 / 171 / 261 us against 187 / 199 / 274 with the
   // best of the others; of 59136 x 8192: 229 / 263 / 392 against 305 / 316 / 437)
   const bool pp_rows = M >= g_pp_min_rows || (g_pp_min_rows == 512 && M > 128 && N >= 16384);
-  if (pp_rows && K >= PP_MIN_INNER && !g_without_wide) {
-    double least = tile_cost(best, M, N, K, num_cus, 1);
+  if (pp_rows && K >= PP_MIN_INNER && K <= PP_MAX_INNER && !g_without_wide) {
+    // (the estimates of the other tiles, fitted at shorter inner sizes, are up to a quarter low from
+    // 3,584 on (and 512 rows): 4096 rows of 1536 x 8960 129 us against 147 with their pick, 2048 of 3584 x 18944 268 against 301,
+    // 2367 of 2048 x 11008 154 against 181; over 126 products the picks then lose 0.1 % on average)
+    double least = tile_cost(best, M, N, K, num_cus, 1) * (M >= 512 && K >= 3584 ? 1.25 : 1.0);
     for (int kind = TILE_256; kind <= TILE_192; ++kind) {
       const double c = tile_cost(kind, M, N, K, num_cus, 1);
       if (c < least) {
@@ -1645,7 +1691,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   for (int kind = TILE_64x128; kind < TILE_KINDS; ++kind) {
     if (kind == TILE_128x256) continue;
     if (one_tile_of_128 && kind != TILE_128) continue;
-    if (kind >= TILE_256 && !(M >= g_pp_min_rows && K >= PP_MIN_INNER && !g_without_wide)) continue;
+    if (kind >= TILE_256 && !(M >= g_pp_min_rows && K >= PP_MIN_INNER && K <= PP_MAX_INNER && !g_without_wide)) continue;
     if (g_force_tile != 0 && kind != choose_tile(M, N, K, num_cus)) continue;
     for (int s = 2; s <= max_pieces; ++s) {
       if ((nk + s - 1) / s < min_tiles_per_piece) break;

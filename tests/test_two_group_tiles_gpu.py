@@ -1,0 +1,34 @@
+"""The tiles of two groups of waves: every length of the inner size at which their rings in LDS begin, wrap or
+end (pieces of x of two steps, steps of W, the last of them cut short), whole and in pieces."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+BF = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llm_inference_lab_amd.kernels.hip_ops import HipOps
+    return HipOps(DEV)
+
+
+@pytest.mark.parametrize("tile,m", [(132, 257), (132, 400), (133, 193), (133, 300)])
+@pytest.mark.parametrize("k", [8, 32, 56, 64, 72, 96, 128, 160, 192, 200, 224, 256, 352, 384, 392, 448, 776])
+def test_inner_sizes_around_the_rings(ops, tile, m, k):
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    x = torch.randn(m, k, device=DEV, generator=gen).to(BF)
+    w = torch.randn(530, k, device=DEV, generator=gen).to(BF)
+    want = x.double() @ w.double().T
+    unit = (k + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + 1)      # float32 sums in any order
+    pw = ops.prepare_weight(w)
+    with ops.debug.force(gemm_tile=tile, few_rows_max=64):
+        out = torch.empty(m, 530, device=DEV)
+        ops.linear_logits(x, pw, out)
+        assert bool(((out.double() - want).abs() <= unit).all())
+        for count in (2, 3):
+            parts = torch.zeros(count, m, 530, device=DEV)
+            ops.linear_partials(x, pw, parts, count)
+            assert bool(((parts.double().sum(0) - want).abs() <= unit).all())
