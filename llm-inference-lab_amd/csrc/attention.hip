@@ -90,8 +90,32 @@ struct AttnArgs {
   int tiles;          // paired kernel: tiles of rows per request (blocks take two each)
   int qlen_lo, qlen_hi;  // only requests that bring so many tokens are worked on (a step may be
                          // served by two launches: its short requests by one, its long ones by the other)
+  int reqs, picked;   // picked > 0: block z of the launch is for the z-th of the `reqs` requests that bring
+                      // so many tokens, of which there are `picked`
   float scale;
 };
+
+// The request of block z of a launch: of a step of both kinds of requests, whose launch has blocks for one
+// kind only, the z-th that brings qlen_lo to qlen_hi tokens (-1: there are fewer).  All waves of a block call
+// it alike; 64 requests a load, found by the ballots.  With a block for every request, most of them for
+// the other kind and ending at once, a portion of 464 tokens beside 48 decoding requests (10,094 blocks of
+// 8 waves and 68 KB, 300 of them alive) took 33 us, most of it the empty ones.  (A loop that would go on
+// to a request `picked` further costs every block 10 registers, and the short kernels a wave a SIMD.)
+__device__ __forceinline__ int request_of(const AttnArgs& a, int z) {
+  if (a.picked <= 0) return z;
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int base = 0; base < a.reqs; base += 64) {
+    const int i = min(base + lane, a.reqs - 1);
+    const int len = a.q_start[i + 1] - a.q_start[i];
+    const bool in = base + lane < a.reqs && len >= a.qlen_lo && len <= a.qlen_hi;
+    const unsigned long long all = __ballot(in);
+    const unsigned long long one = __ballot(in && before + __popcll(all & ((1ull << lane) - 1)) == z);
+    if (one) return __builtin_amdgcn_readfirstlane(base + __ffsll(one) - 1);
+    before += __popcll(all);
+  }
+  return -1;
+}
 
 // ------------------------------------------------------------- bf16, MFMA
 // The fragments of one step of 32 keys: two blocks of 16 keys, and the values of
@@ -775,27 +799,32 @@ template <int QB, bool DECODE, int RING = 1, int PH = 1>
 __global__ __launch_bounds__(DECODE ? 64 * DECODE_WAVES : 256 * PH, (!DECODE && D <= 64 && PH == 1) ? 2 : 1) void attention_bf16_kernel(AttnArgs a) {
   if constexpr (DECODE) {
     __shared__ __attribute__((aligned(16))) float dlds[decode_lds_floats<QB>()];
-    attention_tile<QB, DECODE, RING, PH>(a, (int)(gridDim.x - 1 - blockIdx.x), (int)blockIdx.y, (int)blockIdx.z, dlds);
+    const int b = QB == 1 ? (int)blockIdx.z : request_of(a, (int)blockIdx.z);      // (tiles of 16 rows: decode steps)
+    if (b < 0) return;
+    attention_tile<QB, DECODE, RING, PH>(a, (int)(gridDim.x - 1 - blockIdx.x), (int)blockIdx.y, b, dlds);
   } else {
-    attention_tile<QB, DECODE, RING, PH>(a, (int)(gridDim.x - 1 - blockIdx.x), (int)blockIdx.y, (int)blockIdx.z, nullptr);
+    const int b = request_of(a, (int)blockIdx.z);
+    if (b < 0) return;
+    attention_tile<QB, DECODE, RING, PH>(a, (int)(gridDim.x - 1 - blockIdx.x), (int)blockIdx.y, b, nullptr);
   }
 }
 
-// A mixed step in one launch: the first `long_blocks` blocks of a request (x) are the tiles of
-// rows of a portion times the kv heads, each with the keys of its tile split over its waves; the
-// others are the (kv head, split) pairs of a request of a few tokens, whose keys are split over
-// blocks as in a decode step.  A block finds in its request's length which of the two it is
-// for and ends at once if it is for the other kind.  In two launches the decoding requests'
-// blocks, which stream their histories, wait for the portion's, which are a chain of small
+// A mixed step in one launch: first the portions' blocks, a request's tiles of rows times the kv heads
+// after another's, each with the keys of its tile split over its waves; then the decoding requests' blocks,
+// (kv head, split) pairs, whose keys are split over blocks as in a decode step.  In two launches the decoding
+// requests' blocks, which stream their histories, wait for the portion's, which are a chain of small
 // products, although they need different parts of a compute unit.
 template <int QBL, int RL, int RS>
 __global__ __launch_bounds__(64 * DECODE_WAVES) void attention_bf16_mixed_kernel(AttnArgs al, AttnArgs as, int long_tiles) {
   __shared__ __attribute__((aligned(16))) float dlds[decode_lds_floats<QBL>()];
-  const int x = (int)blockIdx.x, long_blocks = long_tiles * al.nkv;
-  if (x < long_blocks)
-    attention_tile<QBL, true, RL>(al, long_tiles - 1 - x / al.nkv, x % al.nkv, (int)blockIdx.z, dlds);
-  else
-    attention_tile<1, true, RS>(as, 0, x - long_blocks, (int)blockIdx.z, dlds);
+  const int x = (int)blockIdx.x, per_long = long_tiles * al.nkv, longs = per_long * al.picked;
+  if (x < longs) {
+    const int at = x % per_long, b = request_of(al, x / per_long);
+    if (b >= 0) attention_tile<QBL, true, RL>(al, long_tiles - 1 - at / al.nkv, at % al.nkv, b, dlds);
+  } else {
+    const int per_short = as.nkv * as.splits, at = (x - longs) % per_short, b = request_of(as, (x - longs) / per_short);
+    if (b >= 0) attention_tile<1, true, RS>(as, 0, at, b, dlds);
+  }
 }
 
 // Two tiles of rows per block, one after the other: tile t from the end and tile t
@@ -805,9 +834,11 @@ __global__ __launch_bounds__(64 * DECODE_WAVES) void attention_bf16_mixed_kernel
 template <int QB, int PH = 1>
 __global__ __launch_bounds__(256 * PH, (D <= 64 && PH == 1) ? 2 : 1) void attention_bf16_paired_kernel(AttnArgs a) {
   const int late = a.tiles - 1 - (int)blockIdx.x, early = (int)blockIdx.x;
+  const int b = request_of(a, (int)blockIdx.z);
+  if (b < 0) return;
   for (int pass = 0; pass < 2; ++pass) {
     if (pass == 1 && early >= late) break;
-    attention_tile<QB, false, 1, PH>(a, pass == 0 ? late : early, (int)blockIdx.y, (int)blockIdx.z, nullptr);
+    attention_tile<QB, false, 1, PH>(a, pass == 0 ? late : early, (int)blockIdx.y, b, nullptr);
     __syncthreads();
   }
 }
@@ -915,7 +946,8 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int b = blockIdx.z;
+  const int b = request_of(a, (int)blockIdx.z);
+  if (b < 0) return;
   const int kvh = blockIdx.y / a.splits, split = blockIdx.y % a.splits;
   const int G = a.nq / a.nkv;
   const int r0 = a.q_start[b], qlen = a.q_start[b + 1] - r0, sp = a.start_pos[b];
@@ -1327,7 +1359,7 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
                                         workspace_floats, num_cus, row_req, stream);
     if (rc) return rc;
     a.qlen_lo = short_len + 1;
-    live = reqs - n_short;
+    a.picked = live = reqs - n_short;
   }
   constexpr int ROWS = 16 * F32_QB;
   const long tiles = (max_rows + ROWS - 1) / ROWS;
@@ -1341,10 +1373,10 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
   // keys (4 requests of 256 tokens: 58 against 81).
   const int path = choose_many_rows_launch_f32(tiles * a.nkv * live, max_q_len, max_ctx_len, num_cus, g_force_path);
   if (path == 1) {
-    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, true, F32_SPLIT_WAVES>), dim3((unsigned)tiles, a.nkv, reqs),
+    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, true, F32_SPLIT_WAVES>), dim3((unsigned)tiles, a.nkv, live),
                        dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
   } else {
-    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, false, 4>), dim3((unsigned)((tiles + 3) / 4), a.nkv, reqs),
+    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, false, 4>), dim3((unsigned)((tiles + 3) / 4), a.nkv, live),
                        dim3(256), 0, stream, a);
   }
   LLMLAB_LAUNCH_CHECK("attention(float32)");
@@ -1503,6 +1535,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
   a.page_shift = 0;
   a.tiles = 0;
   a.qlen_lo = 0; a.qlen_hi = 0x7fffffff;
+  a.reqs = reqs; a.picked = 0;
   while ((1 << a.page_shift) < page_size) ++a.page_shift;
   if (dtype == DT_F32)
     return launch_attention_f32(a, reqs, max_q_len, max_ctx_len, window, total_rows, workspace, workspace_floats,
@@ -1525,7 +1558,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     shorts = prepare_key_split_decode(s, reqs, n_short, short_ctx, window, total_rows, nq, nkv, workspace,
                                       workspace_floats, num_cus, arrived, arrived_ints);
     a.qlen_lo = short_len + 1;
-    live = reqs - n_short;
+    a.picked = live = reqs - n_short;
   }
   const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, g_force_path);
   if (mixed && path != 1) {
@@ -1553,9 +1586,10 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
       if (rc) return rc;
     }
     if (one_launch) {
-      const long gx = (long)long_tiles * nkv + (long)nkv * shorts.a.splits;
+      shorts.a.picked = n_short;
+      const long gx = (long)long_tiles * nkv * live + (long)nkv * shorts.a.splits * n_short;
       LLMLAB_REQUIRE(gx <= 0x7fffffffL, "attention: grid too large");
-      dim3 mgrid((unsigned)gx, 1, reqs), mblock(64 * DECODE_WAVES);
+      dim3 mgrid((unsigned)gx), mblock(64 * DECODE_WAVES);
       const bool deep = steps_per_wave > 2;
       if (deep && shorts.ring == 2)
         hipLaunchKernelGGL((attention_bf16_mixed_kernel<2, 2, 2>), mgrid, mblock, 0, stream, a, shorts.a, long_tiles);
@@ -1568,7 +1602,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
       LLMLAB_LAUNCH_CHECK("attention(bfloat16, mixed)");
       return launch_split_merge(shorts, total_rows, nq, row_req, out, out_stride, stream);
     }
-    dim3 grid((unsigned)((max_rows + 31) / 32), nkv, reqs), block(64 * DECODE_WAVES);
+    dim3 grid((unsigned)((max_rows + 31) / 32), nkv, live), block(64 * DECODE_WAVES);
     if (steps_per_wave > 2)
       hipLaunchKernelGGL((attention_bf16_kernel<2, true, 2>), grid, block, 0, stream, a);
     else
@@ -1577,25 +1611,25 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     return 0;
   }
   if (path == 2) {
-    dim3 grid((unsigned)((max_rows + 127) / 128), nkv, reqs), block(256);
+    dim3 grid((unsigned)((max_rows + 127) / 128), nkv, live), block(256);
     hipLaunchKernelGGL((attention_bf16_kernel<2, false>), grid, block, 0, stream, a);
   } else if (path == 5) {
     if constexpr (TWO_GROUPS) {
       a.tiles = (int)((max_rows + 63) / 64);
-      dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, reqs), block(512);
+      dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, live), block(512);
       hipLaunchKernelGGL((attention_bf16_paired_kernel<1, 2>), grid, block, 0, stream, a);
     }
   } else if (path == 6) {
     if constexpr (TWO_GROUPS) {
-      dim3 grid((unsigned)((max_rows + 63) / 64), nkv, reqs), block(512);
+      dim3 grid((unsigned)((max_rows + 63) / 64), nkv, live), block(512);
       hipLaunchKernelGGL((attention_bf16_kernel<1, false, 1, 2>), grid, block, 0, stream, a);
     }
   } else if (path == 3) {
     a.tiles = (int)((max_rows + 63) / 64);
-    dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, reqs), block(256);
+    dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, live), block(256);
     hipLaunchKernelGGL((attention_bf16_paired_kernel<1>), grid, block, 0, stream, a);
   } else {
-    dim3 grid((unsigned)((max_rows + 63) / 64), nkv, reqs), block(256);
+    dim3 grid((unsigned)((max_rows + 63) / 64), nkv, live), block(256);
     hipLaunchKernelGGL((attention_bf16_kernel<1, false>), grid, block, 0, stream, a);
   }
   LLMLAB_LAUNCH_CHECK("attention(bfloat16, prefill)");
