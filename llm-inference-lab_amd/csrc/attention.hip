@@ -1466,9 +1466,28 @@ static bool mixed_step_in_one_launch(long long_blocks, long short_blocks, int nu
   return 2 * long_blocks <= places || 4 * (long_blocks + short_blocks) <= 5 * places;
 }
 
+// Whether a mixed step goes in one launch with the portions by tiles of 16 rows, whose waves split the keys with one
+// step on its way: few enough registers (116 at heads of 64, against 157 to 201) that a unit holds two
+// blocks of either kind, so that the decoding requests' streams pass beside the portions' chains.  `blocks16` and
+// `blocks32`: the portions' blocks by tiles of 16 and of 32 rows; `path`: the launch they would take by
+// themselves; `deep`: some wave has more than two steps.  Not where all blocks with 32 rows find a unit at once
+// and have histories for a deeper ring, nor where the portions alone fill the chip several times, the less the longer the
+// histories that each 16 rows walk again.  Measured over 630 mixed steps of one portion of 64 to 1,900
+// tokens behind 0 to 4,096 keys beside 8 to 90 requests decoding at 300 to 3,000 (heads of 64, 14 over 2, and of 128, 28
+// over 4), against the launches below: 64 tokens from their start 23 -> 18 us and 58 -> 38; 464 behind 1,100 beside 48 at 1,400
+// 23.3 -> 17.0; 256 of heads of 128 behind 1,100 70 -> 56; 900 behind 1,100 at heads of 64 40 -> 35; 1,900 of heads of 64 would
+// lose 7 to 13 %, 464 of heads of 128 7 to 25 %.
+static bool mixed_step_by_small_tiles(long blocks16, long blocks32, long short_blocks, int short_ring, bool deep, int path,
+                                      int max_ctx_len, int num_cus) {
+  if (D > 128) return false;                   // (not measured)
+  if (path == 1 && deep && blocks32 + short_blocks <= (D <= 64 ? 1L : 2L) * num_cus) return false;
+  if (D <= 64) return blocks16 <= num_cus || (2 * blocks16 <= 7L * num_cus && max_ctx_len <= 3072);
+  return blocks16 <= (path != 1 && short_ring == 2 ? 1L : 2L) * num_cus;
+}
+
 // How many attention launches a mixed step in bfloat16 takes (the merge of key splits not
-// counted): `n_short` of its requests decode behind at most `short_ctx` keys, the others bring
-// portions of at most `max_q_len` tokens (for tests and tuning; 0: not a mixed step).
+// counted) where its portions do not go by tiles of 16 rows: `n_short` of its requests decode behind at most
+// `short_ctx` keys, the others bring portions of at most `max_q_len` tokens (for tests and tuning; 0: not a mixed step).
 extern "C" int llmlab_attention_mixed_launches(int nq, int nkv, int reqs, int n_short, int max_q_len, int max_ctx_len,
                                                int short_ctx, int window, int num_cus) {
   if (num_cus <= 0) num_cus = 256;
@@ -1561,13 +1580,26 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     a.picked = live = reqs - n_short;
   }
   const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, g_force_path);
+  const int steps32 = (max_ctx_len + 31) / 32 + 1;
+  const int steps_per_wave = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;
+  if (mixed && g_force_path == 0 && g_force_two_launches == 0 &&
+      mixed_step_by_small_tiles((max_rows + 15) / 16 * nkv * live, (max_rows + 31) / 32 * nkv * live,
+                                (long)nkv * shorts.a.splits * n_short, shorts.ring,
+                                steps_per_wave > 2 || shorts.ring == 2, path, max_ctx_len, num_cus)) {
+    const int tiles16 = (int)((max_rows + 15) / 16);
+    shorts.a.picked = n_short;
+    const long gx = (long)tiles16 * nkv * live + (long)nkv * shorts.a.splits * n_short;
+    LLMLAB_REQUIRE(gx <= 0x7fffffffL, "attention: grid too large");
+    hipLaunchKernelGGL((attention_bf16_mixed_kernel<1, 1, 1>), dim3((unsigned)gx), dim3(64 * DECODE_WAVES), 0, stream, a,
+                       shorts.a, tiles16);
+    LLMLAB_LAUNCH_CHECK("attention(bfloat16, mixed, tiles of 16 rows)");
+    return launch_split_merge(shorts, total_rows, nq, row_req, out, out_stride, stream);
+  }
   if (mixed && path != 1) {
     const int rc = launch_key_split_decode(shorts, reqs, total_rows, nq, nkv, row_req, out, out_stride, stream);
     if (rc) return rc;
   }
   if (path == 1) {
-    const int steps32 = (max_ctx_len + 31) / 32 + 1;
-    const int steps_per_wave = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;
     // Both kinds of blocks in one launch (see attention_bf16_mixed_kernel) where the portion's
     // blocks leave half of the chip's places free, or all blocks together hardly exceed the
     // places: every block of the one launch holds the registers of the portion's kind, so the

@@ -26,3 +26,12 @@ def test_every_launch(ops, emu, path):  # noqa: F811
     spec[3], spec[66] = (30, 90), (0, 65)
     with ops.debug.force(attention_path=(64, path)):
         run_attention(ops, emu, torch.bfloat16, 14, 2, 64, 16, None, spec, seed=96)
+
+
+@pytest.mark.parametrize("window", [None, 40])
+@pytest.mark.parametrize("nq,nkv,d,page", [(14, 2, 64, 64), (7, 1, 16, 16), (12, 2, 128, 32), (4, 4, 112, 16)])
+def test_tiles_of_16_rows(ops, emu, window, nq, nkv, d, page):  # noqa: F811
+    """The step in one launch with small tiles: portions that fill no tile, begin in one, or see no key of some waves,
+    behind histories whose keys are split over blocks and not."""
+    for spec in ([(0, 3), (5, 1)], [(0, 17), (900, 1), (64, 1)], [(700, 1), (33, 50), (1500, 1), (0, 129)]):
+        run_attention(ops, emu, torch.bfloat16, nq, nkv, d, page, window, spec, seed=97)
