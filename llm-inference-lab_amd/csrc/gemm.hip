@@ -323,6 +323,43 @@ __device__ __forceinline__ void tile_epilogue(const float* Cs, const EpiArgs& e,
   }
 }
 
+// QKV: what the epilogue needs from global memory per row of the tile (position, and the page of that
+// position for the tiles that hold k or v heads) and per column (bias, rotary frequencies).  `ask`, before
+// the product's first loads: the position, the request and the vectors; `page`, behind those loads: the
+// page, which needs the two; `put`, after the product: into LDS.  Nothing waits for a trip to memory
+// before the product's own first tiles are on their way (put into LDS at once, position, request and page
+// were two trips in a row before them: 512 rows of 1152 x 896 13.5 us, 12.6 now).
+template <int BM, int BN, int NT>
+struct QkvRows {
+  static_assert(BM <= NT && BN <= 2 * NT && NT >= 128, "a row, two columns and a frequency a thread");
+  int pos, at, page_no;
+  float freq, bias[2];
+  __device__ __forceinline__ void ask(const EpiArgs& e, int m0, int n0, int M, int N, int tid) {
+    const int m = min(m0 + min(tid, BM - 1), M - 1);
+    pos = e.positions[m];
+    at = e.kcache && n0 + BN > e.nq * e.d ? e.row_req[m] : -1;
+    freq = e.inv_freq && tid < (e.d >> 1) ? e.inv_freq[tid] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int n = n0 + tid + i * NT;
+      bias[i] = e.bias && tid + i * NT < BN && n < N ? load_vec(e.bias, e.bias_bf16, n) : 0.f;
+    }
+  }
+  __device__ __forceinline__ void page(const EpiArgs& e) {
+    page_no = at >= 0 ? e.table[(size_t)at * e.table_stride + pos / e.page_size] : 0;
+  }
+  __device__ __forceinline__ void put(int tid, int* s_pos, int* s_page, float* s_freq, float* s_bias) const {
+    if (tid < BM) {
+      s_pos[tid] = pos;
+      s_page[tid] = page_no;
+    }
+    if (tid < 128) s_freq[tid] = freq;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (tid + i * NT < BN) s_bias[tid + i * NT] = bias[i];
+  }
+};
+
 // ============================================================ bf16, tiled
 template <int BM, int BN, int BK, int WM, int WN, int EPI, bool GROUPED = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __restrict__ A,
@@ -368,25 +405,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
     W += (size_t)member * e.g_w_stride;
   }
 
-  // QKV: what the epilogue needs from global memory per row of the tile (position, and the
-  // page of that position for the tiles that hold k or v heads) and per column (bias,
-  // rotary frequencies) is fetched now, so that those round trips (the page follows the
-  // position follows the request) pass behind the product instead of after it.
   constexpr bool QKV = EPI == EPI_QKV;
   __shared__ int s_pos[QKV ? BM : 1], s_page[QKV ? BM : 1];
   __shared__ float s_freq[QKV ? 128 : 1], s_bias[QKV ? BN : 1];
-  if constexpr (QKV) {
-    if (tid < BM) {
-      const int m = min(m0 + tid, M - 1);
-      const int pos = e.positions[m];
-      s_pos[tid] = pos;
-      s_page[tid] = (e.kcache && n0 + BN > e.nq * e.d)
-                        ? e.table[(size_t)e.row_req[m] * e.table_stride + pos / e.page_size] : 0;
-    }
-    for (int i = tid; i < (e.d >> 1); i += NT) s_freq[i] = e.inv_freq ? e.inv_freq[i] : 0.f;
-    for (int i = tid; i < BN; i += NT)
-      s_bias[i] = (e.bias && n0 + i < N) ? load_vec(e.bias, e.bias_bf16, n0 + i) : 0.f;
-  }
+  QkvRows<QKV ? BM : 64, QKV ? BN : 64, QKV ? NT : 128> rows;
+  if constexpr (QKV) rows.ask(e, m0, n0, M, N, tid);
 
   floatx4 acc[TM][TN];
 #pragma unroll
@@ -461,6 +484,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
     fetch(p, kbase + p * BK);
     fetch_b(p, kbase + p * BK);
   }
+  if constexpr (QKV) rows.page(e);
   // Tile t lies in stage t % 3.  It is put there during tile t - 2, and its fragments are
   // read into registers half a tile ahead of their products (those of its first 32
   // columns of K during the second half of tile t - 1), so that the reads of LDS pass
@@ -524,6 +548,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
 #pragma unroll
       for (int x = 0; x < 4; ++x)
         Cs[(wm * WTM + i * 16 + g * 4 + x) * C_STRIDE + wn * WTN + j * 16 + c] = acc[i][j][x];
+  if constexpr (QKV) rows.put(tid, s_pos, s_page, s_freq, s_bias);
   __syncthreads();
   tile_epilogue<BM, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
 }
@@ -593,18 +618,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   constexpr bool QKV = EPI == EPI_QKV;
   __shared__ int s_pos[QKV ? BM : 1], s_page[QKV ? BM : 1];
   __shared__ float s_freq[QKV ? 128 : 1], s_bias[QKV ? BN : 1];
-  if constexpr (QKV) {
-    if (tid < BM) {
-      const int m = min(m0 + tid, M - 1);
-      const int pos = e.positions[m];
-      s_pos[tid] = pos;
-      s_page[tid] = (e.kcache && n0 + BN > e.nq * e.d)
-                        ? e.table[(size_t)e.row_req[m] * e.table_stride + pos / e.page_size] : 0;
-    }
-    for (int i = tid; i < (e.d >> 1); i += NT) s_freq[i] = e.inv_freq ? e.inv_freq[i] : 0.f;
-    for (int i = tid; i < BN; i += NT)
-      s_bias[i] = (e.bias && n0 + i < N) ? load_vec(e.bias, e.bias_bf16, n0 + i) : 0.f;
-  }
+  QkvRows<QKV ? BM : 64, QKV ? BN : 64, QKV ? NT : 128> rows;
+  if constexpr (QKV) rows.ask(e, m0, n0, M, N, tid);
 
   // Per step a wave fetches four times 1 KB (three times of x with BM = 192): the even waves of x,
   // the odd ones of W (so that both groups fetch both).  Rows past M, strips past N and numbers past K read a
@@ -697,6 +712,10 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   // step t - 1, at least one barrier ago) or of piece t + NG - 2 of x (into the slot of piece t - 2, read
   // last in step t - 1 or t - 2) and waits for its own loads of step t + 1; the
   // barrier after the other group's same phase then says that step t + 1 is whole.
+  if constexpr (QKV) {
+    rows.page(e);
+    rows.put(tid, s_pos, s_page, s_freq, s_bias);          // (before the direct loads, whose number the waits count)
+  }
   if (fetches_x) {
 #pragma unroll
     for (int q = 0; q < NG - 2; ++q) fetch_x(q, q & 1, q * PIECE);
