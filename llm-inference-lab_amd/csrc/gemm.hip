@@ -712,10 +712,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   // step t - 1, at least one barrier ago) or of piece t + NG - 2 of x (into the slot of piece t - 2, read
   // last in step t - 1 or t - 2) and waits for its own loads of step t + 1; the
   // barrier after the other group's same phase then says that step t + 1 is whole.
-  if constexpr (QKV) {
-    rows.page(e);
-    rows.put(tid, s_pos, s_page, s_freq, s_bias);          // (before the direct loads, whose number the waits count)
-  }
+  if constexpr (QKV) rows.page(e);
   if (fetches_x) {
 #pragma unroll
     for (int q = 0; q < NG - 2; ++q) fetch_x(q, q & 1, q * PIECE);
@@ -763,6 +760,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
 
   // ---- epilogue: the rows 0-127 of the tile through LDS, then the rest
   float* Cs = (float*)smem;
+  if constexpr (QKV) rows.put(tid, s_pos, s_page, s_freq, s_bias);
   auto to_lds = [&](int part) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -783,6 +781,159 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   to_lds(1);
   tile_epilogue<BM - HALF, BN, NT, EPI>(Cs, e, m0 + HALF, n0, M, N, tid, s_pos + (QKV ? HALF : 0),
                                         s_page + (QKV ? HALF : 0), s_freq, s_bias);
+}
+
+// ============================================================ bf16, small tiles by direct loads
+// Small products: four waves 2 x 2 on a tile of BM x BN, both operands by direct loads into LDS as in the kernel
+// above (x 8 rows of 128 bytes a load, W by fragments), in stages of 64 of the inner size, NST of them.  What
+// bounds such a product is its few blocks' way through launch, first trip to memory, K tiles and epilogue; here no
+// operand passes through registers on its way, every stage but one is on its way at any time, a stage
+// takes one barrier, and three blocks of the 64 x 64 tile (48 KB) share a unit.  Against the same tile with x by way of registers and W
+// straight into them, over 182 products of 24 to 2,048 rows whole and in pieces: 18 % less; 512 rows of 896 x 896 8.9 -> 7.8 us,
+// 2,048 11.7 -> 9.2, 512 of 896 x 4864 in four pieces 15.6 -> 12.6, 64 of 3584 x 18944 in eight 39.6 -> 30.8.  Four and five stages (two blocks a
+// unit): 4 % slower.  Larger tiles of this kind: 64 x 128 (three stages) is slower than the tile above with many
+// rows (512 of 9728 x 896 24.8 against 21.4) and faster in pieces of few rows only (64 of 3584 x 18944 28.2 against 32.4), 128 x 160
+// and 128 x 256 as fast as theirs (128 of 37888 x 3584 71.8 against 73.7): not kept.
+template <int BM, int BN, int NST, int EPI>
+__global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                      EpiArgs e, int M, int N, int K) {
+  constexpr int NT = 256, WTM = BM / 2, WTN = BN / 2, TM = WTM / 16, TN = WTN / 16;
+  constexpr int XL = BM / 8, WL = BN / 8, NL = (XL + WL) / 4;      // loads of 1 KB of a stage: of x, of W, of one wave
+  static_assert((XL + WL) % 4 == 0 && WTM % 16 == 0 && WTN % 16 == 0 && NL * (NST - 2) < 64, "shape");
+  constexpr int STAGE = (XL + WL) * 1024, W_AT = XL * 1024;
+  constexpr int C_STRIDE = BN + 4;
+  constexpr size_t C_BYTES = (size_t)BM * C_STRIDE * sizeof(float);
+  __shared__ __attribute__((aligned(1024))) char smem[C_BYTES > NST * STAGE ? C_BYTES : NST * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+  int bx = blockIdx.x, by = blockIdx.y;
+  {                                                      // a band of column tiles per die, as above
+    const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
+    const int lin = by * gx + bx;
+    const int whole = total & ~7;
+    const int mapped = lin < whole ? (lin & 7) * (whole >> 3) + (lin >> 3) : lin;
+    bx = mapped / gy;
+    by = mapped - bx * gy;
+  }
+  const int m0 = by * BM, n0 = bx * BN;
+  const int c = lane & 15, g = lane >> 4;
+  constexpr bool QKV = EPI == EPI_QKV;
+  __shared__ int s_pos[QKV ? BM : 1], s_page[QKV ? BM : 1];
+  __shared__ float s_freq[QKV ? 128 : 1], s_bias[QKV ? BN : 1];
+  QkvRows<QKV ? BM : 64, QKV ? BN : 64, NT> rows;
+  if constexpr (QKV) rows.ask(e, m0, n0, M, N, tid);
+  const int T = (K + 31) >> 5, nstrips = (N + 15) >> 4;
+  unsigned off[NL];
+  int shift[NL];
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  // Load i of a wave is number wave + 4 i of the stage: the first XL take 8 rows of x each, the others a step
+  // of a strip of W.  Rows past M, strips past N and numbers past K read a valid place instead.
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int b = wave + 4 * i;
+    if (4 * i < XL) {                     // (XL % 4 == 0: the same for all waves)
+      shift[i] = ((lane & 7) ^ (((b & 1) << 2) | (lane >> 4))) * 8;
+      off[i] = ((unsigned)(min(m0 + b * 8 + (lane >> 3), M - 1) - m0) * (unsigned)K + shift[i]) * 2u;
+    } else {
+      const int f = (b - XL) >> 1;
+      shift[i] = (b - XL) & 1;
+      off[i] = (unsigned)(min((n0 >> 4) + f, nstrips - 1) - (n0 >> 4)) * (unsigned)T * 1024u + lane * 16u;
+    }
+  }
+  static_assert(XL % 4 == 0, "x first");
+  const char* const xbase = (const char*)(A + (size_t)m0 * K);
+  const char* const wbase = (const char*)(W + (size_t)(n0 >> 4) * T * 512);
+  auto load_to_lds = [&](unsigned at, const char* base, unsigned to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(at), "s"(base), "s"(to) : "memory", "m0");
+  };
+  int first = 0, nk = T;
+  if constexpr (EPI == EPI_PART) {
+    first = (int)blockIdx.z * e.kt_per_split * 2;
+    nk = max(0, min(T - first, e.kt_per_split * 2));
+    e.out = (float*)e.out + (size_t)blockIdx.z * e.part_stride;
+    if (blockIdx.z > 0) e.bias = nullptr;
+  }
+  auto fetch = [&](int stage, unsigned slot) {
+    const int t = first + 2 * stage, k = t * 32;
+    const bool whole = k + 64 <= K;
+    const char* xb = whole ? xbase + (size_t)k * 2 : xbase;
+    const char* w0 = wbase + (size_t)min(t, T - 1) * 1024;
+    const char* w1 = wbase + (size_t)min(t + 1, T - 1) * 1024;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const unsigned to = lds0 + slot + (wave + 4 * i) * 1024;
+      if (4 * i < XL) {
+        if (whole) load_to_lds(off[i], xb, to);
+        else load_to_lds(off[i] + (unsigned)(min(k + shift[i], K - 8) - shift[i]) * 2u, xb, to);
+      } else {
+        load_to_lds(off[i], ((wave + 4 * i - XL) & 1) ? w1 : w0, to);
+      }
+    }
+  };
+  auto barrier = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  };
+  constexpr int VM = NL * (NST - 2);
+  auto wait_loads = [&]() { __builtin_amdgcn_s_waitcnt(0x0070 | (VM & 15) | ((VM >> 4) << 14)); };
+  floatx4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 a[2][TM], b[2][TN];
+  const int at[2] = {c * 128 + ((g ^ (c >> 1)) << 4), c * 128 + (((4 + g) ^ (c >> 1)) << 4)};
+  auto frags = [&](int h, unsigned slot) {
+    const char* xs = smem + slot + wm * WTM * 128 + at[h];
+    const char* ws = smem + slot + W_AT + (wn * TN * 2 + h) * 1024 + lane * 16;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b[h][j] = *(const bf16x8*)(ws + j * 2048);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a[h][i] = *(const bf16x8*)(xs + i * 2048);
+  };
+  auto products = [&](int h) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], b[h][j], acc[i][j], 0, 0, 0);
+  };
+  fetch(0, 0);
+  if constexpr (QKV) rows.page(e);      // (waits for the first stage too, which has to come first in any case)
+#pragma unroll
+  for (int s = 1; s < NST; ++s) fetch(s, s * STAGE);
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NL * (NST - 1)) : "memory");
+  barrier();
+  // Stage s (steps 2 s and 2 s + 1) lies in slot s % NST.  Its first half's fragments are read during the stage
+  // before, its second half's while the first is multiplied; behind the one barrier of a stage it has been
+  // read by all, the next one is there, and stage s + NST is asked for into its place.
+  unsigned slot = 0;
+  frags(0, 0);
+  for (int t = 0; t < nk; t += 2) {
+    const unsigned next = slot == (NST - 1) * STAGE ? 0 : slot + STAGE;
+    frags(1, slot);
+    products(0);
+    wait_loads();                       // stage t / 2 + 1 is there, this stage is read
+    barrier();
+    fetch((t >> 1) + NST, slot);
+    frags(0, next);
+    if (t + 1 < nk) products(1);
+    slot = next;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);                    // the last loads (past K, never read) are in
+  barrier();
+  float* Cs = (float*)smem;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) Cs[(wm * WTM + i * 16 + g * 4 + x) * C_STRIDE + wn * WTN + j * 16 + c] = acc[i][j][x];
+  if constexpr (QKV) rows.put(tid, s_pos, s_page, s_freq, s_bias);
+  __syncthreads();
+  tile_epilogue<BM, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
 }
 
 // ================================================================ float32
@@ -1497,7 +1648,7 @@ static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int mi
   return best;
 }
 
-static int choose_tile(int M, int N, int K, int num_cus) {
+static int estimated_tile(int M, int N, int K, int num_cus) {
   if (g_force_tile == 64) return TILE_64;
   if (g_force_tile == 130) return TILE_64x128;
   if (g_force_tile == 129 || g_force_tile == 128) return TILE_128;
@@ -1577,12 +1728,55 @@ static int choose_tile(int M, int N, int K, int num_cus) {
   return best;
 }
 
+// Up to 1,024 rows of a matrix of less than 32 MB (128 rows: 64 MB): among the three small tiles the
+// estimates above lose 10 % on average (up to 42 %), because they count a block that has its unit to itself, whose
+// chain of K tiles is the time, like one of several that share it.  Here both are weighed: the chain of a block's K tiles, and
+// what a unit takes for all of its blocks.  Fitted to the same sweep (9 to 12 % rms), the pick then loses 2 %,
+// with the fold of the pieces: 512 rows of 896 x 4864 with the norm 17.8 us (64 x 64 in four pieces) against 24.7 (64 x 128 in six),
+// 700 of 2048 x 2048 15.8 against 22.5, 100 of 4608 x 3584 17.5 against 22.4.  Beyond that range the estimates above.
+static bool few_blocks_range(int M, int N, int K) {
+  const double bytes = (double)N * K * 2.0;
+  return g_force_tile == 0 && ((M <= 1024 && bytes < 32e6) || (M <= 128 && bytes < 64e6));
+}
+static double few_blocks_cost(int kind, int M, int N, int K, int num_cus, int pieces) {
+  static const struct {
+    double L, chain, f, tk, stream;
+    int resident;
+  } fit[3] = {{3.10, 0.357, 0.76, 0.227, 30.0e3, 3}, {4.03, 0.482, 1.57, 0.358, 32.4e3, 2}, {2.13, 0.71, 4.25, 0.655, 25.7e3, 1}};
+  const auto& p = fit[kind];
+  const double blocks = (double)((M + TILE_MODELS[kind].bm - 1) / TILE_MODELS[kind].bm) *
+                        ((N + TILE_MODELS[kind].bn - 1) / TILE_MODELS[kind].bn) * pieces;
+  const int nk = ((K + 63) / 64 + pieces - 1) / pieces;
+  const double share = blocks / num_cus, turns = share <= p.resident ? ceil(share - 1e-9) : share;
+  const double rate = blocks * p.stream < CHIP_STREAM ? blocks * p.stream : CHIP_STREAM;
+  double t = turns * (p.f + nk * p.tk);
+  if (nk * p.chain > t) t = nk * p.chain;
+  if ((double)N * K * 2.0 / rate > t) t = (double)N * K * 2.0 / rate;
+  return p.L + t;
+}
+
+static int choose_tile(int M, int N, int K, int num_cus) {
+  int kind = estimated_tile(M, N, K, num_cus);
+  if (kind <= TILE_128 && few_blocks_range(M, N, K))
+    for (int other = TILE_64; other <= TILE_128; ++other)
+      if (few_blocks_cost(other, M, N, K, num_cus, 1) < few_blocks_cost(kind, M, N, K, num_cus, 1)) kind = other;
+  return kind;
+}
+
+// The tile of a product that is written into the cache by heads of d: that, or where no head fits it the
+// estimates' (a head of 128 in a tile of 128 columns saves the kernel that rotates and writes).
+static int heads_tile(int M, int N, int K, int d, int num_cus) {
+  const int kind = choose_tile(M, N, K, num_cus);
+  return TILE_MODELS[kind].bn % d == 0 ? kind : estimated_tile(M, N, K, num_cus);
+}
+
 // The tile of a product that is neither cut into pieces nor written into the cache by heads (those need a
 // width that heads divide): the rule for few rows of a wide matrix, else the estimates.
 static int plain_tile(int M, int N, int K, int num_cus) {
   if (g_force_tile >= 134 && g_force_tile <= 137) return TILE_64x96 + (g_force_tile - 134);
   const int one_round = g_force_tile == 0 && !g_without_wide ? one_round_tile(M, N, K, num_cus) : -1;
-  return one_round >= 0 ? one_round : choose_tile(M, N, K, num_cus);
+  if (one_round >= 0) return one_round;
+  return choose_tile(M, N, K, num_cus);
 }
 // ... its width (for tests)
 extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
@@ -1595,7 +1789,7 @@ static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArg
   const TileModel& t = TILE_MODELS[kind];
   dim3 grid((N + t.bn - 1) / t.bn, (M + t.bm - 1) / t.bm, pieces);
   if (kind == TILE_64)
-    hipLaunchKernelGGL((gemm_bf16_tiled<64, 64, 64, 2, 2, EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
+    hipLaunchKernelGGL((gemm_bf16_ring<64, 64, 3, EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
   else if (kind == TILE_64x128)
     hipLaunchKernelGGL((gemm_bf16_tiled<64, 128, 64, 1, 4, EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
   else if (kind == TILE_128)
@@ -1739,6 +1933,18 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   // 15.8, 15.1 against 18.8 us; with more blocks than units it is the slower one)
   if (M <= 64 && best_pieces > 1 && g_force_tile == 0 && (long)((N + 63) / 64) * best_pieces <= num_cus)
     best_kind = TILE_64;
+  if (best_kind <= TILE_128 && few_blocks_range(M, N, K)) {
+    double least = few_blocks_cost(best_kind, M, N, K, num_cus, best_pieces) + (best_pieces > 1 ? best_pieces * piece : 0.0);
+    for (int kind = TILE_64; kind <= TILE_128; ++kind)
+      for (int s = 1; s <= max_pieces && (s == 1 || (nk + s - 1) / s >= min_tiles_per_piece); ++s) {
+        const double c = few_blocks_cost(kind, M, N, K, num_cus, s) + (s > 1 ? s * piece : 0.0);
+        if (c < least) {
+          least = c;
+          best_kind = kind;
+          best_pieces = s;
+        }
+      }
+  }
   out[0] = best_pieces;
   out[1] = best_kind;
 }
@@ -1771,7 +1977,7 @@ extern "C" int llmlab_linear_qkv(const void* x, const void* w, const void* bias,
   if (num_cus <= 0) num_cus = 256;
   EpiArgs e{q_out, bias, bias_dtype == DT_BF16, ldo, N, 0, 0, inv_freq, positions, row_req, table,
             (bf16_t*)kcache, (bf16_t*)vcache, table_stride, page_size, nq, nkv, d};
-  const int kind = choose_tile(M, N, K, num_cus);
+  const int kind = heads_tile(M, N, K, d, num_cus);
   LLMLAB_REQUIRE(TILE_MODELS[kind].bn % d == 0, "linear_qkv: heads of %d do not divide the tile of %d columns", d,
                  TILE_MODELS[kind].bn);
   launch_tile<EPI_QKV>(kind, (const bf16_t*)x, (const bf16_t*)w, e, M, N, K, 1, stream);
@@ -1779,11 +1985,15 @@ extern "C" int llmlab_linear_qkv(const void* x, const void* w, const void* bias,
   return 0;
 }
 
-// The width of the tile (64, 128 or 256 columns) that a product of these sizes gets: for
-// callers that must know whether a head fits it.
+// The width of the tile (64, 128 or 256 columns) that a product of these sizes gets (for tests) ...
 extern "C" int llmlab_linear_tile(int M, int N, int K, int num_cus) {
   if (num_cus <= 0) num_cus = 256;
   return TILE_MODELS[choose_tile(M, N, K, num_cus)].bn;
+}
+
+// ... and that llmlab_linear_qkv takes for heads of d: for callers that must know whether a head fits it.
+extern "C" int llmlab_linear_heads_tile(int M, int N, int K, int d, int num_cus) {
+  return TILE_MODELS[heads_tile(M, N, K, d > 0 ? d : 1, num_cus > 0 ? num_cus : 256)].bn;
 }
 
 // parts[z] = x[:, K_z] . W[:, K_z]^T for `ksplit` ranges K_z of the inner size (whole K

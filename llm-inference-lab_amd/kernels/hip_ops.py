@@ -245,8 +245,8 @@ class HipOps:
         c.llmlab_linear_qkv.argtypes = [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                         _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr,
                                         _c_int, _c_int, _c_int, _c_int, _c_ptr]
-        c.llmlab_linear_tile.argtypes = [_c_int, _c_int, _c_int, _c_int]
-        c.llmlab_linear_tile.restype = _c_int
+        c.llmlab_linear_heads_tile.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_int]
+        c.llmlab_linear_heads_tile.restype = _c_int
         c.llmlab_linear_partials.argtypes = [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                              _c_int, _c_int, _c_size, _c_int, _c_ptr]
         c.llmlab_qkv_from_pieces.argtypes = [_c_ptr, _c_int, _c_size, _c_int, _c_ptr, _c_int, _c_int, _c_int,
@@ -864,7 +864,7 @@ class HipOps:
                                                 or self._qkv_pieces_plan(rows, n, k) is not None):
             return True
         return (n is not None and k is not None
-                and self._core.llmlab_linear_tile(rows, n, k, self.num_cus) % head_dim == 0)
+                and self._core.llmlab_linear_heads_tile(rows, n, k, head_dim, self.num_cus) % head_dim == 0)
 
     def _qkv_pieces_plan(self, rows: int, n: int, k: int):
         """``(pieces, tile)`` if q/k/v of these sizes goes through pieces along the inner size

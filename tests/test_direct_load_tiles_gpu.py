@@ -1,5 +1,6 @@
-"""The tiles of two groups of waves: every length of the inner size at which their rings in LDS begin, wrap or
-end (pieces of x of two steps, steps of W, the last of them cut short), whole and in pieces."""
+"""The tiles whose operands come by direct loads into LDS (the two of two groups of waves, and 64 x 64): every length of
+the inner size at which their rings begin, wrap or end (pieces of x of two steps, steps of W, the last of them cut
+short), whole and in pieces."""
 import pytest
 import torch
 
@@ -15,7 +16,7 @@ def ops():
     return HipOps(DEV)
 
 
-@pytest.mark.parametrize("tile,m", [(132, 257), (132, 400), (133, 193), (133, 300)])
+@pytest.mark.parametrize("tile,m", [(132, 257), (132, 400), (133, 193), (133, 300), (64, 65), (64, 200)])
 @pytest.mark.parametrize("k", [8, 32, 56, 64, 72, 96, 128, 160, 192, 200, 224, 256, 352, 384, 392, 448, 776])
 def test_inner_sizes_around_the_rings(ops, tile, m, k):
     gen = torch.Generator(device=DEV).manual_seed(k)
