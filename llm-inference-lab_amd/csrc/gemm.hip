@@ -1728,21 +1728,24 @@ static int estimated_tile(int M, int N, int K, int num_cus) {
   return best;
 }
 
-// Up to 1,024 rows of a matrix of less than 32 MB (128 rows: 64 MB): among the three small tiles the
+// Up to 1,024 rows of a matrix of less than 32 MB (128 rows: 64 MB), where the blocks of the 64 x 128 tile find
+// two places a unit (with more, 512 rows of 9728 x 896, the estimates choose better): among the three small tiles the
 // estimates above lose 10 % on average (up to 42 %), because they count a block that has its unit to itself, whose
 // chain of K tiles is the time, like one of several that share it.  Here both are weighed: the chain of a block's K tiles, and
-// what a unit takes for all of its blocks.  Fitted to the same sweep (9 to 12 % rms), the pick then loses 2 %,
+// what a unit takes for all of its blocks.  Fitted to the same sweep (9 to 12 % rms; the two larger
+// tiles 5 and 10 % up, with which fewer picks are wrong), the pick then loses 1 %,
 // with the fold of the pieces: 512 rows of 896 x 4864 with the norm 17.8 us (64 x 64 in four pieces) against 24.7 (64 x 128 in six),
 // 700 of 2048 x 2048 15.8 against 22.5, 100 of 4608 x 3584 17.5 against 22.4.  Beyond that range the estimates above.
-static bool few_blocks_range(int M, int N, int K) {
+static bool few_blocks_range(int M, int N, int K, int num_cus) {
   const double bytes = (double)N * K * 2.0;
+  if ((long)((M + 63) / 64) * ((N + 127) / 128) > 2L * num_cus) return false;
   return g_force_tile == 0 && ((M <= 1024 && bytes < 32e6) || (M <= 128 && bytes < 64e6));
 }
 static double few_blocks_cost(int kind, int M, int N, int K, int num_cus, int pieces) {
   static const struct {
     double L, chain, f, tk, stream;
     int resident;
-  } fit[3] = {{3.10, 0.357, 0.76, 0.227, 30.0e3, 3}, {4.03, 0.482, 1.57, 0.358, 32.4e3, 2}, {2.13, 0.71, 4.25, 0.655, 25.7e3, 1}};
+  } fit[3] = {{3.10, 0.357, 0.76, 0.227, 30.0e3, 3}, {4.23, 0.506, 1.65, 0.376, 30.9e3, 2}, {2.34, 0.781, 4.68, 0.72, 23.4e3, 1}};
   const auto& p = fit[kind];
   const double blocks = (double)((M + TILE_MODELS[kind].bm - 1) / TILE_MODELS[kind].bm) *
                         ((N + TILE_MODELS[kind].bn - 1) / TILE_MODELS[kind].bn) * pieces;
@@ -1757,7 +1760,7 @@ static double few_blocks_cost(int kind, int M, int N, int K, int num_cus, int pi
 
 static int choose_tile(int M, int N, int K, int num_cus) {
   int kind = estimated_tile(M, N, K, num_cus);
-  if (kind <= TILE_128 && few_blocks_range(M, N, K))
+  if (kind <= TILE_128 && few_blocks_range(M, N, K, num_cus))
     for (int other = TILE_64; other <= TILE_128; ++other)
       if (few_blocks_cost(other, M, N, K, num_cus, 1) < few_blocks_cost(kind, M, N, K, num_cus, 1)) kind = other;
   return kind;
@@ -1933,7 +1936,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   // 15.8, 15.1 against 18.8 us; with more blocks than units it is the slower one)
   if (M <= 64 && best_pieces > 1 && g_force_tile == 0 && (long)((N + 63) / 64) * best_pieces <= num_cus)
     best_kind = TILE_64;
-  if (best_kind <= TILE_128 && few_blocks_range(M, N, K)) {
+  if (best_kind <= TILE_128 && few_blocks_range(M, N, K, num_cus)) {
     double least = few_blocks_cost(best_kind, M, N, K, num_cus, best_pieces) + (best_pieces > 1 ? best_pieces * piece : 0.0);
     for (int kind = TILE_64; kind <= TILE_128; ++kind)
       for (int s = 1; s <= max_pieces && (s == 1 || (nk + s - 1) / s >= min_tiles_per_piece); ++s) {
