@@ -1735,11 +1735,15 @@ static int estimated_tile(int M, int N, int K, int num_cus) {
 // what a unit takes for all of its blocks.  Fitted to the same sweep (9 to 12 % rms; the two larger
 // tiles 5 and 10 % up, with which fewer picks are wrong), the pick then loses 1 %,
 // with the fold of the pieces: 512 rows of 896 x 4864 with the norm 17.8 us (64 x 64 in four pieces) against 24.7 (64 x 128 in six),
-// 700 of 2048 x 2048 15.8 against 22.5, 100 of 4608 x 3584 17.5 against 22.4.  Beyond that range the estimates above.
-static bool few_blocks_range(int M, int N, int K, int num_cus) {
+// 700 of 2048 x 2048 15.8 against 22.5, 100 of 4608 x 3584 17.5 against 22.4 (2: all three are weighed).  Up to 2,560
+// rows of less than 16 MB and inner sizes to 2,048 (1) the 64 x 64 tile is weighed against the estimates' tile: 2048 rows of
+// 1152 x 896 12.0 against 13.7, of 896 x 896 9.4 against 10.6; of 896 x 4864 it would be taken whole, 33.3 us by itself against
+// 39.9 in two pieces with their fold, and inside a prompt's step be slower by 4 us a layer.  Beyond that (0) the estimates above.
+static int few_blocks_range(int M, int N, int K, int num_cus) {
   const double bytes = (double)N * K * 2.0;
-  if ((long)((M + 63) / 64) * ((N + 127) / 128) > 2L * num_cus) return false;
-  return g_force_tile == 0 && ((M <= 1024 && bytes < 32e6) || (M <= 128 && bytes < 64e6));
+  if (g_force_tile != 0 || (long)((M + 63) / 64) * ((N + 127) / 128) > 2L * num_cus) return 0;
+  if ((M <= 1024 && bytes < 32e6) || (M <= 128 && bytes < 64e6)) return 2;
+  return M <= 2560 && K <= 2048 && bytes < 16e6 ? 1 : 0;
 }
 static double few_blocks_cost(int kind, int M, int N, int K, int num_cus, int pieces) {
   static const struct {
@@ -1760,8 +1764,9 @@ static double few_blocks_cost(int kind, int M, int N, int K, int num_cus, int pi
 
 static int choose_tile(int M, int N, int K, int num_cus) {
   int kind = estimated_tile(M, N, K, num_cus);
-  if (kind <= TILE_128 && few_blocks_range(M, N, K, num_cus))
-    for (int other = TILE_64; other <= TILE_128; ++other)
+  const int range = kind <= TILE_128 ? few_blocks_range(M, N, K, num_cus) : 0;
+  if (range)
+    for (int other = TILE_64; other <= (range == 2 ? TILE_128 : TILE_64); ++other)
       if (few_blocks_cost(other, M, N, K, num_cus, 1) < few_blocks_cost(kind, M, N, K, num_cus, 1)) kind = other;
   return kind;
 }
@@ -1936,9 +1941,10 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   // 15.8, 15.1 against 18.8 us; with more blocks than units it is the slower one)
   if (M <= 64 && best_pieces > 1 && g_force_tile == 0 && (long)((N + 63) / 64) * best_pieces <= num_cus)
     best_kind = TILE_64;
-  if (best_kind <= TILE_128 && few_blocks_range(M, N, K, num_cus)) {
+  const int range = best_kind <= TILE_128 ? few_blocks_range(M, N, K, num_cus) : 0;
+  if (range) {
     double least = few_blocks_cost(best_kind, M, N, K, num_cus, best_pieces) + (best_pieces > 1 ? best_pieces * piece : 0.0);
-    for (int kind = TILE_64; kind <= TILE_128; ++kind)
+    for (int kind = TILE_64; kind <= (range == 2 ? TILE_128 : TILE_64x128); ++kind)
       for (int s = 1; s <= max_pieces && (s == 1 || (nk + s - 1) / s >= min_tiles_per_piece); ++s) {
         const double c = few_blocks_cost(kind, M, N, K, num_cus, s) + (s > 1 ? s * piece : 0.0);
         if (c < least) {
@@ -1947,6 +1953,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
           best_pieces = s;
         }
       }
+    if (best_pieces == 1) best_kind = estimated_tile(M, N, K, num_cus);      // (a whole product chooses its tile itself)
   }
   out[0] = best_pieces;
   out[1] = best_kind;
