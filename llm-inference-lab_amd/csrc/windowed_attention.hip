@@ -1086,17 +1086,26 @@ __global__ __launch_bounds__(256) void sink_window_attention_mfma_kernel(MfmaArg
 // pieces two tiles ahead and stores them a tile ahead), and the waves take their fragments from
 // there instead of each from L2.  Key rows lie 16 bytes apart from a
 // multiple of 256 bytes and the values' quad rows 128, so that the lanes of a read spread over the
-// banks.  Everything else (the list of tiles, masks, the running softmax, the transposed
-// products) is the kernel's above; all waves of a block walk the same tiles, so the barriers
-// are reached by all.
+// banks.  Two stages of LDS: the next tile is put down while this one is taken, a barrier a
+// tile.  The list of tiles, the masks and the transposed products are the kernel's above; all waves of
+// a block walk the same tiles, so the barriers are reached by all.
+//
+// What bounds it is the chain of a tile (scores, maximum, weights, product) of the block with the most
+// tiles, 34 to 64 of them one after the other, and its waits.  Page numbers come by scalar
+// loads a tile ahead: as vector loads they stood behind the keys and values in flight, and waiting for one was waiting for
+// all; the loads of keys and values have no branch.  1,900 rows over
+// 1,032 keys, 14 heads of 64: 50.5 -> 43.1 us, the same numbers to the bit.  (With the running maximum raised only where a
+// score exceeds it by 2^8 and a lane's weights summed by itself 40.0, but a model of sharp scores is then further off.)
 template <int DC, int EB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void sink_window_attention_shared_kernel(MfmaArgs a) {
   constexpr int D = 32 * DC, E = 16 * EB;
   constexpr int KROW = D + 8, VROW = 4 * E + 64;
   constexpr int KCHUNKS = 4 * D, VCHUNKS = 4 * E;            // 16-byte pieces of a tile's keys / values
   constexpr int KCH = (KCHUNKS + 255) / 256, VCH = (VCHUNKS + 255) / 256;
-  __shared__ __attribute__((aligned(16))) bf16_t ks[2 * 16 * KROW];
-  __shared__ __attribute__((aligned(16))) bf16_t vs[2 * 4 * VROW];
+  constexpr int KSTAGE = 2 * 16 * KROW, VSTAGE = 2 * 4 * VROW;
+  constexpr bool TWO = EB < 14;          // stages of LDS
+  __shared__ __attribute__((aligned(16))) bf16_t ks_all[(TWO ? 2 : 1) * KSTAGE];
+  __shared__ __attribute__((aligned(16))) bf16_t vs_all[(TWO ? 2 : 1) * VSTAGE];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g4 = lane >> 4, wave = tid >> 6;
   const int r0 = blockIdx.x * 16;
   if (r0 >= a.n_rows) return;
@@ -1121,6 +1130,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   const float bias = (sig && a.sink) ? a.sink[h] : 0.f;
   run.m = sig ? 0.f : (a.sink ? a.sink[h] : NEG_INF);
   run.l = (sig || a.sink) ? 1.f : 0.f;
+  // (pages are powers of two in use; any other size is divided by)
+  const int page_shift = (a.page_size & (a.page_size - 1)) == 0 ? __builtin_ctz(a.page_size) : -1;
+  auto page_of = [&](int j) { return page_shift >= 0 ? j >> page_shift : j / a.page_size; };
 #pragma unroll
   for (int eb = 0; eb < EB; ++eb) run.o[eb] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int b_first = __builtin_amdgcn_readfirstlane(a.row_req[r0]);
@@ -1134,46 +1146,63 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       p_lo = min(p_lo, __shfl_xor(p_lo, off, WAVE));
       p_hi = max(p_hi, __shfl_xor(p_hi, off, WAVE));
     }
+    // (the same in every lane: said so, that the tiles' bounds, page numbers and branches are scalar)
+    p_lo = __builtin_amdgcn_readfirstlane(p_lo);
+    p_hi = __builtin_amdgcn_readfirstlane(p_hi);
     if (p_hi < 0) continue;
     const KeyTiles kt(p_lo, p_hi, a.mask);
-    const int* pages = a.table + (size_t)b * a.max_pages;
+    // (the table is not written while the kernel runs: page numbers come by scalar loads, whose wait is not
+    // also one for the keys and values in flight)
+    const auto pages = (const __attribute__((address_space(4))) int*)(a.table + (size_t)b * a.max_pages);
     // Two sets of staging registers: a tile's pieces are asked for TWO tiles ahead and stored one
     // tile ahead, so that their way from memory lies behind the products of a whole tile and
     // more (the longest block's tiles, one after the other, are what a prompt's attention takes).
     bf16x8 k_a[KCH], v_a[VCH], k_b[KCH], v_b[VCH];
-    // the 16-byte pieces of tile t that this thread brings
+    // The pages of a tile's two halves are looked up one fetch ahead (a lookup in front of its own loads
+    // is a trip to memory that every tile would wait for).
+    int page[2];
+    auto look_up = [&](int t) {
+      const int j0 = t < kt.tiles_a ? 32 * t : kt.b_start + 32 * (t - kt.tiles_a);
+      const int end = t < kt.tiles_a ? kt.a_end : kt.end_b;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) page[u] = j0 + 16 * u < end ? pages[page_of(j0 + 16 * u)] : 0;
+    };
+    // the 16-byte pieces of tile t that this thread brings (tiles are fetched in their order)
     auto fetch = [&](int t, bf16x8 (&kreg)[KCH], bf16x8 (&vreg)[VCH]) {
       const int j0 = t < kt.tiles_a ? 32 * t : kt.b_start + 32 * (t - kt.tiles_a);
       const int end = t < kt.tiles_a ? kt.a_end : kt.end_b;
       size_t kbase[2], vbase[2];
-      bool have[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const int ju = j0 + 16 * u;
-        have[u] = ju < end;
-        kbase[u] = vbase[u] = 0;
-        if (have[u]) {
-          const int page = pages[ju / a.page_size];
-          const size_t head = ((size_t)page * a.n_kv + g) * a.page_size;
-          const int off = ju % a.page_size;
-          kbase[u] = (head + off) * D;
-          vbase[u] = head * E + (size_t)(off >> 2) * E * 4;
-        }
+        const size_t head = ((size_t)page[u] * a.n_kv + g) * a.page_size;
+        const int off = ju - page_of(ju) * a.page_size;
+        kbase[u] = (head + off) * D;
+        vbase[u] = head * E + (size_t)(off >> 2) * E * 4;
+      }
+      // Loads are unconditional (one under a branch makes the compiler wait for all in flight where it ends): a
+      // half that the tile does not have, and a piece past the last, are others again; their keys weigh zero.
+      if (j0 + 16 >= end) {
+        kbase[1] = kbase[0];
+        vbase[1] = vbase[0];
       }
 #pragma unroll
       for (int i = 0; i < KCH; ++i) {
-        const int idx = tid + 256 * i;
+        const int idx = min(tid + 256 * i, KCHUNKS - 1);
         const int u = idx / (2 * D), rem = idx % (2 * D);
-        kreg[i] = (idx < KCHUNKS && have[u & 1]) ? *(const bf16x8*)(a.k_cache + kbase[u & 1] + (size_t)rem * 8) : zero8;
+        kreg[i] = *(const bf16x8*)(a.k_cache + (u ? kbase[1] : kbase[0]) + (size_t)rem * 8);
       }
 #pragma unroll
       for (int i = 0; i < VCH; ++i) {
-        const int idx = tid + 256 * i;
+        const int idx = min(tid + 256 * i, VCHUNKS - 1);
         const int u = idx / (2 * E), rem = idx % (2 * E);
-        vreg[i] = (idx < VCHUNKS && have[u & 1]) ? *(const bf16x8*)(a.v_cache + vbase[u & 1] + (size_t)rem * 8) : zero8;
+        vreg[i] = *(const bf16x8*)(a.v_cache + (u ? vbase[1] : vbase[0]) + (size_t)rem * 8);
       }
+      if (t + 1 < kt.tiles) look_up(t + 1);
     };
-    auto stash = [&](const bf16x8 (&kreg)[KCH], const bf16x8 (&vreg)[VCH]) {
+    auto stash = [&](const bf16x8 (&kreg)[KCH], const bf16x8 (&vreg)[VCH], int stage) {
+      bf16_t* const ks = ks_all + stage * KSTAGE;
+      bf16_t* const vs = vs_all + stage * VSTAGE;
 #pragma unroll
       for (int i = 0; i < KCH; ++i) {
         const int idx = tid + 256 * i;
@@ -1194,7 +1223,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       }
     };
     // tile t, which lies in LDS, into the running softmax
-    auto attend = [&](int t) {
+    auto attend = [&](int t, int stage) {
+      const bf16_t* const ks = ks_all + stage * KSTAGE;
+      const bf16_t* const vs = vs_all + stage * VSTAGE;
       const int j0 = t < kt.tiles_a ? 32 * t : kt.b_start + 32 * (t - kt.tiles_a);
       const int end = t < kt.tiles_a ? kt.a_end : kt.end_b;
       const bool have1 = j0 + 16 < end;
@@ -1232,30 +1263,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       }
       float corr = 1.f;
       bf16x8 pf;
-      if (a.mode == MODE_SIGMOID) {
+      if (sig) {
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int i = 0; i < 4; ++i) pf[4 * u + i] = (bf16_t)sigmoid_weight(s[u][i] + bias);      // (masked: -inf -> 0)
       } else {
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-      const float m_new = fmaxf(run.m, tmax);
-      const float m_use = m_new == NEG_INF ? 0.f : m_new;
-      corr = run.m == NEG_INF ? 0.f : __expf(run.m - m_use);
-      float sum = 0.f;
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+        const float m_new = fmaxf(run.m, tmax);
+        const float m_use = m_new == NEG_INF ? 0.f : m_new;
+        corr = run.m == NEG_INF ? 0.f : __expf(run.m - m_use);
+        float sum = 0.f;
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p = __expf(s[u][i] - m_use);       // (exp(-inf) = 0 for a masked key)
-          sum += p;
-          pf[4 * u + i] = (bf16_t)p;
-        }
-      sum += __shfl_xor(sum, 16, WAVE);
-      sum += __shfl_xor(sum, 32, WAVE);
-      run.l = run.l * corr + sum;
-      run.m = m_new;
+          for (int i = 0; i < 4; ++i) {
+            const float p = __expf(s[u][i] - m_use);       // (exp(-inf) = 0 for a masked key)
+            sum += p;
+            pf[4 * u + i] = (bf16_t)p;
+          }
+        sum += __shfl_xor(sum, 16, WAVE);
+        sum += __shfl_xor(sum, 32, WAVE);
+        run.l = run.l * corr + sum;
+        run.m = m_new;
       }
 #pragma unroll
       for (int eb = 0; eb < EB; ++eb) {
@@ -1273,24 +1304,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     };
     const int T = kt.tiles;
     __syncthreads();                                  // (the request before this one has been read)
+    look_up(0);
     fetch(0, k_a, v_a);
-    stash(k_a, v_a);
-    __syncthreads();
-    if (T > 1) fetch(1, k_a, v_a);
-    for (int t = 0; t < T; t += 2) {
-      // tile t lies in LDS, tile t + 1 is on its way into set a
-      if (t + 2 < T) fetch(t + 2, k_b, v_b);
-      attend(t);
-      __syncthreads();                                // (every wave has read the tile)
-      if (t + 1 < T) stash(k_a, v_a);
-      __syncthreads();
-      if (t + 1 >= T) break;
-      // tile t + 1 lies in LDS, tile t + 2 is on its way into set b
-      if (t + 3 < T) fetch(t + 3, k_a, v_a);
-      attend(t + 1);
-      __syncthreads();
-      if (t + 2 < T) stash(k_b, v_b);
-      __syncthreads();
+    stash(k_a, v_a, 0);
+    if constexpr (TWO) {
+      if (T > 1) fetch(1, k_a, v_a);
+      if (T > 2) fetch(2, k_b, v_b);
+      for (int t = 0; t < T; t += 2) {
+        // tile t lies in stage 0, tiles t + 1 and t + 2 are on their way into sets a and b
+        __syncthreads();                              // (tile t is whole, tile t - 1 has been read)
+        if (t + 1 < T) stash(k_a, v_a, 1);
+        if (t + 3 < T) fetch(t + 3, k_a, v_a);
+        attend(t, 0);
+        if (t + 1 >= T) break;
+        __syncthreads();
+        if (t + 2 < T) stash(k_b, v_b, 0);
+        if (t + 4 < T) fetch(t + 4, k_b, v_b);
+        attend(t + 1, 1);
+      }
+    } else {
+      // (values of 224 and more: the registers hold one tile on its way, and it is put down when the one
+      // before has been taken, which for such heads takes longer than the way)
+      for (int t = 0; t < T; ++t) {
+        __syncthreads();                              // (tile t is whole)
+        if (t + 1 < T) fetch(t + 1, k_a, v_a);
+        attend(t, 0);
+        __syncthreads();                              // (every wave has read it)
+        if (t + 1 < T) stash(k_a, v_a, 0);
+      }
     }
   }
   if (!row_ok || !head_ok) return;
