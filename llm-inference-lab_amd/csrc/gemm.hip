@@ -1578,7 +1578,12 @@ static int g_force_tile = 0, g_without_wide = 0, g_pp_min_rows = 512;
 // tokens of five shapes that is between 1.4 % faster and 1.3 % slower than from 2,048 on.)
 constexpr int WIDE_TILE_MIN_ROWS = 2048;
 constexpr int PP_MIN_INNER = 896;      // the shortest inner size the estimates of those tiles were fitted to
-constexpr int PP_MAX_INNER = 1 << 22;  // their loads address a tile's rows by 32 bits of bytes
+// The tiles by direct loads address a tile's rows by 32 bits of bytes, which hold 255 rows (and 15 strips of
+// W) of this inner size; beyond, the 64 x 128 tile, whose addresses have 64.
+constexpr int DIRECT_MAX_INNER = 1 << 22;
+static int addressable(int kind, int K) {
+  return K > DIRECT_MAX_INNER && (kind == TILE_64 || kind == TILE_256 || kind == TILE_192) ? TILE_64x128 : kind;
+}
 extern "C" void llmlab_debug_gemm_tile(int tile) {
   g_force_tile = tile > 0 ? tile : 0;
   g_without_wide = tile == -131;
@@ -1649,12 +1654,12 @@ static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int mi
 }
 
 static int estimated_tile(int M, int N, int K, int num_cus) {
-  if (g_force_tile == 64) return TILE_64;
+  if (g_force_tile == 64) return addressable(TILE_64, K);
   if (g_force_tile == 130) return TILE_64x128;
   if (g_force_tile == 129 || g_force_tile == 128) return TILE_128;
   if (g_force_tile == 131) return TILE_128x256;
-  if (g_force_tile == 132 && K <= PP_MAX_INNER) return TILE_256;
-  if (g_force_tile == 133 && K <= PP_MAX_INNER) return TILE_192;
+  if (g_force_tile == 132) return addressable(TILE_256, K);
+  if (g_force_tile == 133) return addressable(TILE_192, K);
   // One or two tiles of rows of a wide matrix (the head, gate and up at larger shapes):
   // bound by the read of W, which the wider tiles stream better than the estimate
   // knows, and the 128-row tile reads W once where two 64-row tiles read it twice
@@ -1712,7 +1717,7 @@ static int estimated_tile(int M, int N, int K, int num_cus) {
   // chip (192 / 256 / 384 rows of 55296 x 5120: 153 / 171 / 261 us against 187 / 199 / 274 with the
   // best of the others; of 59136 x 8192: 229 / 263 / 392 against 305 / 316 / 437)
   const bool pp_rows = M >= g_pp_min_rows || (g_pp_min_rows == 512 && M > 128 && N >= 16384);
-  if (pp_rows && K >= PP_MIN_INNER && K <= PP_MAX_INNER && !g_without_wide) {
+  if (pp_rows && K >= PP_MIN_INNER && K <= DIRECT_MAX_INNER && !g_without_wide) {
     // (the estimates of the other tiles, fitted at shorter inner sizes, are up to a quarter low from
     // 3,584 on (and 512 rows): 4096 rows of 1536 x 8960 129 us against 147 with their pick, 2048 of 3584 x 18944 268 against 301,
     // 2367 of 2048 x 11008 154 against 181; over 126 products the picks then lose 0.1 % on average)
@@ -1725,7 +1730,7 @@ static int estimated_tile(int M, int N, int K, int num_cus) {
       }
     }
   }
-  return best;
+  return addressable(best, K);
 }
 
 // Up to 1,024 rows of a matrix of less than 32 MB (128 rows: 64 MB), where the blocks of the 64 x 128 tile find
@@ -1768,7 +1773,7 @@ static int choose_tile(int M, int N, int K, int num_cus) {
   if (range)
     for (int other = TILE_64; other <= (range == 2 ? TILE_128 : TILE_64); ++other)
       if (few_blocks_cost(other, M, N, K, num_cus, 1) < few_blocks_cost(kind, M, N, K, num_cus, 1)) kind = other;
-  return kind;
+  return addressable(kind, K);
 }
 
 // The tile of a product that is written into the cache by heads of d: that, or where no head fits it the
@@ -1794,6 +1799,7 @@ extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
 template <int EPI>
 static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArgs& e, int M, int N, int K,
                         int pieces, hipStream_t stream) {
+  kind = addressable(kind, K);             // (a tile that the caller names)
   const TileModel& t = TILE_MODELS[kind];
   dim3 grid((N + t.bn - 1) / t.bn, (M + t.bm - 1) / t.bm, pieces);
   if (kind == TILE_64)
@@ -1912,7 +1918,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   for (int kind = TILE_64x128; kind < TILE_KINDS; ++kind) {
     if (kind == TILE_128x256) continue;
     if (one_tile_of_128 && kind != TILE_128) continue;
-    if (kind >= TILE_256 && !(M >= g_pp_min_rows && K >= PP_MIN_INNER && K <= PP_MAX_INNER && !g_without_wide)) continue;
+    if (kind >= TILE_256 && !(M >= g_pp_min_rows && K >= PP_MIN_INNER && K <= DIRECT_MAX_INNER && !g_without_wide)) continue;
     if (g_force_tile != 0 && kind != choose_tile(M, N, K, num_cus)) continue;
     for (int s = 2; s <= max_pieces; ++s) {
       if ((nk + s - 1) / s < min_tiles_per_piece) break;
@@ -1956,7 +1962,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
     if (best_pieces == 1) best_kind = estimated_tile(M, N, K, num_cus);      // (a whole product chooses its tile itself)
   }
   out[0] = best_pieces;
-  out[1] = best_kind;
+  out[1] = addressable(best_kind, K);
 }
 
 // The same for a float32 product (of more rows than the few-row kernel takes).

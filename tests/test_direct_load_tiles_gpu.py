@@ -33,3 +33,25 @@ def test_inner_sizes_around_the_rings(ops, tile, m, k):
             parts = torch.zeros(count, m, 530, device=DEV)
             ops.linear_partials(x, pw, parts, count)
             assert bool(((parts.double().sum(0) - want).abs() <= unit).all())
+
+
+def test_an_inner_size_beyond_their_addresses(ops):
+    """65 rows of 34,087,048 (4.4 GB; the 64 rows of a tile span more bytes than 32 bits address): rows that are zero but
+    for a few numbers, whose product is that of those columns."""
+    m, n, k = 65, 16, 34_087_048
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    w = torch.randn(n, k, device=DEV, generator=gen).to(BF)
+    at = torch.tensor([0, 33, k // 2 + 1, k - 9, k - 1], device=DEV)
+    x = torch.zeros(m, k, device=DEV, dtype=BF)
+    x[:, at] = torch.randn(m, 5, device=DEV, generator=gen).to(BF)
+    want = x[:, at].double() @ w[:, at].double().T
+    unit = 8 * 2.0 ** -24 * (x[:, at].double().abs() @ w[:, at].double().abs().T + 1)
+    pw = ops.prepare_weight(w)
+    out = torch.empty(m, n, device=DEV)
+    ops.linear_logits(x, pw, out)
+    assert bool(((out.double() - want).abs() <= unit).all())
+    for tile in (0, 4):                    # (kinds named by the caller)
+        parts = torch.zeros(2, m, n, device=DEV)
+        ops._call(ops._core.llmlab_linear_partials, x.data_ptr(), pw.data_ptr(), 1, parts.data_ptr(), None, 0, m, n, k, n,
+                  2, m * n, tile, ops._stream())
+        assert bool(((parts.double().sum(0) - want).abs() <= unit).all()), tile

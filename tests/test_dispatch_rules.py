@@ -137,6 +137,25 @@ def test_one_round_of_blocks_is_one_round(core):
     assert differs > 300
 
 
+@pytest.mark.parametrize("m", [1, 65, 200, 600, 2048])
+@pytest.mark.parametrize("k", [2 ** 22 + 8, 34_087_048, 40_000_000])
+def test_inner_sizes_beyond_the_addresses_of_direct_loads(core, m, k):
+    """The 64 x 64 tile and the two of two groups of waves address a tile's rows by 32 bits of bytes (63 rows of
+    34,087,042 numbers wrap): beyond their limit nothing is given to them, whether estimated, cut or named."""
+    direct = (0, 4, 5)
+    for n in (7, 16, 896):
+        assert core.llmlab_linear_tile(m, n, k, CUS) in (128,) and core.llmlab_plain_tile(m, n, k, CUS) in (128,)
+        assert core.llmlab_linear_heads_tile(m, n, k, 64, CUS) == 128
+        assert plan(core, m, n, k)[1] not in direct and plan(core, m, n, k, 1)[1] not in direct
+        for tile in (64, 132, 133):
+            core.llmlab_debug_gemm_tile(tile)
+            try:
+                assert core.llmlab_linear_tile(m, n, k, CUS) == 128 and plan(core, m, n, k)[1] not in direct
+                assert core.llmlab_linear_tile(m, n, 2 ** 22, CUS) == (64 if tile == 64 else 256)
+            finally:
+                core.llmlab_debug_gemm_tile(0)
+
+
 def test_block_shapes_of_products_of_few_rows(core):
     rng = random.Random(6)
     out = (ctypes.c_int * 5)()
