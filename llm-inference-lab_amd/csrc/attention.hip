@@ -91,7 +91,8 @@ struct AttnArgs {
   int qlen_lo, qlen_hi;  // only requests that bring so many tokens are worked on (a step may be
                          // served by two launches: its short requests by one, its long ones by the other)
   int reqs, picked;   // picked > 0: block z of the launch is for the z-th of the `reqs` requests that bring
-                      // so many tokens, of which there are `picked`
+                      // so many tokens, of which there are `picked`; 0: block z is for request z, and ends at
+                      // once if that brings another number of tokens
   float scale;
 };
 
@@ -817,7 +818,7 @@ __global__ __launch_bounds__(DECODE ? 64 * DECODE_WAVES : 256 * PH, (!DECODE && 
 template <int QBL, int RL, int RS>
 __global__ __launch_bounds__(64 * DECODE_WAVES) void attention_bf16_mixed_kernel(AttnArgs al, AttnArgs as, int long_tiles) {
   __shared__ __attribute__((aligned(16))) float dlds[decode_lds_floats<QBL>()];
-  const int x = (int)blockIdx.x, per_long = long_tiles * al.nkv, longs = per_long * al.picked;
+  const int x = (int)blockIdx.x, per_long = long_tiles * al.nkv, longs = per_long * (al.picked > 0 ? al.picked : al.reqs);
   if (x < longs) {
     const int at = x % per_long, b = request_of(al, x / per_long);
     if (b >= 0) attention_tile<QBL, true, RL>(al, long_tiles - 1 - at / al.nkv, at % al.nkv, b, dlds);
@@ -1341,7 +1342,7 @@ static int choose_many_rows_launch_f32(long blocks, int max_q_len, int max_ctx_l
 
 static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx_len, int window, int total_rows,
                                 float* workspace, size_t workspace_floats, int num_cus, const int* row_req,
-                                int short_len, int n_short, int short_ctx, hipStream_t stream) {
+                                int short_len, int n_short, int short_ctx, bool counted, hipStream_t stream) {
   LLMLAB_REQUIRE(a.q_stride % 4 == 0 && a.out_stride % 4 == 0 && ((uintptr_t)a.q % 16 == 0) &&
                  ((uintptr_t)a.out % 16 == 0) && ((uintptr_t)a.kc % 16 == 0) && ((uintptr_t)a.vc % 16 == 0),
                  "attention(float32): operands are not aligned for 16-byte loads");
@@ -1359,8 +1360,10 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
                                         workspace_floats, num_cus, row_req, stream);
     if (rc) return rc;
     a.qlen_lo = short_len + 1;
-    a.picked = live = reqs - n_short;
+    live = reqs - n_short;
+    a.picked = counted ? live : 0;
   }
+  const unsigned zs = a.picked > 0 ? a.picked : reqs;
   constexpr int ROWS = 16 * F32_QB;
   const long tiles = (max_rows + ROWS - 1) / ROWS;
   // Which launch, from a sweep of 1 to 32 requests of 64 to 8,192 tokens behind 0 to 4,096 keys
@@ -1373,10 +1376,10 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
   // keys (4 requests of 256 tokens: 58 against 81).
   const int path = choose_many_rows_launch_f32(tiles * a.nkv * live, max_q_len, max_ctx_len, num_cus, g_force_path);
   if (path == 1) {
-    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, true, F32_SPLIT_WAVES>), dim3((unsigned)tiles, a.nkv, live),
+    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, true, F32_SPLIT_WAVES>), dim3((unsigned)tiles, a.nkv, zs),
                        dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
   } else {
-    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, false, 4>), dim3((unsigned)((tiles + 3) / 4), a.nkv, live),
+    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, false, 4>), dim3((unsigned)((tiles + 3) / 4), a.nkv, zs),
                        dim3(256), 0, stream, a);
   }
   LLMLAB_LAUNCH_CHECK("attention(float32)");
@@ -1526,7 +1529,10 @@ extern "C" int llmlab_attention_launch(int dtype, int nq, int nkv, int reqs, int
 // among those is short_ctx, and row_req[row] is the request of a row.  Its short
 // requests are then served by the decode-like launch and the others by the tiled one;
 // in one launch the few rows of a decoding request would walk its whole history in
-// one wave while the rest of the chip waits.
+// one wave while the rest of the chip waits.  n_short shapes the launches; with `counted` the
+// caller also stands for it being the number of such requests in q_start, as it does for max_q_len, and the
+// launches have blocks for so many requests of either kind and no more (a request beyond would keep its rows
+// unwritten).  Without, they have blocks for every request, and any n_short gives the same results.
 extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, int nq, int nkv,
                                       const void* kcache, const void* vcache, const int* table,
                                       int table_stride, int page_size, const int* q_start,
@@ -1534,7 +1540,8 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
                                       int window, float scale, void* out, int out_stride,
                                       float* workspace, size_t workspace_floats, int total_rows,
                                       int num_cus, const int* row_req, int short_len, int n_short,
-                                      int short_ctx, int* arrived, size_t arrived_ints, hipStream_t stream) {
+                                      int short_ctx, int counted, int* arrived, size_t arrived_ints,
+                                      hipStream_t stream) {
   LLMLAB_REQUIRE(nq > 0 && nkv > 0 && nq % nkv == 0, "attention: %d heads, %d kv heads", nq, nkv);
   LLMLAB_REQUIRE(page_size >= 16 && (page_size & (page_size - 1)) == 0,
                  "attention: page size %d is not a power of two >= 16", page_size);
@@ -1558,7 +1565,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
   while ((1 << a.page_shift) < page_size) ++a.page_shift;
   if (dtype == DT_F32)
     return launch_attention_f32(a, reqs, max_q_len, max_ctx_len, window, total_rows, workspace, workspace_floats,
-                                num_cus, row_req, short_len, n_short, short_ctx, stream);
+                                num_cus, row_req, short_len, n_short, short_ctx, counted != 0, stream);
   LLMLAB_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16 == 0) && out_stride % 4 == 0 &&
                  ((uintptr_t)out % 8 == 0) && ((uintptr_t)kcache % 16 == 0) && ((uintptr_t)vcache % 16 == 0),
                  "attention(bfloat16): operands are not aligned for vector loads");
@@ -1577,20 +1584,25 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     shorts = prepare_key_split_decode(s, reqs, n_short, short_ctx, window, total_rows, nq, nkv, workspace,
                                       workspace_floats, num_cus, arrived, arrived_ints);
     a.qlen_lo = short_len + 1;
-    a.picked = live = reqs - n_short;
+    live = reqs - n_short;
+    if (counted) {
+      a.picked = live;
+      shorts.a.picked = n_short;         // (read where both kinds share a launch)
+    }
   }
+  const int zs = a.picked > 0 ? a.picked : reqs, short_zs = shorts.a.picked > 0 ? n_short : reqs;
+  // (a launch of both kinds has them all along x, which takes less than 2^32 threads)
+  auto mixed_blocks = [&](long long_tiles) { return long_tiles * nkv * zs + (long)nkv * shorts.a.splits * short_zs; };
+  constexpr long MOST_BLOCKS = 0xffffffffl / (64 * DECODE_WAVES);
   const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, g_force_path);
   const int steps32 = (max_ctx_len + 31) / 32 + 1;
   const int steps_per_wave = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;
-  if (mixed && g_force_path == 0 && g_force_two_launches == 0 &&
+  if (mixed && g_force_path == 0 && g_force_two_launches == 0 && mixed_blocks((max_rows + 15) / 16) <= MOST_BLOCKS &&
       mixed_step_by_small_tiles((max_rows + 15) / 16 * nkv * live, (max_rows + 31) / 32 * nkv * live,
                                 (long)nkv * shorts.a.splits * n_short, shorts.ring,
                                 steps_per_wave > 2 || shorts.ring == 2, path, max_ctx_len, num_cus)) {
     const int tiles16 = (int)((max_rows + 15) / 16);
-    shorts.a.picked = n_short;
-    const long gx = (long)tiles16 * nkv * live + (long)nkv * shorts.a.splits * n_short;
-    LLMLAB_REQUIRE(gx <= 0x7fffffffL, "attention: grid too large");
-    hipLaunchKernelGGL((attention_bf16_mixed_kernel<1, 1, 1>), dim3((unsigned)gx), dim3(64 * DECODE_WAVES), 0, stream, a,
+    hipLaunchKernelGGL((attention_bf16_mixed_kernel<1, 1, 1>), dim3((unsigned)mixed_blocks(tiles16)), dim3(64 * DECODE_WAVES), 0, stream, a,
                        shorts.a, tiles16);
     LLMLAB_LAUNCH_CHECK("attention(bfloat16, mixed, tiles of 16 rows)");
     return launch_split_merge(shorts, total_rows, nq, row_req, out, out_stride, stream);
@@ -1610,7 +1622,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     // 1,024: 68 against 59, hence not there.  Heads of 128, 128 tokens beside 63 at 2,048: 75
     // against 90.
     const int long_tiles = (int)((max_rows + 31) / 32);
-    const bool one_launch = mixed && mixed_step_in_one_launch((long)long_tiles * nkv * live,
+    const bool one_launch = mixed && mixed_blocks(long_tiles) <= MOST_BLOCKS && mixed_step_in_one_launch((long)long_tiles * nkv * live,
                                                               (long)nkv * shorts.a.splits * n_short, num_cus,
                                                               g_force_two_launches);
     if (mixed && !one_launch) {
@@ -1618,10 +1630,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
       if (rc) return rc;
     }
     if (one_launch) {
-      shorts.a.picked = n_short;
-      const long gx = (long)long_tiles * nkv * live + (long)nkv * shorts.a.splits * n_short;
-      LLMLAB_REQUIRE(gx <= 0x7fffffffL, "attention: grid too large");
-      dim3 mgrid((unsigned)gx), mblock(64 * DECODE_WAVES);
+      dim3 mgrid((unsigned)mixed_blocks(long_tiles)), mblock(64 * DECODE_WAVES);
       const bool deep = steps_per_wave > 2;
       if (deep && shorts.ring == 2)
         hipLaunchKernelGGL((attention_bf16_mixed_kernel<2, 2, 2>), mgrid, mblock, 0, stream, a, shorts.a, long_tiles);
@@ -1634,7 +1643,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
       LLMLAB_LAUNCH_CHECK("attention(bfloat16, mixed)");
       return launch_split_merge(shorts, total_rows, nq, row_req, out, out_stride, stream);
     }
-    dim3 grid((unsigned)((max_rows + 31) / 32), nkv, live), block(64 * DECODE_WAVES);
+    dim3 grid((unsigned)((max_rows + 31) / 32), nkv, zs), block(64 * DECODE_WAVES);
     if (steps_per_wave > 2)
       hipLaunchKernelGGL((attention_bf16_kernel<2, true, 2>), grid, block, 0, stream, a);
     else
@@ -1643,25 +1652,25 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     return 0;
   }
   if (path == 2) {
-    dim3 grid((unsigned)((max_rows + 127) / 128), nkv, live), block(256);
+    dim3 grid((unsigned)((max_rows + 127) / 128), nkv, zs), block(256);
     hipLaunchKernelGGL((attention_bf16_kernel<2, false>), grid, block, 0, stream, a);
   } else if (path == 5) {
     if constexpr (TWO_GROUPS) {
       a.tiles = (int)((max_rows + 63) / 64);
-      dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, live), block(512);
+      dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, zs), block(512);
       hipLaunchKernelGGL((attention_bf16_paired_kernel<1, 2>), grid, block, 0, stream, a);
     }
   } else if (path == 6) {
     if constexpr (TWO_GROUPS) {
-      dim3 grid((unsigned)((max_rows + 63) / 64), nkv, live), block(512);
+      dim3 grid((unsigned)((max_rows + 63) / 64), nkv, zs), block(512);
       hipLaunchKernelGGL((attention_bf16_kernel<1, false, 1, 2>), grid, block, 0, stream, a);
     }
   } else if (path == 3) {
     a.tiles = (int)((max_rows + 63) / 64);
-    dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, live), block(256);
+    dim3 grid((unsigned)((a.tiles + 1) / 2), nkv, zs), block(256);
     hipLaunchKernelGGL((attention_bf16_paired_kernel<1>), grid, block, 0, stream, a);
   } else {
-    dim3 grid((unsigned)((max_rows + 63) / 64), nkv, live), block(256);
+    dim3 grid((unsigned)((max_rows + 63) / 64), nkv, zs), block(256);
     hipLaunchKernelGGL((attention_bf16_kernel<1, false>), grid, block, 0, stream, a);
   }
   LLMLAB_LAUNCH_CHECK("attention(bfloat16, prefill)");

@@ -16,7 +16,7 @@ from typing import Dict, Optional
 import torch
 
 from ..config.errors import UnsupportedSizeError
-from ..parts.base import ChosenSums, PendingSums
+from ..parts.base import ChosenSums, PendingSums, ShortRequests
 from . import build
 from .debug import DispatchRules, KernelDebug
 
@@ -149,7 +149,7 @@ class AttentionCall:
     (``HipOps.prepare_attention``)."""
 
     __slots__ = ("ops", "lib", "args", "most_requests", "most_context", "row_req", "heads", "dtype")
-    N_REQS, MAX_Q, MAX_CTX, ROW_REQ, SHORT_LEN, N_SHORT, SHORT_CTX, STREAM = 12, 13, 14, 23, 24, 25, 26, 29
+    N_REQS, MAX_Q, MAX_CTX, ROW_REQ, SHORT_LEN, N_SHORT, SHORT_CTX, COUNTED, STREAM = 12, 13, 14, 23, 24, 25, 26, 27, 30
 
     def __init__(self, ops, lib, args, most_requests, most_context, row_req, heads, dtype):
         self.ops, self.lib, self.args = ops, lib, args
@@ -171,6 +171,7 @@ class AttentionCall:
             a[self.ROW_REQ], a[self.SHORT_LEN], a[self.N_SHORT], a[self.SHORT_CTX] = self.row_req, short_len, n_short, short_ctx
         else:
             a[self.ROW_REQ], a[self.SHORT_LEN], a[self.N_SHORT], a[self.SHORT_CTX] = None, 0, 0, 0
+        a[self.COUNTED] = int(isinstance(short, ShortRequests))
         a[self.STREAM] = self.ops._stream()
         self.ops._call(self.lib.llmlab_paged_attention, *a, lib=self.lib)
 
@@ -192,7 +193,7 @@ class HipOps:
             self.device = torch.device("cuda", torch.cuda.current_device())
         self._core = self._load(build.core_library())
         self._declare_core()
-        if self._core.llmlab_abi_version() != 10:
+        if self._core.llmlab_abi_version() != 11:
             raise RuntimeError("kernel library and Python bindings disagree on the interface")
         self._attn: Dict[int, ctypes.CDLL] = {}
         self._mixer_libs: Dict[str, ctypes.CDLL] = {}
@@ -294,7 +295,7 @@ class HipOps:
             lib.llmlab_paged_attention.argtypes = [
                 _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr,
                 _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr, _c_int, _c_ptr, _c_size,
-                _c_int, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_size, _c_ptr]
+                _c_int, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_size, _c_ptr]
             lib.llmlab_paged_attention.restype = _c_int
             self._attn[head_dim] = lib
             self.loaded_libraries.append(lib._name)
@@ -1021,7 +1022,7 @@ class HipOps:
                         out, short=None) -> None:
         """``short``: ``(row_req, limit, count, longest)`` for a step in which ``count`` of the
         requests (not all) bring at most ``limit = attention_short_limit(...)`` tokens, the
-        longest context among those being ``longest``."""
+        longest context among those being ``longest`` (or what ``ShortRequests.count`` gives)."""
         self.prepare_attention(qkv, num_heads, num_kv_heads, head_dim, k_cache, v_cache, block_table, page_size,
                                q_start, start_pos, window, scale, out,
                                short[0] if short is not None else None).launch(n_reqs, max_q_len, max_ctx_len, short)
@@ -1063,7 +1064,7 @@ class HipOps:
                 self._ptr(q_start), self._ptr(start_pos), 0, 0, 0,
                 int(window) if window else 0, float(scale), self._ptr(out), out.stride(0) if rows > 1 else
                 out.shape[1], self._ptr(self.workspace), self.workspace.numel(), rows, self.num_cus,
-                None, 0, 0, 0, self._ptr(self.arrived), self.arrived.numel(), None]
+                None, 0, 0, 0, 0, self._ptr(self.arrived), self.arrived.numel(), None]
         return AttentionCall(self, lib, args, most_requests=min(q_start.numel() - 1, start_pos.numel(), block_table.shape[0]),
                              most_context=block_table.shape[1] * page_size, row_req=self._ptr(row_req),
                              heads=(num_heads, num_kv_heads), dtype=qkv.dtype)

@@ -8,7 +8,7 @@ import torch
 
 from ..config.spec import PartSpec
 from ..weights.loader import TensorSpec, MATRIX, VECTOR, INIT_NORM
-from .base import Mixer, KVCacheSpec, CacheSpec, PageTensor, NormedInput, PendingSums, pieces_buffer, project_normed
+from .base import Mixer, KVCacheSpec, CacheSpec, PageTensor, NormedInput, PendingSums, ShortRequests, pieces_buffer, project_normed
 from .registry import register_part, build_part
 
 
@@ -248,13 +248,7 @@ class GQAAttention(Mixer):
             return None
         key = ("attention.short", limit)
         if key not in ctx.memo:
-            count = longest = 0
-            for b in range(ctx.n_reqs):
-                n = ctx.host_q_start[b + 1] - ctx.host_q_start[b]
-                if n <= limit:
-                    count += 1
-                    longest = max(longest, ctx.host_start_pos[b] + n)
-            ctx.memo[key] = (ctx.row_req, limit, count, longest) if 0 < count < ctx.n_reqs else None
+            ctx.memo[key] = ShortRequests.count(ctx.row_req, limit, ctx.host_q_start, ctx.host_start_pos, ctx.n_reqs)
         return ctx.memo[key]
 
     @property

@@ -12,7 +12,7 @@ arguments.  No part knows which model it is in.
 from __future__ import annotations
 
 import dataclasses
-from typing import Dict, Optional, Tuple
+from typing import Dict, NamedTuple, Optional, Tuple
 
 import torch
 
@@ -180,6 +180,28 @@ class PendingSums:
 
     def __init__(self, parts: torch.Tensor, splits: int):
         self.parts, self.splits = parts, int(splits)
+
+
+class ShortRequests(NamedTuple):
+    """The short requests of a mixed step as ``ShortRequests.count`` finds them in the step's own lists.  A plain
+    tuple of the same four says the same, but its count only shapes the launches; this one's is taken for the truth,
+    and the launches have blocks for so many requests of either kind and no more."""
+    row_req: object
+    limit: int
+    requests: int
+    longest: int
+
+    @classmethod
+    def count(cls, row_req, limit: int, q_start, start_pos, n_reqs: int) -> Optional["ShortRequests"]:
+        """Of the ``n_reqs`` requests whose rows start at ``q_start`` (host numbers, one more than requests) behind
+        ``start_pos`` keys, those that bring at most ``limit`` tokens; None if none or all do."""
+        requests = longest = 0
+        for b in range(n_reqs):
+            n = q_start[b + 1] - q_start[b]
+            if n <= limit:
+                requests += 1
+                longest = max(longest, start_pos[b] + n)
+        return cls(row_req, limit, requests, longest) if 0 < requests < n_reqs else None
 
 
 def pieces_buffer(ctx, name: str, shape) -> Optional[torch.Tensor]:

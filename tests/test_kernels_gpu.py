@@ -8,6 +8,7 @@ import torch
 
 from emu_ops import EmuOps
 from llm_inference_lab_amd.cache import layout as cache_layout
+from llm_inference_lab_amd.parts.base import ShortRequests
 
 pytestmark = pytest.mark.gpu
 
@@ -680,12 +681,13 @@ def run_attention(ops, emu, dtype, nq, nkv, d, page, window, reqs_spec, seed=30,
     if 0 < len(short_reqs) < reqs:
         row_req = torch.cat([torch.full((n,), b) for b, (_, n) in enumerate(reqs_spec)]).int().to(DEV)
         short = (row_req, limit, len(short_reqs), max(s + n for s, n in short_reqs))
-    got2 = torch.zeros(rows, nq * d, dtype=dtype, device=DEV)
-    ops.paged_attention(qkv.to(DEV), nq, nkv, d, kc.to(DEV), vc.to(DEV), table.to(DEV), page,
-                        q_start_t.to(DEV), start_pos_t.to(DEV), reqs, max(n for _, n in reqs_spec),
-                        max_ctx, window, scale, got2, short)
-    err = (got2.float().cpu() - want.float()).abs().max().item()
-    assert err <= tol * max(1.0, want.float().abs().max().item()), f"attention error {err} (described step)"
+    for described in ([short, ShortRequests(*short)] if short else [None]):      # (claimed, and counted)
+        got2 = torch.zeros(rows, nq * d, dtype=dtype, device=DEV)
+        ops.paged_attention(qkv.to(DEV), nq, nkv, d, kc.to(DEV), vc.to(DEV), table.to(DEV), page,
+                            q_start_t.to(DEV), start_pos_t.to(DEV), reqs, max(n for _, n in reqs_spec),
+                            max_ctx, window, scale, got2, described)
+        err = (got2.float().cpu() - want.float()).abs().max().item()
+        assert err <= tol * max(1.0, want.float().abs().max().item()), f"attention error {err} (described step)"
     # key splits are merged by the last block to arrive; the same with the kernel of its own,
     # and the arrival counters are back at zero whoever merged
     if dtype == torch.bfloat16:
@@ -697,7 +699,7 @@ def run_attention(ops, emu, dtype, nq, nkv, d, page, window, reqs_spec, seed=30,
             with ops.debug.force(**{w: d for w in who}):
                 ops.paged_attention(qkv.to(DEV), nq, nkv, d, kc.to(DEV), vc.to(DEV), table.to(DEV), page,
                                     q_start_t.to(DEV), start_pos_t.to(DEV), reqs, max(n for _, n in reqs_spec),
-                                    max_ctx, window, scale, got3, short)
+                                    max_ctx, window, scale, got3, short and ShortRequests(*short))
             err = (got3.float().cpu() - want.float()).abs().max().item()
             assert err <= tol * max(1.0, want.float().abs().max().item()), f"attention error {err} ({who})"
     assert int(ops.arrived.abs().sum()) == 0

@@ -3,7 +3,9 @@
 import pytest
 import torch
 
-from test_kernels_gpu import emu, ops, run_attention  # noqa: F401 (fixtures)
+from llm_inference_lab_amd.cache import layout as cache_layout
+from llm_inference_lab_amd.parts.base import ShortRequests
+from test_kernels_gpu import DEV, emu, make_cache, ops, rnd, run_attention  # noqa: F401 (fixtures)
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +37,45 @@ def test_tiles_of_16_rows(ops, emu, window, nq, nkv, d, page):  # noqa: F811
     behind histories whose keys are split over blocks and not."""
     for spec in ([(0, 3), (5, 1)], [(0, 17), (900, 1), (64, 1)], [(700, 1), (33, 50), (1500, 1), (0, 129)]):
         run_attention(ops, emu, torch.bfloat16, nq, nkv, d, page, window, spec, seed=97)
+
+
+def step(ops, dtype, nq, nkv, d, page, spec, seed):  # noqa: F811
+    """A step over requests ``(start, tokens)``; a function that takes its description and returns its rows, and
+    the description as it is counted."""
+    per = max(-(-(s + n) // page) for s, n in spec)
+    starts = [0]
+    for _, n in spec:
+        starts.append(starts[-1] + n)
+    q = rnd((starts[-1], (nq + 2 * nkv) * d), dtype, seed).to(DEV)
+    kc, vc = make_cache(per * len(spec) + 1, nkv, page, d, dtype, seed + 1)
+    kc, vc = cache_layout.keys_to_cache_order(kc).to(DEV), cache_layout.values_to_cache_order(vc).to(DEV)
+    table = torch.arange(per * len(spec), dtype=torch.int32, device=DEV).view(len(spec), per)
+    row_req = torch.cat([torch.full((n,), b) for b, (_, n) in enumerate(spec)]).int().to(DEV)
+    q_start, start_pos = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in (starts, [s for s, _ in spec]))
+    longest, most = max(n for _, n in spec), max(s + n for s, n in spec)
+    counted = ShortRequests.count(row_req, ops.attention_short_limit(nq, nkv, dtype, longest), starts, [s for s, _ in spec],
+                                  len(spec))
+
+    def run(short):
+        out = torch.full((starts[-1], nq * d), 777.0, dtype=dtype, device=DEV)
+        ops.paged_attention(q, nq, nkv, d, kc, vc, table, page, q_start, start_pos, len(spec), longest, most, None,
+                            d ** -0.5, out, short)
+        return out.float()
+    return run, counted
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("nq,nkv,d", [(14, 2, 64), (8, 2, 128)])
+@pytest.mark.parametrize("portion", [21, 300])
+def test_a_count_that_the_caller_only_claims(ops, dtype, nq, nkv, d, portion):  # noqa: F811
+    """A count of short requests that is not that of the step (one too many, one too few, nearly all) leaves no row
+    unwritten: only a counted description bounds the blocks of a launch."""
+    spec = [(60 + 7 * i, 1) for i in range(9)] + [(500, portion), (0, 40), (33, portion)]
+    run, counted = step(ops, dtype, nq, nkv, d, 64, spec, 98)
+    assert counted[2:] == (9, 117)
+    want = run(None)
+    bound = (2e-5 if dtype == torch.float32 else 2e-2) * max(1.0, want.abs().max().item())
+    assert (run(counted) - want).abs().max().item() <= bound
+    for claimed in (1, 8, 9, 10, 11):
+        got = run((counted[0], counted[1], claimed, 117))
+        assert (got - want).abs().max().item() <= bound, claimed
