@@ -1720,8 +1720,10 @@ static int estimated_tile(int M, int N, int K, int num_cus) {
   if (pp_rows && K >= PP_MIN_INNER && K <= DIRECT_MAX_INNER && !g_without_wide) {
     // (the estimates of the other tiles, fitted at shorter inner sizes, are up to a quarter low from
     // 3,584 on (and 512 rows): 4096 rows of 1536 x 8960 129 us against 147 with their pick, 2048 of 3584 x 18944 268 against 301,
-    // 2367 of 2048 x 11008 154 against 181; over 126 products the picks then lose 0.1 % on average)
-    double least = tile_cost(best, M, N, K, num_cus, 1) * (M >= 512 && K >= 3584 ? 1.25 : 1.0);
+    // 2367 of 2048 x 11008 154 against 181.  Not where the blocks of the 64 x 128 tile nearly find the three places
+    // a unit that they have, until an inner size of 8,192: 1400 rows of 3584 x 3584 70 us with it against 76, 768 of 6144 x 4096 64 against 70)
+    const bool low = M >= 512 && K >= 3584 && (K >= 8192 || 10 * (long)((M + 63) / 64) * wide > 27L * num_cus);
+    double least = tile_cost(best, M, N, K, num_cus, 1) * (low ? 1.25 : 1.0);
     for (int kind = TILE_256; kind <= TILE_192; ++kind) {
       const double c = tile_cost(kind, M, N, K, num_cus, 1);
       if (c < least) {
@@ -1733,17 +1735,22 @@ static int estimated_tile(int M, int N, int K, int num_cus) {
   return addressable(best, K);
 }
 
-// Up to 1,024 rows of a matrix of less than 32 MB (128 rows: 64 MB), where the blocks of the 64 x 128 tile find
-// two places a unit (with more, 512 rows of 9728 x 896, the estimates choose better): among the three small tiles the
-// estimates above lose 10 % on average (up to 42 %), because they count a block that has its unit to itself, whose
-// chain of K tiles is the time, like one of several that share it.  Here both are weighed: the chain of a block's K tiles, and
-// what a unit takes for all of its blocks.  Fitted to the same sweep (9 to 12 % rms; the two larger
-// tiles 5 and 10 % up, with which fewer picks are wrong), the pick then loses 1 %,
-// with the fold of the pieces: 512 rows of 896 x 4864 with the norm 17.8 us (64 x 64 in four pieces) against 24.7 (64 x 128 in six),
-// 700 of 2048 x 2048 15.8 against 22.5, 100 of 4608 x 3584 17.5 against 22.4 (2: all three are weighed).  Up to 2,560
-// rows of less than 16 MB and inner sizes to 2,048 (1) the 64 x 64 tile is weighed against the estimates' tile: 2048 rows of
-// 1152 x 896 12.0 against 13.7, of 896 x 896 9.4 against 10.6; of 896 x 4864 it would be taken whole, 33.3 us by itself against
-// 39.9 in two pieces with their fold, and inside a prompt's step be slower by 4 us a layer.  Beyond that (0) the estimates above.
+// Few blocks: the estimates above count a block that has its unit to itself, whose chain of K tiles is the time,
+// like one of several that share it, and lose 10 % on average (up to 42 %).  Here a unit holds `resident` blocks at a
+// time; a round of them takes what the unit needs for all of them (f + K tiles x tk each), or the chain of one (K
+// tiles x chain), whichever is more; a block more than the places of a round is a round of its own.  (Counted as a
+// share of one, 1400 rows of 2304 x 768 went to 64 x 64, 792 blocks on 768 places, 19.4 us against 15.2 with 64 x
+// 128, and 700 of 5632 x 1024 to 128 x 128, 264 blocks, 23.7 against 18.2.)  Fitted to 12,000 products: the four of a layer of 14
+// model shapes, 512 to 4096 wide, 65 to 3,000 rows, whole and in two to eight pieces (7, 7 and 6 % rms).  Over 1,200 of them
+// the picks lose 1 % to the best tile of gate and up, and with the fold of the pieces 2 and 3 % of the output and down
+// product: 512 rows of 896 x 4864 with the norm 17.8 us (64 x 64 in four pieces) against 24.7 (64 x 128 in six, the
+// estimates'), 700 of 2048 x 2048 15.8 against 22.5, 100 of 4608 x 3584 17.5 against 22.4.
+// Where they are asked (2): up to 1,024 rows of a matrix of less than 32 MB (128 rows: 64 MB) where the blocks of the 64 x 128
+// tile find two places a unit; with more, 512 rows of 9728 x 896, the estimates choose as well.  Up to 2,560 rows of
+// less than 16 MB and inner sizes to 2,048 (1) a whole product weighs the 64 x 64 tile against the estimates' (2048 rows of
+// 1152 x 896 12.0 against 13.7, of 896 x 896 9.4 against 10.6), one in pieces the two of 64 rows; 2048 rows of 896 x 4864 would be taken
+// whole, 33.3 us by itself against 39.9 in two pieces with their fold, and inside a prompt's step be slower by 4 us a
+// layer.  Beyond that (0) the estimates above.
 static int few_blocks_range(int M, int N, int K, int num_cus) {
   const double bytes = (double)N * K * 2.0;
   if (g_force_tile != 0 || (long)((M + 63) / 64) * ((N + 127) / 128) > 2L * num_cus) return 0;
@@ -1752,19 +1759,23 @@ static int few_blocks_range(int M, int N, int K, int num_cus) {
 }
 static double few_blocks_cost(int kind, int M, int N, int K, int num_cus, int pieces) {
   static const struct {
-    double L, chain, f, tk, stream;
+    double L, chain, f, tk;
     int resident;
-  } fit[3] = {{3.10, 0.357, 0.76, 0.227, 30.0e3, 3}, {4.23, 0.506, 1.65, 0.376, 30.9e3, 2}, {2.34, 0.781, 4.68, 0.72, 23.4e3, 1}};
+  } fit[3] = {{4.78, 0.357, 0.09, 0.234, 3}, {5.87, 0.5, 0.5, 0.327, 3}, {6.89, 0.735, 1.25, 0.478, 2}};
   const auto& p = fit[kind];
   const double blocks = (double)((M + TILE_MODELS[kind].bm - 1) / TILE_MODELS[kind].bm) *
                         ((N + TILE_MODELS[kind].bn - 1) / TILE_MODELS[kind].bn) * pieces;
   const int nk = ((K + 63) / 64 + pieces - 1) / pieces;
-  const double share = blocks / num_cus, turns = share <= p.resident ? ceil(share - 1e-9) : share;
-  const double rate = blocks * p.stream < CHIP_STREAM ? blocks * p.stream : CHIP_STREAM;
-  double t = turns * (p.f + nk * p.tk);
-  if (nk * p.chain > t) t = nk * p.chain;
-  if ((double)N * K * 2.0 / rate > t) t = (double)N * K * 2.0 / rate;
-  return p.L + t;
+  auto round_of = [&](double share) {           // share: blocks a unit
+    const double together = share * (p.f + nk * p.tk), alone = nk * p.chain;
+    return together > alone ? together : alone;
+  };
+  const double share = blocks / num_cus, rounds = floor(share / p.resident + 1e-9);
+  const double last = share - rounds * p.resident;
+  double t = rounds * round_of(p.resident);
+  if (last > 1e-6) t += round_of(ceil(last - 1e-9));
+  const double read = (double)N * K * 2.0 / CHIP_STREAM;
+  return p.L + (t > read ? t : read);
 }
 
 static int choose_tile(int M, int N, int K, int num_cus) {
@@ -1906,14 +1917,18 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
   const int nk = (K + 63) / 64;
   const double piece = (double)M * N * 2.2e-6 + 0.3;
   int best_kind = choose_tile(M, N, K, num_cus), best_pieces = 1;
-  double best_cost = tile_cost(best_kind, M, N, K, num_cus, 1);
+  // (the estimates of the tiles below 256 rows are low at long inner sizes, as in estimated_tile)
+  auto cost = [&](int kind, int pieces) {
+    return tile_cost(kind, M, N, K, num_cus, pieces) * (kind < TILE_256 && M >= 512 && K >= 3584 ? 1.25 : 1.0);
+  };
+  double best_cost = cost(best_kind, 1);
   // 65 to 128 rows: one tile of 128 rows reads W once where two of 64 read it twice, which
   // the estimate does not know (128 rows of 3584 x 18944 in pieces: 45 us against 57, a decode
   // step of 128 requests of that shape 7.11 ms against 7.30)
   const bool one_tile_of_128 = M > 64 && M <= 128 && g_force_tile == 0 && (double)N * K * 2.0 >= 64e6;
   if (one_tile_of_128) {
     best_kind = TILE_128;
-    best_cost = tile_cost(TILE_128, M, N, K, num_cus, 1);
+    best_cost = cost(TILE_128, 1);
   }
   for (int kind = TILE_64x128; kind < TILE_KINDS; ++kind) {
     if (kind == TILE_128x256) continue;
@@ -1922,7 +1937,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
     if (g_force_tile != 0 && kind != choose_tile(M, N, K, num_cus)) continue;
     for (int s = 2; s <= max_pieces; ++s) {
       if ((nk + s - 1) / s < min_tiles_per_piece) break;
-      const double c = tile_cost(kind, M, N, K, num_cus, s) + s * piece;
+      const double c = cost(kind, s) + s * piece;
       if (c < best_cost) {
         best_cost = c;
         best_kind = kind;
@@ -1949,10 +1964,11 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
     best_kind = TILE_64;
   const int range = best_kind <= TILE_128 ? few_blocks_range(M, N, K, num_cus) : 0;
   if (range) {
-    double least = few_blocks_cost(best_kind, M, N, K, num_cus, best_pieces) + (best_pieces > 1 ? best_pieces * piece : 0.0);
+    auto folded = [&](int pieces) { return pieces > 1 ? pieces * ((double)M * N * 1.1e-6 + 0.28) : 0.0; };
+    double least = few_blocks_cost(best_kind, M, N, K, num_cus, best_pieces) + folded(best_pieces);
     for (int kind = TILE_64; kind <= (range == 2 ? TILE_128 : TILE_64x128); ++kind)
       for (int s = 1; s <= max_pieces && (s == 1 || (nk + s - 1) / s >= min_tiles_per_piece); ++s) {
-        const double c = few_blocks_cost(kind, M, N, K, num_cus, s) + (s > 1 ? s * piece : 0.0);
+        const double c = few_blocks_cost(kind, M, N, K, num_cus, s) + folded(s);
         if (c < least) {
           least = c;
           best_kind = kind;

@@ -91,6 +91,41 @@ def test_measured_decisions(core, m, n, k, want):
     assert plan(core, m, n, k) == want
 
 
+@pytest.mark.parametrize("m,n,k,columns", [
+    # (us with this tile and with the best of the others; blocks of 64 x 64 that find no place any more with three
+    # to a unit cost a round, and a block of 128 x 128 more than units as well)
+    (700, 5632, 1024, 128),      # 64 x 128: 18.2 us against 23.7 (128 x 128) and 22.6
+    (576, 6144, 768, 128),       # 14.1 against 16.6
+    (640, 5632, 1024, 128),      # 17.8 against 20.6
+    (640, 5216, 1000, 128),      # 17.9 against 21.1
+    (384, 9216, 1152, 128),      # 20.4 against 24.1
+    (300, 10240, 1280, 128),     # 22.9 against 26.0
+    (1400, 2304, 768, 128),      # 15.2 against 19.4
+    (1536, 2304, 1792, 128),     # 25.1 against 31.3
+    (2048, 1792, 1280, 128),     # 21.1 against 26.0
+    (1801, 2048, 1024, 128),     # 18.5 against 22.6
+    (2300, 1536, 1536, 128),     # 32.2 against 36.4
+    (1400, 3584, 3584, 128),     # 70.4 against 76.3 with the 192 x 256 tile
+    (768, 6144, 4096, 128),      # 64.0 against 69.9
+    (512, 896, 896, 64), (2048, 896, 896, 64), (2048, 1152, 896, 64), (700, 2048, 2048, 64),
+])
+def test_tiles_of_few_blocks(core, m, n, k, columns):
+    assert core.llmlab_linear_tile(m, n, k, CUS) == columns
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (576, 1536, 8960, (4, 1)),       # with the norm 40.9 us against 46.1 (64 x 64 in two pieces)
+    (1024, 1792, 7168, (4, 5)),      # 46.4 against 65.9 (64 x 64 whole)
+    (300, 3584, 3584, (3, 1)),       # 30.6 against 33.3 (64 x 64 in three)
+    (512, 2560, 2560, (3, 1)),       # 26.0 against 30.1 (64 x 64 whole)
+    (512, 896, 4864, (4, 0)),        # 17.8 against 24.7 (64 x 128 in six)
+    (1100, 4096, 4096, (2, 5)),      # 59.3 against 72.3 (64 x 128 whole)
+])
+def test_pieces_of_few_blocks(core, m, n, k, want):
+    assert plan(core, m, n, k) == want
+    assert plan(core, m, n, k, 8) == want
+
+
 def test_one_tile_of_rows_of_a_wide_matrix(core):
     """Up to 128 rows: the tile that the estimates pick, measured inside decode steps of 96 and 128 requests.  (A
     product that is neither cut nor written by heads follows it only where no width makes one round of blocks:
