@@ -1908,9 +1908,28 @@ extern "C" int llmlab_linear_grouped(const void* x, const void* w, int epilogue,
   return 0;
 }
 
+// 65 to 128 rows in pieces: one tile of 128 rows reads W once where two of 64 read it twice, which
+// the estimate does not know (128 rows of 3584 x 18944 in pieces: 45 us against 57, a decode
+// step of 128 requests of that shape 7.11 ms against 7.30)
+static bool takes_one_tile_of_128(int M, int N, int K) {
+  return M > 64 && M <= 128 && g_force_tile == 0 && (double)N * K * 2.0 >= 64e6;
+}
+
+// The tile of a product that its caller cuts into so many pieces, whatever number the plan below would take
+// (q/k/v products of 65 to 384 rows, two at least: 384 rows of 5120 x 3072 33.8 us in two with this tile, 40.5 with that of the whole product).
+extern "C" int llmlab_pieces_tile(int M, int N, int K, int num_cus, int pieces) {
+  if (num_cus <= 0) num_cus = 256;
+  int kind = choose_tile(M, N, K, num_cus);
+  if (takes_one_tile_of_128(M, N, K)) kind = TILE_128;
+  else if (kind <= TILE_128 && few_blocks_range(M, N, K, num_cus) == 2)
+    for (int other = TILE_64; other <= TILE_128; ++other)
+      if (few_blocks_cost(other, M, N, K, num_cus, pieces) < few_blocks_cost(kind, M, N, K, num_cus, pieces)) kind = other;
+  return addressable(kind, K);
+}
+
 // Whether (and into how many pieces along K) a product that adds into float32 rows should
-// be left unsummed, and with which tile: out = {pieces (1: no), tile kind}.  A piece costs
-// a write and a read of the result by whoever sums it up later.
+// be left unsummed, and with which tile: out = {pieces (1: no), tile kind}; in one piece the kind is that
+// of a whole product (choose_tile).  A piece costs a write and a read of the result by whoever sums it up later.
 extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pieces, int min_tiles_per_piece,
                                    int* out) {
   if (num_cus <= 0) num_cus = 256;
@@ -1922,10 +1941,7 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
     return tile_cost(kind, M, N, K, num_cus, pieces) * (kind < TILE_256 && M >= 512 && K >= 3584 ? 1.25 : 1.0);
   };
   double best_cost = cost(best_kind, 1);
-  // 65 to 128 rows: one tile of 128 rows reads W once where two of 64 read it twice, which
-  // the estimate does not know (128 rows of 3584 x 18944 in pieces: 45 us against 57, a decode
-  // step of 128 requests of that shape 7.11 ms against 7.30)
-  const bool one_tile_of_128 = M > 64 && M <= 128 && g_force_tile == 0 && (double)N * K * 2.0 >= 64e6;
+  const bool one_tile_of_128 = takes_one_tile_of_128(M, N, K);
   if (one_tile_of_128) {
     best_kind = TILE_128;
     best_cost = cost(TILE_128, 1);
@@ -1975,8 +1991,8 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
           best_pieces = s;
         }
       }
-    if (best_pieces == 1) best_kind = estimated_tile(M, N, K, num_cus);      // (a whole product chooses its tile itself)
   }
+  if (best_pieces == 1) best_kind = choose_tile(M, N, K, num_cus);
   out[0] = best_pieces;
   out[1] = addressable(best_kind, K);
 }

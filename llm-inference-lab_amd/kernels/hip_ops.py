@@ -248,6 +248,8 @@ class HipOps:
                                         _c_int, _c_int, _c_int, _c_int, _c_ptr]
         c.llmlab_linear_heads_tile.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_int]
         c.llmlab_linear_heads_tile.restype = _c_int
+        c.llmlab_pieces_tile.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_int]
+        c.llmlab_pieces_tile.restype = _c_int
         c.llmlab_linear_partials.argtypes = [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                              _c_int, _c_int, _c_size, _c_int, _c_ptr]
         c.llmlab_qkv_from_pieces.argtypes = [_c_ptr, _c_int, _c_size, _c_int, _c_ptr, _c_int, _c_int, _c_int,
@@ -753,6 +755,13 @@ class HipOps:
         plan(rows, n, k, self.num_cus, self.MAX_SPLITS, self.rules.min_tiles_per_split, out)
         return out[0], out[1]
 
+    def _pieces_tile(self, rows: int, n: int, k: int, dtype, pieces: int) -> int:
+        """The tile of such a product cut into ``pieces``, which need not be the plan's number."""
+        planned, tile = self._linear_plan(rows, n, k, dtype)
+        if dtype != torch.bfloat16 or pieces == planned:
+            return tile
+        return self._core.llmlab_pieces_tile(rows, n, k, self.num_cus, pieces)
+
     def linear_partials(self, x, w, parts: torch.Tensor, splits: int, bias=None) -> PendingSums:
         """``parts[s] = x[:, K_s] w[:, K_s]^T`` for the ``splits`` pieces ``K_s`` of the inner
         size (bias in piece 0): the product without the final sum."""
@@ -778,7 +787,7 @@ class HipOps:
             self._call(self._core.llmlab_linear_partials,
                 self._ptr(x), self._ptr(w), _dt(x), self._ptr(parts), self._ptr(bias),
                 _dt(bias) if bias is not None else 0, m, n, k, parts.stride(1), splits, parts.stride(0),
-                self._linear_plan(m, n, k, x.dtype)[1], self._stream())
+                self._pieces_tile(m, n, k, x.dtype, splits), self._stream())
         return PendingSums(parts, splits)
 
     def add_pending(self, x: torch.Tensor, pending: PendingSums) -> None:
@@ -874,7 +883,7 @@ class HipOps:
             return None
         if rows > self.FEW_ROWS and self.few_rows_take(rows, n, k):
             return None
-        pieces, tile = self._linear_plan(rows, n, k)
+        pieces = self._linear_plan(rows, n, k)[0]
         if rows > self.FEW_ROWS and k >= 2 * 64 * self.rules.min_tiles_per_split:
             # (65 to 384 rows: two pieces at least.  4608 x 3584 at 192 / 256 rows: 24 / 31 us
             # against 33 / 39 whole; 2560 x 2048: 15 / 18.5 against 20.5; the estimate of
@@ -883,7 +892,7 @@ class HipOps:
         if self.rules.forced_tiled_pieces:
             pieces = max(1, min(self.rules.forced_tiled_pieces, (k + 63) // 64, self.MAX_SPLITS))
         if pieces > 1 and pieces * rows * n <= self.workspace.numel():
-            return pieces, tile
+            return pieces, self._pieces_tile(rows, n, k, torch.bfloat16, pieces)
         return None
 
     def qkv_rope_cache(self, h, w_qkv, b_qkv, num_heads, num_kv_heads, head_dim, inv_freq, positions,

@@ -57,6 +57,26 @@ def test_tile_and_pieces_of_products_of_many_rows(core):
             assert (m >= 512 or (m > 128 and n >= 16384 and pieces == 1)) and k >= 896, (m, n, k, kind)
 
 
+def test_a_plan_in_one_piece_names_the_tile_that_is_launched(core):
+    rng = random.Random(9)
+    whole = 0
+    for _ in range(20000):
+        m, n, k = rng.randint(17, 2560), 16 * rng.randint(4, 700), 8 * rng.randint(8, 900)
+        pieces, kind = plan(core, m, n, k)
+        if pieces == 1:
+            whole += 1
+            assert KINDS[kind][1] == core.llmlab_linear_tile(m, n, k, CUS), (m, n, k, kind)
+    assert whole > 5000
+
+
+@pytest.mark.parametrize("m,n,k,pieces,want", [
+    (384, 5120, 3072, 2, 1),          # 33.8 us in two pieces against 40.5 with the tile of the whole product
+    (256, 4608, 3584, 3, 1), (128, 3584, 18944, 4, 2), (192, 2560, 2048, 2, 0),
+])
+def test_tile_of_a_number_of_pieces_that_is_not_the_plans(core, m, n, k, pieces, want):
+    assert core.llmlab_pieces_tile(m, n, k, CUS, pieces) == want
+
+
 def test_limits_of_the_plan_are_kept(core):
     for max_pieces, min_tiles in ((1, 8), (3, 8), (16, 100), (16, 1)):
         for (m, n, k) in ((40, 3584, 18944), (576, 3584, 18944), (2048, 5120, 27648), (100, 896, 4864)):
@@ -81,7 +101,9 @@ def test_limits_of_the_plan_are_kept(core):
     (384, 27648, 5120, (1, 5)),
     (192, 27648, 5120, (1, 1)),       # ... not where half the units would stay idle
     (192, 4608, 3584, (1, 0)),        # 216 blocks of 64 x 64 are one round (26 us against 29 with 64 x 128),
-    (1536, 896, 896, (1, 1)),         # 336 are two: 64 x 128 (11.5 us against 13.3)
+    (1536, 896, 896, (1, 0)),         # ... and so are 336 by direct loads, three to a unit (with the norm 16.5 against 18.7)
+    (2048, 1152, 896, (1, 0)),
+    (1400, 2304, 768, (1, 1)),        # 792 are a round and a bit
     (384, 5120, 27648, (4, 2)),       # three tiles of 128 rows in four pieces (150 us against 183 in two of 64 x 128)
     (256, 8192, 8192, (4, 2)),
     (192, 5120, 27648, (4, 1)),       # ... from 256 rows on (a step of 192 requests of the 32B shape loses 5 % with them)
