@@ -1934,7 +1934,10 @@ extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pie
                                    int* out) {
   if (num_cus <= 0) num_cus = 256;
   const int nk = (K + 63) / 64;
-  const double piece = (double)M * N * 2.2e-6 + 0.3;
+  // (a piece's write and read; the second is the price of large results, where that of the first kept whole what is
+  // faster in pieces: with the norm 900 rows of 3584 x 3584 45 us in three pieces against 53 whole, 1400 of 4096 x 4096 66
+  // in two against 85)
+  const double piece = (double)M * N * (M < 512 || (double)M * N < 2e6 ? 2.2e-6 : 1.5e-6) + 0.3;
   int best_kind = choose_tile(M, N, K, num_cus), best_pieces = 1;
   // (the estimates of the tiles below 256 rows are low at long inner sizes, as in estimated_tile)
   auto cost = [&](int kind, int pieces) {

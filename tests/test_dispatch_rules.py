@@ -142,6 +142,9 @@ def test_tiles_of_few_blocks(core, m, n, k, columns):
     (512, 2560, 2560, (3, 1)),       # 26.0 against 30.1 (64 x 64 whole)
     (512, 896, 4864, (4, 0)),        # 17.8 against 24.7 (64 x 128 in six)
     (1100, 4096, 4096, (2, 5)),      # 59.3 against 72.3 (64 x 128 whole)
+    (900, 3584, 3584, (3, 5)),       # 44.9 against 53.4 (64 x 128 whole)
+    (1400, 4096, 4096, (2, 5)),      # 66.1 against 85.0 (192 x 256 whole)
+    (2048, 896, 4864, (2, 1)),
 ])
 def test_pieces_of_few_blocks(core, m, n, k, want):
     assert plan(core, m, n, k) == want
