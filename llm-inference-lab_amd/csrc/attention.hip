@@ -1279,7 +1279,8 @@ static int launch_key_split_decode(const KeySplitLaunch& k, int reqs, int total_
   return launch_split_merge(k, total_rows, nq, row_req, out, out_stride, stream);
 }
 
-// 1: a mixed step always in two launches; -1: in one wherever a kernel for it exists (measurements)
+// 1: a mixed step always in two launches; -1: in one wherever a kernel for it exists; -2: in one with the
+// portions by tiles of 16 rows (heads up to 128; measurements and tests)
 static int g_force_two_launches = 0;
 extern "C" void llmlab_debug_attention_two_launches(int on) { g_force_two_launches = on; }
 
@@ -1460,15 +1461,6 @@ static int choose_many_rows_launch(long max_rows, int nkv, int live, int max_q_l
   return path;
 }
 
-// Whether the blocks of a mixed step's portions (keys split over the waves of a block) and of its
-// decoding requests go in one launch: see llmlab_paged_attention.
-static bool mixed_step_in_one_launch(long long_blocks, long short_blocks, int num_cus, int forced) {
-  if (forced > 0) return false;
-  if (forced < 0) return true;
-  const long places = (D <= 64 ? 1L : 2L) * num_cus;      // blocks of the portion's kind that the chip holds at a time
-  return 2 * long_blocks <= places || 4 * (long_blocks + short_blocks) <= 5 * places;
-}
-
 // Whether a mixed step goes in one launch with the portions by tiles of 16 rows, whose waves split the keys with one
 // step on its way: few enough registers (116 at heads of 64, against 157 to 201) that a unit holds two
 // blocks of either kind, so that the decoding requests' streams pass beside the portions' chains.  `blocks16` and
@@ -1488,9 +1480,42 @@ static bool mixed_step_by_small_tiles(long blocks16, long blocks32, long short_b
   return blocks16 <= (path != 1 && short_ring == 2 ? 1L : 2L) * num_cus;
 }
 
-// How many attention launches a mixed step in bfloat16 takes (the merge of key splits not
-// counted) where its portions do not go by tiles of 16 rows: `n_short` of its requests decode behind at most
-// `short_ctx` keys, the others bring portions of at most `max_q_len` tokens (for tests and tuning; 0: not a mixed step).
+// Both kinds of blocks in one launch (see attention_bf16_mixed_kernel) with the portions by tiles of 32 rows,
+// where the portion's blocks leave half of the chip's places free, or all blocks together hardly exceed the
+// places: every block of the one launch holds the registers of the portion's kind, so the
+// decoding requests' blocks, which stream and want company on their unit, lose places
+// (a unit holds one block at heads up to 64, two above).  Heads of 64, a portion of 128
+// tokens behind 2,048 keys beside 63 requests decoding at 2,048: 28 us against 38 in two
+// launches; a portion of 512 (224 blocks) beside 31 at 1,024: 27 against 30, beside 127 at
+// 1,024: 68 against 59, hence not there.  Heads of 128, 128 tokens beside 63 at 2,048: 75
+// against 90.
+static bool mixed_step_in_one_launch(long long_blocks, long short_blocks, int num_cus, int forced) {
+  if (forced > 0) return false;
+  if (forced < 0) return true;
+  const long places = (D <= 64 ? 1L : 2L) * num_cus;      // blocks of the portion's kind that the chip holds at a time
+  return 2 * long_blocks <= places || 4 * (long_blocks + short_blocks) <= 5 * places;
+}
+
+// What serves a mixed step in bfloat16 whose `live` portions would by themselves take launch `path`: the one place
+// that decides it, for llmlab_paged_attention and for who asks (llmlab_attention_mixed_launches).
+enum { MIXED_NONE = 0, MIXED_ONE_LAUNCH = 1, MIXED_TWO_LAUNCHES = 2, MIXED_SMALL_TILES = 3 };
+static int mixed_step_launch(const KeySplitLaunch& shorts, int n_short, long max_rows, int nkv, int live, int max_ctx_len,
+                             int path, int num_cus, int forced_path, int forced) {
+  const int steps32 = (max_ctx_len + 31) / 32 + 1;
+  const int steps_per_wave = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;
+  const long blocks16 = (max_rows + 15) / 16 * nkv * live, blocks32 = (max_rows + 31) / 32 * nkv * live;
+  const long short_blocks = (long)nkv * shorts.a.splits * n_short;
+  if (forced == -2 && D <= 128) return MIXED_SMALL_TILES;
+  if (forced_path == 0 && forced == 0 &&
+      mixed_step_by_small_tiles(blocks16, blocks32, short_blocks, shorts.ring, steps_per_wave > 2 || shorts.ring == 2, path,
+                                max_ctx_len, num_cus))
+    return MIXED_SMALL_TILES;
+  return path == 1 && mixed_step_in_one_launch(blocks32, short_blocks, num_cus, forced) ? MIXED_ONE_LAUNCH : MIXED_TWO_LAUNCHES;
+}
+
+// What serves a mixed step in bfloat16: `n_short` of its requests decode behind at most `short_ctx` keys, the
+// others bring portions of at most `max_q_len` tokens.  2: a launch for each kind; 1: one launch, the portions by tiles of
+// 32 rows; 3: one launch, by tiles of 16 rows (the merge of key splits not counted); 0: not a mixed step.
 extern "C" int llmlab_attention_mixed_launches(int nq, int nkv, int reqs, int n_short, int max_q_len, int max_ctx_len,
                                                int short_ctx, int window, int num_cus) {
   if (num_cus <= 0) num_cus = 256;
@@ -1498,12 +1523,11 @@ extern "C" int llmlab_attention_mixed_launches(int nq, int nkv, int reqs, int n_
   const long max_rows = (long)max_q_len * (nq / nkv);
   if (max_rows <= 16) return 0;
   const int live = reqs - n_short;
-  if (choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, 0) != 1) return 2;
+  const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, 0);
   AttnArgs a{};
   const KeySplitLaunch shorts = prepare_key_split_decode(a, reqs, n_short, short_ctx, window, reqs, nq, nkv, nullptr,
                                                          ~(size_t)0 >> 8, num_cus, nullptr, 0);
-  return mixed_step_in_one_launch((max_rows + 31) / 32 * nkv * live, (long)nkv * shorts.a.splits * n_short, num_cus, 0)
-             ? 1 : 2;
+  return mixed_step_launch(shorts, n_short, max_rows, nkv, live, max_ctx_len, path, num_cus, 0, g_force_two_launches);
 }
 
 // The launch that llmlab_paged_attention would take for a step of many rows of these sizes
@@ -1597,39 +1621,25 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
   const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, g_force_path);
   const int steps32 = (max_ctx_len + 31) / 32 + 1;
   const int steps_per_wave = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;
-  if (mixed && g_force_path == 0 && g_force_two_launches == 0 && mixed_blocks((max_rows + 15) / 16) <= MOST_BLOCKS &&
-      mixed_step_by_small_tiles((max_rows + 15) / 16 * nkv * live, (max_rows + 31) / 32 * nkv * live,
-                                (long)nkv * shorts.a.splits * n_short, shorts.ring,
-                                steps_per_wave > 2 || shorts.ring == 2, path, max_ctx_len, num_cus)) {
+  int how = mixed ? mixed_step_launch(shorts, n_short, max_rows, nkv, live, max_ctx_len, path, num_cus, g_force_path,
+                                      g_force_two_launches) : MIXED_NONE;
+  if ((how == MIXED_SMALL_TILES && mixed_blocks((max_rows + 15) / 16) > MOST_BLOCKS) ||
+      (how == MIXED_ONE_LAUNCH && mixed_blocks((max_rows + 31) / 32) > MOST_BLOCKS))
+    how = MIXED_TWO_LAUNCHES;
+  if (how == MIXED_SMALL_TILES) {
     const int tiles16 = (int)((max_rows + 15) / 16);
     hipLaunchKernelGGL((attention_bf16_mixed_kernel<1, 1, 1>), dim3((unsigned)mixed_blocks(tiles16)), dim3(64 * DECODE_WAVES), 0, stream, a,
                        shorts.a, tiles16);
     LLMLAB_LAUNCH_CHECK("attention(bfloat16, mixed, tiles of 16 rows)");
     return launch_split_merge(shorts, total_rows, nq, row_req, out, out_stride, stream);
   }
-  if (mixed && path != 1) {
+  if (how == MIXED_TWO_LAUNCHES) {
     const int rc = launch_key_split_decode(shorts, reqs, total_rows, nq, nkv, row_req, out, out_stride, stream);
     if (rc) return rc;
   }
   if (path == 1) {
-    // Both kinds of blocks in one launch (see attention_bf16_mixed_kernel) where the portion's
-    // blocks leave half of the chip's places free, or all blocks together hardly exceed the
-    // places: every block of the one launch holds the registers of the portion's kind, so the
-    // decoding requests' blocks, which stream and want company on their unit, lose places
-    // (a unit holds one block at heads up to 64, two above).  Heads of 64, a portion of 128
-    // tokens behind 2,048 keys beside 63 requests decoding at 2,048: 28 us against 38 in two
-    // launches; a portion of 512 (224 blocks) beside 31 at 1,024: 27 against 30, beside 127 at
-    // 1,024: 68 against 59, hence not there.  Heads of 128, 128 tokens beside 63 at 2,048: 75
-    // against 90.
-    const int long_tiles = (int)((max_rows + 31) / 32);
-    const bool one_launch = mixed && mixed_blocks(long_tiles) <= MOST_BLOCKS && mixed_step_in_one_launch((long)long_tiles * nkv * live,
-                                                              (long)nkv * shorts.a.splits * n_short, num_cus,
-                                                              g_force_two_launches);
-    if (mixed && !one_launch) {
-      const int rc = launch_key_split_decode(shorts, reqs, total_rows, nq, nkv, row_req, out, out_stride, stream);
-      if (rc) return rc;
-    }
-    if (one_launch) {
+    if (how == MIXED_ONE_LAUNCH) {
+      const int long_tiles = (int)((max_rows + 31) / 32);
       dim3 mgrid((unsigned)mixed_blocks(long_tiles)), mblock(64 * DECODE_WAVES);
       const bool deep = steps_per_wave > 2;
       if (deep && shorts.ring == 2)

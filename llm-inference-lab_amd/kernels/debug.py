@@ -127,7 +127,7 @@ class KernelDebug:
               attention_path: Optional[Tuple[int, int]] = None,
               attention_merge_kernel: Optional[int] = None,
               attention_merge_in_place: Optional[int] = None, attention_two_launches: Optional[int] = None,
-              attention_one_launch: Optional[int] = None,
+              attention_one_launch: Optional[int] = None, attention_small_tiles: Optional[int] = None,
               f32_fma: Optional[bool] = None, **rules):
         """``gemm_tile``: 64 (64 x 64), 130 (64 x 128), 129 (128 x 128), 131 (128 x 256), 132 (256 x
         256), 133 (192 x 256), 134 / 135 / 136 (64 x 96 / 160 / 224) or 137 (128 x 160); -131: the choice among the first three; -256 and below: the
@@ -143,7 +143,8 @@ class KernelDebug:
         key splits of decode attention are merged there by the kernel of its own, or by the
         last block to arrive, whatever their number.  ``attention_two_launches`` / ``attention_one_launch``:
         a head size; a mixed step's decoding requests and its portions get a launch each also
-        where one launch would serve both, or one launch wherever there is a kernel for both.
+        where one launch would serve both, or one launch wherever there is a kernel for both; ``attention_small_tiles``:
+        a head size (up to 128); one launch with the portions by tiles of 16 rows.
         ``f32_fma``: float32 products of many rows by the plain FMA kernel instead of the
         matrix cores.  Other keywords: fields of ``DispatchRules`` for the time of the block."""
         ops = self._ops
@@ -168,6 +169,9 @@ class KernelDebug:
             elif attention_one_launch is not None:
                 tlib = ops._attention_lib(int(attention_one_launch))
                 tlib.llmlab_debug_attention_two_launches(-1)
+            elif attention_small_tiles is not None:
+                tlib = ops._attention_lib(int(attention_small_tiles))
+                tlib.llmlab_debug_attention_two_launches(-2)
             if attention_path is not None:
                 plib = ops._attention_lib(int(attention_path[0]))
                 plib.llmlab_debug_attention_path(int(attention_path[1]))

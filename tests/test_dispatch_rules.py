@@ -366,15 +366,26 @@ def test_measured_attention_launches(head_dim, nq, nkv, dtype, reqs, q, behind, 
 
 
 @pytest.mark.parametrize("head_dim,nq,nkv,portion,behind,decoding,their_keys,want", [
-    # (measured, one launch against two: see the comment in llmlab_paged_attention)
-    (64, 14, 2, 128, 2048, 63, 2048, 1),     # 28 us against 38
-    (64, 14, 2, 256, 1024, 31, 1024, 1),     # 21 against 27
-    (64, 14, 2, 512, 1536, 31, 1024, 1),     # 31 against 34
-    (64, 14, 2, 512, 1536, 127, 1024, 2),    # 70 against 63
-    (64, 14, 2, 512, 1536, 63, 512, 2),      # 43 against 40
-    (128, 28, 4, 128, 2048, 63, 2048, 1),    # 75 against 88
-    (128, 40, 8, 128, 2048, 127, 1024, 1),   # 145 against 164
-    (128, 28, 4, 512, 512, 63, 2048, 2),     # (the portion's launch is not the one with the key split)
+    # (us in two launches / in one with the portion by tiles of 32 rows / in one by tiles of 16; the rules are in
+    # csrc/attention.hip.  2: two launches, 1: one by tiles of 32 rows, 3: one by tiles of 16)
+    (64, 14, 2, 128, 2048, 63, 2048, 1),     # 34.2 / 21.6 / 16.6
+    (64, 14, 2, 256, 1024, 31, 1024, 1),     # 24.1 / 15.5 / 14.5
+    (64, 14, 2, 512, 1536, 31, 1024, 3),     # 28.0 / 19.0 / 20.5
+    (64, 14, 2, 512, 1536, 127, 1024, 3),    # 33.1 / 29.5 / 26.8
+    (64, 14, 2, 512, 1536, 63, 512, 3),      # 25.6 / 23.0 / 21.1
+    (64, 14, 2, 464, 1100, 48, 1400, 3),     # 28.7 / 24.4 / 17.6
+    (64, 14, 2, 64, 0, 48, 300, 3),          # 12.4 / -- / 6.9
+    (64, 14, 2, 1024, 1100, 48, 1400, 3),    # 36.9 / -- / 31.2: 896 blocks, three and a half a unit
+    (64, 14, 2, 1025, 1100, 48, 1400, 2),    # (1,100 tokens: 37.5 / -- / 35.5)
+    (64, 14, 2, 512, 2560, 48, 1400, 3),     # 33.2 / 29.9 / 29.6: 3,072 keys
+    (64, 14, 2, 512, 2600, 48, 1400, 1),     # 34.5 / 29.8 / 30.0
+    (128, 28, 4, 128, 2048, 63, 2048, 1),    # 87.5 / 64.1 / 57.6
+    (128, 40, 8, 128, 2048, 127, 1024, 3),   # 141 / 123 / 115
+    (128, 28, 4, 512, 512, 63, 2048, 2),     # 74.6 / -- / 79.9
+    (128, 28, 4, 146, 0, 48, 1400, 3),       # 38.6 / -- / 28.3: 256 blocks, one a unit
+    (128, 28, 4, 147, 0, 48, 1400, 2),       # 38.1 / -- / 28.0
+    (128, 28, 4, 900, 1100, 48, 1400, 2),    # 93.6 / -- / 101
+    (256, 8, 8, 64, 0, 8, 300, 2),           # (no small tiles at such heads)
 ])
 def test_measured_launches_of_a_mixed_step(head_dim, nq, nkv, portion, behind, decoding, their_keys, want):
     lib = attention_library(head_dim)
@@ -382,6 +393,12 @@ def test_measured_launches_of_a_mixed_step(head_dim, nq, nkv, portion, behind, d
     got = lib.llmlab_attention_mixed_launches(nq, nkv, decoding + 1, decoding, portion, behind + portion,
                                               their_keys, 0, CUS)
     assert got == want
+    lib.llmlab_debug_attention_two_launches(-2)                  # (as the switch forces it; heads up to 128)
+    try:
+        assert lib.llmlab_attention_mixed_launches(nq, nkv, decoding + 1, decoding, portion, behind + portion,
+                                                   their_keys, 0, CUS) == (3 if head_dim <= 128 else want)
+    finally:
+        lib.llmlab_debug_attention_two_launches(0)
     # not a mixed step: nobody decodes, or everybody
     assert lib.llmlab_attention_mixed_launches(nq, nkv, 4, 0, portion, behind + portion, 0, 0, CUS) == 0
     assert lib.llmlab_attention_mixed_launches(nq, nkv, 4, 4, portion, behind + portion, their_keys, 0, CUS) == 0

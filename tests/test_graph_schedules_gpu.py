@@ -160,7 +160,7 @@ def test_portions_behind_a_history_beside_decoding_requests(dtype):
                 return H.run_trace(engine, seqs, steps)
         return H.run_trace(engine, seqs, steps)
 
-    if dtype == "bf16":      # (the schedule is one that the rule serves with one launch)
+    if dtype == "bf16":      # (the schedule's last steps are ones that the rule serves with one launch, by tiles of 32 rows)
         ops = H.make_engine("R", 1, dtype, page_size=64, num_pages=4, max_seq_len=128).ops
         lib = ops._attention_lib(cfg.head_dim)
         assert lib.llmlab_attention_mixed_launches(cfg.num_attention_heads, cfg.num_key_value_heads, 4, 3, portion,
