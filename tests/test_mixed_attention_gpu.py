@@ -34,9 +34,31 @@ def test_every_launch(ops, emu, path):  # noqa: F811
 @pytest.mark.parametrize("nq,nkv,d,page", [(14, 2, 64, 64), (7, 1, 16, 16), (12, 2, 128, 32), (4, 4, 112, 16)])
 def test_tiles_of_16_rows(ops, emu, window, nq, nkv, d, page):  # noqa: F811
     """The step in one launch with small tiles: portions that fill no tile, begin in one, or see no key of some waves,
-    behind histories whose keys are split over blocks and not."""
+    behind histories short and long (the switch takes it to that launch whatever the rule says)."""
     for spec in ([(0, 3), (5, 1)], [(0, 17), (900, 1), (64, 1)], [(700, 1), (33, 50), (1500, 1), (0, 129)]):
-        run_attention(ops, emu, torch.bfloat16, nq, nkv, d, page, window, spec, seed=97)
+        with ops.debug.force(attention_small_tiles=d):
+            run_attention(ops, emu, torch.bfloat16, nq, nkv, d, page, window, spec, seed=97)
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3, 7])
+@pytest.mark.parametrize("nq,nkv,d,portion", [(14, 2, 64, 464), (8, 2, 32, 300), (12, 2, 128, 100)])
+def test_tiles_of_16_rows_beside_split_keys(ops, nq, nkv, d, portion, splits):  # noqa: F811
+    """Steps that the rule itself takes there, with the decoding requests' keys split over blocks and merged by the
+    last block to arrive and by a kernel: the same as in a launch for each kind."""
+    decoding = 60 if d < 128 else 40
+    spec = [(1400 - 23 * i, 1) for i in range(decoding)] + [(150, portion), (0, 33)]
+    run, counted = step(ops, torch.bfloat16, nq, nkv, d, 64, spec, 99)
+    how = ops._attention_lib(d).llmlab_attention_mixed_launches(nq, nkv, len(spec), decoding, portion, 1401, 1401, 0, ops.num_cus)
+    assert how == 3, how
+    with ops.debug.force(attention_two_launches=d):
+        want = run(counted)
+    bound = 2e-2 * max(1.0, want.abs().max().item())
+    assert (run(counted) - want).abs().max().item() <= bound
+    for merged in ("attention_merge_kernel", "attention_merge_in_place"):
+        with ops.debug.force(attention_small_tiles=d, attention_splits=(d, splits), **{merged: d}):
+            for described in (counted, tuple(counted)):
+                assert (run(described) - want).abs().max().item() <= bound, (merged, len(described))
+    assert int(ops.arrived.abs().sum()) == 0
 
 
 def step(ops, dtype, nq, nkv, d, page, spec, seed):  # noqa: F811
