@@ -3,9 +3,12 @@
 // for gfx950, with the epilogues the model needs fused in.
 //
 //   bfloat16:  v_mfma_f32_16x16x32_bf16 everywhere.
-//     * tiled kernel: 256 threads = 4 waves, block tile 64x64 (waves 2x2), 64x128 or
+//     * small products: 64x64, four waves 2x2, both operands loaded from global memory straight
+//       into a ring of three stages of LDS (gemm_bf16_ring).
+//     * tiled kernel: 256 threads = 4 waves, block tile 64x128 or
 //       128x128 (waves 1x4, side by side along the columns), or 512 threads = 8 waves on
-//       128x256 (1x8), K step 64; x staged through
+//       128x256 (1x8; widths of 96 to 224 with a wave per 32 columns; 64x64 with waves 2x2 for grouped
+//       products only), K step 64; x staged through
 //       three stages of LDS (rows padded to 80 elements: a wave's 16-byte fragment reads
 //       then take 8.4 clocks, as lane-contiguous ones do; 9.5 with 72, 16 unpadded), its
 //       fragments read into registers half a tile ahead of their products, the fragments
@@ -328,7 +331,9 @@ __device__ __forceinline__ void tile_epilogue(const float* Cs, const EpiArgs& e,
 // the product's first loads: the position, the request and the vectors; `page`, behind those loads: the
 // page, which needs the two; `put`, after the product: into LDS.  Nothing waits for a trip to memory
 // before the product's own first tiles are on their way (put into LDS at once, position, request and page
-// were two trips in a row before them: 512 rows of 1152 x 896 13.5 us, 12.6 now).
+// were two trips in a row before them: 512 rows of 1152 x 896 13.5 us, 12.6 now).  The tiles of two groups of waves
+// alone ask for the page before their first loads: one trip that their products of 50 us and more do not show (700 to 2,560
+// rows of 4608 x 3584, 2560 x 2048, 1152 x 896 and 6144 x 4096 the other way round: the same within 1 %).
 template <int BM, int BN, int NT>
 struct QkvRows {
   static_assert(BM <= NT && BN <= 2 * NT && NT >= 128, "a row, two columns and a frequency a thread");
@@ -569,7 +574,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
 // one load, one fragment, in a ring of four steps).  A load of x takes 8 rows of 128 bytes, two
 // steps of the inner size, neighbouring lanes in the same row, so that a load touches eight lines
 // and takes them whole; with one fragment a load (16 rows of 64 bytes, neighbouring lanes in
-// different rows) it touched 64 half lines, and 2367 rows of 37888 x 3584 took 597 us instead of 522,
+// different rows) it touched 16 half lines, each by four lanes far apart, and 2367 rows of 37888 x 3584 took 597 us instead of 522,
 // of 3584 x 18944 322 instead of 286, 2048 of 22016 x 2048 191 instead of 169, of 3584 x 18944
 // 317 instead of 273 (16 rows of 64 bytes with neighbouring lanes in one row: 539, 280, 178, 319).
 // A piece of x is half of the tile's rows of two steps: NG of them in a ring, one fetched a step,
@@ -784,8 +789,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
 }
 
 // ============================================================ bf16, small tiles by direct loads
-// Small products: four waves 2 x 2 on a tile of BM x BN, both operands by direct loads into LDS as in the kernel
-// above (x 8 rows of 128 bytes a load, W by fragments), in stages of 64 of the inner size, NST of them.  What
+// Small products: four waves 2 x 2 on a tile of 64 x 64, both operands by direct loads into LDS as in the kernel
+// above (x 8 rows of 128 bytes a load, W by fragments), in stages of 64 of the inner size, three of them.  What
 // bounds such a product is its few blocks' way through launch, first trip to memory, K tiles and epilogue; here no
 // operand passes through registers on its way, every stage but one is on its way at any time, a stage
 // takes one barrier, and three blocks of the 64 x 64 tile (48 KB) share a unit.  Against the same tile with x by way of registers and W
@@ -794,9 +799,10 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
 // unit): 4 % slower.  Larger tiles of this kind: 64 x 128 (three stages) is slower than the tile above with many
 // rows (512 of 9728 x 896 24.8 against 21.4) and faster in pieces of few rows only (64 of 3584 x 18944 28.2 against 32.4), 128 x 160
 // and 128 x 256 as fast as theirs (128 of 37888 x 3584 71.8 against 73.7): not kept.
-template <int BM, int BN, int NST, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                       EpiArgs e, int M, int N, int K) {
+  constexpr int BM = 64, BN = 64, NST = 3;
   constexpr int NT = 256, WTM = BM / 2, WTN = BN / 2, TM = WTM / 16, TN = WTN / 16;
   constexpr int XL = BM / 8, WL = BN / 8, NL = (XL + WL) / 4;      // loads of 1 KB of a stage: of x, of W, of one wave
   static_assert((XL + WL) % 4 == 0 && WTM % 16 == 0 && WTN % 16 == 0 && NL * (NST - 2) < 64, "shape");
@@ -1502,11 +1508,11 @@ static void launch_f32_rows(const float* A, const float* W, const EpiArgs& e, in
 constexpr int F32_ROWS_MAX = 64;     // up to here the few-row kernel (the tiled one would run on N / 64 blocks)
 
 // ================================================================ dispatch
-// Four tile shapes with x through LDS and W straight from the packed matrix: 64 x 64 (four
-// waves 2 x 2) for small products; 64 x 128 and 128 x 128 with four waves and 128 x 256
+// The 64 x 64 tile of gemm_bf16_ring for small products; three tile shapes with x through LDS and W straight
+// from the packed matrix, 64 x 128 and 128 x 128 with four waves and 128 x 256
 // with eight, side by side along the columns (1 x 4, 1 x 8), so that every fragment of W
 // is read by one wave only and the rows of x in LDS are shared by all of them; and the
-// 256 x 256 tile of gemm_bf16_pingpong for the largest products.  The shape
+// 256 x 256 and 192 x 256 tiles of gemm_bf16_pingpong for the largest products.  The shape
 // is picked by an estimate of the time, fitted to sweeps of the four products of a layer
 // at three model shapes and 576 to 8192 rows (its picks cost 0.8 % over the best shape
 // there):
@@ -1528,6 +1534,8 @@ struct TileModel {
   double L, f, tk, resident, stream;
   int whole_rounds;
 };
+// (the 64 x 64 row was fitted to a kernel that took x by way of registers, slower by 18 %; in the range of
+// few_blocks_cost that decides)
 static const TileModel TILE_MODELS[TILE_ALL] = {{64, 64, 6.39, 0.79, 0.289, 1.0, 20e3, 0},
                                                   {64, 128, 6.54, 0.71, 0.5, 1.5, 27e3, 0},
                                                   {128, 128, 8.0, 0.48, 0.66, 1.0, 24e3, 0},
@@ -1814,7 +1822,7 @@ static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArg
   const TileModel& t = TILE_MODELS[kind];
   dim3 grid((N + t.bn - 1) / t.bn, (M + t.bm - 1) / t.bm, pieces);
   if (kind == TILE_64)
-    hipLaunchKernelGGL((gemm_bf16_ring<64, 64, 3, EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
+    hipLaunchKernelGGL((gemm_bf16_ring<EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
   else if (kind == TILE_64x128)
     hipLaunchKernelGGL((gemm_bf16_tiled<64, 128, 64, 1, 4, EPI>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
   else if (kind == TILE_128)

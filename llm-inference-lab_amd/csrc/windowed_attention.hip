@@ -1083,10 +1083,10 @@ __global__ __launch_bounds__(256) void sink_window_attention_mfma_kernel(MfmaArg
 // consecutive rows and up to FOUR heads of one key/value head, a wave a head (a group of seven heads: a
 // block of four and one of three, whose last wave only helps to stage).  The block
 // stages every tile of 32 keys and their values in LDS once (each thread asks for its 16-byte
-// pieces two tiles ahead and stores them a tile ahead), and the waves take their fragments from
+// pieces three tiles ahead and stores them one ahead; values of 224 and more: one ahead), and the waves take their fragments from
 // there instead of each from L2.  Key rows lie 16 bytes apart from a
 // multiple of 256 bytes and the values' quad rows 128, so that the lanes of a read spread over the
-// banks.  Two stages of LDS: the next tile is put down while this one is taken, a barrier a
+// banks.  Two stages of LDS (values of 224 and more: one): the next tile is put down while this one is taken, a barrier a
 // tile.  The list of tiles, the masks and the transposed products are the kernel's above; all waves of
 // a block walk the same tiles, so the barriers are reached by all.
 //
@@ -1094,7 +1094,8 @@ __global__ __launch_bounds__(256) void sink_window_attention_mfma_kernel(MfmaArg
 // tiles, 34 to 64 of them one after the other, and its waits.  Page numbers come by scalar
 // loads a tile ahead: as vector loads they stood behind the keys and values in flight, and waiting for one was waiting for
 // all; the loads of keys and values have no branch.  1,900 rows over
-// 1,032 keys, 14 heads of 64: 50.5 -> 43.1 us, the same numbers to the bit.  (With the running maximum raised only where a
+// 1,032 keys, 14 heads of 64: 50.5 -> 43.1 us, the same numbers to the bit; a prompt of 1,900 rows from its start, 16 heads of 128
+// over 4 96 -> 87, 12 over 3 with keys of 128 and values of 256 119 -> 113, 12 over 2 of 224 133 -> 121, 16 over 4 of 256 138 -> 129.  (With the running maximum raised only where a
 // score exceeds it by 2^8 and a lane's weights summed by itself 40.0, but a model of sharp scores is then further off.)
 template <int DC, int EB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void sink_window_attention_shared_kernel(MfmaArgs a) {
@@ -1154,9 +1155,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     // (the table is not written while the kernel runs: page numbers come by scalar loads, whose wait is not
     // also one for the keys and values in flight)
     const auto pages = (const __attribute__((address_space(4))) int*)(a.table + (size_t)b * a.max_pages);
-    // Two sets of staging registers: a tile's pieces are asked for TWO tiles ahead and stored one
-    // tile ahead, so that their way from memory lies behind the products of a whole tile and
-    // more (the longest block's tiles, one after the other, are what a prompt's attention takes).
+    // Two sets of staging registers: while tile t is taken, t + 1 is put into the other stage, t + 2 is on its way
+    // and t + 3 is asked for, so that their way from memory lies behind the products of two tiles
+    // (the longest block's tiles, one after the other, are what a prompt's attention takes).  One stage: one set,
+    // asked for while tile t is taken and put down behind it.
     bf16x8 k_a[KCH], v_a[VCH], k_b[KCH], v_b[VCH];
     // The pages of a tile's two halves are looked up one fetch ahead (a lookup in front of its own loads
     // is a trip to memory that every tile would wait for).

@@ -1017,9 +1017,9 @@ class HipOps:
 
     # -------------------------------------------------------------- attention
     def attention_short_limit(self, num_heads: int, num_kv_heads: int, dtype, max_q_len: int) -> int:
-        """A mixed step (portions of prompts beside decoding requests) is served by two
-        launches: its requests of a few tokens go to the one that splits their keys over
-        the chip, the portions to the tiled one.  Returns the most tokens a request may
+        """A mixed step (portions of prompts beside decoding requests) has blocks of two kinds, in one
+        launch or in one each: those of its requests of a few tokens split the keys over
+        the chip, those of the portions are tiles of rows.  Returns the most tokens a request may
         bring to count as short in such a step, or 0 if the step is not divided."""
         group = num_heads // num_kv_heads
         if group <= 16 < max_q_len * group:
