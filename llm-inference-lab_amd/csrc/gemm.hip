@@ -1937,7 +1937,8 @@ extern "C" int llmlab_pieces_tile(int M, int N, int K, int num_cus, int pieces) 
 
 // Whether (and into how many pieces along K) a product that adds into float32 rows should
 // be left unsummed, and with which tile: out = {pieces (1: no), tile kind}; in one piece the kind is that
-// of a whole product (choose_tile).  A piece costs a write and a read of the result by whoever sums it up later.
+// of a whole product (choose_tile; up to 128 rows of a wide matrix one_round_tile's widths go before it, which make
+// no pieces).  A piece costs a write and a read of the result by whoever sums it up later.
 extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pieces, int min_tiles_per_piece,
                                    int* out) {
   if (num_cus <= 0) num_cus = 256;

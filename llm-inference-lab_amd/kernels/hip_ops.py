@@ -755,9 +755,9 @@ class HipOps:
         plan(rows, n, k, self.num_cus, self.MAX_SPLITS, self.rules.min_tiles_per_split, out)
         return out[0], out[1]
 
-    def _pieces_tile(self, rows: int, n: int, k: int, dtype, pieces: int) -> int:
-        """The tile of such a product cut into ``pieces``, which need not be the plan's number."""
-        planned, tile = self._linear_plan(rows, n, k, dtype)
+    def _pieces_tile(self, rows: int, n: int, k: int, dtype, pieces: int, plan=None) -> int:
+        """The tile of such a product cut into ``pieces``, which need not be the number of its ``plan``."""
+        planned, tile = plan or self._linear_plan(rows, n, k, dtype)
         if dtype != torch.bfloat16 or pieces == planned:
             return tile
         return self._core.llmlab_pieces_tile(rows, n, k, self.num_cus, pieces)
@@ -883,7 +883,8 @@ class HipOps:
             return None
         if rows > self.FEW_ROWS and self.few_rows_take(rows, n, k):
             return None
-        pieces = self._linear_plan(rows, n, k)[0]
+        plan = self._linear_plan(rows, n, k)
+        pieces = plan[0]
         if rows > self.FEW_ROWS and k >= 2 * 64 * self.rules.min_tiles_per_split:
             # (65 to 384 rows: two pieces at least.  4608 x 3584 at 192 / 256 rows: 24 / 31 us
             # against 33 / 39 whole; 2560 x 2048: 15 / 18.5 against 20.5; the estimate of
@@ -892,7 +893,7 @@ class HipOps:
         if self.rules.forced_tiled_pieces:
             pieces = max(1, min(self.rules.forced_tiled_pieces, (k + 63) // 64, self.MAX_SPLITS))
         if pieces > 1 and pieces * rows * n <= self.workspace.numel():
-            return pieces, self._pieces_tile(rows, n, k, torch.bfloat16, pieces)
+            return pieces, self._pieces_tile(rows, n, k, torch.bfloat16, pieces, plan)
         return None
 
     def qkv_rope_cache(self, h, w_qkv, b_qkv, num_heads, num_kv_heads, head_dim, inv_freq, positions,
