@@ -74,6 +74,24 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// The same for waves whose 64 lanes are all active: within rows of sixteen lanes by the operand swizzles
+// of DPP, across the rows by the lane-swap instructions of gfx950.  (wave_sum above takes six trips through
+// the LDS crossbar, one behind the other.)
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float full_wave_sum(float v) {
+  v += dpp_move<0xB1>(v);       // lanes 1 apart (quad_perm 1, 0, 3, 2)
+  v += dpp_move<0x4E>(v);       // 2 apart (quad_perm 2, 3, 0, 1)
+  v += dpp_move<0x141>(v);      // the other four of eight (row_half_mirror)
+  v += dpp_move<0x140>(v);      // the other eight of sixteen (row_mirror)
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result.
 // `red` is shared memory of at least 17 floats.
 __device__ __forceinline__ float block_sum(float v, float* red) {

@@ -28,8 +28,18 @@
 // of the same read, and inv_rms[m] scales the reduced sums in the epilogue.
 //
 // What the epilogue needs from global memory (bias, positions, page numbers,
-// rotary frequencies, the residual value it adds to) is fetched at the start of the
+// rotary frequencies, the residual value it adds to) is asked for at the start of the
 // kernel, so those latencies overlap the weight stream instead of following it.
+//
+// What a block does before its first load counts: a wave issues about 450 instructions a
+// microsecond, and loads come back in the order they were asked for.  So the rows of x are
+// asked for first, then what the epilogue needs, then the weights; nothing is waited for in between;
+// sizes that need a division come from the host (SkinnyArgs).  By clock stamps inside the kernels
+// (0.5B shape, one row, from a block's start): gate/up has all its loads on their way after 0.5 us and its
+// rows staged after 1.1 (0.9 and 2.9 with the weights first), q/k/v, which waited for positions and pages as
+// well, after 1.5 and 2.7 (2.6 and 3.9).  A decode step of 8 requests in
+// float32 takes 1,286 us where it took 1,371; in bfloat16, together with the merge of the attention's waves, 1 / 8 / 64
+// requests 854 / 942 / 1,461 -> 785 / 906 / 1,392 us, 8 of the 7B shape 3,801 -> 3,697.
 //
 // A compute unit draws only about 50 GB/s from HBM, so a product with a narrow
 // output (few strips, hence few blocks) is bound by the units it uses, not by the
@@ -97,7 +107,16 @@ struct SkinnyArgs {
   int seg_end[7];
   size_t seg_stride;
   int tiles;       // tiles of 16 MB rows
-  int col_blocks;  // blocks that a tile of rows takes (sets of columns, times ksplit)
+  int col_blocks;  // blocks that a tile of rows takes (sets of columns); grid y counts the groups of K
+  // What every block would otherwise work out before its first load:
+  int threads;         // of a block
+  int nsb_inv;         // ceil(65536 / nsb): n / nsb is (n * nsb_inv) >> 16 for n < 4096
+  unsigned tiles_inv;  // ceil(2^32 / tiles), tiles > 1: j / tiles is the upper half of j * tiles_inv
+  unsigned qsplit_inv; // the same of qsplit, qsplit > 1
+  int steps;           // steps of the inner size
+  int group_steps;     // ... of a group of K
+  int wave_steps;      // ... of a wave
+  int wpr_shift;       // log2 of the waves that share a staged row
 };
 
 __device__ __forceinline__ float sk_silu(float z) { return z / (1.f + __expf(-z)); }
@@ -192,16 +211,14 @@ __host__ __device__ constexpr int sk_ring(int mb, bool stage) {
   return stage ? SK_RING_STAGE : (mb >= 4 ? SK_RING_DIRECT / 2 : SK_RING_DIRECT);
 }
 
-constexpr int SK_STAGE_U_PIECES = 1;
 constexpr int SK_APAD = 16;  // padding of a staged row, in bytes: 16-byte reads of 8 lanes cover all banks
 
 // floats of LDS before the staged rows (host and device must agree)
-__host__ __device__ inline size_t sk_float_words(int nsb, int kw, int mb, int M, int epi) {
+__host__ __device__ inline size_t sk_float_words(int nsb, int kw, int mb) {
   size_t f = (size_t)kw * nsb * mb * 256;        // partial sums
   f += (size_t)mb * 16 + 16;                      // inverse rms; sums of squares of the parts of a row
   f += (size_t)16 * nsb;                          // bias
   f += (size_t)mb * 16 * 2 + 128;                 // positions, pages, frequencies
-  if (epi == SK_SWIGLU || epi == SK_QKV) f += (size_t)M * 16 * nsb;
   return (f + 3) & ~(size_t)3;
 }
 
@@ -211,6 +228,9 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   using S = SkStep<T>;
   using Frag = typename S::frag;
   extern __shared__ __attribute__((aligned(16))) float smem[];
+  // (the arguments that the first loads need come in one trip, not in one per branch that leads to them)
+  asm volatile("" :: "s"(a.tiles), "s"(a.nsb), "s"(a.threads), "s"(a.nsb_inv), "s"(a.steps), "s"(a.group_steps),
+               "s"(a.wave_steps), "s"(a.wpr_shift), "s"(a.M), "s"(a.K), "s"(a.x), "s"(a.W), "s"(a.norm_w), "s"(a.pend_splits), "s"(a.norm_w_bf16));
   // Rows in tiles of 16 MB: a block sees its tile as if it were the whole product,
   // through pointers moved to the tile's first row.  The tiles of one set of columns
   // read the same part of W: they get block numbers that are equal modulo 8 (the
@@ -218,8 +238,8 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   int col_block = (int)blockIdx.x;
   if (a.tiles > 1) {
     const int xcd = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
-    const int tile = j % a.tiles;
-    col_block = (j / a.tiles) * 8 + xcd;
+    const int jt = (int)__umulhi((unsigned)j, a.tiles_inv), tile = j - jt * a.tiles;
+    col_block = jt * 8 + xcd;
     if (col_block >= a.col_blocks) return;      // (the grid is rounded up to whole eights)
     const int m0 = tile * (MB * 16);
     a.M = min(MB * 16, a.M - m0);
@@ -238,17 +258,18 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   }
   constexpr int R = sk_ring(MB, STAGE);   // K steps whose loads a wave keeps in flight
   const int nsb = a.nsb, kw = a.kw;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-  const int strip = wave % nsb, ks = wave / nsb;
+  const int lane = threadIdx.x & 63, nwaves = a.threads >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // (what follows from it stays scalar)
+  auto by_nsb = [&](int n) { return (n * a.nsb_inv) >> 16; };
+  const int ks = by_nsb(wave), strip = wave - ks * nsb;
   const int c = lane & 15, g = lane >> 4;
   const int cols = 16 * nsb;
   // SK_PART: the blocks of one K group follow each other
-  const int nblk = (EPI == SK_PART) ? a.col_blocks / a.ksplit : a.col_blocks;
-  const int ksp = (EPI == SK_PART) ? col_block / nblk : 0;
-  const int bidx = (EPI == SK_PART) ? col_block - ksp * nblk : col_block;
+  const int ksp = (EPI == SK_PART) ? (int)blockIdx.y : 0;
+  const int bidx = col_block;
   const int n0 = bidx * cols;
   const int K = a.K, M = a.M;
-  const int steps = (K + S::LEN - 1) / S::LEN;     // bfloat16: W is packed and zero-padded to this; float32: whole steps
+  const int steps = a.steps;     // bfloat16: W is packed and zero-padded to this; float32: whole steps
 
   float* part = smem;                                   // [kw*nsb][MB][64][4]
   float* inv = part + (size_t)kw * nsb * MB * 256;      // [MB*16]
@@ -257,15 +278,14 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   int* s_pos = (int*)(s_bias + cols);                   // [MB*16]
   int* s_page = s_pos + MB * 16;                        // [MB*16]
   float* s_freq = (float*)(s_page + MB * 16);           // [128]
-  float* tile = s_freq + 128;                           // [M][cols]   (SWIGLU, QKV)
-  T* As = (T*)(smem + sk_float_words(nsb, kw, MB, M, EPI));   // [M][steps * S::LEN + padding]
+  T* As = (T*)(smem + sk_float_words(nsb, kw, MB));   // [M][steps * S::LEN + padding]
   const int lda = steps * S::LEN + SK_APAD / (int)sizeof(T);
 
   // QKV with qsplit > 1: block = (head, p); its two strips are columns p*16.. and
   // d/2 + p*16.. of the head, i.e. both halves of the rotary pairs
   int qhead = 0, qp = 0;
   if constexpr (EPI == SK_QKV) {
-    qhead = bidx / a.qsplit;
+    qhead = a.qsplit == 1 ? bidx : (int)__umulhi((unsigned)bidx, a.qsplit_inv);
     qp = bidx - qhead * a.qsplit;
   }
   auto head_col = [&](int col) {   // column of the block -> column of the head
@@ -277,52 +297,74 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   int wstrip = (EPI == SK_QKV) ? (qhead * a.d + head_col(strip * 16)) >> 4 : bidx * nsb + strip;
   wstrip = min(wstrip, ((a.N + 15) >> 4) - 1);
   constexpr bool PACKED = sizeof(T) == 2;
-  const T* wp = PACKED ? (const T*)a.W + (size_t)wstrip * steps * 512 + lane * 8
-                       : (const T*)a.W + (size_t)min(wstrip * 16 + c, a.N - 1) * K + g * S::PER;
+  // (the address of a step: a scalar part and 32 bits of a lane's own)
+  const char* const wstart = (const char*)a.W + (size_t)wstrip * (PACKED ? (size_t)steps * 1024 : (size_t)64 * K);
+  const uint32_t wlane = PACKED ? lane * 16 : ((uint32_t)min(c, a.N - 1 - wstrip * 16) * K + g * S::PER) * 4;
   // this block's K steps (all of them, or its group's share), split over its waves
-  const int gsteps = (EPI == SK_PART) ? (steps + a.ksplit - 1) / a.ksplit : steps;
-  const int g_begin = ksp * gsteps, g_end = min(steps, g_begin + gsteps);
-  const int per = (max(g_end - g_begin, 0) + kw - 1) / kw;
-  const int s_begin = g_begin + ks * per;
-  const int s_end = min(g_end, s_begin + per);
+  const int g_begin = ksp * a.group_steps, g_end = min(steps, g_begin + a.group_steps);
+  const int s_begin = g_begin + ks * a.wave_steps;
+  const int s_end = min(g_end, s_begin + a.wave_steps);
   const Frag zero = {};
   const floatx4 fzero = {0.f, 0.f, 0.f, 0.f};
 
-  // ---- what the epilogue needs from global memory, fetched now
-  for (int i = threadIdx.x; i < cols; i += blockDim.x) {
-    const int nn = (EPI == SK_QKV) ? qhead * a.d + head_col(i) : n0 + i;
-    s_bias[i] = (a.bias && nn < a.N && ksp == 0) ? load_vec(a.bias, a.bias_bf16, nn) : 0.f;
-  }
-  if constexpr (EPI == SK_QKV) {
-    const int head = qhead;
-    for (int m = threadIdx.x; m < M; m += blockDim.x) {
-      const int pos = a.positions[m];
-      s_pos[m] = pos;
-      s_page[m] = (a.kcache && head >= a.nq)
-                      ? a.table[(size_t)a.row_req[m] * a.table_stride + pos / a.page_size] : 0;
+  // ---- What the epilogue needs from global memory is asked for at the start, behind the first rows of x and
+  // before the weights, and used at the end: a thread keeps its bias, frequency, position and residual value in
+  // registers until the sums are there.  Loads come back in the order they were asked for, so nothing of it
+  // may be waited for before the weights are asked for.  All loads are unconditional (indexes clamped,
+  // other arrays in the place of absent ones).
+  // (a block has at least four threads per column, one per row and one per frequency)
+  const int tid = threadIdx.x;
+  const bool has_bias = a.bias && ksp == 0;
+  uint16_t bias_lo = 0, bias_hi = 0;
+  int pos_v = 0, req_v = 0;
+  float freq_v = 0.f;
+  const bool wants_page = EPI == SK_QKV && a.kcache && qhead >= a.nq;
+  // the residual value this thread will add to (its first one), and the first pieces owed to it
+  constexpr int RP = EPI != SK_RESID ? 1 : sizeof(T) == 4 ? 4 : 8;
+  float resid_old = 0.f, resid_pieces[RP];
+  auto ask_for_epilogue = [&] {
+    if constexpr (EPI == SK_QKV) {
+      const int row = min(tid, M - 1);
+      pos_v = a.positions[row];
+      req_v = (a.row_req ? a.row_req : a.positions)[row];
+      freq_v = (a.inv_freq ? a.inv_freq : (const float*)a.W)[min(tid, (a.d >> 1) - 1)];
     }
-    for (int i = threadIdx.x; i < (a.d >> 1); i += blockDim.x)
-      s_freq[i] = a.inv_freq ? a.inv_freq[i] : 0.f;
-  }
-
-  // the residual value this thread will add to (its first one): on its way now, not
-  // after the reduction
-  float resid_old = 0.f;
-  if constexpr (EPI == SK_RESID) {
-    const int idx = threadIdx.x;
-    const int m = idx / cols, nn = n0 + idx - m * cols;
-    if (idx < M * cols && nn < a.N) {
+    if constexpr (EPI != SK_SWIGLU) {
+      const int col = min(tid, cols - 1);
+      const int nn = min((EPI == SK_QKV) ? qhead * a.d + head_col(col) : n0 + col, a.N - 1);
+      const uint16_t* at = has_bias ? (const uint16_t*)a.bias + (size_t)nn * (a.bias_bf16 ? 1 : 2) : (const uint16_t*)a.W;
+      int upper = has_bias && !a.bias_bf16 ? 1 : 0;
+      asm volatile("" : "+v"(upper));      // (else two paths, one of which waits for the first load)
+      bias_lo = at[0];
+      bias_hi = at[upper];
+    }
+    if constexpr (EPI == SK_RESID) {
+      const int m = min(by_nsb(tid >> 4), M - 1), nn = min(n0 + tid - by_nsb(tid >> 4) * cols, a.N - 1);
       resid_old = ((const float*)a.out)[(size_t)m * a.ldo + nn];
-      for (int sp0 = 0; sp0 < a.pend_splits; sp0 += 4) {      // four pieces at a time, as above
-        float pp[4];
+      const float* from = a.pend_splits > 0 ? a.pend + (size_t)m * a.pend_ld + nn : (const float*)a.out;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          pp[j] = a.pend[min(sp0 + j, a.pend_splits - 1) * a.pend_stride + (size_t)m * a.pend_ld + nn];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) resid_old += sp0 + j < a.pend_splits ? pp[j] : 0.f;
-      }
+      for (int j = 0; j < RP; ++j) resid_pieces[j] = from[max(min(j, a.pend_splits - 1), 0) * a.pend_stride];
     }
-  }
+  };
+  // pages of the rows, once their positions are known; and everything to LDS for the epilogue, before
+  // the barrier that the sums wait at
+  int page_v = 0;
+  auto ask_for_pages = [&] {
+    if constexpr (EPI == SK_QKV)
+      if (wants_page) page_v = a.table[(size_t)req_v * a.table_stride + pos_v / a.page_size];
+  };
+  auto leave_for_epilogue = [&] {
+    if (tid < cols)
+      s_bias[tid] = !has_bias ? 0.f : __uint_as_float(((uint32_t)(a.bias_bf16 ? bias_lo : bias_hi) << 16) |
+                                                      (a.bias_bf16 ? 0u : (uint32_t)bias_lo));
+    if constexpr (EPI == SK_QKV) {
+      if (tid < M) {
+        s_pos[tid] = pos_v;
+        s_page[tid] = page_v;
+      }
+      if (tid < (a.d >> 1)) s_freq[tid] = a.inv_freq ? freq_v : 0.f;
+    }
+  };
 
   floatx4 acc[MB][S::SUMS];
 #pragma unroll
@@ -333,127 +375,169 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   // Loads in the ring are unconditional (a step past the end reads the last tile
   // again and is multiplied by zeros): a load under a branch makes the compiler wait
   // for every load in flight at the join, and the stream stalls once per round.
+  const int s_last = max(0, min(s_end, steps) - 1);      // (a wave past the end: any step that is there)
   auto wload = [&](int st) {
-    return *(const Frag*)(wp + (size_t)max(0, min(st, steps - 1)) * (PACKED ? 512 : S::LEN));
+    return *(const Frag*)(wstart + (wlane + (uint32_t)min(st, s_last) * (PACKED ? 1024u : 64u)));
   };
   Frag b[R];
 
   if constexpr (STAGE) {
-#pragma unroll
-    for (int u = 0; u < R; ++u) b[u] = wload(min(s_begin + u, s_end - 1));
-    // ---- the first weight tiles are on their way; stage the rows of x
+    // ---- Stage the rows of x.  Their first loads go out before those of the weights, which follow at
+    // once: loads come back in the order they were asked for, so a wave that asked for its
+    // weights first staged its rows only when its whole ring was there (gate/up of one row of the 0.5B shape:
+    // 2.0 us from the first load to the barrier).
     // Fewer rows than waves: `wpr` waves share a row, each taking every wpr-th run of 64
     // chunks (one wave alone would walk a long row in many trips while the others wait)
     const int chunks = K >> 3, chunks_pad = steps * (S::LEN / 8);
-    int wpr = 1;
-    while (2 * wpr * M <= nwaves) wpr *= 2;
+    const int wpr_shift = a.wpr_shift, wpr = 1 << wpr_shift;
     // A wave walks its part of a row U chunks at a time: the loads of all U (the row, the
-    // norm's weight, the pieces owed) are on their way before the first is used, so a part
+    // norm's weight, the first four pieces owed) are on their way before the first is used, so a part
     // costs one trip to memory per U chunks and not one per chunk.  Loads are unconditional
     // (a chunk past the end reads the last one again and is not stored).
-    auto stage_rows = [&](auto u_tag, auto w_tag) {
+    auto stage_rows = [&](auto u_tag, auto w_tag, auto pieces_tag) {
       constexpr int U = decltype(u_tag)::value;
       constexpr bool W_BF16 = decltype(w_tag)::value;     // (the norm's weight: no branch among the loads)
-      const int stride = 64 * wpr;
-      for (int unit = wave; unit < M * wpr; unit += nwaves) {
-        const int r = unit / wpr, sub = unit - r * wpr;
-        T* dst = As + (size_t)r * lda;
-        if constexpr (NORM) {
-          const float* src = (const float*)a.x + (size_t)(a.x_rows ? a.x_rows[r] : r) * K;
-          float ssq = 0.f;
-          const size_t prow = (size_t)(a.x_rows ? a.x_rows[r] : r) * a.pend_ld;
-          for (int ch0 = sub * 64 + lane; ch0 < chunks; ch0 += U * stride) {
-            floatx4 p[U], q[U], w0[U], w1[U];
-            bf16x8 w8[U];
-            int chs[U];
+      constexpr bool PIECES = decltype(pieces_tag)::value;
+      const int stride = 64 * wpr, units = M * wpr;
+      floatx4 p[U], q[U], w0[U], w1[U], pp[U][4], qq[U][4];
+      bf16x8 w8[U];
+      Sk8<T> v[U];
+      size_t row = 0;
+      auto start_row = [&](int unit) {
+        const int r = unit >> wpr_shift;
+        row = NORM && a.x_rows ? a.x_rows[r] : r;
+      };
+      auto load_pieces = [&](int base, int sp0) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-              chs[u] = min(ch0 + u * stride, chunks - 1);
-              p[u] = *(const floatx4*)(src + chs[u] * 8);
-              q[u] = *(const floatx4*)(src + chs[u] * 8 + 4);
-              if constexpr (W_BF16) {
-                w8[u] = *(const bf16x8*)((const bf16_t*)a.norm_w + chs[u] * 8);
-              } else {
-                w0[u] = *(const floatx4*)((const float*)a.norm_w + chs[u] * 8);
-                w1[u] = *(const floatx4*)((const float*)a.norm_w + chs[u] * 8 + 4);
-              }
-            }
-            // sums still owed to these rows: four pieces at a time for every chunk, loads
-            // unconditional (past the last piece: the last one again, not added)
-            for (int sp0 = 0; sp0 < a.pend_splits; sp0 += 4) {
-              floatx4 pp[U][4], qq[U][4];
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-              for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                  const float* src2 = a.pend + min(sp0 + j, a.pend_splits - 1) * a.pend_stride + prow + chs[u] * 8;
-                  pp[u][j] = *(const floatx4*)src2;
-                  qq[u][j] = *(const floatx4*)(src2 + 4);
-                }
-#pragma unroll
-              for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                  const float on = sp0 + j < a.pend_splits ? 1.f : 0.f;
-                  p[u] += pp[u][j] * on;
-                  q[u] += qq[u][j] * on;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              if (ch0 + u * stride >= chunks) break;
-              float wv[8];
-              if constexpr (W_BF16) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) wv[j] = (float)w8[u][j];
-              } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                  wv[j] = w0[u][j];
-                  wv[4 + j] = w1[u][j];
-                }
-              }
-              Sk8<T> av;
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                ssq += p[u][j] * p[u][j] + q[u][j] * q[u][j];
-                av.set(j, p[u][j] * wv[j]);
-                av.set(4 + j, q[u][j] * wv[4 + j]);
-              }
-              av.store(dst + chs[u] * 8);
-            }
+          for (int j = 0; j < 4; ++j) {
+            const float* src = a.pend + min(sp0 + j, a.pend_splits - 1) * a.pend_stride + row * a.pend_ld +
+                               min(base + u * stride + lane, chunks - 1) * 8;
+            pp[u][j] = *(const floatx4*)src;
+            qq[u][j] = *(const floatx4*)(src + 4);
           }
-          ssq = wave_sum(ssq);
-          if (lane == 0) {
-            if (wpr == 1) inv[r] = rsqrtf(ssq / (float)K + a.eps);
-            else s_ssq[unit] = ssq;       // (M * wpr <= 16 waves)
-          }
-        } else {
-          const T* src = (const T*)a.x + (size_t)r * K;
-          for (int ch0 = sub * 64 + lane; ch0 < chunks; ch0 += U * stride) {
-            Sk8<T> v[U];
+      };
+      auto load = [&](int base) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[u].load(src + min(ch0 + u * stride, chunks - 1) * 8);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-              if (ch0 + u * stride < chunks) v[u].store(dst + (ch0 + u * stride) * 8);
+        for (int u = 0; u < U; ++u) {
+          const int ch = min(base + u * stride + lane, chunks - 1);
+          if constexpr (NORM) {
+            const float* src = (const float*)a.x + row * K + ch * 8;
+            p[u] = *(const floatx4*)src;
+            q[u] = *(const floatx4*)(src + 4);
+            if constexpr (W_BF16) {
+              w8[u] = *(const bf16x8*)((const bf16_t*)a.norm_w + ch * 8);
+            } else {
+              w0[u] = *(const floatx4*)((const float*)a.norm_w + ch * 8);
+              w1[u] = *(const floatx4*)((const float*)a.norm_w + ch * 8 + 4);
+            }
+          } else {
+            v[u].load((const T*)a.x + row * K + ch * 8);
           }
         }
-        if (sub == 0)
+        if constexpr (PIECES) load_pieces(base, 0);
+      };
+      auto store = [&](int base, T* dst, float& ssq) {
+        if constexpr (PIECES) {
+          for (int sp0 = 0; sp0 < a.pend_splits; sp0 += 4) {      // in their order
+            if (sp0 > 0) load_pieces(base, sp0);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const float on = sp0 + j < a.pend_splits ? 1.f : 0.f;
+                p[u] += pp[u][j] * on;
+                q[u] += qq[u][j] * on;
+              }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int ch = base + u * stride + lane;
+          if (ch >= chunks) break;
+          if constexpr (NORM) {
+            float wv[8];
+            if constexpr (W_BF16) {
+#pragma unroll
+              for (int j = 0; j < 8; ++j) wv[j] = (float)w8[u][j];
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                wv[j] = w0[u][j];
+                wv[4 + j] = w1[u][j];
+              }
+            }
+            Sk8<T> av;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              ssq += p[u][j] * p[u][j] + q[u][j] * q[u][j];
+              av.set(j, p[u][j] * wv[j]);
+              av.set(4 + j, q[u][j] * wv[4 + j]);
+            }
+            av.store(dst + ch * 8);
+          } else {
+            v[u].store(dst + ch * 8);
+          }
+        }
+      };
+      // (a wave without a part of its own asks for the last one's again and stores nothing)
+      int unit = min(wave, units - 1);
+      start_row(unit);
+      load((unit & (wpr - 1)) * 64);
+      __builtin_amdgcn_sched_barrier(0);
+      ask_for_epilogue();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < R; ++u) b[u] = wload(s_begin + u);
+      __builtin_amdgcn_sched_barrier(0);
+      if (wave >= units) return;
+      float ssq = 0.f;
+      int base = (unit & (wpr - 1)) * 64;
+      T* dst = As + (size_t)(unit >> wpr_shift) * lda;
+      store(base, dst, ssq);      // (by itself: in the loop below the loads of W behind these would be waited for, too)
+      for (;;) {
+        for (base += U * stride; base < chunks; base += U * stride) {
+          load(base);
+          store(base, dst, ssq);
+        }
+        if constexpr (NORM) {
+          ssq = full_wave_sum(ssq);
+          if (lane == 0) {
+            if (wpr == 1) inv[unit] = rsqrtf(ssq / (float)K + a.eps);
+            else s_ssq[unit] = ssq;       // (M * wpr <= 16 waves)
+          }
+        }
+        if ((unit & (wpr - 1)) == 0)
           for (int ch = chunks + lane; ch < chunks_pad; ch += 64) Sk8<T>{}.store(dst + ch * 8);
+        unit += nwaves;
+        if (unit >= units) return;
+        start_row(unit);
+        ssq = 0.f;
+        dst = As + (size_t)(unit >> wpr_shift) * lda;
+        base = (unit & (wpr - 1)) * 64 - U * stride;
       }
     };
-    // (with pieces owed, two chunks' loads are as many registers as four without)
-    using two = std::integral_constant<int, SK_STAGE_U_PIECES>;
+    // (with pieces owed, a chunk's loads are as many registers as three without; with a float32 weight as
+    // many as two; a part of one run of chunks asks for no more)
+    using one = std::integral_constant<int, 1>;
+    using two = std::integral_constant<int, 2>;
     using four = std::integral_constant<int, 4>;
-    if (NORM && a.pend_splits > 0) {
-      if (a.norm_w_bf16) stage_rows(two{}, std::true_type{});
-      else stage_rows(two{}, std::false_type{});
-    } else if (NORM && !a.norm_w_bf16) {
-      stage_rows(four{}, std::false_type{});
+    if constexpr (NORM) {
+      if (a.pend_splits > 0) {
+        if (a.norm_w_bf16) stage_rows(one{}, std::true_type{}, std::true_type{});
+        else stage_rows(one{}, std::false_type{}, std::true_type{});
+      } else if (!a.norm_w_bf16) {
+        stage_rows(two{}, std::false_type{}, std::false_type{});
+      } else if (chunks <= 64 * wpr) {
+        stage_rows(one{}, std::true_type{}, std::false_type{});
+      } else {
+        stage_rows(four{}, std::true_type{}, std::false_type{});
+      }
     } else {
-      stage_rows(four{}, std::true_type{});
+      stage_rows(four{}, std::true_type{}, std::false_type{});
     }
+    ask_for_pages();
     __syncthreads();
     if constexpr (NORM) {
       // the parts of a row in their order (read by the epilogue, behind the next barrier)
@@ -478,7 +562,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
           const Frag av = *(const Frag*)(arow[mb] + st * S::LEN);
           S::mul(av, b[u], acc[mb], u);
         }
-        b[u] = wload(min(st + R, s_end - 1));
+        b[u] = wload(st + R);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -500,25 +584,30 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
     const T* xb[MB];
     const T* x_rows = (const T*)a.x;
     if constexpr (EPI == SK_PART) {
-      int seg = 0;
+      if (a.segs > 1) {
+        int seg = 0;
 #pragma unroll
-      for (int i = 0; i < 7; ++i) seg += (i + 1 < a.segs && wstrip >= a.seg_end[i]) ? 1 : 0;
-      x_rows += seg * a.seg_stride;
+        for (int i = 0; i < 7; ++i) seg += (i + 1 < a.segs && wstrip >= a.seg_end[i]) ? 1 : 0;
+        x_rows += seg * a.seg_stride;
+      }
     }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) xb[mb] = x_rows + (size_t)min(mb * 16 + c, M - 1) * K;
     auto xload = [&](int st, int mb) {
-      return *(const Frag*)(xb[mb] + min(max(0, min(st, steps - 1)) * S::LEN + g * S::PER, K - S::PER));
+      return *(const Frag*)(xb[mb] + min(st * S::LEN + g * S::PER, K - S::PER));
     };
     Frag ab[R][MB];
+    ask_for_epilogue();
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < R; ++u) {     // in the order in which the loop below refills the ring
-      const int st = min(s_begin + u, s_end - 1);
+      const int st = min(s_begin + u, s_last);
       b[u] = wload(st);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) ab[u][mb] = xload(st, mb);
       __builtin_amdgcn_sched_barrier(0);
     }
+    ask_for_pages();
     int s0 = s_begin;
     for (; s0 + R < s_end; s0 += R) {       // rounds that refill the ring
 #pragma unroll
@@ -527,7 +616,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
           S::mul(ab[u][mb], b[u], acc[mb], u);
-        const int nx = min(st + R, s_end - 1);
+        const int nx = min(st + R, s_last);
         b[u] = wload(nx);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) ab[u][mb] = xload(nx, mb);
@@ -555,59 +644,42 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       for (int i = 0; i < half; ++i) acc[mb][i] += acc[mb][half + i];
     *(floatx4*)(part + (((size_t)wave * MB + mb) * 64 + lane) * 4) = acc[mb][0];
   }
+  leave_for_epilogue();
   __syncthreads();
-  // ---- reduce over the K slices in a fixed order; epilogue
-  for (int idx = threadIdx.x; idx < M * cols; idx += blockDim.x) {
-    const int m = idx / cols, col = idx - m * cols;
-    const int st = col >> 4, cc = col & 15;
-    const int mb = m >> 4, gg = (m & 15) >> 2, xx = m & 3;
+  // ---- reduce over the K slices in a fixed order (four of them read at a time); epilogue
+  auto total = [&](int m, int col) {
+    const float* from = part + (((size_t)(col >> 4) * MB + (m >> 4)) * 64 + ((m & 15) >> 2) * 16 + (col & 15)) * 4 + (m & 3);
+    const int stride = nsb * MB * 256;
     float sum = 0.f;
-    for (int k2 = 0; k2 < kw; ++k2)
-      sum += part[((((size_t)k2 * nsb + st) * MB + mb) * 64 + gg * 16 + cc) * 4 + xx];
-    if constexpr (NORM) sum *= inv[m];
-    sum += s_bias[col];
-    const int nn = n0 + col;
-    if constexpr (EPI == SK_SWIGLU || EPI == SK_QKV) {
-      tile[idx] = sum;
-    } else if (nn < a.N) {
-      const size_t at = (size_t)m * a.ldo + nn;
-      if (EPI == SK_STORE) ((T*)a.out)[at] = from_float<T>(a.act ? fmaxf(sum, 0.f) * fmaxf(sum, 0.f) : sum);
-      else if (EPI == SK_RESID) {
-        float old = resid_old;
-        if (idx != (int)threadIdx.x) {
-          old = ((float*)a.out)[at];
-          for (int sp = 0; sp < a.pend_splits; ++sp) old += a.pend[sp * a.pend_stride + (size_t)m * a.pend_ld + nn];
-        }
-        ((float*)a.out)[at] = old + sum;
-      } else if (EPI == SK_PART) {
-        ((float*)a.out)[ksp * a.part_stride + at] = sum;
-      } else {
-        ((float*)a.out)[at] = sum;
-      }
+    for (int k2 = 0; k2 < kw; k2 += 4) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = from[min(k2 + j, kw - 1) * stride];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum += k2 + j < kw ? v[j] : 0.f;
     }
-  }
+    if constexpr (NORM) sum *= inv[m];
+    return sum + s_bias[col];
+  };
   if constexpr (EPI == SK_SWIGLU) {
-    __syncthreads();
-    const int half = cols >> 1;   // outputs of this block
-    for (int idx = threadIdx.x; idx < M * half; idx += blockDim.x) {
-      const int m = idx / half, j = idx - m * half;
+    const int half = cols >> 1;   // outputs of this block: a thread takes a gate column and its up column
+    for (int idx = tid; idx < M * half; idx += a.threads) {
+      const int m = by_nsb(idx >> 3), j = idx - m * half;
       const int pr = j >> 4, cc = j & 15;
-      const float gv = tile[m * cols + pr * 32 + cc], uv = tile[m * cols + pr * 32 + 16 + cc];
+      const float gv = total(m, pr * 32 + cc), uv = total(m, pr * 32 + 16 + cc);
       const int o = ((n0 >> 5) + pr) * 16 + cc;
       if (o < a.n_out) ((T*)a.out)[(size_t)m * a.ldo + o] = from_float<T>(sk_pair<T>(gv, uv, a));
     }
-  }
-  if constexpr (EPI == SK_QKV) {
-    __syncthreads();
-    // this block is (part of) head `qhead` of [q heads | k heads | v heads]; its tile
-    // holds the low halves of its rotary pairs in the first half of its columns
+  } else if constexpr (EPI == SK_QKV) {
+    // this block is (part of) head `qhead` of [q heads | k heads | v heads]; the low halves of
+    // its rotary pairs are the first half of its columns, and a thread takes both of a pair
     const int head = qhead, d = a.d, dhalf = d >> 1, half = cols >> 1;
     const int i0 = a.qsplit == 1 ? 0 : qp * 16;
     const bool is_q = head < a.nq, is_k = !is_q && head < a.nq + a.nkv;
-    for (int idx = threadIdx.x; idx < M * half; idx += blockDim.x) {
-      const int m = idx / half, il = idx - m * half;
+    for (int idx = tid; idx < M * half; idx += a.threads) {
+      const int m = by_nsb(idx >> 3), il = idx - m * half;
       const int i = i0 + il;                      // pair index within the head
-      float lo = tile[m * cols + il], hi = tile[m * cols + il + half];
+      float lo = total(m, il), hi = total(m, il + half);
       const int pos = s_pos[m];
       if ((is_q || is_k) && a.inv_freq) {
         float s, co;
@@ -642,13 +714,37 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
         }
       }
     }
+  } else {
+    for (int idx = tid; idx < M * cols; idx += a.threads) {
+      const int m = by_nsb(idx >> 4), col = idx - m * cols, nn = n0 + col;
+      const float sum = total(m, col);
+      if (nn >= a.N) continue;
+      const size_t at = (size_t)m * a.ldo + nn;
+      if constexpr (EPI == SK_STORE) {
+        ((T*)a.out)[at] = from_float<T>(a.act ? fmaxf(sum, 0.f) * fmaxf(sum, 0.f) : sum);
+      } else if constexpr (EPI == SK_RESID) {
+        const bool first = idx == tid;
+        const float* from = a.pend + (size_t)m * a.pend_ld + nn;
+        float old = first ? resid_old : ((float*)a.out)[at];
+        if (first) {
+#pragma unroll
+          for (int j = 0; j < RP; ++j) old += j < a.pend_splits ? resid_pieces[j] : 0.f;
+        }
+        for (int sp = first ? RP : 0; sp < a.pend_splits; ++sp) old += from[sp * a.pend_stride];
+        ((float*)a.out)[at] = old + sum;
+      } else if constexpr (EPI == SK_PART) {
+        ((float*)a.out)[ksp * a.part_stride + at] = sum;
+      } else {
+        ((float*)a.out)[at] = sum;
+      }
+    }
   }
 }
 
 // ---------------------------------------------------------------- dispatch
 // (`width`: bytes of a number of W and of the staged rows, 2 or 4)
-static size_t skinny_lds_bytes(int nsb, int kw, int mb, int M, int K, int epi, bool stage, int width) {
-  size_t bytes = sk_float_words(nsb, kw, mb, M, epi) * sizeof(float);
+static size_t skinny_lds_bytes(int nsb, int kw, int mb, int M, int K, bool stage, int width) {
+  size_t bytes = sk_float_words(nsb, kw, mb) * sizeof(float);
   if (stage) bytes += (size_t)M * ((size_t)(K + 31) / 32 * 32 * width + SK_APAD);
   return bytes;
 }
@@ -673,7 +769,7 @@ static int skinny_launch(const SkinnyArgs& a, int blocks, size_t lds, hipStream_
     }
   }
   const int grid = a.tiles > 1 ? (blocks + 7) / 8 * 8 * a.tiles : blocks;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * a.nsb * a.kw), lds, stream, a);
+  hipLaunchKernelGGL(kernel, dim3(grid, EPI == SK_PART ? a.ksplit : 1), dim3(64 * a.nsb * a.kw), lds, stream, a);
   return 0;
 }
 
@@ -742,7 +838,7 @@ static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, in
     for (int kw = 1; kw * nsb <= max_waves && kw <= steps; ++kw) {
       for (int st = norm ? 1 : 0; st < (epilogue == SK_PART ? 1 : 2); ++st) {     // pieces of K: no staging
         const bool stage = st == 1;
-        const size_t lds = skinny_lds_bytes(nsb, kw, mb, M, K, epilogue, stage, width);
+        const size_t lds = skinny_lds_bytes(nsb, kw, mb, M, K, stage, width);
         if (lds > SK_LDS_LIMIT) continue;
         const int blocks = (strips + nsb - 1) / nsb * ksplit * tiles;     // (for QKV: heads, or heads * d/32)
         const int per_cu = (blocks + num_cus - 1) / num_cus;       // blocks the busiest unit runs
@@ -893,7 +989,7 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   LLMLAB_REQUIRE(shape.nsb > 0 && shape.kw > 0,
                  "skinny_linear: no block shape fits N=%d K=%d M=%d (16 rows of x to stage: %zu bytes of LDS)",
                  N, K, M, (size_t)(M < 16 ? M : 16) * ((size_t)(K + 31) / 32 * 32 * width + SK_APAD));
-  const size_t lds = skinny_lds_bytes(shape.nsb, shape.kw, mb, tile_rows, K, epilogue, shape.stage, width);
+  const size_t lds = skinny_lds_bytes(shape.nsb, shape.kw, mb, tile_rows, K, shape.stage, width);
   LLMLAB_REQUIRE(lds <= SK_LDS_LIMIT && shape.nsb * shape.kw <= (mb >= 4 ? 8 : 16),
                  "skinny_linear: block shape %dx%d does not fit", shape.nsb, shape.kw);
   // (only a forced shape can fail these: a gate strip and its up strip share a block, and
@@ -901,7 +997,7 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   LLMLAB_REQUIRE(!(epilogue == SK_SWIGLU && shape.nsb % 2 != 0) &&
                      shape.kw <= ((K + 31) / 32 + ksplit - 1) / ksplit * (width / 2),
                  "skinny_linear: block shape %dx%d does not fit this product", shape.nsb, shape.kw);
-  const int blocks = (N + 16 * shape.nsb - 1) / (16 * shape.nsb) * ksplit;
+  const int blocks = (N + 16 * shape.nsb - 1) / (16 * shape.nsb);
   SkinnyArgs a;
   a.pend = pend; a.pend_splits = pend_splits; a.pend_ld = pend_ld; a.pend_stride = pend_stride;
   a.segs = segs;
@@ -909,6 +1005,14 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   a.seg_stride = seg_stride;
   a.ksplit = ksplit; a.part_stride = part_stride; a.tiles = tiles; a.col_blocks = blocks;
   a.qsplit = shape.qsplit;
+  auto inverse = [](int n) { return n > 1 ? (unsigned)(((1ull << 32) + n - 1) / n) : 0u; };
+  a.tiles_inv = inverse(tiles);
+  a.qsplit_inv = inverse(shape.qsplit);
+  a.steps = (K + 64 / width - 1) / (64 / width);       // (64 bytes of a row a step)
+  a.group_steps = (a.steps + ksplit - 1) / ksplit;
+  a.wave_steps = (a.group_steps + shape.kw - 1) / shape.kw;
+  a.wpr_shift = 0;
+  while ((2 << a.wpr_shift) * tile_rows <= shape.nsb * shape.kw) ++a.wpr_shift;
   a.act = act;
   a.limit = limit; a.slope = slope; a.shift = shift;
   a.x = x; a.x_rows = x_rows; a.norm_w = norm_w; a.W = w; a.bias = bias; a.out = out;
@@ -916,7 +1020,7 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   a.kcache = kcache; a.vcache = vcache;
   a.M = M; a.N = N; a.K = K; a.ldo = ldo; a.n_out = n_out;
   a.norm_w_bf16 = norm_w_dtype == DT_BF16; a.bias_bf16 = bias_dtype == DT_BF16;
-  a.nsb = shape.nsb; a.kw = shape.kw; a.nq = nq; a.nkv = nkv; a.d = d; a.table_stride = table_stride;
+  a.nsb = shape.nsb; a.kw = shape.kw; a.threads = 64 * shape.nsb * shape.kw; a.nsb_inv = (65536 + shape.nsb - 1) / shape.nsb; a.nq = nq; a.nkv = nkv; a.d = d; a.table_stride = table_stride;
   a.page_size = page_size; a.eps = eps;
   int rc = 0;
   if (norm) {
