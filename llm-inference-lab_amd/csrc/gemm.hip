@@ -49,6 +49,8 @@
 // For SWIGLU the rows of W alternate in runs of 16: gate rows of 16 outputs, then
 // the up rows of the same 16 outputs, so fragments j and j+1 hold gate and up of
 // the same outputs in the same lanes.
+#include <type_traits>
+
 #include "common.h"
 
 enum { EPI_STORE = 0, EPI_RESID = 1, EPI_F32 = 2, EPI_SWIGLU = 3, EPI_QKV = 4, EPI_PART = 5 };
@@ -1048,22 +1050,32 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // exact in float32 and the sums are float32; an instruction adds 32 of them where
 // v_mfma_f32_32x32x2_f32 adds 2, so fewer roundings meet in a sum (relative error of a product of
 // normal numbers against 64 bits: inner size 896 4.5e-7, 5.4e-7 with the float32 instructions; 4,864 1.1e-6
-// and 1.25e-6, 6e-7 in three pieces).  Six instructions at 16 times the rate of the float32 ones, measured
-// against tiles of v_mfma_f32_32x32x2_f32 (which this replaces; 157 TFLOP/s is what those could reach): 1,531
-// rows of 9728 x 896 181 us against 266 (147 TFLOP/s of 32-bit products), of 896 x 4864 in three pieces 82
-// against 215, 4,000 rows of 17920 x 1536 1,305 against 1,831, 65 rows of 1536 x 8960 42 in eight pieces against 252.
-// What bounds it: in full rounds the power limit (0.98 PFLOP/s of bfloat16 products), in a round by itself
-// a step's trip through LDS (1.3 us where its matrix instructions need 0.7).
+// and 1.25e-6, 6e-7 in three pieces).
+//
+// Where all numbers of W are bfloat16 numbers, as in checkpoints that were trained and kept in bfloat16, m_w and l_w are
+// zero and with them three of the six products.  A block takes W for such until it meets another number: the first step
+// tells in most cases and the block starts over with all parts, what a later one holds is known at the end and the block
+// takes its outputs again.  Nothing is kept between calls, and both ways give the same sums to the bit (the
+// terms left out are zeros).  (Relative error of a prompt's logits, 1,531 tokens of the 0.5B shape, mean of eight seeds:
+// 2.13e-6; 2.63e-6 before the small products had sums of their own.)
 //
 // BM x BN outputs per block of WM x WN waves, steps of 32 of the inner size.  A thread
-// fetches eight numbers of a row as they lie in memory, three steps ahead, splits them in registers and
-// puts the three parts down in LDS in fragment order, [16 rows][part][lane][8], so that writes
-// and reads are 1 KB of consecutive bytes a wave.  Lane (c, g) of a fragment holds the numbers 4 g
-// .. 4 g + 3 and 16 + 4 g .. of its row's 32 (the order inside a step is free, both operands share
-// it), so that four lanes read 64 consecutive bytes.  Two stages of LDS: the next step is split and put down
-// between the matrix instructions of this one, a barrier a step.  The product is taken transposed, C^T = W
+// fetches eight numbers of a row as they lie in memory, two steps ahead (four neighbouring lanes 64 consecutive bytes: with
+// neighbouring lanes in different rows the way of the loads to the compute unit bounded the small tile, 1,531 rows
+// of 1152 x 896 34 us against 23), splits them in registers and puts the parts down in LDS in fragment order, [16
+// rows][part][64 places][8], where lane (c, g) of a fragment holds the numbers 4 g .. 4 g + 3 and 16 + 4 g .. of its row's 32
+// (the order inside a step is free, both operands share it).  Two stages of LDS: the next step is put down
+// in this one.  With eight waves they form two groups, a wave of each on every SIMD, half a step apart: between two barriers
+// one group reads its fragments and splits and puts down its pieces while the other issues its matrix instructions
+// (128 x 256, one part: 2,550 clocks a step where all waves in step took 4,000; not with three parts in the 128 x 128
+// tile, whose splitting takes longer than its products: 3,100 against 2,900).  The product is taken transposed, C^T = W
 // x^T, so that a lane holds four neighbouring columns of a row, and for SWIGLU the gate and the up
 // value of an output.
+//
+// What bounds it: LDS (128 x 256, one part: 128 KB of reads and 40 of writes a step, 1,850 clocks at the rates of LDS,
+// 1,630 of matrix instructions).  1,531 rows of 9728 x 896 with one / three parts 105 / 158 us (255 / 169 TFLOP/s of
+// 32-bit products; 187 / 184 before these tiles and loads), of 896 x 4864 in five pieces 57 / 87 (in three: 88 / 90), of
+// 1152 x 896 23 / 33 (36), 4,000 of 9728 x 896 250 / 383 (428 / 459).
 //
 // Two ranges have no such parts.  Of numbers below 2^-110 the last bits fall under bfloat16's smallest number, 2^-133
 // (the sum of the parts is then off by 2.4e-7 of the number at 2^-112, 9.5e-4 at 2^-124): it shows in what the third
@@ -1073,18 +1085,19 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // v_mfma_f32_16x16x4_f32, operands straight from memory: true 32-bit products over the whole range (1,531 rows of 9728 x
 // 896 with such a number in every block 654 us).  (The split is the one of Henry, Tang and Heinecke, "Leveraging the
 // bfloat16 artificial intelligence datatype for higher-precision computations", 2019.)
-template <int EPI, int BM, int BN, int WM, int WN>
+template <int EPI, int BM, int BN, int WM, int WN, bool VEC>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const float* __restrict__ A,
                                                                 const float* __restrict__ W, EpiArgs e, int M,
-                                                                int N, int K, int vec) {
+                                                                int N, int K) {
   constexpr int BK = 32, NW = WM * WN;
+  constexpr bool GROUPS = NW == 8;
   constexpr int TM = BM / 16 / WM, TN = BN / 16 / WN;    // 16 x 16 tiles per wave along m and n
   constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW;    // pieces of eight numbers per thread and step
   static_assert(LA >= 1 && LB >= 1 && LA * NW * 16 == BM && LB * NW * 16 == BN && TN % 2 == 0, "pieces");
   constexpr int STAGE = (BM + BN) / 16 * 3072;
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
   __shared__ int s_again;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wn = wave / WM;
   int bx = blockIdx.x, by = blockIdx.y;
   {                                                      // a band of column tiles per die, as above
@@ -1113,121 +1126,233 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
 #pragma unroll
     for (int i = 0; i < TM; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // piece x of a thread: row (wave + NW x) * 16 + c of the tile, numbers 4 g .. and 16 + 4 g .. of the step
-  const float* ap[LA];
-  const float* bp[LB];
+  // piece x of a thread: row (wave + NW x) * 16 + sr of the tile, numbers 4 sg .. and 16 + 4 sg .. of the step (four
+  // neighbouring lanes read 64 consecutive bytes)
+  const int sr = lane >> 2, sg = lane & 3;
+  const char* const abase = (const char*)(A + (size_t)m0 * K);
+  const char* const bbase = (const char*)(W + (size_t)n0 * K);
+  using Offset = std::conditional_t<VEC, uint32_t, size_t>;
+  Offset aoff[LA], boff[LB];     // bytes from the tile's first row of x and of W
 #pragma unroll
-  for (int x = 0; x < LA; ++x) ap[x] = A + (size_t)min(m0 + (wave + NW * x) * 16 + c, M - 1) * K;
+  for (int x = 0; x < LA; ++x) aoff[x] = (Offset)(min(m0 + (wave + NW * x) * 16 + sr, M - 1) - m0) * K * 4;
 #pragma unroll
-  for (int x = 0; x < LB; ++x) bp[x] = W + (size_t)min(n0 + (wave + NW * x) * 16 + c, N - 1) * K;
+  for (int x = 0; x < LB; ++x) boff[x] = (Offset)(min(n0 + (wave + NW * x) * 16 + sr, N - 1) - n0) * K * 4;
   struct Pieces {
     floatx4 a[LA][2], b[LB][2];
   };
-  auto guarded = [&](const float* row, int k) {
+  // Past the range other numbers of the rows are read; stash() puts zeros down for those of x.  Every load is
+  // unconditional and their number the same each time: the compiler then counts what is on its way instead of
+  // waiting for all of it.
+  auto guarded = [&](const float* row, int k) {      // (rows that are not 16-byte aligned)
     floatx4 v;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = k + q < k_end ? row[k + q] : 0.f;
+    for (int q = 0; q < 4; ++q) v[q] = row[min(k + q, k_end - 1)];
     return v;
   };
   auto fetch = [&](Pieces& r, int k0) {
-    if (vec && k0 + BK <= k_end) {
 #pragma unroll
-      for (int x = 0; x < LB; ++x) {
-        r.b[x][0] = *(const floatx4*)(bp[x] + k0 + 4 * g);
-        r.b[x][1] = *(const floatx4*)(bp[x] + k0 + 16 + 4 * g);
-      }
+    for (int h = 0; h < 2; ++h) {
+      const int k = k0 + 16 * h + 4 * sg;
+      if constexpr (VEC) {
+        const uint32_t kb = (uint32_t)min(k, k_end - 4) * 4u;
 #pragma unroll
-      for (int x = 0; x < LA; ++x) {
-        r.a[x][0] = *(const floatx4*)(ap[x] + k0 + 4 * g);
-        r.a[x][1] = *(const floatx4*)(ap[x] + k0 + 16 + 4 * g);
-      }
-    } else {
+        for (int x = 0; x < LA; ++x) r.a[x][h] = *(const floatx4*)(abase + (aoff[x] + kb));
 #pragma unroll
-      for (int x = 0; x < LB; ++x) {
-        r.b[x][0] = guarded(bp[x], k0 + 4 * g);
-        r.b[x][1] = guarded(bp[x], k0 + 16 + 4 * g);
-      }
+        for (int x = 0; x < LB; ++x) r.b[x][h] = *(const floatx4*)(bbase + (boff[x] + kb));
+      } else {
 #pragma unroll
-      for (int x = 0; x < LA; ++x) {
-        r.a[x][0] = guarded(ap[x], k0 + 4 * g);
-        r.a[x][1] = guarded(ap[x], k0 + 16 + 4 * g);
+        for (int x = 0; x < LA; ++x) r.a[x][h] = guarded((const float*)(abase + aoff[x]), k);
+#pragma unroll
+        for (int x = 0; x < LB; ++x) r.b[x][h] = guarded((const float*)(bbase + boff[x]), k);
       }
     }
   };
-  unsigned rest = 0;
-  auto split = [&](const floatx4 (&v)[2], char* to) {
-    bf16x8 h, m, l;
+  // Where row r of a fragment has what lane group q of it holds: 16 bytes, with the rows of a group exchanged by the
+  // group's number, so that eight neighbouring lanes of a write (two rows, four groups) and of a read (one group, eight rows)
+  // meet different banks.
+  auto place = [](int r, int q) { return (q * 16 + (r ^ (2 * q))) * 16; };
+  const int mine = place(c, g);
+  unsigned rest = 0;             // of the numbers of x, what the third part is rounded from
+  unsigned rest_w = 0;           // of the numbers of W, what one bfloat16 number leaves out
+  auto split = [&](const floatx4 (&v)[2], char* to, int k0) {      // (of x the numbers from k0 on; W: k0 < 0)
+    uint32_t part[3][4];
+    float num[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float x = v[q >> 2][q & 3];
-      h[q] = (bf16_t)x;
-      const float r = x - (float)h[q];
-      m[q] = (bf16_t)r;
-      const float s = r - (float)m[q];
-      l[q] = (bf16_t)s;
-      rest |= __float_as_uint(s);      // (its lower half is zero where bfloat16 holds it)
+    for (int q = 0; q < 8; ++q) num[q] = v[q >> 2][q & 3];
+    if (k0 + BK > k_end) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) num[q] = k0 + (q >> 2) * 16 + 4 * sg + (q & 3) < k_end ? num[q] : 0.f;
     }
-    *(bf16x8*)to = h;
-    *(bf16x8*)(to + 1024) = m;
-    *(bf16x8*)(to + 2048) = l;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {      // two numbers at a time
+      float x0 = num[2 * q], x1 = num[2 * q + 1];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+        const bf16x2 both = {(bf16_t)x0, (bf16_t)x1};
+        part[p][q] = __builtin_bit_cast(uint32_t, both);
+        if (p < 2) {
+          x0 -= __uint_as_float(part[p][q] << 16);
+          x1 -= __uint_as_float(part[p][q] & 0xffff0000u);
+        }
+      }
+      rest |= __float_as_uint(x0) | __float_as_uint(x1);      // (their lower halves are zero where bfloat16 holds them)
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      *(bf16x8*)(to + p * 1024) = __builtin_bit_cast(bf16x8, floatx4{__uint_as_float(part[p][0]), __uint_as_float(part[p][1]),
+                                                                     __uint_as_float(part[p][2]), __uint_as_float(part[p][3])});
   };
-  auto stash = [&](const Pieces& r, int stage) {
-    char* to = smem + stage * STAGE + lane * 16;
+  auto upper_halves = [&](const floatx4 (&v)[2], char* to) {      // numbers that are bfloat16 numbers, if rest_w says so
+    uint32_t h[4];
 #pragma unroll
-    for (int x = 0; x < LA; ++x) split(r.a[x], to + (wave + NW * x) * 3072);
-#pragma unroll
-    for (int x = 0; x < LB; ++x) split(r.b[x], to + (BM / 16 + wave + NW * x) * 3072);
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t a = __float_as_uint(v[q >> 1][(q & 1) * 2]), b = __float_as_uint(v[q >> 1][(q & 1) * 2 + 1]);
+      h[q] = __builtin_amdgcn_perm(b, a, 0x07060302);
+      rest_w |= a | b;
+    }
+    *(bf16x8*)to = __builtin_bit_cast(bf16x8, floatx4{__uint_as_float(h[0]), __uint_as_float(h[1]), __uint_as_float(h[2]),
+                                                      __uint_as_float(h[3])});
   };
-  auto multiply = [&](int stage, auto between) {
-    const char* xs = smem + stage * STAGE + lane * 16;
-    const char* ws = xs + BM / 16 * 3072;
-    bf16x8 xf[3][TM], wf[3][TN];
-    auto parts = [&](int p) {
+  // ONE: one part of every number of W is taken, else three
+  auto stash = [&](auto one, const Pieces& r, int k0, int stage) {
+    constexpr bool ONE = decltype(one)::value;
+    char* to = smem + stage * STAGE + place(sr, sg);
 #pragma unroll
-      for (int i = 0; i < TM; ++i) xf[p][i] = *(const bf16x8*)(xs + ((wm * TM + i) * 3 + p) * 1024);
+    for (int x = 0; x < LA; ++x) split(r.a[x], to + (wave + NW * x) * 3072, k0);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) wf[p][j] = *(const bf16x8*)(ws + ((wn * TN + j) * 3 + p) * 1024);
-    };
-    auto products = [&](int pw, int px) {
+    for (int x = 0; x < LB; ++x) {
+      if constexpr (ONE) upper_halves(r.b[x], to + BM / 16 * 3072 + (wave + NW * x) * 1024);
+      else split(r.b[x], to + (BM / 16 + wave + NW * x) * 3072, -BK);
+    }
+  };
+  // the parts of step `t` as a wave multiplies them, and their products, the small ones first
+  // (ONE: the order of the general sum, without its terms that are zero)
+  auto x_part = [&](bf16x8 (&xf)[TM], int stage, int p) {
+    const char* xs = smem + stage * STAGE + mine;
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+    for (int i = 0; i < TM; ++i) xf[i] = *(const bf16x8*)(xs + ((wm * TM + i) * 3 + p) * 1024);
+  };
+  auto w_part = [&](auto one, bf16x8 (&wf)[TN], int stage, int p) {
+    constexpr int PW = decltype(one)::value ? 1 : 3;
+    const char* ws = smem + stage * STAGE + BM / 16 * 3072 + mine;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[pw][j], xf[px][i], acc[j][i], 0, 0, 0);
-    };
-    parts(1);
-    parts(0);
-    parts(2);
-    products(1, 1);            // m_w m_x
-    between();
-    products(1, 0);
-    products(0, 1);
-    products(2, 0);
-    products(0, 2);
-    products(0, 0);            // h_w h_x
+    for (int j = 0; j < TN; ++j) wf[j] = *(const bf16x8*)(ws + ((wn * TN + j) * PW + p) * 1024);
+  };
+  // (the small products in sums of their own where there are registers for them: a sum is rounded at its own size, once
+  // a step and not three or six times; a product of 1,531 rows of 896 x 896 then is 1.9e-7 off 64 bits, 3.1e-7 in one sum)
+  constexpr bool APART = TN * TM <= 8;
+  floatx4 small[APART ? TN : 1][APART ? TM : 1];
+  auto products = [&](auto large, const bf16x8 (&wf)[TN], const bf16x8 (&xf)[TM]) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        floatx4& sum = APART && !decltype(large)::value ? small[APART ? j : 0][APART ? i : 0] : acc[j][i];
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], xf[i], sum, 0, 0, 0);
+      }
+  };
+  auto barrier = [&]() {      // (nothing moves across; a wave's reads and writes of LDS are done)
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  // Step t lies in stage t % 2; it is put there while step t - 1 is multiplied, from registers
-  // that were asked for three steps ahead.
+  // With one part of W: whether that was enough.  The first step tells at once; what a later one tells is
+  // known at the end.
   const int steps = (k_end - k_begin + BK - 1) / BK;
-  if (steps > 0) {
+  auto walk = [&](auto one) -> bool {
+    constexpr bool ONE = decltype(one)::value;
+    constexpr int PW = ONE ? 1 : 3;
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (APART) small[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
     Pieces r0, r1;
     fetch(r0, k_begin);
     fetch(r1, k_begin + BK);
-    stash(r0, 0);
+    stash(one, r0, k_begin, 0);
     fetch(r0, k_begin + 2 * BK);
-    __syncthreads();
-    for (int t = 0; t < steps; t += 2) {
-      const int k0 = k_begin + t * BK;
-      multiply(0, [&]() { stash(r1, 1); });          // (past the last step: zeros, never read)
-      fetch(r1, k0 + 3 * BK);
-      __syncthreads();
-      if (t + 1 >= steps) break;
-      multiply(1, [&]() { stash(r0, 0); });
-      fetch(r0, k0 + 4 * BK);
+    if constexpr (ONE) {
+      if (__syncthreads_or(rest_w & 0xffffu)) return false;
+    } else {
       __syncthreads();
     }
-  }
+    // Step t lies in stage t % 2; it is put there during step t - 1, from registers that were asked for two steps
+    // before that.
+    bf16x8 xf[3][TM], wf[PW][TN];
+    auto read = [&](int stage) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) x_part(xf[p], stage, p);
+#pragma unroll
+      for (int p = 0; p < PW; ++p) w_part(one, wf[p], stage, p);
+    };
+    auto multiply = [&]() {
+      const std::false_type part;
+      if constexpr (ONE) {
+        products(part, wf[0], xf[1]);
+        products(part, wf[0], xf[2]);
+      } else {
+        products(part, wf[1], xf[1]);            // m_w m_x
+        products(part, wf[1], xf[0]);
+        products(part, wf[0], xf[1]);
+        products(part, wf[2], xf[0]);
+        products(part, wf[0], xf[2]);
+      }
+      products(std::true_type{}, wf[0], xf[0]);  // h_w h_x
+    };
+    if constexpr (GROUPS && (ONE || TN > 2)) {
+      if (wave >= NW / 2) barrier();       // the second group runs half a step behind
+      auto step = [&](int t, Pieces& r) {  // (r: step t + 1)
+        read(t & 1);
+        stash(one, r, k_begin + (t + 1) * BK, (t + 1) & 1);
+        barrier();
+        fetch(r, k_begin + (t + 3) * BK);
+        multiply();
+        // (the loads and what they take to address between the matrix instructions)
+#pragma unroll
+        for (int n = 0; n < 2 * (LA + LB); ++n) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 3, 0);      // matrix instructions
+          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);      // vector instructions
+          __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);     // a load
+        }
+        barrier();
+      };
+      for (int t = 0; t < steps; t += 2) {
+        step(t, r1);
+        if (t + 1 >= steps) break;
+        step(t + 1, r0);
+      }
+      if (wave < NW / 2) barrier();
+    } else {
+      auto step = [&](int t, Pieces& r) {
+        read(t & 1);
+        stash(one, r, k_begin + (t + 1) * BK, (t + 1) & 1);
+        multiply();
+        fetch(r, k_begin + (t + 3) * BK);
+        __syncthreads();
+      };
+      for (int t = 0; t < steps; t += 2) {
+        step(t, r1);
+        if (t + 1 >= steps) break;
+        step(t + 1, r0);
+      }
+    }
+    if constexpr (APART) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[j][i] += small[j][i];
+    }
+    return !ONE || !__syncthreads_or(rest_w & 0xffffu);
+  };
+  if (steps > 0 && !walk(std::true_type{})) walk(std::false_type{});
   bool again = (rest & 0xffffu) != 0;
 #pragma unroll
   for (int j = 0; j < TN; ++j)
@@ -1238,6 +1363,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
   if (again) s_again = 1;      // (any thread's; the same value from all)
   __syncthreads();
   if (s_again) {
+    auto checked = [&](const float* row, int k) {
+      floatx4 v = guarded(row, k);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = k + q < k_end ? v[q] : 0.f;
+      return v;
+    };
     // lane (c, g) holds the numbers 4 g .. 4 g + 3 of 16 of its row; an instruction contracts one of each group
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -1246,17 +1377,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
 #pragma unroll 1
     for (int k0 = k_begin; k0 < k_end; k0 += 16) {
       const int k = k0 + 4 * g;
-      const bool whole = vec && k0 + 16 <= k_end;
+      const bool whole = VEC && k0 + 16 <= k_end;
       floatx4 xf[TM], wf[TN];
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const float* row = A + (size_t)min(m0 + (wm * TM + i) * 16 + c, M - 1) * K;
-        xf[i] = whole ? *(const floatx4*)(row + k) : guarded(row, k);
+        xf[i] = whole ? *(const floatx4*)(row + k) : checked(row, k);
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const float* row = W + (size_t)min(n0 + (wn * TN + j) * 16 + c, N - 1) * K;
-        wf[j] = whole ? *(const floatx4*)(row + k) : guarded(row, k);
+        wf[j] = whole ? *(const floatx4*)(row + k) : checked(row, k);
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -1312,22 +1443,54 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
   }
 }
 
+// The tiles of the products of many rows (what the numbers are: below, where a bfloat16 product is given its tile).
+enum { TILE_64 = 0, TILE_64x128 = 1, TILE_128 = 2, TILE_128x256 = 3, TILE_256 = 4, TILE_192 = 5, TILE_KINDS = 6,
+       // chosen by their own rule (one_round_tile) for whole products
+       TILE_64x96 = 6, TILE_64x160 = 7, TILE_64x224 = 8, TILE_128x160 = 9, TILE_ALL = 10 };
+struct TileModel {
+  int bm, bn;
+  double L, f, tk, resident, stream;
+  int whole_rounds;
+};
+// (the 64 x 64 row was fitted to a kernel that took x by way of registers, slower by 18 %; in the range of
+// few_blocks_cost that decides)
+static const TileModel TILE_MODELS[TILE_ALL] = {{64, 64, 6.39, 0.79, 0.289, 1.0, 20e3, 0},
+                                                  {64, 128, 6.54, 0.71, 0.5, 1.5, 27e3, 0},
+                                                  {128, 128, 8.0, 0.48, 0.66, 1.0, 24e3, 0},
+                                                  {128, 256, 0.0, 6.16, 0.945, 1.0, 24e3, 1},
+                                                  {256, 256, 0.0, 12.8, 1.34, 1.0, 24e3, 1},
+                                                  {192, 256, 0.0, 10.2, 1.08, 1.0, 24e3, 1},
+                                                  {64, 96}, {64, 160}, {64, 224}, {128, 160}};
+
 // The tile of a float32 product of many rows, and into how many pieces along the inner size one that adds
 // into the stream is cut.
 struct F32Plan {
-  int bm, pieces;
+  int tile, pieces;      // TILE_64, TILE_128 or TILE_128x256
 };
 static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int min_steps);
 
+// The tiles by direct loads address a tile's rows by 32 bits of bytes, which hold 255 rows (and 15 strips of
+// W) of this inner size; beyond, the 64 x 128 tile, whose addresses have 64.
+constexpr int DIRECT_MAX_INNER = 1 << 22;
+
 template <int EPI>
-static void launch_f32_split(int bm, const float* A, const float* W, const EpiArgs& e, int M, int N, int K, int pieces,
+static void launch_f32_split(int tile, const float* A, const float* W, const EpiArgs& e, int M, int N, int K, int pieces,
                              hipStream_t stream) {
-  const int vec = (K % 4 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);
-  const dim3 grid((N + bm - 1) / bm, (M + bm - 1) / bm, pieces);
-  if (bm == 128)
-    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 128, 128, 2, 4>), grid, dim3(512), 0, stream, A, W, e, M, N, K, vec);
+  // (whole loads of 16 bytes, and 32 bits of offset within 256 rows)
+  const bool vec = (K % 4 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) && K <= DIRECT_MAX_INNER;
+  if (!vec && tile == TILE_128x256) tile = TILE_128;
+  const int bm = TILE_MODELS[tile].bm, bn = TILE_MODELS[tile].bn;
+  const dim3 grid((N + bn - 1) / bn, (M + bm - 1) / bm, pieces);
+  if (tile == TILE_128x256)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 128, 256, 2, 4, true>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  else if (tile == TILE_128 && vec)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 128, 128, 2, 4, true>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  else if (tile == TILE_128)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 128, 128, 2, 4, false>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  else if (vec)
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 64, 64, 2, 2, true>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
   else
-    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 64, 64, 2, 2>), grid, dim3(256), 0, stream, A, W, e, M, N, K, vec);
+    hipLaunchKernelGGL((gemm_f32_split_kernel<EPI, 64, 64, 2, 2, false>), grid, dim3(256), 0, stream, A, W, e, M, N, K);
 }
 
 // Products of many rows in float32: the matrix cores, or (debug) the plain FMA kernel, their reference, with
@@ -1338,7 +1501,7 @@ static void launch_f32_tiled(const float* A, const float* W, const EpiArgs& e, i
   const int vec = (K % 4 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);
   auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (g_f32_fma == 0) {
-    launch_f32_split<EPI>(f32_plan(M, N, K, num_cus, 1, 1).bm, A, W, e, M, N, K, 1, stream);
+    launch_f32_split<EPI>(f32_plan(M, N, K, num_cus, 1, 1).tile, A, W, e, M, N, K, 1, stream);
     return;
   }
   if (blocks(128, 128) >= num_cus)
@@ -1526,23 +1689,6 @@ constexpr int F32_ROWS_MAX = 64;     // up to here the few-row kernel (the tiled
 // bytes a microsecond, the chip 5.3e6 at most (one tile of rows, 17 to 64 of them, of
 // matrices from 9 to 283 MB, in 4 or 8 pieces: the estimate is within 2 us of the
 // measurement).
-enum { TILE_64 = 0, TILE_64x128 = 1, TILE_128 = 2, TILE_128x256 = 3, TILE_256 = 4, TILE_192 = 5, TILE_KINDS = 6,
-       // chosen by their own rule (one_round_tile) for whole products
-       TILE_64x96 = 6, TILE_64x160 = 7, TILE_64x224 = 8, TILE_128x160 = 9, TILE_ALL = 10 };
-struct TileModel {
-  int bm, bn;
-  double L, f, tk, resident, stream;
-  int whole_rounds;
-};
-// (the 64 x 64 row was fitted to a kernel that took x by way of registers, slower by 18 %; in the range of
-// few_blocks_cost that decides)
-static const TileModel TILE_MODELS[TILE_ALL] = {{64, 64, 6.39, 0.79, 0.289, 1.0, 20e3, 0},
-                                                  {64, 128, 6.54, 0.71, 0.5, 1.5, 27e3, 0},
-                                                  {128, 128, 8.0, 0.48, 0.66, 1.0, 24e3, 0},
-                                                  {128, 256, 0.0, 6.16, 0.945, 1.0, 24e3, 1},
-                                                  {256, 256, 0.0, 12.8, 1.34, 1.0, 24e3, 1},
-                                                  {192, 256, 0.0, 10.2, 1.08, 1.0, 24e3, 1},
-                                                  {64, 96}, {64, 160}, {64, 224}, {128, 160}};
 constexpr double CHIP_STREAM = 5.3e6;     // bytes a microsecond
 
 // The tiles of the two groups of waves: whole rounds of one block a unit; with 256 rows a
@@ -1586,9 +1732,6 @@ static int g_force_tile = 0, g_without_wide = 0, g_pp_min_rows = 512;
 // tokens of five shapes that is between 1.4 % faster and 1.3 % slower than from 2,048 on.)
 constexpr int WIDE_TILE_MIN_ROWS = 2048;
 constexpr int PP_MIN_INNER = 896;      // the shortest inner size the estimates of those tiles were fitted to
-// The tiles by direct loads address a tile's rows by 32 bits of bytes, which hold 255 rows (and 15 strips of
-// W) of this inner size; beyond, the 64 x 128 tile, whose addresses have 64.
-constexpr int DIRECT_MAX_INNER = 1 << 22;
 static int addressable(int kind, int K) {
   return K > DIRECT_MAX_INNER && (kind == TILE_64 || kind == TILE_256 || kind == TILE_192) ? TILE_64x128 : kind;
 }
@@ -1627,34 +1770,47 @@ static int one_round_tile(int M, int N, int K, int num_cus) {
   return K >= 3072 && fills(224, 1, 0.8) ? TILE_64x224 : -1;
 }
 
-// By an estimate of the time, fitted to a sweep of seven matrices of two model shapes at 65 to 4,000 rows
-// whole and in up to eight pieces (within 12 % of the measurement; its picks lose 0.1 % on average, 5 % at most, to the best of the sweep).  A block of the 128 x
-// 128 tile is alone on its unit, rounds are whole; of the 64 x 64 tile three share one, whose first is slow by
-// itself (0.86 us a step for its own chain of trips, 0.58 where others fill the gaps).
+// By an estimate of the time, fitted to a sweep of eight matrices of three model shapes at 65 to 4,096 rows
+// whole and in up to eight pieces, each with W's numbers of one part and of three (948 times; 4 to 9 % rms about the
+// geometric mean of the two, since W's numbers are not known here; the picks lose 0.6 % whole and 2.3 % in pieces to the
+// best of the sweep).  Against the tiles and picks before (64 x 64 and 128 x 128, one loop for all numbers, a load of 16
+// rows with neighbouring lanes in different ones) they take 0.60 of the time whole and 0.72 with the fold of their
+// pieces where W has one part, 0.87 and 0.94 where it has three (9 % more at worst, of a product in fewer pieces than
+// before).  A block of the 128 x 128 and 128 x 256 tiles is alone on its unit, rounds are whole; of the 64 x 64 tile
+// three share one, whose first is slow by itself.
+// The 128 x 256 tile, whose small products have no sums of their own, adds at most so many steps where the product may
+// be cut: 7,041 rows of 896 x 4864 whole were 7.4e-7 off 64 bits and a decode step behind such prompts 1.68e-6, in
+// three pieces 4.3e-7 and 1.44e-6 (as before this tile).
+constexpr int F32_WIDE_STEPS = 64;
 static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int min_steps) {
   const int steps = (K + 31) / 32;
-  F32Plan best{0, 1};
+  F32Plan best{-1, 1};
   double least = 0.0;
-  for (int bm = 64; bm <= 128; bm += 64) {
-    if (g_force_tile == 64 && bm != 64) continue;
-    if ((g_force_tile == 128 || g_force_tile == 129) && bm != 128) continue;
+  for (const int tile : {TILE_64, TILE_128, TILE_128x256}) {
+    if (g_force_tile == 64 && tile != TILE_64) continue;
+    if ((g_force_tile == 128 || g_force_tile == 129) && tile != TILE_128) continue;
+    if (g_force_tile == 131 && tile != TILE_128x256) continue;
+    const int bm = TILE_MODELS[tile].bm, bn = TILE_MODELS[tile].bn;
     for (int pieces = 1; pieces <= max_pieces; ++pieces) {
       const int s = (steps + pieces - 1) / pieces;
       if (pieces > 1 && s < min_steps) break;
-      const double share = (double)((M + bm - 1) / bm) * ((N + bm - 1) / bm) * pieces / num_cus;
+      const double share = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * pieces / num_cus;
       const double whole = ceil(share - 1e-9);
       double t;
-      if (bm == 128) {
-        t = whole * (5.4 + s * (1.31 + 0.12 * (share < 1.0 ? share : 1.0)));
+      if (tile == TILE_128x256) {
+        if (s > F32_WIDE_STEPS && pieces < max_pieces) continue;
+        t = 1.65 + whole * (8.9 + s * (1.475 + 0.377 * (share < 1.0 ? share : 1.0)));
+      } else if (tile == TILE_128) {
+        t = 1.4 + whole * (5.9 + s * (0.945 + 0.22 * (share < 1.0 ? share : 1.0)));
       } else {
-        const double shared = (share <= 3.0 ? whole : share) * (1.0 + 0.58 * s);
-        t = 2.0 + 0.863 * s;
+        const double shared = (share <= 3.0 ? whole : share) * (1.25 + 0.394 * s);
+        t = 5.7 + 0.504 * s;
         if (shared > t && whole > 1.0) t = shared;
       }
       if (pieces > 1) t += pieces * ((double)M * N * 2.2e-6 + 0.3);      // (their way through memory to the next reader)
-      if (best.bm == 0 || t < least) {
+      if (best.tile < 0 || t < least) {
         least = t;
-        best = F32Plan{bm, pieces};
+        best = F32Plan{tile, pieces};
       }
     }
   }
@@ -2014,7 +2170,7 @@ extern "C" void llmlab_linear_plan_f32(int M, int N, int K, int num_cus, int max
                                        int* out) {
   const F32Plan plan = f32_plan(M, N, K, num_cus > 0 ? num_cus : 256, max_pieces, min_steps_per_piece);
   out[0] = plan.pieces;
-  out[1] = plan.bm == 128 ? TILE_128 : TILE_64;
+  out[1] = plan.tile;
 }
 
 // q/k/v projection of many rows with bias, rotation and cache write in the epilogue
@@ -2067,11 +2223,11 @@ extern "C" int llmlab_linear_partials(const void* x, const void* w, int dtype, f
                  "linear_partials: %d pieces, row stride %d", ksplit, ldo);
   LLMLAB_REQUIRE(tile >= TILE_64 && tile < TILE_KINDS, "linear_partials: unknown tile %d", tile);
   if (dtype == DT_F32) {
-    LLMLAB_REQUIRE(tile == TILE_64 || tile == TILE_128, "linear_partials(float32): tile %d", tile);
+    LLMLAB_REQUIRE(tile == TILE_64 || tile == TILE_128 || tile == TILE_128x256, "linear_partials(float32): tile %d", tile);
     if (M == 0) return 0;
     const int steps = (K + 31) / 32;
     EpiArgs e{parts, bias, bias_dtype == DT_BF16, ldo, N, (steps + ksplit - 1) / ksplit, part_stride};
-    launch_f32_split<EPI_PART>(tile == TILE_128 ? 128 : 64, (const float*)x, (const float*)w, e, M, N, K, ksplit, stream);
+    launch_f32_split<EPI_PART>(tile, (const float*)x, (const float*)w, e, M, N, K, ksplit, stream);
     LLMLAB_LAUNCH_CHECK("linear_partials(float32)");
     return 0;
   }

@@ -112,3 +112,47 @@ def test_sums_that_overflow(ops, tile):
     fine = want.isfinite()
     assert torch.equal(got[~fine], want[~fine])
     assert bool(((got - want).abs()[fine] <= limit[fine]).all())
+
+
+@pytest.mark.parametrize("tile", [64, 128, 131])
+@pytest.mark.parametrize("m,n,k", [(65, 64, 32), (128, 256, 64), (129, 257, 96), (127, 255, 36), (130, 300, 100), (70, 66, 33),
+                                   (200, 520, 1152)])
+@pytest.mark.parametrize("odd", [None, 0, -1])
+def test_weights_of_one_part(ops, tile, m, n, k, odd):
+    """Matrices whose numbers are bfloat16 numbers take half of the part products; one other number, in the first
+    step of the inner size or in the last, makes its blocks take all.  Whole, in pieces and paired."""
+    x, w = rnd((m, k), 21), rnd((n, k), 22).bfloat16().float()
+    if odd is not None:
+        w[n // 2, odd] = 1.0 + 2.0 ** -20
+    want, limit = x.double() @ w.double().T, bound(x, w)
+    dx, dw = x.to(DEV), ops.prepare_weight(w.to(DEV))
+    with ops.debug.force(gemm_tile=tile):
+        out = torch.empty(m, n, device=DEV)
+        ops.linear_logits(dx, dw, out)
+        assert bool(((out.cpu().double() - want).abs() <= limit).all())
+        parts = torch.full((3, m, n), float("nan"), device=DEV)
+        ops.linear_partials(dx, dw, parts, 3)
+        assert bool(((parts.cpu().double().sum(0) - want).abs() <= limit).all())
+        if n % 32 == 0:
+            paired = torch.empty(m, n // 2, device=DEV)
+            ops.linear_swiglu(dx, dw, paired)
+            both = out.cpu().reshape(m, n // 32, 2, 16).double()
+            want_p = (both[:, :, 0] * torch.sigmoid(both[:, :, 0]) * both[:, :, 1]).reshape(m, n // 2)
+            # (the same sums; the activation and two products in 32 bits: a few roundings of 2^-24, the exponential 2 ulp)
+            assert bool(((paired.cpu().double() - want_p).abs() <= 2.0 ** -20 * want_p.abs() + 1e-30).all())
+
+
+def test_products_of_many_steps_of_one_part_and_three_agree(ops):
+    """The part products left out are zeros: the sums are the same to the bit."""
+    m, n, k = 150, 512, 640
+    x, w = rnd((m, k), 23).to(DEV), rnd((n, k), 24).bfloat16().float().to(DEV)
+    # (a row of other numbers behind every 31: all blocks of this matrix take three parts)
+    mixed = torch.full((n + n // 31 + 1, k), 1.0 + 2.0 ** -20, device=DEV)
+    places = torch.tensor([i for i in range(mixed.shape[0]) if i % 32 != 31][:n], device=DEV)
+    mixed[places] = w
+    for tile in (64, 128, 131):
+        with ops.debug.force(gemm_tile=tile):
+            one, three = torch.empty(m, n, device=DEV), torch.empty(m, mixed.shape[0], device=DEV)
+            ops.linear_logits(x, ops.prepare_weight(w), one)
+            ops.linear_logits(x, ops.prepare_weight(mixed), three)
+            assert torch.equal(one, three[:, places]), f"tile {tile}"
