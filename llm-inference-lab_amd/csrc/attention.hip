@@ -990,6 +990,14 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
   const int c = lane & 15, g = lane >> 4;
   const int b = request_of(a, (int)blockIdx.z);
   if (b < 0) return;
+  // (a short row of the block table as a whole, see the bfloat16 kernel)
+  constexpr int TAB = SPLIT ? 2 : 1;
+  const bool table_here = SPLIT && a.table_stride <= 64 * TAB;
+  int tab[TAB];
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < TAB; ++i) tab[i] = a.table[(size_t)b * a.table_stride + min(i * 64 + lane, a.table_stride - 1)];
+  }
   const int kvh = blockIdx.y / a.splits, split = blockIdx.y % a.splits;
   const int G = a.nq / a.nkv;
   const int r0 = a.q_start[b], qlen = a.q_start[b + 1] - r0, sp = a.start_pos[b];
@@ -1115,7 +1123,18 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
     {
       const int pos16 = (cb + lane) * 16;
       const bool in = cb + lane < ce && pos16 <= key_hi && pos16 + 15 >= key_lo;
-      const int pg = a.table[(size_t)b * a.table_stride + min(pos16 >> pshift, a.table_stride - 1)];
+      const int pi = min(pos16 >> pshift, a.table_stride - 1);
+      int pg;
+      if (table_here) {
+        pg = __shfl(tab[0], pi & 63, WAVE);
+#pragma unroll
+        for (int i = 1; i < TAB; ++i) {
+          const int there = __shfl(tab[i], pi & 63, WAVE);
+          pg = pi >> 6 == i ? there : pg;
+        }
+      } else {
+        pg = a.table[(size_t)b * a.table_stride + pi];
+      }
       pages_v = in ? pg : -1;
     }
     auto fetch = [&](int blk, Step& f) {
@@ -1176,7 +1195,7 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
   } else {
     // ---- merge the waves of the block through LDS (see the bfloat16 kernel)
     __shared__ float s_m[NW][16 * QB], s_l[NW][16 * QB];
-    __shared__ __attribute__((aligned(16))) float s_o[NW][16 * QB][D];
+    __shared__ __attribute__((aligned(16))) float s_o[NW][16 * QB][DS];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       float l = lsum[qb];
@@ -1191,24 +1210,42 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
     }
     __syncthreads();
     const int nrows = min(16 * QB, rows_total - row0);
-    for (int idx = threadIdx.x; idx < nrows * D; idx += blockDim.x) {
-      const int r = idx / D, dd = idx - r * D;
-      float mmax = NEG_INF;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) mmax = fmaxf(mmax, s_m[w][r]);
-      float num = 0.f, den = 0.f;
+    const bool whole_stores = ((uintptr_t)a.o_part & 15) == 0;
+    for (int idx = threadIdx.x; idx < nrows * (D / 4); idx += blockDim.x) {
+      const int r = idx / (D / 4), dd = (idx - r * (D / 4)) * 4;
+      float mw[NW], lw[NW];
+      floatx4 ow[NW];
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        const float wt = s_m[w][r] == NEG_INF ? 0.f : exp2f(s_m[w][r] - mmax);
-        num += wt * s_o[w][r][dd];
-        den += wt * s_l[w][r];
+        mw[w] = s_m[w][r];
+        lw[w] = s_l[w][r];
+        ow[w] = *(const floatx4*)(&s_o[w][r][dd]);
+      }
+      float mmax = NEG_INF;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) mmax = fmaxf(mmax, mw[w]);
+      floatx4 num = {0.f, 0.f, 0.f, 0.f};
+      float den = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float wt = mw[w] == NEG_INF ? 0.f : exp2f(mw[w] - mmax);
+        num += wt * ow[w];
+        den += wt * lw[w];
       }
       const int t = (row0 + r) / G, hh = kvh * G + (row0 + r) % G;
       if (a.splits == 1) {
-        ((float*)a.out)[(size_t)(r0 + t) * a.out_stride + (size_t)hh * D + dd] = den > 0.f ? num / den : 0.f;
+        floatx4 res;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) res[i] = den > 0.f ? num[i] / den : 0.f;
+        *(floatx4*)((float*)a.out + (size_t)(r0 + t) * a.out_stride + (size_t)hh * D + dd) = res;
       } else {
         const size_t at = ((size_t)(r0 + t) * a.nq + hh) * a.splits + split;
-        a.o_part[at * D + dd] = num;
+        if (whole_stores) {
+          *(floatx4*)(a.o_part + at * D + dd) = num;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) a.o_part[at * D + dd + i] = num[i];
+        }
         if (dd == 0) {
           a.ml_part[at * 2] = mmax;
           a.ml_part[at * 2 + 1] = den;
