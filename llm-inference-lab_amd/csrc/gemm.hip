@@ -94,7 +94,9 @@ __device__ __forceinline__ float relu2_f(float z) {
   return z * z;
 }
 
-__device__ __forceinline__ float silu_f(float z) { return z / (1.f + __expf(-z)); }
+// (by the hardware's reciprocal, one unit in the last place of 32 bits, for results of 8 bits: the division is
+// eleven instructions, and an output of a paired product was sixteen)
+__device__ __forceinline__ float silu_f(float z) { return z * __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 
 // tanh form of gelu: 0.5 z (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))), as z * sigmoid(2 t)
 __device__ __forceinline__ float gelu_tanh_f(float z) {
@@ -113,8 +115,8 @@ __device__ __forceinline__ float gate_act_exact_f(float z, int act) {
 
 // A gated pair: act(gate) * up; act 3, the clamped pair: with g = min(gate, limit) and u = up held within
 // -limit .. limit, g * sigmoid(slope * g) * (u + shift).
-__device__ __forceinline__ float pair_f(float g, float u, const EpiArgs& e) {
-  if (e.act != 3) return gate_act_f(g, e.act) * u;
+__device__ __forceinline__ float pair_f(float g, float u, int act, const EpiArgs& e) {
+  if (act != 3) return gate_act_f(g, act) * u;
   g = fminf(g, e.limit);
   return g / (1.f + __expf(-e.slope * g)) * (fminf(fmaxf(u, -e.limit), e.limit) + e.shift);
 }
@@ -137,7 +139,155 @@ __device__ __forceinline__ void epi_store(const EpiArgs& e, int m, int n, float 
     ((float*)e.out)[at] = acc;
 }
 
-// The epilogue of a tile of BM x BN sums that lies in LDS (rows of BN + 4 floats), by the NT
+// The epilogue of a wave's sums where they are: lane (c, g) holds, of the 16 x 16 block (i, j), row m0 + 16 i + c and
+// the columns n0 + 16 j + 4 g .. + 3 (products taken transposed, W x^T).  Sums of 32 bits are written, and the residual
+// read, 16 bytes a lane, a row of blocks on its way while the one before is added; two blocks of bfloat16 results are
+// exchanged between neighbouring groups of lanes so that a lane writes 16 bytes too.  By way of LDS, where a thread found
+// the activation anew for each number, a tile alone on its unit spent 14 us so with a residual (192 x 256, a trip to memory
+// behind the other) and 11 with paired results (256 x 256); here 7, at the rate of memory for what all units then want
+// at once, and 2.3.
+template <int TM, int TN, int EPI>
+__device__ __forceinline__ void register_epilogue(const floatx4 (&acc)[TM][TN], const EpiArgs& e, int m0, int n0, int M,
+                                                  int N, int c, int g) {
+  static_assert(TM % 2 == 0 && TN % 2 == 0, "blocks in pairs");
+  // eight neighbouring results a lane out of four of block a and four of block b: lane groups 0 and 2 get a's, 1 and
+  // 3 b's, the lower half of the block's columns in groups 0 and 1
+  auto exchange = [](const bf16x4& a, const bf16x4& b) {
+    typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2;
+    typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+    const u32x2 x = __builtin_bit_cast(u32x2, a), y = __builtin_bit_cast(u32x2, b);
+    const auto r0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+    const auto r1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+    return __builtin_bit_cast(bf16x8, u32x4{(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]});
+  };
+  if constexpr (EPI == EPI_SWIGLU) {
+    // columns alternate in runs of 16: gate, up of the same 16 outputs
+    bf16_t* out = (bf16_t*)e.out;
+    const int o0 = n0 >> 1;
+    const bool whole = (e.ldo & 7) == 0 && ((uintptr_t)out & 15) == 0 && o0 + TN * 8 <= e.n_out;
+    auto put = [&](int m, int col, const bf16x4& v) {      // (unaligned, or past the last output)
+      if (m < M)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          if (o0 + col + x < e.n_out) out[(size_t)m * e.ldo + o0 + col + x] = v[x];
+    };
+    // (two runs of outputs of a row where a wave has them, else the same run of two rows)
+    constexpr int DI = TN >= 4 ? 1 : 2, DJ = TN >= 4 ? 2 : 1;
+    auto results = [&](auto act) {      // (the activation a constant: no branch a number)
+      auto pair = [&](int i, int jp) {
+        bf16x4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = (bf16_t)pair_f(acc[i][2 * jp][x], acc[i][2 * jp + 1][x], decltype(act)::value, e);
+        return v;
+      };
+#pragma unroll
+      for (int i = 0; i < TM; i += DI)
+#pragma unroll
+        for (int jp = 0; jp < TN / 2; jp += DJ) {
+          const int i1 = i + DI - 1, jp1 = jp + DJ - 1;
+          const bf16x4 a = pair(i, jp), b = pair(i1, jp1);
+          if (whole) {
+            const bf16x8 v = exchange(a, b);
+            const int m = m0 + 16 * ((g & 1) ? i1 : i) + c, col = 16 * ((g & 1) ? jp1 : jp) + (g >> 1) * 8;
+            if (m < M) *(bf16x8*)(out + (size_t)m * e.ldo + o0 + col) = v;
+          } else {
+            put(m0 + 16 * i + c, 16 * jp + 4 * g, a);
+            put(m0 + 16 * i1 + c, 16 * jp1 + 4 * g, b);
+          }
+        }
+    };
+    if (e.act == 3) results(std::integral_constant<int, 3>{});
+    else if (e.act == 2) results(std::integral_constant<int, 2>{});
+    else results(std::integral_constant<int, 0>{});
+  } else if constexpr (EPI != EPI_QKV) {
+    constexpr bool OUT32 = EPI != EPI_STORE;
+    const bool whole = (e.ldo & (OUT32 ? 3 : 7)) == 0 && ((uintptr_t)e.out & 15) == 0 && n0 + TN * 16 <= N;
+    floatx4 bias[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bias[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (e.bias) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) bias[j][x] = load_vec(e.bias, e.bias_bf16, min(n0 + 16 * j + 4 * g + x, N - 1));
+    }
+    if (!whole) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int m = m0 + 16 * i + c;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const int n = n0 + 16 * j + 4 * g + x;
+            if (m >= M || n >= N) continue;
+            const size_t at = (size_t)m * e.ldo + n;
+            float v = acc[i][j][x] + bias[j][x];
+            if constexpr (EPI == EPI_STORE) {
+              if (e.act) v = relu2_f(v);
+              ((bf16_t*)e.out)[at] = (bf16_t)v;
+            } else {
+              ((float*)e.out)[at] = (EPI == EPI_RESID ? ((float*)e.out)[at] : 0.f) + v;
+            }
+          }
+        }
+    } else if constexpr (EPI == EPI_STORE) {
+      auto rounded = [&](int i, int j) {
+        floatx4 v = acc[i][j] + bias[j];
+        if (e.act)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) v[x] = relu2_f(v[x]);
+        return bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+      };
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; j += 2) {
+          const bf16x8 v = exchange(rounded(i, j), rounded(i, j + 1));
+          const int m = m0 + 16 * i + c;
+          if (m < M) *(bf16x8*)((bf16_t*)e.out + (size_t)m * e.ldo + n0 + 16 * (j + (g & 1)) + (g >> 1) * 8) = v;
+        }
+    } else {
+      // neighbouring lanes have neighbouring rows: one takes both halves' columns of the even row's 32, the other of
+      // the odd one's, so that an instruction touches eight rows by 128 bytes and not sixteen by 64
+      const bool odd = c & 1;
+      float* const out = (float*)e.out + n0 + (odd ? 16 : 0) + 4 * g;
+      auto row = [&](int i, int h) { return out + (size_t)min(m0 + 16 * i + (c & ~1) + h, M - 1) * e.ldo; };
+      floatx4 old[2][2][TN / 2];
+      auto ask = [&](int i) {
+        if constexpr (EPI == EPI_RESID) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int jp = 0; jp < TN / 2; ++jp) old[i & 1][h][jp] = *(const floatx4*)(row(i, h) + 32 * jp);
+        }
+      };
+      ask(0);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        if (i + 1 < TM) ask(i + 1);
+#pragma unroll
+        for (int jp = 0; jp < TN / 2; ++jp) {
+          const floatx4 a = acc[i][2 * jp] + bias[2 * jp], b = acc[i][2 * jp + 1] + bias[2 * jp + 1];
+          floatx4 v[2];
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const float a1 = dpp_move<0xB1>(a[x]), b1 = dpp_move<0xB1>(b[x]);      // the neighbour's
+            v[0][x] = odd ? b1 : a[x];
+            v[1][x] = odd ? b[x] : a1;
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if constexpr (EPI == EPI_RESID) v[h] = old[i & 1][h][jp] + v[h];
+            if (m0 + 16 * i + (c & ~1) + h < M) *(floatx4*)(row(i, h) + 32 * jp) = v[h];
+          }
+        }
+      }
+    }
+  }
+}
+
+// The epilogue of a q/k/v tile of BM x BN sums that lies in LDS (rows of BN + 4 floats), by the NT
 // threads of the block: global memory is written (and the residual read) in pieces of 16 bytes,
 // consecutive lanes next to each other.  s_pos, s_page, s_freq and s_bias are what the QKV
 // epilogue fetched per row and per column of the tile before the product.
@@ -261,70 +411,6 @@ __device__ __forceinline__ void tile_epilogue(const float* Cs, const EpiArgs& e,
         }
       }
     }
-  } else if constexpr (EPI == EPI_SWIGLU) {
-    // columns of the tile alternate in runs of 16: gate, up of the same 16 outputs
-    constexpr int OUTS = BN / 2, CH = OUTS / 8;      // outputs per row of the tile, chunks of 8 of them
-    bf16_t* out = (bf16_t*)e.out;
-    const int o0 = n0 >> 1;
-    const bool vec = (e.ldo & 7) == 0 && ((uintptr_t)out & 15) == 0;
-    for (int ch = tid; ch < BM * CH; ch += NT) {
-      const int row = ch / CH, oc = (ch % CH) * 8;      // 8 outputs within one run of 16
-      const int m = m0 + row;
-      if (m >= M) continue;
-      const float* gp = Cs + row * C_STRIDE + (oc >> 4) * 32 + (oc & 15);
-      const floatx4 g0 = *(const floatx4*)gp, g1 = *(const floatx4*)(gp + 4);
-      const floatx4 u0 = *(const floatx4*)(gp + 16), u1 = *(const floatx4*)(gp + 20);
-      bf16x8 v;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[q] = (bf16_t)pair_f(g0[q], u0[q], e);
-        v[4 + q] = (bf16_t)pair_f(g1[q], u1[q], e);
-      }
-      bf16_t* dst = out + (size_t)m * e.ldo + o0 + oc;
-      if (vec && o0 + oc + 8 <= e.n_out) *(bf16x8*)dst = v;
-      else
-        for (int q = 0; q < 8; ++q)
-          if (o0 + oc + q < e.n_out) dst[q] = v[q];
-    }
-  } else {
-    constexpr int CH = BN / 4;                         // chunks of 4 columns per row of the tile
-    constexpr bool OUT32 = EPI != EPI_STORE;
-    const bool vec = (e.ldo & 3) == 0 && ((uintptr_t)e.out & 15) == 0 && (OUT32 || (e.ldo & 7) == 0);
-    for (int ch = tid; ch < BM * CH; ch += NT) {
-      const int row = ch / CH, col = (ch % CH) * 4;
-      const int m = m0 + row, n = n0 + col;
-      if (m >= M || n >= N) continue;
-      floatx4 v = *(const floatx4*)(Cs + row * C_STRIDE + col);
-      if (e.bias)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] += load_vec(e.bias, e.bias_bf16, min(n + q, N - 1));
-      const size_t at = (size_t)m * e.ldo + n;
-      const bool whole = vec && n + 4 <= N;
-      if constexpr (EPI == EPI_STORE) {
-        if (e.act)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] = relu2_f(v[q]);
-        bf16_t* dst = (bf16_t*)e.out + at;
-        if (whole) {
-          bf16x4 o;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) o[q] = (bf16_t)v[q];
-          *(bf16x4*)dst = o;
-        } else {
-          for (int q = 0; q < 4; ++q)
-            if (n + q < N) dst[q] = (bf16_t)v[q];
-        }
-      } else {
-        float* dst = (float*)e.out + at;
-        if (whole) {
-          if constexpr (EPI == EPI_RESID) v += *(const floatx4*)dst;
-          *(floatx4*)dst = v;
-        } else {
-          for (int q = 0; q < 4; ++q)
-            if (n + q < N) dst[q] = (EPI == EPI_RESID ? dst[q] : 0.f) + v[q];
-        }
-      }
-    }
   }
 }
 
@@ -387,7 +473,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
   constexpr int C_STRIDE = BN + 4;           // floats per row of the result tile in LDS
   constexpr size_t STAGE_BYTES = (size_t)(3 * A_STAGE) * sizeof(bf16_t);
   constexpr size_t C_BYTES = (size_t)BM * C_STRIDE * sizeof(float);
-  __shared__ __attribute__((aligned(16))) char smem[STAGE_BYTES > C_BYTES ? STAGE_BYTES : C_BYTES];
+  __shared__ __attribute__((aligned(16))) char smem[EPI != EPI_QKV || STAGE_BYTES > C_BYTES ? STAGE_BYTES : C_BYTES];
   bf16_t* As2 = (bf16_t*)smem;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -526,14 +612,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], rbd[p][0][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rbd[p][0][j], a0[i], acc[i][j], 0, 0, 0);
         frags(a0, stage1, 0);
         if (t + 2 < nk) stash(p2, stage2);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], rbd[p][1][j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rbd[p][1][j], a1[i], acc[i][j], 0, 0, 0);
         __syncthreads();
       }
       // (outside the branch, like every load of the loop: see above)
@@ -543,21 +629,21 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
     }
   }
 
-  // ---- epilogue.  The results go through LDS so that global memory is written (and the
-  // residual read) in pieces of 16 bytes, consecutive lanes next to each other: straight
-  // from the MFMA layout a wave instruction would touch 32 bytes in each of four rows.
-  // (Every live tile ended with a barrier, so the stages are free.)
-  float* Cs = (float*)smem;
+  // ---- epilogue
+  if constexpr (QKV) {      // through LDS, where a thread finds both halves of its pairs
+    // (every live tile ended with a barrier, so the stages are free)
+    float* Cs = (float*)smem;
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        Cs[(wm * WTM + i * 16 + g * 4 + x) * C_STRIDE + wn * WTN + j * 16 + c] = acc[i][j][x];
-  if constexpr (QKV) rows.put(tid, s_pos, s_page, s_freq, s_bias);
-  __syncthreads();
-  tile_epilogue<BM, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
+      for (int j = 0; j < TN; ++j)
+        *(floatx4*)(Cs + (wm * WTM + i * 16 + c) * C_STRIDE + wn * WTN + j * 16 + g * 4) = acc[i][j];
+    rows.put(tid, s_pos, s_page, s_freq, s_bias);
+    __syncthreads();
+    tile_epilogue<BM, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
+  } else {
+    register_epilogue<TM, TN, EPI>(acc, e, m0 + wm * WTM, n0 + wn * WTN, M, N, c, g);
+  }
 }
 
 // ============================================================ bf16, 256 x 256 by two groups of waves
@@ -605,7 +691,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   constexpr int W_AT = NG * PIECE, W_STEP = (BN / 16) * 1024;
   constexpr int C_STRIDE = BN + 4;
   constexpr size_t C_BYTES = (size_t)HALF * C_STRIDE * sizeof(float);
-  __shared__ __attribute__((aligned(1024))) char smem[C_BYTES > W_AT + 4 * W_STEP ? C_BYTES : W_AT + 4 * W_STEP];
+  __shared__ __attribute__((aligned(1024))) char smem[EPI == EPI_QKV && C_BYTES > W_AT + 4 * W_STEP ? C_BYTES : W_AT + 4 * W_STEP];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave >> 2;                             // waves 0-3 and 4-7: one of each on every SIMD
@@ -756,7 +842,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
         barrier();
       }
     }
@@ -765,29 +851,29 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
   __builtin_amdgcn_s_waitcnt(0x0070);                    // the last loads (past K, never read) are in
   barrier();
 
-  // ---- epilogue: the rows 0-127 of the tile through LDS, then the rest
-  float* Cs = (float*)smem;
-  if constexpr (QKV) rows.put(tid, s_pos, s_page, s_freq, s_bias);
-  auto to_lds = [&](int part) {
+  // ---- epilogue
+  if constexpr (QKV) {      // the rows 0-127 of the tile through LDS, then the rest
+    float* Cs = (float*)smem;
+    rows.put(tid, s_pos, s_page, s_freq, s_bias);
+    auto to_lds = [&](int part) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int row = wm * (BM / 2) + i * 16;             // of the tile
-      if (row / HALF == part) {
+      for (int i = 0; i < TM; ++i) {
+        const int row = wm * (BM / 2) + i * 16;             // of the tile
+        if (row / HALF == part) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int x = 0; x < 4; ++x)
-            Cs[(row % HALF + g * 4 + x) * C_STRIDE + wn * 64 + j * 16 + c] = acc[i][j][x];
+          for (int j = 0; j < 4; ++j) *(floatx4*)(Cs + (row % HALF + c) * C_STRIDE + wn * 64 + j * 16 + g * 4) = acc[i][j];
+        }
       }
-    }
+      __syncthreads();
+    };
+    to_lds(0);
+    tile_epilogue<HALF, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
     __syncthreads();
-  };
-  to_lds(0);
-  tile_epilogue<HALF, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
-  __syncthreads();
-  to_lds(1);
-  tile_epilogue<BM - HALF, BN, NT, EPI>(Cs, e, m0 + HALF, n0, M, N, tid, s_pos + (QKV ? HALF : 0),
-                                        s_page + (QKV ? HALF : 0), s_freq, s_bias);
+    to_lds(1);
+    tile_epilogue<BM - HALF, BN, NT, EPI>(Cs, e, m0 + HALF, n0, M, N, tid, s_pos + HALF, s_page + HALF, s_freq, s_bias);
+  } else {
+    register_epilogue<TM, 4, EPI>(acc, e, m0 + wm * (BM / 2), n0 + wn * 64, M, N, c, g);
+  }
 }
 
 // ============================================================ bf16, small tiles by direct loads
@@ -811,7 +897,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__
   constexpr int STAGE = (XL + WL) * 1024, W_AT = XL * 1024;
   constexpr int C_STRIDE = BN + 4;
   constexpr size_t C_BYTES = (size_t)BM * C_STRIDE * sizeof(float);
-  __shared__ __attribute__((aligned(1024))) char smem[C_BYTES > NST * STAGE ? C_BYTES : NST * STAGE];
+  __shared__ __attribute__((aligned(1024))) char smem[EPI == EPI_QKV && C_BYTES > NST * STAGE ? C_BYTES : NST * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   int bx = blockIdx.x, by = blockIdx.y;
@@ -906,7 +992,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], b[h][j], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h][j], a[h][i], acc[i][j], 0, 0, 0);
   };
   fetch(0, 0);
   if constexpr (QKV) rows.page(e);      // (waits for the first stage too, which has to come first in any case)
@@ -932,16 +1018,19 @@ __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__
   }
   __builtin_amdgcn_s_waitcnt(0x0070);                    // the last loads (past K, never read) are in
   barrier();
-  float* Cs = (float*)smem;
+  if constexpr (QKV) {
+    float* Cs = (float*)smem;
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) Cs[(wm * WTM + i * 16 + g * 4 + x) * C_STRIDE + wn * WTN + j * 16 + c] = acc[i][j][x];
-  if constexpr (QKV) rows.put(tid, s_pos, s_page, s_freq, s_bias);
-  __syncthreads();
-  tile_epilogue<BM, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
+      for (int j = 0; j < TN; ++j)
+        *(floatx4*)(Cs + (wm * WTM + i * 16 + c) * C_STRIDE + wn * WTN + j * 16 + g * 4) = acc[i][j];
+    rows.put(tid, s_pos, s_page, s_freq, s_bias);
+    __syncthreads();
+    tile_epilogue<BM, BN, NT, EPI>(Cs, e, m0, n0, M, N, tid, s_pos, s_page, s_freq, s_bias);
+  } else {
+    register_epilogue<TM, TN, EPI>(acc, e, m0 + wm * WTM, n0 + wn * WTN, M, N, c, g);
+  }
 }
 
 // ================================================================ float32
