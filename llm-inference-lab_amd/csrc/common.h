@@ -74,22 +74,34 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// The same for waves whose 64 lanes are all active: within rows of sixteen lanes by the operand swizzles
-// of DPP, across the rows by the lane-swap instructions of gfx950.  (wave_sum above takes six trips through
-// the LDS crossbar, one behind the other.)
+// The same, to the bit, for waves whose 64 lanes are all active: across the rows of sixteen lanes by the lane-swap
+// instructions of gfx950, within a row by the rotations and swizzles of DPP.  (wave_sum above takes six trips
+// through the LDS crossbar, one behind the other.)  A rotation by 8 pairs the lanes that are 8 apart; then a row holds
+// every number twice, and one by 4 pairs what is 4 apart.
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float full_wave_sum(float v) {
-  v += dpp_move<0xB1>(v);       // lanes 1 apart (quad_perm 1, 0, 3, 2)
-  v += dpp_move<0x4E>(v);       // 2 apart (quad_perm 2, 3, 0, 1)
-  v += dpp_move<0x141>(v);      // the other four of eight (row_half_mirror)
-  v += dpp_move<0x140>(v);      // the other eight of sixteen (row_mirror)
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+template <typename F>
+__device__ __forceinline__ float full_wave_reduce(float v, F op) {
   const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  v = op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = op(v, dpp_move<0x128>(v));      // row_ror:8
+  v = op(v, dpp_move<0x124>(v));      // row_ror:4
+  v = op(v, dpp_move<0x4E>(v));       // quad_perm 2, 3, 0, 1
+  return op(v, dpp_move<0xB1>(v));    // quad_perm 1, 0, 3, 2
+}
+__device__ __forceinline__ float full_wave_sum(float v) {
+  return full_wave_reduce(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float full_wave_max(float v) {
+  return full_wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// what lane `from` (the same for the whole wave) holds
+__device__ __forceinline__ float lane_value(float v, int from) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), from));
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.

@@ -1,5 +1,7 @@
 // Embedding gather, RMSNorm, and rotary position encoding fused with the
 // write of keys and values into the paged cache.  gfx950 only.
+#include <type_traits>
+
 #include "common.h"
 
 extern "C" const char* llmlab_last_error() { return g_llmlab_error; }
@@ -70,89 +72,111 @@ extern "C" int llmlab_embed(const void* table, int dtype, int packed, const int*
 // A thread keeps its first KEEP groups of W elements (and their weights) in
 // registers, so a row of up to KEEP * W * blockDim.x elements costs one trip to
 // memory; what lies beyond is read again after the reduction.  VEC: groups of four
-// (hidden % 4 == 0 and 16-byte aligned rows).
-template <typename T, bool VEC, int G>
+// (hidden % 4 == 0 and 16-byte aligned rows).  All loads of a trip are unconditional (past the row's end its last
+// group again, not counted): under a branch each would be waited for before the next is asked for.
+template <typename T, bool VEC, int KEEP, int G>
 __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w, int w_bf16,
                                float eps, T* __restrict__ out, const int* __restrict__ rows,
                                int hidden, const float* __restrict__ pend, int splits, size_t pend_stride) {
-  constexpr int KEEP = 4, W = VEC ? 4 : 1;
-  __shared__ float red[17];
+  constexpr int W = VEC ? 4 : 1;
+  __shared__ float red[16];
   const int i = blockIdx.x;
   const int r = rows ? rows[i] : i;
   float* src = x + (size_t)r * hidden;
   const float* prow = pend + (size_t)r * hidden;
   const int stride = blockDim.x * W;
-  float keep[KEEP][W], wk[KEEP][W];
-  float ss = 0.f;
-  // Pieces come G at a time, loads unconditional (past the last piece: the last one again,
-  // not added), so that they travel together instead of one after the other: G = 4 for
-  // the many pieces that few rows bring (a step bound by latency).  One or two pieces,
-  // which many rows bring, are taken one by one (G = 1, a kernel of its own): that step
+  struct alignas(4 * W) Group {
+    float v[W];
+  };
+  auto get = [](const float* p) {
+    Group g;
+    if constexpr (VEC) *(floatx4*)g.v = *(const floatx4*)p;
+    else g.v[0] = *p;
+    return g;
+  };
+  auto weights = [&](int c) {
+    Group g;
+    if constexpr (VEC) {
+      if (!w_bf16) return get((const float*)w + c);
+      const bf16x4 b = *(const bf16x4*)((const bf16_t*)w + c);
+#pragma unroll
+      for (int e = 0; e < W; ++e) g.v[e] = (float)b[e];
+    } else {
+      g.v[0] = load_vec(w, w_bf16, c);
+    }
+    return g;
+  };
+  // The whole values of N groups from element c on, `stride` apart, written back if pieces came in.  Pieces come G at a
+  // time, so that they travel together: G = 4 for the many pieces that few rows bring (a step bound by
+  // latency).  One or two pieces, which many rows bring, are taken one by one (G = 1): that step
   // is bound by the memory rate, and the registers of a group would cost it waves (2,048
   // rows of 896 with two pieces: 8.8 us one by one, 10.7 in pairs).
-  auto fetch = [&](int c, float* v) {       // the whole values of elements c .. c+W-1, written back if pieces came in
-    if constexpr (VEC) {
-      floatx4 t = *(const floatx4*)(src + c);
-      for (int s0 = 0; s0 < splits; s0 += G) {
-        floatx4 p[G];
+  auto fetch = [&](auto count, int c, Group* g) {
+    constexpr int N = decltype(count)::value;
+    auto at = [&](int j) { return min(c + j * stride, hidden - W); };
 #pragma unroll
-        for (int j = 0; j < G; ++j) p[j] = *(const floatx4*)(prow + (size_t)min(s0 + j, splits - 1) * pend_stride + c);
+    for (int j = 0; j < N; ++j) g[j] = get(src + at(j));
+    for (int s0 = 0; s0 < splits; s0 += G) {
+      Group p[N][G];
 #pragma unroll
-        for (int j = 0; j < G; ++j)
-          if (s0 + j < splits) t += p[j];
-      }
-      if (splits > 0) *(floatx4*)(src + c) = t;
+      for (int j = 0; j < N; ++j)
 #pragma unroll
-      for (int e = 0; e < W; ++e) v[e] = t[e];
-    } else {
-      float t = src[c];
-      for (int s0 = 0; s0 < splits; s0 += G) {
-        float p[G];
+        for (int q = 0; q < G; ++q) p[j][q] = get(prow + (size_t)min(s0 + q, splits - 1) * pend_stride + at(j));
 #pragma unroll
-        for (int j = 0; j < G; ++j) p[j] = prow[(size_t)min(s0 + j, splits - 1) * pend_stride + c];
+      for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int j = 0; j < G; ++j) t += s0 + j < splits ? p[j] : 0.f;
-      }
-      if (splits > 0) src[c] = t;
-      v[0] = t;
+        for (int q = 0; q < G; ++q)
+#pragma unroll
+          for (int e = 0; e < W; ++e) g[j].v[e] += s0 + q < splits ? p[j][q].v[e] : 0.f;
     }
   };
+  auto put_back = [&](int c, const Group& g) {
+    if (splits > 0) {
+      if constexpr (VEC) *(floatx4*)(src + c) = *(const floatx4*)g.v;
+      else src[c] = g.v[0];
+    }
+  };
+  Group keep[KEEP], wk[KEEP];
+  float ss = 0.f;
+  const int c0 = threadIdx.x * W;
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) wk[j] = weights(min(c0 + j * stride, hidden - W));
+  fetch(std::integral_constant<int, KEEP>{}, c0, keep);
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
-    const int c = threadIdx.x * W + j * stride;
-    if (c < hidden) {
-      fetch(c, keep[j]);
+    const int c = c0 + j * stride;
+    if (c < hidden) put_back(c, keep[j]);
 #pragma unroll
-      for (int e = 0; e < W; ++e) { wk[j][e] = load_vec(w, w_bf16, c + e); ss += keep[j][e] * keep[j][e]; }
-    }
+    for (int e = 0; e < W; ++e) ss += c < hidden ? keep[j].v[e] * keep[j].v[e] : 0.f;
   }
-  for (int c = threadIdx.x * W + KEEP * stride; c < hidden; c += stride) {
-    float v[W];
-    fetch(c, v);
+  for (int c = c0 + KEEP * stride; c < hidden; c += stride) {
+    Group g;
+    fetch(std::integral_constant<int, 1>{}, c, &g);
+    put_back(c, g);
 #pragma unroll
-    for (int e = 0; e < W; ++e) ss += v[e] * v[e];
+    for (int e = 0; e < W; ++e) ss += g.v[e] * g.v[e];
   }
-  ss = block_sum(ss, red);      // (a barrier; below a thread reads back only what it wrote itself)
+  ss = full_wave_sum(ss);            // (whole waves, all of whose threads come here)
+  const int waves = blockDim.x >> 6;
+  if (waves > 1) {                   // (a barrier; below a thread reads back only what it wrote itself)
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = 0.f;
+    for (int k = 0; k < waves; ++k) ss += red[k];
+  }
   const float inv = rsqrtf(ss / (float)hidden + eps);
   T* dst = out + (size_t)i * hidden;
+  auto put = [&](int c, const Group& g, const Group& wg) {
+    typedef T Out __attribute__((ext_vector_type(W)));
+    Out o;
 #pragma unroll
-  for (int j = 0; j < KEEP; ++j) {
-    const int c = threadIdx.x * W + j * stride;
-    if (c < hidden) {
-      if constexpr (VEC) {
-        typedef T outx4 __attribute__((ext_vector_type(4)));
-        outx4 o;
+    for (int e = 0; e < W; ++e) o[e] = from_float<T>(g.v[e] * inv * wg.v[e]);
+    *(Out*)(dst + c) = o;
+  };
 #pragma unroll
-        for (int e = 0; e < W; ++e) o[e] = from_float<T>(keep[j][e] * inv * wk[j][e]);
-        *(outx4*)(dst + c) = o;
-      } else {
-        dst[c] = from_float<T>(keep[j][0] * inv * wk[j][0]);
-      }
-    }
-  }
-  for (int c = threadIdx.x * W + KEEP * stride; c < hidden; c += stride)
-#pragma unroll
-    for (int e = 0; e < W; ++e) dst[c + e] = from_float<T>(src[c + e] * inv * load_vec(w, w_bf16, c + e));
+  for (int j = 0; j < KEEP; ++j)
+    if (c0 + j * stride < hidden) put(c0 + j * stride, keep[j], wk[j]);
+  for (int c = c0 + KEEP * stride; c < hidden; c += stride) put(c, get(src + c), weights(c));
 }
 
 extern "C" int llmlab_rmsnorm(float* x, const void* w, int w_dtype, float eps, void* out,
@@ -163,25 +187,30 @@ extern "C" int llmlab_rmsnorm(float* x, const void* w, int w_dtype, float eps, v
                  "rmsnorm: pending sums go with all rows in order");
   if (n_out == 0) return 0;
   const bool vec = hidden % 4 == 0 && pend_stride % 4 == 0 &&
-                   (((uintptr_t)x | (uintptr_t)pend | (uintptr_t)out) & 15) == 0;
-  // few rows are bound by latency, not by the memory rate: then a row is spread over as
-  // many threads as it has groups of four numbers, so that every thread's loads (its
-  // numbers and the pieces owed to them) are one round
-  int threads = hidden >= 8192 ? 512 : 256;
-  if (n_out <= 128)
-    while (threads < 1024 && threads * 4 < hidden) threads *= 2;
+                   (((uintptr_t)x | (uintptr_t)pend | (uintptr_t)out) & 15) == 0 &&
+                   ((uintptr_t)w & (w_dtype == DT_BF16 ? 7 : 15)) == 0;
+  const int groups = hidden / (vec ? 4 : 1);
+  // Few rows are bound by latency (and up to 1,024 narrow ones): a row is spread over as many threads as it has groups,
+  // so that every thread's loads (its numbers and the pieces owed to them) are one round.  Many rows: four groups a thread
+  // (two with many pieces: registers), a row of 1,024 and less a wave of its own without a barrier.  (2,367 rows of 3584
+  // 15.3 -> 11.6 us by that and by loads that travel together; 512 of 896 4.0 a group a thread, 4.4 four.)
+  const int keep = n_out <= 128 || (n_out <= 1024 && groups <= 256) ? 1 : splits > 2 ? 2 : 4;
+  int threads = 64;
+  while (threads < 1024 && threads * keep < groups) threads *= 2;
   dim3 grid(n_out), block(threads);
+#define LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, G)                                                               \
+  hipLaunchKernelGGL((rmsnorm_kernel<T, VEC, KEEP, G>), grid, block, 0, stream, x, w, w_dtype == DT_BF16, eps, \
+                     (T*)out, rows, hidden, pend, splits, pend_stride)
 #define LLMLAB_RMSNORM(T, VEC)                                                                             \
   do {                                                                                                     \
-    if (splits > 2)                                                                                        \
-      hipLaunchKernelGGL((rmsnorm_kernel<T, VEC, 4>), grid, block, 0, stream, x, w, w_dtype == DT_BF16, eps, \
-                         (T*)out, rows, hidden, pend, splits, pend_stride);                                \
-    else                                                                                                   \
-      hipLaunchKernelGGL((rmsnorm_kernel<T, VEC, 1>), grid, block, 0, stream, x, w, w_dtype == DT_BF16, eps, \
-                         (T*)out, rows, hidden, pend, splits, pend_stride);                                \
+    if (keep == 4) LLMLAB_RMSNORM_KEEP(T, VEC, 4, 1);                                                      \
+    else if (keep == 2) LLMLAB_RMSNORM_KEEP(T, VEC, 2, 4);                                                 \
+    else if (splits > 2) LLMLAB_RMSNORM_KEEP(T, VEC, 1, 4);                                                \
+    else LLMLAB_RMSNORM_KEEP(T, VEC, 1, 1);                                                                \
   } while (0)
   if (out_dtype == DT_BF16) { if (vec) LLMLAB_RMSNORM(bf16_t, true); else LLMLAB_RMSNORM(bf16_t, false); }
   else                      { if (vec) LLMLAB_RMSNORM(float, true);  else LLMLAB_RMSNORM(float, false); }
+#undef LLMLAB_RMSNORM_KEEP
 #undef LLMLAB_RMSNORM
   LLMLAB_LAUNCH_CHECK("rmsnorm");
   return 0;
@@ -549,7 +578,7 @@ __global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
     return g;
   };
   auto total = [&](float v, int which) {
-    v = wave_sum(v);
+    v = full_wave_sum(v);      // (whole waves, all of whose threads come here)
     if constexpr (!ONE_WAVE) {
       if ((threadIdx.x & 63) == 0) red[which * 16 + (threadIdx.x >> 6)] = v;
       __syncthreads();
