@@ -937,20 +937,20 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void attention_merge_kernel(
         v[p][u] = (u0 + u < u_hi && dd < D) ? o_part[(at0 + u0 + u) * D + dd] : 0.f;
       }
     if (u0 == u_lo) {     // the weights, while the first loads are under way
-      mmax = wave_max(fmaxf(ms[0], ms[1]));
+      mmax = full_wave_max(fmaxf(ms[0], ms[1]));
 #pragma unroll
       for (int h = 0; h < 2; ++h) w[h] = ms[h] == NEG_INF ? 0.f : exp2f(ms[h] - mmax);
     }
 #pragma unroll
     for (int p = 0; p < PER; ++p)
 #pragma unroll
-      for (int u = 0; u < 16; ++u) num[p] += __shfl(u0 + u < 64 ? w[0] : w[1], (u0 + u) & 63, WAVE) * v[p][u];
+      for (int u = 0; u < 16; ++u) num[p] += lane_value(u0 + u < 64 ? w[0] : w[1], (u0 + u) & 63) * v[p][u];
   }
 #pragma unroll
   for (int p = 0; p < PER; ++p) s_num[wave][p * 64 + lane] = num[p];
   __syncthreads();
   if (wave != 0) return;
-  const float den = wave_sum(w[0] * ls[0] + w[1] * ls[1]);
+  const float den = full_wave_sum(w[0] * ls[0] + w[1] * ls[1]);
   const float inv = den > 0.f ? 1.f / den : 0.f;
 #pragma unroll
   for (int p = 0; p < PER; ++p) {

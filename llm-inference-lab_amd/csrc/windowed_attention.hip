@@ -55,6 +55,12 @@ __global__ __launch_bounds__(512) void project_norm_write_quads_kernel(NormWrite
   const int pos = a.positions ? a.positions[r] : 0;
   const int page = a.own ? a.table[(size_t)a.row_req[r] * a.max_pages + pos / a.page_size] : 0;
   const int slot = pos % a.page_size;
+  // (what the second half reads from memory is on its way from the start: the first quad's weights, the first value)
+  const int quads = a.DK >> 2, heads = a.n_heads + (a.own ? a.n_kv : 0);
+  const int h0 = min((int)threadIdx.x / quads, heads - 1), d0 = min(4 * ((int)threadIdx.x % quads), a.D - 4);
+  floatx4 w0 = floatx4{1.f, 1.f, 1.f, 1.f};
+  if (a.norm) w0 = load4(h0 < a.n_heads ? a.q_w + (size_t)h0 * a.D + d0 : a.k_w + (size_t)(h0 - a.n_heads) * a.D + d0);
+  const float value0 = a.own ? src[turned + min((int)threadIdx.x, a.n_kv * a.E - 1)] : 0.f;
   float sq = 0.f, sk = 0.f;
   for (int c0 = 4 * threadIdx.x; c0 < turned; c0 += 16 * threads) {    // (four loads travel together)
     floatx4 v[4];
@@ -77,8 +83,8 @@ __global__ __launch_bounds__(512) void project_norm_write_quads_kernel(NormWrite
     s_sin[i] = sn;
   }
   if (a.norm) {
-    sq = wave_sum(sq);
-    sk = wave_sum(sk);
+    sq = full_wave_sum(sq);      // (whole waves, all of whose threads come here)
+    sk = full_wave_sum(sk);
     if (lane == 0) {
       red_q[wave] = sq;
       red_k[wave] = sk;
@@ -95,7 +101,6 @@ __global__ __launch_bounds__(512) void project_norm_write_quads_kernel(NormWrite
     inv_q = 1.0f / sqrtf(sq / (float)q_size + a.eps);
     if (k_size > 0) inv_k = 1.0f / sqrtf(sk / (float)k_size + a.eps);
   }
-  const int quads = a.DK >> 2, heads = a.n_heads + (a.own ? a.n_kv : 0);
   for (int i = threadIdx.x; i < heads * quads; i += threads) {
     const int h = i / quads, d = 4 * (i - h * quads);
     const bool query = h < a.n_heads;
@@ -104,7 +109,7 @@ __global__ __launch_bounds__(512) void project_norm_write_quads_kernel(NormWrite
       const float* w = query ? a.q_w + (size_t)h * a.D : a.k_w + (size_t)(h - a.n_heads) * a.D;
       const float inv = query ? inv_q : inv_k;
       v = load4(s_row + h * a.D + d);
-      if (a.norm) v *= inv * load4(w + d);
+      if (a.norm) v *= inv * (i == (int)threadIdx.x ? w0 : load4(w + d));
       if (d < a.rot_dims) {
         const bool first = d < half;
         const int o = first ? d + half : d - half, at = first ? d : d - half;
@@ -120,7 +125,8 @@ __global__ __launch_bounds__(512) void project_norm_write_quads_kernel(NormWrite
   if (!a.own) return;
   for (int c = threadIdx.x; c < a.n_kv * a.E; c += threads) {
     const int g = c / a.E, e = c - g * a.E;
-    v_cache[((size_t)page * a.n_kv + g) * a.page_size * a.E + value_index(slot, e, a.E)] = from_float<T>(src[turned + c]);
+    v_cache[((size_t)page * a.n_kv + g) * a.page_size * a.E + value_index(slot, e, a.E)] =
+        from_float<T>(c == (int)threadIdx.x ? value0 : src[turned + c]);
   }
 }
 
@@ -1414,54 +1420,70 @@ __global__ __launch_bounds__(64) void sink_window_attention_grouped_kernel(MfmaA
 }
 
 // out[r, h] = sum_z exp(m_z - M) o_z / sum_z exp(m_z - M) l_z over the shares of the row's keys.
-// One wave per (row, head).  The shares' maxima and sums are read once, a lane a share; the
-// shares' weights exp(m_z - M) lie in LDS, and the loop over the shares' partial outputs has no
-// branch (an empty share weighs zero and its numbers are dropped), so its loads travel together.
+// One wave per (row, head).  The shares' maxima and sums are read once, a lane a share, and the first CHUNK shares' partial
+// outputs are asked for beside them; the shares' weights exp(m_z - M) lie in LDS, and the loop over the partial outputs
+// has no branch (past the last share that one again; an empty share, or one again, weighs zero and its numbers are
+// dropped), so that a chunk's loads for all of the wave's channels travel together.  (Sixteen rows of 16 heads of 128 in
+// 17 shares: 6.5 us in a decode step with four shares' loads of 64 channels at a time, 4.3 so.)
 constexpr int MERGE_MAX_SPLITS = 256;
+template <int P>       // channels of a lane: E up to 64 P
 __global__ __launch_bounds__(64) void sink_window_attention_merge_kernel(MfmaArgs a, int E) {
+  constexpr int CHUNK = P <= 2 ? 16 : 8;
   __shared__ float s_w[MERGE_MAX_SPLITS];
-  const int r = blockIdx.x, h = blockIdx.y;
-  const int b = a.row_req[r];
-  if (a.long_from > 0 && a.q_start[b + 1] - a.q_start[b] >= a.long_from) return;
+  const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  if (a.long_from > 0) {
+    const int b = a.row_req[r];
+    if (a.q_start[b + 1] - a.q_start[b] >= a.long_from) return;
+  }
   const size_t first = ((size_t)r * a.n_heads + h) * a.splits;
   constexpr int PER_LANE = MERGE_MAX_SPLITS / 64;
-  float m[PER_LANE], l[PER_LANE];
+  float m[PER_LANE], l[PER_LANE], o[P][CHUNK];
+#pragma unroll
+  for (int i = 0; i < PER_LANE; ++i) {
+    const int at = min(lane + 64 * i, a.splits - 1);
+    m[i] = a.part_ml[(first + at) * 2];
+    l[i] = a.part_ml[(first + at) * 2 + 1];
+  }
+  auto ask = [&](int z0) {
+#pragma unroll
+    for (int j = 0; j < CHUNK; ++j)
+#pragma unroll
+      for (int p = 0; p < P; ++p) o[p][j] = a.part_o[(first + min(z0 + j, a.splits - 1)) * E + min(lane + 64 * p, E - 1)];
+  };
+  ask(0);
   float big = NEG_INF;
 #pragma unroll
   for (int i = 0; i < PER_LANE; ++i) {
-    const int z = threadIdx.x + 64 * i;
-    const int at = min(z, a.splits - 1);
-    const float mz = a.part_ml[(first + at) * 2], lz = a.part_ml[(first + at) * 2 + 1];
-    m[i] = z < a.splits ? mz : NEG_INF;
-    l[i] = lz;
+    if (lane + 64 * i >= a.splits) m[i] = NEG_INF;
     big = fmaxf(big, m[i]);
   }
-  big = wave_max(big);
+  big = full_wave_max(big);
   float den = 0.f;
 #pragma unroll
   for (int i = 0; i < PER_LANE; ++i) {
     const float w = m[i] != NEG_INF ? __expf(m[i] - big) : 0.f;
     if (w != 0.f) den = fmaf(w, l[i], den);
-    s_w[threadIdx.x + 64 * i] = w;
+    s_w[lane + 64 * i] = w;
   }
-  den = wave_sum(den);
+  den = full_wave_sum(den);
   __syncthreads();
+  float acc[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) acc[p] = 0.f;
+  for (int z0 = 0; z0 < a.splits; z0 += CHUNK) {
+    if (z0 > 0) ask(z0);
+#pragma unroll
+    for (int j = 0; j < CHUNK; ++j) {
+      const float w = z0 + j < a.splits ? s_w[min(z0 + j, MERGE_MAX_SPLITS - 1)] : 0.f;
+#pragma unroll
+      for (int p = 0; p < P; ++p) acc[p] = fmaf(w, w != 0.f ? o[p][j] : 0.f, acc[p]);
+    }
+  }
   const float inv = a.gate.head(r, h) / den;
-  for (int e = threadIdx.x; e < E; e += 64) {
-    float acc = 0.f;
-    int z = 0;
-    for (; z + 4 <= a.splits; z += 4) {
-      float o[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = a.part_o[(first + z + j) * E + e];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc = fmaf(s_w[z + j], s_w[z + j] != 0.f ? o[j] : 0.f, acc);
-    }
-    for (; z < a.splits; ++z) {
-      const float o = a.part_o[(first + z) * E + e];
-      acc = fmaf(s_w[z], s_w[z] != 0.f ? o : 0.f, acc);
-    }
-    a.out[((size_t)r * a.n_heads + h) * E + e] = (bf16_t)(acc * inv * a.gate.at(r, h * E + e));
+  for (int p = 0; p < P; ++p) {
+    const int e = lane + 64 * p;
+    if (e < E) a.out[((size_t)r * a.n_heads + h) * E + e] = (bf16_t)(acc[p] * inv * a.gate.at(r, h * E + e));
   }
 }
 
@@ -1578,7 +1600,10 @@ extern "C" int llmlab_sink_window_attention(const void* q, int dtype, int rows, 
       launch_mfma_any(D, E, 1, dim3(rows, n_kv * per_group, a.splits), dim3(64), stream, a);
       LLMLAB_LAUNCH_CHECK("sink_window_attention (decoding)");
       if (a.splits > 1) {
-        hipLaunchKernelGGL(sink_window_attention_merge_kernel, dim3(rows, n_heads), dim3(64), 0, stream, a, E);
+        const dim3 grid(rows, n_heads);
+        if (E <= 64) hipLaunchKernelGGL(sink_window_attention_merge_kernel<1>, grid, dim3(64), 0, stream, a, E);
+        else if (E <= 128) hipLaunchKernelGGL(sink_window_attention_merge_kernel<2>, grid, dim3(64), 0, stream, a, E);
+        else hipLaunchKernelGGL(sink_window_attention_merge_kernel<4>, grid, dim3(64), 0, stream, a, E);
         LLMLAB_LAUNCH_CHECK("sink_window_attention (merge)");
       }
     }
