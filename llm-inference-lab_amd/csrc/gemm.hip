@@ -33,8 +33,8 @@
 //       issuing MFMAs, both operands loaded from global memory straight into LDS
 //       (gemm_bf16_pingpong): 1.1 to 1.25 PF/s where the tiles above reach 0.9 to 0.97.
 //     (products of few rows, as in decode steps, have kernels of their own in decode.hip)
-//   float32: numbers split into three bfloat16 parts for the matrix cores, 32-bit products and sums
-//     as exact as plain FMAs (gemm_f32_split_kernel); a plain FMA kernel beside it as its
+//   float32: numbers split into three bfloat16 parts (W in one where its numbers are bfloat16 ones) for the matrix
+//     cores, 32-bit products and sums as exact as plain FMAs (gemm_f32_split_kernel); a plain FMA kernel beside it as its
 //     reference (tiles of 64x64 to 128x128, 4x4 to 8x8 outputs per thread); for up to 64 rows one in
 //     which a wave owns four rows of W and its lanes split the inner size.
 //
@@ -288,8 +288,8 @@ __device__ __forceinline__ void register_epilogue(const floatx4 (&acc)[TM][TN], 
 }
 
 // The epilogue of a q/k/v tile of BM x BN sums that lies in LDS (rows of BN + 4 floats), by the NT
-// threads of the block: global memory is written (and the residual read) in pieces of 16 bytes,
-// consecutive lanes next to each other.  s_pos, s_page, s_freq and s_bias are what the QKV
+// threads of the block: global memory is written in pieces of 16 bytes, consecutive lanes next to
+// each other.  s_pos, s_page, s_freq and s_bias are what the QKV
 // epilogue fetched per row and per column of the tile before the product.
 template <int BM, int BN, int NT, int EPI>
 __device__ __forceinline__ void tile_epilogue(const float* Cs, const EpiArgs& e, int m0, int n0, int M, int N,
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_tiled(const bf16_t* __
 // LDS and the matrix instructions of a compute unit overlap by construction and not by
 // the luck of the scheduler (all eight waves in step: 975 TF/s on 8192 x 37888 x 3584,
 // the groups apart: 1065; the 128 x 256 tile of the kernel above: 966).  A block fills a
-// compute unit; the epilogue takes the two halves of the rows through LDS one after the other.
+// compute unit; the q/k/v epilogue takes the two halves of the rows through LDS one after the other.
 //
 // What bounds it is the way of x to the compute units, line by line: with 1 KB of consecutive
 // memory a load in place of rows the same loop is 20 % faster.  W has such tiles (packed:
