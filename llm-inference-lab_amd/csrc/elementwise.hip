@@ -63,6 +63,36 @@ extern "C" int llmlab_embed(const void* table, int dtype, int packed, const int*
 }
 
 // ----------------------------------------------------------------- RMSNorm
+// W neighbouring weights as they lie in memory, bfloat16 or float32, and their values.  Two loads of 8 bytes without a
+// branch (of the same 8 where the weights are bfloat16): converted on the way, each group was waited for
+// before the next, and the row, were asked for (48 rows of 896, back to back in a graph, 2.7 us so and 2.1 now; 2,048 rows
+// 4.1 and 3.1).
+template <int W>
+struct RawWeights {
+  uint32_t u[W];
+  __device__ __forceinline__ float value(int e, int w_bf16) const {
+    const uint32_t b = W == 1 ? u[0] << 16 : e & 1 ? u[e / 2] & 0xffff0000u : u[e / 2] << 16;
+    return __uint_as_float(w_bf16 ? b : u[e]);
+  }
+};
+
+template <int W>
+__device__ __forceinline__ RawWeights<W> ask_for_weights(const void* w, int w_bf16, int c) {
+  RawWeights<W> raw;
+  if constexpr (W == 4) {
+    typedef uint32_t Pair __attribute__((ext_vector_type(2)));
+    const char* at = (const char*)w + (size_t)c * (w_bf16 ? 2 : 4);
+    const Pair lo = *(const Pair*)at, hi = *(const Pair*)(at + (w_bf16 ? 0 : 8));
+    raw.u[0] = lo[0];
+    raw.u[1] = lo[1];
+    raw.u[2] = hi[0];
+    raw.u[3] = hi[1];
+  } else {
+    raw.u[0] = w_bf16 ? ((const uint16_t*)w)[c] : ((const uint32_t*)w)[c];
+  }
+  return raw;
+}
+
 // out[i, :] = x[row_i, :] * rsqrt(mean(x[row_i]^2) + eps) * w, row_i = rows[i] or
 // i.  The square, the mean, the rsqrt and both products are float32; one
 // rounding to T at the end.
@@ -94,40 +124,32 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w
     else g.v[0] = *p;
     return g;
   };
-  auto weights = [&](int c) {
-    Group g;
-    if constexpr (VEC) {
-      if (!w_bf16) return get((const float*)w + c);
-      const bf16x4 b = *(const bf16x4*)((const bf16_t*)w + c);
-#pragma unroll
-      for (int e = 0; e < W; ++e) g.v[e] = (float)b[e];
-    } else {
-      g.v[0] = load_vec(w, w_bf16, c);
-    }
-    return g;
-  };
+  auto weights = [&](int c) { return ask_for_weights<W>(w, w_bf16, c); };
   // The whole values of N groups from element c on, `stride` apart, written back if pieces came in.  Pieces come G at a
-  // time, so that they travel together: G = 4 for the many pieces that few rows bring (a step bound by
-  // latency).  One or two pieces, which many rows bring, are taken one by one (G = 1): that step
-  // is bound by the memory rate, and the registers of a group would cost it waves (2,048
-  // rows of 896 with two pieces: 8.8 us one by one, 10.7 in pairs).
+  // time (G = 0: there are none), the first G with the groups themselves: behind a loop's head the compiler waits for
+  // what is on its way, so that x and one piece after the other cost a trip each (512 rows of 896 with two pieces
+  // 3.4 us so and 2.7 now, 2,048 6.0 and 5.2).
   auto fetch = [&](auto count, int c, Group* g) {
     constexpr int N = decltype(count)::value;
     auto at = [&](int j) { return min(c + j * stride, hidden - W); };
 #pragma unroll
     for (int j = 0; j < N; ++j) g[j] = get(src + at(j));
-    for (int s0 = 0; s0 < splits; s0 += G) {
-      Group p[N][G];
+    if constexpr (G > 0) {
+      auto pieces = [&](int s0) {
+        Group p[N][G];
 #pragma unroll
-      for (int j = 0; j < N; ++j)
+        for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int q = 0; q < G; ++q) p[j][q] = get(prow + (size_t)min(s0 + q, splits - 1) * pend_stride + at(j));
+          for (int q = 0; q < G; ++q) p[j][q] = get(prow + (size_t)min(s0 + q, splits - 1) * pend_stride + at(j));
 #pragma unroll
-      for (int j = 0; j < N; ++j)
+        for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int q = 0; q < G; ++q)
+          for (int q = 0; q < G; ++q)
 #pragma unroll
-          for (int e = 0; e < W; ++e) g[j].v[e] += s0 + q < splits ? p[j][q].v[e] : 0.f;
+            for (int e = 0; e < W; ++e) g[j].v[e] += s0 + q < splits ? p[j][q].v[e] : 0.f;
+      };
+      pieces(0);
+      for (int s0 = G; s0 < splits; s0 += G) pieces(s0);
     }
   };
   auto put_back = [&](int c, const Group& g) {
@@ -136,7 +158,8 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w
       else src[c] = g.v[0];
     }
   };
-  Group keep[KEEP], wk[KEEP];
+  Group keep[KEEP];
+  RawWeights<W> wk[KEEP];
   float ss = 0.f;
   const int c0 = threadIdx.x * W;
 #pragma unroll
@@ -166,11 +189,11 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w
   }
   const float inv = rsqrtf(ss / (float)hidden + eps);
   T* dst = out + (size_t)i * hidden;
-  auto put = [&](int c, const Group& g, const Group& wg) {
+  auto put = [&](int c, const Group& g, const RawWeights<W>& wg) {
     typedef T Out __attribute__((ext_vector_type(W)));
     Out o;
 #pragma unroll
-    for (int e = 0; e < W; ++e) o[e] = from_float<T>(g.v[e] * inv * wg.v[e]);
+    for (int e = 0; e < W; ++e) o[e] = from_float<T>(g.v[e] * inv * wg.value(e, w_bf16));
     *(Out*)(dst + c) = o;
   };
 #pragma unroll
@@ -195,18 +218,19 @@ extern "C" int llmlab_rmsnorm(float* x, const void* w, int w_dtype, float eps, v
   // (two with many pieces: registers), a row of 1,024 and less a wave of its own without a barrier.  (2,367 rows of 3584
   // 15.3 -> 11.6 us by that and by loads that travel together; 512 of 896 4.0 a group a thread, 4.4 four.)
   const int keep = n_out <= 128 || (n_out <= 1024 && groups <= 256) ? 1 : splits > 2 ? 2 : 4;
-  int threads = 64;
-  while (threads < 1024 && threads * keep < groups) threads *= 2;
+  const int threads = min(1024, max(1, (groups + 64 * keep - 1) / (64 * keep)) * 64);
   dim3 grid(n_out), block(threads);
 #define LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, G)                                                               \
   hipLaunchKernelGGL((rmsnorm_kernel<T, VEC, KEEP, G>), grid, block, 0, stream, x, w, w_dtype == DT_BF16, eps, \
                      (T*)out, rows, hidden, pend, splits, pend_stride)
 #define LLMLAB_RMSNORM(T, VEC)                                                                             \
   do {                                                                                                     \
-    if (keep == 4) LLMLAB_RMSNORM_KEEP(T, VEC, 4, 1);                                                      \
+    if (keep == 4 && splits == 0) LLMLAB_RMSNORM_KEEP(T, VEC, 4, 0);                                       \
+    else if (keep == 4) LLMLAB_RMSNORM_KEEP(T, VEC, 4, 2);                                                 \
     else if (keep == 2) LLMLAB_RMSNORM_KEEP(T, VEC, 2, 4);                                                 \
     else if (splits > 2) LLMLAB_RMSNORM_KEEP(T, VEC, 1, 4);                                                \
-    else LLMLAB_RMSNORM_KEEP(T, VEC, 1, 1);                                                                \
+    else if (splits > 0) LLMLAB_RMSNORM_KEEP(T, VEC, 1, 2);                                                \
+    else LLMLAB_RMSNORM_KEEP(T, VEC, 1, 0);                                                                \
   } while (0)
   if (out_dtype == DT_BF16) { if (vec) LLMLAB_RMSNORM(bf16_t, true); else LLMLAB_RMSNORM(bf16_t, false); }
   else                      { if (vec) LLMLAB_RMSNORM(float, true);  else LLMLAB_RMSNORM(float, false); }
@@ -527,10 +551,11 @@ extern "C" int llmlab_add_pending(float* x, const float* pend, int splits, size_
 // A thread keeps its first KEEP groups of W numbers (of the row, the weight and the stream) in
 // registers, all asked for at once, so that a row costs one trip to memory; what lies beyond is
 // read again.  Few rows are bound by that trip: a row is spread over as many threads as it has
-// groups of four, its pieces come G at a time (16 rows of 2048: in three strided passes of 256 threads
-// 6.2 us back to back and 10.8 in a decode step, 3.0 and 4.2 so).  Many rows are bound by the memory rate:
-// ONE_WAVE, a wave a row and no barrier at all (with the stream's copy, 1,900 rows of 896 7.1 -> 5.4 us, 4.4 TB/s;
-// 2,048 of 2048 14.3 -> 10.2).
+// groups of four, its pieces come G at a time (G = 0: it is whole), the first G with the row, the weights and the stream,
+// without a branch (16 rows of 2048 in two pieces, back to back: in three strided passes of 256 threads 6.2 us, 3.2 with
+// the loads of a group under a branch, 2.7 so).  Many rows are bound by the memory rate:
+// ONE_WAVE, a wave a row and no barrier at all (with the stream's copy, 1,900 rows of 896 7.1 -> 5.2 us by that, 4.5 by
+// loads that travel together; in two pieces 5.9 -> 5.1; 2,048 of 2048 14.3 -> 9.9 -> 8.8).
 template <typename T, bool ADD, bool VEC, bool ONE_WAVE, int KEEP, int G>
 __global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
     const float* __restrict__ x, int splits, size_t stride, const void* __restrict__ w, int w_bf16, float eps,
@@ -551,32 +576,37 @@ __global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
     else g.v[0] = *p;
     return g;
   };
-  // (loads unconditional: past the last piece the last one again, not added)
-  auto whole = [&](int c) {
-    Group sum = get(src + c);
-    for (int s0 = 1; s0 < splits; s0 += G) {
-      Group p[G];
+  // The whole values of N groups from element c on, `step` apart (loads unconditional: past the last piece the last one
+  // again, not added; past the row's end its last group again, not counted).
+  auto fetch = [&](auto count, int c, Group* g) {
+    constexpr int N = decltype(count)::value;
+    auto at = [&](int j) { return min(c + j * step, hidden - W); };
 #pragma unroll
-      for (int j = 0; j < G; ++j) p[j] = get(src + min(s0 + j, splits - 1) * stride + c);
+    for (int j = 0; j < N; ++j) g[j] = get(src + at(j));
+    if constexpr (G > 0) {
+      auto pieces = [&](int s0) {
+        Group p[N][G];
 #pragma unroll
-      for (int j = 0; j < G; ++j)
+        for (int j = 0; j < N; ++j)
 #pragma unroll
-        for (int e = 0; e < W; ++e) sum.v[e] += s0 + j < splits ? p[j].v[e] : 0.f;
+          for (int q = 0; q < G; ++q) p[j][q] = get(src + min(s0 + q, splits - 1) * stride + at(j));
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+#pragma unroll
+          for (int q = 0; q < G; ++q)
+#pragma unroll
+            for (int e = 0; e < W; ++e) g[j].v[e] += s0 + q < splits ? p[j][q].v[e] : 0.f;
+      };
+      pieces(1);
+      for (int s0 = 1 + G; s0 < splits; s0 += G) pieces(s0);
     }
-    return sum;
   };
-  auto weights = [&](int c) {
+  auto whole = [&](int c) {
     Group g;
-    if constexpr (VEC) {
-      if (!w_bf16) return get((const float*)w + c);
-      const bf16x4 b = *(const bf16x4*)((const bf16_t*)w + c);
-#pragma unroll
-      for (int e = 0; e < W; ++e) g.v[e] = (float)b[e];
-    } else {
-      g.v[0] = load_vec(w, w_bf16, c);
-    }
+    fetch(std::integral_constant<int, 1>{}, c, &g);
     return g;
   };
+  auto weights = [&](int c) { return ask_for_weights<W>(w, w_bf16, c); };
   auto total = [&](float v, int which) {
     v = full_wave_sum(v);      // (whole waves, all of whose threads come here)
     if constexpr (!ONE_WAVE) {
@@ -587,19 +617,20 @@ __global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
     }
     return v;
   };
-  Group keep[KEEP], wk[KEEP], old[KEEP];
+  Group keep[KEEP], old[KEEP];
+  RawWeights<W> wk[KEEP];
   float s = 0.f;
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
-    const int c = t * W + j * step;
-    if (c < hidden) {
-      keep[j] = whole(c);
-      wk[j] = weights(c);
-      if (ADD) old[j] = get(resid + (size_t)i * hidden + c);
-#pragma unroll
-      for (int e = 0; e < W; ++e) s += keep[j].v[e];
-    }
+    const int c = min(t * W + j * step, hidden - W);
+    wk[j] = weights(c);
+    if (ADD) old[j] = get(resid + (size_t)i * hidden + c);
   }
+  fetch(std::integral_constant<int, KEEP>{}, t * W, keep);
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j)
+#pragma unroll
+    for (int e = 0; e < W; ++e) s += t * W + j * step < hidden ? keep[j].v[e] : 0.f;
   for (int c = t * W + KEEP * step; c < hidden; c += step) {
     const Group g = whole(c);
 #pragma unroll
@@ -614,18 +645,25 @@ __global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
       v += d * d;
     }
   };
+  if constexpr (KEEP == 1 && W == 4) {
+    // (the roundings of the other instances, whose second square is the first one rounded by itself)
+    if (t * W < hidden) {
+      const float d0 = keep[0].v[0] - mean, d1 = keep[0].v[1] - mean, d2 = keep[0].v[2] - mean, d3 = keep[0].v[3] - mean;
+      v = fmaf(d3, d3, fmaf(d2, d2, fmaf(d0, d0, d1 * d1)));
+    }
+  } else
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
     if (t * W + j * step < hidden) deviate(keep[j]);
   for (int c = t * W + KEEP * step; c < hidden; c += step) deviate(whole(c));
   const float inv = 1.0f / sqrtf(total(v, 1) / (float)hidden + eps);
-  auto put = [&](int c, const Group& g, const Group& wg, const Group& og) {
+  auto put = [&](int c, const Group& g, const RawWeights<W>& wg, const Group& og) {
     typedef T Out __attribute__((ext_vector_type(W)));
     Group y;
     Out o;
 #pragma unroll
     for (int e = 0; e < W; ++e) {
-      y.v[e] = (g.v[e] - mean) * inv * wg.v[e];
+      y.v[e] = (g.v[e] - mean) * inv * wg.value(e, w_bf16);
       if (ADD) y.v[e] += og.v[e];
       o[e] = from_float<T>(y.v[e]);
     }
@@ -654,25 +692,29 @@ static void launch_layernorm(const float* x, int splits, size_t stride, const vo
                    (((uintptr_t)out | (uintptr_t)copy) & (4 * sizeof(T) - 1)) == 0 &&
                    ((uintptr_t)w & (w_bf16 ? 7 : 15)) == 0;
   // A wave a row where the rows fill the chip and a row fits a wave's registers; else a block, whose
-  // threads cover the row in one group each.
+  // threads cover the row in one group each, or in two or three where 1,024 threads (256 for more than 128 rows) do not.
+#define LLMLAB_LAYERNORM(VEC, ONE_WAVE, KEEP, G, grid, threads)                                                     \
+  hipLaunchKernelGGL((layernorm_kernel<T, ADD, VEC, ONE_WAVE, KEEP, G>), dim3(grid), dim3(threads), 0, stream, x,   \
+                     splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden)
   if (vec && n_rows > 512 && hidden <= 2048) {
-    if (hidden <= 1024)
-      hipLaunchKernelGGL((layernorm_kernel<T, ADD, true, true, 4, 1>), dim3((n_rows + 3) / 4), dim3(256), 0, stream, x,
-                         splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
-    else
-      hipLaunchKernelGGL((layernorm_kernel<T, ADD, true, true, 8, 1>), dim3((n_rows + 3) / 4), dim3(256), 0, stream, x,
-                         splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
+    const int blocks = (n_rows + 3) / 4;
+    if (hidden <= 1024 && splits == 1) LLMLAB_LAYERNORM(true, true, 4, 0, blocks, 256);
+    else if (hidden <= 1024) LLMLAB_LAYERNORM(true, true, 4, 1, blocks, 256);
+    else if (splits == 1) LLMLAB_LAYERNORM(true, true, 8, 0, blocks, 256);
+    else LLMLAB_LAYERNORM(true, true, 8, 1, blocks, 256);
     return;
   }
   int threads = 64;
   while (threads < 1024 && threads * (vec ? 4 : 1) < hidden) threads += 64;
   if (n_rows > 128 && threads > 256) threads = 256;
-  if (vec)
-    hipLaunchKernelGGL((layernorm_kernel<T, ADD, true, false, 4, 4>), dim3(n_rows), dim3(threads), 0, stream, x, splits,
-                       stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
-  else
-    hipLaunchKernelGGL((layernorm_kernel<T, ADD, false, false, 4, 4>), dim3(n_rows), dim3(threads), 0, stream, x,
-                       splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden);
+  if (vec && threads * 4 >= hidden && splits == 1) LLMLAB_LAYERNORM(true, false, 1, 0, n_rows, threads);
+  else if (vec && threads * 4 >= hidden) LLMLAB_LAYERNORM(true, false, 1, 4, n_rows, threads);
+  else if (vec && threads * 8 >= hidden && splits == 1) LLMLAB_LAYERNORM(true, false, 2, 0, n_rows, threads);
+  else if (vec && threads * 8 >= hidden) LLMLAB_LAYERNORM(true, false, 2, 2, n_rows, threads);
+  else if (vec && splits == 1) LLMLAB_LAYERNORM(true, false, 3, 0, n_rows, threads);
+  else if (vec) LLMLAB_LAYERNORM(true, false, 3, 2, n_rows, threads);
+  else LLMLAB_LAYERNORM(false, false, 4, 4, n_rows, threads);
+#undef LLMLAB_LAYERNORM
 }
 
 // out: n_out rows of the compute dtype; rows: which rows of x (null: all in order).
