@@ -94,9 +94,8 @@ __device__ __forceinline__ float relu2_f(float z) {
   return z * z;
 }
 
-// (by the hardware's reciprocal, one unit in the last place of 32 bits, for results of 8 bits: the division is
-// eleven instructions, and an output of a paired product was sixteen)
-__device__ __forceinline__ float silu_f(float z) { return z * __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
+// (the function of the few-row kernel, to the bit)
+__device__ __forceinline__ float silu_f(float z) { return z / (1.f + __expf(-z)); }
 
 // tanh form of gelu: 0.5 z (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))), as z * sigmoid(2 t)
 __device__ __forceinline__ float gelu_tanh_f(float z) {

@@ -81,3 +81,26 @@ def test_gates_of_any_size(ops, tile):      # noqa: F811
     assert torch.equal(got[want.isinf()], want[want.isinf()])
     # (one rounding to bfloat16; numbers below 2^-126 may be zero)
     assert bool(((got - want).abs()[fine] <= 2.0 ** -8 * want.abs()[fine] + 2.0 ** -126).all())
+
+
+@pytest.mark.parametrize("tile", [64, 130, 129, 131, 132, 133])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", "clamped"])
+def test_gates_as_in_the_few_row_kernel(ops, tile, activation):      # noqa: F811
+    """The same function of the same sums, to the bit: gates and up values of one term each."""
+    bf, m = torch.bfloat16, 520
+    gen = torch.Generator().manual_seed(8)
+    x = torch.zeros(m, 64, dtype=bf)
+    x[:, 0] = torch.linspace(-100.0, 100.0, m).to(bf)
+    x[:, 1] = torch.randn(m, generator=gen).to(bf)
+    w = torch.zeros(32, 64, dtype=bf)
+    w[:16, 0] = (0.05 + 0.95 * torch.rand(16, generator=gen)).to(bf)
+    w[0, 0] = 0.879                      # (gates of the size at which one over the denominator is no normal number)
+    w[16:, 1] = torch.randn(16, generator=gen).to(bf)
+    constants = (7.0, 1.7, 1.0) if activation == "clamped" else None
+    dx, dw = x.to(DEV), ops.prepare_weight(w.to(DEV))
+    got, want = torch.empty(m, 16, dtype=bf, device=DEV), torch.empty(m, 16, dtype=bf, device=DEV)
+    with ops.debug.force(gemm_tile=tile):
+        ops.linear_swiglu(dx, dw, got, activation, constants)
+    for r in range(0, m, 8):      # (so few rows take the other kernel)
+        ops.linear_swiglu(dx[r:r + 8], dw, want[r:r + 8], activation, constants)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
