@@ -745,7 +745,7 @@ __device__ __forceinline__ void attention_tile(const AttnArgs& a, const int xblk
       float den = 0.f;
 #pragma unroll
       for (int w = 0; w < DECODE_WAVES; ++w) {
-        const float wt = mw[w] == NEG_INF ? 0.f : fast_exp2(mw[w] - mmax);
+        const float wt = mw[w] == NEG_INF ? 0.f : exp2f(mw[w] - mmax);
         num += wt * ow[w];
         den += wt * lw[w];
       }
