@@ -116,6 +116,7 @@ struct SkinnyArgs {
   int steps;           // steps of the inner size
   int group_steps;     // ... of a group of K
   int wave_steps;      // ... of a wave
+  int last_wave_steps; // ... of a wave of the last group that has any, which may be shorter
   int wpr_shift;       // log2 of the waves that share a staged row
 };
 
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   extern __shared__ __attribute__((aligned(16))) float smem[];
   // (the arguments that the first loads need come in one trip, not in one per branch that leads to them)
   asm volatile("" :: "s"(a.tiles), "s"(a.nsb), "s"(a.threads), "s"(a.nsb_inv), "s"(a.steps), "s"(a.group_steps),
-               "s"(a.wave_steps), "s"(a.wpr_shift), "s"(a.M), "s"(a.K), "s"(a.x), "s"(a.W), "s"(a.norm_w), "s"(a.pend_splits), "s"(a.norm_w_bf16));
+               "s"(a.wave_steps), "s"(EPI == SK_PART ? a.last_wave_steps : a.wave_steps), "s"(a.wpr_shift), "s"(a.M), "s"(a.K), "s"(a.x), "s"(a.W), "s"(a.norm_w), "s"(a.pend_splits), "s"(a.norm_w_bf16));
   // Rows in tiles of 16 MB: a block sees its tile as if it were the whole product,
   // through pointers moved to the tile's first row.  The tiles of one set of columns
   // read the same part of W: they get block numbers that are equal modulo 8 (the
@@ -302,8 +303,9 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
   const uint32_t wlane = PACKED ? lane * 16 : ((uint32_t)min(c, a.N - 1 - wstrip * 16) * K + g * S::PER) * 4;
   // this block's K steps (all of them, or its group's share), split over its waves
   const int g_begin = ksp * a.group_steps, g_end = min(steps, g_begin + a.group_steps);
-  const int s_begin = g_begin + ks * a.wave_steps;
-  const int s_end = min(g_end, s_begin + a.wave_steps);
+  const int portion = EPI == SK_PART && g_begin + a.group_steps > steps ? a.last_wave_steps : a.wave_steps;
+  const int s_begin = g_begin + ks * portion;
+  const int s_end = min(g_end, s_begin + portion);
   const Frag zero = {};
   const floatx4 fzero = {0.f, 0.f, 0.f, 0.f};
 
@@ -1011,6 +1013,7 @@ extern "C" int llmlab_skinny_linear(const void* x, int norm, const int* x_rows, 
   a.steps = (K + 64 / width - 1) / (64 / width);       // (64 bytes of a row a step)
   a.group_steps = (a.steps + ksplit - 1) / ksplit;
   a.wave_steps = (a.group_steps + shape.kw - 1) / shape.kw;
+  a.last_wave_steps = (a.steps % a.group_steps + shape.kw - 1) / shape.kw;
   a.wpr_shift = 0;
   while ((2 << a.wpr_shift) * tile_rows <= shape.nsb * shape.kw) ++a.wpr_shift;
   a.act = act;

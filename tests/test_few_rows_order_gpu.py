@@ -48,3 +48,22 @@ def test_owed_pieces_of_any_number(ops, emu, dtype, m, splits):      # noqa: F81
         ops.linear(x.to(DEV), ops.prepare_weight(w.to(DEV)), out, bias.to(DEV))
         emu.linear(x, w, want_o, bias)
         close(out, want_o, dtype, "bias", want_o.float().abs().max().item())
+
+
+@pytest.mark.parametrize("splits,waves,steps,large", [(3, 3, 20, 1), (6, 8, 97, 1), (2, 4, 17, 1), (2, 2, 13, 2)])
+def test_a_shorter_last_group_is_shared_out_evenly(ops, splits, waves, steps, large):      # noqa: F811
+    """The inner size in groups of steps, the last one shorter: its steps, too, go to the waves in equal portions.  One
+    number a step: a large one, one half a unit of its last place, and the large one's negative; the second is lost
+    where it meets the first in one wave and kept where it meets the third there."""
+    group = -(-steps // splits)
+    rest = steps - (splits - 1) * group
+    portion = -(-rest // waves)
+    assert 0 < rest < group and portion < -(-group // waves) and portion == large + 1
+    k, n = 32 * steps, 32
+    w, x = torch.zeros(n, k, dtype=torch.bfloat16), torch.ones(3, k, dtype=torch.bfloat16)
+    first = (splits - 1) * group
+    w[:, 32 * (first + large)], w[:, 32 * (first + large + 1)], w[:, 32 * (first + large + 2)] = 2.0 ** 24, 1.0, -2.0 ** 24
+    parts = torch.full((splits, 3, n), float("nan"), device=DEV)
+    with ops.debug.force(skinny_shape=(1, waves, 0, 1)):
+        ops.linear_partials(x.to(DEV), ops.prepare_weight(w.to(DEV)), parts, splits)
+    assert bool((parts[:-1] == 0).all()) and bool((parts[-1] == 1.0).all())
