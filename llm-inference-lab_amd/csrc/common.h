@@ -103,6 +103,27 @@ __device__ __forceinline__ float full_wave_max(float v) {
 __device__ __forceinline__ float lane_value(float v, int from) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), from));
 }
+// The sums over the wave of N numbers a lane, each to the bit what full_wave_sum gives, number k's in lane
+// full_wave_place(k).  A step between the halves of the wave (between rows of 16 lanes) leaves two sums' halves in one
+// register, so that two or four sums take the steps that follow together.
+template <int N>
+__device__ __forceinline__ float full_wave_sums(const float (&v)[N]) {
+  static_assert(N == 1 || N == 2 || N == 4, "sums");
+  auto halves = [](float a, float b) {      // lanes 0-31: of a, 32-63: of b
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  };
+  const float a = halves(v[0], v[N > 1]), b = N == 4 ? halves(v[N - 2], v[N - 1]) : a;
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  float s = __uint_as_float(r[0]) + __uint_as_float(r[1]);      // rows 0 and 2: of a, 1 and 3: of b
+  s += dpp_move<0x128>(s);
+  s += dpp_move<0x124>(s);
+  s += dpp_move<0x4E>(s);
+  return s + dpp_move<0xB1>(s);
+}
+__device__ __forceinline__ constexpr int full_wave_place(int k) {
+  return (k & 1) * 32 + (k >> 1) * 16;
+}
 
 // Sum over a block of up to 1024 threads; every thread gets the result.
 // `red` is shared memory of at least 17 floats.

@@ -66,7 +66,7 @@ extern "C" int llmlab_embed(const void* table, int dtype, int packed, const int*
 // W neighbouring weights as they lie in memory, bfloat16 or float32, and their values.  Two loads of 8 bytes without a
 // branch (of the same 8 where the weights are bfloat16): converted on the way, each group was waited for
 // before the next, and the row, were asked for (48 rows of 896, back to back in a graph, 2.7 us so and 2.1 now; 2,048 rows
-// 4.1 and 3.1).
+// 4.2 and 3.4).
 template <int W>
 struct RawWeights {
   uint32_t u[W];
@@ -104,11 +104,15 @@ __device__ __forceinline__ RawWeights<W> ask_for_weights(const void* w, int w_bf
 // memory; what lies beyond is read again after the reduction.  VEC: groups of four
 // (hidden % 4 == 0 and 16-byte aligned rows).  All loads of a trip are unconditional (past the row's end its last
 // group again, not counted): under a branch each would be waited for before the next is asked for.
-template <typename T, bool VEC, int KEEP, int G>
+// The order of a row's sum does not depend on how many threads hold it: SHARE threads of a block of SHARE * blockDim.x are
+// one here, with a sum of squares for each (which meet as the waves of that block would: within 64 neighbours,
+// then one after the other).  What that block is: llmlab_rmsnorm.
+template <typename T, bool VEC, int KEEP, int SHARE, int G>
 __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w, int w_bf16,
                                float eps, T* __restrict__ out, const int* __restrict__ rows,
                                int hidden, const float* __restrict__ pend, int splits, size_t pend_stride) {
   constexpr int W = VEC ? 4 : 1;
+  static_assert(KEEP % SHARE == 0, "whole rounds");
   __shared__ float red[16];
   const int i = blockIdx.x;
   const int r = rows ? rows[i] : i;
@@ -160,7 +164,19 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w
   };
   Group keep[KEEP];
   RawWeights<W> wk[KEEP];
-  float ss = 0.f;
+  float ss[SHARE];
+#pragma unroll
+  for (int k = 0; k < SHARE; ++k) ss[k] = 0.f;
+  // (a sum's first group: the second square rounded by itself, the others into the sum; fixed here, since it would be
+  // the compiler's choice, and another one in each instance)
+  auto squares = [](const Group& g, bool first, float sum) {
+    if constexpr (W == 4) {
+      sum = first ? fmaf(g.v[0], g.v[0], g.v[1] * g.v[1]) : fmaf(g.v[1], g.v[1], fmaf(g.v[0], g.v[0], sum));
+      return fmaf(g.v[3], g.v[3], fmaf(g.v[2], g.v[2], sum));
+    } else {
+      return fmaf(g.v[0], g.v[0], sum);
+    }
+  };
   const int c0 = threadIdx.x * W;
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) wk[j] = weights(min(c0 + j * stride, hidden - W));
@@ -169,25 +185,31 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w
   for (int j = 0; j < KEEP; ++j) {
     const int c = c0 + j * stride;
     if (c < hidden) put_back(c, keep[j]);
-#pragma unroll
-    for (int e = 0; e < W; ++e) ss += c < hidden ? keep[j].v[e] * keep[j].v[e] : 0.f;
+    ss[j % SHARE] = c < hidden ? squares(keep[j], j < SHARE, ss[j % SHARE]) : ss[j % SHARE];
   }
-  for (int c = c0 + KEEP * stride; c < hidden; c += stride) {
-    Group g;
-    fetch(std::integral_constant<int, 1>{}, c, &g);
-    put_back(c, g);
-#pragma unroll
-    for (int e = 0; e < W; ++e) ss += g.v[e] * g.v[e];
-  }
-  ss = full_wave_sum(ss);            // (whole waves, all of whose threads come here)
+  if constexpr (SHARE == 1)          // (else the groups held are all)
+    for (int c = c0 + KEEP * stride; c < hidden; c += stride) {
+      Group g;
+      fetch(std::integral_constant<int, 1>{}, c, &g);
+      put_back(c, g);
+      ss[0] = squares(g, false, ss[0]);
+    }
   const int waves = blockDim.x >> 6;
+  const float sums = full_wave_sums(ss);      // (whole waves, all of whose threads come here)
+  float total;
   if (waves > 1) {                   // (a barrier; below a thread reads back only what it wrote itself)
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+#pragma unroll
+    for (int k = 0; k < SHARE; ++k)
+      if ((threadIdx.x & 63) == full_wave_place(k)) red[k * waves + (threadIdx.x >> 6)] = sums;
     __syncthreads();
-    ss = 0.f;
-    for (int k = 0; k < waves; ++k) ss += red[k];
+    total = 0.f;
+    for (int k = 0; k < waves * SHARE; ++k) total += red[k];
+  } else {
+    total = lane_value(sums, 0);
+#pragma unroll
+    for (int k = 1; k < SHARE; ++k) total += lane_value(sums, full_wave_place(k));
   }
-  const float inv = rsqrtf(ss / (float)hidden + eps);
+  const float inv = rsqrtf(total / (float)hidden + eps);
   T* dst = out + (size_t)i * hidden;
   auto put = [&](int c, const Group& g, const RawWeights<W>& wg) {
     typedef T Out __attribute__((ext_vector_type(W)));
@@ -199,7 +221,8 @@ __global__ void rmsnorm_kernel(float* __restrict__ x, const void* __restrict__ w
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
     if (c0 + j * stride < hidden) put(c0 + j * stride, keep[j], wk[j]);
-  for (int c = c0 + KEEP * stride; c < hidden; c += stride) put(c, get(src + c), weights(c));
+  if constexpr (SHARE == 1)
+    for (int c = c0 + KEEP * stride; c < hidden; c += stride) put(c, get(src + c), weights(c));
 }
 
 extern "C" int llmlab_rmsnorm(float* x, const void* w, int w_dtype, float eps, void* out,
@@ -213,28 +236,47 @@ extern "C" int llmlab_rmsnorm(float* x, const void* w, int w_dtype, float eps, v
                    (((uintptr_t)x | (uintptr_t)pend | (uintptr_t)out) & 15) == 0 &&
                    ((uintptr_t)w & (w_dtype == DT_BF16 ? 7 : 15)) == 0;
   const int groups = hidden / (vec ? 4 : 1);
-  // Few rows are bound by latency (and up to 1,024 narrow ones): a row is spread over as many threads as it has groups,
-  // so that every thread's loads (its numbers and the pieces owed to them) are one round.  Many rows: four groups a thread
-  // (two with many pieces: registers), a row of 1,024 and less a wave of its own without a barrier.  (2,367 rows of 3584
-  // 15.3 -> 11.6 us by that and by loads that travel together; 512 of 896 4.0 a group a thread, 4.4 four.)
-  const int keep = n_out <= 128 || (n_out <= 1024 && groups <= 256) ? 1 : splits > 2 ? 2 : 4;
-  const int threads = min(1024, max(1, (groups + 64 * keep - 1) / (64 * keep)) * 64);
+  // The block whose order a row's sum has: 256 threads (512 from 8,192 numbers on), for few rows as many as the row has
+  // groups of four, up to 1,024; and the groups that one of its threads then takes.
+  int order = hidden >= 8192 ? 512 : 256;
+  if (n_out <= 128)
+    while (order < 1024 && order * 4 < hidden) order *= 2;
+  const int rounds = (groups + order - 1) / order;
+  // Few rows are bound by latency (and up to 1,024 narrow ones): a thread a group, so that every thread's loads (its
+  // numbers and the pieces owed to them) are one round; what 1,024 threads do not hold is read again (8 rows of 5120
+  // in eight pieces 4.0 us so, 4.8 with two groups a thread).  Many rows: four groups a thread (two with many pieces:
+  // registers), a row of 1,024 and less a wave of its own without a barrier.  (Back to back, before and now: 2,048 rows of 896
+  // 4.2 and 3.4 us, in eight pieces 14.2 and 12.5; 2,367 of 3584 14.3 and 9.4; 512 of 5120 5.8 and 4.3.)
+  const bool few = n_out <= 128 || (n_out <= 1024 && groups <= 256);
+  int keep = vec && few ? 1 : rounds > 2 ? 4 : rounds, share = 1;
+  if (vec && !few && rounds <= 2) {
+    keep = splits > 2 ? 2 : 4;
+    share = keep / rounds;
+  }
+  const int threads = rounds == 1 && share == 1 ? (groups + 63) / 64 * 64 : order / share;
   dim3 grid(n_out), block(threads);
-#define LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, G)                                                               \
-  hipLaunchKernelGGL((rmsnorm_kernel<T, VEC, KEEP, G>), grid, block, 0, stream, x, w, w_dtype == DT_BF16, eps, \
+#define LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, SHARE, G)                                                        \
+  hipLaunchKernelGGL((rmsnorm_kernel<T, VEC, KEEP, SHARE, G>), grid, block, 0, stream, x, w, w_dtype == DT_BF16, eps, \
                      (T*)out, rows, hidden, pend, splits, pend_stride)
+#define LLMLAB_RMSNORM_PIECES(T, VEC, KEEP, SHARE, MANY)                                                   \
+  do {                                                                                                     \
+    if (splits == 0) LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, SHARE, 0);                                          \
+    else if (splits <= 2) LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, SHARE, 2);                                     \
+    else LLMLAB_RMSNORM_KEEP(T, VEC, KEEP, SHARE, MANY);                                                   \
+  } while (0)
 #define LLMLAB_RMSNORM(T, VEC)                                                                             \
   do {                                                                                                     \
-    if (keep == 4 && splits == 0) LLMLAB_RMSNORM_KEEP(T, VEC, 4, 0);                                       \
-    else if (keep == 4) LLMLAB_RMSNORM_KEEP(T, VEC, 4, 2);                                                 \
-    else if (keep == 2) LLMLAB_RMSNORM_KEEP(T, VEC, 2, 4);                                                 \
-    else if (splits > 2) LLMLAB_RMSNORM_KEEP(T, VEC, 1, 4);                                                \
-    else if (splits > 0) LLMLAB_RMSNORM_KEEP(T, VEC, 1, 2);                                                \
-    else LLMLAB_RMSNORM_KEEP(T, VEC, 1, 0);                                                                \
+    if (VEC && keep == 4 && share == 4) LLMLAB_RMSNORM_PIECES(T, true, 4, 4, 2);                           \
+    else if (VEC && keep == 4 && share == 2) LLMLAB_RMSNORM_PIECES(T, true, 4, 2, 2);                      \
+    else if (VEC && keep == 2 && share == 2) LLMLAB_RMSNORM_KEEP(T, true, 2, 2, 4);                        \
+    else if (keep == 4) LLMLAB_RMSNORM_PIECES(T, VEC, 4, 1, 2);                                            \
+    else if (keep == 2) LLMLAB_RMSNORM_PIECES(T, VEC, 2, 1, 4);                                            \
+    else LLMLAB_RMSNORM_PIECES(T, VEC, 1, 1, 4);                                                           \
   } while (0)
   if (out_dtype == DT_BF16) { if (vec) LLMLAB_RMSNORM(bf16_t, true); else LLMLAB_RMSNORM(bf16_t, false); }
   else                      { if (vec) LLMLAB_RMSNORM(float, true);  else LLMLAB_RMSNORM(float, false); }
 #undef LLMLAB_RMSNORM_KEEP
+#undef LLMLAB_RMSNORM_PIECES
 #undef LLMLAB_RMSNORM
   LLMLAB_LAUNCH_CHECK("rmsnorm");
   return 0;

@@ -29,3 +29,20 @@ def test_against_64_bits(ops, dtype, rows, hidden, splits):      # noqa: F811
         got = torch.empty(len(picked), hidden, dtype=dtype, device=DEV)
         ops.rmsnorm(got_x, w.to(DEV), 1e-6, got, picked.to(DEV))
         close(got, want[picked.long()], dtype, "gathered", want.abs().max().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [4, 33, 64, 260, 512, 772, 896, 1024])
+@pytest.mark.parametrize("splits", [0, 1, 2, 3, 8])
+def test_a_row_is_the_same_among_any_number_of_rows(ops, dtype, hidden, splits):      # noqa: F811
+    """Rows of up to 1,024 numbers: however a launch spreads them, a row's sum meets in one order."""
+    x, w = rnd((2000, hidden), torch.float32, 1), (1 + 0.1 * rnd((hidden,), torch.float32, 2)).to(dtype).to(DEV)
+    pieces = rnd((max(splits, 1), 2000, hidden), torch.float32, 3)
+    got = {}
+    for rows in (1, 100, 129, 1024, 1025, 2000):
+        out = torch.empty(rows, hidden, dtype=dtype, device=DEV)
+        ops.rmsnorm(x[:rows].to(DEV), w, 1e-6, out,
+                    pending=PendingSums(pieces[:, :rows].contiguous().to(DEV), splits) if splits else None)
+        got[rows] = out
+    for rows, out in got.items():
+        assert torch.equal(out, got[2000][:rows]), f"{rows} rows"
