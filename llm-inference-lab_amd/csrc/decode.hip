@@ -146,6 +146,14 @@ __device__ __forceinline__ float sk_pair(float g, float u, const SkinnyArgs& a) 
   return g / (1.f + __expf(-a.slope * g)) * (fminf(fmaxf(u, -a.limit), a.limit) + a.shift);
 }
 
+// A sum of squares and two more, `alone` rounded by itself before the other is added.  The roundings are fixed here: left to
+// the compiler they differ between the places it is inlined at, and a row's norm with the instance that takes it.
+__device__ __forceinline__ float sk_add_squares(float sum, float other, float alone) {
+#pragma clang fp contract(off)
+  const float square = alone * alone;
+  return sum + fmaf(other, other, square);
+}
+
 // What a step of the inner size is: 16 rows of W by 64 bytes, 16 bytes a lane.  bfloat16: 32 numbers, one
 // matrix instruction.  float32: 16 numbers, four (lane (c, g) holds the numbers 4 g .. 4 g + 3 of row c; instruction
 // e contracts the e-th of all four groups, the same four numbers of both operands), 32-bit products and sums in
@@ -440,7 +448,10 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
         }
         if constexpr (PIECES) load_pieces(base, 0);
       };
-      auto store = [&](int base, T* dst, float& ssq) {
+      // (n: how many chunks of its part a lane has behind it.  The first of every four chunks without pieces rounds the
+      // squares of its lower four numbers by themselves, all others those of their upper four, whatever U is; a part taken
+      // one by one without pieces is one chunk)
+      auto store = [&](int base, T* dst, float& ssq, int n) {
         if constexpr (PIECES) {
           for (int sp0 = 0; sp0 < a.pend_splits; sp0 += 4) {      // in their order
             if (sp0 > 0) load_pieces(base, sp0);
@@ -471,9 +482,10 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
               }
             }
             Sk8<T> av;
+            const bool p_alone = !PIECES && u == 0 && (U != 2 || (n & 2) == 0);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              ssq += p[u][j] * p[u][j] + q[u][j] * q[u][j];
+              ssq = p_alone ? sk_add_squares(ssq, q[u][j], p[u][j]) : sk_add_squares(ssq, p[u][j], q[u][j]);
               av.set(j, p[u][j] * wv[j]);
               av.set(4 + j, q[u][j] * wv[4 + j]);
             }
@@ -497,11 +509,11 @@ __global__ __launch_bounds__(MB >= 4 ? 512 : 1024) void skinny_block_kernel(Skin
       float ssq = 0.f;
       int base = (unit & (wpr - 1)) * 64;
       T* dst = As + (size_t)(unit >> wpr_shift) * lda;
-      store(base, dst, ssq);      // (by itself: in the loop below the loads of W behind these would be waited for, too)
-      for (;;) {
-        for (base += U * stride; base < chunks; base += U * stride) {
+      store(base, dst, ssq, 0);      // (by itself: in the loop below the loads of W behind these would be waited for, too)
+      for (int n = U;; n = 0) {
+        for (base += U * stride; base < chunks; base += U * stride, n += U) {
           load(base);
-          store(base, dst, ssq);
+          store(base, dst, ssq, n);
         }
         if constexpr (NORM) {
           ssq = full_wave_sum(ssq);

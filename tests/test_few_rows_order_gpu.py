@@ -67,3 +67,19 @@ def test_a_shorter_last_group_is_shared_out_evenly(ops, splits, waves, steps, la
     with ops.debug.force(skinny_shape=(1, waves, 0, 1)):
         ops.linear_partials(x.to(DEV), ops.prepare_weight(w.to(DEV)), parts, splits)
     assert bool((parts[:-1] == 0).all()) and bool((parts[-1] == 1.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [96, 896, 2048, 3584])
+def test_a_norm_of_weights_in_either_type(ops, dtype, n):      # noqa: F811
+    """Weights of one value in bfloat16 and in float32 are read by instances of their own: a row's squares meet in one
+    order, to the bit."""
+    weight, head = (1 + 0.1 * rnd((n,), torch.float32, 6)).bfloat16().to(DEV), ops.prepare_weight(rnd((48, n), dtype, 7, 0.1).to(DEV))
+    for m in range(1, 65):
+        if not ops.can_fuse(m, dtype, n):
+            continue
+        x = rnd((m, n), torch.float32, m).to(DEV)
+        narrow, wide = torch.empty(m, 48, device=DEV), torch.empty(m, 48, device=DEV)
+        ops.fused_norm_logits(x, None, weight, 1e-6, head, narrow)
+        ops.fused_norm_logits(x, None, weight.float(), 1e-6, head, wide)
+        assert torch.equal(narrow, wide), f"{m} rows"
