@@ -1141,11 +1141,12 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // and 1.25e-6, 6e-7 in three pieces).
 //
 // Where all numbers of W are bfloat16 numbers, as in checkpoints that were trained and kept in bfloat16, m_w and l_w are
-// zero and with them three of the six products.  A block takes W for such until it meets another number: the first step
-// tells in most cases and the block starts over with all parts, what a later one holds is known at the end and the block
-// takes its outputs again.  Nothing is kept between calls, and both ways give the same sums to the bit (the
+// zero and with them three of the six products.  A block takes W for such until it meets another number, and all parts from
+// that step on: a thread that puts such a number down leaves its step in LDS, where every wave looks before it multiplies a
+// step.  Nothing is kept between calls, and both ways give the same sums to the bit (the
 // terms left out are zeros).  (Relative error of a prompt's logits, 1,531 tokens of the 0.5B shape, mean of eight seeds:
-// 2.13e-6; 2.63e-6 before the small products had sums of their own.)
+// 2.13e-6; 2.63e-6 before the small products had sums of their own.  1,531 rows of 9728 x 896 with such a number in the last
+// step 95 us, without one 91, of such numbers 146; when the block found out at the end and started over 209.)
 //
 // BM x BN outputs per block of WM x WN waves, steps of 32 of the inner size.  A thread
 // fetches eight numbers of a row as they lie in memory, two steps ahead (four neighbouring lanes 64 consecutive bytes: with
@@ -1161,9 +1162,9 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // value of an output.
 //
 // What bounds it: LDS (128 x 256, one part: 128 KB of reads and 40 of writes a step, 1,850 clocks at the rates of LDS,
-// 1,630 of matrix instructions).  1,531 rows of 9728 x 896 with one / three parts 105 / 158 us (255 / 169 TFLOP/s of
-// 32-bit products; 187 / 184 before these tiles and loads), of 896 x 4864 in five pieces 57 / 87 (in three: 88 / 90), of
-// 1152 x 896 23 / 33 (36), 4,000 of 9728 x 896 250 / 383 (428 / 459).
+// 1,630 of matrix instructions).  Back to back, with one / three parts (by one loop for all numbers, whose loads had
+// neighbouring lanes in different rows): 1,531 rows of 9728 x 896 91 / 146 us (166 / 174), 293 / 183 TFLOP/s of 32-bit products; of 896 x 4864 in three
+// pieces 57 / 78 (77 / 80), of 1152 x 896 25 / 35 (38 / 38), 4,000 of 9728 x 896 227 / 371 (415 / 447).
 //
 // Two ranges have no such parts.  Of numbers below 2^-110 the last bits fall under bfloat16's smallest number, 2^-133
 // (the sum of the parts is then off by 2.4e-7 of the number at 2^-112, 9.5e-4 at 2^-124): it shows in what the third
@@ -1185,6 +1186,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
   constexpr int STAGE = (BM + BN) / 16 * 3072;
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
   __shared__ int s_again;
+  __shared__ int s_other;      // where the first step begins that holds a number of W of more than one part, of those put down
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wn = wave / WM;
   int bx = blockIdx.x, by = blockIdx.y;
@@ -1206,13 +1208,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
     e.out = (float*)e.out + (size_t)blockIdx.z * e.part_stride;
     if (blockIdx.z > 0) e.bias = nullptr;
   }
-  if (tid == 0) s_again = 0;
+  if (tid == 0) {
+    s_again = 0;
+    s_other = 0x7fffffff;
+  }
 
-  floatx4 acc[TN][TM];
+  // (the small products in sums of their own where there are registers for them: a sum is rounded at its own size, once
+  // a step and not three or six times; a product of 1,531 rows of 896 x 896 then is 1.9e-7 off 64 bits, 3.1e-7 in one sum)
+  constexpr bool APART = TN * TM <= 8;
+  floatx4 acc[TN][TM], small[APART ? TN : 1][APART ? TM : 1];
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TM; ++i) {
+      acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (APART) small[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
 
   // piece x of a thread: row (wave + NW x) * 16 + sr of the tile, numbers 4 sg .. and 16 + 4 sg .. of the step (four
   // neighbouring lanes read 64 consecutive bytes)
@@ -1261,7 +1272,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
   auto place = [](int r, int q) { return (q * 16 + (r ^ (2 * q))) * 16; };
   const int mine = place(c, g);
   unsigned rest = 0;             // of the numbers of x, what the third part is rounded from
-  unsigned rest_w = 0;           // of the numbers of W, what one bfloat16 number leaves out
   auto split = [&](const floatx4 (&v)[2], char* to, int k0) {      // (of x the numbers from k0 on; W: k0 < 0)
     uint32_t part[3][4];
     float num[8];
@@ -1291,28 +1301,32 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
       *(bf16x8*)(to + p * 1024) = __builtin_bit_cast(bf16x8, floatx4{__uint_as_float(part[p][0]), __uint_as_float(part[p][1]),
                                                                      __uint_as_float(part[p][2]), __uint_as_float(part[p][3])});
   };
-  auto upper_halves = [&](const floatx4 (&v)[2], char* to) {      // numbers that are bfloat16 numbers, if rest_w says so
-    uint32_t h[4];
+  auto upper_halves = [&](const floatx4 (&v)[2], char* to) {      // and what they leave out, zero where bfloat16 holds the numbers
+    uint32_t h[4], out = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const uint32_t a = __float_as_uint(v[q >> 1][(q & 1) * 2]), b = __float_as_uint(v[q >> 1][(q & 1) * 2 + 1]);
       h[q] = __builtin_amdgcn_perm(b, a, 0x07060302);
-      rest_w |= a | b;
+      out |= a | b;
     }
     *(bf16x8*)to = __builtin_bit_cast(bf16x8, floatx4{__uint_as_float(h[0]), __uint_as_float(h[1]), __uint_as_float(h[2]),
                                                       __uint_as_float(h[3])});
+    return out & 0xffffu;
   };
-  // ONE: one part of every number of W is taken, else three
+  // The step from k0 on to `stage`.  ONE: one part of every number of W is taken, else three
   auto stash = [&](auto one, const Pieces& r, int k0, int stage) {
     constexpr bool ONE = decltype(one)::value;
     char* to = smem + stage * STAGE + place(sr, sg);
+    uint32_t other = 0;
 #pragma unroll
     for (int x = 0; x < LA; ++x) split(r.a[x], to + (wave + NW * x) * 3072, k0);
 #pragma unroll
     for (int x = 0; x < LB; ++x) {
-      if constexpr (ONE) upper_halves(r.b[x], to + BM / 16 * 3072 + (wave + NW * x) * 1024);
+      if constexpr (ONE) other |= upper_halves(r.b[x], to + BM / 16 * 3072 + (wave + NW * x) * 1024);
       else split(r.b[x], to + (BM / 16 + wave + NW * x) * 3072, -BK);
     }
+    if constexpr (ONE)
+      if (__ballot(other != 0) != 0 && other != 0) atomicMin(&s_other, k0);      // (no branch by lanes where there is none)
   };
   // the parts of step `t` as a wave multiplies them, and their products, the small ones first
   // (ONE: the order of the general sum, without its terms that are zero)
@@ -1327,10 +1341,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
 #pragma unroll
     for (int j = 0; j < TN; ++j) wf[j] = *(const bf16x8*)(ws + ((wn * TN + j) * PW + p) * 1024);
   };
-  // (the small products in sums of their own where there are registers for them: a sum is rounded at its own size, once
-  // a step and not three or six times; a product of 1,531 rows of 896 x 896 then is 1.9e-7 off 64 bits, 3.1e-7 in one sum)
-  constexpr bool APART = TN * TM <= 8;
-  floatx4 small[APART ? TN : 1][APART ? TM : 1];
   auto products = [&](auto large, const bf16x8 (&wf)[TN], const bf16x8 (&xf)[TM]) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
@@ -1349,31 +1359,26 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // With one part of W: whether that was enough.  The first step tells at once; what a later one tells is
-  // known at the end.
-  const int steps = (k_end - k_begin + BK - 1) / BK;
-  auto walk = [&](auto one) -> bool {
+  // The steps from k0 on; with one part of W up to the first that holds a number of more.  Returns where it left off.
+  auto walk = [&](auto one, int k0) -> int {
     constexpr bool ONE = decltype(one)::value;
     constexpr int PW = ONE ? 1 : 3;
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (APART) small[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-      }
+    // (what a wave finds in s_other in its step from k0 on: every piece of that step was put down before the barrier it came
+    // through; what others put down meanwhile is of a later step)
+    // (a relaxed atomic load: of a volatile one each would be waited for at once)
+    auto other_from = [&]() {
+      return ONE ? __hip_atomic_load(&s_other, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0x7fffffff;
+    };
+    auto before = [&](int other) { return ONE && __builtin_amdgcn_readfirstlane(other) <= k0; };
     Pieces r0, r1;
-    fetch(r0, k_begin);
-    fetch(r1, k_begin + BK);
-    stash(one, r0, k_begin, 0);
-    fetch(r0, k_begin + 2 * BK);
-    if constexpr (ONE) {
-      if (__syncthreads_or(rest_w & 0xffffu)) return false;
-    } else {
-      __syncthreads();
-    }
-    // Step t lies in stage t % 2; it is put there during step t - 1, from registers that were asked for two steps
-    // before that.
+    fetch(r0, k0);
+    fetch(r1, k0 + BK);
+    if constexpr (ONE) barrier();      // (s_other is set)
+    stash(one, r0, k0, 0);
+    fetch(r0, k0 + 2 * BK);
+    __syncthreads();
+    if (before(other_from())) return k0;
+    // A step is put down during the one before, from registers that were asked for two steps before that.
     bf16x8 xf[3][TM], wf[PW][TN];
     auto read = [&](int stage) {
 #pragma unroll
@@ -1395,13 +1400,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
       }
       products(std::true_type{}, wf[0], xf[0]);  // h_w h_x
     };
+    // (r: the next step's numbers)
     if constexpr (GROUPS && (ONE || TN > 2)) {
       if (wave >= NW / 2) barrier();       // the second group runs half a step behind
-      auto step = [&](int t, Pieces& r) {  // (r: step t + 1)
-        read(t & 1);
-        stash(one, r, k_begin + (t + 1) * BK, (t + 1) & 1);
+      auto step = [&](int stage, Pieces& r) -> bool {
+        const int other = other_from();
+        read(stage);
+        stash(one, r, k0 + BK, stage ^ 1);
         barrier();
-        fetch(r, k_begin + (t + 3) * BK);
+        if (before(other)) return false;
+        fetch(r, k0 + 3 * BK);
         multiply();
         // (the loads and what they take to address between the matrix instructions)
 #pragma unroll
@@ -1411,36 +1419,38 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
           __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);     // a load
         }
         barrier();
+        k0 += BK;
+        return k0 < k_end;
       };
-      for (int t = 0; t < steps; t += 2) {
-        step(t, r1);
-        if (t + 1 >= steps) break;
-        step(t + 1, r0);
-      }
+      // (both groups leave at the same step, and the first waits for the second's reads of it)
+      while (step(0, r1) && step(1, r0)) {}
       if (wave < NW / 2) barrier();
     } else {
-      auto step = [&](int t, Pieces& r) {
-        read(t & 1);
-        stash(one, r, k_begin + (t + 1) * BK, (t + 1) & 1);
+      auto step = [&](int stage, Pieces& r) -> bool {
+        const int other = other_from();
+        read(stage);
+        if (before(other)) return false;
+        stash(one, r, k0 + BK, stage ^ 1);
         multiply();
-        fetch(r, k_begin + (t + 3) * BK);
+        fetch(r, k0 + 3 * BK);
         __syncthreads();
+        k0 += BK;
+        return k0 < k_end;
       };
-      for (int t = 0; t < steps; t += 2) {
-        step(t, r1);
-        if (t + 1 >= steps) break;
-        step(t + 1, r0);
-      }
+      while (step(0, r1) && step(1, r0)) {}
     }
-    if constexpr (APART) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) acc[j][i] += small[j][i];
-    }
-    return !ONE || !__syncthreads_or(rest_w & 0xffffu);
+    return k0;
   };
-  if (steps > 0 && !walk(std::true_type{})) walk(std::false_type{});
+  if (k_begin < k_end) {
+    const int left_off = walk(std::true_type{}, k_begin);
+    if (left_off < k_end) walk(std::false_type{}, left_off);
+  }
+  if constexpr (APART) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[j][i] += small[j][i];
+  }
   bool again = (rest & 0xffffu) != 0;
 #pragma unroll
   for (int j = 0; j < TN; ++j)

@@ -156,3 +156,51 @@ def test_products_of_many_steps_of_one_part_and_three_agree(ops):
             ops.linear_logits(x, ops.prepare_weight(w), one)
             ops.linear_logits(x, ops.prepare_weight(mixed), three)
             assert torch.equal(one, three[:, places]), f"tile {tile}"
+
+
+@pytest.mark.parametrize("tile", [64, 128, 131])
+@pytest.mark.parametrize("k", [32, 160, 330, 352])
+def test_a_number_of_three_parts_in_any_step(ops, tile, k):
+    """From the step on that holds the first such number a block takes all parts; its sums are those of a block that
+    takes all parts from the start, to the bit."""
+    m, n = 140, 300
+    x, w = rnd((m, k), 25).to(DEV), rnd((n, k), 26).bfloat16().float()
+    rows = [5, 150, 290]      # (one a block of every tile at least)
+    rest = torch.tensor([r for r in range(n) if r not in [b + 1 for b in range(0, n, 64)]], device=DEV)
+    general = w.clone()
+    general[[b + 1 for b in range(0, n, 64)], 0] = 1.0 + 2.0 ** -20      # (a row of every block, left out below)
+    with ops.debug.force(gemm_tile=tile):
+        for at in range(0, k, 32):
+            for row in rows:
+                late, first = w.clone(), general.clone()
+                late[row, min(at + 7, k - 1)] = first[row, min(at + 7, k - 1)] = 1.0 + 2.0 ** -19
+                got, want = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+                ops.linear_logits(x, ops.prepare_weight(late.to(DEV)), got)
+                ops.linear_logits(x, ops.prepare_weight(first.to(DEV)), want)
+                assert torch.equal(got[:, rest], want[:, rest]), f"step {at // 32}, row {row}"
+
+
+@pytest.mark.parametrize("tile", [64, 128, 131])
+def test_a_late_number_of_three_parts_costs_no_second_walk(ops, tile):
+    """A matrix with one such number a block, in the last step, takes little longer than one of such numbers (which
+    takes about as long as a walk by itself; two walks would take 1.6 times as long)."""
+    m, n, k = 1536, 4096, 896
+    x, w = rnd((m, k), 27).to(DEV), rnd((n, k), 28)
+    late = w.bfloat16().float()
+    late[::64, -1] = 1.0 + 2.0 ** -20
+    out = torch.empty(m, n, device=DEV)
+
+    def time(weight):
+        weight, best = ops.prepare_weight(weight.to(DEV)), float("inf")
+        for _ in range(12):
+            marks = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            marks[0].record()
+            for _ in range(10):
+                ops.linear_logits(x, weight, out)
+            marks[1].record()
+            torch.cuda.synchronize()
+            best = min(best, marks[0].elapsed_time(marks[1]))
+        return best
+
+    with ops.debug.force(gemm_tile=tile):
+        assert time(late) < 1.25 * time(w)
