@@ -1871,17 +1871,48 @@ static int one_round_tile(int M, int N, int K, int num_cus) {
 // By an estimate of the time, fitted to a sweep of eight matrices of three model shapes at 65 to 4,096 rows
 // whole and in up to eight pieces, each with W's numbers of one part and of three (948 times; 4 to 9 % rms about the
 // geometric mean of the two, since W's numbers are not known here; the picks lose 0.6 % whole and 2.3 % in pieces to the
-// best of the sweep).  Against the tiles and picks before (64 x 64 and 128 x 128, one loop for all numbers, a load of 16
+// best of the sweep; before the bound below).  Against the tiles and picks before (64 x 64 and 128 x 128, one loop for all numbers, a load of 16
 // rows with neighbouring lanes in different ones) they take 0.60 of the time whole and 0.72 with the fold of their
 // pieces where W has one part, 0.87 and 0.94 where it has three (9 % more at worst, of a product in fewer pieces than
 // before).  A block of the 128 x 128 and 128 x 256 tiles is alone on its unit, rounds are whole; of the 64 x 64 tile
 // three share one, whose first is slow by itself.
-// The 128 x 256 tile, whose small products have no sums of their own, adds at most so many steps where the product may
-// be cut: 7,041 rows of 896 x 4864 whole were 7.4e-7 off 64 bits and a decode step behind such prompts 1.68e-6, in
-// three pieces 4.3e-7 and 1.44e-6 (as before this tile).
+//
+// How many steps a sum may add where the product may be cut: a sum is rounded at its own size once a product and step, so that
+// its error grows as the root of its steps.  The bound is what the estimate of the first kernels gave (64 x 64 and
+// 128 x 128, everything in one sum): the 128 x 256 tile, which adds everything in one sum, holds to it (and to 64 steps: 7,041
+// rows of 896 x 4864 whole were 7.4e-7 off 64 bits and a decode step behind such prompts 1.68e-6, in three pieces 4.3e-7 and
+// 1.44e-6); the others, whose small products have sums of their own and whose error at the same steps is 0.55 of
+// that, may add three times as many.  (Without the bound 4,040 rows of 1536 x 1536 whole 4.2e-7 / 6.0e-7 off 64 bits with one part of
+// W and with three, in two pieces 2.9e-7 / 4.2e-7; 2,312 of 2048 x 2048 4.9e-7 / 7.0e-7 and 3.4e-7 / 4.9e-7; 3,336 of 896 x
+// 4864 by 128 x 128 whole 4.3e-7, in two pieces 3.1e-7, by the first kernel in four 3.7e-7.)
 constexpr int F32_WIDE_STEPS = 64;
+static int f32_sum_steps(int M, int N, int steps, int num_cus, int max_pieces, int min_steps) {
+  int most = steps;
+  double least = 1e30;
+  for (int bm = 64; bm <= 128; bm += 64) {
+    for (int pieces = 1; pieces <= max_pieces; ++pieces) {
+      const int s = (steps + pieces - 1) / pieces;
+      if (pieces > 1 && s < min_steps) break;
+      const double share = (double)((M + bm - 1) / bm) * ((N + bm - 1) / bm) * pieces / num_cus;
+      const double whole = ceil(share - 1e-9);
+      double t = whole * (5.4 + s * (1.31 + 0.12 * (share < 1.0 ? share : 1.0)));
+      if (bm == 64) {
+        const double shared = (share <= 3.0 ? whole : share) * (1.0 + 0.58 * s);
+        t = 2.0 + 0.863 * s;
+        if (shared > t && whole > 1.0) t = shared;
+      }
+      if (pieces > 1) t += pieces * ((double)M * N * 2.2e-6 + 0.3);
+      if (t < least) {
+        least = t;
+        most = s;
+      }
+    }
+  }
+  return most;
+}
 static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int min_steps) {
   const int steps = (K + 31) / 32;
+  const int sum_steps = f32_sum_steps(M, N, steps, num_cus, max_pieces, min_steps);
   F32Plan best{-1, 1};
   double least = 0.0;
   for (const int tile : {TILE_64, TILE_128, TILE_128x256}) {
@@ -1892,11 +1923,13 @@ static F32Plan f32_plan(int M, int N, int K, int num_cus, int max_pieces, int mi
     for (int pieces = 1; pieces <= max_pieces; ++pieces) {
       const int s = (steps + pieces - 1) / pieces;
       if (pieces > 1 && s < min_steps) break;
+      const int most = tile == TILE_128x256 ? (sum_steps < F32_WIDE_STEPS ? sum_steps : F32_WIDE_STEPS) : 3 * sum_steps;
+      const bool finer = pieces < max_pieces && (steps + pieces) / (pieces + 1) >= min_steps;      // (there are more pieces to be had)
+      if (s > most && finer) continue;
       const double share = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * pieces / num_cus;
       const double whole = ceil(share - 1e-9);
       double t;
       if (tile == TILE_128x256) {
-        if (s > F32_WIDE_STEPS && pieces < max_pieces) continue;
         t = 1.65 + whole * (8.9 + s * (1.475 + 0.377 * (share < 1.0 ? share : 1.0)));
       } else if (tile == TILE_128) {
         t = 1.4 + whole * (5.9 + s * (0.945 + 0.22 * (share < 1.0 ? share : 1.0)));

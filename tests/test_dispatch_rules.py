@@ -3,6 +3,7 @@ size, which block shape for few rows) are plain functions of the sizes: they run
 a GPU, over sizes drawn at random, against what every choice must satisfy, and a few
 measured decisions are pinned so that a change of a constant shows."""
 import ctypes
+import math
 import random
 import shutil
 
@@ -402,3 +403,61 @@ def test_measured_launches_of_a_mixed_step(head_dim, nq, nkv, portion, behind, d
     # not a mixed step: nobody decodes, or everybody
     assert lib.llmlab_attention_mixed_launches(nq, nkv, 4, 0, portion, behind + portion, 0, 0, CUS) == 0
     assert lib.llmlab_attention_mixed_launches(nq, nkv, 4, 4, portion, behind + portion, their_keys, 0, CUS) == 0
+
+
+def first_float32_sum(m, n, k, max_pieces, min_steps):
+    """Steps of a sum by the estimate of the kernels that add all part products in one sum (64 x 64 and 128 x 128)."""
+    steps, best = -(-k // 32), None
+    for tile in (64, 128):
+        for pieces in range(1, max_pieces + 1):
+            s = -(-steps // pieces)
+            if pieces > 1 and s < min_steps:
+                break
+            share = -(-m // tile) * -(-n // tile) * pieces / CUS
+            whole = math.ceil(share - 1e-9)
+            if tile == 128:
+                t = whole * (5.4 + s * (1.31 + 0.12 * min(share, 1.0)))
+            else:
+                t, shared = 2.0 + 0.863 * s, (whole if share <= 3 else share) * (1.0 + 0.58 * s)
+                t = shared if shared > t and whole > 1 else t
+            t += pieces * (m * n * 2.2e-6 + 0.3) if pieces > 1 else 0.0
+            if best is None or t < best[0]:
+                best = (t, s)
+    return best[1]
+
+
+def test_float32_sums_are_no_longer_than_their_tile_allows(core):
+    """A product that may be cut: the 128 x 256 tile, which adds everything in one sum, adds no more steps than the first
+    kernels did (nor than 64, where more pieces are to be had), the others three times as many at most."""
+    core.llmlab_linear_plan_f32.restype = None
+    out, rng, kinds = (ctypes.c_int * 2)(), random.Random(9), set()
+    shapes = [(896, 4864), (896, 896), (1536, 1536), (2048, 2048), (1536, 8960), (1024, 4096)]
+    for i in range(6000):
+        n, k = rng.choice(shapes) if i % 2 else (16 * rng.randint(20, 400), 16 * rng.randint(8, 800))
+        m = rng.choice([rng.randint(65, 1024), rng.randint(1025, 9000)])
+        max_pieces, min_steps = rng.choice([(8, 8), (8, 8), (1, 1), (8, 40), (3, 8)])
+        core.llmlab_linear_plan_f32(m, n, k, CUS, max_pieces, min_steps, out)
+        pieces, kind = out
+        steps = -(-k // 32)
+        s = -(-steps // pieces)
+        assert 1 <= pieces <= max_pieces and kind in (0, 2, 3) and (pieces == 1 or s >= min_steps), (m, n, k, pieces, kind)
+        first = first_float32_sum(m, n, k, max_pieces, min_steps)
+        assert s <= (first if kind == 3 else 3 * first), (m, n, k, max_pieces, min_steps, pieces, kind, first)
+        if kind == 3 and pieces < max_pieces and -(-steps // (pieces + 1)) >= min_steps:
+            assert s <= 64, (m, n, k, pieces)
+        kinds.add((kind, pieces > 1))
+    assert len(kinds) == 6
+
+
+@pytest.mark.parametrize("tile,kind", [(64, 0), (128, 2), (131, 3)])
+def test_a_forced_float32_tile_is_planned_at_any_size(core, tile, kind):
+    core.llmlab_linear_plan_f32.restype = None
+    out, rng = (ctypes.c_int * 2)(), random.Random(10)
+    core.llmlab_debug_gemm_tile(tile)
+    try:
+        for _ in range(2000):
+            m, n, k = rng.randint(65, 9000), rng.randint(1, 6000), rng.randint(1, 20000)
+            core.llmlab_linear_plan_f32(m, n, k, CUS, rng.randint(1, 8), rng.choice([1, 8, 40, 500]), out)
+            assert out[1] == kind and 1 <= out[0] <= 8, (m, n, k, out[0], out[1])
+    finally:
+        core.llmlab_debug_gemm_tile(0)
