@@ -680,24 +680,22 @@ __global__ __launch_bounds__(ONE_WAVE ? 256 : 1024) void layernorm_kernel(
   }
   const float mean = total(s, 0) / (float)hidden;
   float v = 0.f;
-  auto deviate = [&](const Group& g) {
+  // (the roundings fixed, and the same in all instances: see rmsnorm_kernel)
+  auto deviate = [&](const Group& g, bool first) {
+    float d[W];
 #pragma unroll
-    for (int e = 0; e < W; ++e) {
-      const float d = g.v[e] - mean;
-      v += d * d;
+    for (int e = 0; e < W; ++e) d[e] = g.v[e] - mean;
+    if constexpr (W == 4) {
+      v = first ? fmaf(d[0], d[0], d[1] * d[1]) : fmaf(d[1], d[1], fmaf(d[0], d[0], v));
+      v = fmaf(d[3], d[3], fmaf(d[2], d[2], v));
+    } else {
+      v = fmaf(d[0], d[0], v);
     }
   };
-  if constexpr (KEEP == 1 && W == 4) {
-    // (the roundings of the other instances, whose second square is the first one rounded by itself)
-    if (t * W < hidden) {
-      const float d0 = keep[0].v[0] - mean, d1 = keep[0].v[1] - mean, d2 = keep[0].v[2] - mean, d3 = keep[0].v[3] - mean;
-      v = fmaf(d3, d3, fmaf(d2, d2, fmaf(d0, d0, d1 * d1)));
-    }
-  } else
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
-    if (t * W + j * step < hidden) deviate(keep[j]);
-  for (int c = t * W + KEEP * step; c < hidden; c += step) deviate(whole(c));
+    if (t * W + j * step < hidden) deviate(keep[j], j == 0);
+  for (int c = t * W + KEEP * step; c < hidden; c += step) deviate(whole(c), false);
   const float inv = 1.0f / sqrtf(total(v, 1) / (float)hidden + eps);
   auto put = [&](int c, const Group& g, const RawWeights<W>& wg, const Group& og) {
     typedef T Out __attribute__((ext_vector_type(W)));
@@ -734,7 +732,7 @@ static void launch_layernorm(const float* x, int splits, size_t stride, const vo
                    (((uintptr_t)out | (uintptr_t)copy) & (4 * sizeof(T) - 1)) == 0 &&
                    ((uintptr_t)w & (w_bf16 ? 7 : 15)) == 0;
   // A wave a row where the rows fill the chip and a row fits a wave's registers; else a block, whose
-  // threads cover the row in one group each, or in two or three where 1,024 threads (256 for more than 128 rows) do not.
+  // threads cover the row in one group each, or in two to four where 1,024 threads (256 for more than 128 rows) do not.
 #define LLMLAB_LAYERNORM(VEC, ONE_WAVE, KEEP, G, grid, threads)                                                     \
   hipLaunchKernelGGL((layernorm_kernel<T, ADD, VEC, ONE_WAVE, KEEP, G>), dim3(grid), dim3(threads), 0, stream, x,   \
                      splits, stride, w, w_bf16, eps, out, resid, copy, rows, n_rows, hidden)
@@ -753,8 +751,10 @@ static void launch_layernorm(const float* x, int splits, size_t stride, const vo
   else if (vec && threads * 4 >= hidden) LLMLAB_LAYERNORM(true, false, 1, 4, n_rows, threads);
   else if (vec && threads * 8 >= hidden && splits == 1) LLMLAB_LAYERNORM(true, false, 2, 0, n_rows, threads);
   else if (vec && threads * 8 >= hidden) LLMLAB_LAYERNORM(true, false, 2, 2, n_rows, threads);
-  else if (vec && splits == 1) LLMLAB_LAYERNORM(true, false, 3, 0, n_rows, threads);
-  else if (vec) LLMLAB_LAYERNORM(true, false, 3, 2, n_rows, threads);
+  else if (vec && threads * 12 >= hidden && splits == 1) LLMLAB_LAYERNORM(true, false, 3, 0, n_rows, threads);
+  else if (vec && threads * 12 >= hidden) LLMLAB_LAYERNORM(true, false, 3, 2, n_rows, threads);
+  else if (vec && splits == 1) LLMLAB_LAYERNORM(true, false, 4, 0, n_rows, threads);
+  else if (vec) LLMLAB_LAYERNORM(true, false, 4, 2, n_rows, threads);
   else LLMLAB_LAYERNORM(false, false, 4, 4, n_rows, threads);
 #undef LLMLAB_LAYERNORM
 }
