@@ -1,5 +1,5 @@
 """The float32 products of many rows that split every number into three bfloat16 parts
-(``gemm_f32_split_kernel``): both tiles, whole and in pieces, against 64 bits at the edges of the
+(``gemm_f32_split_kernel``): all tiles, whole and in pieces, against 64 bits at the edges of the
 tiles, with numbers of very different sizes, and with numbers that have no such parts."""
 import pytest
 import torch
@@ -25,7 +25,7 @@ def bound(x, w):
     return (x.shape[1] + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
 
 
-@pytest.mark.parametrize("tile", [64, 128, None])
+@pytest.mark.parametrize("tile", [64, 128, 131, None])
 @pytest.mark.parametrize("m,n,k", [(65, 64, 32), (66, 65, 33), (127, 63, 31), (128, 128, 64), (129, 130, 100),
                                    (192, 257, 1), (193, 36, 1153)])
 def test_against_64_bits(ops, tile, m, n, k):
@@ -45,13 +45,18 @@ def test_against_64_bits(ops, tile, m, n, k):
             assert bool(((got - want).abs() <= limit).all()), f"{pieces} pieces"
 
 
-@pytest.mark.parametrize("tile", [64, 128])
-def test_numbers_without_parts(ops, tile):
-    """Infinities, numbers that bfloat16 rounds to infinity and NaN: as plain 32-bit FMAs give them."""
+@pytest.mark.parametrize("tile", [64, 128, 131])
+@pytest.mark.parametrize("one_part", [False, True])
+def test_numbers_without_parts(ops, tile, one_part):
+    """Infinities, numbers that bfloat16 rounds to infinity and NaN: as plain 32-bit FMAs give them.  ``one_part``: W's
+    numbers are bfloat16 ones, infinite and NaN among them and one below the smallest normal number."""
     m, n, k = 70, 66, 40
     x, w = rnd((m, k), 5), rnd((n, k), 6)
     x[3, 7], x[10, 0], x[20, 39], x[65, 1] = float("inf"), 3.4e38, float("nan"), -float("inf")
     w[:, 0] = 1e-38 * w[:, 0]
+    if one_part:
+        w[5, 2], w[9, 35], w[40, 39], w[64, 3] = float("inf"), -float("inf"), float("nan"), 2.0 ** -130
+        w = w.bfloat16().float()
     want = x.double() @ w.double().T
     out = torch.empty(m, n, device=DEV)
     with ops.debug.force(gemm_tile=tile):
@@ -64,13 +69,17 @@ def test_numbers_without_parts(ops, tile):
     assert bool(((got - want).abs()[fine] <= limit[fine]).all())
 
 
-@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("tile", [64, 128, 131])
 @pytest.mark.parametrize("m,n,k", [(70, 66, 40), (129, 130, 100), (65, 64, 33)])
 @pytest.mark.parametrize("size", [-100, -104, -107, -110, -111, -112, -116, -120, -124, -126, -140])
-def test_small_numbers(ops, tile, m, n, k, size):
+@pytest.mark.parametrize("one_part", [False, True])
+def test_small_numbers(ops, tile, m, n, k, size, one_part):
     """Numbers whose last bits lie under bfloat16's smallest (or that are below float32's smallest normal number), in
-    one row among ordinary ones, in a few places among zeros, and on the other side of the product."""
+    one row among ordinary ones, in a few places among zeros, and on the other side of the product; beside
+    numbers of three parts and of one."""
     x, w = rnd((m, k), 7), rnd((n, k), 8) * 2.0 ** 90
+    if one_part:
+        w = w.bfloat16().float()
     x[3] *= 2.0 ** size
     alone = torch.arange(m - 9, m)
     x[alone] = 0
@@ -90,10 +99,11 @@ def test_small_numbers(ops, tile, m, n, k, size):
         assert bool(((parts.cpu().double().sum(0) - want).abs() <= limit).all())
 
 
-@pytest.mark.parametrize("tile", [64, 128])
-def test_sums_that_overflow(ops, tile):
+@pytest.mark.parametrize("tile", [64, 128, 131])
+@pytest.mark.parametrize("one_part", [False, True])
+def test_sums_that_overflow(ops, tile, one_part):
     """Numbers that have parts and a product past the largest float32: infinite, not NaN; a product just below it,
-    whose leading parts' product is past it: finite."""
+    whose leading parts' product is past it: finite.  ``one_part``: W's numbers are bfloat16 ones."""
     m, n, k = 70, 66, 40
     x, w = rnd((m, k), 9), rnd((n, k), 10)
     x[0], x[1], x[2] = 0, 0, 0
@@ -101,6 +111,9 @@ def test_sums_that_overflow(ops, tile):
     x[1, 6], w[7, 6] = 1e30, 1.0037e12
     root = 2.0 ** 64 * (1 - 2.0 ** -10)          # (its leading part is 2^64)
     x[2, 9], w[11, 9] = root, root
+    if one_part:
+        w[11, 9] = 2.0 ** 64
+        w = w.bfloat16().float()
     want = (x.double() @ w.double().T)
     limit = bound(x, w)
     want = torch.where(want.abs() >= 2.0 ** 128 * (1 - 2.0 ** -25), want.sign() * float("inf"), want)

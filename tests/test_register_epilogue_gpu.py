@@ -16,10 +16,15 @@ def test_every_tile_into_any_rows(ops, emu, tile, m, n, k, pad, shift):      # n
     x, w, b = rnd((m, k), bf, 1), rnd((n, k), bf, 2, 0.1), rnd((n,), torch.float32, 3)
     dx, dw = x.to(DEV), ops.prepare_weight(w.to(DEV))
 
-    def place(dtype):
-        """Rows of a wider matrix that begin at an odd place of it; what lies around them stays as it is."""
-        whole = torch.full((m, n + pad + shift), 7.0, dtype=dtype, device=DEV)
-        return whole, whole[:, shift:shift + n]
+    def place(dtype, *pieces):
+        """Rows of a wider and longer matrix (a tile's rows longer) that begin at an odd place of it; what lies around
+        them stays as it is."""
+        whole = torch.full((*pieces, m + 256, n + pad + shift), 7.0, dtype=dtype, device=DEV)
+        return whole, whole[..., :m, shift:shift + n]
+
+    def alone(whole, out):
+        out.fill_(7.0)
+        return bool((whole == 7.0).all())
 
     y = x.float() @ w.float().t()
     scale = y.abs().max().item()
@@ -27,20 +32,20 @@ def test_every_tile_into_any_rows(ops, emu, tile, m, n, k, pad, shift):      # n
         whole, out = place(bf)
         ops.linear(dx, dw, out, b.to(DEV))
         close(out, (y + b).to(bf), bf, "store", (y + b).abs().max().item())
-        rest, whole_f, out_f = whole.clone(), *place(torch.float32)
-        rest[:, shift:shift + n] = 7.0
-        assert bool((rest == 7.0).all()), "written beside the output"
+        assert alone(whole, out), "written beside the output"
+        whole_f, out_f = place(torch.float32)
         ops.linear_logits(dx, dw, out_f)
         close(out_f, y, torch.float32, "float32", scale)
+        assert alone(whole_f, out_f), "written beside the output"
         before = rnd((m, n), torch.float32, 4)
         out_f.copy_(before)
         ops.linear_residual(dx, dw, out_f)
         close(out_f, before + y, torch.float32, "into the residual", scale)
-        whole_f[:, shift:shift + n] = 7.0
-        assert bool((whole_f == 7.0).all()), "written beside the output"
-        parts = torch.zeros(3, m, n, device=DEV)
+        assert alone(whole_f, out_f), "written beside the output"
+        whole_p, parts = place(torch.float32, 3)
         ops.linear_partials(dx, dw, parts, 3)
         close(parts.sum(0), y, torch.float32, "pieces", scale)
+        assert alone(whole_p, parts), "written beside the pieces"
 
 
 @pytest.mark.parametrize("tile", [64, 130, 129, 131, 132, 133])
@@ -53,11 +58,11 @@ def test_paired_products(ops, emu, tile, activation, m, inter, k, pad):      # n
     constants = (1.5, 1.7, 1.0) if activation == "clamped" else None
     want = torch.empty(m, inter, dtype=bf)
     emu.linear_swiglu(x, w, want, activation, constants)
-    got = torch.full((m, inter + pad), 7.0, dtype=bf, device=DEV)
+    got = torch.full((m + 256, inter + pad), 7.0, dtype=bf, device=DEV)
     with ops.debug.force(gemm_tile=tile):
-        ops.linear_swiglu(x.to(DEV), ops.prepare_weight(w.to(DEV)), got[:, :inter], activation, constants)
-    close(got[:, :inter], want, bf, "paired", want.float().abs().max().item())
-    assert bool((got[:, inter:] == 7.0).all())
+        ops.linear_swiglu(x.to(DEV), ops.prepare_weight(w.to(DEV)), got[:m, :inter], activation, constants)
+    close(got[:m, :inter], want, bf, "paired", want.float().abs().max().item())
+    assert bool((got[:, inter:] == 7.0).all()) and bool((got[m:] == 7.0).all())
 
 
 @pytest.mark.parametrize("tile", [64, 132])
