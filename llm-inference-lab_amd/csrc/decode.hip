@@ -858,7 +858,11 @@ static SkinnyShape skinny_choose_tile(int epilogue, bool norm, int mb, int M, in
         const int per_cu = (blocks + num_cus - 1) / num_cus;       // blocks the busiest unit runs
         int resident = 16 / (nsb * kw);                             // of which so many at a time
         if (resident > per_cu) resident = per_cu;
-        const int by_lds = (int)((160 * 1024) / (lds > 1024 ? lds : 1024));
+        // (as many as LDS would hold with a block's results there, as where this was fitted; by what is left without
+        // them gate/up of 16 rows of the 1.5B shape takes 2 strips x 2 slices, 21.7 us, and not 8 x 1, 16.6, of 5 of the
+        // 7B shape 2 x 2, 57, and not 2 x 4, 52)
+        const size_t results = epilogue == SK_SWIGLU || epilogue == SK_QKV ? (size_t)M * 16 * nsb * sizeof(float) : 0;
+        const int by_lds = (int)((160 * 1024) / (lds + results > 1024 ? lds + results : 1024));
         if (resident > by_lds) resident = by_lds;
         if (resident < 1) resident = 1;
         const int rounds = (per_cu + resident - 1) / resident;

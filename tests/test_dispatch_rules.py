@@ -237,6 +237,18 @@ def test_block_shapes_of_products_of_few_rows(core):
         assert stage in (0, 1) and qsplit == 1
 
 
+@pytest.mark.parametrize("m,n,k,want", [
+    (16, 17920, 1536, (8, 1, 1, 1, 1)),      # 16.6 us; 2 strips x 2 slices 21.7
+    (5, 37888, 3584, (2, 4, 1, 1, 1)),       # 52; 2 x 2 57
+    (10, 37888, 3584, (16, 1, 1, 1, 1)),     # 55; 4 x 2 59
+])
+def test_measured_block_shapes_of_gate_and_up(core, m, n, k, want):
+    """Behind a norm, weights from memory."""
+    out = (ctypes.c_int * 5)()
+    core.llmlab_skinny_shape(3, 1, m, n, k, 0, CUS, 1, out)
+    assert tuple(out) == want
+
+
 def test_when_a_decode_graph_pays():
     """``graph="auto"``: the rule on measured cases.  At the 0.5B shape (151 calls a step, 1 GB
     of weights) the host cannot keep up and the graph is taken, also with 3.2 GB of cache
