@@ -144,7 +144,8 @@ __device__ __forceinline__ void epi_store(const EpiArgs& e, int m, int n, float 
 // exchanged between neighbouring groups of lanes so that a lane writes 16 bytes too.  By way of LDS, where a thread found
 // the activation anew for each number, a tile alone on its unit spent 14 us so with a residual (192 x 256, a trip to memory
 // behind the other) and 11 with paired results (256 x 256); here 7, at the rate of memory for what all units then want
-// at once, and 2.3.
+// at once, and 2.3 with the hardware's reciprocal in place of the activation's division, which takes 2 more (192 x
+// 256: gate and up of 2,048 rows of the 0.5B shape, two rounds, 54 us by way of LDS, 43 and 47).
 template <int TM, int TN, int EPI>
 __device__ __forceinline__ void register_epilogue(const floatx4 (&acc)[TM][TN], const EpiArgs& e, int m0, int n0, int M,
                                                   int N, int c, int g) {
@@ -1775,10 +1776,11 @@ constexpr int F32_ROWS_MAX = 64;     // up to here the few-row kernel (the tiled
 // is read by one wave only and the rows of x in LDS are shared by all of them; and the
 // 256 x 256 and 192 x 256 tiles of gemm_bf16_pingpong for the largest products.  The shape
 // is picked by an estimate of the time, fitted to sweeps of the four products of a layer
-// at three model shapes and 576 to 8192 rows (its picks cost 0.8 % over the best shape
-// there):
+// at three model shapes and 576 to 8192 rows, when all epilogues went through LDS (its picks then cost
+// 0.8 % over the best shape there; now, over shapes of 0.5B to 7B at 256 to 3,000 rows, 1.2 % for gate and up, 3.4 for output
+// and 3.6 for down products, and constants lowered to what the epilogues take lose more on single output products):
 //   time = L + rounds * (f + K tiles * tk),  rounds = max(1, blocks / (units * resident)).
-// One block of the 128 x 256 tile fills a compute unit (its epilogue stages 133 KB), so
+// One block of the 128 x 256 tile fills a compute unit (eight waves of 220 registers a lane), so
 // its rounds are whole: ceil(blocks / units).  Where its blocks fill their rounds it is
 // the fastest by 5 to 20 % (2048 rows, 3584 x 18944: 301 us against 337 with 128 x 128;
 // 8192 rows, 37888 x 3584: 2320 against 2577), where the last round is nearly empty the
@@ -1791,8 +1793,8 @@ constexpr double CHIP_STREAM = 5.3e6;     // bytes a microsecond
 
 // The tiles of the two groups of waves: whole rounds of one block a unit; with 256 rows a
 // step of 32 of the inner size takes 0.67 us in a full round and from 0.41 us in a round of
-// few blocks (the chip clocks higher), and 12.8 us pass before and after the loop; with 192
-// rows 0.54, 0.37 and 10.2 us (fitted to a sweep of 14 matrices of four model shapes at 512 to 8192
+// few blocks (the chip clocks higher), and 12.8 us were to pass before and after the loop; with 192
+// rows 0.54, 0.37 and 10.2 us (epilogues by way of LDS, as above; fitted to a sweep of 14 matrices of four model shapes at 512 to 8192
 // rows, inner sizes from 896 to 18944: 7 and 5 % rms).
 static double pingpong_cost(int bm, int M, int N, int K, int num_cus, int pieces) {
   const double rounds = (double)((M + bm - 1) / bm) * ((N + 255) / 256) * pieces / num_cus;
@@ -1884,7 +1886,7 @@ static int one_round_tile(int M, int N, int K, int num_cus) {
 // 1.44e-6); the others, whose small products have sums of their own and whose error at the same steps is 0.55 of
 // that, may add three times as many.  (Without the bound 4,040 rows of 1536 x 1536 whole 4.2e-7 / 6.0e-7 off 64 bits with one part of
 // W and with three, in two pieces 2.9e-7 / 4.2e-7; 2,312 of 2048 x 2048 4.9e-7 / 7.0e-7 and 3.4e-7 / 4.9e-7; 3,336 of 896 x
-// 4864 by 128 x 128 whole 4.3e-7, in two pieces 3.1e-7, by the first kernel in four 3.7e-7.)
+// 4864 by 128 x 128 whole 4.3e-7, in four pieces, as planned with it, 2.1e-7, by the first kernel in four 3.7e-7.)
 constexpr int F32_WIDE_STEPS = 64;
 static int f32_sum_steps(int M, int N, int steps, int num_cus, int max_pieces, int min_steps) {
   int most = steps;

@@ -1424,7 +1424,7 @@ __global__ __launch_bounds__(64) void sink_window_attention_grouped_kernel(MfmaA
 // outputs are asked for beside them; the shares' weights exp(m_z - M) lie in LDS, and the loop over the partial outputs
 // has no branch (past the last share that one again; an empty share, or one again, weighs zero and its numbers are
 // dropped), so that a chunk's loads for all of the wave's channels travel together.  (Sixteen rows of 16 heads of 128 in
-// 17 shares: 6.5 us in a decode step with four shares' loads of 64 channels at a time, 4.3 so.)
+// 17 shares: 6.5 us in a decode step with four shares' loads of 64 channels at a time, 4.5 to 4.8 so.)
 constexpr int MERGE_MAX_SPLITS = 256;
 template <int P>       // channels of a lane: E up to 64 P
 __global__ __launch_bounds__(64) void sink_window_attention_merge_kernel(MfmaArgs a, int E) {
