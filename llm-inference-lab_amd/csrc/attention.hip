@@ -30,6 +30,8 @@
 //
 // float32 kernel: the same scheme on the float32 matrix instruction (true 32-bit
 // products and sums), in steps of 16 keys.
+#include <type_traits>
+
 #include "common.h"
 
 #ifndef HEAD_DIM
@@ -885,6 +887,360 @@ __global__ __launch_bounds__(256 * PH, (D <= 64 && PH == 1) ? 2 : 1) void attent
   }
 }
 
+// ------------------------------------------------------------- bf16, rows by keys staged in LDS
+// Steps of many rows at heads of 64 and 128.  A block has RT tiles of 32 rows side by side, and P groups of waves that
+// take the staged keys in turn, GK of every P GK; the groups' sums meet in LDS at the end.  Keys and values come by direct
+// loads from the cache into LDS (the cache's order is the fragments' order) in NST stages of which all but the one being
+// multiplied are on their way, one barrier a stage.
+//
+// Products by v_mfma_f32_32x32x16_bf16, transposed as above (lane l: column = row l % 32 of the tile, h = l / 32):
+//   S^T[key, row] = K . Q^T: element i of the 32 keys of a step is key 8 (i / 4) + 4 h + i % 4;
+//   O^T[d, row] = V^T . P^T: the keys of a block of 16 in the order {4 h .. + 3, 8 + 4 h .. + 3} for half h, which is
+//   what a lane holds of S^T, eight neighbouring elements a product.
+// A lane has one row, whose maximum needs one exchange with the lane 32 on (and none while no maximum grows).  In LDS the
+// four groups of a block of 16 values by an odd 16 of d lie exchanged in pairs (the direct loads' lanes fetch them so): a
+// read takes both halves of 32 numbers of d, which then meet different banks.
+//
+// What bounds it: the vector instructions of the softmax (32 x 32 scores: 538 clocks of a SIMD at heads of 64, 16 of them an
+// exponential) beside 256 (heads of 128: 512) of matrix instructions, which overlap where a SIMD has four waves (heads of 64: two
+// blocks a unit, 455 clocks measured for both) and hardly where it has two (813); and how evenly a prompt's triangle
+// lies on the units.  Against the kernels below it (us, old -> new): 14 heads of 64 over 2, a prompt of 1,024 16.7 -> 12.9, of
+// 2,048 31.3 -> 21.6, of 4,096 78 -> 54; 2,000 tokens behind 3,000 85 -> 52; 28 heads of 128 over 4, three prompts of 1,000, 789
+// and 578 66 -> 35, a prompt of 4,096 268 -> 146, 1,000 tokens behind 1,500 86 -> 46.  The scores of the next stage
+// before the softmax of this one: no faster.  A load from the block table under a branch in the loop (or of the queries before it)
+// makes the compiler wait there for all that is on its way, every step: hence table_entry, and the queries' use before the loop.
+#define STAGED_ROWS (HEAD_DIM == 64 || HEAD_DIM == 128)
+#if STAGED_ROWS
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+// 16 keys (or their values) from the cache to consecutive memory of LDS, 1 KB a load; the offset counts at both ends
+template <int BYTES>
+__device__ __forceinline__ void block_to_lds(unsigned from, const char* base, unsigned to) {
+  static_assert(BYTES % 1024 == 0 && BYTES <= 4096, "offsets of 12 bits");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(to) : "memory", "m0");
+  if constexpr (BYTES >= 1024) asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(from), "s"(base) : "memory");
+  if constexpr (BYTES >= 2048) asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" : : "v"(from), "s"(base) : "memory");
+  if constexpr (BYTES >= 3072) asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" : : "v"(from), "s"(base) : "memory");
+  if constexpr (BYTES >= 4096) asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" : : "v"(from), "s"(base) : "memory");
+}
+
+// A number of the block table, waited for on the spot (the compiler, which does not see it, would wait for all loads on
+// their way wherever a branch with a load of its own ends)
+__device__ __forceinline__ int table_entry(const int* table, int at) {
+  int v;
+  asm volatile("global_load_dword %0, %1, %2\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(at * 4), "s"(table) : "memory");
+  return v;
+}
+
+template <int RT, int P, int GK, int NST>
+__device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk, const int kvh, const int b, char* lds) {
+  constexpr int NW = RT * P;                             // waves
+  constexpr int KT = GK * P, NS = GK / 32, DK = D / 16, DV = D / 32;
+  constexpr int BLK = 16 * D * 2;                        // bytes of 16 keys, and of their values
+  constexpr int V_AT = KT * D * 2, STAGE = 2 * V_AT;     // a stage: keys, then values
+  constexpr int NB = KT / 8 / NW;                        // blocks of 16 keys or of values that a wave brings of a tile
+  static_assert(GK % 32 == 0 && NB * 8 * NW == KT && D % 32 == 0, "steps of 32 keys, whole blocks a wave, loads of 1 KB");
+  constexpr int LOADS = NB * (BLK / 1024);               // ... its loads
+  static_assert(LOADS * (NST - 2) < 64, "loads on their way that can be counted");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rt = wave % RT, ph = wave / RT;
+  const int col = lane & 31, h = lane >> 5;
+  const int G = a.nq / a.nkv;
+  auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };      // (the same for all lanes: kept scalar)
+  const int r0 = uniform(a.q_start[b]), qlen = uniform(a.q_start[b + 1]) - r0, sp = uniform(a.start_pos[b]);
+  const int rows_total = qlen * G;
+  const int blk_row0 = xblk * RT * 32;
+  if (blk_row0 >= rows_total) return;                                   // the whole block is past the rows
+  if (qlen < a.qlen_lo || qlen > a.qlen_hi) return;                     // another launch's request
+  const int row0 = blk_row0 + rt * 32;
+  const float scale2 = a.scale * 1.4426950408889634f;
+  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+
+  // this lane's row (of its query, operand kk holds the numbers 16 kk + 8 h .. + 7)
+  const int rr = row0 + col;
+  const bool valid = rr < rows_total;
+  const int tok = valid ? rr / G : 0, head = kvh * G + (valid ? rr % G : 0);
+  const int pos = valid ? sp + tok : -1, lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  // the keys that the wave's rows see, and the block's; from full_lo on a key is inside the windows of all its rows
+  const int last_row = min(row0 + 32, rows_total) - 1, blk_last = min(blk_row0 + RT * 32, rows_total) - 1;
+  const int p_first = sp + uniform(row0 / G), p_last = sp + uniform(last_row / G);
+  const int full_lo = a.window > 0 ? max(0, p_last - a.window + 1) : 0;
+  const int bkey_hi = sp + uniform(blk_last / G);
+  const int bkey_lo = a.window > 0 ? max(0, sp + uniform(blk_row0 / G) - a.window + 1) : 0;
+
+  __shared__ int s_missing;
+  __shared__ float s_ml[NW * 64];
+  floatx16 o[DV];
+#pragma unroll
+  for (int i = 0; i < DV; ++i)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) o[i][x] = 0.f;
+  float m = NEG_INF, lsum = 0.f;
+
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const unsigned k_from = lane * 16, v_from = (lane ^ (h ? 8 : 0)) * 16;
+  // where a lane reads its keys and its values of a step
+  const int odd = (lane >> 4) & 1;
+  const int k_at = ph * (GK / 16) * BLK + odd * BLK + (h * 16 + (lane & 15)) * 16;
+  const int v_at = V_AT + ph * (GK / 16) * BLK + odd * 512 + (h ^ odd) * 128 + (lane & 15) * 8;
+  auto barrier = [&]() {      // (nothing moves across)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  };
+
+  // A wave brings NB blocks of 16 keys or of values of a tile: with an even number the keys and the values of NB / 2
+  // blocks, with one the keys (odd waves: the values) of a block.  Blocks that nobody sees read one that somebody does.
+  // Where in the caches: of 64 tiles at a time, tile base + l in lane l.
+  const int tile_lo = bkey_lo / KT, tile_hi = bkey_hi / KT;
+  const int pshift = a.page_shift;
+  const int* const table = a.table + (size_t)b * a.table_stride;
+  constexpr int NA = (NB + 1) / 2;
+  size_t where[NA];
+  auto locate = [&](int base) {
+    const int t = min(base + lane, tile_hi);
+#pragma unroll
+    for (int n = 0; n < NA; ++n) {
+      const int at16 = max(min(t * KT + ((wave * NB + 2 * n) >> 1) * 16, bkey_hi & ~15), bkey_lo & ~15), pi = at16 >> pshift;
+      const int page = table_entry(table, min(pi, a.table_stride - 1));
+      if (page < 0 || pi >= a.table_stride) s_missing = 1;
+      where[n] = ((((size_t)max(page, 0) * a.nkv + kvh) << pshift) + (at16 & ((1 << pshift) - 1))) * (D * 2);
+    }
+  };
+  int base = tile_lo;
+  auto fetch = [&](int t, int slot) {
+    if (t - base >= 64) locate(base = t);
+#pragma unroll
+    for (int n = 0; n < NA; ++n) {
+      const int u = wave * NB + 2 * n;
+      const size_t at = ((size_t)(unsigned)__builtin_amdgcn_readlane((int)(where[n] >> 32), t - base) << 32) |
+                        (unsigned)__builtin_amdgcn_readlane((int)where[n], t - base);
+      const unsigned to = lds0 + slot * STAGE + (u >> 1) * BLK;
+      if constexpr (NB > 1) {
+        block_to_lds<BLK>(k_from, (const char*)a.kc + at, to);
+        block_to_lds<BLK>(v_from, (const char*)a.vc + at, to + V_AT);
+      } else {
+        const bool values = u & 1;
+        block_to_lds<BLK>(values ? v_from : k_from, (values ? (const char*)a.vc : (const char*)a.kc) + at, values ? to + V_AT : to);
+      }
+    }
+  };
+  auto there = [&](int k16) {      // is this block of 16 keys in the cache (asked only if some are not)
+    const int pi = max(min(k16, bkey_hi & ~15), bkey_lo & ~15) >> pshift;
+    return pi < a.table_stride && table_entry(table, pi) >= 0;
+  };
+  bf16x8 qf[DK];
+  {
+    const bf16_t* qp = (const bf16_t*)a.q + (size_t)(r0 + tok) * a.q_stride + (size_t)head * D + h * 8;
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk) {
+      qf[kk] = *(const bf16x8*)(qp + kk * 16);
+    }
+  }
+  if (tid == 0) s_missing = 0;
+  __syncthreads();
+  locate(tile_lo);
+  // (waited for here, with the table: in the loop it would be waited for, with all that is on its way, in every step)
+#pragma unroll
+  for (int kk = 0; kk < DK; ++kk) {
+    qf[kk] = valid ? qf[kk] : zero8;
+    asm volatile("" : "+v"(qf[kk]));
+  }
+#pragma unroll
+  for (int t = 0; t < NST - 1; ++t) fetch(tile_lo + t, t);
+  int slot = 0;
+  bool missing = false;
+  int located = -1;
+  for (int tile = tile_lo; tile <= tile_hi; ++tile) {
+    // this tile's loads are in (the wave's own; behind the barrier, all), and the tile before is read by all
+    constexpr int VM = LOADS * (NST - 2);
+    __builtin_amdgcn_s_waitcnt(0x0070 | (VM & 15) | ((VM >> 4) << 14));
+    barrier();
+    if (located != base) missing = uniform(s_missing) != 0, located = base;      // (of the tiles located by now)
+    const char* const ks = lds + slot * STAGE + k_at;
+    const char* const vs = lds + slot * STAGE + v_at;
+    bf16x8 kf[DK][NS];
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk)
+#pragma unroll
+      for (int st = 0; st < NS; ++st) kf[kk][st] = *(const bf16x8*)(ks + st * 2 * BLK + kk * 512);
+    fetch(tile + NST - 1, slot == 0 ? NST - 1 : slot - 1);
+    if (tile * KT + KT - 1 > bkey_hi || missing) {
+      // values of keys that nobody sees yet may be anything: out of the products, although their probability is zero
+      for (int i = tid; i < KT * D / 8; i += 64 * NW) {
+        const int block = i / (2 * D), db = (i / 32) % (D / 16), g = ((i >> 3) & 3) ^ (db & 1);
+        const int k0 = tile * KT + block * 16 + g * 4;
+        const bool ok = !missing || there(k0 & ~15);
+        bf16x8* at = (bf16x8*)(lds + slot * STAGE + V_AT + i * 16);
+        bf16x8 v = *at;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) v[x] = ok && k0 + (x & 3) <= bkey_hi ? v[x] : (bf16_t)0.f;
+        *at = v;
+      }
+      __syncthreads();
+    }
+    const int kb0 = tile * KT + ph * GK;
+    floatx16 s[NS];
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) s[st][x] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk)
+#pragma unroll
+      for (int st = 0; st < NS; ++st) s[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk][st], qf[kk], s[st], 0, 0, 0);
+    // (the values of the first 32 keys travel while the maximum is found)
+    bf16x8 vf[2][DV];
+    auto values = [&](bf16x8 (&f)[DV], int block) {
+#pragma unroll
+      for (int i = 0; i < DV; ++i) {
+        const char* at = vs + block * BLK + i * 1024;
+        const bf16x4 v0 = *(const bf16x4*)at, v1 = *(const bf16x4*)(at + 256);
+        f[i] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+    };
+    values(vf[0], 0);
+    values(vf[1], 1);
+    if (!(kb0 + GK - 1 <= p_first && kb0 >= full_lo && !missing)) {      // some of the keys are not for every row
+#pragma unroll
+      for (int st = 0; st < NS; ++st)
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub) {
+          const int k16 = kb0 + st * 32 + sub * 16;
+          const bool ok = !missing || there(k16);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int j = k16 + 8 * (i >> 2) + 4 * h + (i & 3);
+            s[st][sub * 8 + i] = ok && j <= pos && j >= lo ? s[st][sub * 8 + i] : NEG_INF;
+          }
+        }
+    }
+    // the maximum of the raw scores, then into the units of the exponent (the scale is positive)
+    float mx[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+      for (int x = 0; x < 16; x += 2) mx[(x >> 1) & 3] = max3_raw(s[st][x], s[st][x + 1], mx[(x >> 1) & 3]);
+    mx[0] = max_raw(max3_raw(mx[0], mx[1], mx[2]), mx[3]);
+    if (__any(mx[0] * scale2 > m + LAZY_MAX)) {            // some row's maximum grew: rescale what is summed so far
+      mx[0] = max_across_32(mx[0]) * scale2;
+      const bool grow = mx[0] > m + LAZY_MAX;
+      const float m_new = grow ? mx[0] : m;
+      const float alpha = grow ? fast_exp2(m - m_new) : 1.f;     // 2^-inf = 0 the first time
+      lsum *= alpha;
+#pragma unroll
+      for (int i = 0; i < DV; ++i)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) o[i][x] *= alpha;
+      m = m_new;
+    }
+    const float neg_m = m == NEG_INF ? 0.f : -m;      // (no visible key yet: every p of the row is 2^-inf = 0)
+#pragma unroll
+    for (int block = 0; block < 2 * NS; ++block) {
+      float pv[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pv[i] = fast_exp2(fmaf(s[block >> 1][(block & 1) * 8 + i], scale2, neg_m));
+      lsum += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+      bf16x8 pf;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pf[i] = (bf16_t)pv[i];
+#pragma unroll
+      for (int i = 0; i < DV; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[block & 1][i], pf, o[i], 0, 0, 0);
+      if (block + 2 < 2 * NS) values(vf[block & 1], block + 2);
+    }
+    slot = slot == NST - 1 ? 0 : slot + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);      // the last loads (of tiles past the end) are in, and the stages read
+  __syncthreads();
+  lsum += __shfl_xor(lsum, 32, WAVE);
+
+  // lane (col, h) holds, of a block of 32 of d, the numbers 8 q + 4 h .. + 3 of its row for q = 0 .. 3
+  auto put = [&](int row, int d0, const floatx4& v, float inv) {
+    bf16_t* dst = (bf16_t*)a.out + (size_t)(r0 + row / G) * a.out_stride + (size_t)(kvh * G + row % G) * D + d0;
+    *(bf16x4*)dst = bf16x4{(bf16_t)(v[0] * inv), (bf16_t)(v[1] * inv), (bf16_t)(v[2] * inv), (bf16_t)(v[3] * inv)};
+  };
+  if constexpr (P == 1) {
+    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    if (valid)
+#pragma unroll
+      for (int i = 0; i < DV; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          put(rr, i * 32 + q * 8 + h * 4, floatx4{o[i][4 * q], o[i][4 * q + 1], o[i][4 * q + 2], o[i][4 * q + 3]}, inv);
+  } else {
+    //   o = sum_p 2^(m_p - m) o_p,  l likewise,  m = max_p m_p
+    // Group ph sums up the pieces (four numbers a lane) ph, ph + P, ..; a wave leaves the others in LDS.
+    static_assert(DV * 4 % P == 0, "whole shares");
+    constexpr int SHARES = DV * 4 / P;
+    floatx4* const xo = (floatx4*)lds;                       // [wave][share][group but the wave's own][lane]
+    float* const x_m = s_ml;                                 // [wave][32], then the denominators
+    float* const x_l = x_m + NW * 32;
+    if (h == 0) {
+      x_m[wave * 32 + col] = m;
+      x_l[wave * 32 + col] = lsum;
+    }
+    auto quad = [&](int piece) {
+      const floatx16& v = o[piece >> 2];
+      const int q = (piece & 3) * 4;
+      return floatx4{v[q], v[q + 1], v[q + 2], v[q + 3]};
+    };
+    floatx4 own[SHARES];
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int n = 0; n < SHARES; ++n) {
+        if (p == ph) own[n] = quad(n * P + p);
+        else xo[((wave * SHARES + n) * (P - 1) + (p > ph ? p - 1 : p)) * 64 + lane] = quad(n * P + p);
+      }
+    __syncthreads();
+    float w[P], mx = NEG_INF, den = 0.f;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      w[p] = x_m[(p * RT + rt) * 32 + col];
+      mx = fmaxf(mx, w[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      w[p] = w[p] == NEG_INF ? 0.f : fast_exp2(w[p] - mx);
+      den += w[p] * x_l[(p * RT + rt) * 32 + col];
+    }
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+#pragma unroll
+    for (int n = 0; n < SHARES; ++n) {
+      const int piece = n * P + ph;
+      floatx4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        v += w[p] * (p == ph ? own[n] : xo[(((p * RT + rt) * SHARES + n) * (P - 1) + (ph > p ? ph - 1 : ph)) * 64 + lane]);
+      if (valid) put(rr, (piece >> 2) * 32 + (piece & 3) * 8 + h * 4, v, inv);
+    }
+  }
+}
+template <int RT, int P, int GK, int NST>
+constexpr int rows_lds_bytes() {
+  const int stages = NST * GK * P * D * 4, sums = RT * (P - 1) * 32 * D * 4;
+  return stages > sums ? stages : sums;
+}
+
+// 32 RT rows a block.  Along x, the tiles with the longest histories of all kv heads and requests come first, so that the
+// short ones fill what those leave (more blocks than x takes: tiles, kv heads and requests along x, y and z).
+template <int RT, int P, int GK, int NST, int WAVES>
+__global__ __launch_bounds__(64 * RT * P, WAVES) void attention_rows_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(1024))) char rows_lds[rows_lds_bytes<RT, P, GK, NST>()];
+  int rank = (int)blockIdx.x, kvh = (int)blockIdx.y, z = (int)blockIdx.z;
+  if (gridDim.y == 1 && gridDim.z == 1) {
+    const int per = a.nkv * (a.picked > 0 ? a.picked : a.reqs), at = rank % per;
+    rank /= per;
+    kvh = at % a.nkv;
+    z = at / a.nkv;
+  }
+  const int b = __builtin_amdgcn_readfirstlane(request_of(a, z));
+  if (b < 0) return;
+  attention_rows<RT, P, GK, NST>(a, a.tiles - 1 - rank, kvh, b, rows_lds);
+}
+#endif  // STAGED_ROWS
+
 // Merge of the key splits of a decode step, one block of four waves per (row, head):
 //   out = sum_s w_s acc_s / sum_s w_s l_s,  w_s = 2^(m_s - max m).
 // Every wave takes a quarter of the splits (lane = element of the head), has all of
@@ -1539,6 +1895,35 @@ static int choose_many_rows_launch(long max_rows, int nkv, int live, int max_q_l
   return path;
 }
 
+// Heads of 64 and 128: attention_rows serves what the launches 2 to 6 would, and launch 1 where it is faster: at heads of
+// 128 everywhere (us: 4 / 48 / 96 tokens of 28 heads over 4 behind 1,500 keys 27 / 33 / 33 -> 21 / 23 / 24, behind 4,000 45 / 46 / 47 ->
+// 43), at heads of 64 behind fewer than 1,024 (48 tokens of 14 heads over 2 behind 500 10.4 -> 9.7, behind 1,500 14.8 and 14.5,
+// behind 4,000 24.0 and 27.4).  Not beside decoding requests: one launch for both kinds and two give the same there, to the bit.
+static bool splits_keys(bool mixed, int max_q_len, int max_ctx_len, int forced) {
+  return !STAGED_ROWS || mixed || forced == 1 || (D == 64 && max_ctx_len - max_q_len >= 1024);
+}
+#if STAGED_ROWS
+// ... and by which block, RT tiles of 32 rows by P groups of waves.  The more groups, the shorter a tile's chain of steps;
+// the more rows, the fewer reads of the keys.  By `blocks`, tiles of 64 rows (1, 2 and 4 tiles of 32 rows with 4, 4 / 2 and 2 / 1 groups, us):
+// heads of 64: a prompt of 1,024 (224 blocks) 12.9 / 13.3 / 18.1, of 1,536 (336) 19.6 / 18.3 / 23.7, of 4,096 (896) 67 / 53.9 / 54.4,
+// of 8,192 (1,792) 213 / 171 / 161, two of 2,000 and 1,789 (876) 44 / 34 / 32; heads of 128 (28 over 4), 2 tiles with 4 and 2
+// groups and 4 with one: 512 tokens (224) 14.8 / 14.6 / 18.9, 768 (336) 24 / 20 / 25, 464 behind 3,000 (204) 42.5 / 51 / 81,
+// 2,048 (896) 68 / 51 / 57, 3,072 (1,344) 126 / 98 / 90.  Hardly a step of keys: four tiles, one group (64 prompts of 24 tokens: heads of
+// 64 12.9 / 10.5 / 7.0, of 128 29 / 18 / 12).
+enum { ROWS_1x4 = 1, ROWS_2x4 = 2, ROWS_4x2 = 3, ROWS_4x1 = 4, ROWS_2x2 = 5 };
+static int rows_kind(long max_rows, int nkv, int live, int max_q_len, int max_ctx_len, int num_cus, int forced) {
+  if (forced == 2) return D == 64 ? ROWS_4x2 : ROWS_4x1;      // (32 rows a wave over all keys, or nearly; tests)
+  if (forced == 3) return D == 64 ? ROWS_1x4 : ROWS_2x2;
+  if (forced == 4) return ROWS_4x1;
+  if (forced == 5 || forced == 6) return ROWS_2x4;
+  const long blocks = (max_rows + 63) / 64 * nkv * live;
+  if (max_ctx_len <= (D == 64 ? 64 : 32)) return ROWS_4x1;
+  if (D == 64) return 8 * blocks <= 7L * num_cus ? ROWS_1x4 : blocks <= 3L * num_cus ? ROWS_2x4 : ROWS_4x2;
+  if (blocks > 4L * num_cus) return ROWS_4x1;
+  return blocks <= num_cus && max_ctx_len > 512 ? ROWS_2x4 : ROWS_2x2;
+}
+#endif
+
 // Whether a mixed step goes in one launch with the portions by tiles of 16 rows, whose waves split the keys with one
 // step on its way: few enough registers (116 at heads of 64, against 157 to 201) that a unit holds two
 // blocks of either kind, so that the decoding requests' streams pass beside the portions' chains.  `blocks16` and
@@ -1715,7 +2100,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     const int rc = launch_key_split_decode(shorts, reqs, total_rows, nq, nkv, row_req, out, out_stride, stream);
     if (rc) return rc;
   }
-  if (path == 1) {
+  if (path == 1 && splits_keys(mixed, max_q_len, max_ctx_len, g_force_path)) {
     if (how == MIXED_ONE_LAUNCH) {
       const int long_tiles = (int)((max_rows + 31) / 32);
       dim3 mgrid((unsigned)mixed_blocks(long_tiles)), mblock(64 * DECODE_WAVES);
@@ -1739,6 +2124,26 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     LLMLAB_LAUNCH_CHECK("attention(bfloat16, key split)");
     return 0;
   }
+#if STAGED_ROWS
+  const int kind = rows_kind(max_rows, nkv, live, max_q_len, max_ctx_len, num_cus, g_force_path);
+  auto launch = [&](auto kernel, int rt, int waves) {
+    a.tiles = (int)((max_rows + 32 * rt - 1) / (32 * rt));
+    const long blocks = (long)a.tiles * nkv * zs;
+    const dim3 grid = blocks <= 0xffffffffl / (64 * waves) ? dim3((unsigned)blocks) : dim3((unsigned)a.tiles, nkv, zs);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, stream, a);
+  };
+  if constexpr (D == 64) {
+    if (kind == ROWS_1x4) launch(attention_rows_kernel<1, 4, 32, 2, 2>, 1, 4);
+    if (kind == ROWS_2x4) launch(attention_rows_kernel<2, 4, 32, 2, 4>, 2, 8);
+    if (kind == ROWS_4x2) launch(attention_rows_kernel<4, 2, 32, 3, 4>, 4, 8);
+    if (kind == ROWS_4x1) launch(attention_rows_kernel<4, 1, 32, 3, 4>, 4, 4);
+  } else {
+    if (kind == ROWS_2x4) launch(attention_rows_kernel<2, 4, 32, 2, 2>, 2, 8);
+    if (kind == ROWS_2x2) launch(attention_rows_kernel<2, 2, 32, 2, 2>, 2, 4);
+    if (kind == ROWS_4x1) launch(attention_rows_kernel<4, 1, 32, 3, 2>, 4, 4);
+  }
+  LLMLAB_LAUNCH_CHECK("attention(bfloat16, staged rows)");
+#else
   if (path == 2) {
     dim3 grid((unsigned)((max_rows + 127) / 128), nkv, zs), block(256);
     hipLaunchKernelGGL((attention_bf16_kernel<2, false>), grid, block, 0, stream, a);
@@ -1762,5 +2167,6 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     hipLaunchKernelGGL((attention_bf16_kernel<1, false>), grid, block, 0, stream, a);
   }
   LLMLAB_LAUNCH_CHECK("attention(bfloat16, prefill)");
+#endif
   return 0;
 }
