@@ -4,7 +4,8 @@
 //
 //   bfloat16:  v_mfma_f32_16x16x32_bf16 everywhere.
 //     * small products: 64x64, four waves 2x2, both operands loaded from global memory straight
-//       into a ring of three stages of LDS (gemm_bf16_ring).
+//       into a ring of three stages of LDS (gemm_bf16_ring); 128x128, 128x192 and 192x128 with eight waves 4x2 in the same
+//       way where their blocks find a unit each, or two of them one.
 //     * tiled kernel: 256 threads = 4 waves, block tile 64x128 or
 //       128x128 (waves 1x4, side by side along the columns), or 512 threads = 8 waves on
 //       128x256 (1x8; widths of 96 to 224 with a wave per 32 columns; 64x64 with waves 2x2 for grouped
@@ -149,7 +150,7 @@ __device__ __forceinline__ void epi_store(const EpiArgs& e, int m, int n, float 
 template <int TM, int TN, int EPI>
 __device__ __forceinline__ void register_epilogue(const floatx4 (&acc)[TM][TN], const EpiArgs& e, int m0, int n0, int M,
                                                   int N, int c, int g) {
-  static_assert(TM % 2 == 0 && TN % 2 == 0, "blocks in pairs");
+  static_assert(TN % 2 == 0 && (TN % 4 == 0 || TM % 2 == 0 || EPI != EPI_SWIGLU), "blocks in pairs");
   // eight neighbouring results a lane out of four of block a and four of block b: lane groups 0 and 2 get a's, 1 and
   // 3 b's, the lower half of the block's columns in groups 0 and 1
   auto exchange = [](const bf16x4& a, const bf16x4& b) {
@@ -172,7 +173,7 @@ __device__ __forceinline__ void register_epilogue(const floatx4 (&acc)[TM][TN], 
           if (o0 + col + x < e.n_out) out[(size_t)m * e.ldo + o0 + col + x] = v[x];
     };
     // (two runs of outputs of a row where a wave has them, else the same run of two rows)
-    constexpr int DI = TN >= 4 ? 1 : 2, DJ = TN >= 4 ? 2 : 1;
+    constexpr int DI = TN % 4 == 0 ? 1 : 2, DJ = TN % 4 == 0 ? 2 : 1;
     auto results = [&](auto act) {      // (the activation a constant: no branch a number)
       auto pair = [&](int i, int jp) {
         bf16x4 v;
@@ -884,22 +885,25 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong(const bf16_t* __restri
 // takes one barrier, and three blocks of the 64 x 64 tile (48 KB) share a unit.  Against the same tile with x by way of registers and W
 // straight into them, over 182 products of 24 to 2,048 rows whole and in pieces: 18 % less; 512 rows of 896 x 896 8.9 -> 7.8 us,
 // 2,048 11.7 -> 9.2, 512 of 896 x 4864 in four pieces 15.6 -> 12.6, 64 of 3584 x 18944 in eight 39.6 -> 30.8.  Four and five stages (two blocks a
-// unit): 4 % slower.  Larger tiles of this kind: 64 x 128 (three stages) is slower than the tile above with many
+// unit): 4 % slower.  Larger tiles of this kind with four waves: 64 x 128 (three stages) is slower than the tile above with many
 // rows (512 of 9728 x 896 24.8 against 21.4) and faster in pieces of few rows only (64 of 3584 x 18944 28.2 against 32.4), 128 x 160
 // and 128 x 256 as fast as theirs (128 of 37888 x 3584 71.8 against 73.7): not kept.
-template <int EPI>
-__global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
-                                                      EpiArgs e, int M, int N, int K) {
-  constexpr int BM = 64, BN = 64, NST = 3;
-  constexpr int NT = 256, WTM = BM / 2, WTN = BN / 2, TM = WTM / 16, TN = WTN / 16;
-  constexpr int XL = BM / 8, WL = BN / 8, NL = (XL + WL) / 4;      // loads of 1 KB of a stage: of x, of W, of one wave
-  static_assert((XL + WL) % 4 == 0 && WTM % 16 == 0 && WTN % 16 == 0 && NL * (NST - 2) < 64, "shape");
+// With eight waves, 4 x 2: 128 x 128 and 128 x 192 in three stages (one block a unit) and 192 x 128 in two (two blocks a
+// unit, the end of one behind the loop of the other); which product takes them and what they measure: direct_tile.  What bounds
+// them is LDS (128 x 192: 128 KB of fragments a stage, 1,024 clocks beside 768 of matrix instructions) and, of 16 us
+// that 512 rows of 9728 x 896 take, the half that launch, first trip to memory and epilogue are.
+template <int EPI, int BM = 64, int BN = 64, int NST = 3, int WM = 2, int WN = 2, int WAVES = 1>
+__global__ __launch_bounds__(64 * WM * WN, WAVES) void gemm_bf16_ring(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                      EpiArgs e, int M, int N, int K) {
+  constexpr int NW = WM * WN, NT = 64 * NW, WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
+  constexpr int XL = BM / 8, WL = BN / 8, NL = (XL + WL) / NW;     // loads of 1 KB of a stage: of x, of W, of one wave
+  static_assert((XL + WL) % NW == 0 && WTM % 16 == 0 && WTN % 16 == 0 && NL * (NST - 2) < 64, "shape");
   constexpr int STAGE = (XL + WL) * 1024, W_AT = XL * 1024;
   constexpr int C_STRIDE = BN + 4;
   constexpr size_t C_BYTES = (size_t)BM * C_STRIDE * sizeof(float);
   __shared__ __attribute__((aligned(1024))) char smem[EPI == EPI_QKV && C_BYTES > NST * STAGE ? C_BYTES : NST * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % WM, wn = wave / WM;
   int bx = blockIdx.x, by = blockIdx.y;
   {                                                      // a band of column tiles per die, as above
     const int gx = gridDim.x, gy = gridDim.y, total = gx * gy;
@@ -920,12 +924,12 @@ __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__
   unsigned off[NL];
   int shift[NL];
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-  // Load i of a wave is number wave + 4 i of the stage: the first XL take 8 rows of x each, the others a step
+  // Load i of a wave is number wave + NW i of the stage: the first XL take 8 rows of x each, the others a step
   // of a strip of W.  Rows past M, strips past N and numbers past K read a valid place instead.
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
-    const int b = wave + 4 * i;
-    if (4 * i < XL) {                     // (XL % 4 == 0: the same for all waves)
+    const int b = wave + NW * i;
+    if (NW * i < XL) {                    // (XL % NW == 0: the same for all waves)
       shift[i] = ((lane & 7) ^ (((b & 1) << 2) | (lane >> 4))) * 8;
       off[i] = ((unsigned)(min(m0 + b * 8 + (lane >> 3), M - 1) - m0) * (unsigned)K + shift[i]) * 2u;
     } else {
@@ -934,7 +938,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__
       off[i] = (unsigned)(min((n0 >> 4) + f, nstrips - 1) - (n0 >> 4)) * (unsigned)T * 1024u + lane * 16u;
     }
   }
-  static_assert(XL % 4 == 0, "x first");
+  static_assert(XL % NW == 0, "x first");
   const char* const xbase = (const char*)(A + (size_t)m0 * K);
   const char* const wbase = (const char*)(W + (size_t)(n0 >> 4) * T * 512);
   auto load_to_lds = [&](unsigned at, const char* base, unsigned to) {
@@ -955,12 +959,12 @@ __global__ __launch_bounds__(256) void gemm_bf16_ring(const bf16_t* __restrict__
     const char* w1 = wbase + (size_t)min(t + 1, T - 1) * 1024;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      const unsigned to = lds0 + slot + (wave + 4 * i) * 1024;
-      if (4 * i < XL) {
+      const unsigned to = lds0 + slot + (wave + NW * i) * 1024;
+      if (NW * i < XL) {
         if (whole) load_to_lds(off[i], xb, to);
         else load_to_lds(off[i] + (unsigned)(min(k + shift[i], K - 8) - shift[i]) * 2u, xb, to);
       } else {
-        load_to_lds(off[i], ((wave + 4 * i - XL) & 1) ? w1 : w0, to);
+        load_to_lds(off[i], ((wave + NW * i - XL) & 1) ? w1 : w0, to);
       }
     }
   };
@@ -1545,7 +1549,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_split_kernel(const f
 // The tiles of the products of many rows (what the numbers are: below, where a bfloat16 product is given its tile).
 enum { TILE_64 = 0, TILE_64x128 = 1, TILE_128 = 2, TILE_128x256 = 3, TILE_256 = 4, TILE_192 = 5, TILE_KINDS = 6,
        // chosen by their own rule (one_round_tile) for whole products
-       TILE_64x96 = 6, TILE_64x160 = 7, TILE_64x224 = 8, TILE_128x160 = 9, TILE_ALL = 10 };
+       TILE_64x96 = 6, TILE_64x160 = 7, TILE_64x224 = 8, TILE_128x160 = 9,
+       // by direct loads, eight waves: in place of other tiles where direct_tile says so
+       TILE_DIRECT_128 = 10, TILE_DIRECT_128x192 = 11, TILE_DIRECT_192x128 = 12, TILE_ALL = 13 };
 struct TileModel {
   int bm, bn;
   double L, f, tk, resident, stream;
@@ -1559,7 +1565,8 @@ static const TileModel TILE_MODELS[TILE_ALL] = {{64, 64, 6.39, 0.79, 0.289, 1.0,
                                                   {128, 256, 0.0, 6.16, 0.945, 1.0, 24e3, 1},
                                                   {256, 256, 0.0, 12.8, 1.34, 1.0, 24e3, 1},
                                                   {192, 256, 0.0, 10.2, 1.08, 1.0, 24e3, 1},
-                                                  {64, 96}, {64, 160}, {64, 224}, {128, 160}};
+                                                  {64, 96}, {64, 160}, {64, 224}, {128, 160},
+                                                  {128, 128}, {128, 192}, {192, 128}};
 
 // The tile of a float32 product of many rows, and into how many pieces along the inner size one that adds
 // into the stream is cut.
@@ -1824,7 +1831,7 @@ static double tile_cost(int kind, int M, int N, int K, int num_cus, int pieces) 
 
 // Debug interface (kernels/debug.py): a tile can be forced, for tests and measurements
 // (0 = choose; 64, 130 = 64 x 128, 129 = 128 x 128, 131 = 128 x 256, 132 = 256 x 256, 133 =
-// 192 x 256, 134 / 135 / 136 = 64 x 96 / 160 / 224, 137 = 128 x 160; -131 = choose among the first three; -256 and below: the tiles of two groups
+// 192 x 256, 134 / 135 / 136 = 64 x 96 / 160 / 224, 137 = 128 x 160, 138 / 139 / 140 = 128 x 128, 128 x 192 and 192 x 128 by direct loads; -131 = choose among the first three; -256 and below: the tiles of two groups
 // of waves from so many rows on).
 static int g_force_tile = 0, g_without_wide = 0, g_pp_min_rows = 512;
 // The 128 x 256 tile is weighed from so many rows on.  (By the product alone it would pay from
@@ -2104,10 +2111,50 @@ extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
   return TILE_MODELS[plain_tile(M, N, K, num_cus > 0 ? num_cus : 256)].bn;
 }
 
+// The tiles of eight waves by direct loads in place of the tile that the estimates, the plan or a rule above named: those
+// choose among tiles by their sizes (and answer for them); these are faster where all their blocks find a place at once.
+// Every sum keeps its order, so the results are the same to the bit.
+//   128 x 128, a block a unit, in place of 64 x 128 and 128 x 128 in one round, whole or in pieces (beyond 64 rows; us
+//   before / with it): 384 rows of 9728 x 896 13.6 / 11.8, 256 of 11008 x 2048 24.3 / 21.1, 2,048 of 896 x 4864 in two pieces
+//   32.0 / 26.8, 384 of 2048 x 11008 in four 34.5 / 27.5, 457 of 3584 x 18944 in two 114 / 84.  Beyond one round it loses (512 of
+//   9728 x 896, 304 blocks, 17.6 / 21.2).
+//   192 x 128, two blocks a unit, in place of a 64 x 128 tile of more than two blocks a unit where its own find a unit each: 512 rows
+//   of 9728 x 896 17.6 / 15.0, 1,024 of 4864 x 896 18.2 / 15.2, 384 of 11008 x 2048 32.5 / 28.5; and of 192 x 256 whose last round is
+//   less than half full, of up to three, at inner sizes to 2,048: 1,900 of 9728 x 896 43.8 / 39.0, 900 of 17920 x 1536 63.4 / 56.1, 1,536
+//   of 11008 x 2048 77.9 / 74.2 (not 1,024 of 17920 x 1536, 1.64 rounds, 66.8 / 69.2; 384 of 37888 x 3584 137 / 141).
+//   128 x 192, a block a unit, where 192 x 128 has more than units: 640 of 9728 x 896 18.7 / 16.7, 256 of 17920 x 1536 26.8 / 23.3,
+//   512 of 11008 x 2048 34.2 / 32.0.
+// (Weights from memory and not from the caches.  An MI355X has 256 units.)
+static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads) {
+  constexpr long UNITS = 256;
+  if (K > DIRECT_MAX_INNER) return kind;
+  if (g_force_tile >= 138 && g_force_tile <= 140) {
+    const int forced = TILE_DIRECT_128 + (g_force_tile - 138);
+    return heads && forced != TILE_DIRECT_128 ? kind : forced;
+  }
+  if (g_force_tile != 0 || g_without_wide || M <= 64) return kind;
+  auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * pieces; };
+  if ((kind == TILE_64x128 || kind == TILE_128) && blocks(128, 128) <= UNITS) return TILE_DIRECT_128;
+  if (heads) return kind;
+  if (kind == TILE_64x128 && blocks(64, 128) > 2 * UNITS) {
+    if (blocks(192, 128) <= UNITS) return TILE_DIRECT_192x128;
+    if (blocks(128, 192) <= UNITS) return TILE_DIRECT_128x192;
+  }
+  const long large = blocks(192, 256), last = large % UNITS;
+  if (kind == TILE_192 && pieces == 1 && K <= 2048 && large > UNITS && large < 3 * UNITS && last > 0 && 2 * last <= UNITS)
+    return TILE_DIRECT_192x128;
+  return kind;
+}
+// ... its code above (for tests; -1: the tile stays)
+extern "C" int llmlab_direct_tile(int kind, int M, int N, int K, int pieces, int heads) {
+  const int tile = direct_tile(kind, M, N, K, pieces, heads != 0);
+  return tile == kind ? -1 : tile;
+}
+
 template <int EPI>
 static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArgs& e, int M, int N, int K,
                         int pieces, hipStream_t stream) {
-  kind = addressable(kind, K);             // (a tile that the caller names)
+  kind = direct_tile(addressable(kind, K), M, N, K, pieces, EPI == EPI_QKV);      // (a tile that the caller names)
   const TileModel& t = TILE_MODELS[kind];
   dim3 grid((N + t.bn - 1) / t.bn, (M + t.bm - 1) / t.bm, pieces);
   if (kind == TILE_64)
@@ -2122,6 +2169,14 @@ static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArg
     hipLaunchKernelGGL((gemm_bf16_pingpong<256, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
   else if (kind == TILE_192)
     hipLaunchKernelGGL((gemm_bf16_pingpong<192, EPI>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  else if (kind == TILE_DIRECT_128)
+    hipLaunchKernelGGL((gemm_bf16_ring<EPI, 128, 128, 3, 4, 2, 2>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  if constexpr (EPI != EPI_QKV) {
+    if (kind == TILE_DIRECT_128x192)
+      hipLaunchKernelGGL((gemm_bf16_ring<EPI, 128, 192, 3, 4, 2, 2>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+    else if (kind == TILE_DIRECT_192x128)
+      hipLaunchKernelGGL((gemm_bf16_ring<EPI, 192, 128, 2, 4, 2, 4>), grid, dim3(512), 0, stream, A, W, e, M, N, K);
+  }
   if constexpr (EPI != EPI_QKV && EPI != EPI_PART) {      // (plain_tile: whole products only)
     if (kind == TILE_64x96)
       hipLaunchKernelGGL((gemm_bf16_tiled<64, 96, 64, 1, 3, EPI>), grid, dim3(192), 0, stream, A, W, e, M, N, K);

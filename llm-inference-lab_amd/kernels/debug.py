@@ -130,7 +130,8 @@ class KernelDebug:
               attention_one_launch: Optional[int] = None, attention_small_tiles: Optional[int] = None,
               f32_fma: Optional[bool] = None, **rules):
         """``gemm_tile``: 64 (64 x 64), 130 (64 x 128), 129 (128 x 128), 131 (128 x 256), 132 (256 x
-        256), 133 (192 x 256), 134 / 135 / 136 (64 x 96 / 160 / 224) or 137 (128 x 160); -131: the choice among the first three; -256 and below: the
+        256), 133 (192 x 256), 134 / 135 / 136 (64 x 96 / 160 / 224), 137 (128 x 160) or 138 / 139 / 140 (128 x 128, 128 x 192,
+        192 x 128 by direct loads, eight waves); -131: the choice among the first three; -256 and below: the
         tiles of two groups of waves (132, 133) from so many rows on.  ``skinny_shape``:
         (strips per block, K slices, staged rows 0/1 or -1, rows per tile) of the few-row
         product kernel, 0 = chosen by the kernel.  ``skinny_epilogue``: the force holds for

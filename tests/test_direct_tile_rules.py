@@ -1,0 +1,39 @@
+"""Which products the tiles of eight waves by direct loads take over from the tile that was named for them (here without a
+GPU): the measured ones, and over sizes drawn at random only where all their blocks find a place at once."""
+import random
+
+import pytest
+
+from test_dispatch_rules import core      # noqa: F401 (fixture)
+
+UNITS = 256
+SHAPES = {10: (128, 128), 11: (128, 192), 12: (192, 128)}
+
+
+@pytest.mark.parametrize("kind,m,n,k,pieces,want", [
+    # (us before / with it: csrc/gemm.hip)
+    (1, 384, 9728, 896, 1, 10), (1, 256, 11008, 2048, 1, 10), (1, 2048, 896, 4864, 2, 10), (2, 457, 3584, 18944, 2, 10),
+    (1, 512, 9728, 896, 1, 12), (1, 1024, 4864, 896, 1, 12), (5, 1900, 9728, 896, 1, 12), (5, 900, 17920, 1536, 1, 12),
+    (1, 640, 9728, 896, 1, 11), (1, 256, 17920, 1536, 1, 11),
+    (5, 1024, 17920, 1536, 1, -1), (5, 384, 37888, 3584, 1, -1), (1, 64, 896, 4864, 2, -1), (0, 512, 896, 896, 1, -1),
+    (4, 2048, 37888, 3584, 1, -1), (1, 384, 9728, 2 ** 22 + 8, 1, -1),
+])
+def test_measured(core, kind, m, n, k, pieces, want):      # noqa: F811
+    assert core.llmlab_direct_tile(kind, m, n, k, pieces, 0) == want
+
+
+def test_only_where_their_blocks_find_a_place(core):      # noqa: F811
+    rng, seen = random.Random(11), set()
+    for _ in range(20000):
+        kind, heads = rng.randint(0, 5), rng.randint(0, 1)
+        m, n, k = rng.randint(1, 3000), rng.randint(1, 40000), 8 * rng.randint(1, 2500)
+        pieces = rng.choice([1, 1, 2, 4, 8])
+        tile = core.llmlab_direct_tile(kind, m, n, k, pieces, heads)
+        if tile < 0:
+            continue
+        seen.add((kind, tile))
+        bm, bn = SHAPES[tile]
+        blocks = -(-m // bm) * -(-n // bn) * pieces
+        assert m > 64 and (not heads or tile == 10)
+        assert blocks <= UNITS or (kind == 5 and pieces == 1 and k <= 2048), (kind, m, n, k, pieces, tile)
+    assert seen == {(1, 10), (2, 10), (1, 11), (1, 12), (5, 12)}
