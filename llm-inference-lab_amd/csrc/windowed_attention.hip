@@ -679,6 +679,9 @@ static int g_force_plain = 0;      // tests and measurements: no matrix-core ker
 extern "C" void llmlab_debug_windowed_attention_plain(int on) { g_force_plain = on; }
 static int g_private_tiles = 0;    // tests and measurements: prompts by the kernel whose waves fetch their own tiles
 extern "C" void llmlab_debug_windowed_attention_private_tiles(int on) { g_private_tiles = on; }
+// ... and 1 or 2 groups of waves a block in the kernel that shares tiles (0: by the rule)
+static int g_groups = 0;
+extern "C" void llmlab_debug_windowed_attention_groups(int groups) { g_groups = groups; }
 
 // ------------------------------------------------------------------ attention
 // The query at position i of its request attends to the keys i - window < j <= i and to the
@@ -852,6 +855,16 @@ __global__ __launch_bounds__(64) void sink_window_attention_kernel(
   }
 }
 
+// Over the four lanes l, l ^ 16, l ^ 32, l ^ 48 that hold a column's keys, by the lane swaps of gfx950: to the bit what two
+// shuffles give, without their two trips through the LDS crossbar, which every tile's chain had twice (all lanes active).
+template <typename F>
+__device__ __forceinline__ float across_groups(float v, F op) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
+
 // ---- matrix-core kernels (bfloat16; D a multiple of 32, E of 16).  A wave serves 16 queries
 // that share their keys: 16 consecutive rows of the step for one head (prompts), or the
 // heads of one key/value head for one row (decoding: the keys are read once for the group).
@@ -989,8 +1002,7 @@ __device__ __forceinline__ void attend_tiles(const KeyTiles& kt, int t_begin, in
       for (int eb = 0; eb < EB; ++eb)
         run.o[eb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[eb], pf, run.o[eb], 0, 0, 0);
     } else {
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    tmax = across_groups(tmax, [](float x, float y) { return fmaxf(x, y); });
     const float m_new = fmaxf(run.m, tmax);
     const float m_use = m_new == NEG_INF ? 0.f : m_new;
     const float corr = run.m == NEG_INF ? 0.f : __expf(run.m - m_use);
@@ -1003,8 +1015,7 @@ __device__ __forceinline__ void attend_tiles(const KeyTiles& kt, int t_begin, in
         sum += p;
         pf[4 * u + i] = (bf16_t)p;
       }
-    sum += __shfl_xor(sum, 16, WAVE);
-    sum += __shfl_xor(sum, 32, WAVE);
+    sum = across_groups(sum, [](float x, float y) { return x + y; });
     run.l = run.l * corr + sum;
     run.m = m_new;
 #pragma unroll
@@ -1103,17 +1114,21 @@ __global__ __launch_bounds__(256) void sink_window_attention_mfma_kernel(MfmaArg
 // 1,032 keys, 14 heads of 64: 50.5 -> 43.1 us, the same numbers to the bit; a prompt of 1,900 rows from its start, 16 heads of 128
 // over 4 96 -> 87, 12 over 3 with keys of 128 and values of 256 119 -> 113, 12 over 2 of 224 133 -> 121, 16 over 4 of 256 138 -> 129.  (With the running maximum raised only where a
 // score exceeds it by 2^8 and a lane's weights summed by itself 40.0, but a model of sharp scores is then further off.)
-template <int DC, int EB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void sink_window_attention_shared_kernel(MfmaArgs a) {
+template <int DC, int EB, int GROUPS = 1>
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(2))) void sink_window_attention_shared_kernel(MfmaArgs a) {
   constexpr int D = 32 * DC, E = 16 * EB;
   constexpr int KROW = D + 8, VROW = 4 * E + 64;
   constexpr int KCHUNKS = 4 * D, VCHUNKS = 4 * E;            // 16-byte pieces of a tile's keys / values
   constexpr int KCH = (KCHUNKS + 255) / 256, VCH = (VCHUNKS + 255) / 256;
   constexpr int KSTAGE = 2 * 16 * KROW, VSTAGE = 2 * 4 * VROW;
   constexpr bool TWO = EB < 14;          // stages of LDS
-  __shared__ __attribute__((aligned(16))) bf16_t ks_all[(TWO ? 2 : 1) * KSTAGE];
-  __shared__ __attribute__((aligned(16))) bf16_t vs_all[(TWO ? 2 : 1) * VSTAGE];
-  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g4 = lane >> 4, wave = tid >> 6;
+  static_assert(GROUPS == 1 || (GROUPS == 2 && TWO), "one or two groups of four waves");
+  constexpr int STAGES = (TWO ? 2 : 1) * (KSTAGE + VSTAGE), SUMS = GROUPS > 1 ? 4 * 64 * (EB * 4 + 2) * 2 : 0;      // (in bf16_t)
+  __shared__ __attribute__((aligned(16))) bf16_t lds_all[GROUPS * STAGES > SUMS ? GROUPS * STAGES : SUMS];
+  const int tid = threadIdx.x & 255, lane = tid & 63, c = lane & 15, g4 = lane >> 4, wave = tid >> 6;
+  const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;      // this wave's group
+  bf16_t* const ks_all = lds_all + grp * STAGES;
+  bf16_t* const vs_all = ks_all + (TWO ? 2 : 1) * KSTAGE;
   const int r0 = blockIdx.x * 16;
   if (r0 >= a.n_rows) return;
   const int group = a.n_heads / a.n_kv, per_group = (group + 3) >> 2;      // blocks a key/value head's heads take
@@ -1135,8 +1150,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   Running<EB> run;
   const bool sig = a.mode == MODE_SIGMOID;
   const float bias = (sig && a.sink) ? a.sink[h] : 0.f;
-  run.m = sig ? 0.f : (a.sink ? a.sink[h] : NEG_INF);
-  run.l = (sig || a.sink) ? 1.f : 0.f;
+  run.m = sig ? 0.f : (a.sink && grp == 0 ? a.sink[h] : NEG_INF);      // (the sink enters the first group only)
+  run.l = (sig || a.sink) && grp == 0 ? 1.f : 0.f;
   // (pages are powers of two in use; any other size is divided by)
   const int page_shift = (a.page_size & (a.page_size - 1)) == 0 ? __builtin_ctz(a.page_size) : -1;
   auto page_of = [&](int j) { return page_shift >= 0 ? j >> page_shift : j / a.page_size; };
@@ -1169,14 +1184,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     // The pages of a tile's two halves are looked up one fetch ahead (a lookup in front of its own loads
     // is a trip to memory that every tile would wait for).
     int page[2];
-    auto look_up = [&](int t) {
+    // (the group's u-th tile: every GROUPS-th of them)
+    auto look_up = [&](int u0) {
+      const int t = u0 * GROUPS + grp;
       const int j0 = t < kt.tiles_a ? 32 * t : kt.b_start + 32 * (t - kt.tiles_a);
       const int end = t < kt.tiles_a ? kt.a_end : kt.end_b;
 #pragma unroll
       for (int u = 0; u < 2; ++u) page[u] = j0 + 16 * u < end ? pages[page_of(j0 + 16 * u)] : 0;
     };
     // the 16-byte pieces of tile t that this thread brings (tiles are fetched in their order)
-    auto fetch = [&](int t, bf16x8 (&kreg)[KCH], bf16x8 (&vreg)[VCH]) {
+    const int T = (kt.tiles - grp + GROUPS - 1) / GROUPS, T_most = (kt.tiles + GROUPS - 1) / GROUPS;      // (of the group; of any)
+    auto fetch = [&](int u0, bf16x8 (&kreg)[KCH], bf16x8 (&vreg)[VCH]) {
+      const int t = u0 * GROUPS + grp;
       const int j0 = t < kt.tiles_a ? 32 * t : kt.b_start + 32 * (t - kt.tiles_a);
       const int end = t < kt.tiles_a ? kt.a_end : kt.end_b;
       size_t kbase[2], vbase[2];
@@ -1206,7 +1225,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
         const int u = idx / (2 * E), rem = idx % (2 * E);
         vreg[i] = *(const bf16x8*)(a.v_cache + (u ? vbase[1] : vbase[0]) + (size_t)rem * 8);
       }
-      if (t + 1 < kt.tiles) look_up(t + 1);
+      if (u0 + 1 < T) look_up(u0 + 1);
     };
     auto stash = [&](const bf16x8 (&kreg)[KCH], const bf16x8 (&vreg)[VCH], int stage) {
       bf16_t* const ks = ks_all + stage * KSTAGE;
@@ -1231,7 +1250,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       }
     };
     // tile t, which lies in LDS, into the running softmax
-    auto attend = [&](int t, int stage) {
+    auto attend = [&](int u0, int stage) {
+      const int t = u0 * GROUPS + grp;
       const bf16_t* const ks = ks_all + stage * KSTAGE;
       const bf16_t* const vs = vs_all + stage * VSTAGE;
       const int j0 = t < kt.tiles_a ? 32 * t : kt.b_start + 32 * (t - kt.tiles_a);
@@ -1277,8 +1297,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
 #pragma unroll
           for (int i = 0; i < 4; ++i) pf[4 * u + i] = (bf16_t)sigmoid_weight(s[u][i] + bias);      // (masked: -inf -> 0)
       } else {
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+        tmax = across_groups(tmax, [](float x, float y) { return fmaxf(x, y); });
         const float m_new = fmaxf(run.m, tmax);
         const float m_use = m_new == NEG_INF ? 0.f : m_new;
         corr = run.m == NEG_INF ? 0.f : __expf(run.m - m_use);
@@ -1291,8 +1310,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
             sum += p;
             pf[4 * u + i] = (bf16_t)p;
           }
-        sum += __shfl_xor(sum, 16, WAVE);
-        sum += __shfl_xor(sum, 32, WAVE);
+        sum = across_groups(sum, [](float x, float y) { return x + y; });
         run.l = run.l * corr + sum;
         run.m = m_new;
       }
@@ -1310,25 +1328,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
         run.o[eb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, run.o[eb], 0, 0, 0);
       }
     };
-    const int T = kt.tiles;
     __syncthreads();                                  // (the request before this one has been read)
-    look_up(0);
-    fetch(0, k_a, v_a);
-    stash(k_a, v_a, 0);
+    if (GROUPS == 1 || T > 0) {
+      look_up(0);
+      fetch(0, k_a, v_a);
+      stash(k_a, v_a, 0);
+    }
     if constexpr (TWO) {
       if (T > 1) fetch(1, k_a, v_a);
       if (T > 2) fetch(2, k_b, v_b);
-      for (int t = 0; t < T; t += 2) {
+      for (int t = 0; t < T_most; t += 2) {
         // tile t lies in stage 0, tiles t + 1 and t + 2 are on their way into sets a and b
         __syncthreads();                              // (tile t is whole, tile t - 1 has been read)
         if (t + 1 < T) stash(k_a, v_a, 1);
         if (t + 3 < T) fetch(t + 3, k_a, v_a);
-        attend(t, 0);
-        if (t + 1 >= T) break;
+        if (GROUPS == 1 || t < T) attend(t, 0);
+        if (t + 1 >= T_most) break;
         __syncthreads();
         if (t + 2 < T) stash(k_b, v_b, 0);
         if (t + 4 < T) fetch(t + 4, k_b, v_b);
-        attend(t + 1, 1);
+        if (GROUPS == 1 || t + 1 < T) attend(t + 1, 1);
       }
     } else {
       // (values of 224 and more: the registers hold one tile on its way, and it is put down when the one
@@ -1340,6 +1359,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
         __syncthreads();                              // (every wave has read it)
         if (t + 1 < T) stash(k_a, v_a, 0);
       }
+    }
+  }
+  if constexpr (GROUPS > 1) {
+    // the second group's sums to the first, lane to lane:  o = e^(m0 - m) o0 + e^(m1 - m) o1,  l likewise,  m = max(m0, m1)
+    floatx4* const sums = (floatx4*)lds_all;                  // [wave][piece][lane], then the maxima and denominators
+    float* const s_m = (float*)(sums + 4 * EB * 64) + wave * 128 + lane;
+    __syncthreads();                                          // (every stage has been read)
+    if (grp > 0) {
+      s_m[0] = run.m;
+      s_m[64] = run.l;
+#pragma unroll
+      for (int eb = 0; eb < EB; ++eb) sums[(wave * EB + eb) * 64 + lane] = run.o[eb];
+    }
+    __syncthreads();
+    if (grp > 0) return;
+    const float m1 = s_m[0], m = fmaxf(run.m, m1);
+    const float w0 = run.m == NEG_INF ? 0.f : __expf(run.m - m), w1 = m1 == NEG_INF ? 0.f : __expf(m1 - m);
+    run.l = run.l * w0 + s_m[64] * w1;
+#pragma unroll
+    for (int eb = 0; eb < EB; ++eb) {
+      const floatx4 o1 = sums[(wave * EB + eb) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) run.o[eb][i] = run.o[eb][i] * w0 + o1[i] * w1;
     }
   }
   if (!row_ok || !head_ok) return;
@@ -1496,12 +1538,20 @@ extern "C" int llmlab_sink_window_attention_has_mfma(int dtype, int D, int E, in
   return (D <= 128 && E <= 128) || (D >= 64 && D <= 128 && (E == 192 || E == 256)) || (D == E && D <= 256);
 }
 
+// (heads up to 128: wider ones' registers and stages do not fit)
+template <int DC, int EB>
+static void launch_two_groups(dim3 grid, hipStream_t stream, const MfmaArgs& a) {
+  if constexpr (DC <= 4 && EB <= 8)
+    hipLaunchKernelGGL((sink_window_attention_shared_kernel<DC, EB, 2>), grid, dim3(512), 0, stream, a);
+}
+
 template <int DC>
 static void launch_mfma(int EBv, int which, dim3 grid, dim3 block, hipStream_t stream, const MfmaArgs& a) {
 #define LLMLAB_MFMA(EBC)                                                                                      \
   case EBC:                                                                                                   \
     if (which == 0) hipLaunchKernelGGL((sink_window_attention_mfma_kernel<DC, EBC>), grid, block, 0, stream, a); \
     else if (which == 2) hipLaunchKernelGGL((sink_window_attention_shared_kernel<DC, EBC>), grid, block, 0, stream, a); \
+    else if (which == 3) launch_two_groups<DC, EBC>(grid, stream, a);                                           \
     else hipLaunchKernelGGL((sink_window_attention_grouped_kernel<DC, EBC>), grid, block, 0, stream, a);      \
     break;
   switch (EBv) {
@@ -1531,6 +1581,17 @@ static void launch_mfma_any(int D, int E, int which, dim3 grid, dim3 block, hipS
     case 3: launch_mfma<3>(E / 16, which, grid, block, stream, a); break;
     default: launch_mfma<4>(E / 16, which, grid, block, stream, a); break;
   }
+}
+
+// Whether a block that shares its tiles has two groups of four waves, each with every second tile and stages of its own,
+// whose sums meet at the end: a block's chain of tiles is half as long, and a unit holds fewer blocks.  One group / two, us:
+// heads of 64 (14 over 2), 512 rows (128 blocks) 18.8 / 14.5, 1,000 (252) 32.7 / 24.2, 1,900 over a window of 1,024 (476) 41.6 / 35.0,
+// three prompts of 2,367 rows (592) 39.8 / 33.2, 4,096 (1,024) 58.7 / 64.6; of 128 (16 over 2), 64 rows 7.3 / 7.6, 200 12.5 / 11.3, 1,000 (252)
+// 40.5 / 30.1, 1,900 (476) 51.2 / 60.1: their registers let a unit hold one block of two groups.
+static bool two_groups(int D, int E, int rows, long blocks, int num_cus) {
+  if (num_cus <= 0) num_cus = 256;
+  if (D <= 64 && E <= 64) return 2 * blocks <= 5L * num_cus;
+  return rows >= 96 && blocks <= num_cus;
 }
 
 // q [rows, heads * D], out [rows, heads * E] in the compute dtype; sink: float32 [heads] or null.
@@ -1572,8 +1633,11 @@ extern "C" int llmlab_sink_window_attention(const void* q, int dtype, int rows, 
     if (launches & 2) {
       // heads that read the same keys and values share the tiles a block stages in LDS
       const int group = n_heads / n_kv;
+      const long blocks = (long)((rows + 15) / 16) * n_kv * ((group + 3) / 4);
+      const bool fit = D <= 128 && E <= 128;
       if (!g_private_tiles && group >= 3)
-        launch_mfma_any(D, E, 2, dim3((rows + 15) / 16, n_kv * ((group + 3) / 4)), dim3(256), stream, a);
+        launch_mfma_any(D, E, fit && (g_groups > 0 ? g_groups == 2 : two_groups(D, E, rows, blocks, num_cus)) ? 3 : 2,
+                        dim3((rows + 15) / 16, n_kv * ((group + 3) / 4)), dim3(256), stream, a);
       else
         launch_mfma_any(D, E, 0, dim3((rows + 63) / 64, n_heads), dim3(256), stream, a);
       LLMLAB_LAUNCH_CHECK("sink_window_attention (prompts)");
