@@ -33,31 +33,48 @@ __device__ __forceinline__ float log_decay_of(float z, int kind, float inv_tau) 
   return -(fmaxf(u, 0.f) + log1pf(expf(-fabsf(u)))) * inv_tau;
 }
 __device__ __forceinline__ float decay_of(float z, int kind, float inv_tau) { return expf(log_decay_of(z, kind, inv_tau)); }
-__global__ __launch_bounds__(256) void gla_decay_kernel(const float* __restrict__ low, int ld, int rank,
+// ROWS rows and 256 channels a block, a thread a channel.  What bounds it is a thread's chain (its row of the second factor,
+// the sum, the logarithm) and, of many rows, that every block reads the second factor again: 1,900 rows of 448 channels and rank
+// 32 with one / two / four / eight rows a block 15.8 / 9.8 / 8.5 / 9.6 us (16.5 with one and all channels a block), 512 rows 6.0 / 5.0 /
+// 5.0 / 7.1, 16 rows 4.3 / 4.0 / 4.7 / 6.8 (5.1).  A number's sum has the same order.
+template <int ROWS>
+__global__ __launch_bounds__(256) void gla_decay_kernel(const float* __restrict__ low, int ld, int rows, int rank,
                                                         const float* __restrict__ w2, const float* __restrict__ bias,
                                                         int kind, float inv_tau, float* __restrict__ decay, int channels,
                                                         int as_log) {
-  extern __shared__ float s_low[];
-  const int r = blockIdx.x;
-  const float* t = low + (size_t)r * ld;
-  for (int j = threadIdx.x; j < rank; j += blockDim.x) s_low[j] = kind == DECAY_DOUBLE_EXP ? tanhf(t[j]) : t[j];
+  extern __shared__ __attribute__((aligned(16))) float s_low[];      // [rank][ROWS]
+  const int r0 = blockIdx.x * ROWS;
+  for (int i = threadIdx.x; i < rank * ROWS; i += blockDim.x) {
+    const int k = i / rank, j = i - k * rank;
+    const float t = low[(size_t)min(r0 + k, rows - 1) * ld + j];
+    s_low[j * ROWS + k] = kind == DECAY_DOUBLE_EXP ? tanhf(t) : t;
+  }
   __syncthreads();
-  for (int c = threadIdx.x; c < channels; c += blockDim.x) {
-    float z = bias ? bias[c] : 0.f;
+  const int c = blockIdx.y * 256 + threadIdx.x;
+  if (c < channels) {
+    float z[ROWS];
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k) z[k] = bias ? bias[c] : 0.f;
     const float* w = w2 + (size_t)c * rank;
     if ((rank & 3) == 0) {                       // (a row of the second factor 16 bytes a load, all on their way together)
       for (int j = 0; j < rank; j += 4) {
         const floatx4 w4 = *(const floatx4*)(w + j);
-        z = fmaf(w4[0], s_low[j], z);
-        z = fmaf(w4[1], s_low[j + 1], z);
-        z = fmaf(w4[2], s_low[j + 2], z);
-        z = fmaf(w4[3], s_low[j + 3], z);
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int k = 0; k < ROWS; ++k) z[k] = fmaf(w4[x], s_low[(j + x) * ROWS + k], z[k]);
       }
     } else {
-      for (int j = 0; j < rank; ++j) z = fmaf(w[j], s_low[j], z);
+      for (int j = 0; j < rank; ++j)
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k) z[k] = fmaf(w[j], s_low[j * ROWS + k], z[k]);
     }
-    const float lg = log_decay_of(z, kind, inv_tau);
-    decay[(size_t)r * channels + c] = as_log ? fmaxf(lg * LOG2_E, LOG_FLOOR) : expf(lg);
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k) {
+      if (r0 + k >= rows) break;
+      const float lg = log_decay_of(z[k], kind, inv_tau);
+      decay[(size_t)(r0 + k) * channels + c] = as_log ? fmaxf(lg * LOG2_E, LOG_FLOOR) : expf(lg);
+    }
   }
 }
 
@@ -68,8 +85,15 @@ extern "C" int llmlab_gla_decay(const float* low, int ld, int rows, int rank, co
                  "gla_decay: bad sizes rows=%d rank=%d channels=%d ld=%d kind=%d tau=%g", rows, rank, channels, ld, kind,
                  (double)tau);
   if (rows == 0) return 0;
-  hipLaunchKernelGGL(gla_decay_kernel, dim3(rows), dim3(256), rank * sizeof(float), stream, low, ld, rank, w2, bias, kind,
-                     1.0f / tau, decay, channels, as_log);
+  const unsigned chunks = (unsigned)((channels + 255) / 256);
+  auto launch = [&](auto kernel, int per) {
+    hipLaunchKernelGGL(kernel, dim3((rows + per - 1) / per, chunks), dim3(256), rank * per * sizeof(float), stream, low, ld, rows,
+                       rank, w2, bias, kind, 1.0f / tau, decay, channels, as_log);
+  };
+  const long blocks = (long)rows * chunks;
+  if (blocks <= 512 || rank > 1024) launch(gla_decay_kernel<1>, 1);      // (ranks beyond: LDS)
+  else if (blocks <= 1400) launch(gla_decay_kernel<2>, 2);
+  else launch(gla_decay_kernel<4>, 4);
   LLMLAB_LAUNCH_CHECK("gla_decay");
   return 0;
 }
