@@ -95,8 +95,19 @@ struct AttnArgs {
   int reqs, picked;   // picked > 0: block z of the launch is for the z-th of the `reqs` requests that bring
                       // so many tokens, of which there are `picked`; 0: block z is for request z, and ends at
                       // once if that brings another number of tokens
+  int units;          // compute units of the chip
   float scale;
 };
+
+// Which tile block `number` of `total` takes, tiles counted from the longest histories on, where a unit holds `slots` blocks
+// at a time: the first block of every unit in their order, the second in the opposite one and so on, so that what a unit
+// starts with is about the same load on all units; the others, which start where a place is free first, in their order again.
+__device__ __forceinline__ int rank_of(int number, int total, int units, int slots) {
+  const int round = number / units;
+  if (!(round & 1) || round >= slots) return number;
+  const int first = round * units, last = min(first + units, total) - 1;
+  return first + last - number;
+}
 
 // The request of block z of a launch: of a step of both kinds of requests, whose launch has blocks for one
 // kind only, the z-th that brings qlen_lo to qlen_hi tokens (-1: there are fewer).  All waves of a block call
@@ -1338,13 +1349,34 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void attention_merge_kernel(
 // waves of a block share one tile and split its keys, merge through LDS (all other steps of
 // many rows), and blockIdx.y also counts splits over blocks whose partial results the merge
 // kernel sums (decode steps).
+// Heads up to 64 in blocks of four waves (`f32_lean`) keep one step of keys and values in registers and ask for the next keys
+// behind the scores, for the next values behind the second product: a SIMD has four waves, and a unit four blocks, whose
+// first trips to memory and merges pass behind each other's products.  What bounds it: the matrix cores in float32 (141 TFLOP/s
+// measured in a loop of such products alone: 30 us for a prompt of 1,531 of 14 heads), and 6 us of launch, first trips
+// and merge.  Against tiles of 32 rows by eight waves, two steps in registers and a maximum exchanged every step (us): that
+// prompt 65.7 -> 47.2, one of 8,000 1,213 -> 1,024, of 150 10.6 -> 6.2, three of 700 to 500 46.7 -> 30.1, 8 of up to 512 79 -> 40,
+// 100 tokens behind 3,000 keys 72 -> 36; the prompt's error against 64 bits
+// 2.60e-7 -> 2.55e-7.  Tiles of 32 rows in the lean form: 49.4 to 49.7 for the first, 38.6 (here 30.9) for 512 behind
+// 1,000; five waves a SIMD spill registers.
+constexpr bool f32_lean(bool split, int waves) { return split && waves == 4 && D <= 64; }
 template <int QB, bool SPLIT, int NW>
-__global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
+__global__ __launch_bounds__(64 * NW, f32_lean(SPLIT, NW) ? 4 : 1) void attention_f32_kernel(AttnArgs a) {
+  constexpr bool LEAN = f32_lean(SPLIT, NW);
   constexpr int DQ = D / 16;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int b = request_of(a, (int)blockIdx.z);
+  // Along x, the tiles with the longest histories of all kv heads and requests come first (where they share x: more blocks
+  // than x takes, or decode steps, lie along x, y and z).
+  int tiles = gridDim.x, from_last = blockIdx.x, column = blockIdx.y, z = blockIdx.z;
+  if (SPLIT && gridDim.y == 1 && gridDim.z == 1) {
+    const int per = a.nkv * (a.picked > 0 ? a.picked : a.reqs), rank = rank_of(from_last, tiles, a.units, 16 / NW);
+    tiles /= per;
+    from_last = rank / per;
+    column = rank % per % a.nkv * a.splits;
+    z = rank % per / a.nkv;
+  }
+  const int b = request_of(a, z);
   if (b < 0) return;
   // (a short row of the block table as a whole, see the bfloat16 kernel)
   constexpr int TAB = SPLIT ? 2 : 1;
@@ -1354,13 +1386,12 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
 #pragma unroll
     for (int i = 0; i < TAB; ++i) tab[i] = a.table[(size_t)b * a.table_stride + min(i * 64 + lane, a.table_stride - 1)];
   }
-  const int kvh = blockIdx.y / a.splits, split = blockIdx.y % a.splits;
+  const int kvh = column / a.splits, split = column % a.splits;
   const int G = a.nq / a.nkv;
   const int r0 = a.q_start[b], qlen = a.q_start[b + 1] - r0, sp = a.start_pos[b];
   const int rows_total = qlen * G;
   if (qlen < a.qlen_lo || qlen > a.qlen_hi) return;                  // another launch's request
-  // tiles with the longest histories (the last rows) first
-  const int xblk = (int)(gridDim.x - 1 - blockIdx.x);
+  const int xblk = tiles - 1 - from_last;
   const int row0 = (SPLIT ? xblk : xblk * NW + wave) * (16 * QB);
   if (row0 >= rows_total) {
     if (!SPLIT || xblk * 16 * QB >= rows_total) return;              // (without SPLIT no wave waits for another)
@@ -1385,9 +1416,17 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
     lo[qb] = a.window > 0 ? max(0, pos[qb] - a.window + 1) : 0;
     const float* qp = q + (size_t)(r0 + tok[qb]) * a.q_stride + (size_t)head[qb] * D + g * 4;
 #pragma unroll
-    for (int mb = 0; mb < DQ; ++mb)
-      qf[qb][mb] = valid[qb] ? *(const floatx4*)(qp + mb * 16) : floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < DQ; ++mb) qf[qb][mb] = *(const floatx4*)(qp + mb * 16);
   }
+  // (the rows past the end read the first one: a load under a condition would be waited for where it stands)
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int mb = 0; mb < DQ; ++mb) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) qf[qb][mb][t] = valid[qb] ? qf[qb][mb][t] : 0.f;
+      asm volatile("" : "+v"(qf[qb][mb]));      // (waited for here: in the loop it would be, in every step, with all that is on its way)
+    }
   const int last_row = min(row0 + 16 * QB, rows_total) - 1;
   const int p_first = sp + row0 / G, p_last = sp + last_row / G;
   const int key_lo = a.window > 0 ? max(0, p_first - a.window + 1) : 0;
@@ -1403,69 +1442,103 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
     my1 = min(my0 + per_wave, my1);
   }
 
-  floatx4 o[QB][DQ];
-  float m[QB], lsum[QB];
+  // (the lean form has a second set of sums, for every other step: a wave's sums are as short as those of eight waves)
+  constexpr int SETS = LEAN ? 2 : 1;
+  floatx4 o_set[SETS][QB][DQ];
+  float m[QB], l_set[SETS][QB];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     m[qb] = NEG_INF;
-    lsum[qb] = 0.f;
 #pragma unroll
-    for (int mb = 0; mb < DQ; ++mb) o[qb][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int set = 0; set < SETS; ++set) {
+      l_set[set][qb] = 0.f;
+#pragma unroll
+      for (int mb = 0; mb < DQ; ++mb) o_set[set][qb][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
   }
+  floatx4 (&o)[QB][DQ] = o_set[0];
+  float (&lsum)[QB] = l_set[0];
 
   struct Step {
     floatx4 k[DQ], v[DQ];
     bool ok;
   };
-  auto compute = [&](int blk, const Step& f) {
-    if (!f.ok) return;                      // (the same for the whole wave)
+  auto scores = [&](const Step& f, floatx4 (&sc)[QB]) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) sc[qb] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mb = 0; mb < DQ; ++mb)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+          sc[qb] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[mb][t], qf[qb][mb][t], sc[qb], 0, 0, 0);
+  };
+  auto finish = [&](int blk, Step& f, floatx4 (&sc)[QB], floatx4 (&o)[QB][DQ], float (&lsum)[QB]) {
     const int kb = blk << 4;
-    const bool all_visible = kb + 15 <= p_first && kb >= full_lo;
-    const bool tail = kb + 15 > key_hi;
+    if (!(kb + 15 <= p_first && kb >= full_lo)) {      // some of the keys are not for every row
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = kb + g * 4 + i;
+          sc[qb][i] = valid[qb] && j <= pos[qb] && j >= lo[qb] ? sc[qb][i] : NEG_INF;
+        }
+      // (a position past the last one written holds whatever was there: kept out of
+      // the product although its weight is zero)
+      if (kb + 15 > key_hi)
+#pragma unroll
+        for (int mb = 0; mb < DQ; ++mb)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) f.v[mb][u] = kb + g * 4 + u > key_hi ? 0.f : f.v[mb][u];
+    }
+    // The running maximum, in units of the binary exponent (score * scale * log2 e, the scale is positive), is raised
+    // only where some score stands out by more than LAZY_MAX, as in bfloat16: what is summed is then
+    // as exact, since a float32 keeps its digits at any size.
+    float mx[QB];
+    bool grows = false;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-      floatx4 sc = {0.f, 0.f, 0.f, 0.f};
+      mx[qb] = max_raw(max3_raw(sc[qb][0], sc[qb][1], sc[qb][2]), sc[qb][3]) * scale2;
+      grows |= mx[qb] > m[qb] + LAZY_MAX;
+    }
+    if (__any(grows)) {                     // some row's maximum grew: rescale what is summed so far
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const float top = max_across_16(max_across_32(mx[qb]));
+        const bool grow = top > m[qb] + LAZY_MAX;
+        const float alpha = grow ? fast_exp2(m[qb] - top) : 1.f;      // 2^-inf = 0 the first time
+#pragma unroll
+        for (int set = 0; set < SETS; ++set) {
+          l_set[set][qb] *= alpha;
+#pragma unroll
+          for (int mb = 0; mb < DQ; ++mb) o_set[set][qb][mb] *= alpha;
+        }
+        m[qb] = grow ? top : m[qb];
+      }
+    }
+    // the exponentials by the hardware's 2^x (one unit in the last place; a softmax asks no more of them)
+    float pv[QB][4];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      const float from = m[qb] == NEG_INF ? 0.f : m[qb];      // (no visible key yet: every p of the row is 2^-inf = 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pv[qb][i] = fast_exp2(sc[qb][i] * scale2 - from);
+      lsum[qb] += (pv[qb][0] + pv[qb][1]) + (pv[qb][2] + pv[qb][3]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int mb = 0; mb < DQ; ++mb)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          sc = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[mb][t], qf[qb][mb][t], sc, 0, 0, 0);
-      // scores in units of the binary exponent (score * scale * log2 e); the exponentials by
-      // the hardware's 2^x (one unit in the last place; a softmax asks no more of them)
-      float sv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = kb + g * 4 + i;
-        const bool vis = all_visible || (valid[qb] && j <= pos[qb] && j >= lo[qb]);
-        sv[i] = vis ? sc[i] * scale2 : NEG_INF;
-      }
-      float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-      mx = max_across_32(mx);
-      mx = max_across_16(mx);
-      const float m_new = fmaxf(m[qb], mx);
-      if (__any(m_new != m[qb])) {        // some row's maximum grew: rescale what is summed so far
-        // (nothing visible yet, m_new = -inf: the sums are 0 and stay 0)
-        const float alpha = m_new == NEG_INF ? 1.f : fast_exp2(m[qb] - m_new);
-        lsum[qb] *= alpha;
-#pragma unroll
-        for (int mb = 0; mb < DQ; ++mb) o[qb][mb] *= alpha;
-        m[qb] = m_new;
-      }
-      float pv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) pv[i] = sv[i] == NEG_INF ? 0.f : fast_exp2(sv[i] - m_new);
-      lsum[qb] += (pv[0] + pv[1]) + (pv[2] + pv[3]);
-#pragma unroll
-      for (int mb = 0; mb < DQ; ++mb) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          // (a position past the last one written holds whatever was there: kept out of
-          // the product although its weight is zero)
-          const float vv = (tail && kb + g * 4 + u > key_hi) ? 0.f : f.v[mb][u];
-          o[qb][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv, pv[u], o[qb][mb], 0, 0, 0);
-        }
-      }
-    }
+        for (int qb = 0; qb < QB; ++qb)
+          o[qb][mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.v[mb][u], pv[qb][u], o[qb][mb], 0, 0, 0);
+  };
+  auto compute = [&](int blk, Step& f) {
+    if (!f.ok) return;                      // (the same for the whole wave)
+    floatx4 sc[QB];
+    scores(f, sc);
+    finish(blk, f, sc, o, lsum);
   };
 
   // The next steps' keys and values are on their way while this one is multiplied; the
@@ -1493,19 +1566,51 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
       }
       pages_v = in ? pg : -1;
     }
-    auto fetch = [&](int blk, Step& f) {
+    auto find = [&](int blk, bool& ok) {       // where step `blk` lies in the cache
       const int bl = min(blk, ce - 1);
       const int page = __builtin_amdgcn_readlane(pages_v, bl - cb);
-      f.ok = blk < ce && page >= 0;
-      const size_t base = ((size_t)max(page, 0) * a.nkv + kvh) * P * D + (size_t)(((bl << 4) & (P - 1)) >> 4) * (16 * D);
+      ok = blk < ce && page >= 0;
+      return ((size_t)max(page, 0) * a.nkv + kvh) * P * D + (size_t)(((bl << 4) & (P - 1)) >> 4) * (16 * D);
+    };
+    auto fetch_keys = [&](size_t base, Step& f) {
       const float* kp = kc + base + (size_t)((g >> 1) * 16 + c) * 8 + 4 * (g & 1);
+#pragma unroll
+      for (int mb = 0; mb < DQ; ++mb) f.k[mb] = *(const floatx4*)(kp + mb * 256);      // two octets of d further
+    };
+    auto fetch_values = [&](size_t base, Step& f) {
       const float* vp = vc + base + (size_t)(g * 16 + c) * 4;
 #pragma unroll
-      for (int mb = 0; mb < DQ; ++mb) {
-        f.k[mb] = *(const floatx4*)(kp + mb * 256);      // two octets of d further
-        f.v[mb] = *(const floatx4*)(vp + mb * 256);      // the next 16-wide block of d
-      }
+      for (int mb = 0; mb < DQ; ++mb) f.v[mb] = *(const floatx4*)(vp + mb * 256);      // the next 16-wide block of d
     };
+    auto fetch = [&](int blk, Step& f) {
+      const size_t base = find(blk, f.ok);
+      fetch_keys(base, f);
+      fetch_values(base, f);
+    };
+    if constexpr (LEAN) {
+      // Keys and values of one step in registers: the next step's keys are asked for behind the scores, its values
+      // behind the second product.  So few registers that a SIMD has four waves, which fill each other's waits.
+      Step f;
+      fetch(cb, f);
+      auto step = [&](int blk, int set) {
+        const bool ok = f.ok;                 // (the same for the whole wave)
+        const size_t next = find(blk + 1, f.ok);
+        floatx4 sc[QB];
+        scores(f, sc);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_keys(next, f);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ok) finish(blk, f, sc, o_set[set], l_set[set]);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_values(next, f);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      for (int blk = cb; blk < ce; blk += 2) {
+        step(blk, 0);
+        if (blk + 1 < ce) step(blk + 1, SETS - 1);
+      }
+      continue;
+    }
     // a ring of three: two steps are on their way while one is multiplied (a wave's step is
     // about a microsecond of matrix instructions, a trip to memory takes longer, and a
     // prompt gives a SIMD fewer than two waves to fill the wait with)
@@ -1536,6 +1641,14 @@ __global__ __launch_bounds__(64 * NW) void attention_f32_kernel(AttnArgs a) {
     }
   }
 
+  if constexpr (SETS == 2) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      lsum[qb] += l_set[SETS - 1][qb];
+#pragma unroll
+      for (int mb = 0; mb < DQ; ++mb) o[qb][mb] += o_set[SETS - 1][qb][mb];
+    }
+  }
   if constexpr (!SPLIT) {
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -1770,8 +1883,10 @@ static int choose_many_rows_launch_f32(long blocks, int max_q_len, int max_ctx_l
   // 184, of 2,048 453 against 512, two of 1,024 290 against 305; four of 1,024 562 against 501)
   if (D > 64) few_keys = blocks > (max_q_len >= 1024 ? 7L : 2L) * num_cus ? 0x7fffffff
                          : blocks >= (7L * num_cus) / 4 && max_q_len < 1024 ? 128 : 0;
-  else few_keys = blocks >= 14L * num_cus ? 1024 : blocks >= 7L * num_cus ? 768 : blocks >= (7L * num_cus) / 2 ? 256
-                  : blocks >= (7L * num_cus) / 4 ? 128 : 0;
+  // (heads of 64: the key split takes 16 rows a block and loses only over a step or two of keys a wave, and where there are
+  // tiles for many rounds over few keys: 60 / 24 prompts of 128 tokens 46 / 21 us against 40 / 23, 100 / 40 of 64 33 / 16 against
+  // 31 / 17, 16 of 272 to 512 83 against 74; 32 of 200 46 both, 14 of 512 84 against 115, 8 of 1,000 151 against 191)
+  else few_keys = blocks >= 14L * num_cus ? 512 : blocks >= 10L * num_cus ? 128 : blocks >= (7L * num_cus) / 4 ? 64 : 0;
   return max_ctx_len <= few_keys ? 2 : 1;
 }
 
@@ -1801,18 +1916,27 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
   const unsigned zs = a.picked > 0 ? a.picked : reqs;
   constexpr int ROWS = 16 * F32_QB;
   const long tiles = (max_rows + ROWS - 1) / ROWS;
-  // Which launch, from a sweep of 1 to 32 requests of 64 to 8,192 tokens behind 0 to 4,096 keys
+  // Which launch, from a sweep of 1 to 100 requests of 32 to 8,192 tokens behind 0 to 4,096 keys
   // (14 heads of 64 over 2, 28 of 128 over 4).  A block whose waves split the keys of a tile
   // (1) wins wherever a wave per tile (2) would leave compute units idle or walk a long
-  // history alone: 512 tokens behind 1,024 keys at heads of 64 take 43 us so and 162 with a
-  // wave per tile, a prompt of 2,048 tokens 117 against 217.  A wave per tile wins once the
-  // tiles fill the chip and the keys are few (16 requests of 512 tokens from their start,
-  // heads of 64: 137 us against 187), at heads above 64 from two tiles a unit on whatever the
+  // history alone: 512 tokens behind 1,024 keys at heads of 64 take 31 us so and 120 with a
+  // wave per tile, a prompt of 1,531 tokens 49 against 122.  A wave per tile wins once the
+  // tiles fill the chip and the keys are few, at heads above 64 from two tiles a unit on whatever the
   // keys (4 requests of 256 tokens: 58 against 81).
   const int path = choose_many_rows_launch_f32(tiles * a.nkv * live, max_q_len, max_ctx_len, num_cus, g_force_path);
   if (path == 1) {
-    hipLaunchKernelGGL((attention_f32_kernel<F32_QB, true, F32_SPLIT_WAVES>), dim3((unsigned)tiles, a.nkv, zs),
-                       dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
+    // Heads up to 64: blocks of four waves and 16 rows, four to a unit; eight waves where the tiles leave units idle and
+    // have histories to walk (us, four / eight waves: 100 tokens behind 1,000 keys 20.2 / 16.0, behind 3,000 48.5 / 35.5; 300
+    // behind 1,000 (264 tiles) 27.9 / 31; a prompt of 150 6.3 / 7.0).
+    constexpr int PATH1_QB = D <= 64 ? 1 : F32_QB;
+    const long path1_tiles = (max_rows + 16 * PATH1_QB - 1) / (16 * PATH1_QB), blocks = path1_tiles * a.nkv * zs;
+    // (along x, the longest tiles of all requests first, where every request is this launch's)
+    const bool along_x = live == (long)zs && blocks <= 0xffffffffl / (64 * F32_SPLIT_WAVES);
+    const dim3 grid = along_x ? dim3((unsigned)blocks) : dim3((unsigned)path1_tiles, a.nkv, zs);
+    if (D <= 64 && !(path1_tiles * a.nkv * live <= num_cus && max_ctx_len >= 768))
+      hipLaunchKernelGGL((attention_f32_kernel<PATH1_QB, true, 4>), grid, dim3(64 * 4), 0, stream, a);
+    else
+      hipLaunchKernelGGL((attention_f32_kernel<PATH1_QB, true, F32_SPLIT_WAVES>), grid, dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
   } else {
     hipLaunchKernelGGL((attention_f32_kernel<F32_QB, false, 4>), dim3((unsigned)((tiles + 3) / 4), a.nkv, zs),
                        dim3(256), 0, stream, a);
@@ -2049,6 +2173,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
   a.tiles = 0;
   a.qlen_lo = 0; a.qlen_hi = 0x7fffffff;
   a.reqs = reqs; a.picked = 0;
+  a.units = num_cus;
   while ((1 << a.page_shift) < page_size) ++a.page_shift;
   if (dtype == DT_F32)
     return launch_attention_f32(a, reqs, max_q_len, max_ctx_len, window, total_rows, workspace, workspace_floats,
