@@ -1241,6 +1241,7 @@ __global__ __launch_bounds__(64 * RT * P, WAVES) void attention_rows_kernel(Attn
   __shared__ __attribute__((aligned(1024))) char rows_lds[rows_lds_bytes<RT, P, GK, NST>()];
   int rank = (int)blockIdx.x, kvh = (int)blockIdx.y, z = (int)blockIdx.z;
   if (gridDim.y == 1 && gridDim.z == 1) {
+    rank = rank_of(rank, (int)gridDim.x, a.units, 2);
     const int per = a.nkv * (a.picked > 0 ? a.picked : a.reqs), at = rank % per;
     rank /= per;
     kvh = at % a.nkv;
