@@ -1773,14 +1773,18 @@ static KeySplitLaunch prepare_key_split_decode(AttnArgs a, int reqs, int live, i
   const int most = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;      // one step per wave at least
   if (splits > most) splits = most;
   if (splits > MAX_KEY_SPLITS) splits = MAX_KEY_SPLITS;       // what the merge kernel takes: two per lane
-  // A split costs the merge kernel (4 to 5 us with its launch), which a short history does
-  // not earn back: one block reads 256 KB of keys and values in about that time, and with
-  // few splits to be had (many blocks already) twice as much (64 requests of 2 kv heads of
-  // 64 over 1,024 keys: 10.3 us unsplit, 13.2 in two splits; 32 requests of 4 kv heads of
-  // 128 over 1,024 keys: 20.3 and 22.8; 8 requests of those over 1,024 keys: 14.8 unsplit,
-  // 13.5 in eight splits).
+  // A split costs the merge (4 to 5 us with a kernel's launch, 2 to 3 in place), which a short history does not earn
+  // back: a block reads 320 KB of keys and values in about that time.  Where two splits are to be had, the unsplit
+  // blocks draw half of the memory's rate and more already and gain less.  Unsplit / split, us: heads of 64 over 2, 20
+  // requests behind 1,400 keys (350 KB) 12.0 / 9.7, 28 12.7 / 10.8, behind 2,100 16.9 / 13.0; 40 behind 1,700 (425 KB) 15.8 / 14.1,
+  // 64 17.1 / 16.2, behind 1,300 13.9 / 14.0; heads of 128 over 2, 28 behind 900 (450 KB) 15.1 / 12.6; 40 behind 1,400 (700 KB) 22.5 / 18.2,
+  // 48 behind 1,000 16.8 / 16.5, 56 behind 1,400 24.1 / 27, behind 1,700 27.7 / 24.8.
+  // Beside portions the units have other work: there a split asks for twice as much (48 requests at 1,500 beside 464 tokens
+  // 15.2 / 20.7, 32 at 2,000 17.5 / 19.1).
   const size_t block_bytes = (size_t)visible * D * 2 * sizeof(bf16_t);
-  if (block_bytes < (384u << 10) || (splits <= 4 && block_bytes < (768u << 10))) splits = 1;
+  const size_t least = live < reqs ? (splits <= 4 ? 768 : 384)
+                       : splits > 2 ? 320 : D <= 64 ? 384 : 8 * base <= 3L * num_cus ? 600 : 768;      // KB
+  if (block_bytes < least << 10) splits = 1;
   if (g_force_splits > 0) splits = min(g_force_splits, MAX_KEY_SPLITS);
   if (splits < 1) splits = 1;
   const size_t per_split = (size_t)total_rows * nq * (D + 2);
