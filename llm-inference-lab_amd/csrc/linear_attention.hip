@@ -641,18 +641,21 @@ __device__ __forceinline__ void chunk_log_sums(const float* __restrict__ logs, s
 // SLAB columns at a time; a slab's numbers are asked for into registers while the products before it run.
 constexpr int SLAB = 64, SLAB_STRIDE = SLAB + 16;
 __host__ __device__ inline int product_stride(int columns) { return (columns + 63) / 64 * 64 + 16; }
-// the slab e0 .. of the chunk's values (this thread's 16 numbers: one row of 64 columns a wave at a time)
-__device__ __forceinline__ void fetch_values(const ChunkArgs& a, int first, int n, int h, int e0, float (&reg)[16]) {
+// the slab e0 .. of the chunk's values (this thread's 16 numbers, of PAIR times four waves 16 / PAIR: one row of 64 columns a wave
+// at a time)
+template <int PAIR = 1>
+__device__ __forceinline__ void fetch_values(const ChunkArgs& a, int first, int n, int h, int e0, float (&reg)[16 / PAIR]) {
   const int e = e0 + (int)(threadIdx.x & 63), ec = e < a.E ? e : a.E - 1;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int s = 4 * i + (int)(threadIdx.x >> 6);      // (past the end: the last row, which weighs nothing)
+  for (int i = 0; i < 16 / PAIR; ++i) {
+    const int s = 4 * PAIR * i + (int)(threadIdx.x >> 6);      // (past the end: the last row, which weighs nothing)
     reg[i] = a.proj[(size_t)(first + (s < n ? s : n - 1)) * a.ld + a.off_v + h * a.E + ec];
   }
 }
-__device__ __forceinline__ void stash_slab(float* buf, const float (&reg)[16], int row0) {
+template <int PAIR = 1>
+__device__ __forceinline__ void stash_slab(float* buf, const float (&reg)[16 / PAIR], int row0) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) buf[(row0 + 4 * i + (int)(threadIdx.x >> 6)) * SLAB_STRIDE + (int)(threadIdx.x & 63)] = reg[i];
+  for (int i = 0; i < 16 / PAIR; ++i) buf[(row0 + 4 * PAIR * i + (int)(threadIdx.x >> 6)) * SLAB_STRIDE + (int)(threadIdx.x & 63)] = reg[i];
 }
 
 template <int KIND>
@@ -758,8 +761,14 @@ __global__ __launch_bounds__(256) void chunk_local_kernel(ChunkArgs a) {
     }
 }
 
-template <int KIND, int ET, typename T>
-__global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __restrict__ out) {
+// PAIR = 2: two waves a sub-block of rows, each with half of the channels of the weights (their sums meet in LDS, in the
+// place of the keys, which are read by then) and half of the columns of every slab; a SIMD has a long and a short sub-block.
+// A block's chain (first trips to memory, the diagonal's exponentials, the slabs) is what the pass takes, one block a unit: 1,900 rows of 7
+// heads of 64 x 128 34.6 us by four waves, 29.9 by eight, 29.1 with the first values and the gates asked for ahead of it.
+template <int KIND, int ET, typename T, int PAIR = 1>
+__global__ __launch_bounds__(256 * PAIR) void chunk_finish_kernel(ChunkArgs a, T* __restrict__ out) {
+  static_assert(PAIR == 1 || (KIND == KIND_DECAY && ET >= 2), "pairs of waves");
+  constexpr int NT = 256 * PAIR, REGS = 16 / PAIR, TILES = ET < 4 ? ET : 4, TH = TILES / PAIR, MINE = ET / PAIR;
   extern __shared__ __attribute__((aligned(16))) float chunk_lds[];
   int first, n;
   if (!chunk_rows(a.q_start, a.n_reqs, blockIdx.x, first, n)) return;
@@ -774,21 +783,22 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
   const size_t at = (size_t)blockIdx.x * a.n_heads + h;
   const float* S0 = a.chunk_state + at * D * E;
   // a slab of the state: 64 rows d a time, as many times as it takes
-  auto fetch_state = [&](int d0, int e0, float (&reg)[16]) {
+  auto fetch_state = [&](int d0, int e0, float (&reg)[REGS]) {
     const int e = e0 + (int)(threadIdx.x & 63), ec = e < E ? e : E - 1;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int d = d0 + 4 * i + (int)(threadIdx.x >> 6);      // (past the end: the last row, which meets zeros)
+    for (int i = 0; i < REGS; ++i) {
+      const int d = d0 + 4 * PAIR * i + (int)(threadIdx.x >> 6);      // (past the end: the last row, which meets zeros)
       reg[i] = S0[(size_t)(d < D ? d : D - 1) * E + ec];
     }
   };
-  float sreg[2][16], vreg[16];
+  float sreg[2][REGS], vreg[REGS];
   fetch_state(0, 0, sreg[0]);
   if (DK > 64) fetch_state(64, 0, sreg[1]);
+  fetch_values<PAIR>(a, first, n, h, 0, vreg);
   for (int i0 = 0; i0 < CK * DK; i0 += 1024)
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {                  // (CK * DK is a multiple of 1,024)
-    const int i = i0 + 256 * u + (int)threadIdx.x;
+  for (int u = 0; u < 4 / PAIR; ++u) {           // (CK * DK is a multiple of 1,024)
+    const int i = i0 + NT * u + (int)threadIdx.x;
     const int row = i / DK, d = i - row * DK;
     const bool in = row < n && d < D;
     const float* p = a.proj + (size_t)(first + (row < n ? row : n - 1)) * a.ld + h * D + (d < D ? d : D - 1);
@@ -799,7 +809,7 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
   if (KIND == KIND_MEMORY) chunk_log_sums(a.logs + (size_t)first * a.n_heads + h, a.n_heads, 1, 1, n, s_lb, 1, s_tot);
   else chunk_log_sums(a.logs + ((size_t)first * a.n_heads + h) * D, (size_t)a.n_heads * D, D, DK, n, s_lb, stride, s_tot);
   if (KIND != KIND_DECAY)
-    for (int d = threadIdx.x; d < DK; d += 256) {
+    for (int d = threadIdx.x; d < DK; d += NT) {
       const int dc = d < D ? d : D - 1;
       s_one[d] = d < D ? (KIND == KIND_BONUS ? a.bonus[h * D + dc] : a.chunk_norm[at * D + dc]) : 0.f;
     }
@@ -808,14 +818,16 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
     s_one[DK + row] = row < n ? a.take[(size_t)(first + row) * a.n_heads + h] : 0.f;
   }
   auto stash_state = [&]() {
-    stash_slab(s_buf, sreg[0], 0);
-    if (DK > 64) stash_slab(s_buf, sreg[1], 64);
+    stash_slab<PAIR>(s_buf, sreg[0], 0);
+    if (DK > 64) stash_slab<PAIR>(s_buf, sreg[1], 64);
   };
   stash_state();
   __syncthreads();
-  fetch_values(a, first, n, h, 0, vreg);
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const int i0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));      // this wave's sub-block
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), half = PAIR == 2 ? wave >> 2 : 0;
+  const int i0 = half ? 7 - wave : wave;         // this wave's sub-block
+  // ... and its channels of the weights
+  const int d_half = PAIR == 2 ? (DK / 16 + 1) / 2 * 16 : DK, d_lo = half ? d_half : 0, d_hi = half ? DK : d_half;
   const bool busy = i0 * SUB < n;                // (a wave without rows takes part in the barriers only)
   const int t = i0 * SUB + c;                    // this lane's row (as a row of an operand)
   const float* q_t = s_q + t * DS;
@@ -848,7 +860,7 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
         nq += p[j][r];
       }
     } else if (j < i0) {
-      for (int k0 = 0; k0 < DK; k0 += 16)
+      for (int k0 = d_lo; k0 < d_hi; k0 += 16)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int d = k0 + 4 * u + g;
@@ -858,7 +870,7 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
       }
     } else {
       const int s0 = j * SUB + 4 * g;
-      for (int d = 0; d < DK; d += 4) {
+      for (int d = d_lo; d < d_hi; d += 4) {
         const floatx4 q4 = *(const floatx4*)(q_t + d);
         floatx4 see4;
         if (KIND == KIND_BONUS && c == 0) see4 = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -885,12 +897,26 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
       }
     }
   }
-  // ---- slab by slab: what the state before the chunk gives, and what the chunk's rows give
-  floatx4 acc[ET];
+  if constexpr (PAIR == 2) {                     // the other half's channels, two sub-blocks' weights a time
+    floatx4* const meet = (floatx4*)s_k;         // [wave][2][lane] (DK >= 64: the keys take so much)
+    const int other = 7 - wave;
 #pragma unroll
-  for (int et = 0; et < ET; ++et) acc[et] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 4; j += 2) {
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < 2; ++x) meet[(wave * 2 + x) * 64 + lane] = p[j + x];
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < 2; ++x) p[j + x] += meet[(other * 2 + x) * 64 + lane];
+    }
+  }
+  // ---- slab by slab: what the state before the chunk gives, and what the chunk's rows give
+  floatx4 acc[MINE];
+  auto tile_of = [&](int et) { return et / TH * 4 + half * TH + et % TH; };      // of 16 columns, this wave's et-th
+#pragma unroll
+  for (int et = 0; et < MINE; ++et) acc[et] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto slab = [&](auto number) {                 // (returns whether there is another one behind it)
-    constexpr int TILES = ET < 4 ? ET : 4, X0 = 4 * decltype(number)::value, e0 = 16 * X0;
+    constexpr int X0 = 4 * decltype(number)::value, e0 = 16 * X0, A0 = TH * decltype(number)::value;
     const bool more = X0 + 4 < ET && e0 + SLAB < E;
     if (busy) {
       for (int k0 = 0; k0 < DK; k0 += 16)
@@ -901,14 +927,14 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
         for (int j = 0; j < i0; ++j) lg += s_tot[j * width + dl];
         const float q = q_t[d] * exp2_(lg);
         if (KIND == KIND_MEMORY && e0 == 0) nq = fmaf(q, s_one[d], nq);
-        const float* srow = s_buf + d * SLAB_STRIDE + c;
+        const float* srow = s_buf + d * SLAB_STRIDE + half * TH * 16 + c;
 #pragma unroll
-        for (int x = 0; x < TILES; ++x)
-          acc[X0 + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, srow[16 * x], acc[X0 + x], 0, 0, 0);
+        for (int x = 0; x < TH; ++x)
+          acc[A0 + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q, srow[16 * x], acc[A0 + x], 0, 0, 0);
       }
     }
     __syncthreads();
-    stash_slab(s_buf, vreg, 0);
+    stash_slab<PAIR>(s_buf, vreg, 0);
     __syncthreads();
     if (more) {
       fetch_state(0, e0 + SLAB, sreg[0]);
@@ -920,10 +946,10 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
         if (j > i0) continue;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float* v = s_buf + (j * SUB + 4 * g + r) * SLAB_STRIDE + c;
+          const float* v = s_buf + (j * SUB + 4 * g + r) * SLAB_STRIDE + half * TH * 16 + c;
 #pragma unroll
-          for (int x = 0; x < TILES; ++x)
-            acc[X0 + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[j][r], v[16 * x], acc[X0 + x], 0, 0, 0);
+          for (int x = 0; x < TH; ++x)
+            acc[A0 + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[j][r], v[16 * x], acc[A0 + x], 0, 0, 0);
         }
       }
     }
@@ -931,20 +957,14 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
     __syncthreads();
     stash_state();
     __syncthreads();
-    fetch_values(a, first, n, h, e0 + SLAB, vreg);
+    fetch_values<PAIR>(a, first, n, h, e0 + SLAB, vreg);
     return true;
   };
-  bool again = slab(std::integral_constant<int, 0>{});
-  if constexpr (ET > 4) again = again && slab(std::integral_constant<int, 1>{});
-  if constexpr (ET > 8) again = again && slab(std::integral_constant<int, 2>{});
-  if constexpr (ET > 12) again = again && slab(std::integral_constant<int, 3>{});
-  if (!busy) return;
-  // ---- norm, gate, rounding: this lane now holds the columns 16 et + c of the rows 4 g + r
-  // (all gates and weights are asked for together; past the end the last ones, dropped)
-  float gates[ET][4], ws[ET];
+  // (all gates and weights are asked for together, and travel while the slabs are multiplied; past the end the last ones, dropped)
+  float gates[MINE][4], ws[MINE];
 #pragma unroll
-  for (int et = 0; et < ET; ++et) {
-    const int e = 16 * et + c < E ? 16 * et + c : E - 1;
+  for (int et = 0; et < MINE; ++et) {
+    const int e = 16 * tile_of(et) + c < E ? 16 * tile_of(et) + c : E - 1;
     ws[et] = a.w[a.w_per_head ? h * E + e : e];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -952,29 +972,45 @@ __global__ __launch_bounds__(256) void chunk_finish_kernel(ChunkArgs a, T* __res
       gates[et][r] = a.proj[(size_t)(first + (row < n ? row : n - 1)) * a.ld + a.off_g + h * E + e];
     }
   }
+  bool again = slab(std::integral_constant<int, 0>{});
+  if constexpr (ET > 4) again = again && slab(std::integral_constant<int, 1>{});
+  if constexpr (ET > 8) again = again && slab(std::integral_constant<int, 2>{});
+  if constexpr (ET > 12) again = again && slab(std::integral_constant<int, 3>{});
+  if (PAIR == 1 && !busy) return;
+  // ---- norm, gate, rounding: this lane now holds the columns 16 et + c of the rows 4 g + r
   if (KIND == KIND_MEMORY) {
     nq += __shfl_xor(nq, 16, WAVE);
     nq += __shfl_xor(nq, 32, WAVE);
   }
-  float inv[4];
+  float inv[4], squares[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int row = i0 * SUB + 4 * g + r;
     if (KIND == KIND_MEMORY) {
       const float size = memory_size(__shfl(nq, 4 * g + r, WAVE), a.maxima[(size_t)(first + (row < n ? row : n - 1)) * a.n_heads + h]);
 #pragma unroll
-      for (int et = 0; et < ET; ++et) acc[et][r] /= size;
+      for (int et = 0; et < MINE; ++et) acc[et][r] /= size;
     }
     float ss = 0.f;
 #pragma unroll
-    for (int et = 0; et < ET; ++et) ss = fmaf(acc[et][r], 16 * et + c < E ? acc[et][r] : 0.f, ss);
+    for (int et = 0; et < MINE; ++et) ss = fmaf(acc[et][r], 16 * tile_of(et) + c < E ? acc[et][r] : 0.f, ss);
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
-    inv[r] = 1.0f / sqrtf(ss / (float)a.count + a.eps);
+    squares[r] = ss;
+  }
+  if constexpr (PAIR == 2) {                     // the other half's columns
+    __syncthreads();
+    if (c == 0) *(floatx4*)(s_k + (half * 4 + i0) * SUB + 4 * g) = floatx4{squares[0], squares[1], squares[2], squares[3]};
+    __syncthreads();
+    if (!busy) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) squares[r] = s_k[i0 * SUB + 4 * g + r] + s_k[(4 + i0) * SUB + 4 * g + r];
   }
 #pragma unroll
-  for (int et = 0; et < ET; ++et) {
-    const int e = 16 * et + c;
+  for (int r = 0; r < 4; ++r) inv[r] = 1.0f / sqrtf(squares[r] / (float)a.count + a.eps);
+#pragma unroll
+  for (int et = 0; et < MINE; ++et) {
+    const int e = 16 * tile_of(et) + c;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = i0 * SUB + 4 * g + r;
@@ -1031,11 +1067,11 @@ extern "C" int llmlab_chunk_scan(const float* proj, int ld, int off_q, int off_k
       raised = true;                                                                                                      \
     }                                                                                                                     \
   } while (0)
-#define LLMLAB_CHUNK_FINISH(KIND, ETV, T)                                                                                 \
+#define LLMLAB_CHUNK_FINISH(KIND, ETV, T, PAIR)                                                                           \
   do {                                                                                                                    \
-    auto kernel = chunk_finish_kernel<KIND, ETV, T>;                                                                      \
+    auto kernel = chunk_finish_kernel<KIND, ETV, T, PAIR>;                                                                \
     LLMLAB_CHUNK_LDS(kernel, lds_finish);                                                                                 \
-    hipLaunchKernelGGL(kernel, grid, block, lds_finish, stream, a, (T*)out);                                              \
+    hipLaunchKernelGGL(kernel, grid, dim3(256 * PAIR), lds_finish, stream, a, (T*)out);                                   \
   } while (0)
 #define LLMLAB_CHUNK_LOCAL(KIND)                                              \
   do {                                                                        \
@@ -1045,8 +1081,12 @@ extern "C" int llmlab_chunk_scan(const float* proj, int ld, int off_q, int off_k
   } while (0)
 #define LLMLAB_CHUNK(KIND, ETV)                                                                                  \
   do {                                                                                                           \
-    if (dtype == DT_BF16) LLMLAB_CHUNK_FINISH(KIND, ETV, bf16_t);                                           \
-    else LLMLAB_CHUNK_FINISH(KIND, ETV, float);                                                                  \
+    constexpr int PAIRS = KIND == KIND_DECAY ? 2 : 1;                                                            \
+    const bool paired = KIND == KIND_DECAY && DK >= 64;                                                          \
+    if (dtype == DT_BF16 && paired) LLMLAB_CHUNK_FINISH(KIND, ETV, bf16_t, PAIRS);                               \
+    else if (dtype == DT_BF16) LLMLAB_CHUNK_FINISH(KIND, ETV, bf16_t, 1);                                        \
+    else if (paired) LLMLAB_CHUNK_FINISH(KIND, ETV, float, PAIRS);                                               \
+    else LLMLAB_CHUNK_FINISH(KIND, ETV, float, 1);                                                               \
   } while (0)
 #define LLMLAB_CHUNK_ET(KIND)                 \
   do {                                        \
