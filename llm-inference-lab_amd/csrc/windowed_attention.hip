@@ -1002,7 +1002,9 @@ __device__ __forceinline__ void attend_tiles(const KeyTiles& kt, int t_begin, in
       for (int eb = 0; eb < EB; ++eb)
         run.o[eb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[eb], pf, run.o[eb], 0, 0, 0);
     } else {
-    tmax = across_groups(tmax, [](float x, float y) { return fmaxf(x, y); });
+    // (through LDS: a wave here is alone on its SIMD, and the decoding launch takes 7.8 us so and 8.3 by lane swaps)
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
     const float m_new = fmaxf(run.m, tmax);
     const float m_use = m_new == NEG_INF ? 0.f : m_new;
     const float corr = run.m == NEG_INF ? 0.f : __expf(run.m - m_use);
@@ -1015,7 +1017,8 @@ __device__ __forceinline__ void attend_tiles(const KeyTiles& kt, int t_begin, in
         sum += p;
         pf[4 * u + i] = (bf16_t)p;
       }
-    sum = across_groups(sum, [](float x, float y) { return x + y; });
+    sum += __shfl_xor(sum, 16, WAVE);
+    sum += __shfl_xor(sum, 32, WAVE);
     run.l = run.l * corr + sum;
     run.m = m_new;
 #pragma unroll
