@@ -924,15 +924,18 @@ __global__ __launch_bounds__(256 * PH, (D <= 64 && PH == 1) ? 2 : 1) void attent
 #define STAGED_ROWS (HEAD_DIM == 64 || HEAD_DIM == 128)
 #if STAGED_ROWS
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
-// 16 keys (or their values) from the cache to consecutive memory of LDS, 1 KB a load; the offset counts at both ends
+// 16 keys (or their values) from the cache to consecutive memory of LDS, 1 KB a load; the offset counts at both ends.
+// One statement with the m0 that its loads read: between two the compiler may use m0 itself.
 template <int BYTES>
 __device__ __forceinline__ void block_to_lds(unsigned from, const char* base, unsigned to) {
-  static_assert(BYTES % 1024 == 0 && BYTES <= 4096, "offsets of 12 bits");
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(to) : "memory", "m0");
-  if constexpr (BYTES >= 1024) asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(from), "s"(base) : "memory");
-  if constexpr (BYTES >= 2048) asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" : : "v"(from), "s"(base) : "memory");
-  if constexpr (BYTES >= 3072) asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" : : "v"(from), "s"(base) : "memory");
-  if constexpr (BYTES >= 4096) asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" : : "v"(from), "s"(base) : "memory");
+  static_assert(BYTES == 2048 || BYTES == 4096, "16 keys of 64 or 128 numbers");
+  if constexpr (BYTES == 2048)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024"
+                 : : "v"(from), "s"(base), "s"(to) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %0, %1 offset:2048\n\tglobal_load_lds_dwordx4 %0, %1 offset:3072"
+                 : : "v"(from), "s"(base), "s"(to) : "memory", "m0");
 }
 
 // A number of the block table, waited for on the spot (the compiler, which does not see it, would wait for all loads on
