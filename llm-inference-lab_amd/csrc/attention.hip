@@ -924,6 +924,7 @@ __global__ __launch_bounds__(256 * PH, (D <= 64 && PH == 1) ? 2 : 1) void attent
 #define STAGED_ROWS (HEAD_DIM == 64 || HEAD_DIM == 128)
 #if STAGED_ROWS
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned uintx4;
 // 16 keys (or their values) from the cache to consecutive memory of LDS, 1 KB a load; the offset counts at both ends.
 // One statement with the m0 that its loads read: between two the compiler may use m0 itself.
 template <int BYTES>
@@ -953,7 +954,7 @@ __device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk
   constexpr int BLK = 16 * D * 2;                        // bytes of 16 keys, and of their values
   constexpr int V_AT = KT * D * 2, STAGE = 2 * V_AT;     // a stage: keys, then values
   constexpr int NB = KT / 8 / NW;                        // blocks of 16 keys or of values that a wave brings of a tile
-  static_assert(GK % 32 == 0 && NB * 8 * NW == KT && D % 32 == 0, "steps of 32 keys, whole blocks a wave, loads of 1 KB");
+  static_assert(GK == 32 && NB * 8 * NW == KT && D % 32 == 0, "a step of 32 keys a group, whole blocks a wave, loads of 1 KB");
   constexpr int LOADS = NB * (BLK / 1024);               // ... its loads
   static_assert(LOADS * (NST - 2) < 64, "loads on their way that can be counted");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -977,8 +978,8 @@ __device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk
   const int pos = valid ? sp + tok : -1, lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
   // the keys that the wave's rows see, and the block's; from full_lo on a key is inside the windows of all its rows
   const int last_row = min(row0 + 32, rows_total) - 1, blk_last = min(blk_row0 + RT * 32, rows_total) - 1;
-  const int p_first = sp + uniform(row0 / G), p_last = sp + uniform(last_row / G);
-  const int full_lo = a.window > 0 ? max(0, p_last - a.window + 1) : 0;
+  const int p_first = sp + uniform(row0 / G), p_last = row0 < rows_total ? sp + uniform(last_row / G) : -1;
+  const int key_lo = a.window > 0 ? max(0, p_first - a.window + 1) : 0, full_lo = a.window > 0 ? max(0, p_last - a.window + 1) : 0;
   const int bkey_hi = sp + uniform(blk_last / G);
   const int bkey_lo = a.window > 0 ? max(0, sp + uniform(blk_row0 / G) - a.window + 1) : 0;
 
@@ -1081,88 +1082,98 @@ __device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk
 #pragma unroll
       for (int st = 0; st < NS; ++st) kf[kk][st] = *(const bf16x8*)(ks + st * 2 * BLK + kk * 512);
     fetch(tile + NST - 1, slot == 0 ? NST - 1 : slot - 1);
-    if (tile * KT + KT - 1 > bkey_hi || missing) {
-      // values of keys that nobody sees yet may be anything: out of the products, although their probability is zero
+    if (missing) {
+      // what stands for the values of keys that are not in the cache: out of the products, although their probability is zero
       for (int i = tid; i < KT * D / 8; i += 64 * NW) {
-        const int block = i / (2 * D), db = (i / 32) % (D / 16), g = ((i >> 3) & 3) ^ (db & 1);
-        const int k0 = tile * KT + block * 16 + g * 4;
-        const bool ok = !missing || there(k0 & ~15);
-        bf16x8* at = (bf16x8*)(lds + slot * STAGE + V_AT + i * 16);
-        bf16x8 v = *at;
-#pragma unroll
-        for (int x = 0; x < 8; ++x) v[x] = ok && k0 + (x & 3) <= bkey_hi ? v[x] : (bf16_t)0.f;
-        *at = v;
+        const int k16 = tile * KT + i / (2 * D) * 16;
+        if (!there(k16)) *(bf16x8*)(lds + slot * STAGE + V_AT + i * 16) = zero8;
       }
       __syncthreads();
     }
     const int kb0 = tile * KT + ph * GK;
-    floatx16 s[NS];
-#pragma unroll
-    for (int st = 0; st < NS; ++st)
-#pragma unroll
-      for (int x = 0; x < 16; ++x) s[st][x] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < DK; ++kk)
-#pragma unroll
-      for (int st = 0; st < NS; ++st) s[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk][st], qf[kk], s[st], 0, 0, 0);
-    // (the values of the first 32 keys travel while the maximum is found)
-    bf16x8 vf[2][DV];
-    auto values = [&](bf16x8 (&f)[DV], int block) {
-#pragma unroll
-      for (int i = 0; i < DV; ++i) {
-        const char* at = vs + block * BLK + i * 1024;
-        const bf16x4 v0 = *(const bf16x4*)at, v1 = *(const bf16x4*)(at + 256);
-        f[i] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-      }
-    };
-    values(vf[0], 0);
-    values(vf[1], 1);
-    if (!(kb0 + GK - 1 <= p_first && kb0 >= full_lo && !missing)) {      // some of the keys are not for every row
+    if (kb0 <= p_last && kb0 + GK > key_lo) {      // (else none of the wave's rows sees any of these keys)
+      floatx16 s[NS];
 #pragma unroll
       for (int st = 0; st < NS; ++st)
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-          const int k16 = kb0 + st * 32 + sub * 16;
-          const bool ok = !missing || there(k16);
+        for (int x = 0; x < 16; ++x) s[st][x] = 0.f;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int j = k16 + 8 * (i >> 2) + 4 * h + (i & 3);
-            s[st][sub * 8 + i] = ok && j <= pos && j >= lo ? s[st][sub * 8 + i] : NEG_INF;
-          }
+      for (int kk = 0; kk < DK; ++kk)
+#pragma unroll
+        for (int st = 0; st < NS; ++st) s[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk][st], qf[kk], s[st], 0, 0, 0);
+      // (the values of the first 32 keys travel while the maximum is found)
+      bf16x8 vf[2][DV];
+      auto values = [&](bf16x8 (&f)[DV], int block) {
+#pragma unroll
+        for (int i = 0; i < DV; ++i) {
+          const char* at = vs + block * BLK + i * 1024;
+          const bf16x4 v0 = *(const bf16x4*)at, v1 = *(const bf16x4*)(at + 256);
+          f[i] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
-    }
-    // the maximum of the raw scores, then into the units of the exponent (the scale is positive)
-    float mx[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};
+      };
+      values(vf[0], 0);
+      values(vf[1], 1);
+      if (!(kb0 + GK - 1 <= p_first && kb0 >= full_lo && !missing)) {      // some of the keys are not for every row
 #pragma unroll
-    for (int st = 0; st < NS; ++st)
+        for (int st = 0; st < NS; ++st)
 #pragma unroll
-      for (int x = 0; x < 16; x += 2) mx[(x >> 1) & 3] = max3_raw(s[st][x], s[st][x + 1], mx[(x >> 1) & 3]);
-    mx[0] = max_raw(max3_raw(mx[0], mx[1], mx[2]), mx[3]);
-    if (__any(mx[0] * scale2 > m + LAZY_MAX)) {            // some row's maximum grew: rescale what is summed so far
-      mx[0] = max_across_32(mx[0]) * scale2;
-      const bool grow = mx[0] > m + LAZY_MAX;
-      const float m_new = grow ? mx[0] : m;
-      const float alpha = grow ? fast_exp2(m - m_new) : 1.f;     // 2^-inf = 0 the first time
-      lsum *= alpha;
+          for (int sub = 0; sub < 2; ++sub) {
+            const int k16 = kb0 + st * 32 + sub * 16;
+            const bool ok = !missing || there(k16);
 #pragma unroll
-      for (int i = 0; i < DV; ++i)
+            for (int i = 0; i < 8; ++i) {
+              const int j = k16 + 8 * (i >> 2) + 4 * h + (i & 3);
+              s[st][sub * 8 + i] = ok && j <= pos && j >= lo ? s[st][sub * 8 + i] : NEG_INF;
+            }
+          }
+        // behind the wave's last position values may be anything (another row's may be infinite): out of the products,
+        // although their probability is zero
+        if (kb0 + GK - 1 > p_last)
 #pragma unroll
-        for (int x = 0; x < 16; ++x) o[i][x] *= alpha;
-      m = m_new;
-    }
-    const float neg_m = m == NEG_INF ? 0.f : -m;      // (no visible key yet: every p of the row is 2^-inf = 0)
+        for (int block = 0; block < 2; ++block) {
+          const int seen = p_last - (kb0 + block * 16 + 4 * h);      // of the lane's keys {0 .. 3, 8 .. 11} those up to this one
+          uintx4 keep;
 #pragma unroll
-    for (int block = 0; block < 2 * NS; ++block) {
-      float pv[8];
+          for (int x = 0; x < 4; ++x) {
+            const int at = 8 * (x >> 1) + 2 * (x & 1);
+            keep[x] = seen > at ? 0xffffffffu : seen == at ? 0xffffu : 0u;
+          }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) pv[i] = fast_exp2(fmaf(s[block >> 1][(block & 1) * 8 + i], scale2, neg_m));
-      lsum += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
-      bf16x8 pf;
+          for (int i = 0; i < DV; ++i) vf[block][i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(uintx4, vf[block][i]) & keep);
+        }
+      }
+      // the maximum of the raw scores, then into the units of the exponent (the scale is positive)
+      float mx[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};
 #pragma unroll
-      for (int i = 0; i < 8; ++i) pf[i] = (bf16_t)pv[i];
+      for (int st = 0; st < NS; ++st)
 #pragma unroll
-      for (int i = 0; i < DV; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[block & 1][i], pf, o[i], 0, 0, 0);
-      if (block + 2 < 2 * NS) values(vf[block & 1], block + 2);
+        for (int x = 0; x < 16; x += 2) mx[(x >> 1) & 3] = max3_raw(s[st][x], s[st][x + 1], mx[(x >> 1) & 3]);
+      mx[0] = max_raw(max3_raw(mx[0], mx[1], mx[2]), mx[3]);
+      if (__any(mx[0] * scale2 > m + LAZY_MAX)) {            // some row's maximum grew: rescale what is summed so far
+        mx[0] = max_across_32(mx[0]) * scale2;
+        const bool grow = mx[0] > m + LAZY_MAX;
+        const float m_new = grow ? mx[0] : m;
+        const float alpha = grow ? fast_exp2(m - m_new) : 1.f;     // 2^-inf = 0 the first time
+        lsum *= alpha;
+#pragma unroll
+        for (int i = 0; i < DV; ++i)
+#pragma unroll
+          for (int x = 0; x < 16; ++x) o[i][x] *= alpha;
+        m = m_new;
+      }
+      const float neg_m = m == NEG_INF ? 0.f : -m;      // (no visible key yet: every p of the row is 2^-inf = 0)
+#pragma unroll
+      for (int block = 0; block < 2 * NS; ++block) {
+        float pv[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pv[i] = fast_exp2(fmaf(s[block >> 1][(block & 1) * 8 + i], scale2, neg_m));
+        lsum += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+        bf16x8 pf;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pf[i] = (bf16_t)pv[i];
+#pragma unroll
+        for (int i = 0; i < DV; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[block & 1][i], pf, o[i], 0, 0, 0);
+      }
     }
     slot = slot == NST - 1 ? 0 : slot + 1;
   }
