@@ -975,7 +975,11 @@ __device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk
   const int rr = row0 + col;
   const bool valid = rr < rows_total;
   const int tok = valid ? rr / G : 0, head = kvh * G + (valid ? rr % G : 0);
-  const int pos = valid ? sp + tok : -1, lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  // (a key is seen if it is no further than pos - lo behind lo: one comparison, as two hold so many masks at once that registers
+  // are spilled; a row that sees none, past the end or in front of the first key, has its lo behind all keys)
+  const int pos = valid ? sp + tok : -1, lo = pos < 0 ? 1 << 30 : a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  const int lane_key = 4 * h - lo;
+  const unsigned span = pos < 0 ? 0 : pos - lo;
   // the keys that the wave's rows see, and the block's; from full_lo on a key is inside the windows of all its rows
   const int last_row = min(row0 + 32, rows_total) - 1, blk_last = min(blk_row0 + RT * 32, rows_total) - 1;
   const int p_first = sp + uniform(row0 / G), p_last = row0 < rows_total ? sp + uniform(last_row / G) : -1;
@@ -1122,25 +1126,29 @@ __device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk
             const bool ok = !missing || there(k16);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-              const int j = k16 + 8 * (i >> 2) + 4 * h + (i & 3);
-              s[st][sub * 8 + i] = ok && j <= pos && j >= lo ? s[st][sub * 8 + i] : NEG_INF;
+              const unsigned from_lo = (unsigned)(k16 + 8 * (i >> 2) + (i & 3) + lane_key);
+              s[st][sub * 8 + i] = ok && from_lo <= span ? s[st][sub * 8 + i] : NEG_INF;
             }
           }
         // behind the wave's last position values may be anything (another row's may be infinite): out of the products,
         // although their probability is zero
         if (kb0 + GK - 1 > p_last)
 #pragma unroll
-        for (int block = 0; block < 2; ++block) {
-          const int seen = p_last - (kb0 + block * 16 + 4 * h);      // of the lane's keys {0 .. 3, 8 .. 11} those up to this one
-          uintx4 keep;
+          for (int block = 0; block < 2; ++block) {
+            int past = kb0 + block * 16 + 4 * h - p_last;      // how far the first of the lane's keys {0 .. 3, 8 .. 11} lies behind it
+            asm volatile("" : "+v"(past));
 #pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const int at = 8 * (x >> 1) + 2 * (x & 1);
-            keep[x] = seen > at ? 0xffffffffu : seen == at ? 0xffffu : 0u;
+            for (int x = 0; x < 4; ++x) {
+              const int at = past + 8 * (x >> 1) + 2 * (x & 1);
+              const unsigned keep = ((unsigned)((at - 1) >> 31) & 0xffffu) | ((unsigned)(at >> 31) & 0xffff0000u);
+#pragma unroll
+              for (int i = 0; i < DV; ++i) {
+                uintx4 v = __builtin_bit_cast(uintx4, vf[block][i]);
+                v[x] &= keep;
+                vf[block][i] = __builtin_bit_cast(bf16x8, v);
+              }
+            }
           }
-#pragma unroll
-          for (int i = 0; i < DV; ++i) vf[block][i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(uintx4, vf[block][i]) & keep);
-        }
       }
       // the maximum of the raw scores, then into the units of the exponent (the scale is positive)
       float mx[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};

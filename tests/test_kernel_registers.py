@@ -42,6 +42,8 @@ def library(make):
 
 @pytest.mark.parametrize("make,kernel,waves,least", [
     (lambda: build.mixer_library("linear_attention"), "chunk_finish_kernel", 2, 24),
+    (lambda: build.attention_library(64), "attention_rows_kernel", 2, 4),
+    (lambda: build.attention_library(128), "attention_rows_kernel", 2, 3),
 ])
 def test_waves_a_simd_holds(make, kernel, waves, least):
     """As many waves a SIMD as the kernels' notes count on, and nothing spilled."""
