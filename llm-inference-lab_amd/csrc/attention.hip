@@ -1760,7 +1760,8 @@ extern "C" void llmlab_debug_attention_splits(int splits) { g_force_splits = spl
 // ... and the launch that steps of many rows take: 1 = the waves of a block split the keys of
 // a tile of 32 rows, 2 = tiles of 32 rows per wave, 3 = late and early tiles in pairs,
 // 4 = tiles of 16 rows per wave, 5 and 6 = 3 and 4 with two groups of waves that take the
-// staged keys in turn (0: chosen here).
+// staged keys in turn; 7 to 11 = keys staged in LDS, blocks of 1, 2 and 4 tiles of 32 rows by 4, 4, 2, 1 groups of waves and 2 by
+// 2, at heads of 64 (not 11) and 128 (not 7 and 9), where 2 to 6 stand for one of them (0: chosen here).
 static int g_force_path = 0;
 extern "C" void llmlab_debug_attention_path(int path) { g_force_path = path; }
 // ... and who merges the key splits: 1 = the merge kernel even where the last block could.
@@ -1975,8 +1976,10 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
 
 constexpr bool TWO_GROUPS = D <= 128;      // (the staged keys and values of two groups at larger heads: more LDS than there is)
 
-// Which launch a step of many rows takes (bfloat16): `max_rows` (token, head of the group) pairs
-// at most per request and kv head, `live` requests, the longest portion and context, the window.
+// Which of the launches without staged keys a step of many rows takes (bfloat16): `max_rows` (token, head of the group) pairs
+// at most per request and kv head, `live` requests, the longest portion and context, the window.  Heads of 64 and 128 take
+// launch 1 of them, where many_rows_launch says so, and no other; the figures are theirs, from before that, and stand in for
+// the heads beside them.
 static int choose_many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int max_ctx_len, int window,
                                    int num_cus, int forced) {
   // The launch, from measurements of 64 to 4,096 tokens behind 0 and 4,096 keys, one to
@@ -2047,34 +2050,43 @@ static int choose_many_rows_launch(long max_rows, int nkv, int live, int max_q_l
   return path;
 }
 
-// Heads of 64 and 128: attention_rows serves what the launches 2 to 6 would, and launch 1 where it is faster: at heads of
-// 128 everywhere (us: 4 / 48 / 96 tokens of 28 heads over 4 behind 1,500 keys 27 / 33 / 33 -> 21 / 23 / 24, behind 4,000 45 / 46 / 47 ->
-// 43), at heads of 64 behind fewer than 1,024 (48 tokens of 14 heads over 2 behind 500 10.4 -> 9.7, behind 1,500 14.8 and 14.5,
+// The launch that a step of many rows takes (bfloat16), and that llmlab_attention_launch answers with.  `mixed`: its portions
+// have a launch of their own beside decoding requests.
+// Heads of 64 and 128: keys staged in LDS (attention_rows, ROWS_ below), and launch 1 where it is faster: at heads of
+// 128 nowhere (us: 4 / 48 / 96 tokens of 28 heads over 4 behind 1,500 keys 27 / 33 / 33 -> 21 / 23 / 24, behind 4,000 45 / 46 / 47 ->
+// 43), at heads of 64 behind 1,024 and more (48 tokens of 14 heads over 2 behind 500 10.4 -> 9.7, behind 1,500 14.8 and 14.5,
 // behind 4,000 24.0 and 27.4).  Not beside decoding requests: one launch for both kinds and two give the same there, to the bit.
-static bool splits_keys(bool mixed, int max_q_len, int max_ctx_len, int forced) {
-  return !STAGED_ROWS || mixed || forced == 1 || (D == 64 && max_ctx_len - max_q_len >= 1024);
-}
-#if STAGED_ROWS
-// ... and by which block, RT tiles of 32 rows by P groups of waves.  The more groups, the shorter a tile's chain of steps;
+// By which block, RT tiles of 32 rows by P groups of waves: the more groups, the shorter a tile's chain of steps;
 // the more rows, the fewer reads of the keys.  By `blocks`, tiles of 64 rows (1, 2 and 4 tiles of 32 rows with 4, 4 / 2 and 2 / 1 groups, us):
 // heads of 64: a prompt of 1,024 (224 blocks) 12.9 / 13.3 / 18.1, of 1,536 (336) 19.6 / 18.3 / 23.7, of 4,096 (896) 67 / 53.9 / 54.4,
 // of 8,192 (1,792) 213 / 171 / 161, two of 2,000 and 1,789 (876) 44 / 34 / 32; heads of 128 (28 over 4), 2 tiles with 4 and 2
 // groups and 4 with one: 512 tokens (224) 14.8 / 14.6 / 18.9, 768 (336) 24 / 20 / 25, 464 behind 3,000 (204) 42.5 / 51 / 81,
 // 2,048 (896) 68 / 51 / 57, 3,072 (1,344) 126 / 98 / 90.  Hardly a step of keys: four tiles, one group (64 prompts of 24 tokens: heads of
 // 64 12.9 / 10.5 / 7.0, of 128 29 / 18 / 12).
-enum { ROWS_1x4 = 1, ROWS_2x4 = 2, ROWS_4x2 = 3, ROWS_4x1 = 4, ROWS_2x2 = 5 };
-static int rows_kind(long max_rows, int nkv, int live, int max_q_len, int max_ctx_len, int num_cus, int forced) {
-  if (forced == 2) return D == 64 ? ROWS_4x2 : ROWS_4x1;      // (32 rows a wave over all keys, or nearly; tests)
+enum { KEY_SPLIT = 1, ROWS_1x4 = 7, ROWS_2x4 = 8, ROWS_4x2 = 9, ROWS_4x1 = 10, ROWS_2x2 = 11 };
+static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int max_ctx_len, int window, bool mixed,
+                            int num_cus, int forced) {
+#if STAGED_ROWS
+  if (forced >= ROWS_1x4 && forced <= ROWS_2x2 && forced != (D == 64 ? ROWS_2x2 : ROWS_4x2) && !(D == 128 && forced == ROWS_1x4))
+    return forced;
+  // (what stands in for launches 2 to 6)
+  if (forced == 2) return D == 64 ? ROWS_4x2 : ROWS_4x1;
   if (forced == 3) return D == 64 ? ROWS_1x4 : ROWS_2x2;
   if (forced == 4) return ROWS_4x1;
   if (forced == 5 || forced == 6) return ROWS_2x4;
+  if (forced > 6) forced = 0;
+  if (choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, forced) == KEY_SPLIT &&
+      (mixed || forced == KEY_SPLIT || (D == 64 && max_ctx_len - max_q_len >= 1024)))
+    return KEY_SPLIT;
   const long blocks = (max_rows + 63) / 64 * nkv * live;
   if (max_ctx_len <= (D == 64 ? 64 : 32)) return ROWS_4x1;
   if (D == 64) return 8 * blocks <= 7L * num_cus ? ROWS_1x4 : blocks <= 3L * num_cus ? ROWS_2x4 : ROWS_4x2;
   if (blocks > 4L * num_cus) return ROWS_4x1;
   return blocks <= num_cus && max_ctx_len > 512 ? ROWS_2x4 : ROWS_2x2;
-}
+#else
+  return choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, forced > 6 ? 0 : forced);
 #endif
+}
 
 // Whether a mixed step goes in one launch with the portions by tiles of 16 rows, whose waves split the keys with one
 // step on its way: few enough registers (116 at heads of 64, against 157 to 201) that a unit holds two
@@ -2138,15 +2150,16 @@ extern "C" int llmlab_attention_mixed_launches(int nq, int nkv, int reqs, int n_
   const long max_rows = (long)max_q_len * (nq / nkv);
   if (max_rows <= 16) return 0;
   const int live = reqs - n_short;
-  const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, 0);
+  const int path = many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, true, num_cus, 0);
   AttnArgs a{};
   const KeySplitLaunch shorts = prepare_key_split_decode(a, reqs, n_short, short_ctx, window, reqs, nq, nkv, nullptr,
                                                          ~(size_t)0 >> 8, num_cus, nullptr, 0);
   return mixed_step_launch(shorts, n_short, max_rows, nkv, live, max_ctx_len, path, num_cus, 0, g_force_two_launches);
 }
 
-// The launch that llmlab_paged_attention would take for a step of many rows of these sizes
-// (for tests and tuning; 0: the sizes make a decode step, whose keys are split over blocks).
+// The launch that llmlab_paged_attention takes for a step of many rows of these sizes, none of whose requests decodes (for
+// tests and tuning).  0: the sizes make a decode step, whose keys are split over blocks; 1 to 6: as llmlab_debug_attention_path
+// names them; 7 to 11: keys staged in LDS, in blocks of 1, 2 and 4 tiles of 32 rows by 4, 4, 2, 1 groups of waves, and 2 by 2.
 extern "C" int llmlab_attention_launch(int dtype, int nq, int nkv, int reqs, int max_q_len, int max_ctx_len, int window,
                                        int num_cus) {
   if (num_cus <= 0) num_cus = 256;
@@ -2157,7 +2170,7 @@ extern "C" int llmlab_attention_launch(int dtype, int nq, int nkv, int reqs, int
     constexpr int ROWS = 16 * F32_QB;
     return choose_many_rows_launch_f32((max_rows + ROWS - 1) / ROWS * nkv * reqs, max_q_len, max_ctx_len, num_cus, 0);
   }
-  return choose_many_rows_launch(max_rows, nkv, reqs, max_q_len, max_ctx_len, window, num_cus, 0);
+  return many_rows_launch(max_rows, nkv, reqs, max_q_len, max_ctx_len, window, false, num_cus, 0);
 }
 
 // q rows are the step's packed rows; reqs requests; max_q_len / max_ctx_len are
@@ -2234,7 +2247,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
   // (a launch of both kinds has them all along x, which takes less than 2^32 threads)
   auto mixed_blocks = [&](long long_tiles) { return long_tiles * nkv * zs + (long)nkv * shorts.a.splits * short_zs; };
   constexpr long MOST_BLOCKS = 0xffffffffl / (64 * DECODE_WAVES);
-  const int path = choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, g_force_path);
+  const int path = many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, mixed, num_cus, g_force_path);
   const int steps32 = (max_ctx_len + 31) / 32 + 1;
   const int steps_per_wave = (steps32 + DECODE_WAVES - 1) / DECODE_WAVES;
   int how = mixed ? mixed_step_launch(shorts, n_short, max_rows, nkv, live, max_ctx_len, path, num_cus, g_force_path,
@@ -2253,7 +2266,7 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     const int rc = launch_key_split_decode(shorts, reqs, total_rows, nq, nkv, row_req, out, out_stride, stream);
     if (rc) return rc;
   }
-  if (path == 1 && splits_keys(mixed, max_q_len, max_ctx_len, g_force_path)) {
+  if (path == KEY_SPLIT) {
     if (how == MIXED_ONE_LAUNCH) {
       const int long_tiles = (int)((max_rows + 31) / 32);
       dim3 mgrid((unsigned)mixed_blocks(long_tiles)), mblock(64 * DECODE_WAVES);
@@ -2278,7 +2291,6 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     return 0;
   }
 #if STAGED_ROWS
-  const int kind = rows_kind(max_rows, nkv, live, max_q_len, max_ctx_len, num_cus, g_force_path);
   auto launch = [&](auto kernel, int rt, int waves) {
     a.tiles = (int)((max_rows + 32 * rt - 1) / (32 * rt));
     const long blocks = (long)a.tiles * nkv * zs;
@@ -2286,14 +2298,14 @@ extern "C" int llmlab_paged_attention(const void* q, int dtype, int q_stride, in
     hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, stream, a);
   };
   if constexpr (D == 64) {
-    if (kind == ROWS_1x4) launch(attention_rows_kernel<1, 4, 32, 2, 2>, 1, 4);
-    if (kind == ROWS_2x4) launch(attention_rows_kernel<2, 4, 32, 2, 4>, 2, 8);
-    if (kind == ROWS_4x2) launch(attention_rows_kernel<4, 2, 32, 3, 4>, 4, 8);
-    if (kind == ROWS_4x1) launch(attention_rows_kernel<4, 1, 32, 3, 4>, 4, 4);
+    if (path == ROWS_1x4) launch(attention_rows_kernel<1, 4, 32, 2, 2>, 1, 4);
+    if (path == ROWS_2x4) launch(attention_rows_kernel<2, 4, 32, 2, 4>, 2, 8);
+    if (path == ROWS_4x2) launch(attention_rows_kernel<4, 2, 32, 3, 4>, 4, 8);
+    if (path == ROWS_4x1) launch(attention_rows_kernel<4, 1, 32, 3, 4>, 4, 4);
   } else {
-    if (kind == ROWS_2x4) launch(attention_rows_kernel<2, 4, 32, 2, 2>, 2, 8);
-    if (kind == ROWS_2x2) launch(attention_rows_kernel<2, 2, 32, 2, 2>, 2, 4);
-    if (kind == ROWS_4x1) launch(attention_rows_kernel<4, 1, 32, 3, 2>, 4, 4);
+    if (path == ROWS_2x4) launch(attention_rows_kernel<2, 4, 32, 2, 2>, 2, 8);
+    if (path == ROWS_2x2) launch(attention_rows_kernel<2, 2, 32, 2, 2>, 2, 4);
+    if (path == ROWS_4x1) launch(attention_rows_kernel<4, 1, 32, 3, 2>, 4, 4);
   }
   LLMLAB_LAUNCH_CHECK("attention(bfloat16, staged rows)");
 #else

@@ -140,7 +140,8 @@ class KernelDebug:
         block split the keys of a tile of 32 rows, 2 = tiles of 32 rows per wave, 3 = late and
         early tiles in pairs, 4 = tiles of 16 rows per wave, 5 and 6 = 3 and 4 with two groups of
         waves that take the staged keys in turn; heads above 128 have no 5 and 6 and choose
-        for themselves).  ``attention_merge_kernel`` / ``attention_merge_in_place``: a head size; the
+        for themselves; heads of 64 and 128 have 1 and, with keys staged in LDS, 7 to 11 = blocks of 1, 2 and 4 tiles of 32 rows by
+        4, 4, 2, 1 groups of waves and 2 by 2 (64: not 11; 128: not 7 and 9), for one of which 2 to 6 stand there).  ``attention_merge_kernel`` / ``attention_merge_in_place``: a head size; the
         key splits of decode attention are merged there by the kernel of its own, or by the
         last block to arrive, whatever their number.  ``attention_two_launches`` / ``attention_one_launch``:
         a head size; a mixed step's decoding requests and its portions get a launch each also
