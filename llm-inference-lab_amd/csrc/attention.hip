@@ -2052,17 +2052,22 @@ static int choose_many_rows_launch(long max_rows, int nkv, int live, int max_q_l
 
 // The launch that a step of many rows takes (bfloat16), and that llmlab_attention_launch answers with.  `mixed`: its portions
 // have a launch of their own beside decoding requests.
-// Heads of 64 and 128: keys staged in LDS (attention_rows, ROWS_ below), and launch 1 where it is faster: at heads of
-// 128 nowhere (us: 4 / 48 / 96 tokens of 28 heads over 4 behind 1,500 keys 27 / 33 / 33 -> 21 / 23 / 24, behind 4,000 45 / 46 / 47 ->
-// 43), at heads of 64 behind 1,024 and more (48 tokens of 14 heads over 2 behind 500 10.4 -> 9.7, behind 1,500 14.8 and 14.5,
-// behind 4,000 24.0 and 27.4).  Not beside decoding requests: one launch for both kinds and two give the same there, to the bit.
-// By which block, RT tiles of 32 rows by P groups of waves: the more groups, the shorter a tile's chain of steps;
-// the more rows, the fewer reads of the keys.  By `blocks`, tiles of 64 rows (1, 2 and 4 tiles of 32 rows with 4, 4 / 2 and 2 / 1 groups, us):
-// heads of 64: a prompt of 1,024 (224 blocks) 12.9 / 13.3 / 18.1, of 1,536 (336) 19.6 / 18.3 / 23.7, of 4,096 (896) 67 / 53.9 / 54.4,
-// of 8,192 (1,792) 213 / 171 / 161, two of 2,000 and 1,789 (876) 44 / 34 / 32; heads of 128 (28 over 4), 2 tiles with 4 and 2
-// groups and 4 with one: 512 tokens (224) 14.8 / 14.6 / 18.9, 768 (336) 24 / 20 / 25, 464 behind 3,000 (204) 42.5 / 51 / 81,
-// 2,048 (896) 68 / 51 / 57, 3,072 (1,344) 126 / 98 / 90.  Hardly a step of keys: four tiles, one group (64 prompts of 24 tokens: heads of
-// 64 12.9 / 10.5 / 7.0, of 128 29 / 18 / 12).
+// Heads of 64 and 128: keys staged in LDS (attention_rows, ROWS_ below), and launch 1 where it is faster: at heads of 64 few tiles behind
+// 1,024 keys and more (48 tokens of 14 heads over 2 behind 500 10.4 / 9.7 us with staged keys, behind 1,500 14.5 / 14.8,
+// behind 4,000 24.0 / 27.4); at heads of 128 few tiles whose keys and values together are more than the caches of the dies hold, 25 MB (32
+// requests of 7 tokens behind 5,500 keys at 8 heads over 1 64 / 78, 16 of 35 at 1 over 1 behind 7,284 80 / 98, 49 over 32 behind 1,891 28.0 / 32.9;
+// below, 28 heads over 4, 4 / 48 / 96 tokens behind 1,500 27 / 33 / 33 and 21 / 23 / 24; with more tiles than half the units 16 x 116 of 4
+// heads behind 5,873 71.4 / 70.0).  Not beside decoding requests: one launch for both kinds and two give the same there, to the bit.
+// By which block, RT tiles of 32 rows by P groups of waves: the more groups, the shorter a tile's chain of steps; the more rows
+// and the fewer groups, the fewer reads of the keys, the smaller the merge and the less work for a last tile's padding.  So by `blocks`, tiles of
+// 64 rows, and `walk`, the keys that a tile walks on average (us, 1x4 / 2x4 / 4x2 / 4x1 at heads of 64): a prompt of 1,024 of 14 heads
+// over 2 (224 blocks) 12.9 / 13.3 / 18.1 / --, of 1,536 (336) 19.6 / 18.3 / 23.7 / --; 64 requests of 93 tokens of 2 over 1 x 4 (768, walk 47)
+// 16.2 / 13.6 / 9.3 / 7.9, 8 of 318 of 16 over 4 (640, 159) 17.1 / 14.4 / 11.0 / 10.3, 64 of 229 of 1 over 1 (256, 115) 7.4 / 7.4 / 8.8 / 9.6;
+// 32 of 512 of 16 over 2 (4,096, 256) 99 / 63 / 42 / 31; 1,210 of 28 over 4 (532, 641) 22.4 / 17.8 / 20.0 / 23.6.  At heads of 128 (2x4 / 2x2
+// / 4x1): 512 tokens of 28 over 4 (224) 14.8 / 14.6 / 18.9, 768 (336) 24 / 20 / 25, 464 behind 3,000 (204) 42.5 / 51 / 81, 2,048 (896) 68 / 51 /
+// 57, 3,072 (1,344) 126 / 98 / 90; 64 of 186 of 4 over 2 (768, walk 93) 28.3 / 18.6 / 13.6, 336 of 64 over 16 in a window of 251 (336, 168)
+// 17.6 / 11.6 / 13.0.  Hardly a step of keys: 4x1.  (Over 1,250 steps drawn at random the picks lose 1.1 and 0.5 % to the best of
+// all, and against the launches 1 to 6 that these took the place of they take 0.77 and 0.74 of the time, 1.05 at worst.)
 enum { KEY_SPLIT = 1, ROWS_1x4 = 7, ROWS_2x4 = 8, ROWS_4x2 = 9, ROWS_4x1 = 10, ROWS_2x2 = 11 };
 static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int max_ctx_len, int window, bool mixed,
                             int num_cus, int forced) {
@@ -2075,14 +2080,25 @@ static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int
   if (forced == 4) return ROWS_4x1;
   if (forced == 5 || forced == 6) return ROWS_2x4;
   if (forced > 6) forced = 0;
-  if (choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, forced) == KEY_SPLIT &&
-      (mixed || forced == KEY_SPLIT || (D == 64 && max_ctx_len - max_q_len >= 1024)))
-    return KEY_SPLIT;
+  if (forced == KEY_SPLIT) return KEY_SPLIT;
+  const int history = max_ctx_len - max_q_len, seen = window > 0 ? min(max_ctx_len, window + max_q_len) : max_ctx_len;
+  const int middle = max_ctx_len - max_q_len / 2, walk = window > 0 ? min(window, middle) : middle;
   const long blocks = (max_rows + 63) / 64 * nkv * live;
-  if (max_ctx_len <= (D == 64 ? 64 : 32)) return ROWS_4x1;
-  if (D == 64) return 8 * blocks <= 7L * num_cus ? ROWS_1x4 : blocks <= 3L * num_cus ? ROWS_2x4 : ROWS_4x2;
-  if (blocks > 4L * num_cus) return ROWS_4x1;
-  return blocks <= num_cus && max_ctx_len > 512 ? ROWS_2x4 : ROWS_2x2;
+  if (mixed || D == 64) {
+    if ((mixed || history >= 1024) &&
+        choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, 0) == KEY_SPLIT)
+      return KEY_SPLIT;
+  } else if (2 * ((max_rows + 31) / 32) * nkv * live <= num_cus && (long)nkv * live * seen * D * 4 >= 25L << 20) {
+    return KEY_SPLIT;
+  }
+  if (D == 64) {
+    if (max_ctx_len <= 64) return ROWS_4x1;
+    if (8 * blocks <= 7L * num_cus) return ROWS_1x4;
+    if ((blocks > num_cus && walk <= 160) || (blocks > 2L * num_cus && walk <= 512)) return ROWS_4x1;
+    return blocks <= 3L * num_cus ? ROWS_2x4 : blocks <= 4L * num_cus ? ROWS_4x2 : ROWS_4x1;
+  }
+  if (max_ctx_len <= 32 || blocks > 4L * num_cus || (blocks >= 2L * num_cus && walk <= 224)) return ROWS_4x1;
+  return blocks <= num_cus && walk > 384 ? ROWS_2x4 : ROWS_2x2;
 #else
   return choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, forced > 6 ? 0 : forced);
 #endif

@@ -358,14 +358,34 @@ def test_attention_launch_is_one_the_head_size_has(head_dim, nq, nkv):
     (64, 14, 2, BF16, 1, 1024, 0, 7),        # a prompt from its start, 224 tiles of 64 rows: 12.9 us against 13.3 and 18.1
     (64, 14, 2, BF16, 1, 1025, 0, 8),
     (64, 14, 2, BF16, 1, 1536, 0, 8),        # 18.3 against 19.6 and 23.7
-    (64, 14, 2, BF16, 1, 8192, 0, 9),        # 161 against 213 and 171
     (64, 14, 2, BF16, 64, 24, 0, 10),        # many short prompts: 7.0 against 12.9 and 10.5
+    (64, 8, 4, BF16, 64, 93, 0, 10),         # 7.9 against 13.6 with 2 x 4
+    (64, 16, 4, BF16, 8, 318, 0, 10),        # 10.3 against 14.4
+    (64, 1, 1, BF16, 64, 229, 0, 8),         # a block a unit: 7.4 against 9.6 with 4 x 1
+    (64, 28, 4, BF16, 1, 1210, 36, 8),       # 17.8 against 23.6 with 4 x 1
+    (64, 16, 2, BF16, 32, 512, 0, 10),       # 31 against 42 with 4 x 2
+    (64, 1, 1, BF16, 224, 64, 1, 7), (64, 1, 1, BF16, 225, 64, 1, 8), (64, 1, 1, BF16, 64, 64, 0, 10),
+    (64, 1, 1, BF16, 257, 64, 128, 10), (64, 1, 1, BF16, 257, 64, 129, 8), (64, 1, 1, BF16, 256, 64, 128, 8),
+    (64, 1, 1, BF16, 513, 64, 480, 10), (64, 1, 1, BF16, 513, 64, 481, 8), (64, 1, 1, BF16, 512, 64, 480, 8),
+    (64, 1, 1, BF16, 768, 64, 481, 8), (64, 1, 1, BF16, 769, 64, 481, 9), (64, 1, 1, BF16, 1024, 64, 481, 9),
+    (64, 1, 1, BF16, 1025, 64, 481, 10),
     (128, 28, 4, BF16, 1, 4, 1500, 8),       # 21 us against 27 with the key split
     (128, 28, 4, BF16, 1, 96, 4000, 8),      # 43 against 47
     (128, 28, 4, BF16, 1, 128, 2560, 8),
     (128, 28, 4, BF16, 1, 464, 3000, 8),     # 42.5 against 51 and 81
     (128, 28, 4, BF16, 1, 768, 0, 11),       # 20 against 24 and 25
     (128, 28, 4, BF16, 1, 3072, 0, 10),      # 90 against 126 and 98
+    (128, 8, 1, BF16, 32, 7, 5500, 1),       # keys of many requests from memory: 64 us against 78 with 2 x 4
+    (128, 1, 1, BF16, 16, 35, 7284, 1),      # 80 against 98
+    (128, 4, 4, BF16, 8, 49, 1891, 1),       # 28.0 against 32.9
+    (128, 4, 1, BF16, 16, 116, 5873, 8),     # 70.0 against 71.4: more tiles than half the units
+    (128, 1, 1, BF16, 32, 32, 1568, 1), (128, 1, 1, BF16, 32, 32, 1567, 8), (128, 1, 1, BF16, 128, 32, 1568, 1),
+    (128, 1, 1, BF16, 129, 32, 1568, 8),
+    (128, 4, 2, BF16, 64, 186, 0, 10),       # 13.6 against 18.6 with 2 x 2
+    (128, 1, 1, BF16, 512, 64, 192, 10), (128, 1, 1, BF16, 512, 64, 193, 11), (128, 1, 1, BF16, 511, 64, 192, 11),
+    (128, 1, 1, BF16, 256, 64, 353, 8), (128, 1, 1, BF16, 256, 64, 352, 11), (128, 1, 1, BF16, 257, 64, 353, 11),
+    (128, 1, 1, BF16, 1024, 64, 193, 11), (128, 1, 1, BF16, 1025, 64, 193, 10),
+    (128, 1, 1, BF16, 8, 32, 0, 10), (128, 1, 1, BF16, 8, 32, 1, 11),
     (128, 28, 4, BF16, 64, 24, 0, 10),       # 12 against 29 and 18
     (96, 28, 4, BF16, 1, 128, 1024, 6),      # (heads beside them: as those were measured without staged keys)
     (96, 28, 4, BF16, 1, 128, 2560, 1), (96, 28, 4, BF16, 8, 128, 0, 2), (96, 28, 4, BF16, 1, 64, 0, 4),
@@ -382,6 +402,20 @@ def test_attention_launch_is_one_the_head_size_has(head_dim, nq, nkv):
 def test_measured_attention_launches(head_dim, nq, nkv, dtype, reqs, q, behind, want):
     lib = attention_library(head_dim)
     assert lib.llmlab_attention_launch(dtype, nq, nkv, reqs, q, behind + q, 0, CUS) == want
+
+
+@pytest.mark.parametrize("head_dim,nq,nkv,reqs,q,behind,window,want", [
+    # (a window bounds what a tile walks, and what all requests read)
+    (64, 14, 2, 2, 1521, 0, 33, 10),         # 9.1 us against 14.0 with 2 x 4
+    (64, 16, 8, 8, 298, 0, 32, 10),          # 7.9 against 11.9
+    (64, 1, 1, 513, 64, 4000, 512, 10), (64, 1, 1, 513, 64, 4000, 513, 8),
+    (128, 8, 2, 1, 80, 6665, 50, 11),        # 7.7 against 9.5
+    (128, 1, 1, 16, 35, 7284, 1000, 8),
+    (128, 16, 4, 2, 1827, 0, 49, 10),        # 15.7 against 21.2 with 2 x 2
+])
+def test_launches_in_a_window(head_dim, nq, nkv, reqs, q, behind, window, want):
+    lib = attention_library(head_dim)
+    assert lib.llmlab_attention_launch(BF16, nq, nkv, reqs, q, behind + q, window, CUS) == want
 
 
 @pytest.mark.parametrize("head_dim,nq,nkv,portion,behind,decoding,their_keys,want", [
