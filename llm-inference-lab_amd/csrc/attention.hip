@@ -1900,6 +1900,15 @@ static int launch_f32_key_split(AttnArgs a, int reqs, int live, int ctx_len, int
   return 0;
 }
 
+// Whether the blocks of a float32 step, keys split over a block's waves, come in the order of their tiles, the longest of all kv heads and
+// requests first, or request by request.  By tiles the units end together; but then the blocks of a request's kv head are far
+// apart, and once the keys and values of all of them, `pairs` times `seen` keys, are more than the caches of the dies hold, every tile reads them from
+// beyond (us, by tiles / by requests: 400 pairs of 741 keys of 64 numbers (152 MB) 2,389 / 1,430, 512 of 634 of 48 (125 MB) 1,889 / 1,150, 200 of
+// 1,194 of 48 (92 MB) 1,108 / 746; 128 of 1,021 of 32 (33 MB) 108 / 145; from 64 to 128 MB 0.82 of the time over 26 steps drawn at random, from 32 to 64 0.98, below
+// 1.03 to 1.06).
+static bool f32_tiles_first(long pairs, long seen) { return pairs * seen * D * 8 < 64L << 20; }
+extern "C" int llmlab_attention_f32_tiles_first(int pairs, int seen) { return f32_tiles_first(pairs, seen); }      // (for tests)
+
 // Which launch a float32 step of many rows takes: 1 = the waves of a block split the keys of a
 // tile, anything else = a wave per tile.  `blocks`: tiles of rows times kv heads times requests.
 static int choose_many_rows_launch_f32(long blocks, int max_q_len, int max_ctx_len, int num_cus, int forced) {
@@ -1960,7 +1969,9 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
     constexpr int PATH1_QB = D <= 64 ? 1 : F32_QB;
     const long path1_tiles = (max_rows + 16 * PATH1_QB - 1) / (16 * PATH1_QB), blocks = path1_tiles * a.nkv * zs;
     // (along x, the longest tiles of all requests first, where every request is this launch's)
-    const bool along_x = live == (long)zs && blocks <= 0xffffffffl / (64 * F32_SPLIT_WAVES);
+    const int seen = window > 0 ? min(max_ctx_len, window + max_q_len) : max_ctx_len;
+    const bool along_x = live == (long)zs && blocks <= 0xffffffffl / (64 * F32_SPLIT_WAVES) &&
+                         f32_tiles_first((long)a.nkv * zs, seen);
     const dim3 grid = along_x ? dim3((unsigned)blocks) : dim3((unsigned)path1_tiles, a.nkv, zs);
     if (D <= 64 && !(path1_tiles * a.nkv * live <= num_cus && max_ctx_len >= 768))
       hipLaunchKernelGGL((attention_f32_kernel<PATH1_QB, true, 4>), grid, dim3(64 * 4), 0, stream, a);

@@ -418,6 +418,16 @@ def test_launches_in_a_window(head_dim, nq, nkv, reqs, q, behind, window, want):
     assert lib.llmlab_attention_launch(BF16, nq, nkv, reqs, q, behind + q, window, CUS) == want
 
 
+@pytest.mark.parametrize("head_dim,pairs,seen,want", [
+    (64, 400, 741, 0),         # 2,389 us in the order of the tiles, 1,430 request by request
+    (48, 200, 1194, 0),        # 1,108 and 746
+    (32, 128, 1021, 1),        # 108 and 145
+    (64, 2, 65535, 1), (64, 2, 65536, 0), (16, 8, 65535, 1), (16, 8, 65536, 0),      # 64 MB of keys and values
+])
+def test_order_of_float32_blocks(head_dim, pairs, seen, want):
+    assert attention_library(head_dim).llmlab_attention_f32_tiles_first(pairs, seen) == want
+
+
 @pytest.mark.parametrize("head_dim,nq,nkv,portion,behind,decoding,their_keys,want", [
     # (us in two launches / in one with the portion by tiles of 32 rows / in one by tiles of 16; the rules are in
     # csrc/attention.hip.  2: two launches, 1: one by tiles of 32 rows, 3: one by tiles of 16)
