@@ -1910,8 +1910,8 @@ static bool f32_tiles_first(long pairs, long seen) { return pairs * seen * D * 8
 extern "C" int llmlab_attention_f32_tiles_first(int pairs, int seen) { return f32_tiles_first(pairs, seen); }      // (for tests)
 
 // Which launch a float32 step of many rows takes: 1 = the waves of a block split the keys of a
-// tile, anything else = a wave per tile.  `blocks`: tiles of rows times kv heads times requests.
-static int choose_many_rows_launch_f32(long blocks, int max_q_len, int max_ctx_len, int num_cus, int forced) {
+// tile, anything else = a wave per tile.  `max_rows`: of a request and kv head; `blocks`: tiles of rows times kv heads times requests.
+static int choose_many_rows_launch_f32(long max_rows, long blocks, int max_q_len, int max_ctx_len, int num_cus, int forced) {
   if (forced != 0) return forced;
   // (how few the keys must be for a wave per tile, by how many times the tiles fill the chip)
   int few_keys;
@@ -1921,10 +1921,18 @@ static int choose_many_rows_launch_f32(long blocks, int max_q_len, int max_ctx_l
   // 184, of 2,048 453 against 512, two of 1,024 290 against 305; four of 1,024 562 against 501)
   if (D > 64) few_keys = blocks > (max_q_len >= 1024 ? 7L : 2L) * num_cus ? 0x7fffffff
                          : blocks >= (7L * num_cus) / 4 && max_q_len < 1024 ? 128 : 0;
-  // (heads of 64: the key split takes 16 rows a block and loses only over a step or two of keys a wave, and where there are
-  // tiles for many rounds over few keys: 60 / 24 prompts of 128 tokens 46 / 21 us against 40 / 23, 100 / 40 of 64 33 / 16 against
-  // 31 / 17, 16 of 272 to 512 83 against 74; 32 of 200 46 both, 14 of 512 84 against 115, 8 of 1,000 151 against 191)
-  else few_keys = blocks >= 14L * num_cus ? 512 : blocks >= 10L * num_cus ? 128 : blocks >= (7L * num_cus) / 4 ? 64 : 0;
+  // (heads up to 64: the key split takes 16 rows a block and reads a tile's keys twice as often; it loses where tiles for many rounds
+  // walk few keys, us, key split / a wave per tile: heads of 64, 200 x 1 prompts of 45 tokens of 7 heads (2,000 blocks) 25.7 / 21.2, 256 of
+  // 121 of 2 (2,048) 33.6 / 26.4, 256 x 629 of 4 (20,224) 613 / 594, 64 of 456 of 7 (5,600) 150 / 153, 64 of 505 of 7 (7,200) 181 / 194; heads of 32, 128 x 123 of 4 (2,048)
+  // 22.6 / 16.6, 512 of 529 of 8 (59,392) 1,002 / 754, 128 of 749 of 2 (6,100) 127 / 152, 128 of 571 of 7 (16,000) 263 / 355; 256 of 134 of 2 heads of 64, whose last block of 128 rows is nearly empty, 35.5 / 41.9; 100 of 129 of 4 heads of 16 (1,700) 14.4 / 11.6.  Over 950 steps drawn at random
+  // the picks lose 1.1 % to the better one, 12 % at most)
+  else {
+    const long quarters = 4 * blocks / num_cus;      // (of a block a unit)
+    if (D == 64) few_keys = quarters >= 224 ? 1024 : quarters >= 56 ? 512 : quarters >= 28 ? 192 : quarters >= 14 ? 128 : quarters >= 7 ? 48 : 0;
+    else few_keys = quarters >= 400 ? 1024 : quarters >= 56 ? 512 : quarters >= 28 ? 256 : quarters >= 14 ? 192 : quarters >= 7 ? 64 : 0;
+    // (a block of four waves whose tiles are less than three quarters full)
+    if (few_keys > 128 && 4 * max_rows < 3 * ((max_rows + 127) / 128 * 128)) few_keys = 128;
+  }
   return max_ctx_len <= few_keys ? 2 : 1;
 }
 
@@ -1961,7 +1969,7 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
   // wave per tile, a prompt of 1,531 tokens 49 against 122.  A wave per tile wins once the
   // tiles fill the chip and the keys are few, at heads above 64 from two tiles a unit on whatever the
   // keys (4 requests of 256 tokens: 58 against 81).
-  const int path = choose_many_rows_launch_f32(tiles * a.nkv * live, max_q_len, max_ctx_len, num_cus, g_force_path);
+  const int path = choose_many_rows_launch_f32(max_rows, tiles * a.nkv * live, max_q_len, max_ctx_len, num_cus, g_force_path);
   if (path == 1) {
     // Heads up to 64: blocks of four waves and 16 rows, four to a unit; eight waves where the tiles leave units idle and
     // have histories to walk (us, four / eight waves: 100 tokens behind 1,000 keys 20.2 / 16.0, behind 3,000 48.5 / 35.5; 300
@@ -2195,7 +2203,7 @@ extern "C" int llmlab_attention_launch(int dtype, int nq, int nkv, int reqs, int
   if (max_rows <= 16) return 0;
   if (dtype == DT_F32) {
     constexpr int ROWS = 16 * F32_QB;
-    return choose_many_rows_launch_f32((max_rows + ROWS - 1) / ROWS * nkv * reqs, max_q_len, max_ctx_len, num_cus, 0);
+    return choose_many_rows_launch_f32(max_rows, (max_rows + ROWS - 1) / ROWS * nkv * reqs, max_q_len, max_ctx_len, num_cus, 0);
   }
   return many_rows_launch(max_rows, nkv, reqs, max_q_len, max_ctx_len, window, false, num_cus, 0);
 }

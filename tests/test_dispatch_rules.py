@@ -390,9 +390,27 @@ def test_attention_launch_is_one_the_head_size_has(head_dim, nq, nkv):
     (96, 28, 4, BF16, 1, 128, 1024, 6),      # (heads beside them: as those were measured without staged keys)
     (96, 28, 4, BF16, 1, 128, 2560, 1), (96, 28, 4, BF16, 8, 128, 0, 2), (96, 28, 4, BF16, 1, 64, 0, 4),
     (48, 14, 2, BF16, 1, 512, 1536, 1), (48, 14, 2, BF16, 1, 2048, 0, 6), (48, 14, 2, BF16, 1, 8192, 0, 2), (48, 14, 2, BF16, 16, 64, 0, 4),
-    (64, 14, 2, F32, 1, 512, 1024, 1),       # 43 us against 162
-    (64, 14, 2, F32, 1, 2048, 0, 1),         # 117 against 217
-    (64, 14, 2, F32, 16, 512, 0, 2),         # 137 against 187
+    (64, 14, 2, F32, 1, 512, 1024, 1),       # 31 us against 120
+    (64, 14, 2, F32, 1, 1531, 0, 1),         # 49 against 122
+    (64, 14, 2, F32, 16, 512, 0, 2),         # (3,584 blocks of 32 rows)
+    (64, 8, 4, F32, 64, 121, 0, 2),          # 26.4 against 33.6 with the key split
+    (64, 16, 4, F32, 64, 629, 0, 2),         # 594 against 613
+    (64, 56, 8, F32, 8, 505, 0, 2), (64, 56, 8, F32, 8, 513, 0, 1),
+    (64, 8, 4, F32, 64, 134, 0, 1),          # 35.5 against 41.9: a last block of 12 rows
+    (32, 32, 8, F32, 16, 123, 0, 2),         # 16.6 against 22.6
+    (32, 64, 8, F32, 64, 464, 65, 2),        # 754 against 1,002
+    (32, 4, 2, F32, 64, 749, 0, 1),          # 127 against 152
+    (32, 14, 2, F32, 64, 571, 0, 1),         # 263 against 355
+    # (borders, tiles of 32 rows by fours)
+    (64, 4, 1, F32, 112, 32, 16, 2), (64, 4, 1, F32, 111, 32, 16, 1), (64, 4, 1, F32, 112, 32, 17, 1),
+    (64, 4, 1, F32, 224, 32, 96, 2), (64, 4, 1, F32, 223, 32, 96, 1), (64, 4, 1, F32, 224, 32, 97, 1),
+    (64, 4, 1, F32, 448, 32, 160, 2), (64, 4, 1, F32, 447, 32, 160, 1), (64, 4, 1, F32, 448, 32, 161, 1),
+    (64, 4, 1, F32, 896, 32, 480, 2), (64, 4, 1, F32, 895, 32, 480, 1), (64, 4, 1, F32, 896, 32, 481, 1),
+    (64, 4, 1, F32, 3584, 32, 992, 2), (64, 4, 1, F32, 3583, 32, 992, 1), (64, 4, 1, F32, 3584, 32, 993, 1),
+    (64, 3, 1, F32, 600, 32, 160, 2), (64, 3, 1, F32, 600, 31, 161, 1), (64, 3, 1, F32, 600, 31, 97, 2),
+    (32, 4, 1, F32, 112, 32, 32, 2), (32, 4, 1, F32, 112, 32, 33, 1), (32, 4, 1, F32, 224, 32, 160, 2), (32, 4, 1, F32, 224, 32, 161, 1),
+    (32, 4, 1, F32, 448, 32, 224, 2), (32, 4, 1, F32, 448, 32, 225, 1), (32, 4, 1, F32, 6400, 32, 992, 2), (32, 4, 1, F32, 6400, 32, 993, 1),
+    (32, 4, 1, F32, 6399, 32, 481, 1),
     (128, 28, 4, F32, 4, 256, 0, 2),         # 58 against 81
     (128, 28, 4, F32, 1, 256, 1024, 1),      # 77 against 226
     (128, 28, 4, F32, 1, 1024, 0, 1),        # a long portion's tiles are uneven: 148 against 184
