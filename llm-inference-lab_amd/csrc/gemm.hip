@@ -2124,9 +2124,9 @@ extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
 //   of 11008 x 2048 77.9 / 74.2 (not 1,024 of 17920 x 1536, 1.64 rounds, 66.8 / 69.2; 384 of 37888 x 3584 137 / 141).
 //   128 x 192, a block a unit, where 192 x 128 has more than units: 640 of 9728 x 896 18.7 / 16.7, 256 of 17920 x 1536 26.8 / 23.3,
 //   512 of 11008 x 2048 34.2 / 32.0.
-// (Weights from memory and not from the caches.  An MI355X has 256 units.)
-static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads) {
-  constexpr long UNITS = 256;
+// (Weights from memory and not from the caches.)
+static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads, int num_cus) {
+  const long UNITS = num_cus;
   if (K > DIRECT_MAX_INNER) return kind;
   if (g_force_tile >= 138 && g_force_tile <= 140) {
     const int forced = TILE_DIRECT_128 + (g_force_tile - 138);
@@ -2146,15 +2146,15 @@ static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads) {
   return kind;
 }
 // ... its code above (for tests; -1: the tile stays)
-extern "C" int llmlab_direct_tile(int kind, int M, int N, int K, int pieces, int heads) {
-  const int tile = direct_tile(kind, M, N, K, pieces, heads != 0);
+extern "C" int llmlab_direct_tile(int kind, int M, int N, int K, int pieces, int heads, int num_cus) {
+  const int tile = direct_tile(kind, M, N, K, pieces, heads != 0, num_cus > 0 ? num_cus : 256);
   return tile == kind ? -1 : tile;
 }
 
 template <int EPI>
 static void launch_tile(int kind, const bf16_t* A, const bf16_t* W, const EpiArgs& e, int M, int N, int K,
-                        int pieces, hipStream_t stream) {
-  kind = direct_tile(addressable(kind, K), M, N, K, pieces, EPI == EPI_QKV);      // (a tile that the caller names)
+                        int pieces, int num_cus, hipStream_t stream) {
+  kind = direct_tile(addressable(kind, K), M, N, K, pieces, EPI == EPI_QKV, num_cus);      // (a tile that the caller names)
   const TileModel& t = TILE_MODELS[kind];
   dim3 grid((N + t.bn - 1) / t.bn, (M + t.bm - 1) / t.bm, pieces);
   if (kind == TILE_64)
@@ -2384,7 +2384,7 @@ extern "C" int llmlab_linear_qkv(const void* x, const void* w, const void* bias,
   const int kind = heads_tile(M, N, K, d, num_cus);
   LLMLAB_REQUIRE(TILE_MODELS[kind].bn % d == 0, "linear_qkv: heads of %d do not divide the tile of %d columns", d,
                  TILE_MODELS[kind].bn);
-  launch_tile<EPI_QKV>(kind, (const bf16_t*)x, (const bf16_t*)w, e, M, N, K, 1, stream);
+  launch_tile<EPI_QKV>(kind, (const bf16_t*)x, (const bf16_t*)w, e, M, N, K, 1, num_cus, stream);
   LLMLAB_LAUNCH_CHECK("linear_qkv");
   return 0;
 }
@@ -2398,6 +2398,17 @@ extern "C" int llmlab_linear_tile(int M, int N, int K, int num_cus) {
 // ... and that llmlab_linear_qkv takes for heads of d: for callers that must know whether a head fits it.
 extern "C" int llmlab_linear_heads_tile(int M, int N, int K, int d, int num_cus) {
   return TILE_MODELS[heads_tile(M, N, K, d > 0 ? d : 1, num_cus > 0 ? num_cus : 256)].bn;
+}
+
+// The compute units of the chip (for a call that does not name them).
+static int chip_units() {
+  static const int units = [] {
+    int device = 0, n = 0;
+    const bool known = hipGetDevice(&device) == hipSuccess &&
+                       hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess;
+    return known && n > 0 ? n : 256;
+  }();
+  return units;
 }
 
 // parts[z] = x[:, K_z] . W[:, K_z]^T for `ksplit` ranges K_z of the inner size (whole K
@@ -2425,7 +2436,7 @@ extern "C" int llmlab_linear_partials(const void* x, const void* w, int dtype, f
   const int nk = (K + 63) / 64;
   EpiArgs e{parts, bias, bias_dtype == DT_BF16, ldo, N, (nk + ksplit - 1) / ksplit, part_stride,
             nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
-  launch_tile<EPI_PART>(tile, (const bf16_t*)x, (const bf16_t*)w, e, M, N, K, ksplit, stream);
+  launch_tile<EPI_PART>(tile, (const bf16_t*)x, (const bf16_t*)w, e, M, N, K, ksplit, chip_units(), stream);
   LLMLAB_LAUNCH_CHECK("linear_partials");
   return 0;
 }
@@ -2462,10 +2473,10 @@ extern "C" int llmlab_linear(const void* x, const void* w, int dtype, int epilog
     const bf16_t* W = (const bf16_t*)w;
     const int kind = plain_tile(M, N, K, num_cus);
     switch (epilogue) {
-      case EPI_STORE: launch_tile<EPI_STORE>(kind, A, W, e, M, N, K, 1, stream); break;
-      case EPI_RESID: launch_tile<EPI_RESID>(kind, A, W, e, M, N, K, 1, stream); break;
-      case EPI_F32: launch_tile<EPI_F32>(kind, A, W, e, M, N, K, 1, stream); break;
-      default: launch_tile<EPI_SWIGLU>(kind, A, W, e, M, N, K, 1, stream); break;
+      case EPI_STORE: launch_tile<EPI_STORE>(kind, A, W, e, M, N, K, 1, num_cus, stream); break;
+      case EPI_RESID: launch_tile<EPI_RESID>(kind, A, W, e, M, N, K, 1, num_cus, stream); break;
+      case EPI_F32: launch_tile<EPI_F32>(kind, A, W, e, M, N, K, 1, num_cus, stream); break;
+      default: launch_tile<EPI_SWIGLU>(kind, A, W, e, M, N, K, 1, num_cus, stream); break;
     }
   } else {
     const float* A = (const float*)x;

@@ -6,7 +6,6 @@ import pytest
 
 from test_dispatch_rules import core      # noqa: F401 (fixture)
 
-UNITS = 256
 SHAPES = {10: (128, 128), 11: (128, 192), 12: (192, 128)}
 
 
@@ -19,7 +18,13 @@ SHAPES = {10: (128, 128), 11: (128, 192), 12: (192, 128)}
     (4, 2048, 37888, 3584, 1, -1), (1, 384, 9728, 2 ** 22 + 8, 1, -1),
 ])
 def test_measured(core, kind, m, n, k, pieces, want):      # noqa: F811
-    assert core.llmlab_direct_tile(kind, m, n, k, pieces, 0) == want
+    assert core.llmlab_direct_tile(kind, m, n, k, pieces, 0, 256) == want
+
+
+def test_units_are_the_callers(core):      # noqa: F811
+    """228 blocks of 128 x 128 on chips of 228 units and of one less; 228 of 192 x 128 likewise."""
+    assert core.llmlab_direct_tile(1, 384, 9728, 896, 1, 0, 228) == 10 and core.llmlab_direct_tile(1, 384, 9728, 896, 1, 0, 227) != 10
+    assert core.llmlab_direct_tile(1, 512, 9728, 896, 1, 0, 228) == 12 and core.llmlab_direct_tile(1, 512, 9728, 896, 1, 0, 227) == 11
 
 
 def test_only_where_their_blocks_find_a_place(core):      # noqa: F811
@@ -27,13 +32,13 @@ def test_only_where_their_blocks_find_a_place(core):      # noqa: F811
     for _ in range(20000):
         kind, heads = rng.randint(0, 5), rng.randint(0, 1)
         m, n, k = rng.randint(1, 3000), rng.randint(1, 40000), 8 * rng.randint(1, 2500)
-        pieces = rng.choice([1, 1, 2, 4, 8])
-        tile = core.llmlab_direct_tile(kind, m, n, k, pieces, heads)
+        pieces, units = rng.choice([1, 1, 2, 4, 8]), rng.choice([256, 256, 304, 228, 64])
+        tile = core.llmlab_direct_tile(kind, m, n, k, pieces, heads, units)
         if tile < 0:
             continue
         seen.add((kind, tile))
         bm, bn = SHAPES[tile]
         blocks = -(-m // bm) * -(-n // bn) * pieces
         assert m > 64 and (not heads or tile == 10)
-        assert blocks <= UNITS or (kind == 5 and pieces == 1 and k <= 2048), (kind, m, n, k, pieces, tile)
+        assert blocks <= units or (kind == 5 and pieces == 1 and k <= 2048), (kind, m, n, k, pieces, tile)
     assert seen == {(1, 10), (2, 10), (1, 11), (1, 12), (5, 12)}

@@ -35,7 +35,7 @@ def test_paired_products(ops, emu, tile, activation, m, inter, k, pad):      # n
                                             (1900, 9728, 896, 133, 12)])
 def test_same_results_as_the_tile_before(ops, m, n, k, old, tile):      # noqa: F811
     kind = {130: 1, 133: 5}[old]
-    assert ops._core.llmlab_direct_tile(kind, m, n, k, 1, 0) == tile
+    assert ops._core.llmlab_direct_tile(kind, m, n, k, 1, 0, ops.num_cus) == tile
     gen = torch.Generator(device=DEV).manual_seed(m)
     x = torch.randn(m, k, device=DEV, generator=gen).bfloat16()
     w = ops.prepare_weight(torch.randn(n, k, device=DEV, generator=gen).bfloat16())
