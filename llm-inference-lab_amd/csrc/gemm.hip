@@ -2117,7 +2117,10 @@ extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
 //   128 x 128, a block a unit, in place of 64 x 128 and 128 x 128 in one round, whole or in pieces (beyond 64 rows; us
 //   before / with it): 384 rows of 9728 x 896 13.6 / 11.8, 256 of 11008 x 2048 24.3 / 21.1, 2,048 of 896 x 4864 in two pieces
 //   32.0 / 26.8, 384 of 2048 x 11008 in four 34.5 / 27.5, 457 of 3584 x 18944 in two 114 / 84.  Beyond one round it loses (512 of
-//   9728 x 896, 304 blocks, 17.6 / 21.2).
+//   9728 x 896, 304 blocks, 17.6 / 21.2), and where the blocks of 64 x 128 find a unit each, whose chains are half as long,
+//   as long as the matrix is small (656 of 2048 x 1536, 176 blocks, as q/k/v 16.0 / 17.2, 762 of 2560 x 2048 19.8 / 21.3, 1,384 of 896 x 4864
+//   36.4 / 37.6; from 24 MB on W read once a tile of rows counts for more: 154 of 4608 x 3584, 108, 25.1 / 22.8, 520 of 2048 x 11008, 144, 90.9 / 81.8).
+//   Over 376 products drawn at random 0.83 of the time, 1.04 at most.
 //   192 x 128, two blocks a unit, in place of a 64 x 128 tile of more than two blocks a unit where its own find a unit each: 512 rows
 //   of 9728 x 896 17.6 / 15.0, 1,024 of 4864 x 896 18.2 / 15.2, 384 of 11008 x 2048 32.5 / 28.5; and of 192 x 256 whose last round is
 //   less than half full, of up to three, at inner sizes to 2,048: 1,900 of 9728 x 896 43.8 / 39.0, 900 of 17920 x 1536 63.4 / 56.1, 1,536
@@ -2134,7 +2137,9 @@ static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads, in
   }
   if (g_force_tile != 0 || g_without_wide || M <= 64) return kind;
   auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * pieces; };
-  if ((kind == TILE_64x128 || kind == TILE_128) && blocks(128, 128) <= UNITS) return TILE_DIRECT_128;
+  if ((kind == TILE_128 || (kind == TILE_64x128 && (blocks(64, 128) > UNITS || (double)N * K * 2.0 >= 24e6))) &&
+      blocks(128, 128) <= UNITS)
+    return TILE_DIRECT_128;
   if (heads) return kind;
   if (kind == TILE_64x128 && blocks(64, 128) > 2 * UNITS) {
     if (blocks(192, 128) <= UNITS) return TILE_DIRECT_192x128;

@@ -14,6 +14,9 @@ SHAPES = {10: (128, 128), 11: (128, 192), 12: (192, 128)}
     (1, 384, 9728, 896, 1, 10), (1, 256, 11008, 2048, 1, 10), (1, 2048, 896, 4864, 2, 10), (2, 457, 3584, 18944, 2, 10),
     (1, 512, 9728, 896, 1, 12), (1, 1024, 4864, 896, 1, 12), (5, 1900, 9728, 896, 1, 12), (5, 900, 17920, 1536, 1, 12),
     (1, 640, 9728, 896, 1, 11), (1, 256, 17920, 1536, 1, 11),
+    (1, 656, 2048, 1536, 1, -1), (1, 762, 2560, 2048, 1, -1), (1, 1384, 896, 4864, 1, -1),      # 64 x 128 finds a unit for every block
+    (1, 520, 2048, 11008, 1, 10), (1, 154, 4608, 3584, 1, 10), (2, 656, 2048, 1536, 1, 10),
+    (1, 1024, 2048, 1536, 1, -1), (1, 1025, 2048, 1536, 1, 10), (1, 1024, 2048, 5856, 1, -1), (1, 1024, 2048, 5864, 1, 10),
     (5, 1024, 17920, 1536, 1, -1), (5, 384, 37888, 3584, 1, -1), (1, 64, 896, 4864, 2, -1), (0, 512, 896, 896, 1, -1),
     (4, 2048, 37888, 3584, 1, -1), (1, 384, 9728, 2 ** 22 + 8, 1, -1),
 ])
