@@ -2133,7 +2133,8 @@ static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads, in
   if (K > DIRECT_MAX_INNER) return kind;
   if (g_force_tile >= 138 && g_force_tile <= 140) {
     const int forced = TILE_DIRECT_128 + (g_force_tile - 138);
-    return heads && forced != TILE_DIRECT_128 ? kind : forced;
+    // (heads: columns that they divide, as they divide those of the tile that was named)
+    return heads && (forced != TILE_DIRECT_128 || TILE_MODELS[kind].bn > 128) ? kind : forced;
   }
   if (g_force_tile != 0 || g_without_wide || M <= 64) return kind;
   auto blocks = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * pieces; };

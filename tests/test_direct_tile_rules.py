@@ -45,3 +45,15 @@ def test_only_where_their_blocks_find_a_place(core):      # noqa: F811
         assert m > 64 and (not heads or tile == 10)
         assert blocks <= units or (kind == 5 and pieces == 1 and k <= 2048), (kind, m, n, k, pieces, tile)
     assert seen == {(1, 10), (2, 10), (1, 11), (1, 12), (5, 12)}
+
+
+def test_a_forced_tile_holds_whole_heads(core):      # noqa: F811
+    """Forced for a product written by heads: 128 x 128 where the named tile is no wider (a head of 256 fits one of 256 columns)."""
+    for force, tile in ((138, 10), (139, 11), (140, 12)):
+        core.llmlab_debug_gemm_tile(force)
+        try:
+            for kind in range(6):
+                assert core.llmlab_direct_tile(kind, 200, 1024, 256, 1, 0, 256) == tile
+                assert core.llmlab_direct_tile(kind, 200, 1024, 256, 1, 1, 256) == (10 if force == 138 and kind < 3 else -1)
+        finally:
+            core.llmlab_debug_gemm_tile(0)

@@ -1,12 +1,12 @@
 """The tiles of eight waves whose operands come by direct loads (138: 128 x 128, 139: 128 x 192, 140: 192 x 128): inner sizes
-around their rings, rows and columns that fill no block, every epilogue; and to the bit what the tile gives that they
-stand in for, since every sum has the same order."""
+around their rings, rows and columns that fill no block, every epilogue (q, k and v by heads: 128 x 128, the one of them that
+takes it); and to the bit what the tile gives that they stand in for, since every sum has the same order."""
 import pytest
 import torch
 
 import test_direct_load_tiles_gpu as direct
 import test_register_epilogue_gpu as epilogue
-from test_kernels_gpu import DEV, emu, ops      # noqa: F401 (fixtures)
+from test_kernels_gpu import DEV, check_qkv_rope_cache, emu, ops      # noqa: F401 (fixtures)
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,56 @@ def test_same_results_as_the_tile_before(ops, m, n, k, old, tile):      # noqa: 
     with ops.debug.force(gemm_tile=old):
         ops.linear_swiglu(x, w, want)
     assert torch.equal(got, want)
+
+
+QKV_STARTS = [([70, 1, 130], (3, 40, 0, 7)), ([300, 2, 2, 90], (3, 40, 0, 7)),
+              # (values of four positions written together: starts and rows that line up, that do not, and short requests between)
+              ([72, 4, 124], (0, 64, 8)), ([70, 6, 125], (2, 61, 9)), ([8, 4, 4, 180], (12, 0, 28, 100))]
+MORE_ROWS = [([300, 2, 2, 90], (3, 40, 0, 7)), ([272, 4, 124], (0, 64, 8)), ([270, 6, 125], (2, 61, 9)), ([200, 4, 4, 190], (12, 0, 28, 100))]
+
+
+@pytest.mark.parametrize("nq,nkv,d,page,hidden", [(4, 2, 16, 16, 64), (7, 1, 32, 16, 72), (14, 2, 64, 64, 896)])
+@pytest.mark.parametrize("rows_per,starts", QKV_STARTS)
+def test_queries_keys_and_values(ops, emu, nq, nkv, d, page, hidden, rows_per, starts):      # noqa: F811
+    """Bias, rotation and the write into the cache; two to eight heads a tile of 128 columns, rows that end inside a tile."""
+    with ops.debug.force(gemm_tile=138, few_rows_max=64, qkv_pieces_min_rows=1 << 30):
+        assert ops.can_fuse_qkv_rope(sum(rows_per), torch.bfloat16, d, (nq + 2 * nkv) * d, hidden)
+        check_qkv_rope_cache(ops, emu, nq, nkv, d, page, hidden, rows_per, starts)
+
+
+def qkv_by(ops, tile, nq, nkv, d, page, hidden, rows_per, starts):      # noqa: F811
+    """q, the keys and the values of a step by this tile (0: by the rule), what was there before included."""
+    rows, n, reqs = sum(rows_per), (nq + 2 * nkv) * d, len(rows_per)
+    ints, gen = dict(dtype=torch.int32, device=DEV), torch.Generator(device=DEV).manual_seed(rows)
+    h, b = (torch.randn(*s, device=DEV, generator=gen).bfloat16() for s in ((rows, hidden), (n,)))
+    w = ops.prepare_weight(torch.randn(n, hidden, device=DEV, generator=gen).bfloat16())
+    need = [(s + r + page - 1) // page for s, r in zip(starts, rows_per)]
+    table = torch.full((reqs, max(need)), -1, dtype=torch.int32)
+    for i in range(reqs):
+        table[i, :need[i]] = torch.arange(sum(need[:i]), sum(need[:i + 1])).int()
+    positions = torch.cat([torch.arange(s, s + r) for s, r in zip(starts, rows_per)]).to(**ints)
+    row_req = torch.cat([torch.full((r,), i) for i, r in enumerate(rows_per)]).to(**ints)
+    kc, vc = (torch.randn(sum(need), nkv, *s, device=DEV, generator=gen).bfloat16() for s in ((page, d), (d, page)))
+    q = torch.zeros(rows, nq * d, device=DEV, dtype=torch.bfloat16)
+    inv_freq = (1e4 ** (-torch.arange(0, d, 2, device=DEV).double() / d)).float()
+    with ops.debug.force(gemm_tile=tile, few_rows_max=64, qkv_pieces_min_rows=1 << 30):
+        assert ops._core.llmlab_linear_heads_tile(rows, n, hidden, d, ops.num_cus) == 128
+        ops.qkv_rope_cache(h, w, b, nq, nkv, d, inv_freq, positions, row_req, table.to(DEV), page, kc, vc, q)
+    return q, kc, vc
+
+
+@pytest.mark.parametrize("nq,nkv,page", [(22, 1, 16), (8, 8, 64)])
+@pytest.mark.parametrize("rows_per,starts", MORE_ROWS)
+def test_a_head_a_tile(ops, nq, nkv, page, rows_per, starts):      # noqa: F811
+    """Heads of 128: to the bit what the tile of four waves gives, everywhere in the caches."""
+    hidden = 1536
+    got, want = (qkv_by(ops, tile, nq, nkv, 128, page, hidden, rows_per, starts) for tile in (138, 129))
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+@pytest.mark.parametrize("rows,nq,nkv,hidden", [(1093, 16, 2, 2048), (1242, 12, 2, 1536), (603, 32, 8, 4096)])
+def test_queries_keys_and_values_by_the_rule(ops, rows, nq, nkv, hidden):      # noqa: F811
+    """Sizes that the rule sends to 128 x 128: to the bit what the tile before gives."""
+    assert ops._core.llmlab_direct_tile(1, rows, (nq + 2 * nkv) * 128, hidden, 1, 1, ops.num_cus) == 10
+    got, want = (qkv_by(ops, tile, nq, nkv, 128, 64, hidden, [rows - 7, 7], (5, 90)) for tile in (0, 130))
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
