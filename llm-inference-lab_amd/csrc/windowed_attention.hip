@@ -1591,10 +1591,19 @@ static void launch_mfma_any(int D, int E, int which, dim3 grid, dim3 block, hipS
 // heads of 64 (14 over 2), 512 rows (128 blocks) 18.8 / 14.5, 1,000 (252) 32.7 / 24.2, 1,900 over a window of 1,024 (476) 41.6 / 35.0,
 // three prompts of 2,367 rows (592) 39.8 / 33.2, 4,096 (1,024) 58.7 / 64.6; of 128 (16 over 2), 64 rows 7.3 / 7.6, 200 12.5 / 11.3, 1,000 (252)
 // 40.5 / 30.1, 1,900 (476) 51.2 / 60.1: their registers let a unit hold one block of two groups.
-static bool two_groups(int D, int E, int rows, long blocks, int num_cus) {
+// Not where the second group has nothing or little to do, by `max_keys`, the most keys that a row sees (0: not known): a tile at heads up
+// to 64 (20 rows from their start 5.15 / 5.61, 384 rows of 16 requests 6.92 / 7.41; 38 keys 7.1 / 6.9), two and a bit of wider ones (27 keys
+// 7.0 / 7.9, 53 9.35 / 9.79, 72 equal, a window of 64 and 8 kept 9.5 / 8.7), and four where units have more than a block (4,144 rows over a window of 64,
+// 518 blocks, 10.9 / 12.9, 1,504 of 94 keys, 376, 8.8 / 9.2; 152 keys, 416, 0.95).
+static bool two_groups(int D, int E, int rows, long blocks, int max_keys, int num_cus) {
   if (num_cus <= 0) num_cus = 256;
-  if (D <= 64 && E <= 64) return 2 * blocks <= 5L * num_cus;
-  return rows >= 96 && blocks <= num_cus;
+  if (max_keys <= 0) max_keys = 1 << 30;
+  if (D <= 64 && E <= 64) return 2 * blocks <= 5L * num_cus && max_keys > (blocks > num_cus ? 128 : 32);
+  return rows >= 96 && blocks <= num_cus && max_keys >= 72;
+}
+static long shared_blocks(int rows, int n_heads, int n_kv) { return (long)((rows + 15) / 16) * n_kv * ((n_heads / n_kv + 3) / 4); }
+extern "C" int llmlab_windowed_two_groups(int D, int E, int rows, int n_heads, int n_kv, int max_keys, int num_cus) {      // (for tests)
+  return two_groups(D, E, rows, shared_blocks(rows, n_heads, n_kv), max_keys, num_cus);
 }
 
 // q [rows, heads * D], out [rows, heads * E] in the compute dtype; sink: float32 [heads] or null.
@@ -1602,8 +1611,8 @@ static bool two_groups(int D, int E, int rows, long blocks, int num_cus) {
 // long_from > 0 (sizes that the matrix-core kernels take only): requests that bring at least so
 // many rows (q_start[b + 1] - q_start[b]) go to the prompts' kernel, the others to the decoding
 // one; `launches` says which of the two the step needs (bit 0 decoding, bit 1 prompts).
-// max_keys: the most keys a decoding row of this step sees (it sets how many shares a row's
-// keys are cut into); workspace: float32 scratch for the shares' partial results.
+// max_keys: the most keys a row of this step sees (it sets how many shares a decoding row's
+// keys are cut into, and how many groups of waves a prompts' block has; 0: not known); workspace: float32 scratch for the shares' partial results.
 extern "C" int llmlab_sink_window_attention(const void* q, int dtype, int rows, int n_heads, int n_kv, int D, int E,
                                             const void* k_cache, const void* v_cache, const int* table, int max_pages,
                                             int page_size, const int* positions, const int* row_req, int window,
@@ -1636,10 +1645,10 @@ extern "C" int llmlab_sink_window_attention(const void* q, int dtype, int rows, 
     if (launches & 2) {
       // heads that read the same keys and values share the tiles a block stages in LDS
       const int group = n_heads / n_kv;
-      const long blocks = (long)((rows + 15) / 16) * n_kv * ((group + 3) / 4);
+      const long blocks = shared_blocks(rows, n_heads, n_kv);
       const bool fit = D <= 128 && E <= 128;
       if (!g_private_tiles && group >= 3)
-        launch_mfma_any(D, E, fit && (g_groups > 0 ? g_groups == 2 : two_groups(D, E, rows, blocks, num_cus)) ? 3 : 2,
+        launch_mfma_any(D, E, fit && (g_groups > 0 ? g_groups == 2 : two_groups(D, E, rows, blocks, max_keys, num_cus)) ? 3 : 2,
                         dim3((rows + 15) / 16, n_kv * ((group + 3) / 4)), dim3(256), stream, a);
       else
         launch_mfma_any(D, E, 0, dim3((rows + 63) / 64, n_heads), dim3(256), stream, a);

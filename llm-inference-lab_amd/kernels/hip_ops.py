@@ -1612,7 +1612,8 @@ class HipOps:
         requests that bring at least so many rows (by ``q_start``) are served in tiles of 16 rows
         of a head, the others a row and a group of heads at a time with the row's keys cut into
         shares; ``launches``: which of the two this step needs (bit 0 few rows, bit 1 many);
-        ``max_keys``: the most keys a row of this step sees (sets the number of shares)."""
+        ``max_keys``: the most keys a row of this step sees (sets the number of shares, and of groups of waves a block; 0: not
+        known)."""
         lib = self._mixer_lib("windowed_attention")
         if long_from:
             self._need(q_start, "request row starts", torch.int32)

@@ -541,3 +541,27 @@ def test_a_forced_float32_tile_is_planned_at_any_size(core, tile, kind):
             assert out[1] == kind and 1 <= out[0] <= 8, (m, n, k, out[0], out[1])
     finally:
         core.llmlab_debug_gemm_tile(0)
+
+
+@pytest.mark.parametrize("dim,values,rows,heads,kv_heads,keys,want", [
+    # (us with one group of waves a block / with two: csrc/windowed_attention.hip)
+    (64, 64, 20, 14, 2, 20, 0),              # 5.15 / 5.61
+    (64, 64, 384, 14, 2, 24, 0),             # 6.92 / 7.41
+    (64, 64, 512, 14, 2, 512, 1),            # 18.8 / 14.5
+    (64, 64, 1900, 14, 2, 1032, 1),          # 41.6 / 35.0
+    (64, 64, 4096, 14, 2, 4096, 0),          # 58.7 / 64.6
+    (64, 64, 4144, 8, 1, 72, 0),             # 10.85 / 12.89
+    (64, 64, 1024, 14, 2, 32, 0), (64, 64, 1024, 14, 2, 33, 1), (64, 64, 1025, 14, 2, 128, 0), (64, 64, 1025, 14, 2, 129, 1),
+    (64, 64, 2560, 14, 2, 2560, 1), (64, 64, 2561, 14, 2, 2561, 0), (64, 64, 20, 14, 2, 0, 1),
+    (128, 64, 120, 8, 2, 30, 0),             # 6.96 / 7.90
+    (128, 128, 1000, 16, 2, 1000, 1),        # 40.5 / 30.1
+    (128, 128, 1900, 16, 2, 1032, 0),        # 51.2 / 60.1
+    (96, 96, 164, 28, 4, 72, 1),              # 9.51 / 8.66
+    (128, 128, 96, 16, 2, 72, 1), (128, 128, 96, 16, 2, 71, 0), (128, 128, 95, 16, 2, 72, 0),
+])
+def test_groups_of_waves_of_windowed_attention(dim, values, rows, heads, kv_heads, keys, want):
+    try:
+        lib = ctypes.CDLL(build.mixer_library("windowed_attention"))
+    except (OSError, RuntimeError) as err:
+        pytest.skip(f"the library does not load here: {err}")
+    assert lib.llmlab_windowed_two_groups(dim, values, rows, heads, kv_heads, keys, CUS) == want
