@@ -1813,8 +1813,10 @@ static KeySplitLaunch prepare_key_split_decode(AttnArgs a, int reqs, int live, i
   // requests behind 1,400 keys (350 KB) 12.0 / 9.7, 28 12.7 / 10.8, behind 2,100 16.9 / 13.0; 40 behind 1,700 (425 KB) 15.8 / 14.1,
   // 64 17.1 / 16.2, behind 1,300 13.9 / 14.0; heads of 128 over 2, 28 behind 900 (450 KB) 15.1 / 12.6; 40 behind 1,400 (700 KB) 22.5 / 18.2,
   // 48 behind 1,000 16.8 / 16.5, 56 behind 1,400 24.1 / 27, behind 1,700 27.7 / 24.8.
-  // Beside portions the units have other work: there a split asks for twice as much (48 requests at 1,500 beside 464 tokens
-  // 15.2 / 20.7, 32 at 2,000 17.5 / 19.1).
+  // (Over 300 steps of 300 to 800 KB a block drawn at random, heads of 16 to 256, 4 to 128 requests times kv heads, 0.88 of the time with
+  // 384 KB, and 768 for up to four splits; 1.04 at most.)
+  // Beside portions the units have other work (48 requests at 1,500 beside 464 tokens 15.2 / 20.7, 32 at 2,000 17.5 / 19.1): there
+  // up to four splits ask for 768 KB and more for 384, as decoding steps did before they were measured alone.
   const size_t block_bytes = (size_t)visible * D * 2 * sizeof(bf16_t);
   const size_t least = live < reqs ? (splits <= 4 ? 768 : 384)
                        : splits > 2 ? 320 : D <= 64 ? 384 : 8 * base <= 3L * num_cus ? 600 : 768;      // KB
@@ -1842,6 +1844,13 @@ static KeySplitLaunch prepare_key_split_decode(AttnArgs a, int reqs, int live, i
   }
   const int steps_per_wave = ((steps32 + splits - 1) / splits + DECODE_WAVES - 1) / DECODE_WAVES;
   return KeySplitLaunch{a, steps_per_wave > 2 ? 2 : 1, splits > 1 && !merge_in_place};
+}
+
+// Into how many splits a step goes whose `live` requests of `reqs` decode, behind at most `ctx_len` keys (for tests).
+extern "C" int llmlab_attention_decode_splits(int nq, int nkv, int reqs, int live, int ctx_len, int window, int num_cus) {
+  if (nq <= 0 || nkv <= 0 || nq % nkv != 0 || live <= 0 || live > reqs || ctx_len <= 0) return -1;
+  return prepare_key_split_decode(AttnArgs{}, reqs, live, ctx_len, window, reqs, nq, nkv, nullptr, ~(size_t)0 >> 8,
+                                  num_cus > 0 ? num_cus : 256, nullptr, 0).a.splits;
 }
 
 static int launch_split_merge(const KeySplitLaunch& k, int total_rows, int nq, const int* row_req, void* out,

@@ -485,6 +485,28 @@ def test_measured_launches_of_a_mixed_step(head_dim, nq, nkv, portion, behind, d
     assert lib.llmlab_attention_mixed_launches(nq, nkv, 4, 4, portion, behind + portion, their_keys, 0, CUS) == 0
 
 
+@pytest.mark.parametrize("head_dim,nkv,reqs,beside,keys,want", [
+    # (a block reads keys times 4 times the head size bytes; us unsplit / split in csrc/attention.hip)
+    (64, 2, 20, 0, 1400, 6),                 # 12.0 / 9.7
+    (64, 2, 20, 0, 1280, 6), (64, 2, 20, 0, 1279, 1),         # 320 KB where three splits and more are to be had
+    (64, 2, 42, 0, 1280, 3), (64, 2, 42, 0, 1279, 1),
+    (64, 2, 43, 0, 1536, 2), (64, 2, 43, 0, 1535, 1),         # 384 KB with two, at heads up to 64
+    (64, 2, 64, 0, 1700, 2),                 # 17.1 / 16.2
+    (64, 2, 65, 0, 4096, 1),                 # (more blocks than half the units)
+    (128, 2, 40, 0, 1400, 3),                # 22.5 / 18.2
+    (128, 2, 43, 0, 1200, 2), (128, 2, 43, 0, 1199, 1),       # 600 KB with two at heads above, up to three eighths of the units
+    (128, 2, 48, 0, 1200, 2), (128, 2, 49, 0, 1535, 1), (128, 2, 49, 0, 1536, 2),      # 768 KB beyond
+    (128, 2, 56, 0, 1400, 1),                # 24.1 / 27
+    (256, 2, 40, 0, 320, 3), (256, 2, 40, 0, 319, 1), (32, 2, 20, 0, 2560, 6), (32, 2, 20, 0, 2559, 1),
+    # beside portions: 384 KB from five splits on, 768 below
+    (64, 2, 20, 1, 1536, 6), (64, 2, 20, 1, 1535, 1), (64, 2, 48, 1, 1500, 1), (64, 2, 32, 1, 2000, 1),
+    (64, 2, 32, 1, 3071, 1), (64, 2, 32, 1, 3072, 4), (128, 2, 43, 1, 1535, 1), (128, 2, 43, 1, 1536, 2),
+])
+def test_key_splits_of_decoding_requests(head_dim, nkv, reqs, beside, keys, want):
+    lib = attention_library(head_dim)
+    assert lib.llmlab_attention_decode_splits(7 * nkv, nkv, reqs + beside, reqs, keys, 0, CUS) == want
+
+
 def first_float32_sum(m, n, k, max_pieces, min_steps):
     """Steps of a sum by the estimate of the kernels that add all part products in one sum (64 x 64 and 128 x 128)."""
     steps, best = -(-k // 32), None
