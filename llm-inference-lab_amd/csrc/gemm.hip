@@ -2106,13 +2106,8 @@ static int plain_tile(int M, int N, int K, int num_cus) {
   if (one_round >= 0) return one_round;
   return choose_tile(M, N, K, num_cus);
 }
-// ... its width (for tests)
-extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
-  return TILE_MODELS[plain_tile(M, N, K, num_cus > 0 ? num_cus : 256)].bn;
-}
-
-// The tiles of eight waves by direct loads in place of the tile that the estimates, the plan or a rule above named: those
-// choose among tiles by their sizes (and answer for them); these are faster where all their blocks find a place at once.
+// The tiles of eight waves by direct loads in place of the tile that the estimates, the plan or a rule above named, whose prices
+// and answers are those of the tiles that they choose among; these are faster where all their blocks find a place at once.
 // Every sum keeps its order, so the results are the same to the bit.
 //   128 x 128, a block a unit, in place of 64 x 128 and 128 x 128 in one round, whole or in pieces (beyond 64 rows; us
 //   before / with it): 384 rows of 9728 x 896 13.6 / 11.8, 256 of 11008 x 2048 24.3 / 21.1, 2,048 of 896 x 4864 in two pieces
@@ -2155,6 +2150,12 @@ static int direct_tile(int kind, int M, int N, int K, int pieces, bool heads, in
 extern "C" int llmlab_direct_tile(int kind, int M, int N, int K, int pieces, int heads, int num_cus) {
   const int tile = direct_tile(kind, M, N, K, pieces, heads != 0, num_cus > 0 ? num_cus : 256);
   return tile == kind ? -1 : tile;
+}
+
+// The width of the tile that such a product is launched with (for tests).
+extern "C" int llmlab_plain_tile(int M, int N, int K, int num_cus) {
+  if (num_cus <= 0) num_cus = 256;
+  return TILE_MODELS[direct_tile(addressable(plain_tile(M, N, K, num_cus), K), M, N, K, 1, false, num_cus)].bn;
 }
 
 template <int EPI>
@@ -2286,7 +2287,7 @@ extern "C" int llmlab_pieces_tile(int M, int N, int K, int num_cus, int pieces) 
 }
 
 // Whether (and into how many pieces along K) a product that adds into float32 rows should
-// be left unsummed, and with which tile: out = {pieces (1: no), tile kind}; in one piece the kind is that
+// be left unsummed, and with which tile: out = {pieces (1: no), tile kind}, before direct_tile; in one piece the kind is that
 // of a whole product (choose_tile; up to 128 rows of a wide matrix one_round_tile's widths go before it, which make
 // no pieces).  A piece costs a write and a read of the result by whoever sums it up later.
 extern "C" void llmlab_linear_plan(int M, int N, int K, int num_cus, int max_pieces, int min_tiles_per_piece,
@@ -2395,13 +2396,15 @@ extern "C" int llmlab_linear_qkv(const void* x, const void* w, const void* bias,
   return 0;
 }
 
-// The width of the tile (64, 128 or 256 columns) that a product of these sizes gets (for tests) ...
+// The width of the tile (64, 128 or 256 columns) that the estimates name for a product of these sizes (for tests; direct_tile may
+// put another in its place) ...
 extern "C" int llmlab_linear_tile(int M, int N, int K, int num_cus) {
   if (num_cus <= 0) num_cus = 256;
   return TILE_MODELS[choose_tile(M, N, K, num_cus)].bn;
 }
 
-// ... and that llmlab_linear_qkv takes for heads of d: for callers that must know whether a head fits it.
+// ... and that llmlab_linear_qkv takes for heads of d, and keeps where direct_tile puts another in its place: for callers that must
+// know whether a head fits it.
 extern "C" int llmlab_linear_heads_tile(int M, int N, int K, int d, int num_cus) {
   return TILE_MODELS[heads_tile(M, N, K, d > 0 ? d : 1, num_cus > 0 ? num_cus : 256)].bn;
 }

@@ -58,16 +58,31 @@ def test_tile_and_pieces_of_products_of_many_rows(core):
             assert (m >= 512 or (m > 128 and n >= 16384 and pieces == 1)) and k >= 896, (m, n, k, kind)
 
 
-def test_a_plan_in_one_piece_names_the_tile_that_is_launched(core):
+DIRECT = {10: (128, 128), 11: (128, 192), 12: (192, 128)}      # (by direct loads: put in the place of a tile of KINDS)
+
+
+def launched_width(core, m, n, k, cus=CUS):
+    """Of a whole product whose tile the estimates name."""
+    out = (ctypes.c_int * 2)()
+    core.llmlab_linear_plan(m, n, k, cus, 1, 8, out)
+    direct = core.llmlab_direct_tile(out[1], m, n, k, 1, 0, cus)
+    return (KINDS[out[1]] if direct < 0 else DIRECT[direct])[1]
+
+
+def test_a_plan_in_one_piece_names_the_tile_of_the_whole_product(core):
+    """That the estimates name, and with the direct tiles in their place that which is launched."""
     rng = random.Random(9)
-    whole = 0
+    whole = direct = 0
     for _ in range(20000):
         m, n, k = rng.randint(17, 2560), 16 * rng.randint(4, 700), 8 * rng.randint(8, 900)
         pieces, kind = plan(core, m, n, k)
         if pieces == 1:
             whole += 1
             assert KINDS[kind][1] == core.llmlab_linear_tile(m, n, k, CUS), (m, n, k, kind)
-    assert whole > 5000
+            if m > 128 or k < 1024:      # (else one_round_tile is asked first)
+                assert core.llmlab_plain_tile(m, n, k, CUS) == launched_width(core, m, n, k), (m, n, k, kind)
+                direct += launched_width(core, m, n, k) != KINDS[kind][1]
+    assert whole > 5000 and direct > 100
 
 
 @pytest.mark.parametrize("m,n,k,pieces,want", [
@@ -178,15 +193,15 @@ def test_one_round_of_blocks(core, m, n, k, columns):
 
 
 def test_one_round_of_blocks_is_one_round(core):
-    """Over sizes drawn at random: where the tile is not the one that the estimates pick, its blocks find a compute unit
-    each and leave few without one; beyond 128 rows and at short inner sizes it is the estimates' always."""
+    """Over sizes drawn at random: where the tile is not the one that the estimates pick (or the direct one in its place), its blocks
+    find a compute unit each and leave few without one; beyond 128 rows and at short inner sizes it is the estimates' always."""
     rng = random.Random(7)
     differs = 0
     for _ in range(5000):
         m = rng.choice([rng.randint(17, 64), rng.randint(65, 128), rng.randint(129, 3000)])
         n, k = rng.randint(64, 70000), 8 * rng.randint(16, 1500)
         cus = rng.choice([CUS, 304, 64])
-        columns, estimates = core.llmlab_plain_tile(m, n, k, cus), core.llmlab_linear_tile(m, n, k, cus)
+        columns, estimates = core.llmlab_plain_tile(m, n, k, cus), launched_width(core, m, n, k, cus)
         if m > 128 or k < 1024:
             assert columns == estimates, (m, n, k)
         if columns == estimates:
