@@ -1095,93 +1095,93 @@ __device__ __forceinline__ void attention_rows(const AttnArgs& a, const int xblk
       __syncthreads();
     }
     const int kb0 = tile * KT + ph * GK;
-    if (kb0 <= p_last && kb0 + GK > key_lo) {      // (else none of the wave's rows sees any of these keys)
-      floatx16 s[NS];
+    floatx16 s[NS];
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) s[st][x] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk)
+#pragma unroll
+      for (int st = 0; st < NS; ++st) s[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk][st], qf[kk], s[st], 0, 0, 0);
+    // (the values of the first 32 keys travel while the maximum is found)
+    bf16x8 vf[2][DV];
+    auto values = [&](bf16x8 (&f)[DV], int block) {
+#pragma unroll
+      for (int i = 0; i < DV; ++i) {
+        const char* at = vs + block * BLK + i * 1024;
+        const bf16x4 v0 = *(const bf16x4*)at, v1 = *(const bf16x4*)(at + 256);
+        f[i] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+    };
+    values(vf[0], 0);
+    values(vf[1], 1);
+    if (!(kb0 + GK - 1 <= p_first && kb0 >= full_lo && !missing)) {      // some of the keys are not for every row
 #pragma unroll
       for (int st = 0; st < NS; ++st)
 #pragma unroll
-        for (int x = 0; x < 16; ++x) s[st][x] = 0.f;
+        for (int sub = 0; sub < 2; ++sub) {
+          const int k16 = kb0 + st * 32 + sub * 16;
+          const bool ok = !missing || there(k16);
 #pragma unroll
-      for (int kk = 0; kk < DK; ++kk)
-#pragma unroll
-        for (int st = 0; st < NS; ++st) s[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk][st], qf[kk], s[st], 0, 0, 0);
-      // (the values of the first 32 keys travel while the maximum is found)
-      bf16x8 vf[2][DV];
-      auto values = [&](bf16x8 (&f)[DV], int block) {
-#pragma unroll
-        for (int i = 0; i < DV; ++i) {
-          const char* at = vs + block * BLK + i * 1024;
-          const bf16x4 v0 = *(const bf16x4*)at, v1 = *(const bf16x4*)(at + 256);
-          f[i] = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+          for (int i = 0; i < 8; ++i) {
+            const unsigned from_lo = (unsigned)(k16 + 8 * (i >> 2) + (i & 3) + lane_key);
+            s[st][sub * 8 + i] = ok && from_lo <= span ? s[st][sub * 8 + i] : NEG_INF;
+          }
         }
-      };
-      values(vf[0], 0);
-      values(vf[1], 1);
-      if (!(kb0 + GK - 1 <= p_first && kb0 >= full_lo && !missing)) {      // some of the keys are not for every row
+      // Behind the wave's last position, and where no window of its rows reaches, values may be anything (another row's may be
+      // infinite): out of the products, although their probability is zero.  (Steps that none of the wave's rows sees could be left out;
+      // but a branch around all of a step costs every step: a prompt of 4,096 at heads of 64 51.2 us with it, 49.3 so.)
+      if (kb0 + GK - 1 > p_last || kb0 + GK <= key_lo)
 #pragma unroll
-        for (int st = 0; st < NS; ++st)
+        for (int block = 0; block < 2; ++block) {
+          // how far the first of the lane's keys {0 .. 3, 8 .. 11} lies behind the last that is kept
+          int past = kb0 + GK <= key_lo ? GK : kb0 + block * 16 + 4 * h - p_last;
+          asm volatile("" : "+v"(past));
 #pragma unroll
-          for (int sub = 0; sub < 2; ++sub) {
-            const int k16 = kb0 + st * 32 + sub * 16;
-            const bool ok = !missing || there(k16);
+          for (int x = 0; x < 4; ++x) {
+            const int at = past + 8 * (x >> 1) + 2 * (x & 1);
+            const unsigned keep = ((unsigned)((at - 1) >> 31) & 0xffffu) | ((unsigned)(at >> 31) & 0xffff0000u);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              const unsigned from_lo = (unsigned)(k16 + 8 * (i >> 2) + (i & 3) + lane_key);
-              s[st][sub * 8 + i] = ok && from_lo <= span ? s[st][sub * 8 + i] : NEG_INF;
+            for (int i = 0; i < DV; ++i) {
+              uintx4 v = __builtin_bit_cast(uintx4, vf[block][i]);
+              v[x] &= keep;
+              vf[block][i] = __builtin_bit_cast(bf16x8, v);
             }
           }
-        // behind the wave's last position values may be anything (another row's may be infinite): out of the products,
-        // although their probability is zero
-        if (kb0 + GK - 1 > p_last)
+        }
+    }
+    // the maximum of the raw scores, then into the units of the exponent (the scale is positive)
+    float mx[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};
 #pragma unroll
-          for (int block = 0; block < 2; ++block) {
-            int past = kb0 + block * 16 + 4 * h - p_last;      // how far the first of the lane's keys {0 .. 3, 8 .. 11} lies behind it
-            asm volatile("" : "+v"(past));
+    for (int st = 0; st < NS; ++st)
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              const int at = past + 8 * (x >> 1) + 2 * (x & 1);
-              const unsigned keep = ((unsigned)((at - 1) >> 31) & 0xffffu) | ((unsigned)(at >> 31) & 0xffff0000u);
+      for (int x = 0; x < 16; x += 2) mx[(x >> 1) & 3] = max3_raw(s[st][x], s[st][x + 1], mx[(x >> 1) & 3]);
+    mx[0] = max_raw(max3_raw(mx[0], mx[1], mx[2]), mx[3]);
+    if (__any(mx[0] * scale2 > m + LAZY_MAX)) {            // some row's maximum grew: rescale what is summed so far
+      mx[0] = max_across_32(mx[0]) * scale2;
+      const bool grow = mx[0] > m + LAZY_MAX;
+      const float m_new = grow ? mx[0] : m;
+      const float alpha = grow ? fast_exp2(m - m_new) : 1.f;     // 2^-inf = 0 the first time
+      lsum *= alpha;
 #pragma unroll
-              for (int i = 0; i < DV; ++i) {
-                uintx4 v = __builtin_bit_cast(uintx4, vf[block][i]);
-                v[x] &= keep;
-                vf[block][i] = __builtin_bit_cast(bf16x8, v);
-              }
-            }
-          }
-      }
-      // the maximum of the raw scores, then into the units of the exponent (the scale is positive)
-      float mx[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};
+      for (int i = 0; i < DV; ++i)
 #pragma unroll
-      for (int st = 0; st < NS; ++st)
+        for (int x = 0; x < 16; ++x) o[i][x] *= alpha;
+      m = m_new;
+    }
+    const float neg_m = m == NEG_INF ? 0.f : -m;      // (no visible key yet: every p of the row is 2^-inf = 0)
 #pragma unroll
-        for (int x = 0; x < 16; x += 2) mx[(x >> 1) & 3] = max3_raw(s[st][x], s[st][x + 1], mx[(x >> 1) & 3]);
-      mx[0] = max_raw(max3_raw(mx[0], mx[1], mx[2]), mx[3]);
-      if (__any(mx[0] * scale2 > m + LAZY_MAX)) {            // some row's maximum grew: rescale what is summed so far
-        mx[0] = max_across_32(mx[0]) * scale2;
-        const bool grow = mx[0] > m + LAZY_MAX;
-        const float m_new = grow ? mx[0] : m;
-        const float alpha = grow ? fast_exp2(m - m_new) : 1.f;     // 2^-inf = 0 the first time
-        lsum *= alpha;
+    for (int block = 0; block < 2 * NS; ++block) {
+      float pv[8];
 #pragma unroll
-        for (int i = 0; i < DV; ++i)
+      for (int i = 0; i < 8; ++i) pv[i] = fast_exp2(fmaf(s[block >> 1][(block & 1) * 8 + i], scale2, neg_m));
+      lsum += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+      bf16x8 pf;
 #pragma unroll
-          for (int x = 0; x < 16; ++x) o[i][x] *= alpha;
-        m = m_new;
-      }
-      const float neg_m = m == NEG_INF ? 0.f : -m;      // (no visible key yet: every p of the row is 2^-inf = 0)
+      for (int i = 0; i < 8; ++i) pf[i] = (bf16_t)pv[i];
 #pragma unroll
-      for (int block = 0; block < 2 * NS; ++block) {
-        float pv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pv[i] = fast_exp2(fmaf(s[block >> 1][(block & 1) * 8 + i], scale2, neg_m));
-        lsum += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
-        bf16x8 pf;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pf[i] = (bf16_t)pv[i];
-#pragma unroll
-        for (int i = 0; i < DV; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[block & 1][i], pf, o[i], 0, 0, 0);
-      }
+      for (int i = 0; i < DV; ++i) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[block & 1][i], pf, o[i], 0, 0, 0);
     }
     slot = slot == NST - 1 ? 0 : slot + 1;
   }
@@ -2101,7 +2101,7 @@ static int choose_many_rows_launch(long max_rows, int nkv, int live, int max_q_l
 // 64 rows, and `walk`, the keys that a tile walks on average (us, 1x4 / 2x4 / 4x2 / 4x1 at heads of 64): a prompt of 1,024 of 14 heads
 // over 2 (224 blocks) 12.9 / 13.3 / 18.1 / --, of 1,536 (336) 19.6 / 18.3 / 23.7 / --; 64 requests of 93 tokens of 2 over 1 x 4 (768, walk 47)
 // 16.2 / 13.6 / 9.3 / 7.9, 8 of 318 of 16 over 4 (640, 159) 17.1 / 14.4 / 11.0 / 10.3, 64 of 229 of 1 over 1 (256, 115) 7.4 / 7.4 / 8.8 / 9.6;
-// 32 of 512 of 16 over 2 (4,096, 256) 99 / 63 / 42 / 31; 1,210 of 28 over 4 (532, 641) 22.4 / 17.8 / 20.0 / 23.6.  At heads of 128 (2x4 / 2x2
+// 32 of 512 of 16 over 2 (4,096, 256) 99 / 63 / 42 / 31; 8,192 of 14 over 2 (1,792, 4,096) -- / 160 / 148 / 153; 1,210 of 28 over 4 (532, 641) 22.4 / 17.8 / 20.0 / 23.6.  At heads of 128 (2x4 / 2x2
 // / 4x1): 512 tokens of 28 over 4 (224) 14.8 / 14.6 / 18.9, 768 (336) 24 / 20 / 25, 464 behind 3,000 (204) 42.5 / 51 / 81, 2,048 (896) 68 / 51 /
 // 57, 3,072 (1,344) 126 / 98 / 90; 64 of 186 of 4 over 2 (768, walk 93) 28.3 / 18.6 / 13.6, 336 of 64 over 16 in a window of 251 (336, 168)
 // 17.6 / 11.6 / 13.0.  Hardly a step of keys: 4x1.  (Over 1,250 steps drawn at random the picks lose 1.1 and 0.5 % to the best of
@@ -2133,7 +2133,8 @@ static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int
     if (max_ctx_len <= 64) return ROWS_4x1;
     if (8 * blocks <= 7L * num_cus) return ROWS_1x4;
     if ((blocks > num_cus && walk <= 160) || (blocks > 2L * num_cus && walk <= 512)) return ROWS_4x1;
-    return blocks <= 3L * num_cus ? ROWS_2x4 : blocks <= 4L * num_cus ? ROWS_4x2 : ROWS_4x1;
+    if (blocks <= 3L * num_cus) return ROWS_2x4;
+    return blocks > 8L * num_cus || (blocks > 4L * num_cus && walk <= 1536) ? ROWS_4x1 : ROWS_4x2;
   }
   if (max_ctx_len <= 32 || blocks > 4L * num_cus || (blocks >= 2L * num_cus && walk <= 224)) return ROWS_4x1;
   return blocks <= num_cus && walk > 384 ? ROWS_2x4 : ROWS_2x2;

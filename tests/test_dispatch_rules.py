@@ -383,7 +383,9 @@ def test_attention_launch_is_one_the_head_size_has(head_dim, nq, nkv):
     (64, 1, 1, BF16, 257, 64, 128, 10), (64, 1, 1, BF16, 257, 64, 129, 8), (64, 1, 1, BF16, 256, 64, 128, 8),
     (64, 1, 1, BF16, 513, 64, 480, 10), (64, 1, 1, BF16, 513, 64, 481, 8), (64, 1, 1, BF16, 512, 64, 480, 8),
     (64, 1, 1, BF16, 768, 64, 481, 8), (64, 1, 1, BF16, 769, 64, 481, 9), (64, 1, 1, BF16, 1024, 64, 481, 9),
-    (64, 1, 1, BF16, 1025, 64, 481, 10),
+    (64, 1, 1, BF16, 1025, 64, 481, 10), (64, 1, 1, BF16, 1025, 64, 1504, 10), (64, 1, 1, BF16, 1025, 64, 1505, 9),
+    (64, 1, 1, BF16, 2048, 64, 1505, 9), (64, 1, 1, BF16, 2049, 64, 1505, 10),
+    (64, 14, 2, BF16, 1, 8192, 0, 9),        # a long prompt: 148 us against 153 with 4 x 1 and 160 with 2 x 4
     (128, 28, 4, BF16, 1, 4, 1500, 8),       # 21 us against 27 with the key split
     (128, 28, 4, BF16, 1, 96, 4000, 8),      # 43 against 47
     (128, 28, 4, BF16, 1, 128, 2560, 8),
