@@ -913,12 +913,14 @@ __global__ __launch_bounds__(256 * PH, (D <= 64 && PH == 1) ? 2 : 1) void attent
 // four groups of a block of 16 values by an odd 16 of d lie exchanged in pairs (the direct loads' lanes fetch them so): a
 // read takes both halves of 32 numbers of d, which then meet different banks.
 //
-// What bounds it: the vector instructions of the softmax (32 x 32 scores: 538 clocks of a SIMD at heads of 64, 16 of them an
-// exponential) beside 256 (heads of 128: 512) of matrix instructions, which overlap where a SIMD has four waves (heads of 64: two
-// blocks a unit, 455 clocks measured for both) and hardly where it has two (813); and how evenly a prompt's triangle
-// lies on the units.  Against the kernels below it (us, old -> new): 14 heads of 64 over 2, a prompt of 1,024 16.7 -> 12.9, of
-// 2,048 31.3 -> 21.6, of 4,096 78 -> 54; 2,000 tokens behind 3,000 85 -> 52; 28 heads of 128 over 4, three prompts of 1,000, 789
-// and 578 66 -> 35, a prompt of 4,096 268 -> 146, 1,000 tokens behind 1,500 86 -> 46.  The scores of the next stage
+// What bounds it: no unit alone, but each wave's chain from barrier to barrier.  A step of a wave, 32 keys by 32 rows, is 8 matrix
+// instructions at heads of 64 (256 clocks of a SIMD; of 128: 16, 512), 75 vector instructions and 16 exponentials, and 8 KB
+// (16) read from LDS.  A prompt of 4,096 of 14 heads of 64 over 2 would take 12 us by its matrix instructions alone (at 2.4 GHz) and
+// 12 by LDS; it takes 53, and 44 without maxima and exponentials; of 28 heads of 128 over 4 133, 120 without them, 48 by the matrix
+// instructions; and how evenly a prompt's triangle lies on the units counts.  Against the launches that these took the place of (us, old ->
+// new): 14 heads of 64 over 2, a prompt of 1,024 15.8 -> 11.2, of 2,048 31.3 -> 20.4, of 4,096 79 -> 53, of 8,192 217 -> 146; 2,000 tokens
+// behind 3,000 78 -> 46; 28 heads of 128 over 4, three prompts of 1,000, 789 and 578 64 -> 30, a prompt of 4,096 267 -> 133, 1,000 tokens
+// behind 1,500 79 -> 43.  The scores of the next stage
 // before the softmax of this one: no faster.  A load from the block table under a branch in the loop (or of the queries before it)
 // makes the compiler wait there for all that is on its way, every step: hence table_entry, and the queries' use before the loop.
 #define STAGED_ROWS (HEAD_DIM == 64 || HEAD_DIM == 128)
