@@ -2156,6 +2156,12 @@ static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int
 // over 4), against the launches below: 64 tokens from their start 23 -> 18 us and 58 -> 38; 464 behind 1,100 beside 48 at 1,400
 // 23.3 -> 17.0; 256 of heads of 128 behind 1,100 70 -> 56; 900 behind 1,100 at heads of 64 40 -> 35; 1,900 of heads of 64 would
 // lose 7 to 13 %, 464 of heads of 128 7 to 25 %.
+// That was before the second of two launches took keys staged in LDS.  Against those (200 steps drawn at random, heads of 64 and
+// 128) this one takes 0.74 and 0.69 of the time where the rule sends a step here; at heads of 64 it is equal (0.97) from 620
+// blocks on where the portions begin their prompts, and loses where they have histories (938 tokens behind 2,121 beside 70 at 359 37.6 / 28.7 us,
+// 717 behind 2,198 beside 8 at 787 32.9 / 30.7): the call's longest context may be a decoding request's, so the rule cannot
+// tell the two apart.  Where it does not send a step here, this launch would win with few tiles (128 tokens behind 2,048 beside 63
+// at 2,048 15.3 / 19.1 and 45.2 / 51.7, at heads of 128 150 from their start beside 48 at 300 10.5 / 17.3).
 static bool mixed_step_by_small_tiles(long blocks16, long blocks32, long short_blocks, int short_ring, bool deep, int path,
                                       int max_ctx_len, int num_cus) {
   if (D > 128) return false;                   // (not measured)
@@ -2172,7 +2178,8 @@ static bool mixed_step_by_small_tiles(long blocks16, long blocks32, long short_b
 // tokens behind 2,048 keys beside 63 requests decoding at 2,048: 28 us against 38 in two
 // launches; a portion of 512 (224 blocks) beside 31 at 1,024: 27 against 30, beside 127 at
 // 1,024: 68 against 59, hence not there.  Heads of 128, 128 tokens beside 63 at 2,048: 75
-// against 90.
+// against 90.  (With keys staged in LDS in the second launch, 15 steps drawn at random where the rule takes the one: 0.73
+// of the time, 0.88 at most; the first of these 19 us against 31, the last 52 against 72.)
 static bool mixed_step_in_one_launch(long long_blocks, long short_blocks, int num_cus, int forced) {
   if (forced > 0) return false;
   if (forced < 0) return true;

@@ -466,23 +466,23 @@ def test_order_of_float32_blocks(head_dim, pairs, seen, want):
 @pytest.mark.parametrize("head_dim,nq,nkv,portion,behind,decoding,their_keys,want", [
     # (us in two launches / in one with the portion by tiles of 32 rows / in one by tiles of 16; the rules are in
     # csrc/attention.hip.  2: two launches, 1: one by tiles of 32 rows, 3: one by tiles of 16)
-    (64, 14, 2, 128, 2048, 63, 2048, 1),     # 34.2 / 21.6 / 16.6
-    (64, 14, 2, 256, 1024, 31, 1024, 1),     # 24.1 / 15.5 / 14.5
-    (64, 14, 2, 512, 1536, 31, 1024, 3),     # 28.0 / 19.0 / 20.5
-    (64, 14, 2, 512, 1536, 127, 1024, 3),    # 33.1 / 29.5 / 26.8
-    (64, 14, 2, 512, 1536, 63, 512, 3),      # 25.6 / 23.0 / 21.1
-    (64, 14, 2, 464, 1100, 48, 1400, 3),     # 28.7 / 24.4 / 17.6
-    (64, 14, 2, 64, 0, 48, 300, 3),          # 12.4 / -- / 6.9
-    (64, 14, 2, 1024, 1100, 48, 1400, 3),    # 36.9 / -- / 31.2: 896 blocks, three and a half a unit
-    (64, 14, 2, 1025, 1100, 48, 1400, 2),    # (1,100 tokens: 37.5 / -- / 35.5)
-    (64, 14, 2, 512, 2560, 48, 1400, 3),     # 33.2 / 29.9 / 29.6: 3,072 keys
-    (64, 14, 2, 512, 2600, 48, 1400, 1),     # 34.5 / 29.8 / 30.0
-    (128, 28, 4, 128, 2048, 63, 2048, 1),    # 87.5 / 64.1 / 57.6
-    (128, 40, 8, 128, 2048, 127, 1024, 3),   # 141 / 123 / 115
-    (128, 28, 4, 512, 512, 63, 2048, 2),     # 74.6 / -- / 79.9
-    (128, 28, 4, 146, 0, 48, 1400, 3),       # 38.6 / -- / 28.3: 256 blocks, one a unit
-    (128, 28, 4, 147, 0, 48, 1400, 2),       # 38.1 / -- / 28.0
-    (128, 28, 4, 900, 1100, 48, 1400, 2),    # 93.6 / -- / 101
+    (64, 14, 2, 128, 2048, 63, 2048, 1),     # 30.9 / 19.1 / 15.3
+    (64, 14, 2, 256, 1024, 31, 1024, 1),     # 20.0 / 12.7 / 13.2
+    (64, 14, 2, 512, 1536, 31, 1024, 3),     # 23.4 / 16.5 / 18.6
+    (64, 14, 2, 512, 1536, 127, 1024, 3),    # 31.6 / 27.3 / 25.7
+    (64, 14, 2, 512, 1536, 63, 512, 3),      # 21.0 / 19.3 / 19.4
+    (64, 14, 2, 464, 1100, 48, 1400, 3),     # 24.9 / 21.0 / 16.4
+    (64, 14, 2, 64, 0, 48, 300, 3),          # 11.6 / -- / 6.8
+    (64, 14, 2, 1024, 1100, 48, 1400, 3),    # 28.6 / -- / 30.4: 896 blocks, three and a half a unit (from its start 17.2 / 17.7)
+    (64, 14, 2, 1025, 1100, 48, 1400, 2),    # 29.1 / -- / 30.1
+    (64, 14, 2, 512, 2560, 48, 1400, 3),     # 30.7 / 27.7 / 25.7: 3,072 keys
+    (64, 14, 2, 512, 2600, 48, 1400, 1),     # 31.6 / 27.8 / 28.3
+    (128, 28, 4, 128, 2048, 63, 2048, 1),    # 72.0 / 51.7 / 45.2
+    (128, 40, 8, 128, 2048, 127, 1024, 3),   # 130 / 119 / 116
+    (128, 28, 4, 512, 512, 63, 2048, 2),     # 62.2 / -- / 69.3
+    (128, 28, 4, 146, 0, 48, 1400, 3),       # 36.0 / -- / 25.5: 256 blocks, one a unit
+    (128, 28, 4, 147, 0, 48, 1400, 2),       # 35.7 / -- / 25.4
+    (128, 28, 4, 900, 1100, 48, 1400, 2),    # 59 / -- / 85
     (256, 8, 8, 64, 0, 8, 300, 2),           # (no small tiles at such heads)
 ])
 def test_measured_launches_of_a_mixed_step(head_dim, nq, nkv, portion, behind, decoding, their_keys, want):
