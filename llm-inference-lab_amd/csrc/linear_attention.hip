@@ -91,7 +91,7 @@ extern "C" int llmlab_gla_decay(const float* low, int ld, int rows, int rank, co
     hipLaunchKernelGGL(kernel, dim3((rows + per - 1) / per, chunks), dim3(256), rank * per * sizeof(float), stream, low, ld, rows,
                        rank, w2, bias, kind, 1.0f / tau, decay, channels, as_log);
   };
-  const long blocks = (long)rows * chunks;
+  const long blocks = (long)rows * chunks;      // (of one row; two and five and a half a unit of an MI355X)
   if (blocks <= 512 || rank > 1024) launch(gla_decay_kernel<1>, 1);      // (ranks beyond: LDS)
   else if (blocks <= 1400) launch(gla_decay_kernel<2>, 2);
   else launch(gla_decay_kernel<4>, 4);
