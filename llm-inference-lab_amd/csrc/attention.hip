@@ -1921,18 +1921,37 @@ static int launch_f32_key_split(AttnArgs a, int reqs, int live, int ctx_len, int
   return 0;
 }
 
-// Whether the blocks of a float32 step, keys split over a block's waves, come in the order of their tiles, the longest of all kv heads and
-// requests first, or request by request.  By tiles the units end together; but then the blocks of a request's kv head are far
-// apart, and once the keys and values of all of them, `pairs` times `seen` keys, are more than the caches of the dies hold, every tile reads them from
-// beyond (us, by tiles / by requests: 400 pairs of 741 keys of 64 numbers (152 MB) 2,389 / 1,430, 512 of 634 of 48 (125 MB) 1,889 / 1,150, 200 of
-// 1,194 of 48 (92 MB) 1,108 / 746; 128 of 1,021 of 32 (33 MB) 108 / 145; from 64 to 128 MB 0.82 of the time over 26 steps drawn at random, from 32 to 64 0.98, below
-// 1.03 to 1.06).
-static bool f32_tiles_first(long pairs, long seen) { return pairs * seen * D * 8 < 64L << 20; }
-extern "C" int llmlab_attention_f32_tiles_first(int pairs, int seen) { return f32_tiles_first(pairs, seen); }      // (for tests)
+// By which blocks a float32 step whose waves split the keys of a tile goes, and in which order.
+// Heads up to 64: 16 rows by four waves, four blocks a unit (see `f32_lean`); 16 rows by eight where the tiles leave units idle
+// and have keys to walk (us, four / eight waves: 100 tokens behind 1,000 keys 20.2 / 16.0, behind 3,000 48.5 / 35.5; 300 behind 1,000 (264 tiles)
+// 27.9 / 31; a prompt of 150 6.3 / 7.0); 32 rows by eight, which read a tile's keys half as often, behind histories, where such tiles fill a
+// round of the units or more than one and a half (us, 16 rows / 32: 5 x 160 behind 5,847 of 8 heads of 16 over 2 60 / 43; between the two either may win), or where all keys and values together are 128 MB and more
+// (22 x 61 behind 5,007 of 16 heads of 64 over 8 531 / 380, 17 x 322 behind 5,255 of 8 over 8 945 / 733).  Wider heads have one form.
+// The order: the tiles with the longest histories of all kv heads and requests first, along x, so that the units end together, while the
+// chip holds most of the blocks at a time or their keys lie in the caches; beyond, blocks of far requests share a unit's time and every one reads
+// its keys from beyond the caches (us, by tiles / by requests: 8 x 1,786 behind 4,794 of 14 heads of 64 over 2 1,733 / 850, 16 x 599 behind 2,412 503 / 351;
+// one of 867 of 16 heads over 8 28.5 / 38.4, 972 x 2 of 8 heads of 16 13.6 / 18.8).  Tiles of 32 rows and wider heads go by requests: by tiles
+// they gained nothing together and lost up to twice (8 x 1,033 behind 2,226 of 28 heads of 128 over 4 1,081 / 549).
+// Against tiles of 32 rows by eight waves in the order of the requests for all of them: heads of 16 to 64, 2,774 steps drawn at
+// random 0.84 of the time, 1 % of them more than 5 % slower (11 % with the order by the total of keys alone), at most 1.3; 500 steps of prompts of 800 to 8,000 0.88, 1.07 at most.
+enum { F32_ROWS_16x4 = 1, F32_ROWS_16x8 = 2, F32_ROWS_32x8 = 3, F32_BY_TILES = 16 };
+static int f32_blocks(long max_rows, int nkv, int live, int max_q_len, int max_ctx_len, int window, int num_cus) {
+  if (D > 64) return F32_ROWS_32x8;          // (their one form)
+  const long blocks16 = (max_rows + 15) / 16 * nkv * live, blocks32 = (max_rows + 31) / 32 * nkv * live;
+  auto in_window = [&](int keys) { return window > 0 ? min(window, keys) : keys; };
+  const int history = in_window(max_ctx_len - max_q_len), walk = in_window(max_ctx_len - max_q_len / 2);
+  const int seen = window > 0 ? (int)min((long)max_ctx_len, (long)window + max_q_len) : max_ctx_len;
+  const long bytes = (long)nkv * live * seen * D * 8;
+  const bool rounds32 = 2 * blocks32 > num_cus && (20 * blocks32 <= 21L * num_cus || 2 * blocks32 > 3L * num_cus);
+  if ((history >= 768 && rounds32) || bytes >= 128L << 20) return blocks16 <= num_cus ? F32_ROWS_16x8 : F32_ROWS_32x8;
+  const int form = blocks16 <= num_cus && max_ctx_len >= 768 ? F32_ROWS_16x8 : F32_ROWS_16x4;
+  return form + (live == 1 || blocks16 <= 8L * num_cus || (walk <= 512 && bytes <= 8L << 20) ? F32_BY_TILES : 0);
+}
 
 // Which launch a float32 step of many rows takes: 1 = the waves of a block split the keys of a
 // tile, anything else = a wave per tile.  `max_rows`: of a request and kv head; `blocks`: tiles of rows times kv heads times requests.
-static int choose_many_rows_launch_f32(long max_rows, long blocks, int max_q_len, int max_ctx_len, int num_cus, int forced) {
+static int choose_many_rows_launch_f32(long max_rows, long blocks, int max_q_len, int max_ctx_len, int window, int num_cus,
+                                       int forced) {
   if (forced != 0) return forced;
   // (how few the keys must be for a wave per tile, by how many times the tiles fill the chip)
   int few_keys;
@@ -1953,6 +1972,8 @@ static int choose_many_rows_launch_f32(long max_rows, long blocks, int max_q_len
     else few_keys = quarters >= 400 ? 1024 : quarters >= 56 ? 512 : quarters >= 28 ? 256 : quarters >= 14 ? 192 : quarters >= 7 ? 64 : 0;
     // (a block of four waves whose tiles are less than three quarters full)
     if (few_keys > 128 && 4 * max_rows < 3 * ((max_rows + 127) / 128 * 128)) few_keys = 128;
+    // (a window bounds what a tile walks: 11 x 794 tokens of 32 heads of 64 over 8 in a window of 32 75 / 54)
+    if (window > 0) max_ctx_len = (int)min((long)max_ctx_len, (long)window + 16);
   }
   return max_ctx_len <= few_keys ? 2 : 1;
 }
@@ -1990,22 +2011,23 @@ static int launch_attention_f32(AttnArgs a, int reqs, int max_q_len, int max_ctx
   // wave per tile, a prompt of 1,531 tokens 49 against 122.  A wave per tile wins once the
   // tiles fill the chip and the keys are few, at heads above 64 from two tiles a unit on whatever the
   // keys (4 requests of 256 tokens: 58 against 81).
-  const int path = choose_many_rows_launch_f32(max_rows, tiles * a.nkv * live, max_q_len, max_ctx_len, num_cus, g_force_path);
+  const int path = choose_many_rows_launch_f32(max_rows, tiles * a.nkv * live, max_q_len, max_ctx_len, window, num_cus, g_force_path);
   if (path == 1) {
-    // Heads up to 64: blocks of four waves and 16 rows, four to a unit; eight waves where the tiles leave units idle and
-    // have histories to walk (us, four / eight waves: 100 tokens behind 1,000 keys 20.2 / 16.0, behind 3,000 48.5 / 35.5; 300
-    // behind 1,000 (264 tiles) 27.9 / 31; a prompt of 150 6.3 / 7.0).
-    constexpr int PATH1_QB = D <= 64 ? 1 : F32_QB;
-    const long path1_tiles = (max_rows + 16 * PATH1_QB - 1) / (16 * PATH1_QB), blocks = path1_tiles * a.nkv * zs;
-    // (along x, the longest tiles of all requests first, where every request is this launch's)
-    const int seen = window > 0 ? min(max_ctx_len, window + max_q_len) : max_ctx_len;
-    const bool along_x = live == (long)zs && blocks <= 0xffffffffl / (64 * F32_SPLIT_WAVES) &&
-                         f32_tiles_first((long)a.nkv * zs, seen);
+    const int how = f32_blocks(max_rows, a.nkv, live, max_q_len, max_ctx_len, window, num_cus), form = how & ~F32_BY_TILES;
+    const int rows = form == F32_ROWS_32x8 ? ROWS : 16;
+    const long path1_tiles = (max_rows + rows - 1) / rows, blocks = path1_tiles * a.nkv * zs;
+    // (by tiles where every request is this launch's)
+    const bool along_x = (how & F32_BY_TILES) && live == (long)zs && blocks <= 0xffffffffl / (64 * F32_SPLIT_WAVES);
+    if (!along_x) a.units = 0x7fffffff;      // (all in one order)
     const dim3 grid = along_x ? dim3((unsigned)blocks) : dim3((unsigned)path1_tiles, a.nkv, zs);
-    if (D <= 64 && !(path1_tiles * a.nkv * live <= num_cus && max_ctx_len >= 768))
-      hipLaunchKernelGGL((attention_f32_kernel<PATH1_QB, true, 4>), grid, dim3(64 * 4), 0, stream, a);
-    else
-      hipLaunchKernelGGL((attention_f32_kernel<PATH1_QB, true, F32_SPLIT_WAVES>), grid, dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
+    if (form == F32_ROWS_32x8)
+      hipLaunchKernelGGL((attention_f32_kernel<F32_QB, true, F32_SPLIT_WAVES>), grid, dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
+    else if constexpr (D <= 64) {
+      if (form == F32_ROWS_16x4)
+        hipLaunchKernelGGL((attention_f32_kernel<1, true, 4>), grid, dim3(64 * 4), 0, stream, a);
+      else
+        hipLaunchKernelGGL((attention_f32_kernel<1, true, F32_SPLIT_WAVES>), grid, dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
+    }
   } else {
     hipLaunchKernelGGL((attention_f32_kernel<F32_QB, false, 4>), dim3((unsigned)((tiles + 3) / 4), a.nkv, zs),
                        dim3(256), 0, stream, a);
@@ -2232,9 +2254,16 @@ extern "C" int llmlab_attention_launch(int dtype, int nq, int nkv, int reqs, int
   if (max_rows <= 16) return 0;
   if (dtype == DT_F32) {
     constexpr int ROWS = 16 * F32_QB;
-    return choose_many_rows_launch_f32(max_rows, (max_rows + ROWS - 1) / ROWS * nkv * reqs, max_q_len, max_ctx_len, num_cus, 0);
+    return choose_many_rows_launch_f32(max_rows, (max_rows + ROWS - 1) / ROWS * nkv * reqs, max_q_len, max_ctx_len, window, num_cus, 0);
   }
   return many_rows_launch(max_rows, nkv, reqs, max_q_len, max_ctx_len, window, false, num_cus, 0);
+}
+
+// By which blocks it goes in float32 where launch 1 is taken (for tests): 1 and 2 = 16 rows by four and by eight waves, 3 = the tile of
+// the wave that takes one by itself; 16 more: in the order of the tiles of all requests.
+extern "C" int llmlab_attention_f32_blocks(int nq, int nkv, int reqs, int max_q_len, int max_ctx_len, int window, int num_cus) {
+  if (nq <= 0 || nkv <= 0 || nq % nkv != 0 || reqs <= 0 || max_q_len <= 0) return -1;
+  return f32_blocks((long)max_q_len * (nq / nkv), nkv, reqs, max_q_len, max_ctx_len, window, num_cus > 0 ? num_cus : 256);
 }
 
 // q rows are the step's packed rows; reqs requests; max_q_len / max_ctx_len are

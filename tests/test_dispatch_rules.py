@@ -453,14 +453,30 @@ def test_launches_in_a_window(head_dim, nq, nkv, reqs, q, behind, window, want):
     assert lib.llmlab_attention_launch(BF16, nq, nkv, reqs, q, behind + q, window, CUS) == want
 
 
-@pytest.mark.parametrize("head_dim,pairs,seen,want", [
-    (64, 400, 741, 0),         # 2,389 us in the order of the tiles, 1,430 request by request
-    (48, 200, 1194, 0),        # 1,108 and 746
-    (32, 128, 1021, 1),        # 108 and 145
-    (64, 2, 65535, 1), (64, 2, 65536, 0), (16, 8, 65535, 1), (16, 8, 65536, 0),      # 64 MB of keys and values
+@pytest.mark.parametrize("head_dim,nq,nkv,reqs,q,behind,window,want", [
+    # (us by 16 rows in the order of the tiles / by 16 rows request by request / by 32 rows request by request; 1 and 2 are 16 rows by
+    # four and eight waves, 3 the tile of 32, 16 more the order of the tiles)
+    (64, 14, 2, 1, 1531, 0, 0, 17),
+    (64, 16, 8, 1, 867, 0, 0, 17),              # 28.5 / 38.4 / --
+    (64, 14, 2, 8, 1786, 4794, 0, 3),           # 1,733 / 850 / 887 (portions of up to so many)
+    (64, 14, 2, 21, 444, 4141, 0, 3),           # 2,446 / 1,308 / 1,365
+    (64, 16, 8, 22, 61, 5007, 0, 3),            # 531 with 16 rows, 380 with 32: 457 MB of keys and values
+    (16, 8, 2, 5, 160, 5847, 0, 3),             # 60 / 59 / 43: 200 tiles of 32 rows
+    (64, 8, 8, 1, 100, 3000, 0, 18), (64, 8, 8, 1, 100, 667, 0, 17), (64, 8, 8, 1, 100, 668, 0, 18),     # 768 keys in all
+    (64, 8, 8, 4, 129, 767, 0, 17), (64, 8, 8, 4, 129, 768, 0, 3),      # 768 keys of history
+    (64, 8, 8, 4, 128, 5000, 0, 18),                                    # (half a tile of 32 rows a unit)
+    (64, 8, 8, 1, 1056, 768, 0, 3), (64, 8, 8, 1, 1088, 768, 0, 17),    # 264 and 272 tiles: a round of the units and a bit
+    (64, 8, 8, 1, 1536, 768, 0, 17), (64, 8, 8, 1, 1537, 768, 0, 3),    # 384 and 392: one and a half
+    (64, 8, 8, 1, 1537, 768, 767, 17), (64, 8, 8, 1, 1537, 768, 768, 3),
+    (64, 8, 8, 16, 256, 0, 0, 17), (64, 8, 8, 16, 257, 0, 0, 1),        # 2,048 and 2,176 tiles of 16 rows
+    (32, 8, 2, 32, 513, 0, 0, 1), (32, 8, 2, 32, 500, 0, 0, 17),        # 8 MB of keys and values
+    (16, 8, 2, 16, 1025, 0, 0, 1), (16, 8, 2, 16, 1024, 0, 0, 17),      # 512 keys that a tile walks
+    (64, 8, 8, 32, 1023, 0, 0, 1), (64, 8, 8, 32, 1024, 0, 0, 3),       # 128 MB
+    (128, 28, 4, 1, 1500, 0, 0, 3), (256, 8, 8, 4, 100, 0, 0, 3),
 ])
-def test_order_of_float32_blocks(head_dim, pairs, seen, want):
-    assert attention_library(head_dim).llmlab_attention_f32_tiles_first(pairs, seen) == want
+def test_blocks_of_float32(head_dim, nq, nkv, reqs, q, behind, window, want):
+    lib = attention_library(head_dim)
+    assert lib.llmlab_attention_f32_blocks(nq, nkv, reqs, q, behind + q, window, CUS) == want
 
 
 @pytest.mark.parametrize("head_dim,nq,nkv,portion,behind,decoding,their_keys,want", [

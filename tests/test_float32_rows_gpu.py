@@ -50,3 +50,21 @@ def test_missing_pages_stay_out(ops, start):  # noqa: F811
         got.append(out)
     assert got[0].isfinite().all()
     assert (got[0] - got[1]).abs().max().item() <= 2e-5 * max(1.0, got[1].abs().max().item())
+
+
+@pytest.mark.parametrize("window", [None, 768])
+@pytest.mark.parametrize("nq,nkv,d", [(8, 8, 64), (8, 8, 48), (8, 4, 32), (8, 8, 16)])
+def test_wide_tiles_behind_histories(ops, emu, window, nq, nkv, d):  # noqa: F811
+    """Tiles of 32 rows by eight waves, which the rule takes behind histories: rows that end inside a tile and in its first half,
+    one row, histories of other lengths in one launch."""
+    spec = [(768, 129), (700, 33), (3, 17), (760, 128), (0, 1 + 16 * nkv // nq)]
+    assert ops._attention_lib(d).llmlab_attention_f32_blocks(nq, nkv, len(spec), 129, 768 + 129, window or 0, ops.num_cus) == 3
+    run_attention(ops, emu, torch.float32, nq, nkv, d, 64, window, spec, seed=117, amplify=(0, 300, 30.0))
+
+
+@pytest.mark.parametrize("nq,nkv,d,reqs,longest,how", [(8, 8, 64, 16, 257, 1), (8, 8, 64, 8, 257, 17), (16, 16, 32, 8, 300, 1)])
+def test_order_of_blocks(ops, emu, nq, nkv, d, reqs, longest, how):  # noqa: F811
+    """More tiles than the chip holds, request by request, and the same kernel by tiles: ragged portions, the longest last."""
+    assert ops._attention_lib(d).llmlab_attention_f32_blocks(nq, nkv, reqs, longest, longest, 0, ops.num_cus) == how
+    with ops.debug.force(attention_path=(d, 1)):
+        run_attention(ops, emu, torch.float32, nq, nkv, d, 64, None, [(0, 1 + 31 * i % 97) for i in range(reqs - 1)] + [(0, longest)], seed=118)
