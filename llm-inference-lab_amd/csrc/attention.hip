@@ -1385,8 +1385,16 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void attention_merge_kernel(
 // 2.60e-7 -> 2.55e-7.  Tiles of 32 rows in the lean form: 49.4 to 49.7 for the first, 38.6 (here 30.9) for 512 behind
 // 1,000; five waves a SIMD spill registers.
 constexpr bool f32_lean(bool split, int waves) { return split && waves == 4 && D <= 64; }
-template <int QB, bool SPLIT, int NW>
-__global__ __launch_bounds__(64 * NW, f32_lean(SPLIT, NW) ? 4 : 1) void attention_f32_kernel(AttnArgs a) {
+// The waves that a SIMD is to hold: the lean form's four; of decode steps' blocks (16 rows) two at heads of 96 to 128 and three at 80, which the
+// compiler otherwise misses by 8 registers (105 requests at 397 beside two portions, 12 heads of 128 over 12, 73.5 us so, 64 as they are).  At heads of
+// 32 and 64 what they would hold but for 4 registers costs one spilled: there DENSE, a kernel of its own, is for steps of more blocks
+// than units hold otherwise over few keys (f32_dense).
+constexpr int f32_waves(int qb, bool split, int waves, bool dense) {
+  return f32_lean(split, waves) ? 4 : qb > 1 || !split ? 1 : D > 128 ? 1 : D > 80 ? 2 : D > 64 ? 3 : !dense ? 1 : D > 32 ? 4 : 6;
+}
+constexpr bool F32_DENSE = D == 64 || D == 32;
+template <int QB, bool SPLIT, int NW, bool DENSE = false>
+__global__ __launch_bounds__(64 * NW, f32_waves(QB, SPLIT, NW, DENSE)) void attention_f32_kernel(AttnArgs a) {
   constexpr bool LEAN = f32_lean(SPLIT, NW);
   constexpr int DQ = D / 16;
   const int lane = threadIdx.x & 63;
@@ -1889,6 +1897,17 @@ extern "C" void llmlab_debug_attention_two_launches(int on) { g_force_two_launch
 // wave per tile (launch_attention_f32 says when).
 constexpr int F32_SPLIT_WAVES = D <= 64 ? 8 : 4;
 constexpr int F32_QB = D <= 128 ? 2 : 1;
+// Whether a float32 decode step's blocks are those of which a unit holds more (heads of 64: two for one, of 32: three for two).  Left alone
+// they are 3 to 6 % faster by themselves and over long histories, whose streams fill a unit; over few keys, and where the step otherwise goes
+// on with a round of few blocks, so many more at a time win (us, alone / dense: 255 requests of 32 heads of 64 over 8 at 88 30.2 / 24.6; 33
+// of 8 over 8 at 71, 264 blocks, 9.5 / 8.1; 1 of 8 over 1 at 1,012 5.6 / 6.1).  Of 230 steps of one to five blocks a unit 0.90 of the time up to 200
+// keys, 0.98 up to 1,000, 1.05 beyond.
+static bool f32_dense(long blocks, int visible, int num_cus) {
+  if (!F32_DENSE || visible > 1024) return false;
+  return D == 64 ? 2 * blocks > (visible <= 256 ? 2L : 3L) * num_cus : blocks > 2L * num_cus;
+}
+extern "C" int llmlab_attention_f32_dense(int blocks, int visible, int num_cus) { return f32_dense(blocks, visible, num_cus); }      // (for tests)
+
 static int launch_f32_key_split(AttnArgs a, int reqs, int live, int ctx_len, int window, int total_rows,
                                 float* workspace, size_t workspace_floats, int num_cus, const int* row_req,
                                 hipStream_t stream) {
@@ -1909,8 +1928,11 @@ static int launch_f32_key_split(AttnArgs a, int reqs, int live, int ctx_len, int
     a.o_part = workspace;
     a.ml_part = workspace + (size_t)total_rows * a.nq * splits * D;
   }
-  hipLaunchKernelGGL((attention_f32_kernel<1, true, F32_SPLIT_WAVES>), dim3(1, a.nkv * splits, reqs),
-                     dim3(64 * F32_SPLIT_WAVES), 0, stream, a);
+  const dim3 grid(1, a.nkv * splits, reqs), block(64 * F32_SPLIT_WAVES);
+  if (f32_dense((long)live * a.nkv * splits, visible, num_cus))
+    hipLaunchKernelGGL((attention_f32_kernel<1, true, F32_SPLIT_WAVES, F32_DENSE>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((attention_f32_kernel<1, true, F32_SPLIT_WAVES>), grid, block, 0, stream, a);
   LLMLAB_LAUNCH_CHECK("attention(float32, decode)");
   if (splits > 1) {
     hipLaunchKernelGGL(attention_merge_kernel<float>, dim3(total_rows, a.nq), dim3(splits > 16 ? 64 * MERGE_WAVES : 64),

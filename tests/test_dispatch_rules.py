@@ -479,6 +479,17 @@ def test_blocks_of_float32(head_dim, nq, nkv, reqs, q, behind, window, want):
     assert lib.llmlab_attention_f32_blocks(nq, nkv, reqs, q, behind + q, window, CUS) == want
 
 
+@pytest.mark.parametrize("head_dim,blocks,keys,want", [
+    (64, 256, 71, 0), (64, 257, 71, 1),              # 33 requests of 8 heads over 8 9.5 us alone, 8.1 dense
+    (64, 257, 256, 1), (64, 257, 257, 0), (64, 384, 257, 0), (64, 385, 257, 1),
+    (64, 2040, 1024, 1), (64, 2040, 1025, 0),
+    (32, 512, 65, 0), (32, 513, 65, 1), (32, 513, 1025, 0),
+    (16, 4096, 65, 0), (48, 4096, 65, 0), (128, 4096, 65, 0),
+])
+def test_dense_decode_blocks_of_float32(head_dim, blocks, keys, want):
+    assert attention_library(head_dim).llmlab_attention_f32_dense(blocks, keys, CUS) == want
+
+
 @pytest.mark.parametrize("head_dim,nq,nkv,portion,behind,decoding,their_keys,want", [
     # (us in two launches / in one with the portion by tiles of 32 rows / in one by tiles of 16; the rules are in
     # csrc/attention.hip.  2: two launches, 1: one by tiles of 32 rows, 3: one by tiles of 16)

@@ -68,3 +68,11 @@ def test_order_of_blocks(ops, emu, nq, nkv, d, reqs, longest, how):  # noqa: F81
     assert ops._attention_lib(d).llmlab_attention_f32_blocks(nq, nkv, reqs, longest, longest, 0, ops.num_cus) == how
     with ops.debug.force(attention_path=(d, 1)):
         run_attention(ops, emu, torch.float32, nq, nkv, d, 64, None, [(0, 1 + 31 * i % 97) for i in range(reqs - 1)] + [(0, longest)], seed=118)
+
+
+@pytest.mark.parametrize("nq,nkv,d,reqs", [(8, 8, 64, 33), (16, 8, 64, 49), (16, 16, 32, 33), (14, 2, 32, 300)])
+@pytest.mark.parametrize("window", [None, 20])
+def test_dense_decode(ops, emu, nq, nkv, d, reqs, window):  # noqa: F811
+    """Decode steps of more blocks than units hold by the plain kernel: histories of one key and of all waves' shares and one more."""
+    assert ops._attention_lib(d).llmlab_attention_f32_dense(reqs * nkv, window or 130, ops.num_cus) == 1
+    run_attention(ops, emu, torch.float32, nq, nkv, d, 16, window, [((0, 1, 15, 16, 127, 128, 129)[i % 7], 1) for i in range(reqs)], seed=119)
