@@ -2167,17 +2167,19 @@ static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int
   if (forced == KEY_SPLIT) return KEY_SPLIT;
   const int history = max_ctx_len - max_q_len, seen = window > 0 ? min(max_ctx_len, window + max_q_len) : max_ctx_len;
   const int middle = max_ctx_len - max_q_len / 2, walk = window > 0 ? min(window, middle) : middle;
-  const long blocks = (max_rows + 63) / 64 * nkv * live;
+  const long blocks = (max_rows + 63) / 64 * nkv * live, bytes = (long)nkv * live * seen * D * 4;
   if (mixed || D == 64) {
     if ((mixed || history >= 1024) &&
         choose_many_rows_launch(max_rows, nkv, live, max_q_len, max_ctx_len, window, num_cus, 0) == KEY_SPLIT)
       return KEY_SPLIT;
-  } else if (2 * ((max_rows + 31) / 32) * nkv * live <= num_cus && (long)nkv * live * seen * D * 4 >= 25L << 20) {
+  } else if (2 * ((max_rows + 31) / 32) * nkv * live <= num_cus && bytes >= 25L << 20) {
     return KEY_SPLIT;
   }
   if (D == 64) {
     if (max_ctx_len <= 64) return ROWS_4x1;
-    if (8 * blocks <= 7L * num_cus) return ROWS_1x4;
+    // (tiles of 32 rows read the keys twice: not where most units have a tile of 64 and keys and values are 24 MB and more, 25 requests of 45 tokens
+    // of 8 heads over 8 behind 5,578 78 us by 1x4, 53 by 2x4; 36 such steps of 160 to 224 tiles 0.87, of 128 to 160 0.98, below 1.1)
+    if (8 * blocks <= (bytes >= 24L << 20 ? 5L : 7L) * num_cus) return ROWS_1x4;
     if ((blocks > num_cus && walk <= 160) || (blocks > 2L * num_cus && walk <= 512)) return ROWS_4x1;
     if (blocks <= 3L * num_cus) return ROWS_2x4;
     return blocks > 8L * num_cus || (blocks > 4L * num_cus && walk <= 1536) ? ROWS_4x1 : ROWS_4x2;

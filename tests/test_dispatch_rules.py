@@ -442,6 +442,8 @@ def test_measured_attention_launches(head_dim, nq, nkv, dtype, reqs, q, behind, 
 @pytest.mark.parametrize("head_dim,nq,nkv,reqs,q,behind,window,want", [
     # (a window bounds what a tile walks, and what all requests read)
     (64, 14, 2, 2, 1521, 0, 33, 10),         # 9.1 us against 14.0 with 2 x 4
+    (64, 8, 8, 25, 45, 5578, 0, 8), (64, 8, 8, 20, 45, 5578, 0, 7),       # 200 and 160 tiles of 64 rows: 78 us by 1 x 4 for the first, 53
+    (64, 8, 8, 25, 45, 447, 0, 8), (64, 8, 8, 25, 45, 446, 0, 7), (64, 8, 8, 25, 45, 600, 447, 8), (64, 8, 8, 25, 45, 600, 446, 7),      # 24 MB
     (64, 16, 8, 8, 298, 0, 32, 10),          # 7.9 against 11.9
     (64, 1, 1, 513, 64, 4000, 512, 10), (64, 1, 1, 513, 64, 4000, 513, 8),
     (128, 8, 2, 1, 80, 6665, 50, 11),        # 7.7 against 9.5
