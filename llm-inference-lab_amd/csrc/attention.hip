@@ -1899,9 +1899,9 @@ constexpr int F32_SPLIT_WAVES = D <= 64 ? 8 : 4;
 constexpr int F32_QB = D <= 128 ? 2 : 1;
 // Whether a float32 decode step's blocks are those of which a unit holds more (heads of 64: two for one, of 32: three for two).  Left alone
 // they are 3 to 6 % faster by themselves and over long histories, whose streams fill a unit; over few keys, and where the step otherwise goes
-// on with a round of few blocks, so many more at a time win (us, alone / dense: 255 requests of 32 heads of 64 over 8 at 88 30.2 / 24.6; 33
-// of 8 over 8 at 71, 264 blocks, 9.5 / 8.1; 1 of 8 over 1 at 1,012 5.6 / 6.1).  Of 230 steps of one to five blocks a unit 0.90 of the time up to 200
-// keys, 0.98 up to 1,000, 1.05 beyond.
+// on with a round of few blocks, so many more at a time win (us, alone / dense, heads of 64: 62 requests of 16 heads over 8 at 159 15.1 / 12.2, 34 of 8
+// over 8 at 95, 272 blocks, 9.5 / 8.9, 78 of 32 over 8 at 2,017 122 / 126).  Of 260 steps of one to five blocks a unit 0.95 of the time on the dense side
+// of the lines at either size, 1.05 and 1.03 on the other.
 static bool f32_dense(long blocks, int visible, int num_cus) {
   if (!F32_DENSE || visible > 1024) return false;
   return D == 64 ? 2 * blocks > (visible <= 256 ? 2L : 3L) * num_cus : blocks > 2L * num_cus;
@@ -2178,7 +2178,7 @@ static int many_rows_launch(long max_rows, int nkv, int live, int max_q_len, int
   if (D == 64) {
     if (max_ctx_len <= 64) return ROWS_4x1;
     // (tiles of 32 rows read the keys twice: not where most units have a tile of 64 and keys and values are 24 MB and more, 25 requests of 45 tokens
-    // of 8 heads over 8 behind 5,578 78 us by 1x4, 53 by 2x4; 36 such steps of 160 to 224 tiles 0.87, of 128 to 160 0.98, below 1.1)
+    // of 8 heads over 8 behind 5,578 78 us by 1x4, 62.5 by 2x4, beside 5 decoding; 15 such steps of 160 to 224 tiles 0.85, 10 of 128 to 160 0.96, below more than 1.04)
     if (8 * blocks <= (bytes >= 24L << 20 ? 5L : 7L) * num_cus) return ROWS_1x4;
     if ((blocks > num_cus && walk <= 160) || (blocks > 2L * num_cus && walk <= 512)) return ROWS_4x1;
     if (blocks <= 3L * num_cus) return ROWS_2x4;
